@@ -1,20 +1,17 @@
 // Linear layer for the few rows of a decode step: out[M, N] = x[M, K] W[N, K]^T + bias, M <= 64, bf16 / fp16.
 // The caller's projections around the attention path (src/myvllm/models/qwen3.py:90-94, 118 and the MLP, :121-160;
-// layers/linear.py) are library GEMMs in the reference.  With a handful of rows such a product reads a few MB of
-// weights once, from HBM (a model's layers do not fit the caches together), and is pure latency: a tiled GEMM walks
-// K in a serial loop of small loads.  Here a workgroup owns 16 output columns, its W waves split K, and a wave asks
-// for its whole share of the weights (and of x, which stays in L2) in one or a few bursts before the first MFMA, so
-// a call costs about one memory round trip.
-//   per wave and 32-wide k step: A = W (row n0 + lane%16, 16 B = 8 k values of class lane/16), B = x^T (column m =
-//   lane%16, the same k values), v_mfma_f32_16x16x32: lane l ends with out[m = l%16][n0 + 4 (l/16) + r], r < 4.
-//   The partial sums meet in LDS; wave 0 adds them, adds the bias and stores 8 bytes per lane.
-// From 17 rows on every 16 rows get workgroups of their own (the same code; the workgroups of one column tile run on
-// one XCD and share the weights in its L2) rather than one workgroup holding up to four row tiles in registers.
+// layers/linear.py) are library GEMMs in the reference.  Such a product reads a few MB to a few hundred MB of weights
+// once, from HBM: what bounds it is that stream, and beside it the address unit of a CU, which takes a 16-byte load of a
+// wave at 64 B per clock where four neighbouring lanes share 64 bytes and at 16 B where they do not (a matrix
+// operand's lanes are sixteen different rows).  Hence two kernels:
+//   linear_rows_kernel (very few rows): weights and x straight into registers, eight rows x 128 bytes per load.
+//   linear_ring_kernel (more rows): W and x through a ring of tiles in LDS, copied as whole 128-byte lines.
+// Both read a weight once.  A sum's order depends on (M, N, K) only, not on what follows the product.
 // mvllm_norm_linear_small_m is the same product with the launches around it folded in: the residual add + RMSNorm in
 // front of the layer's first projections (src/myvllm/models/qwen3.py:197-212 through layers/layernorm.py:9-28) as
-// the kernel's prologue, and SiluAndMul behind the gate/up projection (layers/activation.py:15-18) as its epilogue,
-// each rounding where the separate launch rounds.
-#include "common.h"
+// the kernel's prologue (linear_norm_kernel), and SiluAndMul behind the gate/up projection (layers/activation.py:15-18) as
+// its epilogue, each rounding where the separate launch rounds.
+#include "prefill_tiles.h"
 
 #pragma clang fp contract(off)
 
@@ -27,13 +24,12 @@ struct LinearArgs {
   const void* bias;       // [N] in the element type, or null
   int64_t x_row_stride;   // elements between rows of x
   int M, N, K;
-  int cols;               // output columns per workgroup: 16, or 8 / 4 (plain product only) to spread few columns over more CUs
-  int row_tiles;          // > 1: the grid holds this many workgroups per column tile, one per 16 rows of x (MT == 1)
-  // NORM: x is first replaced by rms_norm(x + residual) * gamma, as mvllm_add_rms_norm computes it
+  // norm: x is first replaced by rms_norm(x + residual) * gamma, as mvllm_add_rms_norm computes it
   const void* residual;   // [M, K] contiguous, or null (then the norm of x alone)
   void* residual_out;     // [M, K] contiguous: x + residual in the element type; must not alias x or residual
   const float* gamma;     // [K]
   float eps;
+  int row_tiles;          // norm: workgroups per column tile, one per 16 rows of x
   int gelu;               // plain product only: the result through the tanh form of gelu
 };
 
@@ -53,33 +49,245 @@ __device__ __forceinline__ void unpack8(uint4 w, float (&x)[8]) {
   x[4] = lo_to_float<T>(w.z); x[5] = hi_to_float<T>(w.z);
   x[6] = lo_to_float<T>(w.w); x[7] = hi_to_float<T>(w.w);
 }
-typedef __attribute__((ext_vector_type(2))) float v2f;
-typedef __attribute__((ext_vector_type(2))) __bf16 v2bf16;
-typedef __attribute__((ext_vector_type(2))) _Float16 v2f16;
-template <typename T> __device__ __forceinline__ uint32_t pack2(float a, float b);
-template <> __device__ __forceinline__ uint32_t pack2<bf16_t>(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f){a, b}, v2bf16));
-}
-template <> __device__ __forceinline__ uint32_t pack2<f16_t>(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f){a, b}, v2f16));
-}
 template <typename T>
 __device__ __forceinline__ uint4 pack8(const float (&x)[8]) {
   return make_uint4(pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]), pack2<T>(x[4], x[5]), pack2<T>(x[6], x[7]));
 }
 
-// NORM (the wave's whole share of K is one burst, K / W == 32 U): the rows are normalised on their way into the
-// product.  Every workgroup needs every row, so each of them forms h = x + residual for all rows, the waves add
+// What follows a product: bias, gelu or the gated unit, rounding.  `s`: out[m][j .. j + 3]; GLU: `u` the up columns that meet them.
+template <typename T, bool GLU>
+__device__ __forceinline__ void finish_four(const LinearArgs& a, int m, int j, float (&s)[4], float (&u)[4]) {
+  const int out_cols = GLU ? a.N / 2 : a.N;
+  if (m >= a.M || j >= out_cols) return;
+  if (a.bias) {
+    const T* bp = reinterpret_cast<const T*>(a.bias) + j;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      s[r] += to_float(bp[r]);
+      if (GLU) u[r] += to_float(bp[out_cols + r]);
+    }
+  }
+  T r4[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if constexpr (GLU) r4[r] = silu_mul_rounded<T>(from_float<T>(s[r]), from_float<T>(u[r]));
+    else r4[r] = from_float<T>(a.gelu ? gelu_tanh(s[r]) : s[r]);
+  }
+  *reinterpret_cast<uint2*>(reinterpret_cast<T*>(a.out) + (int64_t)m * out_cols + j) = *reinterpret_cast<const uint2*>(r4);
+}
+
+// Very few rows.  A load of a wave covers 8 rows x 64 values of K, whole 128-byte lines: lane l holds 8 values of row
+// l % 8 from piece 4 (l / 8 % 2) + l / 16 on.  As operands of v_mfma_f32_16x16x32 such registers are 16 "rows" (row, half of the 64
+// values), so that a product of a weight and an x register is valid where the halves agree, half of the results: the matrix
+// unit, idle otherwise, does twice the work, and the halves meet in the sum over the waves.  (Sixteen rows x 64 bytes per
+// load, the operand's own layout: 26.7 against 20.1 us at N 4096, K 12288 with all else equal; the kernel as a whole against the one it
+// replaces, one row, us: 18.8 / 30.2 there, 33.7 / 40.0 at 24576 x 4096 (6.0 TB/s), 10.9 / 16.1 at 6144 x 4096, 3.5 / 4.4 at 1024 x 2048.)
+// Waves split K; each walks its share in chunks of U loads per weight tile, the next chunk on its way while this one is multiplied.
+// WT tiles of 8 weight rows per workgroup; GLU: the first half of them gate columns, the second half the up columns that meet them.
+template <typename T, int WT, int U, int W, bool GLU>
+__global__ __launch_bounds__(64 * W) void linear_rows_kernel(const LinearArgs a) {
+  static_assert(!GLU || WT % 2 == 0, "gate and up tiles come in pairs");
+  __shared__ float4 part[W * WT * 64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row8 = lane & 7, piece = ((lane >> 3) & 1) * 4 + (lane >> 4);
+  const int ksl = a.K / W;
+  const int koff = wave * ksl + piece * 8;
+  const int out_cols = GLU ? a.N / 2 : a.N;
+  const int j0 = blockIdx.x * (GLU ? WT * 4 : WT * 8);     // first output column
+  const T* wp[WT];
+#pragma unroll
+  for (int wt = 0; wt < WT; ++wt) {
+    const int t = GLU ? wt % (WT / 2) : wt;
+    const int row = min(j0 + 8 * t + row8, out_cols - 1) + (GLU && wt >= WT / 2 ? out_cols : 0);     // rows past the last repeat it
+    wp[wt] = reinterpret_cast<const T*>(a.w) + (int64_t)row * a.K + koff;
+  }
+  const T* xp = reinterpret_cast<const T*>(a.x) + (int64_t)min(row8, a.M - 1) * a.x_row_stride + koff;
+  v4f acc[WT];
+#pragma unroll
+  for (int wt = 0; wt < WT; ++wt) acc[wt] = (v4f){0.f, 0.f, 0.f, 0.f};
+  struct Chunk { uint4 w[WT][U], x[U]; };
+  Chunk even, odd;
+  auto load = [&](Chunk& c, int k) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int wt = 0; wt < WT; ++wt) c.w[wt][u] = load16_stream(wp[wt] + k + 64 * u);
+#pragma unroll
+    for (int u = 0; u < U; ++u) c.x[u] = *reinterpret_cast<const uint4*>(xp + k + 64 * u);
+  };
+  auto multiply = [&](const Chunk& c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int wt = 0; wt < WT; ++wt) acc[wt] = mfma16x16x32<T>(c.w[wt][u], c.x[u], acc[wt]);
+  };
+  constexpr int kStep = 64 * U;
+  int k = 0;
+  load(even, 0);
+  for (; k + 2 * kStep < ksl; k += 2 * kStep) {            // loads stay in front of the products of the chunk before
+    load(odd, k + kStep);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(even);
+    __builtin_amdgcn_sched_barrier(0);
+    load(even, k + 2 * kStep);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(odd);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (k + kStep < ksl) {
+    load(odd, k + kStep);
+    multiply(even);
+    multiply(odd);
+  } else {
+    multiply(even);
+  }
+#pragma unroll
+  for (int wt = 0; wt < WT; ++wt) part[(wave * WT + wt) * 64 + lane] = make_float4(acc[wt][0], acc[wt][1], acc[wt][2], acc[wt][3]);
+  __syncthreads();
+  // 16 threads a tile: row m, columns 4 quad .. + 3; the first half's result is in lane 16 quad + m, the second's in 16 (quad + 2) + 8 + m
+  auto sum = [&](int wt, int m, int quad, float (&s)[4]) __attribute__((always_inline)) {
+    s[0] = s[1] = s[2] = s[3] = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float4 lo = part[(w * WT + wt) * 64 + 16 * quad + m], hi = part[(w * WT + wt) * 64 + 16 * quad + 40 + m];
+      s[0] += lo.x + hi.x; s[1] += lo.y + hi.y; s[2] += lo.z + hi.z; s[3] += lo.w + hi.w;
+    }
+  };
+  constexpr int kOutTiles = GLU ? WT / 2 : WT;
+  const int t = threadIdx.x;
+  if (t < kOutTiles * 16) {
+    const int quad = t & 1, wt = (t >> 1) % kOutTiles, m = (t >> 1) / kOutTiles;
+    float s[4], u[4];
+    sum(wt, m, quad, s);
+    if constexpr (GLU) sum(wt + WT / 2, m, quad, u);
+    finish_four<T, GLU>(a, m, j0 + 8 * wt + 4 * quad, s, u);
+  }
+}
+
+// More rows: a workgroup owns 16 CT SC output columns and all MT * 16 rows.  SK waves split the 64 SK values of a stage
+// between them, SC such groups the columns; a stage is WB + XB blocks of 8 rows x 128 bytes per 64 values, copied into a ring of
+// S of them (buffer loads to LDS: eight lines a wave and copy, no registers, S - 1 stages under way; a row's eight pieces
+// trade places by the row's number, which spreads both the copies' and the reads' banks).  One barrier a stage: behind it
+// this stage's copies are there and the stage before has been read by all, so its place takes the next copies.  Past the last stage
+// copies go on with an empty descriptor, which keeps the count that a wave waits for.
+// us against the form before it (a workgroup per 16 columns and 16 rows, operands straight into registers), 16 / 32 / 64 rows: 4096 x 1024 4.0 / 4.7 / 5.6
+// against 4.7 / 6.4 / 9.7, 4096 x 12288 21.5 / 28.1 / 36.4 against 34.8 / 50 / 90 (16.8 at 6 TB/s), 24576 x 4096 with GLU 35.7 / 39.4 / 46.6 (4.3 TB/s)
+// against 58 / 95 / 178.
+// GLU: gate and up rows in turns of eight, so that a tile's lanes hold gates (l / 16 < 2) and, 32 lanes on, what meets them.
+// NT: the weights' lines are marked as read once, +5 to 10 % where the call's weights are a stream from HBM; small
+// weights of a small model may still be in the memory-side cache from the step before (4.4 against 5.8 us at 1024 x 3072, 16 rows).
+template <typename T, int MT, int CT, int SK, int SC, int S, bool NT, bool GLU>
+__global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearArgs a) {
+  constexpr int NW = SK * SC, WB = 2 * CT * SC, XB = 2 * MT;
+  constexpr int kPanel = (WB + XB) * 1024, kStage = SK * kPanel, kCopies = (WB + XB) / SC;
+  static_assert((WB + XB) % SC == 0 && S >= 2 && kCopies * (S - 2) <= 63 && S * kStage <= 160 * 1024, "copies of a wave, waits, LDS");
+  static_assert(NW * MT * CT * 1024 <= S * kStage, "the sums reuse the ring");
+  __shared__ __attribute__((aligned(1024))) char lds[S * kStage];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sk = wave % SK, sc = wave / SK;
+  const int out_cols = GLU ? a.N / 2 : a.N;
+  constexpr int kSpan = (GLU ? 8 : 16) * CT * SC;          // output columns of the workgroup
+  const int first = blockIdx.x * kSpan, left = out_cols - first;
+  const uint32_t row_bytes = (uint32_t)a.K * 2u;
+  const char* w0 = reinterpret_cast<const char*>(a.w) + (int64_t)first * row_bytes;
+  const uint32_t w_bytes = (uint32_t)min(left, kSpan) * row_bytes;
+  const uint32_t x_bytes = ((uint32_t)(a.M - 1) * (uint32_t)a.x_row_stride + (uint32_t)a.K) * 2u;
+  const int r8 = lane >> 3;
+  const uint32_t piece = (uint32_t)(sk * 128 + (((lane & 7) ^ r8) << 4));
+  uint32_t from[kCopies];                                  // rows past the last repeat it
+  static_for<kCopies>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+    const int b = i * SC + sc;
+    if constexpr (i < 2 * CT) from[i] = (uint32_t)min(8 * (GLU ? b >> 1 : b) + r8, left - 1) * row_bytes + piece;
+    else from[i] = (uint32_t)min(8 * (b - WB) + r8, a.M - 1) * (uint32_t)a.x_row_stride * 2u + piece;
+  });
+  const int steps = a.K / (64 * SK);
+  const uint32_t lds0 = lds_address(lds) + sk * kPanel + sc * 1024;
+  auto copy = [&](int step, int buffer) __attribute__((always_inline)) {
+    const bool live = step < steps;
+    const v4i x_rows = make_rsrc(reinterpret_cast<const char*>(a.x), live ? x_bytes : 0u);
+    const v4i w_rows = make_rsrc(w0, live ? w_bytes : 0u);
+    const v4i up_rows = GLU ? make_rsrc(w0 + (int64_t)out_cols * row_bytes, live ? w_bytes : 0u) : w_rows;
+    const uint32_t at = live ? (uint32_t)step * (SK * 128) : 0u, base = lds0 + buffer * kStage;
+    static_for<kCopies>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if constexpr (i < 2 * CT) dma16_to_lds_at<i * SC * 1024, NT>(GLU && ((i * SC + sc) & 1) ? up_rows : w_rows, from[i], at, base);
+      else dma16_to_lds_at<i * SC * 1024>(x_rows, from[i], at, base);
+    });
+  };
+  v4f acc[MT][CT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) acc[mt][ct] = (v4f){0.f, 0.f, 0.f, 0.f};
+  static_for<S - 1>([&](auto I) { copy(decltype(I)::value, decltype(I)::value); });
+  // fragments of v_mfma_f32_16x16x32: row l % 16 of a tile (row l % 8 of one of its two blocks), piece 4 kk + l / 16
+  const char* frag = lds + sk * kPanel + ((lane >> 3) & 1) * 1024 + (lane & 7) * 128;
+  const int p0 = ((lane >> 4) ^ (lane & 7)) << 4, p1 = p0 ^ 64;
+  int buffer = 0;
+  for (int step = 0; step < steps; ++step) {
+    dma_wait_but<kCopies * (S - 2)>();
+    workgroup_barrier();
+    copy(step + S - 1, buffer == 0 ? S - 1 : buffer - 1);
+    const char* st = frag + buffer * kStage;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int p = kk ? p1 : p0;
+      uint4 wf[CT], xf[MT];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) wf[ct] = *reinterpret_cast<const uint4*>(st + (sc * CT + ct) * 2048 + p);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) xf[mt] = *reinterpret_cast<const uint4*>(st + (WB + 2 * mt) * 1024 + p);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt][ct] = mfma16x16x32<T>(wf[ct], xf[mt], acc[mt][ct]);
+    }
+    buffer = buffer + 1 == S ? 0 : buffer + 1;
+  }
+  // lane l of a tile holds out[16 mt + l % 16][weight rows 4 (l / 16) .. + 3 of the tile]
+  const int col = lane & 15, cls = lane >> 4;
+  dma_wait_all();
+  workgroup_barrier();                                     // the ring is read and written to its end
+  float4* part = reinterpret_cast<float4*>(lds);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+      part[((wave * MT + mt) * CT + ct) * 64 + lane] = make_float4(acc[mt][ct][0], acc[mt][ct][1], acc[mt][ct][2], acc[mt][ct][3]);
+  __syncthreads();
+  for (int t = wave; t < SC * MT * CT; t += NW) {
+    const int c = t / (MT * CT), mc = t % (MT * CT);
+    float s[4] = {0.f, 0.f, 0.f, 0.f}, u[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < SK; ++k) {
+      const float4 p = part[((c * SK + k) * MT * CT + mc) * 64 + lane];
+      s[0] += p.x; s[1] += p.y; s[2] += p.z; s[3] += p.w;
+    }
+    if constexpr (GLU) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[r] = __shfl_xor(s[r], 32, 64);
+      if (cls >= 2) continue;
+    }
+    finish_four<T, GLU>(a, 16 * (mc / CT) + col, first + (GLU ? 8 : 16) * (c * CT + mc % CT) + 4 * cls, s, u);
+  }
+}
+
+// The product behind the residual add and norm.  The wave's whole share of K is one burst, K / W == 32 U: the rows are normalised
+// on their way into the product.  Every workgroup needs every row, so each of them forms h = x + residual for all its rows, the waves add
 // their shares of the sums of squares through LDS, and the rounded h / sqrt(mean h^2 + eps) * gamma is the B operand:
 // the value the separate norm launch would have written, without the launch.  Workgroup b < M also writes row b of h
-// (the next residual).
-// GLU (N = 2 F, out is [M, F]): a workgroup owns 8 gate columns and the 8 up columns that meet them, and wave 0
-// finishes with out = silu(gate) * up instead of storing both halves for one more launch to read back.
-template <typename T, int MT, int U, int W, bool NORM, bool GLU>
-__global__ __launch_bounds__(64 * W) void linear_small_kernel(const LinearArgs a) {
-  __shared__ float4 part[(W - 1) * MT * 64];
-  __shared__ float sumsq[NORM ? W * MT * 16 : 1];
-  __shared__ __align__(16) float gam[NORM ? W * 32 * U : 4];
+// (the next residual).  A workgroup owns 16 weight rows and up to 16 rows of x:
+//   per wave and 32-wide k step: A = W (row n0 + lane%16, 16 B = 8 k values of class lane/16), B = x^T (column m =
+//   lane%16, the same k values), v_mfma_f32_16x16x32: lane l ends with out[m = l%16][n0 + 4 (l/16) + r], r < 4.
+//   The partial sums meet in LDS; wave 0 adds them.
+// GLU (N = 2 F, out is [M, F]): a workgroup owns 8 gate columns and the 8 up columns that meet them.
+template <typename T, int U, int W, bool GLU>
+__global__ __launch_bounds__(64 * W) void linear_norm_kernel(const LinearArgs a) {
+  __shared__ float4 part[(W - 1) * 64];
+  __shared__ float sumsq[W * 16];
+  __shared__ __align__(16) float gam[W * 32 * U];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int col = lane & 15, cls = lane >> 4;
@@ -89,7 +297,7 @@ __global__ __launch_bounds__(64 * W) void linear_small_kernel(const LinearArgs a
   // weights: consecutive workgroups go to the eight XCDs in turn, so the row tiles of a column tile are dealt 8
   // apart and meet in one L2.
   int ct = blockIdx.x, m0 = 0;
-  if (MT == 1 && a.row_tiles > 1) {
+  if (a.row_tiles > 1) {
     const int tiles = gridDim.x / a.row_tiles;
     if ((tiles & 7) == 0) {
       const int g = ct >> 3;
@@ -100,258 +308,216 @@ __global__ __launch_bounds__(64 * W) void linear_small_kernel(const LinearArgs a
       ct = ct / a.row_tiles;
     }
   }
-  const int mrows = min(a.M - m0, 16 * MT);              // rows of this workgroup
-  int wrow, n0;                                          // weight row of this lane; first output column of the workgroup
-  if constexpr (GLU) {
-    n0 = ct * 8;
-    wrow = col < 8 ? n0 + col : a.N / 2 + n0 + col - 8;
-  } else {
-    n0 = ct * a.cols;
-    wrow = n0 + min(col, a.cols - 1);
-  }
-  const bool wlive = GLU || col < a.cols;                // weight rows of a narrow tile: the other lanes load nothing
+  const int mrows = min(a.M - m0, 16);                   // rows of this workgroup
+  const int n0 = ct * (GLU ? 8 : 16);                    // first output column of the workgroup
+  const int wrow = GLU && col >= 8 ? a.N / 2 + n0 + col - 8 : n0 + col;
   const T* wp = reinterpret_cast<const T*>(a.w) + (int64_t)wrow * a.K + koff;
-  int rowm[MT];
-  const T* xp[MT];
+  const int rowm = m0 + min(col, mrows - 1);             // rows past the last repeat it; they are not stored
+  const T* xp = reinterpret_cast<const T*>(a.x) + (int64_t)rowm * a.x_row_stride + koff;
+  uint4 wf[U], xf[U];
+  if (a.row_tiles > 1) {                                 // the other row tiles' workgroups read the same weights: keep them in L2
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    rowm[mt] = m0 + min(16 * mt + col, mrows - 1);       // rows past the last repeat it; they are not stored
-    xp[mt] = reinterpret_cast<const T*>(a.x) + (int64_t)rowm[mt] * a.x_row_stride + koff;
+    for (int u = 0; u < U; ++u) wf[u] = *reinterpret_cast<const uint4*>(wp + 32 * u);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) wf[u] = load16_stream(wp + 32 * u);      // weights are read once: stream them
   }
-  v4f acc[MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) acc[mt] = (v4f){0.f, 0.f, 0.f, 0.f};
-  for (int k = 0; k < ksl; k += 32 * U) {
-    uint4 wf[U], xf[MT][U];
-    if (MT == 1 && a.row_tiles > 1) {                    // the other row tiles' workgroups read the same weights: keep them in L2
+  for (int u = 0; u < U; ++u) xf[u] = *reinterpret_cast<const uint4*>(xp + 32 * u);
+  // gamma does not depend on the data: the wave's share of it is asked for with the rows (one coalesced load)
+  // and waits in LDS until the sums of squares are known
+  float4 gl = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (4 * lane < 32 * U) gl = *reinterpret_cast<const float4*>(a.gamma + wave * ksl + 4 * lane);
+  float ss = 0.f;
+  const T* rp = a.residual ? reinterpret_cast<const T*>(a.residual) + (int64_t)rowm * a.K + koff : nullptr;
+  uint4 rf[U];
+  if (rp) {
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        wf[u] = wlive ? *reinterpret_cast<const uint4*>(wp + k + 32 * u) : make_uint4(0u, 0u, 0u, 0u);
-    } else {
+    for (int u = 0; u < U; ++u) rf[u] = *reinterpret_cast<const uint4*>(rp + 32 * u);
+  }
 #pragma unroll
-      for (int u = 0; u < U; ++u)                        // weights are read once: stream them
-        wf[u] = wlive ? load16_stream(wp + k + 32 * u) : make_uint4(0u, 0u, 0u, 0u);
+  for (int u = 0; u < U; ++u) {
+    float h[8];
+    unpack8<T>(xf[u], h);
+    if (rp) {
+      float r[8];
+      unpack8<T>(rf[u], r);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = to_float(from_float<T>(h[e] + r[e]));     // the sum lives in T
+      xf[u] = pack8<T>(h);
     }
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int u = 0; u < U; ++u) xf[mt][u] = *reinterpret_cast<const uint4*>(xp[mt] + k + 32 * u);
-    if constexpr (NORM) {
-      // gamma does not depend on the data: the wave's share of it is asked for with the rows (one coalesced load)
-      // and waits in LDS until the sums of squares are known
-      float4 gl = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (4 * lane < 32 * U) gl = *reinterpret_cast<const float4*>(a.gamma + wave * ksl + 4 * lane);
-      float ss[MT];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        ss[mt] = 0.f;
-        const T* rp = a.residual ? reinterpret_cast<const T*>(a.residual) + (int64_t)rowm[mt] * a.K + koff : nullptr;
-        uint4 rf[U];
-        if (rp) {
-#pragma unroll
-          for (int u = 0; u < U; ++u) rf[u] = *reinterpret_cast<const uint4*>(rp + 32 * u);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          float h[8];
-          unpack8<T>(xf[mt][u], h);
-          if (rp) {
-            float r[8];
-            unpack8<T>(rf[u], r);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) h[e] = to_float(from_float<T>(h[e] + r[e]));   // the sum lives in T
-            xf[mt][u] = pack8<T>(h);
-          }
-#pragma unroll
-          for (int e = 0; e < 8; ++e) ss[mt] = ss[mt] + h[e] * h[e];
-        }
-        // the next residual: row b of the workgroup's rows is written by the workgroup of column tile b (all of
-        // them hold these rows)
-        if (a.residual_out && 16 * mt + col == ct && ct < mrows) {
-          T* hp = reinterpret_cast<T*>(a.residual_out) + (int64_t)(m0 + ct) * a.K + koff;
-#pragma unroll
-          for (int u = 0; u < U; ++u) *reinterpret_cast<uint4*>(hp + 32 * u) = xf[mt][u];
-        }
-        ss[mt] = ss[mt] + __shfl_xor(ss[mt], 16, 64);
-        ss[mt] = ss[mt] + __shfl_xor(ss[mt], 32, 64);
-        if (cls == 0) sumsq[(wave * MT + mt) * 16 + col] = ss[mt];
-      }
-      if (4 * lane < 32 * U) *reinterpret_cast<float4*>(&gam[wave * 32 * U + 4 * lane]) = gl;
-      __syncthreads();
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        float tot = 0.f;
-        for (int w = 0; w < W; ++w) tot = tot + sumsq[(w * MT + mt) * 16 + col];
-        const SharedDivisor denom(sqrtf(tot / (float)a.K + a.eps));
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          float h[8];
-          unpack8<T>(xf[mt][u], h);
-          const float4 g0 = *reinterpret_cast<const float4*>(&gam[wave * 32 * U + 32 * u + 8 * cls]);
-          const float4 g1 = *reinterpret_cast<const float4*>(&gam[wave * 32 * U + 32 * u + 8 * cls + 4]);
-          const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-#pragma unroll
-          for (int e = 0; e < 8; ++e) h[e] = denom.divide(h[e]) * g[e];
-          xf[mt][u] = pack8<T>(h);
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma16x16x32<T>(wf[u], xf[mt][u], acc[mt]);
+    for (int e = 0; e < 8; ++e) ss = ss + h[e] * h[e];
   }
-  if (wave > 0) {
+  // the next residual: row b of the workgroup's rows is written by the workgroup of column tile b (all of
+  // them hold these rows)
+  if (a.residual_out && col == ct && ct < mrows) {
+    T* hp = reinterpret_cast<T*>(a.residual_out) + (int64_t)(m0 + ct) * a.K + koff;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      part[((wave - 1) * MT + mt) * 64 + lane] = make_float4(acc[mt][0], acc[mt][1], acc[mt][2], acc[mt][3]);
+    for (int u = 0; u < U; ++u) *reinterpret_cast<uint4*>(hp + 32 * u) = xf[u];
   }
+  ss = ss + __shfl_xor(ss, 16, 64);
+  ss = ss + __shfl_xor(ss, 32, 64);
+  if (cls == 0) sumsq[wave * 16 + col] = ss;
+  if (4 * lane < 32 * U) *reinterpret_cast<float4*>(&gam[wave * 32 * U + 4 * lane]) = gl;
+  __syncthreads();
+  float tot = 0.f;
+  for (int w = 0; w < W; ++w) tot = tot + sumsq[w * 16 + col];
+  const SharedDivisor denom(sqrtf(tot / (float)a.K + a.eps));
+  v4f acc = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    float h[8];
+    unpack8<T>(xf[u], h);
+    const float4 g0 = *reinterpret_cast<const float4*>(&gam[wave * 32 * U + 32 * u + 8 * cls]);
+    const float4 g1 = *reinterpret_cast<const float4*>(&gam[wave * 32 * U + 32 * u + 8 * cls + 4]);
+    const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] = denom.divide(h[e]) * g[e];
+    acc = mfma16x16x32<T>(wf[u], pack8<T>(h), acc);
+  }
+  if (wave > 0) part[(wave - 1) * 64 + lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
   __syncthreads();
   if (wave > 0) return;
-  // lane l holds out[m = l % 16][weight row 4 (l / 16) + r of the workgroup], r < 4
-  float b4[4] = {0.f, 0.f, 0.f, 0.f};
-  if (a.bias && (GLU || 4 * cls < a.cols)) {
-    const int brow = GLU ? (cls < 2 ? n0 + 4 * cls : a.N / 2 + n0 + 4 * (cls - 2)) : n0 + 4 * cls;
-    const T* bp = reinterpret_cast<const T*>(a.bias) + brow;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) b4[r] = to_float(bp[r]);
+  float s[4] = {acc[0], acc[1], acc[2], acc[3]}, up[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int w = 0; w < W - 1; ++w) {
+    const float4 p = part[w * 64 + lane];
+    s[0] += p.x; s[1] += p.y; s[2] += p.z; s[3] += p.w;
   }
-  T* out = reinterpret_cast<T*>(a.out);
+  if constexpr (GLU) {
+    // classes 0, 1 hold the gate columns, classes 2, 3 the up columns that meet them 32 lanes further on
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    float s[4] = {acc[mt][0], acc[mt][1], acc[mt][2], acc[mt][3]};
-    for (int w = 0; w < W - 1; ++w) {
-      const float4 p = part[(w * MT + mt) * 64 + lane];
-      s[0] += p.x; s[1] += p.y; s[2] += p.z; s[3] += p.w;
-    }
-    const int m = m0 + 16 * mt + col;
-    T r4[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) s[r] += b4[r];
-    if (!NORM && !GLU && a.gelu) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s[r] = gelu_tanh(s[r]);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) r4[r] = from_float<T>(s[r]);
-    if constexpr (GLU) {
-      // classes 0, 1 hold the gate columns, classes 2, 3 the up columns that meet them 32 lanes further on
-      const uint2 mine = *reinterpret_cast<const uint2*>(r4);
-      uint2 other;
-      other.x = (uint32_t)__shfl_xor((int)mine.x, 32, 64);
-      other.y = (uint32_t)__shfl_xor((int)mine.y, 32, 64);
-      if (cls < 2 && m < a.M) {
-        const T* u4 = reinterpret_cast<const T*>(&other);
-        T y4[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) y4[r] = silu_mul_rounded<T>(r4[r], u4[r]);
-        *reinterpret_cast<uint2*>(out + (int64_t)m * (a.N / 2) + n0 + 4 * cls) = *reinterpret_cast<const uint2*>(y4);
-      }
-    } else {
-      if (m < a.M && 4 * cls < a.cols)
-        *reinterpret_cast<uint2*>(out + (int64_t)m * a.N + n0 + 4 * cls) = *reinterpret_cast<const uint2*>(r4);
-    }
+    for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(s[r], 32, 64);
+    if (cls >= 2) return;
   }
+  finish_four<T, GLU>(a, m0 + col, n0 + 4 * cls, s, up);
 }
 
-// NORM variants that exist: W waves per workgroup, mt row tiles, `steps` 32-wide k steps per wave
-static bool norm_fits(int W, int mt, int steps) {
-  if (mt > 2 || (steps != 4 && steps != 8)) return false;
-  if (steps == 8) return W == 4 || (W == 8 && mt == 1);
-  return W <= 8 || mt == 1;
+// ---- which kernel ----
+// linear_rows_kernel up to here: from then on its lanes' different rows of x cost more than the ring's detour through LDS.  us at 1 / 3 / 4 rows,
+// in registers against through the ring: 6144 x 4096 10.9 / 11.8 / 12.8 against 13.9, 2048 x 6144 6.8 / 7.2 / 7.5 against 10.0, 4096 x 12288 18.7 /
+// 20.7 / 22.6 against 19.6, 24576 x 4096 33.7 / 34.5 / 35.0 against 35.4.
+constexpr int kFewRows = 3;
+constexpr int64_t kStreamBytes = 12 << 20;                 // weights from this size on are marked as read once (see linear_ring_kernel)
+
+// Columns per workgroup of the ring form: the narrowest tile with which the copies of a CU (its workgroups one after the other,
+// each bringing `columns + rows` rows of K values, at the 30 B per clock measured for such copies) take no longer than the weights take from
+// HBM, N / 100 in these units; else the tile with which they take the least.  us at 64 rows with 16 / 32 / 64 / 96 columns: 4096 x 4096 13.3 / 15.8 / 21.1 / 33,
+// 6144 x 4096 22.3 / 17.2 / 22.0 / 34, 12288 x 2048 22 / 19.2 / 15.4 / 18.8, 24576 x 4096 75 / 53.8 / 53 / 44.2.
+static int ring_columns(int M, int N) {
+  if (N <= 4096) return 16;
+  const int rows = (M + 15) / 16 * 16, widths[3] = {32, 64, 96};
+  int best = 0, best_cost = 0;
+  for (int c : widths) {
+    const int cost = ((N + c - 1) / c + 255) / 256 * (c + rows);
+    if (cost * 100 <= N) return c;
+    if (!best || cost < best_cost) { best = c; best_cost = cost; }
+  }
+  return best;
 }
 
-template <typename T, int W, bool NORM, bool GLU>
-static int launch_linear_w(const LinearArgs& a, hipStream_t stream) {
-  const int tiles = GLU ? a.N / 16 : a.N / a.cols;       // GLU: 8 gate + 8 up columns each
-  const dim3 grid((unsigned)(tiles * a.row_tiles)), block(64 * W);
-  const int mt = a.row_tiles > 1 ? 1 : (a.M + 15) / 16;  // row tiles per workgroup
-  const int steps = a.K / W / 32;                        // 32-wide k steps per wave
-  if constexpr (NORM) {
-    // the wave's whole share of K in one burst, at most two row tiles; the combinations left out would not fit the
-    // registers of their workgroup size
-    if (!norm_fits(W, mt, steps) || tiles < (a.M < 16 * mt ? a.M : 16 * mt)) return MVLLM_ERR_UNSUPPORTED;
-    if (steps == 8) {
-      if constexpr (W <= 8) {
-        if (mt == 1) linear_small_kernel<T, 1, 8, W, true, GLU><<<grid, block, 0, stream>>>(a);
-        else if constexpr (W == 4) linear_small_kernel<T, 2, 8, W, true, GLU><<<grid, block, 0, stream>>>(a);
-      }
-    } else {
-      if (mt == 1) linear_small_kernel<T, 1, 4, W, true, GLU><<<grid, block, 0, stream>>>(a);
-      else if constexpr (W <= 8) linear_small_kernel<T, 2, 4, W, true, GLU><<<grid, block, 0, stream>>>(a);
-    }
-    return launch_status();
+template <typename T, bool GLU>
+static int launch_rows(const LinearArgs& a, hipStream_t stream) {
+  // few columns: narrow tiles and more waves on a tile's K, to have more loads under way.  us at one row with 8 columns and 8 / 4 waves, 16 columns
+  // and 4 waves: 1024 x 3072 4.0 / 4.1 / 5.2, 4096 x 4096 7.7 / 7.3 / 7.9, 12288 x 2048 - / 11 / 10.8.  The order of a sum follows
+  // from the number of waves: it does not depend on GLU.
+  constexpr int WT = GLU ? 2 : 1;
+  const auto grid = [&](int wt) { const int c = wt * (GLU ? 4 : 8); return dim3((unsigned)(((GLU ? a.N / 2 : a.N) + c - 1) / c)); };
+  if (a.N <= 2048) {
+    if (a.K % 1024 == 0) linear_rows_kernel<T, WT, 2, 8, GLU><<<grid(WT), dim3(512), 0, stream>>>(a);
+    else linear_rows_kernel<T, WT, 1, 8, GLU><<<grid(WT), dim3(512), 0, stream>>>(a);
+  } else if (a.N <= 8192) {
+    linear_rows_kernel<T, WT, 2, 4, GLU><<<grid(WT), dim3(256), 0, stream>>>(a);
   } else {
-    // loads in flight per burst: 8 steps of W and x for up to 32 rows, 4 for more (registers)
-    if (mt <= 2 && steps % 8 == 0) {
-      if (mt == 1) linear_small_kernel<T, 1, 8, W, false, GLU><<<grid, block, 0, stream>>>(a);
-      else linear_small_kernel<T, 2, 8, W, false, GLU><<<grid, block, 0, stream>>>(a);
-    } else if (steps % 4 == 0) {
-      if (mt == 1) linear_small_kernel<T, 1, 4, W, false, GLU><<<grid, block, 0, stream>>>(a);
-      else if (mt == 2) linear_small_kernel<T, 2, 4, W, false, GLU><<<grid, block, 0, stream>>>(a);
-      else if (mt == 3) linear_small_kernel<T, 3, 4, W, false, GLU><<<grid, block, 0, stream>>>(a);
-      else linear_small_kernel<T, 4, 4, W, false, GLU><<<grid, block, 0, stream>>>(a);
-    } else {
-      return MVLLM_ERR_UNSUPPORTED;
-    }
-    return launch_status();
+    linear_rows_kernel<T, 2, 2, 4, GLU><<<grid(2), dim3(256), 0, stream>>>(a);
   }
+  return launch_status();
 }
 
-constexpr int kLinearNarrowCols = 8;
-// columns per workgroup of the plain product: narrower tiles when 16-column tiles would leave most CUs without
-// a workgroup (what a CU can keep in flight bounds its share of the weight stream)
-static int linear_cols(int N, bool plain) {
-  return plain && N / 16 < 128 ? kLinearNarrowCols : 16;
-}
-
-constexpr int kLinearRowTileFrom = 17;
-// workgroups per column tile: from this many rows on, every 16 rows of x get a workgroup of their own (the code of
-// the 16-row case, which holds few registers and asks for everything at once) instead of one workgroup that walks
-// all rows; the weights are then read once from HBM and again from L2
-static int linear_row_tiles(int M) {
-  return M >= kLinearRowTileFrom ? (M + 15) / 16 : 1;
-}
-
-// waves per workgroup: more of them share a column tile's K when the column tiles alone give too few workgroups to
-// keep the memory system busy; 12 where 16 do not divide K but 12 do, each with one burst of 256 values (K = 3072:
-// the MLP's down projection)
-static int linear_waves(int tiles, int K, bool plain, bool norm, int mt) {
-  if (norm) {
-    // a wave's share of K must be one burst of 4 or 8 steps: the fewest waves that give 1024 of them in all, else the
-    // most that fit; 0 when no split does
-    int best = 0;
-    for (int w = 4; w <= 16; w *= 2) {
-      if (K % (32 * w) != 0 || !norm_fits(w, mt, K / w / 32)) continue;
-      best = w;
-      if ((int64_t)tiles * w >= 1024) break;
-    }
-    return best;
+template <typename T, int MT, bool GLU>
+static int launch_ring(const LinearArgs& a, hipStream_t stream) {
+  const bool stream_weights = (int64_t)a.N * a.K * 2 >= kStreamBytes;
+  const int columns = ring_columns(a.M, a.N);
+  const dim3 grid((unsigned)((a.N + columns - 1) / columns));
+  constexpr int S = MT > 2 ? 3 : 4;
+  switch (columns) {
+    case 16:
+      if (stream_weights) linear_ring_kernel<T, MT, 1, 4, 1, S, true, GLU><<<grid, dim3(256), 0, stream>>>(a);
+      else linear_ring_kernel<T, MT, 1, 4, 1, S, false, GLU><<<grid, dim3(256), 0, stream>>>(a);
+      break;
+    case 32:
+      if (stream_weights) linear_ring_kernel<T, MT, 1, 2, 2, 4, true, GLU><<<grid, dim3(256), 0, stream>>>(a);
+      else linear_ring_kernel<T, MT, 1, 2, 2, 4, false, GLU><<<grid, dim3(256), 0, stream>>>(a);
+      break;
+    case 64: linear_ring_kernel<T, MT, 2, 2, 2, 3, true, GLU><<<grid, dim3(256), 0, stream>>>(a); break;
+    default: linear_ring_kernel<T, MT, 3, 2, 2, 4, true, GLU><<<grid, dim3(256), 0, stream>>>(a);
   }
-  int w = 4;
-  while (w < 16 && (int64_t)tiles * w < 1024 && K % (2 * w * 128) == 0) w *= 2;
-  if (plain && w == 8 && (int64_t)tiles * w < 1024 && K == 12 * 256) w = 12;
-  return w;
+  return launch_status();
 }
 
-template <typename T, bool NORM, bool GLU>
-static int launch_linear_small(const LinearArgs& a, hipStream_t stream) {
-  switch (linear_waves((GLU ? a.N / 16 : a.N / a.cols) * a.row_tiles, a.K, !NORM && !GLU, NORM,
-                       a.row_tiles > 1 ? 1 : (a.M + 15) / 16)) {
-    case 0: return MVLLM_ERR_UNSUPPORTED;
-    case 4: return launch_linear_w<T, 4, NORM, GLU>(a, stream);
-    case 8: return launch_linear_w<T, 8, NORM, GLU>(a, stream);
-    case 12:
-      if constexpr (!NORM && !GLU) return launch_linear_w<T, 12, false, false>(a, stream);
-      else return MVLLM_ERR_UNSUPPORTED;
-    default: return launch_linear_w<T, 16, NORM, GLU>(a, stream);
+template <typename T, bool GLU>
+static int launch_plain(const LinearArgs& a, hipStream_t stream) {
+  if (a.M <= kFewRows) return launch_rows<T, GLU>(a, stream);
+  if (((int64_t)(a.M - 1) * a.x_row_stride + a.K) * 2 > 0xffffffffll) {      // past a buffer descriptor's offsets: eight rows at a time
+    LinearArgs part = a;
+    for (int m = 0; m < a.M; m += kFewRows) {
+      part.x = reinterpret_cast<const T*>(a.x) + (int64_t)m * a.x_row_stride;
+      part.out = reinterpret_cast<T*>(a.out) + (int64_t)m * (GLU ? a.N / 2 : a.N);
+      part.M = a.M - m < kFewRows ? a.M - m : kFewRows;
+      const int bad = launch_rows<T, GLU>(part, stream);
+      if (bad) return bad;
+    }
+    return MVLLM_OK;
+  }
+  if (a.M <= 16) return launch_ring<T, 1, GLU>(a, stream);
+  if (a.M <= 32) return launch_ring<T, 2, GLU>(a, stream);
+  if (a.M <= 48) return launch_ring<T, 3, GLU>(a, stream);
+  return launch_ring<T, 4, GLU>(a, stream);
+}
+
+// norm variants that exist: W waves per workgroup, `steps` 32-wide k steps per wave in one burst
+static bool norm_fits(int W, int steps) { return steps == 4 || (steps == 8 && W <= 8); }
+
+static int norm_row_tiles(int M) { return (M + 15) / 16; }
+
+// waves per workgroup: the fewest that give 1024 of them in all, else the most that fit; 0 when no split does
+static int norm_waves(int tiles, int K) {
+  int best = 0;
+  for (int w = 4; w <= 16; w *= 2) {
+    if (K % (32 * w) != 0 || !norm_fits(w, K / w / 32)) continue;
+    best = w;
+    if ((int64_t)tiles * w >= 1024) break;
+  }
+  return best;
+}
+
+template <typename T, int W, bool GLU>
+static int launch_norm_w(const LinearArgs& a, hipStream_t stream) {
+  const int tiles = a.N / 16;
+  const dim3 grid((unsigned)(tiles * a.row_tiles)), block(64 * W);
+  if (tiles < (a.M < 16 ? a.M : 16)) return MVLLM_ERR_UNSUPPORTED;
+  if (a.K / W / 32 == 8) {
+    if constexpr (W <= 8) linear_norm_kernel<T, 8, W, GLU><<<grid, block, 0, stream>>>(a);
+  } else {
+    linear_norm_kernel<T, 4, W, GLU><<<grid, block, 0, stream>>>(a);
+  }
+  return launch_status();
+}
+
+template <typename T, bool GLU>
+static int launch_norm(const LinearArgs& a, hipStream_t stream) {
+  switch (norm_waves(a.N / 16 * a.row_tiles, a.K)) {
+    case 4: return launch_norm_w<T, 4, GLU>(a, stream);
+    case 8: return launch_norm_w<T, 8, GLU>(a, stream);
+    case 16: return launch_norm_w<T, 16, GLU>(a, stream);
+    default: return MVLLM_ERR_UNSUPPORTED;
   }
 }
 
 template <typename T>
 static int launch_linear_fused(const LinearArgs& a, bool glu, hipStream_t stream) {
-  if (a.gamma) return glu ? launch_linear_small<T, true, true>(a, stream) : launch_linear_small<T, true, false>(a, stream);
-  return glu ? launch_linear_small<T, false, true>(a, stream) : launch_linear_small<T, false, false>(a, stream);
+  if (a.gamma) return glu ? launch_norm<T, true>(a, stream) : launch_norm<T, false>(a, stream);
+  return glu ? launch_plain<T, true>(a, stream) : launch_plain<T, false>(a, stream);
 }
 
 static int linear_check(const void* out, const void* x, const void* w, const void* bias, int64_t x_row_stride, int M,
@@ -377,8 +543,6 @@ static int linear_plain(void* out, const void* x, const void* w, const void* bia
   LinearArgs a{};
   a.out = out; a.x = x; a.w = w; a.bias = bias; a.x_row_stride = x_row_stride; a.M = M; a.N = N; a.K = K;
   a.gelu = gelu;
-  a.cols = linear_cols(N, true);
-  a.row_tiles = linear_row_tiles(M);
   return dtype == MVLLM_BF16 ? launch_linear_fused<bf16_t>(a, false, (hipStream_t)stream)
                              : launch_linear_fused<f16_t>(a, false, (hipStream_t)stream);
 }
@@ -397,11 +561,11 @@ extern "C" int mvllm_linear_small_m_plan(int M, int N, int K, int norm, int glu,
   if (dtype != MVLLM_BF16 && dtype != MVLLM_F16) return dtype_size(dtype) == 0 ? MVLLM_ERR_BAD_DTYPE : MVLLM_ERR_UNSUPPORTED;
   if (M <= 0 || N <= 0 || K <= 0) return MVLLM_ERR_BAD_SHAPE;
   if (M > 64 || N % 16 != 0 || K % 512 != 0 || (glu && N % 32 != 0)) return MVLLM_ERR_UNSUPPORTED;
-  const int rt = linear_row_tiles(M), mt = rt > 1 ? 1 : (M + 15) / 16;
-  const int w = linear_waves(N / linear_cols(N, !norm && !glu) * rt, K, !norm && !glu, norm != 0, mt);
-  if (w == 0) return MVLLM_ERR_UNSUPPORTED;
-  const int steps = K / w / 32;
-  if (norm ? (!norm_fits(w, mt, steps) || N / 16 < (M < 16 * mt ? M : 16 * mt)) : (steps % 4 != 0)) return MVLLM_ERR_UNSUPPORTED;
+  int w = M <= kFewRows && N <= 2048 ? 8 : 4;
+  if (norm) {
+    w = norm_waves(N / 16 * norm_row_tiles(M), K);
+    if (w == 0 || N / 16 < (M < 16 ? M : 16)) return MVLLM_ERR_UNSUPPORTED;
+  }
   if (waves) *waves = w;
   return MVLLM_OK;
 }
@@ -421,8 +585,7 @@ extern "C" int mvllm_norm_linear_small_m(void* out, void* residual_out, const vo
   LinearArgs a{};
   a.out = out; a.x = x; a.w = w; a.bias = bias; a.x_row_stride = x_row_stride; a.M = M; a.N = N; a.K = K;
   a.residual = residual; a.residual_out = residual_out; a.gamma = gamma; a.eps = eps;
-  a.cols = linear_cols(N, !gamma && !glu);
-  a.row_tiles = linear_row_tiles(M);
+  a.row_tiles = norm_row_tiles(M);
   return dtype == MVLLM_BF16 ? launch_linear_fused<bf16_t>(a, glu != 0, (hipStream_t)stream)
                              : launch_linear_fused<f16_t>(a, glu != 0, (hipStream_t)stream);
 }

@@ -84,10 +84,13 @@ template <int LDS_IMM>   // LDS destination = lds_base + LDS_IMM: one scalar reg
 __device__ __forceinline__ void dma16_to_lds(v4i rsrc, uint32_t lane_off, uint32_t lds_base) {
   asm volatile("s_add_u32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(lane_off), "s"(rsrc), "n"(LDS_IMM) : "scc", "m0");
 }
-// The same with one more offset for all lanes (it counts in the bounds check).
-template <int LDS_IMM>
+// The same with one more offset for all lanes (it counts in the bounds check); NT: lines that are read once.
+template <int LDS_IMM, bool NT = false>
 __device__ __forceinline__ void dma16_to_lds_at(v4i rsrc, uint32_t lane_off, uint32_t wave_off, uint32_t lds_base) {
-  asm volatile("s_add_u32 m0, %0, %4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_base), "v"(lane_off), "s"(rsrc), "s"(wave_off), "n"(LDS_IMM) : "scc", "m0");
+  if constexpr (NT)
+    asm volatile("s_add_u32 m0, %0, %4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds_base), "v"(lane_off), "s"(rsrc), "s"(wave_off), "n"(LDS_IMM) : "scc", "m0");
+  else
+    asm volatile("s_add_u32 m0, %0, %4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_base), "v"(lane_off), "s"(rsrc), "s"(wave_off), "n"(LDS_IMM) : "scc", "m0");
 }
 // The same from a 64-bit address per lane (no bounds check).
 __device__ __forceinline__ void dma16_to_lds_from(const void* p, uint32_t lds_base) {

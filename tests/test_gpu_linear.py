@@ -38,6 +38,25 @@ def test_linear_small_m_vs_fp32_product(dtype, m, n, k, bias):
     assert slack <= 2e-3, slack
 
 
+@pytest.mark.parametrize("m", [2, 3, 4, 9, 31, 47, 64])
+@pytest.mark.parametrize("n,k", [(32, 512), (4128, 1536), (12320, 512), (24608, 512)])
+def test_linear_small_m_tile_edges(m, n, k):
+    """Every column tile (16, 32, 64 and 96 wide, a last one that is not full), fewer stages of K than the ring holds, rows that end
+    inside a tile and strided rows, plain, with gelu and with the gated unit (whose two roundings add two units in the last place)."""
+    x, w, b = _case(500 + m, m, n, k, torch.bfloat16, True, stride=k + 24)
+    full = x.float() @ w.float().T + b.float()
+    for gelu in (False, True):
+        want = F.gelu(full, approximate="tanh") if gelu else full
+        err = (linear_small_m(x, w, b, gelu).float() - want).abs() - want.abs() * 2.0 ** -8
+        assert err.max().item() <= 2e-3
+    gate, up = full.bfloat16().float().chunk(2, 1)
+    want = F.silu(gate) * up
+    got = norm_linear_small_m(x.contiguous(), w, b, glu=True).float()
+    # a unit of the gate or of the up value that rounds the other way, and the two roundings behind them
+    slack = (got - want).abs() - 4 * 2.0 ** -8 * (F.silu(gate).abs() + gate.abs() + 1) * (up.abs() + 1)
+    assert slack.max().item() <= 2e-3
+
+
 def test_linear_small_m_strided_rows_and_module_dispatch():
     """Rows of x may be slices of a wider tensor; the module takes the HIP launch up to its row limit and the
     library GEMM beyond, with the same result up to the rounding of the output."""
