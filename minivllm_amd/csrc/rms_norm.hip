@@ -7,8 +7,11 @@
 // correctly rounded square root and the quotient x / denominator taken with one correction step from the
 // correctly rounded reciprocal (SharedDivisor); only the order of the sum of squares is free.
 //
-// One wave per row; lane l holds elements [8 (l + 64 c), +8) for chunks c = 0 .. CHUNKS-1 in registers, so the
-// row is read once and written once (16-byte accesses).
+// WAVES waves per row; thread l of them holds elements [8 (l + 64 WAVES c), +8) for chunks c = 0 .. CHUNKS-1 in registers, so the
+// row is read once and written once (16-byte accesses).  Up to 1024 numbers a row takes one wave; longer ones four, because a wave with
+// 32 numbers or more per lane to take through the norm is what few rows wait for, and holds too many registers to have enough rows
+// under way where there are many (us with one wave and with four: 61 rows of 4096 6.6 / 3.1, 1024 rows 8.8 / 6.5, 8192 rows 44.7 / 39.6;
+// 8192 rows of 8192 135 / 103 = 5.2 TB/s).
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -46,26 +49,28 @@ template <typename T16> struct Row8 {
 
 constexpr int kNormThreads = 256;   // 4 rows per workgroup
 
-template <typename T, int CHUNKS>
+template <typename T, int CHUNKS, int WAVES>
 __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
     T* __restrict__ out, T* __restrict__ residual_out, const T* __restrict__ x, const T* __restrict__ residual,
     const float* __restrict__ gamma, float eps, int64_t rows, int hidden, int64_t x_stride, int64_t res_stride) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (kNormThreads / 64) + (threadIdx.x >> 6);
-  if (row >= rows) return;
+  constexpr int kRows = kNormThreads / 64 / WAVES;
+  __shared__ float part[WAVES > 1 ? kNormThreads / 64 : 1];
+  const int lane = threadIdx.x & (64 * WAVES - 1);
+  const int64_t row = (int64_t)blockIdx.x * kRows + threadIdx.x / (64 * WAVES);
+  if (row >= rows) return;                            // (WAVES > 1: one row per workgroup, so all of it)
+  static_assert(WAVES == 1 || kRows == 1, "the workgroup's barrier is the row's");
   const T* xp = x + row * x_stride;
   float v[CHUNKS][8];
-  // gamma does not depend on the row: for short rows it is fetched together with the row instead of after the
+  // gamma does not depend on the row: it is fetched together with the row instead of after the
   // reduction, which takes one memory latency out of a kernel that is all latency at decode batch sizes
-  constexpr bool kEarlyGamma = CHUNKS <= 4;
-  float gam[kEarlyGamma ? CHUNKS : 1][8];
+  float gam[CHUNKS][8];
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int e0 = 8 * (lane + 64 * c);
+    const int e0 = 8 * (lane + 64 * WAVES * c);
     if (e0 < hidden) {
       Row8<T>::load(xp + e0, v[c]);
-      if constexpr (kEarlyGamma) Row8<float>::load(gamma + e0, gam[c]);
+      Row8<float>::load(gamma + e0, gam[c]);
       if (residual) {
         float r[8];
         Row8<T>::load(residual + row * res_stride + e0, r);
@@ -77,22 +82,22 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
       for (int e = 0; e < 8; ++e) ss = ss + v[c][e] * v[c][e];
     }
   }
+  ss = four_rows_sum(row16_sum(ss));
+  if constexpr (WAVES > 1) {
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = part[0];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ss = ss + __shfl_xor(ss, o, 64);
+    for (int w = 1; w < WAVES; ++w) ss = ss + part[w];
+  }
   const SharedDivisor denom(sqrtf(ss / (float)hidden + eps));
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int e0 = 8 * (lane + 64 * c);
+    const int e0 = 8 * (lane + 64 * WAVES * c);
     if (e0 < hidden) {
-      float g[8], y[8];
-      if constexpr (kEarlyGamma) {
+      float y[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) g[e] = gam[c][e];
-      } else {
-        Row8<float>::load(gamma + e0, g);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = denom.divide(v[c][e]) * g[e];
+      for (int e = 0; e < 8; ++e) y[e] = denom.divide(v[c][e]) * gam[c][e];
       Row8<T>::store(out + row * (int64_t)hidden + e0, y);
     }
   }
@@ -102,15 +107,16 @@ template <typename T>
 static int launch_norm(void* out, void* residual_out, const void* x, const void* residual, const float* gamma, float eps,
                        int64_t rows, int hidden, int64_t x_stride, int64_t res_stride, hipStream_t s) {
   const int chunks = (hidden + 511) / 512;
-  const dim3 grid((unsigned)((rows + kNormThreads / 64 - 1) / (kNormThreads / 64))), block(kNormThreads);
-#define MVLLM_LAUNCH_N(C)                                                                                      \
-  add_rms_norm_kernel<T, C><<<grid, block, 0, s>>>((T*)out, (T*)residual_out, (const T*)x, (const T*)residual, \
-                                                   gamma, eps, rows, hidden, x_stride, res_stride)
-  if (chunks <= 1) MVLLM_LAUNCH_N(1);
-  else if (chunks <= 2) MVLLM_LAUNCH_N(2);
-  else if (chunks <= 4) MVLLM_LAUNCH_N(4);
-  else if (chunks <= 8) MVLLM_LAUNCH_N(8);
-  else MVLLM_LAUNCH_N(16);
+  const int per_group = chunks > 2 ? 1 : kNormThreads / 64;
+  const dim3 grid((unsigned)((rows + per_group - 1) / per_group)), block(kNormThreads);
+#define MVLLM_LAUNCH_N(C, W)                                                                                      \
+  add_rms_norm_kernel<T, C, W><<<grid, block, 0, s>>>((T*)out, (T*)residual_out, (const T*)x, (const T*)residual, \
+                                                      gamma, eps, rows, hidden, x_stride, res_stride)
+  if (chunks <= 1) MVLLM_LAUNCH_N(1, 1);
+  else if (chunks <= 2) MVLLM_LAUNCH_N(2, 1);
+  else if (chunks <= 4) MVLLM_LAUNCH_N(1, 4);
+  else if (chunks <= 8) MVLLM_LAUNCH_N(2, 4);
+  else MVLLM_LAUNCH_N(4, 4);
 #undef MVLLM_LAUNCH_N
   return launch_status();
 }
