@@ -442,8 +442,8 @@ int mvllm_linear_small_m(void* out, const void* x, const void* w, const void* bi
  *   glu != 0:       W is [2F, K] (gate rows, then up rows, as layers/activation.py:15-18 chunks the output), out is
  *                   [M, F] = silu(x' Wg^T + bg) * (x' Wu^T + bu) with the roundings of mvllm_silu_and_mul on the
  *                   rounded projection; N = 2F, N % 32 == 0.
- * Shapes as mvllm_linear_small_m, and for gamma != NULL: N / 16 >= min(M, 16), K / waves one burst of 128 or 256
- * values with 4, 8 or 16 waves (mvllm_linear_small_m_plan says whether a shape is taken); otherwise MVLLM_ERR_UNSUPPORTED and the caller
+ * Shapes as mvllm_linear_small_m, and for gamma != NULL: N / 16 >= min(M, 16) and K 512, 1024 or 2048
+ * (mvllm_linear_small_m_plan says whether a shape is taken); otherwise MVLLM_ERR_UNSUPPORTED and the caller
  * runs the separate launches.
  */
 int mvllm_norm_linear_small_m(void* out, void* residual_out, const void* x, const void* residual,
@@ -452,7 +452,8 @@ int mvllm_norm_linear_small_m(void* out, void* residual_out, const void* x, cons
 
 /*
  * Whether mvllm_linear_small_m (norm == 0 && glu == 0) or mvllm_norm_linear_small_m takes a shape, without a
- * launch: MVLLM_OK and the waves per workgroup in *waves (may be NULL), or MVLLM_ERR_UNSUPPORTED.  No counterpart
+ * launch: MVLLM_OK and in *waves (may be NULL) the number of parts K is cut into for this shape (with the norm: the fewest of 4, 8
+ * or 16 whose 128 or 256 values each give 1024 parts in all), or MVLLM_ERR_UNSUPPORTED.  No counterpart
  * in the reference (its projections are library GEMMs of any shape).
  */
 int mvllm_linear_small_m_plan(int M, int N, int K, int norm, int glu, int dtype, int* waves);

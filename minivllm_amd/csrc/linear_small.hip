@@ -29,7 +29,7 @@ struct LinearArgs {
   void* residual_out;     // [M, K] contiguous: x + residual in the element type; must not alias x or residual
   const float* gamma;     // [K]
   float eps;
-  int row_tiles;          // norm: workgroups per column tile, one per 16 rows of x
+  int row_tiles;          // norm: tiles of 16 rows, a workgroup per column tile each
   int gelu;               // plain product only: the result through the tanh form of gelu
 };
 
@@ -274,123 +274,135 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
   }
 }
 
-// The product behind the residual add and norm.  The wave's whole share of K is one burst, K / W == 32 U: the rows are normalised
-// on their way into the product.  Every workgroup needs every row, so each of them forms h = x + residual for all its rows, the waves add
-// their shares of the sums of squares through LDS, and the rounded h / sqrt(mean h^2 + eps) * gamma is the B operand:
-// the value the separate norm launch would have written, without the launch.  Workgroup b < M also writes row b of h
-// (the next residual).  A workgroup owns 16 weight rows and up to 16 rows of x:
-//   per wave and 32-wide k step: A = W (row n0 + lane%16, 16 B = 8 k values of class lane/16), B = x^T (column m =
-//   lane%16, the same k values), v_mfma_f32_16x16x32: lane l ends with out[m = l%16][n0 + 4 (l/16) + r], r < 4.
-//   The partial sums meet in LDS; wave 0 adds them.
-// GLU (N = 2 F, out is [M, F]): a workgroup owns 8 gate columns and the 8 up columns that meet them.
-template <typename T, int U, int W, bool GLU>
-__global__ __launch_bounds__(64 * W) void linear_norm_kernel(const LinearArgs a) {
-  __shared__ float4 part[(W - 1) * 64];
-  __shared__ float sumsq[W * 16];
-  __shared__ __align__(16) float gam[W * 32 * U];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int col = lane & 15, cls = lane >> 4;
-  const int ksl = a.K / W;                               // this wave's share of K
-  const int koff = wave * ksl + cls * 8;                 // first k of this lane in every 32-wide step
-  // column tile and first row of this workgroup.  With row tiles the workgroups of one column tile read the same
-  // weights: consecutive workgroups go to the eight XCDs in turn, so the row tiles of a column tile are dealt 8
-  // apart and meet in one L2.
-  int ct = blockIdx.x, m0 = 0;
-  if (a.row_tiles > 1) {
-    const int tiles = gridDim.x / a.row_tiles;
-    if ((tiles & 7) == 0) {
-      const int g = ct >> 3;
-      m0 = 16 * (g % a.row_tiles);
-      ct = (g / a.row_tiles) * 8 + (ct & 7);
-    } else {
-      m0 = 16 * (ct % a.row_tiles);
-      ct = ct / a.row_tiles;
+// The product behind the residual add and norm: K = 512 P, eight waves, each with 64 P values of K, 16 rows of x and 16 CT weight rows per
+// workgroup.  Every workgroup needs every row, so each of them forms h = x + residual for its rows, a wave per row, and leaves the rounded
+// h / sqrt(mean h^2 + eps) * gamma in LDS as the second operand: the value the separate norm launch would have written, without
+// the launch.  Workgroup b < M also writes row b of h (the next residual).  The wave's weights are asked for behind the rows and are on their
+// way meanwhile; they go through a place in LDS of the wave's own, because whole lines are loaded (see the top of this file).
+// us at 1 / 16 rows, before (operands straight into registers, rows normalised once per 16 lanes that share them) and now:
+// 4096 x 1024 6.2 / 7.4 and 4.0 / 5.5 (the product alone 3.8 / 4.0), 6144 x 1024 with GLU 8.4 / 10.7 and 5.1 / 6.6, 4096 x 2048 9.3 /
+// 11.3 and 5.8 / 8.7.
+template <typename T, int CT, int P, bool GLU>
+__global__ __launch_bounds__(512) void linear_norm_kernel(const LinearArgs a) {
+  constexpr int W = 8, kPanel = 2048;                      // waves; bytes of 16 rows x 64 values: two blocks of 8 rows, as in linear_ring_kernel
+  constexpr int kX = W * P * kPanel, kW = W * CT * kPanel;
+  __shared__ __attribute__((aligned(1024))) char lds[kX + kW];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = 16 * blockIdx.y, mrows = min(a.M - m0, 16);
+  const int out_cols = GLU ? a.N / 2 : a.N, K = 512 * P;
+  const int first = blockIdx.x * (GLU ? 8 : 16) * CT, left = out_cols - first;
+  // ---- loads: rows wave and wave + 8 (8 values of K per lane and chunk of 512), gamma, then the weights of 64 P values ----
+  uint4 x[2][P], res[2][P];
+  float4 gam[P][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = wave + 8 * i;
+    if (row < mrows) {
+      const T* xp = reinterpret_cast<const T*>(a.x) + (int64_t)(m0 + row) * a.x_row_stride + 8 * lane;
+      const T* rp = reinterpret_cast<const T*>(a.residual) + (int64_t)(m0 + row) * K + 8 * lane;
+#pragma unroll
+      for (int c = 0; c < P; ++c) {
+        x[i][c] = *reinterpret_cast<const uint4*>(xp + 512 * c);
+        if (a.residual) res[i][c] = *reinterpret_cast<const uint4*>(rp + 512 * c);
+      }
     }
   }
-  const int mrows = min(a.M - m0, 16);                   // rows of this workgroup
-  const int n0 = ct * (GLU ? 8 : 16);                    // first output column of the workgroup
-  const int wrow = GLU && col >= 8 ? a.N / 2 + n0 + col - 8 : n0 + col;
-  const T* wp = reinterpret_cast<const T*>(a.w) + (int64_t)wrow * a.K + koff;
-  const int rowm = m0 + min(col, mrows - 1);             // rows past the last repeat it; they are not stored
-  const T* xp = reinterpret_cast<const T*>(a.x) + (int64_t)rowm * a.x_row_stride + koff;
-  uint4 wf[U], xf[U];
-  if (a.row_tiles > 1) {                                 // the other row tiles' workgroups read the same weights: keep them in L2
 #pragma unroll
-    for (int u = 0; u < U; ++u) wf[u] = *reinterpret_cast<const uint4*>(wp + 32 * u);
-  } else {
-#pragma unroll
-    for (int u = 0; u < U; ++u) wf[u] = load16_stream(wp + 32 * u);      // weights are read once: stream them
+  for (int c = 0; c < P; ++c) {
+    gam[c][0] = *reinterpret_cast<const float4*>(a.gamma + 512 * c + 8 * lane);
+    gam[c][1] = *reinterpret_cast<const float4*>(a.gamma + 512 * c + 8 * lane + 4);
   }
+  const int r8 = lane >> 3;
+  uint4 w[P][CT][2];
 #pragma unroll
-  for (int u = 0; u < U; ++u) xf[u] = *reinterpret_cast<const uint4*>(xp + 32 * u);
-  // gamma does not depend on the data: the wave's share of it is asked for with the rows (one coalesced load)
-  // and waits in LDS until the sums of squares are known
-  float4 gl = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (4 * lane < 32 * U) gl = *reinterpret_cast<const float4*>(a.gamma + wave * ksl + 4 * lane);
-  float ss = 0.f;
-  const T* rp = a.residual ? reinterpret_cast<const T*>(a.residual) + (int64_t)rowm * a.K + koff : nullptr;
-  uint4 rf[U];
-  if (rp) {
+  for (int p = 0; p < P; ++p)
 #pragma unroll
-    for (int u = 0; u < U; ++u) rf[u] = *reinterpret_cast<const uint4*>(rp + 32 * u);
-  }
+    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    float h[8];
-    unpack8<T>(xf[u], h);
-    if (rp) {
-      float r[8];
-      unpack8<T>(rf[u], r);
+      for (int b = 0; b < 2; ++b) {                        // GLU: block 0 of a tile gate rows, block 1 up rows; rows past the last repeat it
+        const int row = GLU ? min(8 * ct + r8, left - 1) + first + (b ? out_cols : 0) : first + min(16 * ct + 8 * b + r8, left - 1);
+        const T* wp = reinterpret_cast<const T*>(a.w) + (int64_t)row * K + 64 * (wave * P + p) + 8 * (lane & 7);
+        w[p][ct][b] = a.row_tiles > 1 ? *reinterpret_cast<const uint4*>(wp) : load16_stream(wp);
+      }
+  // ---- rows: sum, norm, into LDS: panel k / 64, block row / 8, row row % 8, piece k / 8 % 8 with its place changed by the row ----
 #pragma unroll
-      for (int e = 0; e < 8; ++e) h[e] = to_float(from_float<T>(h[e] + r[e]));     // the sum lives in T
-      xf[u] = pack8<T>(h);
+  for (int i = 0; i < 2; ++i) {
+    const int row = wave + 8 * i;
+    if (row >= mrows) continue;                            // rows that do not exist leave what is there: their results are not stored
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < P; ++c) {
+      float h[8];
+      unpack8<T>(x[i][c], h);
+      if (a.residual) {
+        float r[8];
+        unpack8<T>(res[i][c], r);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h[e] = to_float(from_float<T>(h[e] + r[e]));       // the sum lives in T
+        x[i][c] = pack8<T>(h);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = ss + h[e] * h[e];
     }
+    if (a.residual_out && (int)blockIdx.x == row) {
+      T* hp = reinterpret_cast<T*>(a.residual_out) + (int64_t)(m0 + row) * K + 8 * lane;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss = ss + h[e] * h[e];
-  }
-  // the next residual: row b of the workgroup's rows is written by the workgroup of column tile b (all of
-  // them hold these rows)
-  if (a.residual_out && col == ct && ct < mrows) {
-    T* hp = reinterpret_cast<T*>(a.residual_out) + (int64_t)(m0 + ct) * a.K + koff;
+      for (int c = 0; c < P; ++c) *reinterpret_cast<uint4*>(hp + 512 * c) = x[i][c];
+    }
+    const SharedDivisor denom(sqrtf(four_rows_sum(row16_sum(ss)) / (float)K + a.eps));
+    char* place = lds + r8 * kPanel + i * 1024 + wave * 128 + (((lane & 7) ^ wave) << 4);
 #pragma unroll
-    for (int u = 0; u < U; ++u) *reinterpret_cast<uint4*>(hp + 32 * u) = xf[u];
+    for (int c = 0; c < P; ++c) {
+      float h[8];
+      unpack8<T>(x[i][c], h);
+      const float g[8] = {gam[c][0].x, gam[c][0].y, gam[c][0].z, gam[c][0].w, gam[c][1].x, gam[c][1].y, gam[c][1].z, gam[c][1].w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = denom.divide(h[e]) * g[e];
+      *reinterpret_cast<uint4*>(place + 8 * kPanel * c) = pack8<T>(h);
+    }
   }
-  ss = ss + __shfl_xor(ss, 16, 64);
-  ss = ss + __shfl_xor(ss, 32, 64);
-  if (cls == 0) sumsq[wave * 16 + col] = ss;
-  if (4 * lane < 32 * U) *reinterpret_cast<float4*>(&gam[wave * 32 * U + 4 * lane]) = gl;
   __syncthreads();
-  float tot = 0.f;
-  for (int w = 0; w < W; ++w) tot = tot + sumsq[w * 16 + col];
-  const SharedDivisor denom(sqrtf(tot / (float)a.K + a.eps));
-  v4f acc = (v4f){0.f, 0.f, 0.f, 0.f};
+  // ---- products: panels wave * P .. of x, the wave's weights through its own place (a wave's LDS accesses stay in order) ----
+  v4f acc[CT];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    float h[8];
-    unpack8<T>(xf[u], h);
-    const float4 g0 = *reinterpret_cast<const float4*>(&gam[wave * 32 * U + 32 * u + 8 * cls]);
-    const float4 g1 = *reinterpret_cast<const float4*>(&gam[wave * 32 * U + 32 * u + 8 * cls + 4]);
-    const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+  for (int ct = 0; ct < CT; ++ct) acc[ct] = (v4f){0.f, 0.f, 0.f, 0.f};
+  char* own = lds + kX + wave * CT * kPanel;
+  const int frag = ((lane >> 3) & 1) * 1024 + (lane & 7) * 128, p0 = ((lane >> 4) ^ (lane & 7)) << 4;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] = denom.divide(h[e]) * g[e];
-    acc = mfma16x16x32<T>(wf[u], pack8<T>(h), acc);
+  for (int p = 0; p < P; ++p) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        *reinterpret_cast<uint4*>(own + ct * kPanel + b * 1024 + r8 * 128 + (((lane & 7) ^ r8) << 4)) = w[p][ct][b];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const uint4 xf = *reinterpret_cast<const uint4*>(lds + (wave * P + p) * kPanel + frag + (p0 ^ (64 * kk)));
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        acc[ct] = mfma16x16x32<T>(*reinterpret_cast<const uint4*>(own + ct * kPanel + frag + (p0 ^ (64 * kk))), xf, acc[ct]);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
-  if (wave > 0) part[(wave - 1) * 64 + lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  float4* part = reinterpret_cast<float4*>(lds + kX);      // the wave's own place again: CT KB of CT * 2
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) part[(2 * wave * CT + ct) * 64 + lane] = make_float4(acc[ct][0], acc[ct][1], acc[ct][2], acc[ct][3]);
   __syncthreads();
-  if (wave > 0) return;
-  float s[4] = {acc[0], acc[1], acc[2], acc[3]}, up[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int w = 0; w < W - 1; ++w) {
-    const float4 p = part[w * 64 + lane];
-    s[0] += p.x; s[1] += p.y; s[2] += p.z; s[3] += p.w;
+  if (wave >= CT) return;
+  float s[4] = {0.f, 0.f, 0.f, 0.f}, up[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < W; ++k) {
+    const float4 q = part[(2 * k * CT + wave) * 64 + lane];
+    s[0] += q.x; s[1] += q.y; s[2] += q.z; s[3] += q.w;
   }
+  const int cls = lane >> 4, m = lane & 15;
   if constexpr (GLU) {
-    // classes 0, 1 hold the gate columns, classes 2, 3 the up columns that meet them 32 lanes further on
 #pragma unroll
     for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(s[r], 32, 64);
     if (cls >= 2) return;
   }
-  finish_four<T, GLU>(a, m0 + col, n0 + 4 * cls, s, up);
+  finish_four<T, GLU>(a, m < mrows ? m0 + m : a.M, first + (GLU ? 8 : 16) * wave + 4 * cls, s, up);
 }
 
 // ---- which kernel ----
@@ -475,12 +487,11 @@ static int launch_plain(const LinearArgs& a, hipStream_t stream) {
   return launch_ring<T, 4, GLU>(a, stream);
 }
 
-// norm variants that exist: W waves per workgroup, `steps` 32-wide k steps per wave in one burst
+// Shapes the norm form takes: K of 512, 1024 or 2048 (512 P), at least as many column tiles as rows of a row tile.  The number reported for a shape
+// is the split of K that defined the set: the fewest waves that give 1024 of them in all with one burst of 128 or 256 values
+// each; 0 when there is none.
 static bool norm_fits(int W, int steps) { return steps == 4 || (steps == 8 && W <= 8); }
-
 static int norm_row_tiles(int M) { return (M + 15) / 16; }
-
-// waves per workgroup: the fewest that give 1024 of them in all, else the most that fit; 0 when no split does
 static int norm_waves(int tiles, int K) {
   int best = 0;
   for (int w = 4; w <= 16; w *= 2) {
@@ -490,33 +501,34 @@ static int norm_waves(int tiles, int K) {
   }
   return best;
 }
+static bool norm_takes(int M, int N, int K) {
+  return norm_waves(N / 16 * norm_row_tiles(M), K) != 0 && N / 16 >= (M < 16 ? M : 16);
+}
 
-template <typename T, int W, bool GLU>
-static int launch_norm_w(const LinearArgs& a, hipStream_t stream) {
-  const int tiles = a.N / 16;
-  const dim3 grid((unsigned)(tiles * a.row_tiles)), block(64 * W);
-  if (tiles < (a.M < 16 ? a.M : 16)) return MVLLM_ERR_UNSUPPORTED;
-  if (a.K / W / 32 == 8) {
-    if constexpr (W <= 8) linear_norm_kernel<T, 8, W, GLU><<<grid, block, 0, stream>>>(a);
-  } else {
-    linear_norm_kernel<T, 4, W, GLU><<<grid, block, 0, stream>>>(a);
-  }
+template <typename T, int P, bool GLU>
+static int launch_norm(const LinearArgs& a, hipStream_t stream) {
+  // 32 columns halve what the rows cost where 16 would give a CU more than one workgroup
+  const int wide = a.N > 4096;
+  const dim3 grid((unsigned)((a.N + (wide ? 31 : 15)) / (wide ? 32 : 16)), (unsigned)a.row_tiles);
+  if (wide) linear_norm_kernel<T, 2, P, GLU><<<grid, dim3(512), 0, stream>>>(a);
+  else linear_norm_kernel<T, 1, P, GLU><<<grid, dim3(512), 0, stream>>>(a);
   return launch_status();
 }
 
 template <typename T, bool GLU>
-static int launch_norm(const LinearArgs& a, hipStream_t stream) {
-  switch (norm_waves(a.N / 16 * a.row_tiles, a.K)) {
-    case 4: return launch_norm_w<T, 4, GLU>(a, stream);
-    case 8: return launch_norm_w<T, 8, GLU>(a, stream);
-    case 16: return launch_norm_w<T, 16, GLU>(a, stream);
+static int launch_norm_k(const LinearArgs& a, hipStream_t stream) {
+  if (!norm_takes(a.M, a.N, a.K)) return MVLLM_ERR_UNSUPPORTED;
+  switch (a.K) {
+    case 512: return launch_norm<T, 1, GLU>(a, stream);
+    case 1024: return launch_norm<T, 2, GLU>(a, stream);
+    case 2048: return launch_norm<T, 4, GLU>(a, stream);
     default: return MVLLM_ERR_UNSUPPORTED;
   }
 }
 
 template <typename T>
 static int launch_linear_fused(const LinearArgs& a, bool glu, hipStream_t stream) {
-  if (a.gamma) return glu ? launch_norm<T, true>(a, stream) : launch_norm<T, false>(a, stream);
+  if (a.gamma) return glu ? launch_norm_k<T, true>(a, stream) : launch_norm_k<T, false>(a, stream);
   return glu ? launch_plain<T, true>(a, stream) : launch_plain<T, false>(a, stream);
 }
 
@@ -563,8 +575,8 @@ extern "C" int mvllm_linear_small_m_plan(int M, int N, int K, int norm, int glu,
   if (M > 64 || N % 16 != 0 || K % 512 != 0 || (glu && N % 32 != 0)) return MVLLM_ERR_UNSUPPORTED;
   int w = M <= kFewRows && N <= 2048 ? 8 : 4;
   if (norm) {
+    if (!norm_takes(M, N, K)) return MVLLM_ERR_UNSUPPORTED;
     w = norm_waves(N / 16 * norm_row_tiles(M), K);
-    if (w == 0 || N / 16 < (M < 16 ? M : 16)) return MVLLM_ERR_UNSUPPORTED;
   }
   if (waves) *waves = w;
   return MVLLM_OK;

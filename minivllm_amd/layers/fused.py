@@ -18,7 +18,7 @@ import torch
 
 from minivllm_amd import _C
 
-__all__ = ["qk_norm_rope_store", "sample_tokens", "sample_tokens_into", "decode_advance", "add_rms_norm", "silu_and_mul", "linear_small_m", "linear_small_m_takes", "norm_linear_small_m", "norm_linear_small_m_takes",
+__all__ = ["qk_norm_rope_store", "sample_tokens", "sample_tokens_into", "decode_advance", "add_rms_norm", "silu_and_mul", "linear_small_m", "linear_small_m_takes", "norm_linear_small_m", "norm_linear_small_m_pays", "norm_linear_small_m_takes",
            "lm_head_sample", "lm_head_sample_takes", "lm_head_sample_workspace_bytes", "norm_conv", "head_rope_store",
            "head_unrotate_gate", "chunk_decode_step", "stream_embed_norm", "stream_norm", "gated_unit", "gelu_tanh", "post_norm",
            "embed_rows"]
@@ -335,6 +335,14 @@ def norm_linear_small_m_takes(x: torch.Tensor, weight: torch.Tensor, max_rows: i
         st = _C.load().mvllm_linear_small_m_plan(key[0], key[1], key[2], int(norm), int(glu), _C.dtype_code(x.dtype), None)
         _PLAN_CACHE[key] = st == 0
     return _PLAN_CACHE[key]
+
+
+def norm_linear_small_m_pays(rows: int, weight: torch.Tensor) -> bool:
+    """Whether the norm inside the product beats its own launch in front of it: every workgroup norms all rows again, which
+    costs less than a launch up to 16 of them if a CU has one workgroup or two (us together / apart: 4096 x 1024 4.0 / 6.4 at one row,
+    5.5 / 6.7 at 16, 7.5 / 7.4 at 32; 6144 x 1024 gated 5.1 / 7.8, 6.6 / 7.6, 9.0 / 8.1; 4096 x 2048 5.8 / 7.4, 8.7 / 8.3; 12288 x 2048 15.5 / 13.3)."""
+    n, k = weight.shape
+    return rows <= 16 and n * k <= (8 << 20)
 
 
 def norm_linear_small_m(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,

@@ -15,7 +15,7 @@ import torch.nn.functional as F
 
 from minivllm_amd.layers.attention import Attention
 from minivllm_amd.layers.basic import Linear, RMSNorm, RotaryEmbedding, SiluAndMul
-from minivllm_amd.layers.fused import norm_linear_small_m, norm_linear_small_m_takes
+from minivllm_amd.layers.fused import norm_linear_small_m, norm_linear_small_m_pays, norm_linear_small_m_takes
 from minivllm_amd.utils.context import get_context
 
 
@@ -82,40 +82,36 @@ class Qwen3DecoderLayer(nn.Module):
                                         small_rows=small_rows, **attn_kwargs)
         self.post_attention_layernorm = RMSNorm(hidden_size, rms_norm_epsilon, fused_elementwise)
         self.mlp = Qwen3MLP(hidden_size, intermediate_size, ffn_bias, fused_elementwise, small_rows)
-        # the norm prologue normalises a workgroup's rows once per column tile: it pays up to about 32 rows
         self.norm_rows, self.fused_elementwise = min(small_rows, norm_rows), fused_elementwise
 
-    def _forward_few_rows(self, x, residual, positions):
-        """A decode step's few rows: the two residual norms run as the prologues of the projections that follow them
-        and SiluAndMul as the epilogue of the gate/up projection (``norm_linear_small_m``): 6 launches per layer
-        instead of 9, same roundings."""
-        attn, mlp = self.self_attn, self.mlp
-        ln1, ln2 = self.input_layernorm, self.post_attention_layernorm
-        proj = attn.qkv_projection
-        if residual is None:
-            qkv = norm_linear_small_m(x, proj.weight, proj.bias, ln1.weight_fp32(), ln1.eps)
-            residual = x
-        else:
-            qkv, residual = norm_linear_small_m(x, proj.weight, proj.bias, ln1.weight_fp32(), ln1.eps, residual, True)
-        x = attn.forward_qkv(qkv, positions)
-        act, residual = norm_linear_small_m(x, mlp.gate_up.weight, mlp.gate_up.bias, ln2.weight_fp32(), ln2.eps,
-                                            residual, True, glu=True)
-        return mlp.gate_down(act), residual
+    def _norm_in_product(self, x, weight, glu=False):
+        """A decode step's few rows: the residual norm runs as the prologue of the projection behind it (and SiluAndMul as its
+        epilogue) where that is faster than a launch of its own, with the same roundings."""
+        return (self.norm_rows and self.fused_elementwise and x.dim() == 2 and x.shape[0] <= self.norm_rows and x.is_contiguous()
+                and norm_linear_small_m_pays(x.shape[0], weight) and norm_linear_small_m_takes(x, weight, self.norm_rows, glu=glu))
 
     def forward(self, x, residual, positions):
-        rows = self.norm_rows
-        if (rows and self.fused_elementwise and x.dim() == 2 and x.shape[0] <= rows and x.is_contiguous()
-                and norm_linear_small_m_takes(x, self.self_attn.qkv_projection.weight, rows)
-                and norm_linear_small_m_takes(x, self.mlp.gate_up.weight, rows, glu=True)):
-            return self._forward_few_rows(x, residual, positions)
-        if residual is None:
-            residual = x
-            x = self.input_layernorm(x)
+        attn, mlp, norm = self.self_attn, self.mlp, self.input_layernorm
+        proj = attn.qkv_projection
+        if self._norm_in_product(x, proj.weight):
+            if residual is None:
+                qkv, residual = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps), x
+            else:
+                qkv, residual = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps, residual, True)
+            x = attn.forward_qkv(qkv, positions)
         else:
-            x, residual = self.input_layernorm(x, residual)
-        x = self.self_attn(x, positions)
-        x, residual = self.post_attention_layernorm(x, residual)
-        return self.mlp(x), residual
+            if residual is None:
+                residual = x
+                x = norm(x)
+            else:
+                x, residual = norm(x, residual)
+            x = attn(x, positions)
+        norm = self.post_attention_layernorm
+        if self._norm_in_product(x, mlp.gate_up.weight, glu=True):
+            act, residual = norm_linear_small_m(x, mlp.gate_up.weight, mlp.gate_up.bias, norm.weight_fp32(), norm.eps, residual, True, glu=True)
+            return mlp.gate_down(act), residual
+        x, residual = norm(x, residual)
+        return mlp(x), residual
 
 
 class Qwen3ForCausalLM(nn.Module):

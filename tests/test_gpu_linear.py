@@ -169,3 +169,23 @@ def test_decode_advance_moves_the_step_metadata_forward():
         decode_advance(ids, ctx, pos, slots, sampled, step=step, host_ids=torch.zeros(2, 6, dtype=torch.int64))   # not pinned
     with pytest.raises(ValueError):
         decode_advance(ids, ctx, pos, slots, sampled, host_ids=host)                                             # no counter
+
+
+@pytest.mark.parametrize("m", [1, 8, 9, 20])
+@pytest.mark.parametrize("n,k,glu", [(4112, 512, False), (4128, 1024, True), (4112, 2048, False)])
+def test_norm_linear_last_columns(m, n, k, glu):
+    """Tiles of 32 columns whose last one is half full, one row per wave and two, rows that end inside the second row tile: within two
+    units in the last place of the row's largest output of the separate launches (four behind the activation), as above."""
+    x, w, b = _case(600 + m, m, n, k, torch.bfloat16, True)
+    x = x.contiguous()
+    g = torch.Generator().manual_seed(m)
+    gamma = (1 + 0.2 * torch.randn(k, generator=g)).to(DEV)
+    res = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    assert norm_linear_small_m_takes(x, w, 64, glu=glu)
+    normed, want_res = add_rms_norm(x, gamma, 1e-6, res)
+    want = linear_small_m(normed, w, b)
+    want = silu_and_mul(want) if glu else want
+    got, got_res = norm_linear_small_m(x, w, b, gamma, 1e-6, res, want_residual=True, glu=glu)
+    assert torch.equal(got_res, want_res)
+    worst = ((got.float() - want.float()).abs() / want.float().abs().amax(dim=1, keepdim=True)).max().item()
+    assert worst <= (4 if glu else 2) * 2.0 ** -8, worst
