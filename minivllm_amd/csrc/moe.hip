@@ -3,11 +3,11 @@
 //               largest choice scores, the best `keep` groups stay open; the `top` largest choice scores of those are chosen,
 //               weights s / (sum of the chosen s + 1e-20); or s = softmax(z), the weights s as they are; the last outputs may
 //               stand for no expert but for the input itself: their id is -1
-//   moe_plan    (token, choice) pairs sorted by expert, and tiles of 128 or 256 sorted rows per expert
+//   moe_plan    (token, choice) pairs sorted by expert, and tiles of 64, 128 or 256 sorted rows per expert
 //   moe_linear  out[row] = x[row] W_e^T, optionally silu(gate) * up or its clamped form behind it: W_e [2 F, K] with gate and up rows in turns of
 //               32, so that both halves of an output are in one lane
-// Products, by the number of rows: very few (no plan; a workgroup finds its expert's rows itself, its waves share K), many (bf16: 128 x 128 or 256 x 256
-// tiles on the matrix unit over sorted rows), any (fp32, over sorted rows).
+// Products, by the number of rows: very few (no plan; a workgroup finds its expert's rows itself, its waves share K), many (bf16: tiles of 64 x 128,
+// 128 x 128 or 256 x 256 on the matrix unit over sorted rows), any (fp32, over sorted rows).
 #include "prefill_tiles.h"
 
 #pragma clang fp contract(off)
@@ -124,6 +124,9 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const RouteArgs a) {
 // ---- pairs sorted by expert ----
 constexpr int kPlanPairs = 2048, kMaxExperts = 1024;
 constexpr int kLargeTileRows = 384;      // rows per expert from which tiles are large
+// ... up to which they are small: at 47 per expert (500 rows, top 6 of 64, width 2048) 76 + 42 us against 98 + 44 as tiles of 128, at
+// 65 121 + 73 against 100 + 48: experts of two tiles read their weights twice.
+constexpr int kSmallTileRows = 48;
 
 struct PlanArgs {
   const int32_t* ids;      // [pairs]
@@ -381,15 +384,21 @@ __global__ __launch_bounds__(256) void moe_linear_any_kernel(const ExpertLinearA
   }
 }
 
-// many: 128 sorted rows x 128 weight rows per workgroup, four waves of 64 x 64 on v_mfma_f32_32x32x16_bf16.  Weights are the
-// row operand and x the column operand, so that a lane ends with runs of four outputs of one row.  Steps of 64 along K, two
-// buffers in LDS that the copies of the next step fill during this one; a row's eight 16-byte chunks trade places by half
+// many: 128 weight rows x 32 kRows sorted rows per workgroup, four waves on v_mfma_f32_32x32x16_bf16.  Weights are the row
+// operand and x the column operand, so that a lane ends with runs of four outputs of one row.  Steps of 64 along K through a
+// ring of buffers in LDS that copies of later steps fill during this one; a row's eight 16-byte chunks trade places by half
 // the row's number.  Consecutive workgroups of an XCD go through four row tiles for every weight tile.
-template <int kGlu>
+// kRows 4: a wave has 64 x 64, two buffers.  kRows 2, where experts have so few rows that the stream of weights is the bound: a
+// wave has 64 x 32, the small tile leaves LDS for three buffers of two workgroups per CU (72 KB of copies in flight or use each),
+// and weights, read once by one workgroup, pass the caches by (nt).  900 pairs, 64 experts of 1536 x 2048 and 2048 x 768,
+// weights from memory: 95 + 41 us as 128 x 128 tiles, 72 + 35 us (5.6 and 5.8 TB/s) as these; without nt 80 + 40, six buffers of one
+// workgroup 70 + 41.
+template <int kGlu, int kRows>
 __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLinearArgs a) {
-  constexpr int kTile = 128, kK = 64, kStage = kTile * kK * 2;       // bytes of one operand's step
-  constexpr int kTogether = 4;
-  __shared__ __attribute__((aligned(16))) char lds[4 * kStage];      // [buffer][weights, x]
+  constexpr int kStages = kRows == 4 ? 2 : 3, kTile = 128, kK = 64;
+  constexpr int kW = kTile * kK * 2, kStage = kW + 32 * kRows * kK * 2;   // bytes of the weights' part of a step, of a step
+  constexpr int kTogether = 4, kM = kRows / 2, kCopies = 4 + kRows;       // 32-row blocks per wave; copies per thread and step
+  __shared__ __attribute__((aligned(16))) char lds[kStages * kStage];     // [buffer][weights, x]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
   // ---- which tile ----
   const int total = a.num_tiles[0], per = (total + 7) / 8;
@@ -397,71 +406,77 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
   const int group = j / (kTogether * a.n_tiles), in_group = j % (kTogether * a.n_tiles);
   const int local = group * kTogether + in_group % kTogether, tile = xcd * per + local, n_tile = in_group / kTogether;
   if (local >= per || tile >= total) return;
-  const int e = a.tile_expert[tile], row0 = a.tile_row[tile], row_end = min(row0 + kTile, a.row_start[e + 1]);
+  const int e = a.tile_expert[tile], row0 = a.tile_row[tile], row_end = min(row0 + 32 * kRows, a.row_start[e + 1]);
   const int n0 = n_tile * kTile;
 
-  // ---- copies: four chunks of either operand per thread and step ----
+  // ---- copies: chunks of either operand per thread and step ----
   const v4i w_rows = make_rsrc(reinterpret_cast<const char*>(a.w) + (int64_t)e * a.N * a.K * 2, (uint32_t)((int64_t)a.N * a.K * 2));
   const v4i x_rows = make_rsrc(reinterpret_cast<const char*>(a.x), a.x_bytes);
-  uint32_t from_w[4], from_x[4];
+  uint32_t from_w[4], from_x[kRows];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int c = 256 * i + tid, r = c >> 3, p = (c & 7) ^ ((r >> 1) & 7);
     from_w[i] = (uint32_t)(min(n0 + r, a.N - 1) * a.K + 8 * p) * 2u;
+  }
+#pragma unroll
+  for (int i = 0; i < kRows; ++i) {
+    const int c = 256 * i + tid, r = c >> 3, p = (c & 7) ^ ((r >> 1) & 7);
     const int at = min(row0 + r, row_end - 1);
     const uint32_t xr = (uint32_t)(a.per_token ? a.sorted_pair[at] / a.per_token : at);
     from_x[i] = (xr * (uint32_t)a.x_stride + 8u * p) * 2u;
   }
-  auto copy = [&](int buffer) __attribute__((always_inline)) {
-    const uint32_t base = lds_address(lds) + buffer * 2 * kStage + 1024 * wave;
-    static_for<4>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      dma16_to_lds<4096 * i>(w_rows, from_w[i], base);
-      dma16_to_lds<kStage + 4096 * i>(x_rows, from_x[i], base);
-      from_w[i] += 2 * kK;
-      from_x[i] += 2 * kK;
-    });
+  const int steps = a.K / kK;
+  const uint32_t lds_wave = lds_address(lds) + 1024 * wave;
+  auto copy = [&](int step, int buffer) __attribute__((always_inline)) {      // past the last step nothing is read, and the count stays
+    v4i w = w_rows, x = x_rows;
+    if (kStages > 2) {
+      w[2] = step < steps ? w[2] : 0;
+      x[2] = step < steps ? x[2] : 0;
+    }
+    const uint32_t at = (uint32_t)step * (2 * kK), base = lds_wave + buffer * kStage;
+    static_for<4>([&](auto I) { dma16_to_lds_at<4096 * decltype(I)::value, kRows == 2>(w, from_w[decltype(I)::value], at, base); });
+    static_for<kRows>([&](auto I) { dma16_to_lds_at<kW + 4096 * decltype(I)::value>(x, from_x[decltype(I)::value], at, base); });
   };
   const int wn = wave & 1, wm = wave >> 1;          // the wave's half of the weight rows and of the rows
   // places of this lane's fragments: row l32 of a 32-row block, chunk 2 st + hi
   const int sw = (l32 >> 1) & 7;
   const char* frag = lds + l32 * 128;
-  v16f acc[2][2];
+  v16f acc[2][kM];
 #pragma unroll
   for (int n = 0; n < 2; ++n)
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+    for (int m = 0; m < kM; ++m)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[n][m][r] = 0.f;
 
-  copy(0);
-  const int steps = a.K / kK;
+  static_for<kStages - 1>([&](auto I) { copy(decltype(I)::value, decltype(I)::value); });
+  int buffer = 0;
   for (int step = 0; step < steps; ++step) {
-    const int buffer = step & 1;
-    dma_wait_all();
-    __syncthreads();                                // this step's operands are there, the other buffer is free
-    if (step + 1 < steps) copy(buffer ^ 1);
-    const char* wb = frag + buffer * 2 * kStage + wn * 64 * 128;
-    const char* xb = frag + buffer * 2 * kStage + kStage + wm * 64 * 128;
+    dma_wait_but<kCopies * (kStages - 2)>();
+    workgroup_barrier();                            // this step's operands are there, the buffer of the step before is free
+    if (kStages > 2 || step + 1 < steps) copy(step + kStages - 1, buffer == 0 ? kStages - 1 : buffer - 1);
+    const char* wb = frag + buffer * kStage + wn * 64 * 128;
+    const char* xb = frag + buffer * kStage + kW + wm * (32 * kM) * 128;
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
       const int p = ((2 * st + hi) ^ sw) << 4;
-      uint4 wf[2], xf[2];
+      uint4 wf[2], xf[kM];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        wf[i] = *reinterpret_cast<const uint4*>(wb + i * 32 * 128 + p);
-        xf[i] = *reinterpret_cast<const uint4*>(xb + i * 32 * 128 + p);
-      }
+      for (int i = 0; i < 2; ++i) wf[i] = *reinterpret_cast<const uint4*>(wb + i * 32 * 128 + p);
+#pragma unroll
+      for (int i = 0; i < kM; ++i) xf[i] = *reinterpret_cast<const uint4*>(xb + i * 32 * 128 + p);
 #pragma unroll
       for (int n = 0; n < 2; ++n)
 #pragma unroll
-        for (int m = 0; m < 2; ++m) acc[n][m] = mfma32x32x16<bf16_t>(wf[n], xf[m], acc[n][m]);
+        for (int m = 0; m < kM; ++m) acc[n][m] = mfma32x32x16<bf16_t>(wf[n], xf[m], acc[n][m]);
     }
+    buffer = buffer + 1 == kStages ? 0 : buffer + 1;
   }
+  if (kStages > 2) dma_wait_all();                  // (copies past the last step)
   // ---- lane: row l32 of a block, weight rows 8 (r / 4) + 4 hi + r % 4 ----
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    const int row = row0 + wm * 64 + 32 * m + l32;
+  for (int m = 0; m < kM; ++m) {
+    const int row = row0 + (wm * kM + m) * 32 + l32;
     if (row >= row_end) continue;
     bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (int64_t)row * a.out_stride;
 #pragma unroll
@@ -477,7 +492,8 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
         for (int n = 0; n < 2; ++n) {
           const int col = n0 + wn * 64 + 32 * n + 2 * r + 4 * hi;
           if (col < a.N)
-            *reinterpret_cast<uint2*>(out + col) = make_uint2(pack2<bf16_t>(acc[n][m][r], acc[n][m][r + 1]), pack2<bf16_t>(acc[n][m][r + 2], acc[n][m][r + 3]));
+            *reinterpret_cast<uint2*>(out + col) = make_uint2(pack2<bf16_t>(acc[n][m][r], acc[n][m][r + 1]),
+                                                              pack2<bf16_t>(acc[n][m][r + 2], acc[n][m][r + 3]));
         }
       }
     }
@@ -631,8 +647,10 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
   }
 }
 
-// Rows of a tile: large ones where experts have enough rows on average to fill them.
-static int tile_rows(int64_t pairs, int experts) { return pairs >= kLargeTileRows * (int64_t)experts ? 256 : 128; }
+// Rows of a tile: large ones where experts have enough rows on average to fill them, small ones where most experts fit in one.
+static int tile_rows(int64_t pairs, int experts) {
+  return pairs >= kLargeTileRows * (int64_t)experts ? 256 : pairs > kSmallTileRows * (int64_t)experts ? 128 : 64;
+}
 static int64_t max_tiles(int64_t pairs, int experts) { return (pairs + tile_rows(pairs, experts) - 1) / tile_rows(pairs, experts) + experts; }
 static int plan_blocks(int64_t pairs) { return (int)((pairs + kPlanPairs - 1) / kPlanPairs); }
 
@@ -750,18 +768,18 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
   a.num_tiles = p.num_tiles;
   if (dtype == MVLLM_BF16) {
     a.max_tiles = (int)max_tiles(pairs, experts);
-    a.n_tiles = (N + p.tile_rows - 1) / p.tile_rows;
+    a.n_tiles = p.tile_rows == 256 ? (N + 255) / 256 : (N + 127) / 128;
     if (p.tile_rows == 256 && out_row_stride % 8 != 0) return MVLLM_ERR_UNSUPPORTED;
     const int64_t x_rows = per_token ? (pairs + per_token - 1) / per_token : pairs, x_bytes = ((x_rows - 1) * x_row_stride + K) * 2;
     if (x_bytes >= (int64_t)1 << 32 || (int64_t)N * K * 2 >= (int64_t)1 << 31) return MVLLM_ERR_UNSUPPORTED;
     a.x_bytes = (uint32_t)x_bytes;
     const int64_t per = (a.max_tiles + 7) / 8, groups = (per + 3) / 4, blocks = 8 * groups * 4 * a.n_tiles;
     if (blocks > 0x7fffffff) return MVLLM_ERR_BAD_SHAPE;
-    const bool large = p.tile_rows == 256;
     with_glu(glu, [&](auto G) {
       constexpr int kGlu = decltype(G)::value;
-      if (large) moe_linear_large_kernel<kGlu><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
-      else moe_linear_many_kernel<kGlu><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      if (p.tile_rows == 256) moe_linear_large_kernel<kGlu><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      else if (p.tile_rows == 128) moe_linear_many_kernel<kGlu, 4><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      else moe_linear_many_kernel<kGlu, 2><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
     });
   } else {
     int64_t z = pairs / (16 * (int64_t)experts) + 1;

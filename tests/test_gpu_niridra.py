@@ -513,6 +513,22 @@ def test_moe_linear(rows, top, experts, n, k, path):
     assert row_rel(out, want) < tol(dtype, 1e-5, 1e-2)
 
 
+@pytest.mark.parametrize("n,k", [(64, 64), (80, 128), (336, 192)])
+def test_moe_linear_row_tile_edges(n, k):
+    """Few pairs per expert on average, so tiles of 64 rows, and experts one short of a tile, at it, past it and of several; fewer
+    steps along K than the ring has buffers."""
+    counts, g = [63, 64, 65, 0, 1, 129, 2, 32, 33, 5], gen(n + k)
+    experts, pairs = len(counts), sum(counts)
+    ids = torch.cat([torch.full((c,), i) for i, c in enumerate(counts)])[torch.randperm(pairs, generator=g)].int().view(-1, 1)
+    x = torch.randn(pairs, k, generator=g).bfloat16()
+    w = (torch.randn(experts, n, k, generator=g) * k ** -0.5).bfloat16()
+    plan = moe_plan(ids.to(DEV), experts)
+    place = plan.place.cpu().long()
+    out = moe_linear(x.to(DEV), w.to(DEV), ids.to(DEV), plan, 1).cpu()[place]
+    want = torch.einsum("pk,pnk->pn", x.double(), w.double()[ids.view(-1).long()])
+    assert row_rel(out, want) < 1e-2
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("cfg", [moe(), moe(experts=12, top=5, groups=(3, 2), ff=72, shared=100), moe(experts=5, top=1, groups=None, shared=None),
                                  moe(experts=40, top=8, groups=(8, 3), ff=64, shared=16)], ids=["a", "b", "c", "d"])
