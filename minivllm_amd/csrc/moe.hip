@@ -136,7 +136,7 @@ struct PlanArgs {
   int32_t* row_start;      // [E + 1]
   int32_t* tile_expert;    // [max tiles]
   int32_t* tile_row;       // [max tiles]: first sorted row
-  int32_t* num_tiles;      // [1]
+  int32_t* num_tiles;      // [2] those in order, those behind them (see find_tile)
   int pairs, experts, blocks, tile_rows;
 };
 
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void moe_count_kernel(const PlanArgs a) {
 }
 
 __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
-  __shared__ int32_t total[kMaxExperts + 1], tiles[kMaxExperts + 1], cursor[kMaxExperts];
+  __shared__ int32_t total[kMaxExperts + 1], tiles[kMaxExperts + 1], parts[kMaxExperts + 1], cursor[kMaxExperts];
   const int e = threadIdx.x;
   int n = 0, mine = 0;
   if (a.blocks == 1) {                              // counted here
@@ -174,14 +174,17 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
     }
   // inclusive sums over the experts
   total[e + 1] = n;
-  tiles[e + 1] = (n + a.tile_rows - 1) / a.tile_rows;
-  if (e == 0) total[0] = tiles[0] = 0;
+  const bool apart = a.tile_rows == 256 && n % 256 != 0;      // the last tile, not whole, goes behind all whole ones
+  tiles[e + 1] = (n + a.tile_rows - 1) / a.tile_rows - apart;
+  parts[e + 1] = apart;
+  if (e == 0) total[0] = tiles[0] = parts[0] = 0;
   __syncthreads();
   for (int o = 1; o < 1024; o <<= 1) {
-    const int x = e + 1 > o ? total[e + 1 - o] : 0, y = e + 1 > o ? tiles[e + 1 - o] : 0;
+    const int x = e + 1 > o ? total[e + 1 - o] : 0, y = e + 1 > o ? tiles[e + 1 - o] : 0, z = e + 1 > o ? parts[e + 1 - o] : 0;
     __syncthreads();
     total[e + 1] += x;
     tiles[e + 1] += y;
+    parts[e + 1] += z;
     __syncthreads();
   }
   if (e < a.experts) cursor[e] = total[e] + mine;
@@ -202,10 +205,16 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
     if (e == a.experts - 1) {
       a.row_start[e + 1] = total[e + 1];
       a.num_tiles[0] = tiles[e + 1];
+      a.num_tiles[1] = parts[e + 1];
     }
     for (int t = tiles[e]; t < tiles[e + 1]; ++t) {
       a.tile_expert[t] = e;
       a.tile_row[t] = total[e] + (t - tiles[e]) * a.tile_rows;
+    }
+    if (apart) {
+      const int t = tiles[kMaxExperts] + parts[e];
+      a.tile_expert[t] = e;
+      a.tile_row[t] = total[e + 1] - n % 256;
     }
   }
 }
@@ -384,6 +393,28 @@ __global__ __launch_bounds__(256) void moe_linear_any_kernel(const ExpertLinearA
   }
 }
 
+// The tile of rows and of weights that a workgroup of the tiled products takes; false: none.  Each XCD has an eighth of the (row tile,
+// weight tile) pairs, to one: shares of whole row tiles left the last XCD a third of the others' work (66 tiles: seven of 9, one of 3).
+// Row tiles go in fours: workgroups of a four with the same weight tile follow one another.  Large tiles that are not whole, and so take
+// less time, come behind all whole ones, in turns over the XCDs: the chip's last round is made of short ones.  600 rows, top 6 of 64
+// with uneven routing, width 2048: 132 + 71 -> 101 + 62 us; 8192 rows with what follows at the large kernel: 387 + 239 -> 376 + 222.
+__device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, int& n_tile) {
+  constexpr int kTogether = 4;
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int whole = a.num_tiles[0], rest = a.num_tiles[1], per = (whole * a.n_tiles + 7) / 8;
+  if (j < per) {
+    const int at = xcd * per + j;
+    if (at >= whole * a.n_tiles) return false;
+    const int first = at / (kTogether * a.n_tiles) * kTogether, in = at - first * a.n_tiles, together = min(kTogether, whole - first);
+    tile = first + in % together;
+    n_tile = in / together;
+    return true;
+  }
+  tile = whole + xcd + 8 * ((j - per) / a.n_tiles);
+  n_tile = (j - per) % a.n_tiles;
+  return tile < whole + rest;
+}
+
 // many: 128 weight rows x 32 kRows sorted rows per workgroup, four waves on v_mfma_f32_32x32x16_bf16.  Weights are the row
 // operand and x the column operand, so that a lane ends with runs of four outputs of one row.  Steps of 64 along K through a
 // ring of buffers in LDS that copies of later steps fill during this one; a row's eight 16-byte chunks trade places by half
@@ -397,15 +428,12 @@ template <int kGlu, int kRows>
 __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLinearArgs a) {
   constexpr int kStages = kRows == 4 ? 2 : 3, kTile = 128, kK = 64;
   constexpr int kW = kTile * kK * 2, kStage = kW + 32 * kRows * kK * 2;   // bytes of the weights' part of a step, of a step
-  constexpr int kTogether = 4, kM = kRows / 2, kCopies = 4 + kRows;       // 32-row blocks per wave; copies per thread and step
+  constexpr int kM = kRows / 2, kCopies = 4 + kRows;       // 32-row blocks per wave; copies per thread and step
   __shared__ __attribute__((aligned(16))) char lds[kStages * kStage];     // [buffer][weights, x]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
   // ---- which tile ----
-  const int total = a.num_tiles[0], per = (total + 7) / 8;
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  const int group = j / (kTogether * a.n_tiles), in_group = j % (kTogether * a.n_tiles);
-  const int local = group * kTogether + in_group % kTogether, tile = xcd * per + local, n_tile = in_group / kTogether;
-  if (local >= per || tile >= total) return;
+  int tile, n_tile;
+  if (!find_tile(a, tile, n_tile)) return;
   const int e = a.tile_expert[tile], row0 = a.tile_row[tile], row_end = min(row0 + 32 * kRows, a.row_start[e + 1]);
   const int n0 = n_tile * kTile;
 
@@ -508,14 +536,10 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
 template <int kGlu>
 __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLinearArgs a) {
   constexpr int kTile = 256, kK = 64, kStage = kTile * kK * 2;       // bytes of one operand's step
-  constexpr int kTogether = 4;
   __shared__ __attribute__((aligned(16))) char lds[5 * kStage];      // weights three times, x twice
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
-  const int total = a.num_tiles[0], per = (total + 7) / 8;
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  const int group = j / (kTogether * a.n_tiles), in_group = j % (kTogether * a.n_tiles);
-  const int local = group * kTogether + in_group % kTogether, tile = xcd * per + local, n_tile = in_group / kTogether;
-  if (local >= per || tile >= total) return;
+  int tile, n_tile;
+  if (!find_tile(a, tile, n_tile)) return;
   const int e = a.tile_expert[tile], row0 = a.tile_row[tile], row_end = min(row0 + kTile, a.row_start[e + 1]);
   const int n0 = n_tile * kTile;
 
@@ -560,73 +584,92 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
 #pragma unroll
   for (int st = 0; st < 4; ++st) place[st] = ((2 * st + hi) ^ sw) << 4;
   const char* w_frag = frag + wn * (128 * 128);
-  const char* x_frag = frag + wm * (128 * 128) + kX;
-  // The products of a 16-wide step one by one; after each of them one of the next step's reads (every kEvery-th from product
-  // kFirst on, those that are needed first come first) and whatever `also` does: the matrix unit must not wait for a queue of
-  // reads or copies.
-  auto products = [&](auto SET, auto FIRST, auto EVERY, const char* wb, const char* xb, auto&& also) __attribute__((always_inline)) {
-    constexpr int set = decltype(SET)::value, next = set ^ 1, kFirst = decltype(FIRST)::value, kEvery = decltype(EVERY)::value;
-    static_for<16>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      acc[i / 4][i % 4] = mfma32x32x16<bf16_t>(wf[set][i / 4], xf[set][i % 4], acc[i / 4][i % 4]);
-      also(I);
-      if constexpr (i >= kFirst && (i - kFirst) % kEvery == 0 && (i - kFirst) / kEvery < 8) {
-        constexpr int j = (i - kFirst) / kEvery;
-        if constexpr (j >= 1 && j <= 4) xf[next][j - 1] = *reinterpret_cast<const uint4*>(xb + (j - 1) * 32 * 128);
-        else wf[next][j == 0 ? 0 : j - 4] = *reinterpret_cast<const uint4*>(wb + (j == 0 ? 0 : j - 4) * 32 * 128);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  };
+  const char* x_frag = frag + wm * (32 * 128) + kX;
   constexpr std::integral_constant<int, 0> c0{};
   constexpr std::integral_constant<int, 1> c1{};
-  constexpr std::integral_constant<int, 2> c2{};
-  constexpr std::integral_constant<int, 4> c4{};
-  auto nothing = [](auto) {};
+  // The product with kBlocks blocks of 32 rows for each wave, those of the two halves in turns: a tile that is not whole takes no more
+  // time than its rows do.
+  auto run = [&](auto BLOCKS) __attribute__((always_inline)) {
+    constexpr int kBlocks = decltype(BLOCKS)::value, kProducts = 4 * kBlocks, kPer = kBlocks == 1 ? 2 : 1;
+    // The products of a 16-wide step one by one; after each of them one of the next step's reads (every kEvery-th from product
+    // kFirst on, those that are needed first come first) and whatever `also` does: the matrix unit must not wait for a queue of
+    // reads or copies.
+    auto products = [&](auto SET, auto FIRST, auto EVERY, const char* wb, const char* xb, auto&& also) __attribute__((always_inline)) {
+      constexpr int set = decltype(SET)::value, next = set ^ 1, kFirst = decltype(FIRST)::value, kEvery = decltype(EVERY)::value;
+      static_for<kProducts>([&](auto I) {
+        constexpr int i = decltype(I)::value, n = i / kBlocks, m = i % kBlocks;
+        acc[n][m] = mfma32x32x16<bf16_t>(wf[set][n], xf[set][m], acc[n][m]);
+        also(I);
+        if constexpr (i >= kFirst && (i - kFirst) % kEvery == 0) {
+          static_for<kPer>([&](auto Q) {
+            constexpr int j = (i - kFirst) / kEvery * kPer + decltype(Q)::value;
+            if constexpr (j >= 1 && j <= kBlocks) xf[next][j - 1] = *reinterpret_cast<const uint4*>(xb + (j - 1) * 64 * 128);
+            else if constexpr (j < 4 + kBlocks) {
+              constexpr int w = j == 0 ? 0 : j - kBlocks;
+              wf[next][w] = *reinterpret_cast<const uint4*>(wb + w * 32 * 128);
+            }
+          });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    constexpr std::integral_constant<int, kBlocks == 4 ? 2 : 1> spread{};
+    auto nothing = [](auto) {};
 
-  static_for<8>([&](auto I) {
-    copy_w(I, 0, 0);
-    copy_x(I, 0);
-    copy_w(I, 1, kStage);
-  });
-  dma_wait_all();
-  __syncthreads();
-  static_for<8>([&](auto I) { copy_x(I, 1); });
+    static_for<8>([&](auto I) {
+      copy_w(I, 0, 0);
+      if constexpr (decltype(I)::value < 2 * kBlocks) copy_x(I, 0);
+      copy_w(I, 1, kStage);
+    });
+    dma_wait_all();
+    __syncthreads();
+    static_for<2 * kBlocks>([&](auto I) { copy_x(I, 1); });
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    wf[0][i] = *reinterpret_cast<const uint4*>(w_frag + place[0] + i * 32 * 128);
-    xf[0][i] = *reinterpret_cast<const uint4*>(x_frag + place[0] + i * 32 * 128);
+    for (int i = 0; i < 4; ++i) {
+      wf[0][i] = *reinterpret_cast<const uint4*>(w_frag + place[0] + i * 32 * 128);
+      if (i < kBlocks) xf[0][i] = *reinterpret_cast<const uint4*>(x_frag + place[0] + i * 64 * 128);
+    }
+    uint32_t w_at = 0;                              // the weights' buffer of this step, in bytes
+    for (int step = 0; step < steps; ++step) {
+      const uint32_t w_next = w_at == 2 * kStage ? 0 : w_at + kStage, w_free = w_at == 0 ? 2 * kStage : w_at - kStage;
+      const char* wb = w_frag + w_at;
+      const char* xb = x_frag + (step & 1) * kStage;
+      // the weights two steps ahead, into the buffer that the step before this one has left
+      products(c0, c1, spread, wb + place[1], xb + place[1], [&](auto I) {
+        constexpr int i = decltype(I)::value;
+        if constexpr (kBlocks == 4) {
+          if constexpr (i % 2 == 0) copy_w(std::integral_constant<int, i / 2>{}, step + 2, w_free);
+        } else if constexpr (i * kPer < 8)
+          static_for<kPer>([&](auto Q) { copy_w(std::integral_constant<int, i * kPer + decltype(Q)::value>{}, step + 2, w_free); });
+      });
+      products(c1, c1, spread, wb + place[2], xb + place[2], nothing);
+      products(c0, c1, spread, wb + place[3], xb + place[3], nothing);
+      // the next step's operands have to be there before its first reads, and this step's have been read: then x two steps
+      // ahead follows into its buffer.  What may be in flight until then are the eight copies of weights from above.
+      products(c1, BLOCKS, c1, w_frag + w_next + place[0], x_frag + ((step & 1) ^ 1) * kStage + place[0], [&](auto I) {
+        constexpr int i = decltype(I)::value;
+        if constexpr (i == kBlocks - 1) {
+          dma_wait_but<8>();
+          workgroup_barrier();
+        }
+        if constexpr (i >= 2 * kBlocks) copy_x(std::integral_constant<int, i - 2 * kBlocks>{}, step + 2);
+      });
+      w_at = w_next;
+    }
+    dma_wait_all();                                 // (copies past the last step)
+  };
+  switch ((row_end - row0 + 63) / 64) {
+    case 1: run(c1); break;
+    case 2: run(std::integral_constant<int, 2>{}); break;
+    case 3: run(std::integral_constant<int, 3>{}); break;
+    default: run(std::integral_constant<int, 4>{});
   }
-  uint32_t w_at = 0;                                // the weights' buffer of this step, in bytes
-  for (int step = 0; step < steps; ++step) {
-    const uint32_t w_next = w_at == 2 * kStage ? 0 : w_at + kStage, w_free = w_at == 0 ? 2 * kStage : w_at - kStage;
-    const char* wb = w_frag + w_at;
-    const char* xb = x_frag + (step & 1) * kStage;
-    // the weights two steps ahead, into the buffer that the step before this one has left
-    products(c0, c1, c2, wb + place[1], xb + place[1], [&](auto I) {
-      constexpr int i = decltype(I)::value;
-      if constexpr (i % 2 == 0) copy_w(std::integral_constant<int, i / 2>{}, step + 2, w_free);
-    });
-    products(c1, c1, c2, wb + place[2], xb + place[2], nothing);
-    products(c0, c1, c2, wb + place[3], xb + place[3], nothing);
-    // the next step's operands have to be there before its first reads, and this step's have been read: then x two steps
-    // ahead follows into its buffer.  What may be in flight until then are the eight copies of weights from above.
-    products(c1, c4, c1, w_frag + w_next + place[0], x_frag + ((step & 1) ^ 1) * kStage + place[0], [&](auto I) {
-      constexpr int i = decltype(I)::value;
-      if constexpr (i == 3) {
-        dma_wait_but<8>();
-        workgroup_barrier();
-      }
-      if constexpr (i >= 8) copy_x(std::integral_constant<int, i - 8>{}, step + 2);
-    });
-    w_at = w_next;
-  }
-  dma_wait_all();                                   // (copies past the last step)
   // ---- lane: row l32 of a block, weight rows 8 (r / 4) + 4 hi + r % 4; halves of the wave trade runs of four, so that a lane
   // stores eight outputs in a row ----
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
-    const int row = row0 + wm * 128 + 32 * m + l32;
+    if (row0 + 32 * (wm + 2 * m) >= row_end) break;
+    const int row = row0 + 32 * (wm + 2 * m) + l32;
     bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (int64_t)min(row, row_end - 1) * a.out_stride;
 #pragma unroll
     for (int n = 0; n < (kGlu ? 2 : 4); ++n) {
@@ -697,7 +740,7 @@ extern "C" int mvllm_moe_route_softmax(int32_t* ids, float* weights, const float
 
 extern "C" size_t mvllm_moe_plan_bytes(int64_t pairs, int experts) {
   if (pairs <= 0 || experts <= 0) return 0;
-  return (size_t)(2 * pairs + experts + 1 + 2 * max_tiles(pairs, experts) + 1 + (int64_t)plan_blocks(pairs) * experts + 4) * sizeof(int32_t);
+  return (size_t)(2 * pairs + experts + 1 + 2 * max_tiles(pairs, experts) + 2 + (int64_t)plan_blocks(pairs) * experts + 4) * sizeof(int32_t);
 }
 
 // the parts of a plan, in order
@@ -710,7 +753,7 @@ static PlanArgs plan_parts_of(void* plan, const int32_t* ids, int64_t pairs, int
   a.tile_expert = a.row_start + experts + 1;
   a.tile_row = a.tile_expert + max_tiles(pairs, experts);
   a.num_tiles = a.tile_row + max_tiles(pairs, experts);
-  a.hist = a.num_tiles + 1;
+  a.hist = a.num_tiles + 2;
   a.pairs = (int)pairs; a.experts = experts; a.blocks = plan_blocks(pairs);
   a.tile_rows = tile_rows(pairs, experts);
   return a;
@@ -773,7 +816,7 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
     const int64_t x_rows = per_token ? (pairs + per_token - 1) / per_token : pairs, x_bytes = ((x_rows - 1) * x_row_stride + K) * 2;
     if (x_bytes >= (int64_t)1 << 32 || (int64_t)N * K * 2 >= (int64_t)1 << 31) return MVLLM_ERR_UNSUPPORTED;
     a.x_bytes = (uint32_t)x_bytes;
-    const int64_t per = (a.max_tiles + 7) / 8, groups = (per + 3) / 4, blocks = 8 * groups * 4 * a.n_tiles;
+    const int64_t blocks = 8 * (((int64_t)a.max_tiles * a.n_tiles + 7) / 8 + 1 + a.n_tiles);
     if (blocks > 0x7fffffff) return MVLLM_ERR_BAD_SHAPE;
     with_glu(glu, [&](auto G) {
       constexpr int kGlu = decltype(G)::value;

@@ -514,10 +514,11 @@ def test_moe_linear(rows, top, experts, n, k, path):
 
 
 @pytest.mark.parametrize("n,k", [(64, 64), (80, 128), (336, 192)])
-def test_moe_linear_row_tile_edges(n, k):
-    """Few pairs per expert on average, so tiles of 64 rows, and experts one short of a tile, at it, past it and of several; fewer
-    steps along K than the ring has buffers."""
-    counts, g = [63, 64, 65, 0, 1, 129, 2, 32, 33, 5], gen(n + k)
+@pytest.mark.parametrize("counts", [[63, 64, 65, 0, 1, 129, 2, 32, 33, 5], [256, 0, 257, 513, 320, 321, 640, 700, 1023, 449, 128, 2]], ids=["small", "large"])
+def test_moe_linear_row_tile_edges(counts, n, k):
+    """Few pairs per expert on average, so tiles of 64 rows, or many, so tiles of 256: experts one short of a tile, at it, past it and of
+    several, and every number of 64-row parts of a last one; fewer steps along K than the ring has buffers."""
+    g = gen(n + k)
     experts, pairs = len(counts), sum(counts)
     ids = torch.cat([torch.full((c,), i) for i, c in enumerate(counts)])[torch.randperm(pairs, generator=g)].int().view(-1, 1)
     x = torch.randn(pairs, k, generator=g).bfloat16()
