@@ -573,6 +573,8 @@ int mvllm_gate_linear(float* out, const void* x, int64_t x_row_stride, const voi
  *   first row, rows, flags (1 first, 2 last, 4 the only one of its entry), the segments of an entry in order and next to
  *   each other, all but the last a multiple of 64 rows.  split != 0 (some entry has several): workspace of
  *   mvllm_mlstm_chunked_workspace_bytes.
+ * mvllm_mlstm_chunked_output: the same for dim <= 128 and vdim <= 256 with mvllm_mlstm_output behind it, in one pass: out's rows
+ *   of these entries (16-byte aligned, like weight), m_state[slot].  gate: rows proj_row_stride apart, 8-byte aligned.
  */
 int mvllm_mlstm_recurrent(float* num, float* den, float* m_next, const void* proj, int64_t proj_row_stride,
                           const float* gates, float* s_state, float* n_state, const float* m_state,
@@ -584,6 +586,11 @@ int mvllm_mlstm_chunked(float* num, float* den, float* m_next, const void* proj,
                         const int32_t* cu_seqlens, const int32_t* slots, const int64_t* positions,
                         const int32_t* segments, int num_segments, int split, int num_heads, int dim, int vdim,
                         float q_scale, float floor, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+int mvllm_mlstm_chunked_output(void* out, const float* weight, const void* gate, float eps, const void* proj,
+                               int64_t proj_row_stride, const float* gates, float* s_state, float* n_state, float* m_state,
+                               const int32_t* cu_seqlens, const int32_t* slots, const int64_t* positions,
+                               const int32_t* segments, int num_segments, int split, int num_heads, int dim, int vdim,
+                               float q_scale, float floor, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 int mvllm_mlstm_output(void* out, const float* num, const float* den, const float* weight, const void* gate,
                        int64_t gate_row_stride, float eps, const float* m_next, float* m_state,
                        const int32_t* cu_seqlens, const int32_t* row_entry, const int32_t* slots, int64_t rows,

@@ -48,6 +48,12 @@ struct MemoryChunkArgs {
   float q_scale, floor;
   const float* log_decay;    // [H], without gates
   int silu;                  // q, k and v are taken through z * sigmoid(z)
+  // with kOut
+  bf16_t* out;               // [T, H * vdim]
+  const float* weight;       // [H * vdim]
+  const bf16_t* gate;        // [T, proj_stride]: H * vdim pre-activations per row
+  float* m_out;              // [slots, H]: m_state
+  float eps;
 };
 
 // eight packed values through z * sigmoid(z), rounded again
@@ -77,7 +83,27 @@ __device__ __forceinline__ Split8 split8(const float* x) {
   return {make_uint4(h[0], h[1], h[2], h[3]), make_uint4(l[0], l[1], l[2], l[3])};
 }
 
-template <int DIMP, int kWaves, bool kStateOnly, bool kGates>
+// Sums and maxima of this lane and all before it, in registers: within rows of 16 lanes, then over the rows.  (Six steps of 8 cycles; through
+// the LDS' permutes, six of over 100, every block waited 8 us in all over 1024 rows for its two scans.)
+template <typename F> __device__ __forceinline__ float wave_scan(float x, float nothing, F f) {
+  auto from = [&](auto CTRL, auto ROWS) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(nothing), __float_as_int(x), decltype(CTRL)::value, decltype(ROWS)::value, 0xf, false));
+  };
+  x = f(x, from(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{}));    // 1, 2, 4, 8 lanes on
+  x = f(x, from(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{}));
+  x = f(x, from(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{}));
+  x = f(x, from(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{}));
+  x = f(x, from(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{}));    // rows 0 and 2 to the next ones
+  return f(x, from(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{})); // the first half to the second
+}
+
+// kOut (with gates, vdim <= 256, eight waves: whole heads): the results go through the norm and the output gate here, out = rms(num / den)
+// weight sigmoid(gate), and the sums never leave the chip.  8 x 1024 rows, 16 heads of 128 x 256: 155 us where the sums' pass took 119
+// and their norm 56 (two times 134 MB).  The vector unit bounds it: two waves per SIMD issue 16 of a block's 20 thousand cycles, a
+// quarter of them for norm and gate (116 us without), and 128 workgroups leave half the CUs idle; segments to fill them cost as much as
+// they bring (158 us), since their states are a pass of their own.  Scores are 16 x 16 tiles so that all waves have some (143 without
+// them), the normaliser and n are spread over all threads.
+template <int DIMP, int kWaves, bool kStateOnly, bool kGates, bool kOut>
 __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk_kernel(const MemoryChunkArgs a) {
   constexpr int kThreads = 64 * kWaves;
   constexpr int VT = 32 * kWaves;                  // value columns of the workgroup
@@ -89,7 +115,12 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
   __shared__ __attribute__((aligned(16))) uint16_t vs[kBlock * kVRow];
   __shared__ __attribute__((aligned(16))) uint16_t ph[kStateOnly ? 8 : kBlock * kPRow], pl[kStateOnly ? 8 : kBlock * kPRow];
   __shared__ float sc_a[kBlock], sc_M[kBlock], sc_in[kBlock], sc_w[kBlock], sc_floor[kBlock];
-  __shared__ float n_lds[kGates ? DIMP : 1], n_part[kGates ? kThreads * 2 : 1];
+  __shared__ __attribute__((aligned(16))) float n_lds[kGates ? DIMP : 4];
+  __shared__ float n_part[kGates ? kThreads * 2 : 1];
+  constexpr int kORow = VT + 8;
+  __shared__ __attribute__((aligned(16))) float os[kOut ? kBlock * kORow : 4];
+  __shared__ float sc_den[kOut ? kBlock : 1];
+  static_assert(!kOut || (kGates && !kStateOnly && kWaves == 8), "whole heads, with gates");
 
   const int seg = blockIdx.x, h = blockIdx.y, tile = blockIdx.z;
   const int entry = a.segments[4 * seg], row0 = a.segments[4 * seg + 1], rows = a.segments[4 * seg + 2];
@@ -135,6 +166,17 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
         s[td][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(state, s_first + (uint32_t)((32 * td + 8 * (r >> 2) + (r & 3)) * vdim) * 4u, 0, 0));
       __builtin_amdgcn_sched_barrier(0);
     });
+  }
+  const int out_c = 4 * lane;                       // kOut: this lane's columns of a row
+  float4 out_w = make_float4(0.f, 0.f, 0.f, 0.f);
+  uint2 gr[kOut ? kBlock / kWaves : 1];             // ... its part of the output gate, of rows kBlock / kWaves * wave + i
+  if constexpr (kOut) {
+    if (out_c < vdim) out_w = *reinterpret_cast<const float4*>(a.weight + (int64_t)h * vdim + out_c);
+    // of the scores' 16 x 16 tiles past the diagonal the products read two
+    for (int i = tid; i < 2 * 16 * 16; i += kThreads) {
+      const int t = 32 * (i >> 8) + ((i >> 4) & 15), x = 32 * (i >> 8) + 16 + (i & 15);
+      ph[t * kPRow + x] = pl[t * kPRow + x] = 0;
+    }
   }
   if (n_owner)
     for (int d = tid; d < DIMP; d += kThreads) n_lds[d] = n_in != nullptr && d < dim ? n_in[d] : 0.f;
@@ -201,25 +243,16 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
     for (int i = 0; i < kVLoads; ++i) *reinterpret_cast<uint4*>(&vs[(v_r + i * kVStep) * kVRow + v_d]) = vr[i];
     float decay;                                    // of the state over the block
     if constexpr (kGates) {
-      float F = gate_f;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const float t = __shfl_up(F, o, 64);
-        if (lane >= o) F += t;
-      }
+      const float F = wave_scan(gate_f, 0.f, [](float x, float y) { return x + y; });
       const float av = gate_i - F;
-      float M = fmaxf(av, m);
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const float t = __shfl_up(M, o, 64);
-        if (lane >= o) M = fmaxf(M, t);
-      }
-      const float M_last = __shfl(M, 63, 64), F_last = __shfl(F, 63, 64);
+      const float M = wave_scan(fmaxf(av, m), -INFINITY, [](float x, float y) { return fmaxf(x, y); });
+      const float M_last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(M), 63));
+      const float F_last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(F), 63));
       decay = __expf(m - M_last);
       if (wave == 0) {
         sc_a[lane] = av;
         sc_M[lane] = M;
-        sc_in[lane] = __expf(m - M);
+        sc_in[lane] = __expf(m - M) * a.q_scale;
         sc_w[lane] = __expf(av - M_last);
         sc_floor[lane] = __expf(-(F + M));
       }
@@ -232,17 +265,117 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
       if (wave == 0) {
         sc_a[lane] = -(float)lane * log_decay;
         sc_M[lane] = -(float)lane * log_decay;
-        sc_in[lane] = __expf((float)(lane + 1) * log_decay);
+        sc_in[lane] = __expf((float)(lane + 1) * log_decay) * a.q_scale;
         sc_w[lane] = lane < n ? __expf((float)(n - 1 - lane) * log_decay) : 0.f;
       }
     }
     __syncthreads();
+    if constexpr (kOut) {
+      uint32_t pitch = pitch_in;
+      asm volatile("" : "+s"(pitch));
+      const auto g_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(a.gate + (int64_t)(row0 + at) * a.proj_stride + (int64_t)h * vdim), 0,
+                                                            (uint32_t)(min(kBlock, rows - at) - 1) * pitch + (uint32_t)vdim * 2u, 0x00020000);
+      const uint32_t g_first = out_c < vdim ? (uint32_t)(kBlock / kWaves * wave) * pitch + (uint32_t)out_c * 2u : 0x80000000u;
+#pragma unroll
+      for (int i = 0; i < kBlock / kWaves; ++i)
+        gr[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(g_rows, g_first + (uint32_t)i * pitch, 0, 0));
+    }
     if (at + kBlock < rows) fetch(at + kBlock);     // the next block's rows, on their way during this one
+
+    // kOut: what the normaliser and n take of this block before the scores are there
+    constexpr int kPer = kThreads / kBlock;         // threads per row
+    const int n_t = tid / kPer, n_x = tid % kPer;   // this thread's row, its share of it
+    float nq = 0.f;
+    auto n_dot = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < DIMP / (8 * kPer); ++i) {
+        const int d = 8 * (n_x + kPer * i);
+        const uint4 q4 = *reinterpret_cast<const uint4*>(&qs[n_t * kQRow + d]);
+        const float4 n0 = *reinterpret_cast<const float4*>(&n_lds[d]), n1 = *reinterpret_cast<const float4*>(&n_lds[d + 4]);
+        const uint32_t w[4] = {q4.x, q4.y, q4.z, q4.w};
+        const float nn[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          nq = fmaf(lo_to_float<bf16_t>(w[e]), nn[2 * e], nq);
+          nq = fmaf(hi_to_float<bf16_t>(w[e]), nn[2 * e + 1], nq);
+        }
+      }
+      nq *= sc_in[n_t];
+    };
+    auto den_of = [&]() __attribute__((always_inline)) {       // the row's normaliser, in the row's first thread
+      float sum = 0.f;
+      for (int x = 8 * n_x; x <= n_t; x += 8 * kPer) {
+        const uint4 h4 = *reinterpret_cast<const uint4*>(&ph[n_t * kPRow + x]), l4 = *reinterpret_cast<const uint4*>(&pl[n_t * kPRow + x]);
+        const uint32_t wh[4] = {h4.x, h4.y, h4.z, h4.w}, wl[4] = {l4.x, l4.y, l4.z, l4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          sum += (lo_to_float<bf16_t>(wh[e]) + lo_to_float<bf16_t>(wl[e])) + (hi_to_float<bf16_t>(wh[e]) + hi_to_float<bf16_t>(wl[e]));
+      }
+      nq += sum;
+      // over the row's two, four or eight lanes
+      auto moved = [&](auto CTRL) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(nq), decltype(CTRL)::value, 0xf, 0xf, false)); };
+      nq += moved(std::integral_constant<int, 0xB1>{});
+      if constexpr (kPer >= 4) nq += moved(std::integral_constant<int, 0x4E>{});
+      if constexpr (kPer >= 8) nq += moved(std::integral_constant<int, 0x141>{});
+      static_assert(kPer <= 8, "eight threads per row at most");
+      return fmaxf(fabsf(nq), sc_floor[n_t]) + a.floor;
+    };
+    constexpr int kPairs = DIMP / 2, kShares = kThreads / kPairs > 0 ? kThreads / kPairs : 1;
+    auto n_shares = [&]() __attribute__((always_inline)) {     // thread: one pair of dims, one share of the rows
+      static_assert(kPairs <= kThreads, "one pair of dims per thread");
+      const int pair = tid % kPairs, share = tid / kPairs;
+      float x0 = 0.f, x1 = 0.f;
+#pragma unroll 8
+      for (int i = 0; i < kBlock / kShares; ++i) {
+        const int t = share + i * kShares;
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(&ks[t * kQRow + 2 * pair]);
+        x0 = fmaf(sc_w[t], lo_to_float<bf16_t>(w), x0);
+        x1 = fmaf(sc_w[t], hi_to_float<bf16_t>(w), x1);
+      }
+      n_part[2 * (share * kPairs + pair)] = x0;
+      n_part[2 * (share * kPairs + pair) + 1] = x1;
+    };
+    auto n_update = [&]() __attribute__((always_inline)) {
+      for (int d = tid; d < DIMP; d += kThreads) {
+        float x = 0.f;
+#pragma unroll
+        for (int i = 0; i < kShares; ++i) x += n_part[2 * (i * kPairs) + d];
+        n_lds[d] = fmaf(decay, n_lds[d], x);
+      }
+    };
+    if constexpr (kOut) {
+      n_dot();
+      n_shares();
+    }
 
     v16f o[2];
     if constexpr (!kStateOnly) {
-      // ---- weighted scores: the three 32 x 32 quarters at and below the diagonal ----
-      static_for<3>([&](auto Q) {
+      // ---- weighted scores: the ten 16 x 16 tiles at and below the diagonal ----
+      if constexpr (kOut) {
+        const int g4 = 4 * (lane >> 4);
+        for (int t16 = wave; t16 < 10; t16 += kWaves) {
+          const int rt = t16 < 1 ? 0 : t16 < 3 ? 1 : t16 < 6 ? 2 : 3, ct = t16 - rt * (rt + 1) / 2;
+          const uint16_t* qp = &qs[(16 * rt + i16) * kQRow + 2 * g4];
+          const uint16_t* kp = &ks[(16 * ct + i16) * kQRow + 2 * g4];
+          v4f p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int st = 0; st < DIMP / 32; ++st)
+            p = mfma16x16x32<bf16_t>(*reinterpret_cast<const uint4*>(qp + 32 * st), *reinterpret_cast<const uint4*>(kp + 32 * st), p);
+          // key column sx of the lane, rows 16 rt + g4 + r; past the diagonal the weight is exp(-inf)
+          const int sx = 16 * ct + i16, t0 = 16 * rt + g4;
+          const float as = sc_a[sx];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            constexpr float kNever = -INFINITY;
+            const float x = p[r] * (a.q_scale * __expf(sx > t0 + r ? kNever : as - sc_M[t0 + r]));
+            const bf16_t top = from_float<bf16_t>(x);
+            ph[(t0 + r) * kPRow + sx] = top.bits;
+            pl[(t0 + r) * kPRow + sx] = from_float<bf16_t>(x - to_float(top)).bits;
+          }
+        }
+      }
+      // ... or the three 32 x 32 quarters
+      if constexpr (!kOut) static_for<3>([&](auto Q) {
         constexpr int quarter = decltype(Q)::value;
         if (quarter % kWaves != wave) return;
         constexpr int rt = quarter == 0 ? 0 : 1, ct = quarter == 2 ? 1 : 0;
@@ -302,7 +435,7 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[rt][r] *= sc_in[32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3)] * a.q_scale;
+        for (int r = 0; r < 16; ++r) o[rt][r] *= sc_in[32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3)];
     }
     __builtin_amdgcn_sched_barrier(0);
     // this wave's 64 x 32 values as operand fragments (k-slot order as above)
@@ -330,6 +463,16 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
           o[rt] = mfma32x32x16<bf16_t>(make_uint4(l0.x, l0.y, l1.x, l1.y), vf[st], o[rt]);
           __builtin_amdgcn_sched_barrier(0);
         }
+      if constexpr (kOut) {
+        float* p = &os[4 * hi * kORow + 32 * wave + l32];
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) p[(32 * rt + 8 * (r >> 2) + (r & 3)) * kORow] = o[rt][r];
+        const float den = den_of();
+        if (n_x == 0) sc_den[n_t] = den;
+        n_update();
+      }
     }
     // ---- the state behind the block ----
     Split8 wv[4];
@@ -361,56 +504,17 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
       __builtin_amdgcn_sched_barrier(0);
     });
     // ---- normaliser and n: the head's first workgroup ----
-    if constexpr (kGates) if (n_owner) {
+    if constexpr (kGates && !kOut) if (n_owner) {
       if constexpr (!kStateOnly) {
-        constexpr int kPer = kThreads / kBlock;     // threads per row: 2 or 4
-        const int t = tid / kPer, part = tid % kPer;
-        float nq = 0.f, sum = 0.f;
-        for (int d = 8 * part; d < DIMP; d += 8 * kPer) {
-          const uint4 q4 = *reinterpret_cast<const uint4*>(&qs[t * kQRow + d]);
-          const uint32_t w[4] = {q4.x, q4.y, q4.z, q4.w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            nq = fmaf(lo_to_float<bf16_t>(w[e]), n_lds[d + 2 * e], nq);
-            nq = fmaf(hi_to_float<bf16_t>(w[e]), n_lds[d + 2 * e + 1], nq);
-          }
-        }
-        nq *= sc_in[t] * a.q_scale;
-        for (int x = 8 * part; x <= t; x += 8 * kPer) {
-          const uint4 h4 = *reinterpret_cast<const uint4*>(&ph[t * kPRow + x]), l4 = *reinterpret_cast<const uint4*>(&pl[t * kPRow + x]);
-          const uint32_t wh[4] = {h4.x, h4.y, h4.z, h4.w}, wl[4] = {l4.x, l4.y, l4.z, l4.w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            sum += (lo_to_float<bf16_t>(wh[e]) + lo_to_float<bf16_t>(wl[e])) + (hi_to_float<bf16_t>(wh[e]) + hi_to_float<bf16_t>(wl[e]));
-        }
-        nq += sum;
-#pragma unroll
-        for (int x = 1; x < kPer; x <<= 1) nq += __shfl_xor(nq, x, 64);
-        if (part == 0 && at + t < rows) a.den[(int64_t)(row0 + at + t) * H + h] = fmaxf(fabsf(nq), sc_floor[t]) + a.floor;
+        n_dot();
+        const float den = den_of();
+        if (n_x == 0 && at + n_t < rows) a.den[(int64_t)(row0 + at + n_t) * H + h] = den;
       }
-      // thread: one pair of dims, one share of the rows
-      constexpr int kPairs = DIMP / 2, kShares = kThreads / kPairs > 0 ? kThreads / kPairs : 1, kSweeps = (kPairs + kThreads - 1) / kThreads;
-#pragma unroll
-      for (int sw = 0; sw < kSweeps; ++sw) {
-        const int pair = (tid + sw * kThreads) % kPairs, share = kSweeps > 1 ? 0 : tid / kPairs;
-        float x0 = 0.f, x1 = 0.f;
-        for (int t = share; t < kBlock; t += kShares) {
-          const uint32_t w = *reinterpret_cast<const uint32_t*>(&ks[t * kQRow + 2 * pair]);
-          x0 = fmaf(sc_w[t], lo_to_float<bf16_t>(w), x0);
-          x1 = fmaf(sc_w[t], hi_to_float<bf16_t>(w), x1);
-        }
-        n_part[2 * (share * kPairs + pair)] = x0;
-        n_part[2 * (share * kPairs + pair) + 1] = x1;
-        static_assert(kSweeps == 1, "one pair of dims per thread");
-      }
+      n_shares();
       __syncthreads();                              // n has been read, the shares are there (uniform: the whole workgroup)
-      for (int d = tid; d < DIMP; d += kThreads) {
-        float x = 0.f;
-        for (int i = 0; i < kShares; ++i) x += n_part[2 * (i * kPairs) + d];
-        n_lds[d] = fmaf(decay, n_lds[d], x);
-      }
+      n_update();
     }
-    if constexpr (!kStateOnly) {
+    if constexpr (!kStateOnly && !kOut) {
       // bounds-checked stores: rows past the segment and columns past vdim are dropped
       uint32_t pitch = (uint32_t)(H * vdim) * 4u;
       asm volatile("" : "+s"(pitch));
@@ -426,6 +530,31 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[rt][r]), rsrc, voff + (uint32_t)(32 * rt + 8 * (r >> 2) + (r & 3)) * pitch, 0, 2 /* nt */);
     }
     __syncthreads();                                // everybody is done with this block's LDS
+    if constexpr (kOut) {                           // (os and sc_den are next written behind two more barriers)
+      const float inv_vdim = 1.0f / (float)vdim;
+      const int first = kBlock / kWaves * wave;
+      // bounds-checked stores: rows past the segment and columns past vdim are dropped, but their sums are taken with the others
+      uint32_t pitch = (uint32_t)(H * vdim) * 2u;
+      asm volatile("" : "+s"(pitch));
+      const auto out = __builtin_amdgcn_make_buffer_rsrc(a.out + ((int64_t)(row0 + at) * H + h) * vdim, 0,
+                                                         (uint32_t)(min(kBlock, rows - at) - 1) * pitch + (uint32_t)vdim * 2u, 0x00020000);
+      const uint32_t out_first = out_c < vdim ? (uint32_t)first * pitch + (uint32_t)out_c * 2u : 0x80000000u;
+#pragma unroll
+      for (int i = 0; i < kBlock / kWaves; ++i) {
+        const float inv_den = __builtin_amdgcn_rcpf(sc_den[first + i]);
+        const float4 num = *reinterpret_cast<const float4*>(&os[(first + i) * kORow + out_c]);
+        const float x[4] = {num.x * inv_den, num.y * inv_den, num.z * inv_den, num.w * inv_den};
+        const float ss = four_rows_sum(row16_sum(x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3]));
+        const float sc = __builtin_amdgcn_rsqf(ss * inv_vdim + a.eps);
+        const float y[4] = {x[0] * sc * out_w.x, x[1] * sc * out_w.y, x[2] * sc * out_w.z, x[3] * sc * out_w.w};
+        const float z[4] = {lo_to_float<bf16_t>(gr[i].x), hi_to_float<bf16_t>(gr[i].x), lo_to_float<bf16_t>(gr[i].y), hi_to_float<bf16_t>(gr[i].y)};
+        float o4[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o4[e] = y[e] * __builtin_amdgcn_rcpf(1.0f + __expf(-z[e]));
+        const uint2 packed = make_uint2(pack2<bf16_t>(o4[0], o4[1]), pack2<bf16_t>(o4[2], o4[3]));
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, packed), out, out_first + (uint32_t)i * pitch, 0, 2 /* nt */);
+      }
+    }
   }
 
   // ---- the state behind the segment: contribution -> workspace (kStateOnly), the last one -> the slot ----
@@ -448,6 +577,8 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
       if constexpr (kStateOnly) {
         a.ws_m[(int64_t)seg * H + h] = m;
         a.ws_f[(int64_t)seg * H + h] = f_total;
+      } else if constexpr (kOut) {
+        a.m_out[(int64_t)slot * H + h] = m;         // (who else of this head reads the old one has ended: the kernels before)
       } else {
         a.m_next[(int64_t)entry * H + h] = m;
       }
@@ -531,12 +662,12 @@ static __global__ __launch_bounds__(64) void memory_combine_max_kernel(const Mem
   }
 }
 
-template <int DIMP, int kWaves, bool kGates>
+template <int DIMP, int kWaves, bool kGates, bool kOut>
 static int launch_chunked(const MemoryChunkArgs& a, bool split, hipStream_t s) {
   const dim3 grid((unsigned)a.num_segments, (unsigned)a.heads, (unsigned)((a.vdim + 32 * kWaves - 1) / (32 * kWaves)));
   const dim3 block(64 * kWaves);
   if (split) {
-    memory_chunk_kernel<DIMP, kWaves, true, kGates><<<grid, block, 0, s>>>(a);
+    memory_chunk_kernel<DIMP, kWaves, true, kGates, false><<<grid, block, 0, s>>>(a);
     int status = launch_status();
     if (status != 0) return status;
     const int slices = (a.dim * a.vdim + (kGates ? a.dim : 0) + kCombineElements - 1) / kCombineElements;
@@ -547,20 +678,21 @@ static int launch_chunked(const MemoryChunkArgs& a, bool split, hipStream_t s) {
     status = launch_status();
     if (status != 0) return status;
   }
-  memory_chunk_kernel<DIMP, kWaves, false, kGates><<<grid, block, 0, s>>>(a);
+  if constexpr (kOut) memory_chunk_kernel<DIMP, 8, false, true, true><<<dim3(grid.x, grid.y), dim3(512), 0, s>>>(a);
+  else memory_chunk_kernel<DIMP, kWaves, false, kGates, false><<<grid, block, 0, s>>>(a);
   return launch_status();
 }
 
 template <bool kGates>
 static int launch_chunked_sizes(const MemoryChunkArgs& a, bool split, hipStream_t s) {
   if (a.vdim <= 64) {
-    if (a.dim <= 64) return launch_chunked<64, 2, kGates>(a, split, s);
-    if (a.dim <= 128) return launch_chunked<128, 2, kGates>(a, split, s);
-    return launch_chunked<256, 2, kGates>(a, split, s);
+    if (a.dim <= 64) return launch_chunked<64, 2, kGates, false>(a, split, s);
+    if (a.dim <= 128) return launch_chunked<128, 2, kGates, false>(a, split, s);
+    return launch_chunked<256, 2, kGates, false>(a, split, s);
   }
-  if (a.dim <= 64) return launch_chunked<64, 4, kGates>(a, split, s);
-  if (a.dim <= 128) return launch_chunked<128, 4, kGates>(a, split, s);
-  return launch_chunked<256, 4, kGates>(a, split, s);
+  if (a.dim <= 64) return launch_chunked<64, 4, kGates, false>(a, split, s);
+  if (a.dim <= 128) return launch_chunked<128, 4, kGates, false>(a, split, s);
+  return launch_chunked<256, 4, kGates, false>(a, split, s);
 }
 
 }  // namespace mvllm

@@ -90,7 +90,8 @@ class RaggedStep:
     state_slots: torch.Tensor                         # int32 [entries]
     windows: list = field(default_factory=list)       # WindowStep (LatentStep, RingStep) per window
     multi_rows: int = 0                               # rows of entries with more than one token
-    num_short: int = 0                                # entries below LONG_ROWS (the first ones)
+    num_short: int = 0                                # entries below LONG_ROWS (the first ones) ...
+    short_rows: Optional[int] = None                  # ... and their rows
     segments: Optional[torch.Tensor] = None           # int32 [n, 4] of long entries: entry, first row, rows, flags
     split: bool = False                               # some long entry has more than one segment
     order: list = field(default_factory=list)         # entry e of the packing is sequence order[e] of the caller
@@ -100,7 +101,10 @@ class RaggedStep:
 
 BLOCK_ROWS = 64                # rows per block of a recurrence's block form: segments are whole blocks
 FILL_WORKGROUPS = 512          # segments are made shorter until there are this many workgroups ...
-MIN_SEGMENT_ROWS = 256         # ... but not shorter than this
+# ... but not shorter than this, and portions below two of them stay whole: the states' own pass, two launches and their way through
+# memory have to pay.  One portion of 700 rows, 16 heads of 128 x 256: 43 us (256: 55, 64: 40), 2000 rows, 8 heads: 50 (60, 57), 200
+# rows in two segments 36 against 31 whole.
+MIN_SEGMENT_ROWS = 128
 
 
 def _segments(lens, cu, units):
@@ -113,7 +117,7 @@ def _segments(lens, cu, units):
     out = []
     for e in long_entries:
         n, at = int(lens[e]), int(cu[e])
-        pieces = max(-(-n // length), 1)
+        pieces = max(-(-n // length), 1) if n >= 2 * MIN_SEGMENT_ROWS else 1
         size = -(-n // (pieces * BLOCK_ROWS)) * BLOCK_ROWS
         cuts = list(range(0, n, size)) + [n]
         for i, (lo, hi) in enumerate(zip(cuts, cuts[1:])):
@@ -295,7 +299,7 @@ def ragged_arrays(seqs, windows, block_size, memory_units=0, latent=False):
     if segments:
         arrays["segments"] = np.asarray(segments, dtype=np.int32)
     facts = dict(num_tokens=int(cu[-1]), num_entries=len(items), num_single=singles, multi_rows=int(cu[-1]) - singles,
-                 num_short=num_short, split=any(not s[3] & 4 for s in segments), order=order, starts=starts)
+                 num_short=num_short, short_rows=int(cu[num_short]), split=any(not s[3] & 4 for s in segments), order=order, starts=starts)
     return arrays, [a for a, _ in per_window], [c for _, c in per_window], facts
 
 

@@ -57,6 +57,17 @@ def chunked_takes(proj: torch.Tensor, dim: int, vdim: int) -> bool:
             and proj.shape[1] % 8 == 0 and (proj.shape[0] == 1 or proj.stride(0) % 8 == 0))
 
 
+def chunked_output_takes(segments: int, rows: int, heads: int, dim: int, vdim: int, gate: int, weight: torch.Tensor) -> bool:
+    """Whether ``rows`` of long entries in ``segments`` go through the norm and the output gate in the block form's own pass.
+
+    A workgroup holds all columns of a head, so heads up to 128 x 256, but not those up to 128 columns, of which half its waves
+    would have none.  It takes longer per block of rows than two workgroups of the other form (9.5 us against 8), which have twice as
+    many CUs while there are few of them, and saves a launch and the sums' way through memory.  Heads of 128 x 256: 64 segments of
+    200 rows and heads 40 us against 36, 128 of them 44 against 48, 8 x 16 of 1024 rows 145 against 159, 32 of 100 rows 21 against 25."""
+    fits = dim <= 128 and 128 < vdim <= 256 and gate % 8 == 0 and weight.data_ptr() % 16 == 0
+    return fits and (segments * heads >= 96 or rows <= 128 * segments)
+
+
 def mlstm(step, proj: torch.Tensor, gates: torch.Tensor, gate_col: int, weight: torch.Tensor, state: MlstmState,
           eps: float) -> torch.Tensor:
     """The mLSTM mixer between its projections: (T, H * vdim) = rms(recurrence) * weight * sigmoid(gate).
@@ -77,29 +88,39 @@ def mlstm(step, proj: torch.Tensor, gates: torch.Tensor, gate_col: int, weight: 
     dev, code = proj.device, _C.dtype_code(proj.dtype)
     stream = _C.current_stream_ptr(dev)
     stride = proj.stride(0) if rows > 1 else proj.shape[1]
-    num = torch.empty((rows, heads, vdim), dtype=torch.float32, device=dev)
-    den = torch.empty((rows, heads), dtype=torch.float32, device=dev)
-    m_next = torch.empty((step.num_entries, heads), dtype=torch.float32, device=dev)
     out = torch.empty((rows, heads * vdim), dtype=proj.dtype, device=dev)
+    gate = proj.data_ptr() + gate_col * proj.element_size()
     lib = _C.load()
     scale = dim ** -0.5
-    common = (_ptr(num), _ptr(den), _ptr(m_next), _ptr(proj), stride, _ptr(gates), _ptr(state.s), _ptr(state.n), _ptr(state.m),
-              _ptr(step.cu_seqlens), _ptr(step.state_slots), _ptr(step.positions))
     blocks = step.segments is not None and chunked_takes(proj, dim, vdim)
-    row_by_row = step.num_short if blocks else step.num_entries
-    if row_by_row:
-        _C.check(lib.mvllm_mlstm_recurrent(*common, row_by_row, heads, dim, vdim, scale, DEN_FLOOR, code, stream),
-                 "mlstm_recurrent")
+    # rows of long entries straight to their outputs
+    whole = blocks and step.short_rows is not None and \
+        chunked_output_takes(step.segments.shape[0], rows - step.short_rows, heads, dim, vdim, gate, weight)
+    plain = step.short_rows if whole else rows                # rows whose norm and gate are a pass of their own
+    state_of = (_ptr(state.s), _ptr(state.n), _ptr(state.m), _ptr(step.cu_seqlens), _ptr(step.state_slots), _ptr(step.positions))
+    if plain:
+        num = torch.empty((plain, heads, vdim), dtype=torch.float32, device=dev)
+        den = torch.empty((plain, heads), dtype=torch.float32, device=dev)
+        m_next = torch.empty((step.num_entries, heads), dtype=torch.float32, device=dev)
+        common = (_ptr(num), _ptr(den), _ptr(m_next), _ptr(proj), stride, _ptr(gates), *state_of)
+        row_by_row = step.num_short if blocks else step.num_entries
+        if row_by_row:
+            _C.check(lib.mvllm_mlstm_recurrent(*common, row_by_row, heads, dim, vdim, scale, DEN_FLOOR, code, stream),
+                     "mlstm_recurrent")
     if blocks:
         count = step.segments.shape[0]
         nbytes = lib.mvllm_mlstm_chunked_workspace_bytes(count, heads, dim, vdim) if step.split else 0
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
-        _C.check(lib.mvllm_mlstm_chunked(*common, _ptr(step.segments), count, int(step.split), heads, dim, vdim, scale,
-                                         DEN_FLOOR, code, _ptr(ws), nbytes, stream), "mlstm_chunked")
-    _C.check(lib.mvllm_mlstm_output(
-        _ptr(out), _ptr(num), _ptr(den), _ptr(weight), proj.data_ptr() + gate_col * proj.element_size(), stride, float(eps),
-        _ptr(m_next), _ptr(state.m), _ptr(step.cu_seqlens), _ptr(step.row_entry), _ptr(step.state_slots), rows, heads, vdim,
-        code, stream), "mlstm_output")
+        tail = (_ptr(step.segments), count, int(step.split), heads, dim, vdim, scale, DEN_FLOOR, code, _ptr(ws), nbytes, stream)
+        if whole:
+            _C.check(lib.mvllm_mlstm_chunked_output(_ptr(out), _ptr(weight), gate, float(eps), _ptr(proj), stride, _ptr(gates),
+                                                    *state_of, *tail), "mlstm_chunked_output")
+        else:
+            _C.check(lib.mvllm_mlstm_chunked(*common, *tail), "mlstm_chunked")
+    if plain:
+        _C.check(lib.mvllm_mlstm_output(
+            _ptr(out), _ptr(num), _ptr(den), _ptr(weight), gate, stride, float(eps), _ptr(m_next), _ptr(state.m),
+            _ptr(step.cu_seqlens), _ptr(step.row_entry), _ptr(step.state_slots), plain, heads, vdim, code, stream), "mlstm_output")
     return out
 
 

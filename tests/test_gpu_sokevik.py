@@ -458,6 +458,15 @@ def test_mlstm_segments_side_by_side(monkeypatch, heads, dim, vdim):
         assert rel(torch.cat(outs[i]), want) < 4e-3, i
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 256), (3, 24, 136), (1, 64, 200), (2, 72, 144)])
+def test_mlstm_whole_heads(monkeypatch, heads, dim, vdim):
+    """Heads whose norm and gate belong to the block form: the largest, odd numbers of columns and dims; whole blocks, one row past
+    them, portions behind others, next to short entries, in segments side by side.  The other form's tolerances."""
+    for cuts in ([300], [64, 65, 128, 43], [1, 33, 20, 246]):
+        test_mlstm_portions(torch.bfloat16, heads, dim, vdim, cuts)
+    test_mlstm_segments_side_by_side(monkeypatch, heads, dim, vdim)
+
+
 # ---- the model ----
 _runners: dict = {}
 
