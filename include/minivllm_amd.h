@@ -303,6 +303,24 @@ int mvllm_prefill_paged_int8_split(void* out, const void* q,
                                    void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * mvllm_prefill_varlen (block_size 0; block_tables, cu_seqlens_k NULL, k and v packed) or mvllm_prefill_paged with the keys of every
+ * row tile cut into ranges of `range_tiles` tiles of 64 (an even number), walked side by side: 16-bit element types, head_dim 64 and
+ * 128, block_size a multiple of 16, up to 64 sequences.  Partial results are fp32.  sink: fp32 [Hq] or NULL.
+ *   _ranges_plan: the range the library would use for a batch of these sizes; 0 = run the calls above.
+ *   _ranges_workspace_bytes: 16-byte aligned device memory the call needs.
+ * max_kv_len: the host's upper bound of every sequence's key count (keys past it are walked by the last range).
+ */
+int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads,
+                              int head_dim, int block_size, int dtype);
+size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim,
+                                            int range_tiles);
+int mvllm_prefill_ranges(void* out, const void* q, const void* k, const void* v, const int32_t* block_tables,
+                         int max_num_blocks, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int num_seqs,
+                         int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads, int head_dim, int block_size,
+                         int64_t num_blocks, float scale, const float* sink, int dtype, int range_tiles, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
+/*
  * The caller's per-layer chain between the QKV projection and the attention kernels, fused:
  *   q = rms_norm(q); k = rms_norm(k)      src/myvllm/models/qwen3.py:104-106, layers/layernorm.py:9-17
  *   q, k = rotary_emb(positions, q, k)    qwen3.py:108, layers/rotary_embedding.py:4-23, 77-83

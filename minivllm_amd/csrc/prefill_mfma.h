@@ -44,6 +44,11 @@ struct PrefillArgs {
   int64_t q_period = 0;
   const float* sink = nullptr;   // optional, [num_heads]: one more exp(sink) in a row's denominator (not with lse: the merge adds it)
   int band_shift = 0;   // MFMA path: log2 of the row tiles per band of the item order (locate_banded)
+  // Key ranges (prefill_ranges.hip): workgroup y walks the key tiles [y range_tiles, (y + 1) range_tiles) of its rows, the last one all
+  // that are left; a row tile with several writes their results here, fp32 [ranges, total_tokens, num_heads, head_dim], with lse
+  // [ranges, total_tokens, num_heads] as above (-inf: no keys), others go straight to out.
+  int range_tiles = 0;
+  float* part = nullptr;
 };
 
 constexpr unsigned kXcdChunk = 32;      // consecutive work items handed to one XCD
@@ -150,9 +155,11 @@ __device__ __forceinline__ bool locate_banded(const int32_t* __restrict__ cu, in
 // follows the head in memory (the next head, the next token, zeros past the descriptor's end); the first product runs
 // over ceil(DD / 16) steps and never reads them (kHalfStep below: the last step of DD = 16 n + 8), the second one
 // carries them through the output columns DD .. 32 ceil(DD / 32) - 1 of its last block, which are not stored.
-template <typename T, int HPW, bool PAGED, int D, bool I8 = false, int DD = D>
+// RANGES: see PrefillArgs::range_tiles; head_dim 64 and 128, 16-bit keys and values.
+template <typename T, int HPW, bool PAGED, int D, bool I8 = false, int DD = D, bool RANGES = false>
 __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_kernel(const PrefillArgs a) {
   static_assert(!I8 || PAGED, "INT8 caches are paged");
+  static_assert(!RANGES || (!I8 && DD == D && D <= 128), "key ranges: plain layouts");
   static_assert(DD % 8 == 0 && DD <= D && (!I8 || DD == D), "head dims in steps of 8, INT8 only at 64 and 128");
   constexpr int kRowB = D * 2;                  // bytes per tile row
   constexpr int kChunks = kRowB / 16;           // 16-byte chunks per row: 16 or 8
@@ -189,7 +196,13 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   const unsigned round = slot / kXcdChunk;
   const unsigned item = (round * 8 + ((xcd + round) & 7)) * kXcdChunk + slot % kXcdChunk;
   int item_y, seq_start, seq_len, row0, seq_index;
-  if (a.num_seqs <= 64) {
+  if constexpr (RANGES) {
+    // slices fastest: with a multiple of eight of them all that reads the keys of one is on one XCD; nothing is padded, which would
+    // count once per range (in the other order 195 rows behind 3700 keys in 11 ranges took 92 us, 4000 workgroups without work among them;
+    // in this one 37)
+    item_y = (int)(id % (unsigned)a.heads_y);
+    if (!locate_tile(a.cu_seqlens, a.num_seqs, tiles_x - 1 - (int)(id / (unsigned)a.heads_y), BM, seq_start, seq_len, row0, seq_index)) return;
+  } else if (a.num_seqs <= 64) {
     if (!locate_banded<BM>(a.cu_seqlens, a.num_seqs, item, a.heads_y, a.band_bits, a.band_shift, seq_start, seq_len, row0, seq_index, item_y)) return;
   } else {
     // more sequences than one wave holds: memory order, inside a sequence the latest (heaviest) tiles first
@@ -221,10 +234,19 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   const bool active = r0 < seq_len;
   const int pos0 = cached + r0;                      // position of that row among the keys
   // tiles every row of the wave sees completely (a row sees keys up to its position, and never past the last key)
-  const int n_full = min((pos0 + 1) / kBN, kv_len / kBN);
-  const int j_last = min(pos0 + kWaveRows - 1, kv_len - 1) / kBN;   // last tile any row of the wave sees
+  int n_full = min((pos0 + 1) / kBN, kv_len / kBN);
+  int j_last = min(pos0 + kWaveRows - 1, kv_len - 1) / kBN;         // last tile any row of the wave sees
   const int wg_last = min(row0 + BM, seq_len) - 1;
-  const int ntiles = min((cached + wg_last) / kBN, (kv_len - 1) / kBN) + 1;
+  int ntiles = min((cached + wg_last) / kBN, (kv_len - 1) / kBN) + 1;
+  // RANGES: this workgroup's tiles are [t0, ntiles), t0 even (tile j lies in buffer j % 2); the others belong to other workgroups
+  const int t0 = RANGES ? (int)blockIdx.y * a.range_tiles : 0;
+  const bool in_ranges = RANGES && gridDim.y > 1 && ntiles > a.range_tiles;      // (one range: no partial results, whatever the bound)
+  if constexpr (RANGES) {
+    if (t0 >= ntiles) return;
+    if (blockIdx.y + 1 < gridDim.y) ntiles = min(ntiles, t0 + a.range_tiles);
+    n_full = min(n_full, ntiles);
+    j_last = min(j_last, ntiles - 1);
+  }
   const int l32 = lane & 31;
   const int hi = lane >> 5;                          // 0/1: which half of the k-slots / rows
   const int qrow = r0 + l32;                         // query row of this lane
@@ -276,11 +298,11 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   const int rows_4g = (int)(0xffffffffu / (uint32_t)row_bytes);   // rows whose bytes no longer fit 32 bits
   const int bs = PAGED ? a.block_size : 1;
   const int32_t* table = PAGED ? a.block_tables + (int64_t)seq_index * a.max_num_blocks : nullptr;
-  int pg_pos = ROWS_PER_WAVE * wave;                 // key position of this wave's piece in the next tile asked for
+  int pg_pos = ROWS_PER_WAVE * wave + t0 * kBN;      // key position of this wave's piece in the next tile asked for
   int pg_bi = pg_pos / bs, pg_off = pg_pos - pg_bi * bs;
-  int win_base = 0;
+  int win_base = RANGES ? pg_bi : 0;
   int win = -1;
-  if (PAGED) win = lane < a.max_num_blocks ? table[lane] : -1;
+  if (PAGED) win = win_base + lane < a.max_num_blocks ? table[win_base + lane] : -1;
   auto tile_src = [&](int j, bool enable) {
     TileSrc t;
     if constexpr (PAGED) {
@@ -378,7 +400,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   };
   Scales sc_cur = {0.f, 0.f};
   if constexpr (I8) sc_cur = issue_codes(0, true);
-  else issue_tile(0, 0);
+  else issue_tile(t0, 0);
 
   // Q fragments (B operand): column = query row l32, k = 16*ks + 8*hi ..
   uint4 qf[kKS];
@@ -564,7 +586,8 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
     // head_dim 256: marked unlikely, so that the rescale sits out of line and the register allocator does not plan the
     // tile loop around it (for the other head dims the hint only moves blocks about: measured, no gain)
     if (D == 256 ? __builtin_expect(__any(grow), 0) : __any(grow)) {
-      const float d = grow ? mx : 0.f;                 // the running maximum moves up by d (any finite d on the first tile)
+      // the running maximum moves up by d (any finite d on the first tile; a row may see no key of its range)
+      const float d = grow && !(RANGES && mx == -INFINITY) ? mx : 0.f;
       const float alpha = first ? 1.f : fast_exp2(-d); // nothing is accumulated yet on the first tile
       l *= alpha;
       if constexpr (D == 256) {
@@ -658,7 +681,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
     if (pos0 + kWaveRows - 1 < j * kBN + 32) tile_step(j, BUF, std::true_type{}, H1{}, j + 1 < ntiles);
     else tile_step(j, BUF, std::true_type{}, H2{}, j + 1 < ntiles);
   };
-  int j = 0;
+  int j = t0;
   if constexpr (I8) {
     // codes of tile j have landed and tile j - 1 is no longer read: send for tile j + 1, convert tile j
     auto stage = [&](int jj) {
@@ -711,12 +734,36 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   dma_wait_all();                                    // the zero fill issued during the last tile has landed
   __syncthreads();                                   // every wave is done reading K/V tiles
   if (!active) return;
+  if constexpr (RANGES) {
+    if (in_ranges) {
+      // the same in fp32: a wave's 32 rows of D * 4 bytes take a quarter of all buffers
+      constexpr int kRow32 = D * 4, kChunks32 = D / 4;
+      char* ot = &lds.k[0][0] + wave * (kWaveRows * kRow32);
+      const float lt = l + __shfl_xor(l, 32, 64);
+      const float inv = lt > 0.f ? 1.f / lt : 0.f;   // (no keys: a wave whose rows end before this range)
+      const int64_t part_row = (int64_t)blockIdx.y * a.total_tokens + seq_start + r0;
+      if (hi == 0 && qrow < seq_len) a.lse[(part_row + l32) * a.num_heads + h] = lt > 0.f ? __log2f(lt) - neg_m[0] : -INFINITY;
+#pragma unroll
+      for (int td = 0; td < kTD; ++td)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+          *reinterpret_cast<float4*>(ot + l32 * kRow32 + (((8 * td + 2 * r4 + hi) ^ (l32 & 15)) << 4)) =
+              make_float4(o[td][4 * r4] * inv, o[td][4 * r4 + 1] * inv, o[td][4 * r4 + 2] * inv, o[td][4 * r4 + 3] * inv);
+#pragma unroll
+      for (int i = 0; i < kWaveRows * kChunks32 / 64; ++i) {
+        const int row = (64 * i + lane) / kChunks32, c = lane % kChunks32;
+        const float4 w = *reinterpret_cast<const float4*>(ot + row * kRow32 + ((c ^ (row & 15)) << 4));
+        if (r0 + row < seq_len) *reinterpret_cast<float4*>(a.part + ((part_row + row) * a.num_heads + h) * D + 4 * c) = w;
+      }
+      return;
+    }
+  }
   char* ot = &lds.k[0][0] + wave * (kWaveRows * kRowB);   // 4 waves x 32 rows = both K buffers
   {
     float lt = l + __shfl_xor(l, 32, 64);
     if (a.sink != nullptr) lt = add_sink(lt, -neg_m[0], a.sink[h]);
     const float inv = 1.f / lt;
-    if (PAGED && a.lse != nullptr && hi == 0 && qrow < seq_len)
+    if (PAGED && !RANGES && a.lse != nullptr && hi == 0 && qrow < seq_len)
       a.lse[(int64_t)(seq_start + qrow) * a.num_heads + h] = __log2f(lt) - neg_m[0];
 #pragma unroll
     for (int td = 0; td < kTD; ++td)
@@ -741,8 +788,8 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
 }
 
 // D: the LDS layout (64, 128 or 256), DD: the data's head dimension.
-template <typename T, bool PAGED, bool I8, int D, int DD>
-static int launch_prefill_mfma_as(const PrefillArgs& a, hipStream_t stream) {
+template <typename T, bool PAGED, bool I8, int D, int DD, bool RANGES = false>
+static int launch_prefill_mfma_as(const PrefillArgs& a, hipStream_t stream, int ranges = 1) {
   const int group = a.num_heads / a.num_kv_heads;
   // query heads of a kv head per workgroup: 4 or 2 where they divide the group, else 1 (the workgroup is then four
   // row tiles of one head)
@@ -751,7 +798,7 @@ static int launch_prefill_mfma_as(const PrefillArgs& a, hipStream_t stream) {
   PrefillArgs b = a;
   // upper bound on the query tiles: every sequence may end with a partial tile; in the banded order (at most 64
   // sequences) every sequence may also end with a partial band of kBandRows / bm tiles
-  b.band_shift = band_shift_for(a.total_tokens, a.num_seqs, bm, PAGED);
+  b.band_shift = RANGES ? 0 : band_shift_for(a.total_tokens, a.num_seqs, bm, PAGED);
   b.tiles_x = a.num_seqs <= 64 ? (int)(a.total_tokens / bm + ((int64_t)a.num_seqs << b.band_shift))
                                : (int)(a.total_tokens / bm + a.num_seqs);
   b.heads_y = a.num_kv_heads * (group / hpw);
@@ -759,11 +806,11 @@ static int launch_prefill_mfma_as(const PrefillArgs& a, hipStream_t stream) {
   while (((int64_t)1 << b.band_bits) <= a.total_tokens / (bm << b.band_shift) + 1) ++b.band_bits;
   const int64_t items = (int64_t)b.tiles_x * b.heads_y;
   const int64_t span = 8 * (int64_t)kXcdChunk;
-  dim3 grid((unsigned)((items + span - 1) / span * span));
+  dim3 grid(RANGES ? (unsigned)items : (unsigned)((items + span - 1) / span * span), (unsigned)ranges);
   const dim3 block(64 * kPfWaves);
-  if (hpw == 4) prefill_mfma_kernel<T, 4, PAGED, D, I8, DD><<<grid, block, 0, stream>>>(b);
-  else if (hpw == 2) prefill_mfma_kernel<T, 2, PAGED, D, I8, DD><<<grid, block, 0, stream>>>(b);
-  else prefill_mfma_kernel<T, 1, PAGED, D, I8, DD><<<grid, block, 0, stream>>>(b);
+  if (hpw == 4) prefill_mfma_kernel<T, 4, PAGED, D, I8, DD, RANGES><<<grid, block, 0, stream>>>(b);
+  else if (hpw == 2) prefill_mfma_kernel<T, 2, PAGED, D, I8, DD, RANGES><<<grid, block, 0, stream>>>(b);
+  else prefill_mfma_kernel<T, 1, PAGED, D, I8, DD, RANGES><<<grid, block, 0, stream>>>(b);
   return launch_status();
 }
 template <typename T, bool PAGED, bool I8 = false>
@@ -776,6 +823,8 @@ static int launch_prefill_mfma(const PrefillArgs& a, hipStream_t stream) {
 int launch_prefill_paged_16bit(const PrefillArgs& a, int dtype, hipStream_t stream);
 // the paged form over an INT8 cache (codes + fp32 scales), head_dim 64 or 128, bf16 / fp16 queries (prefill_varlen.hip)
 int launch_prefill_paged_int8(const PrefillArgs& a, int dtype, hipStream_t stream);
+// key ranges side by side, head_dim 64 or 128, bf16 / fp16, packed or paged (prefill_ranges.hip)
+int launch_prefill_ranges(const PrefillArgs& a, int dtype, bool paged, int ranges, hipStream_t stream);
 // fp32 tensors, head_dim 128 or 64, packed or over a paged fp32 cache (prefill_f32.hip)
 int launch_prefill_f32(const PrefillArgs& a, bool paged, hipStream_t stream);
 // every other multiple of 8 from 32 to 120, and 256 (prefill_other_dims.hip, prefill_half_step_dims.hip); 16-bit element types only

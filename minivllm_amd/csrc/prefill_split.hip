@@ -164,6 +164,70 @@ __global__ __launch_bounds__(256) void split_merge_kernel(const MergeArgs a) {
   *reinterpret_cast<uint4*>(reinterpret_cast<T*>(a.out) + ((int64_t)t * a.num_heads + h) * a.head_dim + 8 * c) = o;
 }
 
+// The merge behind prefill_ranges.hip, with fp32 partial results: a wave merges one query row's heads, 256 / D of them at a time; rows
+// whose tile has one range are complete already.
+struct RangeMergeArgs {
+  void* out;               // [total_q, Hq, D]
+  const float* part;       // [ranges, total_q, Hq, D]
+  const float* lse;        // [ranges, total_q, Hq]
+  const int32_t* cu_seqlens_q;
+  const int32_t* cu_seqlens_k;   // null: packed
+  const float* sink;
+  int num_seqs, ranges, range_tiles, rows_per_tile, total_q, num_heads;
+};
+template <typename T, int D>
+__global__ __launch_bounds__(256) void range_merge_kernel(const RangeMergeArgs a) {
+  constexpr int kHeads = 256 / D, kLanes = D / 4;  // heads of a wave, lanes of a head
+  const int lane = threadIdx.x & 63, t = blockIdx.x;
+  // the row's sequence: at most 64 of them, one per lane
+  int lo = 0, end = 0x7fffffff;
+  if (lane < a.num_seqs) {
+    lo = a.cu_seqlens_q[lane];
+    end = a.cu_seqlens_q[lane + 1];
+  }
+  const int s = __popcll(__ballot(end <= t));
+  if (s >= a.num_seqs) return;                     // behind the last sequence
+  const int start = __builtin_amdgcn_readlane(lo, s), len = __builtin_amdgcn_readlane(end, s) - start;
+  const int kv = a.cu_seqlens_k ? a.cu_seqlens_k[s + 1] - a.cu_seqlens_k[s] : len, cached = max(kv - len, 0);
+  const int last = min((t - start) / a.rows_per_tile * a.rows_per_tile + a.rows_per_tile, len) - 1;
+  const int tiles = min((cached + last) / 64, (kv - 1) / 64) + 1;
+  if (tiles <= a.range_tiles) return;
+  const int n = min((tiles + a.range_tiles - 1) / a.range_tiles, a.ranges);
+  const int h = (blockIdx.y * 4 + (threadIdx.x >> 6)) * kHeads + lane / kLanes, c = 4 * (lane % kLanes);
+  if (h >= a.num_heads) return;
+  const int64_t at = (int64_t)t * a.num_heads + h, pitch = (int64_t)a.total_q * a.num_heads;
+  // the weights: a range per lane of the head's, then through LDS (a wave's own: no barrier)
+  __shared__ float weights[4 * kHeads][kMaxRanges];
+  float* w_of = weights[(threadIdx.x >> 6) * kHeads + lane / kLanes];
+  float lse[kMaxRanges / kLanes], top = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < kMaxRanges / kLanes; ++j) {
+    const int i = lane % kLanes + kLanes * j;
+    lse[j] = i < n ? a.lse[i * pitch + at] : -INFINITY;
+    top = fmaxf(top, lse[j]);
+  }
+#pragma unroll
+  for (int o = 1; o < kLanes; o <<= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
+#pragma unroll
+  for (int j = 0; j < kMaxRanges / kLanes; ++j) w_of[lane % kLanes + kLanes * j] = exp2f(lse[j] - top);
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  float den = 0.f;
+#pragma unroll 8
+  for (int i = 0; i < n; ++i) {
+    const float w = w_of[i];
+    const float4 p = *reinterpret_cast<const float4*>(a.part + (i * pitch + at) * D + c);
+    den += w;
+    acc.x = fmaf(w, p.x, acc.x);
+    acc.y = fmaf(w, p.y, acc.y);
+    acc.z = fmaf(w, p.z, acc.z);
+    acc.w = fmaf(w, p.w, acc.w);
+  }
+  if (a.sink != nullptr) den = add_sink(den, top, a.sink[h]);
+  const float inv = 1.f / den;
+  *reinterpret_cast<uint2*>(reinterpret_cast<T*>(a.out) + at * D + c) =
+      make_uint2(pack2<T>(acc.x * inv, acc.y * inv), pack2<T>(acc.z * inv, acc.w * inv));
+}
+
 int gcd_int(int x, int y) {
   while (y != 0) {
     const int r = x % y;
@@ -350,4 +414,108 @@ extern "C" int mvllm_prefill_paged_int8_split(void* out, const void* q, const in
   return run_split(out, q, k_cache, v_cache, k_scale, v_scale, true, block_tables, max_num_blocks, cu_seqlens_q, cu_seqlens_k,
                    num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, num_blocks, scale, nullptr, dtype,
                    splits, workspace, workspace_bytes, stream);
+}
+
+// ---- key ranges with their tables left where they are (prefill_ranges.hip) ----
+
+// shapes the form takes: prefill_kernel_for's LDS-tiled kernel at head_dim 64 and 128, 64 sequences at most
+static bool ranges_shape_ok(int num_seqs, int64_t total_q, int max_kv_len, int num_heads, int num_kv_heads, int head_dim, int block_size,
+                            int dtype) {
+  if (num_seqs <= 0 || num_seqs > 64 || total_q <= 0 || max_kv_len <= 0 || num_heads <= 0 || num_kv_heads <= 0 || block_size < 0) return false;
+  if (num_heads % num_kv_heads != 0 || num_heads > 65535 || (dtype != MVLLM_BF16 && dtype != MVLLM_F16)) return false;
+  if ((head_dim != 128 && head_dim != 64) || block_size % 16 != 0) return false;
+  if ((int64_t)block_size * num_kv_heads * head_dim * 2 >= ((int64_t)1 << 31) || (int64_t)num_kv_heads * head_dim * 2 * 64 >= ((int64_t)1 << 31)) return false;
+  return total_q <= ((int64_t)1 << 24);
+}
+static int rows_of_tile(int group) { return 32 * (group % 4 == 0 ? 1 : group % 2 == 0 ? 2 : 4); }
+static int ranges_of(int max_kv_len, int range_tiles) { return ((max_kv_len + 63) / 64 + range_tiles - 1) / range_tiles; }
+
+// The range for a batch of these sizes, at least every sequence's tiles where none is cut; 0: the other kernels.
+// Which kernel: the two-group kernel holds one workgroup per CU and runs faster once it has started (906 TFLOP/s against 680), but takes
+// 6 us longer until then, and its longest item decides when there are few.  So this form takes what fits on the chip about at once, two
+// workgroups per CU, four heads per workgroup (whose row tiles are half as long, and read the keys twice as often) somewhat less.  us on
+// either side, bf16, without the store: 16 heads over 8 kv heads of 128, two prompts of 270 rows 20.5 -> 14.5, one of 3000 67 -> 60, of 4000
+// (512 workgroups) 92 -> 82, ten of 406 (488) 32 -> 30, two of 2330 (592) 66 -> 68,
+// seven of 965 (900) 51 -> 56; 32 heads, one of 1500 (384) 38.6 -> 35.7, four of 875 (904) 42 -> 51.  At head_dim
+// 64 the other form is this kernel over its banded order, which pays for packed batches as soon as their tiles differ (3500 rows,
+// 448 workgroups: 30 us, here 33) and costs cached ones its padding (1000 rows behind as many 26 -> 24).
+// Which range: a tile takes a workgroup 0.9 us (0.8 at head_dim 64), workgroups of 0.6 of the longest sequence's tiles each fill 256 CUs;
+// a range brings every row's fp32 partial result into memory and back, about 0.7 of the ranges are there on average.  Batches of more
+// than 192 workgroups gain nothing that the partial results do not cost (1500 rows behind 1500, 32 heads, 376 workgroups: whole 72, two
+// ranges 86).  Measured, whole -> ranges: 343 rows behind 6500, 16 heads 64 -> 35; 870 behind 7800 50 -> 40; 132 behind 32768, 32
+// heads: 104, two-group kernel with split keys 155.
+extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads,
+                                         int head_dim, int block_size, int dtype) {
+  if (!ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype)) return 0;
+  const int group = num_heads / num_kv_heads, bm = rows_of_tile(group);
+  const int64_t wgs = (total_q_tokens / bm + num_seqs) * ((int64_t)num_heads * bm / 128), tiles = (max_kv_len + 63) / 64;
+  const int limit = head_dim == 64 ? (block_size > 0 ? 768 : tiles >= 16 ? 384 : 0) : group % 4 != 0 ? (tiles >= 16 ? 512 : 640) : tiles >= 12 ? 384 : 320;
+  if (wgs > limit) return 0;
+  int64_t p = (tiles + 1) / 2 * 2;
+  if (wgs > 192) return (int)p;
+  const float per_tile = head_dim == 64 ? 0.8f : 0.9f, per_range = 0.3f + 0.7f * 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f;
+  float best = 3.f;
+  for (int64_t x = 6; x < tiles; x += 2) {
+    const int64_t n = (tiles + x - 1) / x;
+    if (n > kMaxRanges) continue;
+    const float gain = per_tile * ((float)tiles - fmaxf((float)x, 0.6f * (float)(wgs * tiles) / 256.f)) - 4.f - per_range * (float)n;
+    if (gain > best) {
+      best = gain;
+      p = x;
+    }
+  }
+  return (int)p;
+}
+
+extern "C" size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim, int range_tiles) {
+  if (total_q_tokens <= 0 || max_kv_len <= 0 || num_heads <= 0 || head_dim <= 0 || range_tiles <= 0) return 0;
+  const int ranges = ranges_of(max_kv_len, range_tiles);
+  return ranges < 2 ? 0 : (size_t)ranges * total_q_tokens * num_heads * (head_dim + 1) * sizeof(float);
+}
+
+extern "C" int mvllm_prefill_ranges(void* out, const void* q, const void* k, const void* v, const int32_t* block_tables,
+                                    int max_num_blocks, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int num_seqs,
+                                    int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads, int head_dim, int block_size,
+                                    int64_t num_blocks, float scale, const float* sink, int dtype, int range_tiles, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  if (dtype_size(dtype) == 0) return MVLLM_ERR_BAD_DTYPE;
+  const bool paged = block_size > 0;
+  if (num_seqs < 0 || total_q_tokens < 0 || max_kv_len < 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || block_size < 0 ||
+      num_blocks < 0 || max_num_blocks < 0 || num_heads % num_kv_heads != 0 || !(scale > 0.f) || range_tiles <= 0)
+    return MVLLM_ERR_BAD_SHAPE;
+  if (num_seqs == 0 || total_q_tokens == 0) return MVLLM_OK;
+  if (!out || !q || !k || !v || !cu_seqlens_q || (paged && (!block_tables || !cu_seqlens_k))) return MVLLM_ERR_NULL_POINTER;
+  if (range_tiles % 2 != 0 || !ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype))
+    return MVLLM_ERR_UNSUPPORTED;
+  const int ranges = ranges_of(max_kv_len, range_tiles);
+  if (ranges > kMaxRanges) return MVLLM_ERR_UNSUPPORTED;
+  if (!aligned16(q) || !aligned16(out) || !aligned16(k) || !aligned16(v)) return MVLLM_ERR_MISALIGNED;
+  if (ranges > 1 && (!workspace || !aligned16(workspace)) ||
+      workspace_bytes < mvllm_prefill_ranges_workspace_bytes(total_q_tokens, max_kv_len, num_heads, head_dim, range_tiles))
+    return MVLLM_ERR_WORKSPACE;
+  hipStream_t s = (hipStream_t)stream;
+  PrefillArgs a = {};
+  a.out = out; a.q = q; a.k = k; a.v = v; a.cu_seqlens = cu_seqlens_q; a.total_tokens = total_q_tokens; a.num_seqs = num_seqs;
+  a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.head_dim = head_dim; a.scale_log2 = scale * kLog2e;
+  a.cu_seqlens_k = paged ? cu_seqlens_k : nullptr; a.block_tables = paged ? block_tables : nullptr; a.max_num_blocks = max_num_blocks;
+  a.block_size = block_size; a.num_blocks = num_blocks; a.sink = sink;
+  a.range_tiles = range_tiles;
+  a.part = reinterpret_cast<float*>(workspace);
+  a.lse = ranges > 1 ? a.part + (int64_t)ranges * total_q_tokens * num_heads * head_dim : nullptr;
+  const int status = launch_prefill_ranges(a, dtype, paged, ranges, s);
+  if (status != MVLLM_OK || ranges == 1) return status;
+  RangeMergeArgs m;
+  m.out = out; m.part = a.part; m.lse = a.lse; m.cu_seqlens_q = cu_seqlens_q; m.cu_seqlens_k = a.cu_seqlens_k; m.sink = sink;
+  m.num_seqs = num_seqs; m.ranges = ranges; m.range_tiles = range_tiles; m.rows_per_tile = rows_of_tile(num_heads / num_kv_heads);
+  m.total_q = (int)total_q_tokens; m.num_heads = num_heads;
+  const int per = 4 * (256 / head_dim);
+  const dim3 grid((unsigned)total_q_tokens, (unsigned)((num_heads + per - 1) / per));
+  if (dtype == MVLLM_BF16) {
+    if (head_dim == 128) range_merge_kernel<bf16_t, 128><<<grid, dim3(256), 0, s>>>(m);
+    else range_merge_kernel<bf16_t, 64><<<grid, dim3(256), 0, s>>>(m);
+  } else {
+    if (head_dim == 128) range_merge_kernel<f16_t, 128><<<grid, dim3(256), 0, s>>>(m);
+    else range_merge_kernel<f16_t, 64><<<grid, dim3(256), 0, s>>>(m);
+  }
+  return launch_status();
 }

@@ -175,13 +175,15 @@ def store_kvcache_int8(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Te
 
 def flash_attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens: torch.Tensor,
                             scale: float, num_heads: int, num_kv_heads: int, head_dim: int, *,
-                            sink: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+                            sink: torch.Tensor | None = None, out: torch.Tensor | None = None,
+                            max_seqlen: int | None = None) -> torch.Tensor:
     """Causal attention over a packed ragged batch.  Reference: attention.py:212-280.
 
     q: (total_tokens, num_heads, head_dim); k, v: (total_tokens, num_kv_heads,
     head_dim); cu_seqlens: int32 (num_seqs + 1,).  Returns a tensor like q.
     ``sink`` (float32 (num_heads,), not in the reference): one more exp(sink) per head in the softmax denominators;
-    ``out``: contiguous tensor like q to write to.
+    ``out``: contiguous tensor like q to write to.  ``max_seqlen``: the host's upper bound of every sequence's length, with
+    which a batch too small to fill the chip has its keys cut into ranges that are walked side by side.
     No device->host synchronisation happens here.
     """
     _C.require_cuda(q, k, v, cu_seqlens)
@@ -203,6 +205,9 @@ def flash_attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, c
     num_seqs = cu_seqlens.shape[0] - 1
     _warn_if_generic("prefill", num_heads, num_kv_heads, head_dim, 0, q.dtype, False)
     lib = _C.load()
+    if max_seqlen is not None and _prefill_ranges(lib, output, q, k, v, None, cu_seqlens, None, num_seqs, int(max_seqlen), scale,
+                                                  num_heads, num_kv_heads, head_dim, 0, 0, sink):
+        return output
     if sink is not None:
         st = lib.mvllm_prefill_varlen_sink(_ptr(output), _ptr(q), _ptr(k), _ptr(v), _ptr(cu_seqlens), num_seqs, total,
                                            num_heads, num_kv_heads, head_dim, float(scale), _sink_ptr(sink, num_heads),
@@ -214,6 +219,25 @@ def flash_attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, c
                                   _C.current_stream_ptr(q.device))
     _C.check(st, "flash_attention_prefill")
     return output
+
+
+def _prefill_ranges(lib, output, q, k, v, block_tables, cu_seqlens_q, cu_seqlens_k, num_seqs, max_seqlen, scale, num_heads,
+                    num_kv_heads, head_dim, block_size, num_blocks, sink) -> bool:
+    """Runs the call over key ranges if the library's plan says so."""
+    code = _C.dtype_code(q.dtype)
+    tiles = lib.mvllm_prefill_ranges_plan(num_seqs, q.shape[0], max_seqlen, num_heads, num_kv_heads, head_dim, block_size, code)
+    need = lib.mvllm_prefill_ranges_workspace_bytes(q.shape[0], max_seqlen, num_heads, head_dim, tiles) if tiles else 0
+    if not tiles or need > STAGED_PREFILL_MAX_BYTES or not scale > 0 or any(t.data_ptr() % 16 for t in (output, q, k, v)):
+        return False
+    workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None      # none: one range
+    st = lib.mvllm_prefill_ranges(_ptr(output), _ptr(q), _ptr(k), _ptr(v), 0 if block_tables is None else _ptr(block_tables),
+                                  0 if block_tables is None else block_tables.shape[1], _ptr(cu_seqlens_q),
+                                  0 if cu_seqlens_k is None else _ptr(cu_seqlens_k), num_seqs, q.shape[0], max_seqlen, num_heads,
+                                  num_kv_heads, head_dim, block_size, num_blocks, float(scale),
+                                  0 if sink is None else _sink_ptr(sink, num_heads), code, tiles, 0 if workspace is None else _ptr(workspace), need,
+                                  _C.current_stream_ptr(q.device))
+    _C.check(st, "prefill over key ranges")
+    return True
 
 
 def flash_attention_prefill_paged(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -275,6 +299,10 @@ def flash_attention_prefill_paged(q: torch.Tensor, k_cache: torch.Tensor, v_cach
             _C.check(st, "flash_attention_prefill_paged (staged)")
             return output
     if max_seqlen_k is not None and int(max_seqlen_k) > 0 and q.dtype != torch.float32:
+        if key_splits is None and _prefill_ranges(lib, output, q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, num_seqs,
+                                                  int(max_seqlen_k), scale, num_heads, num_kv_heads, head_dim, block_size,
+                                                  k_cache.shape[0], sink):
+            return output
         code = _C.dtype_code(q.dtype)
         splits = key_splits
         if splits is None:
@@ -606,7 +634,7 @@ class Attention(nn.Module):
                 o = flash_attention_prefill(q.reshape(bsz * n, self.num_heads, self.head_dim),
                                             k.reshape(bsz * n, self.num_kv_heads, self.head_dim),
                                             v.reshape(bsz * n, self.num_kv_heads, self.head_dim), cu, scale,
-                                            self.num_heads, self.num_kv_heads, self.head_dim)
+                                            self.num_heads, self.num_kv_heads, self.head_dim, max_seqlen=n)
                 return o.reshape(bsz, n, self.num_heads * self.head_dim)
             if q.dim() != 3:
                 raise ValueError("prefill expects q of shape (total_tokens, num_heads, head_dim) or "
@@ -630,7 +658,7 @@ class Attention(nn.Module):
                                                       self.head_dim, self.block_size, context.max_seqlen_k or None)
                 return o.reshape(o.shape[0], self.num_heads * self.head_dim)
             o = flash_attention_prefill(q, k, v, cu_seqlens, scale, self.num_heads, self.num_kv_heads,
-                                        self.head_dim)
+                                        self.head_dim, max_seqlen=context.max_seqlen_q or None)
             return o.reshape(o.shape[0], self.num_heads * self.head_dim)
 
         if q.dim() == 4:          # (B, 1, Hq, D) -> (B, Hq, D)

@@ -36,7 +36,7 @@ def kernel_sources(config: dict) -> list[str]:
         sources.append("decay_memory.hip")
     latent = [e["mixer"] for e in config["layers"] if e["type"] == "latent_attention"]
     if latent:
-        sources += ["latent.hip", "paged_decode.hip", "prefill_varlen.hip", "prefill_split.hip", "prefill_f32.hip"]
+        sources += ["latent.hip", "paged_decode.hip", "prefill_varlen.hip", "prefill_split.hip", "prefill_ranges.hip", "prefill_f32.hip"]
         if any(attention_head_dim(m["dim"], m["vdim"], torch.bfloat16) not in (64, 128) for m in latent):
             sources.append("prefill_other_dims.hip")
     if any(e.get("mlp") is not None for e in config["layers"]):

@@ -50,7 +50,7 @@ def kernel_sources(config: dict) -> list[str]:
         sources += ["gate_linear.hip", "mlstm.hip", "mlstm_chunk.hip"]
     attention = [e["mixer"] for e in config["layers"] if e["type"] == "attention"]
     if attention:
-        sources += ["head_rope.hip", "store_kvcache.hip", "paged_decode.hip", "prefill_varlen.hip", "prefill_split.hip",
+        sources += ["head_rope.hip", "store_kvcache.hip", "paged_decode.hip", "prefill_varlen.hip", "prefill_split.hip", "prefill_ranges.hip",
                     "prefill_f32.hip"]
         if any(attention_head_dim(m["dim"], m["vdim"], torch.bfloat16) not in (64, 128) for m in attention):
             sources.append("prefill_other_dims.hip")

@@ -1,0 +1,73 @@
+"""Prefill over ranges of key tiles (mvllm_prefill_ranges) against the CPU oracle and the other kernels."""
+import math
+
+import pytest
+import torch
+
+import oracle
+from helpers import error_stats, make_paged_prefill_case
+from minivllm_amd import _C
+from minivllm_amd.layers import attention
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+MAX_ABS_16, MEAN_ABS_16 = 2e-2, 2e-3                                   # the other forms' bounds: 16-bit weights and results
+
+
+def _run(c, hq, hkv, d, bs, tiles, max_k, paged, sink=None):
+    class Forced:
+        def __getattr__(self, name):
+            return getattr(_C.load(), name) if name != "mvllm_prefill_ranges_plan" else lambda *sizes: tiles
+    out = torch.full_like(c["q_new"] if paged else c["q"], float("nan")).to(DEV)
+    on = lambda name: c[name].to(DEV)
+    q, k, v, tables, cu_k = (on("q_new"), on("k_cache"), on("v_cache"), on("block_tables"), on("cu_k")) if paged \
+        else (on("q"), on("k"), on("v"), None, None)
+    took = attention._prefill_ranges(Forced(), out, q, k, v, tables, on("cu_q") if paged else on("cu_k"), cu_k, len(c["cu_k"]) - 1, max_k,
+                                     1 / math.sqrt(d), hq, hkv, d, bs if paged else 0, k.shape[0] if paged else 0, sink)
+    assert took
+    return out.cpu()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d,bs,lengths,cached,tiles", [
+    (8, 2, 128, 16, [128, 129, 127, 1], [64, 100, 126, 0], 2),         # a last tile that ends a range, starts one, falls short of it
+    (8, 4, 128, 32, [160, 700], [96, 690], 2),                         # a range that only the later of two row tiles reaches
+    (5, 5, 64, 48, [600, 300, 64], [470, 10, 63], 4),                  # one head per workgroup, row tiles over several waves
+    (4, 2, 64, 256, [1000, 30], [0, 7], 6),                            # nothing cached: every row tile its own number of ranges
+    (8, 2, 128, 16, [4200], [4190], 2),                                # 33 ranges
+    (16, 8, 128, 16, [500, 200], [400, 150], 8),                       # whole: one range
+])
+@pytest.mark.parametrize("paged", [True, False])
+def test_prefill_over_key_ranges(hq, hkv, d, bs, lengths, cached, tiles, paged, dtype):
+    c = make_paged_prefill_case(61, lengths, cached, hq, hkv, d, bs, dtype=dtype)
+    want = oracle.prefill_paged_oracle(c["q_new"].float(), torch.nan_to_num(c["k_cache"].float()), torch.nan_to_num(c["v_cache"].float()),
+                                       c["block_tables"], c["cu_q"], c["cu_k"], 1 / math.sqrt(d), hq, hkv, d, bs)
+    for bound in (max(lengths), max(1, max(lengths) - 150)):           # also a bound that is too low: the last range takes the rest
+        got = _run(c, hq, hkv, d, bs, tiles, bound, paged)
+        got = got if paged else got[c["new_rows"]]
+        mx, mean = error_stats(got, want)
+        assert torch.isfinite(got.float()).all() and mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (bound, mx, mean)
+
+
+@pytest.mark.parametrize("lengths", [[0, 300, 0, 77], [200]])
+def test_prefill_over_key_ranges_sinks_and_empty_sequences(lengths):
+    """Against the kernel without ranges: the sink counts once, sequences without tokens have no rows."""
+    c = make_paged_prefill_case(7, lengths, [0] * len(lengths), 8, 4, 128, 16, dtype=torch.bfloat16)
+    sink = torch.randn(8, generator=torch.Generator().manual_seed(1)).to(DEV)
+    got = _run(c, 8, 4, 128, 16, 2, max(lengths), False, sink)
+    want = attention.flash_attention_prefill(*(c[n].to(DEV) for n in ("q", "k", "v", "cu_k")), 128 ** -0.5, 8, 4, 128, sink=sink).cpu()
+    mx, mean = error_stats(got, want.float())
+    assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
+
+
+def test_prefill_ranges_plan_and_rejections():
+    lib = _C.load()
+    bf, f32 = _C.dtype_code(torch.bfloat16), _C.dtype_code(torch.float32)
+    plan = lib.mvllm_prefill_ranges_plan
+    assert plan(2, 343, 3435, 16, 8, 128, 16, bf) in range(6, 20, 2)     # few rows behind many keys: ranges
+    assert plan(2, 541, 275, 16, 8, 128, 0, bf) == 6                     # a small batch: whole (five tiles, an even number)
+    assert plan(16, 16000, 2048, 32, 8, 128, 0, bf) == 0                 # the chip is full
+    assert plan(65, 650, 4000, 16, 8, 128, 16, bf) == 0 and plan(1, 100, 4000, 16, 8, 128, 16, f32) == 0
+    assert plan(1, 100, 4000, 16, 8, 80, 16, bf) == 0 and plan(1, 100, 4000, 16, 8, 128, 8, bf) == 0
+    assert lib.mvllm_prefill_ranges_workspace_bytes(100, 640, 16, 128, 10) == 0
+    assert lib.mvllm_prefill_ranges_workspace_bytes(100, 641, 16, 128, 10) == 2 * 100 * 16 * 129 * 4
