@@ -120,10 +120,18 @@ inline int largest_divisor_le(int n, int cap) {
 // contexts are long, although up to 2x slower when they are much shorter than the table is wide, which the
 // host cannot know.
 // The partition is never shorter than partition_tokens_for's, so a workspace sized from it is always enough.
-constexpr int kSplitWaves = 4;            // 8 waves: 1-3 us slower per call except at 16 sequences (merge cost, one workgroup per CU)
+constexpr int kSplitWaves = 4;
+// Eight waves where that leaves no CU with more than one workgroup: a chain of half as many tiles (1 sequence of 300 tokens 7.3 -> 6.8 us,
+// 16 of 32-352 9.0 -> 8.3, 32 of 500-2000 38.1 -> 36.6; 64 of 32-352, two workgroups per CU, 12.9 -> 15.1).
+constexpr int kSplitManyWaves = 8;
 constexpr int kSplitMinGroups = 512;
 constexpr int kSplitMaxPart = 4096;
 constexpr int kSplitOnePartCtx = 512;
+// Tables of at most this many tokens (16-bit caches) are one partition from kSplitOnePartPairs (sequence, kv head) pairs on, and
+// below that cut into no less than kSplitNarrowPart tokens: us with partitions to fill the chip / so, 61 sequences of 64-1500 tokens
+// 51.5 / 37.6, 40 of 32-700 21.7 / 16.6, 32 of 500-2000 41.1 / 37.9 (16 of them 23.9 / 31.7); 1 of 2000 12.6 / 10.3, 4 of 1000-2000
+// 13.0 / 12.3, 8 of 100-1000 10.5 / 10.7.
+constexpr int kSplitNarrowCtx = 2048, kSplitNarrowPart = 256, kSplitOnePartPairs = 256;
 inline bool split_wanted(int64_t max_ctx, int batch, int num_kv_heads, bool int8) {
   const int part = partition_tokens_for(max_ctx, batch);
   const int64_t parts = (max_ctx + part - 1) / part;
@@ -136,14 +144,16 @@ inline bool split_wanted(int64_t max_ctx, int batch, int num_kv_heads, bool int8
   if (int8) return few_groups || ((short_parts || narrow_table) && (int64_t)batch * num_kv_heads <= 512);
   return few_groups || short_parts || narrow_table;
 }
-inline int split_partition_tokens(int64_t max_ctx, int batch, int num_kv_heads) {
+inline int split_partition_tokens(int64_t max_ctx, int batch, int num_kv_heads, bool sixteen_bit) {
   const int64_t pairs = (int64_t)batch * num_kv_heads;
   const int64_t want_parts = (kSplitMinGroups + pairs - 1) / pairs;
   int64_t part = ((max_ctx + want_parts - 1) / want_parts + 63) / 64 * 64;
   // a table of at most 512 tokens is one partition whatever the batch: four waves walk it in a few tiles each, and
   // the merge launch that several partitions need costs more than they save (16 sequences of 32-352 tokens:
   // 10.1 -> 8.0 us per call; from 1024-token tables on the finer split wins)
-  if (max_ctx <= kSplitOnePartCtx) part = (max_ctx + 63) / 64 * 64;
+  const bool narrow = sixteen_bit && max_ctx <= kSplitNarrowCtx;
+  if (narrow && part < kSplitNarrowPart) part = kSplitNarrowPart;
+  if (max_ctx <= kSplitOnePartCtx || (narrow && pairs >= kSplitOnePartPairs)) part = (max_ctx + 63) / 64 * 64;
   if (part > kSplitMaxPart) part = kSplitMaxPart;
   const int64_t floor_part = partition_tokens_for(max_ctx, batch);
   return (int)(part < floor_part ? floor_part : part);
@@ -463,49 +473,6 @@ struct DecodeHead {
       }
   }
 
-  // W waves hold partial results of the same heads over different tokens: waves 1 .. W-1 leave theirs in LDS
-  // (1 + kAcc float4 per lane: m, l and the accumulators), wave 0 folds them into its own with the usual
-  // log-sum-exp weights and is the only one to return true.  Every wave of the workgroup must call this.
-  template <int W>
-  __device__ __forceinline__ bool merge(int w, int lane) {
-    constexpr int kSlots = 1 + kAcc;
-    __shared__ float4 part[(W - 1) * kSlots * 64];
-    const int cls = lane >> 4;
-    if (w > 0) {
-      float4* dst = part + (w - 1) * kSlots * 64 + lane;
-      dst[0] = make_float4(m, l, 0.f, 0.f);
-#pragma unroll
-      for (int e = 0; e < kAcc; ++e) dst[(1 + e) * 64] = make_float4(o[e][0], o[e][1], o[e][2], o[e][3]);
-    }
-    __syncthreads();
-    if (w > 0) return false;
-#pragma unroll 1
-    for (int x = 0; x < W - 1; ++x) {
-      const float4* src = part + x * kSlots * 64 + lane;
-      const float4 ml = src[0];
-      const float m_new = fmaxf(m, ml.x);
-      const float f0 = safe_exp2_diff(m, m_new);          // both are 0 while neither wave has seen a token
-      const float f1 = safe_exp2_diff(ml.x, m_new);
-      m = m_new;
-      l = l * f0 + ml.y * f1;
-      float a0[4], a1[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {                        // accumulator row j is head 4*cls + j
-        a0[j] = __shfl(f0, 4 * cls + j, 64);
-        a1[j] = __shfl(f1, 4 * cls + j, 64);
-      }
-#pragma unroll
-      for (int e = 0; e < kAcc; ++e) {
-        const float4 ow = src[(1 + e) * 64];
-        o[e][0] = o[e][0] * a0[0] + ow.x * a1[0];
-        o[e][1] = o[e][1] * a0[1] + ow.y * a1[1];
-        o[e][2] = o[e][2] * a0[2] + ow.z * a1[2];
-        o[e][3] = o[e][3] * a0[3] + ow.w * a1[3];
-      }
-    }
-    return true;
-  }
-
   // write the output row (direct) or this partition's partial result
   __device__ __forceinline__ void finish(const DecodeArgs& a, int b, int p, int head0, int group, bool direct, int lane) {
     finish_head(*this, a, b, p, head0, group, direct, lane);
@@ -619,45 +586,6 @@ struct DecodeHead<float, D> {
       }
   }
 
-  template <int W>
-  __device__ __forceinline__ bool merge(int w, int lane) {
-    __shared__ float4 part[(W - 1) * (1 + kAcc) * 64];
-    const int cls = lane >> 4;
-    if (w > 0) {
-      float4* dst = part + (w - 1) * (1 + kAcc) * 64 + lane;
-      dst[0] = make_float4(m, l, 0.f, 0.f);
-#pragma unroll
-      for (int e = 0; e < kAcc; ++e) dst[(1 + e) * 64] = make_float4(o[e][0], o[e][1], o[e][2], o[e][3]);
-    }
-    __syncthreads();
-    if (w > 0) return false;
-#pragma unroll 1
-    for (int x = 0; x < W - 1; ++x) {
-      const float4* src = part + x * (1 + kAcc) * 64 + lane;
-      const float4 ml = src[0];
-      const float m_new = fmaxf(m, ml.x);
-      const float f0 = safe_exp2_diff(m, m_new);
-      const float f1 = safe_exp2_diff(ml.x, m_new);
-      m = m_new;
-      l = l * f0 + ml.y * f1;
-      float a0[4], a1[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        a0[j] = __shfl(f0, 4 * cls + j, 64);
-        a1[j] = __shfl(f1, 4 * cls + j, 64);
-      }
-#pragma unroll
-      for (int e = 0; e < kAcc; ++e) {
-        const float4 ow = src[(1 + e) * 64];
-        o[e][0] = o[e][0] * a0[0] + ow.x * a1[0];
-        o[e][1] = o[e][1] * a0[1] + ow.y * a1[1];
-        o[e][2] = o[e][2] * a0[2] + ow.z * a1[2];
-        o[e][3] = o[e][3] * a0[3] + ow.w * a1[3];
-      }
-    }
-    return true;
-  }
-
   __device__ __forceinline__ void write_row(float* row_ptr, int j, float scale, int lane) const {
     const int col = lane & 15;
 #pragma unroll
@@ -670,6 +598,61 @@ struct DecodeHead<float, D> {
     finish_head(*this, a, b, p, head0, group, direct, lane);
   }
 };
+
+// W waves hold partial results of the same heads over different tokens: all of them leave theirs in LDS, a row per live head, and
+// then share the log-sum-exp merge and the output, four dims of a head per thread.  (One wave folding the others' accumulators into
+// its own, 16 heads whether live or not, was a chain of 0.3 us per wave.)  Every wave of the workgroup must call this.
+template <int W, typename HEAD>
+__device__ __forceinline__ void finish_waves(HEAD& hd, const DecodeArgs& a, int b, int p, int head0, int group, bool direct, int w, int lane) {
+  using T = typename HEAD::Elem;
+  constexpr int D = HEAD::kDim;
+  __shared__ __attribute__((aligned(16))) float rows[W][16][D];
+  __shared__ float2 ml[W][16];
+  hd.l += __shfl_xor(hd.l, 16, 64);                 // the four token classes
+  hd.l += __shfl_xor(hd.l, 32, 64);
+  if (lane < 16) ml[w][lane] = make_float2(hd.m, hd.l);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int h = 4 * (lane >> 4) + j;
+    if (h < group) hd.write_partial(rows[w][h], j, lane);
+  }
+  __syncthreads();
+  for (int i = 64 * w + lane; i < group * (D / 4); i += 64 * W) {
+    const int h = i / (D / 4), c = 4 * (i % (D / 4));
+    float2 of[W];
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int x = 0; x < W; ++x) {
+      of[x] = ml[x][h];
+      m = fmaxf(m, of[x].x);
+    }
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int x = 0; x < W; ++x) {
+      const float f = safe_exp2_diff(of[x].x, m);   // 0 for a wave that has seen no token
+      const float4 r = *reinterpret_cast<const float4*>(&rows[x][h][c]);
+      l += of[x].y * f;
+      o.x += r.x * f;
+      o.y += r.y * f;
+      o.z += r.z * f;
+      o.w += r.w * f;
+    }
+    if (direct) {
+      if (a.sink != nullptr) l = add_sink(l, m, a.sink[head0 + h]);
+      const float linv = l > 0.f ? 1.f / l : 0.f;
+      T* out = reinterpret_cast<T*>(a.out) + ((int64_t)b * a.num_heads + head0 + h) * D + c;
+      if constexpr (sizeof(T) == 4) *reinterpret_cast<float4*>(out) = make_float4(o.x * linv, o.y * linv, o.z * linv, o.w * linv);
+      else {
+        const T r[4] = {from_float<T>(o.x * linv), from_float<T>(o.y * linv), from_float<T>(o.z * linv), from_float<T>(o.w * linv)};
+        *reinterpret_cast<uint2*>(out) = *reinterpret_cast<const uint2*>(r);
+      }
+    } else {
+      const int64_t slot = ((int64_t)b * a.num_parts + p) * a.num_heads + head0 + h;
+      *reinterpret_cast<float4*>(a.ws_acc + slot * D + c) = o;
+      if (c == 0) *reinterpret_cast<float2*>(a.ws_ml + slot * 2) = make_float2(m, l);
+    }
+  }
+}
 
 // W = 1: the wave walks all tiles of its partition.  W > 1 (the workgroup is W waves on one kv head): wave w takes
 // tiles w, w + W, ... and the partial results meet in LDS (DecodeHead::merge), so a short context costs a few tiles
@@ -798,10 +781,8 @@ __device__ __forceinline__ void decode_mfma_item(const DecodeArgs& a, int b, int
     head.consume(tb, part_end, a.scale_log2, lane);
   }
   if (tile < ntiles) head.consume(ta, part_end, a.scale_log2, lane);
-  if constexpr (W > 1) {
-    if (!head.template merge<W>(w, lane)) return;
-  }
-  head.finish(a, b, p, hs.head0, group, direct, lane);
+  if constexpr (W > 1) finish_waves<W>(head, a, b, p, hs.head0, group, direct, w, lane);
+  else head.finish(a, b, p, hs.head0, group, direct, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1562,13 +1543,15 @@ static int head_chunks_of(int num_heads, int num_kv_heads) { return (num_heads /
 struct DecodePlan {
   int part_tokens, num_parts, waves_per_head;
 };
-static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, int block_size, bool fast_ok, bool int8) {
+static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, int block_size, bool fast_ok, bool int8, int head_dim, int dtype) {
   const int64_t max_ctx = (int64_t)max_num_blocks * block_size;
   const bool split = fast_ok && split_wanted(max_ctx, batch, num_kv_heads, int8);
   DecodePlan plan;
-  plan.part_tokens = split ? split_partition_tokens(max_ctx, batch, num_kv_heads) : partition_tokens_for(max_ctx, batch);
+  plan.part_tokens = split ? split_partition_tokens(max_ctx, batch, num_kv_heads, !int8 && dtype != MVLLM_F32) : partition_tokens_for(max_ctx, batch);
   plan.num_parts = (int)((max_ctx + plan.part_tokens - 1) / plan.part_tokens);
-  plan.waves_per_head = !fast_ok ? 0 : split ? kSplitWaves : 1;
+  const bool many = !int8 && dtype != MVLLM_F32 && (head_dim == 128 || head_dim == 64) && block_size % kTile == 0 &&
+                    (int64_t)batch * num_kv_heads * plan.num_parts <= (plan.num_parts == 1 ? 256 : 64);
+  plan.waves_per_head = !fast_ok ? 0 : !split ? 1 : many ? kSplitManyWaves : kSplitWaves;
   return plan;
 }
 
@@ -1576,7 +1559,8 @@ template <typename T> struct IsSixteenBit { static constexpr bool value = true; 
 template <> struct IsSixteenBit<float> { static constexpr bool value = false; };
 
 template <typename T>
-static int launch_decode(DecodeArgs a, bool int8, bool fast_ok, bool split, hipStream_t stream) {
+static int launch_decode(DecodeArgs a, bool int8, bool fast_ok, int waves, hipStream_t stream) {
+  const bool split = waves > 1;
   bool launched = false;
   // kv heads (waves) per workgroup of the one-wave-per-head form: as many as allowed, so that a workgroup streams
   // whole token rows; fewer when the grid would otherwise leave most CUs without a workgroup
@@ -1592,6 +1576,13 @@ static int launch_decode(DecodeArgs a, bool int8, bool fast_ok, bool split, hipS
     const dim3 grid((unsigned)a.num_parts, (unsigned)a.batch, groups);
     auto go = [&](auto DIM) {
       constexpr int D = decltype(DIM)::value;
+      if constexpr (IsSixteenBit<T>::value && (D == 64 || D == 128)) {
+        if (waves == kSplitManyWaves) {
+          decode_mfma_split_kernel<T, kSplitManyWaves, D><<<split_grid, dim3(64 * kSplitManyWaves), 0, stream>>>(a);
+          launched = true;
+          return;
+        }
+      }
       if (split) decode_mfma_split_kernel<T, kSplitWaves, D><<<split_grid, split_block, 0, stream>>>(a);
       else decode_mfma_kernel<T, D><<<grid, block, 0, stream>>>(a);
       launched = true;
@@ -1675,8 +1666,7 @@ static int decode_entry(void* out, const void* q, const void* k_cache, const voi
   const bool fast_ok = fast_shape(num_heads, num_kv_heads, head_dim, block_size, dtype, int8) &&
                        aligned16(q) && aligned16(out) && aligned16(k_cache) && aligned16(v_cache);
   a.head_chunks = head_chunks_of(num_heads, num_kv_heads);
-  const DecodePlan plan = plan_decode(batch, num_kv_heads * a.head_chunks, max_num_blocks, block_size, fast_ok, int8);
-  const bool split = plan.waves_per_head > 1;
+  const DecodePlan plan = plan_decode(batch, num_kv_heads * a.head_chunks, max_num_blocks, block_size, fast_ok, int8, head_dim, dtype);
   a.part_tokens = plan.part_tokens;
   a.num_parts = plan.num_parts;
   a.scale_log2 = scale * kLog2e;
@@ -1690,9 +1680,9 @@ static int decode_entry(void* out, const void* q, const void* k_cache, const voi
   }
   hipStream_t s = (hipStream_t)stream;
   switch (dtype) {
-    case MVLLM_F32: return launch_decode<float>(a, int8, fast_ok, split, s);
-    case MVLLM_BF16: return launch_decode<bf16_t>(a, int8, fast_ok, split, s);
-    default: return launch_decode<f16_t>(a, int8, fast_ok, split, s);
+    case MVLLM_F32: return launch_decode<float>(a, int8, fast_ok, plan.waves_per_head, s);
+    case MVLLM_BF16: return launch_decode<bf16_t>(a, int8, fast_ok, plan.waves_per_head, s);
+    default: return launch_decode<f16_t>(a, int8, fast_ok, plan.waves_per_head, s);
   }
 }
 
@@ -1750,7 +1740,7 @@ extern "C" int mvllm_paged_decode_plan(int batch, int num_heads, int num_kv_head
       num_heads % num_kv_heads != 0)
     return MVLLM_ERR_BAD_SHAPE;
   const DecodePlan plan = plan_decode(batch, num_kv_heads * head_chunks_of(num_heads, num_kv_heads), max_num_blocks, block_size,
-                                      fast_shape(num_heads, num_kv_heads, head_dim, block_size, dtype, int8_cache != 0), int8_cache != 0);
+                                      fast_shape(num_heads, num_kv_heads, head_dim, block_size, dtype, int8_cache != 0), int8_cache != 0, head_dim, dtype);
   if (part_tokens) *part_tokens = plan.part_tokens;
   if (num_parts) *num_parts = plan.num_parts;
   if (waves_per_head) *waves_per_head = plan.waves_per_head;

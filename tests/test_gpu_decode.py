@@ -74,6 +74,22 @@ def test_context_length_boundaries(ctx_list, bs):
     assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
 
 
+@pytest.mark.parametrize("hq,hkv,d,bs,ctx_list", [
+    (16, 1, 128, 16, [1, 5, 16, 17, 127, 128, 129, 511, 512]),        # waves without a token, every wave its first, one its second; 16 heads
+    (4, 2, 64, 32, [300]),                                            # two heads of 64 dims: fewer outputs than threads
+    (40, 2, 128, 16, [500, 33]),                                      # 20 heads per kv head: two slices, the second of four
+    (16, 2, 128, 256, [2000]),                                        # partitions of eight waves each
+    (8, 2, 128, 16, [1500]),
+])
+def test_eight_waves_per_head(hq, hkv, d, bs, ctx_list):
+    case = make_paged_case(39, len(ctx_list), 1, 1, hq, hkv, d, bs, dtype=torch.bfloat16, ctx_list=ctx_list)
+    scale = 1 / math.sqrt(d)
+    assert paged_decode_plan(len(ctx_list), hq, hkv, d, case[3].shape[1], bs)[2] == 8
+    got = _run(*case, scale, hq, hkv, d, bs)
+    mx, mean = error_stats(got, _oracle32(*case, scale, hq, hkv, d, bs))
+    assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
+
+
 @pytest.mark.parametrize("dtype,hq,hkv,d,bs", [
     (torch.float32, 4, 2, 64, 4),       # generic kernel: fp32 with a block size of 4
     (torch.float32, 6, 2, 96, 16),      # fp32, head_dim 96
