@@ -655,7 +655,7 @@ __device__ __forceinline__ void finish_waves(HEAD& hd, const DecodeArgs& a, int 
 }
 
 // W = 1: the wave walks all tiles of its partition.  W > 1 (the workgroup is W waves on one kv head): wave w takes
-// tiles w, w + W, ... and the partial results meet in LDS (DecodeHead::merge), so a short context costs a few tiles
+// tiles w, w + W, ... and the partial results meet in LDS (finish_waves), so a short context costs a few tiles
 // of latency per wave and no second launch.
 // SUB: blocks of 1, 2, 4 or 8 tokens.  A 16-token tile then spans several blocks, and every lane looks up the blocks
 // of its own tokens (one for its K row, up to four for its V rows) in the block-table window.
@@ -990,20 +990,81 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
   const int ntiles = W == 1 ? tiles_all : (tiles_all > w ? (tiles_all - w + W - 1) / W : 0);   // this wave's
   if constexpr (W == 1) win = (win_base + lane < a.max_num_blocks) ? table[win_base + lane] : -1;
 
+  // the query's and the first tile's loads set out together: a workgroup's first keys arrive while the query becomes int8 (one after the
+  // other the same batch took 251 us, not 240)
+  uint4 qr[2 * kSteps];                // this lane's 16 dims of each 64-dim step of its head
+  {
+    const bool live = col < group;
+    const T* src = reinterpret_cast<const T*>(a.q) + ((int64_t)b * a.num_heads + hs.head0 + (live ? col : 0)) * D + 16 * q4;
+#pragma unroll
+    for (int j = 0; j < 2 * kSteps; ++j)
+      qr[j] = live ? *reinterpret_cast<const uint4*>(src + 64 * (j / 2) + 8 * (j % 2)) : make_uint4(0u, 0u, 0u, 0u);
+  }
+  const int64_t row = (int64_t)a.num_kv_heads * D;          // bytes per token row
+  const char* kc = reinterpret_cast<const char*>(a.k_cache) + (int64_t)g * D;
+  const char* vc = reinterpret_cast<const char*>(a.v_cache) + (int64_t)g * D;
+  // W == 1, a stream of many tiles: K arrives in whole rows, D / 16 lanes each, and goes through LDS into the first product's operands;
+  // in the operands' own order, token lane%16 and bytes 16*q4 (+64 j), a load's lanes are 16 bytes of 16 rows, and 128 sequences of
+  // 256-16384 tokens took 240 us instead of 230
+  constexpr bool kRows = W == 1;
+  constexpr int kChunks = D / 16, kRowsPer = 64 / kChunks;   // 16-byte chunks of a row, rows of a load
+  const int k_lane_off = kRows ? lane / kChunks * (int)row + lane % kChunks * 16 : col * (int)row + q4 * 16;
+  const int64_t k_step = kRows ? (int64_t)kRowsPer * row : 64;
+  const int v_lane_off = 4 * q4 * (int)row + col * 8;       // tokens 4*q4 + i, dims 8*(lane%16)
+  const int s_lane_tok = 4 * q4 + (lane & 3);               // token whose scales this lane loads
+
+  auto load_tile = [&](KVTileI8& t, int tile) {
+    t.t0 = first + tile * (W * kTile);
+    if (bi - win_base >= 64) {
+      win_base = bi;
+      win = (win_base + lane < a.max_num_blocks) ? table[win_base + lane] : -1;
+    }
+    const int phys = __builtin_amdgcn_readlane(win, bi - win_base);
+    t.ok = (bi < a.max_num_blocks) && phys >= 0 && (int64_t)phys < a.num_blocks;
+    if (t.ok) {
+      const int64_t tok0 = (int64_t)phys * bs + off;
+      const char* kp = kc + tok0 * row + k_lane_off;
+      const char* vp = vc + tok0 * row + v_lane_off;
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j) t.k[j] = kRows ? load16_stream(kp + j * k_step) : *reinterpret_cast<const uint4*>(kp + j * k_step);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) t.v[i] = owns ? load8_stream(vp + i * row) : make_uint2(0u, 0u);
+      const int64_t sidx = (tok0 + s_lane_tok) * a.num_kv_heads + g;
+      t.ks = a.k_scale[sidx];
+      t.vs = a.v_scale[sidx];
+    } else {
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j) t.k[j] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) t.v[i] = make_uint2(0u, 0u);
+      t.ks = t.vs = 0.f;
+    }
+    if constexpr (W == 1) {
+      off += kTile;
+      if (off >= bs) { off = 0; ++bi; }
+    } else {
+      off += W * kTile;
+      while (off >= bs) { off -= bs; ++bi; }
+    }
+  };
+
+  KVTileI8 ta, tb;
+  if (ntiles > 0) load_tile(ta, 0);
+  __builtin_amdgcn_sched_barrier(0);
+
   // ---- query -> int8 hi/lo planes (B operand: column lane%16 -> head, bytes 16*q4.. of each 64-dim step)
   v4i qhi[kSteps], qlo[kSteps];
   float qscale;                        // amax/16256 * scale*log2e of this lane's head
   {
-    const T* q = reinterpret_cast<const T*>(a.q);
-    const bool live = col < group;
-    const T* src = q + ((int64_t)b * a.num_heads + hs.head0 + (live ? col : 0)) * D;
     float x[kSteps][16];
     float amax = 0.f;
 #pragma unroll
     for (int j = 0; j < kSteps; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        x[j][e] = live ? to_float(src[64 * j + 16 * q4 + e]) : 0.f;
+        const uint32_t w = e < 8 ? (e < 2 ? qr[2 * j].x : e < 4 ? qr[2 * j].y : e < 6 ? qr[2 * j].z : qr[2 * j].w)
+                                 : (e < 10 ? qr[2 * j + 1].x : e < 12 ? qr[2 * j + 1].y : e < 14 ? qr[2 * j + 1].z : qr[2 * j + 1].w);
+        x[j][e] = e & 1 ? hi_to_float<T>(w) : lo_to_float<T>(w);
         amax = fmaxf(amax, fabsf(x[j][e]));
       }
     amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
@@ -1033,48 +1094,8 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-  const int64_t row = (int64_t)a.num_kv_heads * D;          // bytes per token row
-  const char* kc = reinterpret_cast<const char*>(a.k_cache) + (int64_t)g * D;
-  const char* vc = reinterpret_cast<const char*>(a.v_cache) + (int64_t)g * D;
-  const int k_lane_off = col * (int)row + q4 * 16;          // token lane%16, bytes 16*q4 (+64 j)
-  const int v_lane_off = 4 * q4 * (int)row + col * 8;       // tokens 4*q4 + i, dims 8*(lane%16)
-  const int s_lane_tok = 4 * q4 + (lane & 3);               // token whose scales this lane loads
-
-  auto load_tile = [&](KVTileI8& t, int tile) {
-    t.t0 = first + tile * (W * kTile);
-    if (bi - win_base >= 64) {
-      win_base = bi;
-      win = (win_base + lane < a.max_num_blocks) ? table[win_base + lane] : -1;
-    }
-    const int phys = __builtin_amdgcn_readlane(win, bi - win_base);
-    t.ok = (bi < a.max_num_blocks) && phys >= 0 && (int64_t)phys < a.num_blocks;
-    if (t.ok) {
-      const int64_t tok0 = (int64_t)phys * bs + off;
-      const char* kp = kc + tok0 * row + k_lane_off;
-      const char* vp = vc + tok0 * row + v_lane_off;
-#pragma unroll
-      for (int j = 0; j < kSteps; ++j) t.k[j] = *reinterpret_cast<const uint4*>(kp + 64 * j);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) t.v[i] = owns ? load8_stream(vp + i * row) : make_uint2(0u, 0u);
-      const int64_t sidx = (tok0 + s_lane_tok) * a.num_kv_heads + g;
-      t.ks = a.k_scale[sidx];
-      t.vs = a.v_scale[sidx];
-    } else {
-#pragma unroll
-      for (int j = 0; j < kSteps; ++j) t.k[j] = make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) t.v[i] = make_uint2(0u, 0u);
-      t.ks = t.vs = 0.f;
-    }
-    if constexpr (W == 1) {
-      off += kTile;
-      if (off >= bs) { off = 0; ++bi; }
-    } else {
-      off += W * kTile;
-      while (off >= bs) { off -= bs; ++bi; }
-    }
-  };
-
+  __shared__ __attribute__((aligned(16))) char k_tiles[kRows ? kDecodeI8Wpb : 1][kRows ? kTile * D : 16];
+  char* k_lds = k_tiles[kRows ? threadIdx.x >> 6 : 0];        // this wave's (no barrier: the LDS keeps a wave's order)
   auto consume = [&](const KVTileI8& t) {
     if constexpr (MVLLM_DECODE_LOADS_ONLY) {
       uint32_t x = __float_as_uint(t.ks) ^ __float_as_uint(t.vs);
@@ -1101,9 +1122,17 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
 #pragma unroll
     for (int r = 0; r < 4; ++r) lv4[r] = __log2f(fmaxf(vs4[r], 9.094947e-13f));
     v4i shi = {0, 0, 0, 0}, slo = {0, 0, 0, 0};
+    if constexpr (kRows) {
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j) {
+        const int tok = kRowsPer * j + lane / kChunks;
+        *reinterpret_cast<uint4*>(k_lds + (tok * kChunks + ((lane ^ tok) & (kChunks - 1))) * 16) = t.k[j];
+      }
+    }
 #pragma unroll
     for (int j = 0; j < kSteps; ++j) {
-      const v4i kf = (v4i){(int)t.k[j].x, (int)t.k[j].y, (int)t.k[j].z, (int)t.k[j].w};
+      const uint4 k16 = kRows ? *reinterpret_cast<const uint4*>(k_lds + (col * kChunks + ((q4 + 4 * j) ^ (col & (kChunks - 1)))) * 16) : t.k[j];
+      const v4i kf = (v4i){(int)k16.x, (int)k16.y, (int)k16.z, (int)k16.w};
       shi = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qhi[j], shi, 0, 0, 0);
       slo = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qlo[j], slo, 0, 0, 0);
     }
@@ -1161,8 +1190,6 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
   };
 
   // tiles in pairs, the odd one after the loop (see the 16-bit kernel)
-  KVTileI8 ta, tb;
-  if (ntiles > 0) load_tile(ta, 0);
   int tile = 0;
   for (; tile + 1 < ntiles; tile += 2) {
     load_tile(tb, tile + 1);
@@ -1173,8 +1200,7 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
   if (tile < ntiles) consume(ta);
 
   if constexpr (W > 1) {
-    // waves 1 .. W-1 leave m, l, the weight sum and their accumulators in LDS, wave 0 folds them in (as in
-    // DecodeHead::merge) and goes on alone
+    // waves 1 .. W-1 leave m, l, the weight sum and their accumulators in LDS, wave 0 folds them in and goes on alone
     __shared__ float4 part[(W - 1) * 9 * 64];
     if (w > 0) {
       float4* dst = part + (w - 1) * 9 * 64 + lane;
