@@ -798,6 +798,15 @@ int mvllm_linear_small_m_gelu(void* out, const void* x, const void* w, const voi
                               int dtype, void* stream);
 
 /*
+ * mvllm_linear_small_m (gelu != 0: mvllm_linear_small_m_gelu) with room for sums over parts of K, which a long K with few columns takes.
+ * mvllm_linear_small_m_split_bytes says how much for a shape, 0 where the product runs in one launch and the workspace is not looked at.
+ * The workspace is 16-byte aligned and free again after the call's work on the stream; too little: MVLLM_ERR_WORKSPACE.
+ */
+size_t mvllm_linear_small_m_split_bytes(int M, int N, int K, int64_t x_row_stride);
+int mvllm_linear_small_m_split(void* out, const void* x, const void* w, const void* bias, int64_t x_row_stride,
+                               int M, int N, int K, int gelu, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Between the sublayers of a decoder that norms what they return (csrc/post_norm.hip): x_out = x + norm(y) * gain (fp32
  * [rows, width]; may be x itself, or NULL), out = x_out, or norm(x_out) * final_gain where that is not NULL, in dtype, zeros from
  * `width` to out_row_stride.  norm divides by sqrt(mean of squares + eps), with `centred` after taking the mean off.

@@ -6,7 +6,8 @@
 // operand's lanes are sixteen different rows).  Hence two kernels:
 //   linear_rows_kernel (very few rows): weights and x straight into registers, eight rows x 128 bytes per load.
 //   linear_ring_kernel (more rows): W and x through a ring of tiles in LDS, copied as whole 128-byte lines.
-// Both read a weight once.  A sum's order depends on (M, N, K) only, not on what follows the product.
+// Both read a weight once.  A sum's order depends on (M, N, K), not on what follows the product; a long K with few columns is cut into
+// parts where the caller brings room for their sums (linear_split).
 // mvllm_norm_linear_small_m is the same product with the launches around it folded in: the residual add + RMSNorm in
 // front of the layer's first projections (src/myvllm/models/qwen3.py:197-212 through layers/layernorm.py:9-28) as
 // the kernel's prologue (linear_norm_kernel), and SiluAndMul behind the gate/up projection (layers/activation.py:15-18) as
@@ -31,6 +32,7 @@ struct LinearArgs {
   float eps;
   int row_tiles;          // norm: tiles of 16 rows, a workgroup per column tile each
   int gelu;               // plain product only: the result through the tanh form of gelu
+  float* part;            // plain product only: partial sums [gridDim.y, M, N] of the splits of K, or null
 };
 
 // silu(g) * u with the roundings of the two tensor operations (activation.hip): silu in fp32 rounded to T, then the
@@ -202,14 +204,15 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
     if constexpr (i < 2 * CT) from[i] = (uint32_t)min(8 * (GLU ? b >> 1 : b) + r8, left - 1) * row_bytes + piece;
     else from[i] = (uint32_t)min(8 * (b - WB) + r8, a.M - 1) * (uint32_t)a.x_row_stride * 2u + piece;
   });
-  const int steps = a.K / (64 * SK);
+  const int steps_all = a.K / (64 * SK), per_split = (steps_all + (int)gridDim.y - 1) / (int)gridDim.y, step0 = per_split * (int)blockIdx.y;
+  const int steps = max(min(steps_all - step0, per_split), 0);      // of this workgroup's share of K
   const uint32_t lds0 = lds_address(lds) + sk * kPanel + sc * 1024;
   auto copy = [&](int step, int buffer) __attribute__((always_inline)) {
     const bool live = step < steps;
     const v4i x_rows = make_rsrc(reinterpret_cast<const char*>(a.x), live ? x_bytes : 0u);
     const v4i w_rows = make_rsrc(w0, live ? w_bytes : 0u);
     const v4i up_rows = GLU ? make_rsrc(w0 + (int64_t)out_cols * row_bytes, live ? w_bytes : 0u) : w_rows;
-    const uint32_t at = live ? (uint32_t)step * (SK * 128) : 0u, base = lds0 + buffer * kStage;
+    const uint32_t at = live ? (uint32_t)(step0 + step) * (SK * 128) : 0u, base = lds0 + buffer * kStage;
     static_for<kCopies>([&](auto I) {
       constexpr int i = decltype(I)::value;
       if constexpr (i < 2 * CT) dma16_to_lds_at<i * SC * 1024, NT>(GLU && ((i * SC + sc) & 1) ? up_rows : w_rows, from[i], at, base);
@@ -270,8 +273,28 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
       for (int r = 0; r < 4; ++r) u[r] = __shfl_xor(s[r], 32, 64);
       if (cls >= 2) continue;
     }
-    finish_four<T, GLU>(a, 16 * (mc / CT) + col, first + (GLU ? 8 : 16) * (c * CT + mc % CT) + 4 * cls, s, u);
+    const int m = 16 * (mc / CT) + col, j = first + (GLU ? 8 : 16) * (c * CT + mc % CT) + 4 * cls;
+    if (!GLU && a.part) {
+      if (m < a.M && j < a.N) *reinterpret_cast<float4*>(a.part + ((int64_t)blockIdx.y * a.M + m) * a.N + j) = make_float4(s[0], s[1], s[2], s[3]);
+    } else {
+      finish_four<T, GLU>(a, m, j, s, u);
+    }
   }
+}
+
+// The sums of the splits of K, four outputs a thread.
+template <typename T>
+__global__ __launch_bounds__(256) void linear_sum_kernel(const LinearArgs a, int splits) {
+  const int64_t at = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x), size = (int64_t)a.M * a.N;
+  if (at >= size) return;
+  float s[4] = {0.f, 0.f, 0.f, 0.f}, u[4];
+#pragma unroll 4
+  for (int i = 0; i < splits; ++i) {
+    const float4 p = *reinterpret_cast<const float4*>(a.part + i * size + at);
+    s[0] += p.x; s[1] += p.y; s[2] += p.z; s[3] += p.w;
+  }
+  const int m = (int)(at / a.N);
+  finish_four<T, false>(a, m, (int)(at - (int64_t)m * a.N), s, u);
 }
 
 // The product behind the residual add and norm: K = 512 P, eight waves, each with 64 P values of K, 16 rows of x and 16 CT weight rows per
@@ -428,6 +451,24 @@ static int ring_columns(int M, int N) {
   return best;
 }
 
+// Splits of K: with narrow tiles every workgroup reads all of x, rows * K values, and the CUs' copies of it, not the weights, take the time
+// once K is long; with wider tiles and three or four splits of K the workgroups are as many and each reads a part of x, for
+// a second launch (2.5 us) that adds the partial sums up.  us at 16 / 33 / 64 rows, whole and split: 4096 x 12288 22.1 / 30.7 / 37.1 and
+// 21.1 / 23.0 / 27.0, 5120 x 8192 23.6 / 27.6 / 32.0 and 20.5 / 21.4 / 24.5, 4096 x 6144 12.9 / 17.6 / 20.9 and 13.0 / 14.4 / 17.4,
+// 2048 x 6144 10.0 / 13.9 / 18.0 and 8.6 / 9.7 / 11.7, 1024 x 6144 9.2 / 13.3 / 17.2 and 6.8 / 8.5 / 9.6.  No gain: 4 to 24 rows of 2736 to 4096
+// columns and K of 6144 to 8192 (3072 x 8192 at 16 rows 13.8 and 14.8), 4096 x 4096 (13.6 and 13.2 at 64 rows), more columns
+// (6144 x 4096 18.5 and 18.3), 1024 x 3072 up to 32 rows (5.4 and 6.2 at 16; 9.0 and 7.4 at 64).
+struct LinearSplit { int columns, splits; };               // splits 1: whole
+static LinearSplit linear_split(int M, int N, int K) {
+  constexpr int kTiles = 256 / 3;                           // at most so many, for three splits of each over 256 CUs
+  if (M <= kFewRows || N < 1024 || N > 64 * kTiles) return {0, 1};
+  const bool narrow = N <= 2048, many = M > 32;
+  if (!(K >= 12288 || (K >= 6144 && (narrow || N > 4096 || many)) || (K >= 3072 && narrow && many))) return {0, 1};
+  const int columns = N <= 16 * kTiles ? 16 : N <= 32 * kTiles ? 32 : 64;
+  const int splits = 256 / ((N + columns - 1) / columns);
+  return {columns, splits < 4 ? splits : 4};
+}
+
 template <typename T, bool GLU>
 static int launch_rows(const LinearArgs& a, hipStream_t stream) {
   // few columns: narrow tiles and more waves on a tile's K, to have more loads under way.  us at one row with 8 columns and 8 / 4 waves, 16 columns
@@ -449,8 +490,9 @@ static int launch_rows(const LinearArgs& a, hipStream_t stream) {
 template <typename T, int MT, bool GLU>
 static int launch_ring(const LinearArgs& a, hipStream_t stream) {
   const bool stream_weights = (int64_t)a.N * a.K * 2 >= kStreamBytes;
-  const int columns = ring_columns(a.M, a.N);
-  const dim3 grid((unsigned)((a.N + columns - 1) / columns));
+  const LinearSplit split = a.part ? linear_split(a.M, a.N, a.K) : LinearSplit{ring_columns(a.M, a.N), 1};
+  const int columns = split.columns;
+  const dim3 grid((unsigned)((a.N + columns - 1) / columns), (unsigned)split.splits);
   constexpr int S = MT > 2 ? 3 : 4;
   switch (columns) {
     case 16:
@@ -464,6 +506,9 @@ static int launch_ring(const LinearArgs& a, hipStream_t stream) {
     case 64: linear_ring_kernel<T, MT, 2, 2, 2, 3, true, GLU><<<grid, dim3(256), 0, stream>>>(a); break;
     default: linear_ring_kernel<T, MT, 3, 2, 2, 4, true, GLU><<<grid, dim3(256), 0, stream>>>(a);
   }
+  const int status = launch_status();
+  if (status != MVLLM_OK || !a.part) return status;
+  linear_sum_kernel<T><<<dim3((unsigned)(((int64_t)a.M * a.N / 4 + 255) / 256)), dim3(256), 0, stream>>>(a, split.splits);
   return launch_status();
 }
 
@@ -549,12 +594,12 @@ static int linear_check(const void* out, const void* x, const void* w, const voi
 using namespace mvllm;
 
 static int linear_plain(void* out, const void* x, const void* w, const void* bias, int64_t x_row_stride, int M, int N, int K,
-                        int gelu, int dtype, void* stream) {
+                        int gelu, int dtype, void* stream, float* part = nullptr) {
   const int bad = linear_check(out, x, w, bias, x_row_stride, M, N, K, dtype);
   if (bad || M == 0) return bad;
   LinearArgs a{};
   a.out = out; a.x = x; a.w = w; a.bias = bias; a.x_row_stride = x_row_stride; a.M = M; a.N = N; a.K = K;
-  a.gelu = gelu;
+  a.gelu = gelu; a.part = part;
   return dtype == MVLLM_BF16 ? launch_linear_fused<bf16_t>(a, false, (hipStream_t)stream)
                              : launch_linear_fused<f16_t>(a, false, (hipStream_t)stream);
 }
@@ -567,6 +612,19 @@ extern "C" int mvllm_linear_small_m(void* out, const void* x, const void* w, con
 extern "C" int mvllm_linear_small_m_gelu(void* out, const void* x, const void* w, const void* bias, int64_t x_row_stride,
                                          int M, int N, int K, int dtype, void* stream) {
   return linear_plain(out, x, w, bias, x_row_stride, M, N, K, 1, dtype, stream);
+}
+
+extern "C" size_t mvllm_linear_small_m_split_bytes(int M, int N, int K, int64_t x_row_stride) {
+  if (M <= 0 || M > 64 || N <= 0 || N % 16 != 0 || K <= 0 || K % 512 != 0 || ((int64_t)(M - 1) * x_row_stride + K) * 2 > 0xffffffffll) return 0;
+  const int splits = linear_split(M, N, K).splits;
+  return splits < 2 ? 0 : (size_t)splits * M * N * sizeof(float);
+}
+
+extern "C" int mvllm_linear_small_m_split(void* out, const void* x, const void* w, const void* bias, int64_t x_row_stride,
+                                          int M, int N, int K, int gelu, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  const size_t need = mvllm_linear_small_m_split_bytes(M, N, K, x_row_stride);
+  if (need != 0 && (!workspace || !aligned16(workspace) || workspace_bytes < need)) return MVLLM_ERR_WORKSPACE;
+  return linear_plain(out, x, w, bias, x_row_stride, M, N, K, gelu != 0, dtype, stream, need != 0 ? reinterpret_cast<float*>(workspace) : nullptr);
 }
 
 extern "C" int mvllm_linear_small_m_plan(int M, int N, int K, int norm, int glu, int dtype, int* waves) {

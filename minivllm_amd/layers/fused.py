@@ -300,8 +300,8 @@ def linear_small_m_takes(x: torch.Tensor, weight: torch.Tensor, max_rows: int = 
 
 def linear_small_m(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, gelu: bool = False) -> torch.Tensor:
     """``F.linear(x, weight, bias)`` for the few rows of a decode step (the reference's projections,
-    models/qwen3.py:90-94, 118, 121-160, are library GEMMs): one HIP launch in which every wave asks for its whole
-    share of the weights at once, so the call costs about one memory round trip.  x (M <= 64, K), weight (N, K)
+    models/qwen3.py:90-94, 118, 121-160, are library GEMMs): one HIP launch that reads every weight once (two
+    where a long K is cut into parts).  x (M <= 64, K), weight (N, K)
     contiguous, bias (N,) or None, all in one 16-bit dtype; fp32 accumulation.  ``gelu``: the result through the tanh form
     of gelu, rounded once.  Returns (M, N)."""
     _C.require_cuda(x, weight, bias)
@@ -315,9 +315,15 @@ def linear_small_m(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
     n = weight.shape[0]
     out = torch.empty(m, n, dtype=x.dtype, device=x.device)
     lib = _C.load()
-    st = (lib.mvllm_linear_small_m_gelu if gelu else lib.mvllm_linear_small_m)(
-        _ptr(out), _ptr(x), _ptr(weight), _ptr(bias), x.stride(0) if m > 1 else k, m, n, k, _C.dtype_code(x.dtype),
-        _C.current_stream_ptr(x.device))
+    stride = x.stride(0) if m > 1 else k
+    head = (_ptr(out), _ptr(x), _ptr(weight), _ptr(bias), stride, m, n, k)
+    tail = (_C.dtype_code(x.dtype), _C.current_stream_ptr(x.device))
+    need = lib.mvllm_linear_small_m_split_bytes(m, n, k, stride)
+    if need:                                                  # a long K, cut into parts: their sums before they are added up
+        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+        st = lib.mvllm_linear_small_m_split(*head, int(gelu), tail[0], _ptr(workspace), need, tail[1])
+    else:
+        st = (lib.mvllm_linear_small_m_gelu if gelu else lib.mvllm_linear_small_m)(*head, *tail)
     _C.check(st, "linear_small_m")
     return out
 

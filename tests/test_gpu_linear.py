@@ -5,6 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from minivllm_amd import _C
 from minivllm_amd.layers.basic import Linear
 from minivllm_amd.layers.fused import (add_rms_norm, decode_advance, linear_small_m, linear_small_m_takes,
                                        norm_linear_small_m, norm_linear_small_m_takes, silu_and_mul)
@@ -55,6 +56,20 @@ def test_linear_small_m_tile_edges(m, n, k):
     # a unit of the gate or of the up value that rounds the other way, and the two roundings behind them
     slack = (got - want).abs() - 4 * 2.0 ** -8 * (F.silu(gate).abs() + gate.abs() + 1) * (up.abs() + 1)
     assert slack.max().item() <= 2e-3
+
+
+@pytest.mark.parametrize("m", [4, 17, 33, 64])
+@pytest.mark.parametrize("n,k", [(1360, 6656), (2032, 6656), (4112, 12800), (5440, 6144), (1024, 3072)])
+def test_linear_small_m_splits_of_k(m, n, k):
+    """Every column tile with K in parts: parts of unequal length, a last tile that is not full, the most and the fewest columns."""
+    split = _C.load().mvllm_linear_small_m_split_bytes(m, n, k, k + 24) // (4 * m * n)
+    assert split == {1360: 3, 2032: 4, 4112: 3, 5440: 3, 1024: 4 if m > 32 else 0}[n]
+    x, w, b = _case(700 + m, m, n, k, torch.bfloat16, True, stride=k + 24)
+    full = x.float() @ w.float().T + b.float()
+    for gelu in (False, True):
+        want = F.gelu(full, approximate="tanh") if gelu else full
+        err = (linear_small_m(x, w, b, gelu).float() - want).abs() - want.abs() * 2.0 ** -8
+        assert err.max().item() <= 2e-3
 
 
 def test_linear_small_m_strided_rows_and_module_dispatch():
