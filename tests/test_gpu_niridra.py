@@ -448,6 +448,18 @@ def test_router_logits(dtype, rows, n, k):
     assert row_rel(gate_linear(x.to(DEV), w.to(DEV), None, n, 0.0), x.double() @ w.double().T) < 1e-5
 
 
+@pytest.mark.parametrize("rows", [1, 17, 512, 513, 4113])
+@pytest.mark.parametrize("n,k", [(5, 576), (32, 1024), (33, 640), (64, 1088), (65, 2048), (90, 704)])
+def test_router_logits_long_rows(rows, n, k):
+    """Whole rows through LDS: every number of column tiles, 16 and 32 rows, parts of K of unequal length, strided rows."""
+    x, w = torch.randn(rows, k + 40, generator=gen(n)).bfloat16()[:, 8:k + 8], (torch.randn(n, k, generator=gen(k)) * k ** -0.5).bfloat16()
+    b = torch.randn(n, generator=gen(rows))
+    x_gpu = x.to(DEV) if rows == 1 else torch.empty(rows, k + 40, dtype=x.dtype, device=DEV)[:, 8:k + 8].copy_(x)
+    z = x.double() @ w.double().T + b.double()
+    want = torch.cat([z[:, :n // 2], torch.nn.functional.logsigmoid(z[:, n // 2:])], dim=1)
+    assert row_rel(gate_linear(x_gpu, w.to(DEV), b.to(DEV), n // 2, 0.0), want) < 1e-5
+
+
 ROUTERS = [(10, 3, 2, 1), (12, 5, 3, 2), (5, 1, 1, 1), (64, 6, 8, 3), (128, 8, 16, 4), (200, 9, 4, 2), (1000, 12, 50, 7), (6, 6, 1, 1), (16, 2, 16, 3), (7, 4, 7, 5)]
 
 
