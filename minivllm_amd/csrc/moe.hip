@@ -153,8 +153,10 @@ __global__ __launch_bounds__(256) void moe_count_kernel(const PlanArgs a) {
   for (int e = threadIdx.x; e < a.experts; e += 256) a.hist[(int64_t)blockIdx.x * a.experts + e] = count[e];
 }
 
+// A chain of latencies, not bytes: the counts of the blocks, sums over the experts, places.  With the counts' loads one by one and the sums in ten rounds
+// with two barriers each 14 us at 49152 pairs of 64 experts, so 5.9; 1800 pairs 5.1 and 3.5.
 __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
-  __shared__ int32_t total[kMaxExperts + 1], tiles[kMaxExperts + 1], parts[kMaxExperts + 1], cursor[kMaxExperts];
+  __shared__ int32_t total[kMaxExperts + 1], tiles[kMaxExperts + 1], parts[kMaxExperts + 1], cursor[kMaxExperts], of_wave[3][16];
   const int e = threadIdx.x;
   int n = 0, mine = 0;
   if (a.blocks == 1) {                              // counted here
@@ -167,26 +169,41 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
     __syncthreads();
     n = cursor[e];
     __syncthreads();
-  } else if (e < a.experts)
-    for (int b = 0; b < a.blocks; ++b) {
-      if (b == (int)blockIdx.x) mine = n;
-      n += a.hist[(int64_t)b * a.experts + e];
+  } else if (e < a.experts) {
+#pragma unroll 8
+    for (int b = 0; b < a.blocks; ++b) {            // (loads of several blocks under way)
+      const int of_block = a.hist[(int64_t)b * a.experts + e];
+      mine += b < (int)blockIdx.x ? of_block : 0;
+      n += of_block;
     }
-  // inclusive sums over the experts
-  total[e + 1] = n;
+  }
+  // inclusive sums over the experts: within a wave, then over the waves before it
   const bool apart = a.tile_rows == 256 && n % 256 != 0;      // the last tile, not whole, goes behind all whole ones
-  tiles[e + 1] = (n + a.tile_rows - 1) / a.tile_rows - apart;
-  parts[e + 1] = apart;
+  int sums[3] = {n, (n + a.tile_rows - 1) / a.tile_rows - apart, apart};
+  const int lane = e & 63, wave = __builtin_amdgcn_readfirstlane(e >> 6);
+  const bool some = 64 * wave < a.experts;
+  if (some) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int before = __shfl_up(sums[i], o, 64);
+        sums[i] += lane >= o ? before : 0;
+      }
+    if (lane == 63)
+      for (int i = 0; i < 3; ++i) of_wave[i][wave] = sums[i];
+  }
+  __syncthreads();
+  if (some) {
+    for (int w = 0; w < wave; ++w)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) sums[i] += of_wave[i][w];
+    total[e + 1] = sums[0];
+    tiles[e + 1] = sums[1];
+    parts[e + 1] = sums[2];
+  }
   if (e == 0) total[0] = tiles[0] = parts[0] = 0;
   __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    const int x = e + 1 > o ? total[e + 1 - o] : 0, y = e + 1 > o ? tiles[e + 1 - o] : 0, z = e + 1 > o ? parts[e + 1 - o] : 0;
-    __syncthreads();
-    total[e + 1] += x;
-    tiles[e + 1] += y;
-    parts[e + 1] += z;
-    __syncthreads();
-  }
   if (e < a.experts) cursor[e] = total[e] + mine;
   __syncthreads();
   const int end = min((int)(blockIdx.x + 1) * kPlanPairs, a.pairs);
@@ -212,7 +229,7 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
       a.tile_row[t] = total[e] + (t - tiles[e]) * a.tile_rows;
     }
     if (apart) {
-      const int t = tiles[kMaxExperts] + parts[e];
+      const int t = tiles[a.experts] + parts[e];
       a.tile_expert[t] = e;
       a.tile_row[t] = total[e + 1] - n % 256;
     }
