@@ -6,7 +6,7 @@
 // operand's lanes are sixteen different rows).  Hence two kernels:
 //   linear_rows_kernel (very few rows): weights and x straight into registers, eight rows x 128 bytes per load.
 //   linear_ring_kernel (more rows): W and x through a ring of tiles in LDS, copied as whole 128-byte lines.
-// Both read a weight once.  A sum's order depends on (M, N, K), not on what follows the product; a long K with few columns is cut into
+// Both read a weight once.  A sum's order depends on (M, N, K) and, from kStreamBytes of weights on, on the column; a long K with few columns is cut into
 // parts where the caller brings room for their sums (linear_split).
 // mvllm_norm_linear_small_m is the same product with the launches around it folded in: the residual add + RMSNorm in
 // front of the layer's first projections (src/myvllm/models/qwen3.py:197-212 through layers/layernorm.py:9-28) as
@@ -206,13 +206,17 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
   });
   const int steps_all = a.K / (64 * SK), per_split = (steps_all + (int)gridDim.y - 1) / (int)gridDim.y, step0 = per_split * (int)blockIdx.y;
   const int steps = max(min(steps_all - step0, per_split), 0);      // of this workgroup's share of K
+  // Rows a multiple of 4 KB long start in the same channel of the L2 and of the memory: workgroups that walk K in step would all read
+  // from a few of them, so neighbours on an XCD start a quarter of the steps apart.  us at 16 / 33 / 64 rows without and with: 24576 x 4096 with GLU 34.2 /
+  // 41.8 / 45.9 and 32.3 / 41.0 / 39.0, 6144 x 4096 14.3 / 14.9 / 17.2 and 12.4 / 13.5 / 16.6, 12288 x 2048 with GLU 13.1 / 13.8 / 15.5 and 12.5 / 13.0 / 14.7.
+  const int turn = NT && a.K % 2048 == 0 ? (int)(blockIdx.x >> 3 & 3) * (steps >> 2) : 0;
   const uint32_t lds0 = lds_address(lds) + sk * kPanel + sc * 1024;
   auto copy = [&](int step, int buffer) __attribute__((always_inline)) {
     const bool live = step < steps;
     const v4i x_rows = make_rsrc(reinterpret_cast<const char*>(a.x), live ? x_bytes : 0u);
     const v4i w_rows = make_rsrc(w0, live ? w_bytes : 0u);
     const v4i up_rows = GLU ? make_rsrc(w0 + (int64_t)out_cols * row_bytes, live ? w_bytes : 0u) : w_rows;
-    const uint32_t at = live ? (uint32_t)(step0 + step) * (SK * 128) : 0u, base = lds0 + buffer * kStage;
+    const uint32_t at = live ? (uint32_t)(step0 + (step < steps - turn ? step + turn : step + turn - steps)) * (SK * 128) : 0u, base = lds0 + buffer * kStage;
     static_for<kCopies>([&](auto I) {
       constexpr int i = decltype(I)::value;
       if constexpr (i < 2 * CT) dma16_to_lds_at<i * SC * 1024, NT>(GLU && ((i * SC + sc) & 1) ? up_rows : w_rows, from[i], at, base);

@@ -432,6 +432,15 @@ __device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, 
   return tile < whole + rest;
 }
 
+// Step of K that a workgroup starts with; it comes round to the ones before it at its end.  Rows a multiple of 4 KB long start in the same channel
+// of the L2 and of the memory, and workgroups that walk K in step read the same place of all rows at a time: a few channels serve
+// everybody.  Four groups of experts start a quarter of K apart and the weight tiles of an expert a step apart: x stays shared, and the
+// order of a sum depends on expert and column alone.  us from the first step on and so: 300 rows, top 6 of 64 experts of 1536 x 2048 84 / 68, 600
+// rows 115 / 94, 8192 rows 354 / 336; of 2560 x 4096, 8192 rows 1390 / 1345, 32 rows 211 / 209.  Other rows (K of 768 and 1280): no difference.
+__device__ __forceinline__ int first_step(const ExpertLinearArgs& a, int e, int n_tile, int steps) {
+  return a.K % 2048 == 0 ? ((e & 3) * (steps >> 2) + n_tile) % steps : 0;
+}
+
 // many: 128 weight rows x 32 kRows sorted rows per workgroup, four waves on v_mfma_f32_32x32x16_bf16.  Weights are the row
 // operand and x the column operand, so that a lane ends with runs of four outputs of one row.  Steps of 64 along K through a
 // ring of buffers in LDS that copies of later steps fill during this one; a row's eight 16-byte chunks trade places by half
@@ -440,7 +449,7 @@ __device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, 
 // wave has 64 x 32, the small tile leaves LDS for three buffers of two workgroups per CU (72 KB of copies in flight or use each),
 // and weights, read once by one workgroup, pass the caches by (nt).  900 pairs, 64 experts of 1536 x 2048 and 2048 x 768,
 // weights from memory: 95 + 41 us as 128 x 128 tiles, 72 + 35 us (5.6 and 5.8 TB/s) as these; without nt 80 + 40, six buffers of one
-// workgroup 70 + 41.
+// workgroup 70 + 41 (all before first_step).
 template <int kGlu, int kRows>
 __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLinearArgs a) {
   constexpr int kStages = kRows == 4 ? 2 : 3, kTile = 128, kK = 64;
@@ -470,7 +479,7 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
     const uint32_t xr = (uint32_t)(a.per_token ? a.sorted_pair[at] / a.per_token : at);
     from_x[i] = (xr * (uint32_t)a.x_stride + 8u * p) * 2u;
   }
-  const int steps = a.K / kK;
+  const int steps = a.K / kK, turn = first_step(a, e, n_tile, steps);
   const uint32_t lds_wave = lds_address(lds) + 1024 * wave;
   auto copy = [&](int step, int buffer) __attribute__((always_inline)) {      // past the last step nothing is read, and the count stays
     v4i w = w_rows, x = x_rows;
@@ -478,7 +487,7 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
       w[2] = step < steps ? w[2] : 0;
       x[2] = step < steps ? x[2] : 0;
     }
-    const uint32_t at = (uint32_t)step * (2 * kK), base = lds_wave + buffer * kStage;
+    const uint32_t at = (uint32_t)(step < steps - turn ? step + turn : step + turn - steps) * (2 * kK), base = lds_wave + buffer * kStage;
     static_for<4>([&](auto I) { dma16_to_lds_at<4096 * decltype(I)::value, kRows == 2>(w, from_w[decltype(I)::value], at, base); });
     static_for<kRows>([&](auto I) { dma16_to_lds_at<kW + 4096 * decltype(I)::value>(x, from_x[decltype(I)::value], at, base); });
   };
@@ -573,17 +582,18 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
   }
   constexpr int kX = 3 * kStage;                    // where x begins
   const uint32_t lds_wave = lds_address(lds) + 1024 * wave;
-  const int steps = a.K / kK;
+  const int steps = a.K / kK, turn = first_step(a, e, n_tile, steps);
+  auto k_of = [&](int step) __attribute__((always_inline)) { return (uint32_t)(step < steps - turn ? step + turn : step + turn - steps) * (2 * kK); };
   // copy i of eight of a step's operand; past the last step nothing is read (the buffer is not used again)
   auto copy_w = [&](auto I, int step, uint32_t buffer) __attribute__((always_inline)) {
     v4i rows = w_rows;
     rows[2] = step < steps ? rows[2] : 0;
-    dma16_to_lds_at<4096 * decltype(I)::value>(rows, from_w[decltype(I)::value], (uint32_t)step * (2 * kK), lds_wave + buffer);
+    dma16_to_lds_at<4096 * decltype(I)::value>(rows, from_w[decltype(I)::value], k_of(step), lds_wave + buffer);
   };
   auto copy_x = [&](auto I, int step) __attribute__((always_inline)) {
     v4i rows = x_rows;
     rows[2] = step < steps ? rows[2] : 0;
-    dma16_to_lds_at<4096 * decltype(I)::value>(rows, from_x[decltype(I)::value], (uint32_t)step * (2 * kK), lds_wave + kX + (step & 1) * kStage);
+    dma16_to_lds_at<4096 * decltype(I)::value>(rows, from_x[decltype(I)::value], k_of(step), lds_wave + kX + (step & 1) * kStage);
   };
   const int wn = wave & 1, wm = wave >> 1;
   const int sw = (l32 >> 1) & 7;
