@@ -32,6 +32,7 @@ struct LinearArgs {
   float eps;
   int row_tiles;          // norm: tiles of 16 rows, a workgroup per column tile each
   int gelu;               // plain product only: the result through the tanh form of gelu
+  int part_steps;         // steps of the ring in a part of K
   float* part;            // plain product only: partial sums [gridDim.y, M, N] of the splits of K, or null
 };
 
@@ -204,8 +205,7 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
     if constexpr (i < 2 * CT) from[i] = (uint32_t)min(8 * (GLU ? b >> 1 : b) + r8, left - 1) * row_bytes + piece;
     else from[i] = (uint32_t)min(8 * (b - WB) + r8, a.M - 1) * (uint32_t)a.x_row_stride * 2u + piece;
   });
-  const int steps_all = a.K / (64 * SK), per_split = (steps_all + (int)gridDim.y - 1) / (int)gridDim.y, step0 = per_split * (int)blockIdx.y;
-  const int steps = max(min(steps_all - step0, per_split), 0);      // of this workgroup's share of K
+  const int step0 = a.part_steps * (int)blockIdx.y, steps = min(a.K / (64 * SK) - step0, a.part_steps);    // of this workgroup's part of K
   // Rows a multiple of 4 KB long start in the same channel of the L2 and of the memory: workgroups that walk K in step would all read
   // from a few of them, so neighbours on an XCD start a quarter of the steps apart.  us at 16 / 33 / 64 rows without and with: 24576 x 4096 with GLU 34.2 /
   // 41.8 / 45.9 and 32.3 / 41.0 / 39.0, 6144 x 4096 14.3 / 14.9 / 17.2 and 12.4 / 13.5 / 16.6, 12288 x 2048 with GLU 13.1 / 13.8 / 15.5 and 12.5 / 13.0 / 14.7.
@@ -492,10 +492,11 @@ static int launch_rows(const LinearArgs& a, hipStream_t stream) {
 }
 
 template <typename T, int MT, bool GLU>
-static int launch_ring(const LinearArgs& a, hipStream_t stream) {
+static int launch_ring(LinearArgs a, hipStream_t stream) {
   const bool stream_weights = (int64_t)a.N * a.K * 2 >= kStreamBytes;
   const LinearSplit split = a.part ? linear_split(a.M, a.N, a.K) : LinearSplit{ring_columns(a.M, a.N), 1};
-  const int columns = split.columns;
+  const int columns = split.columns, steps = a.K / (columns == 16 ? 256 : 128);
+  a.part_steps = (steps + split.splits - 1) / split.splits;
   const dim3 grid((unsigned)((a.N + columns - 1) / columns), (unsigned)split.splits);
   constexpr int S = MT > 2 ? 3 : 4;
   switch (columns) {
