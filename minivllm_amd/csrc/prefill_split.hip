@@ -435,10 +435,14 @@ static int ranges_of(int max_kv_len, int range_tiles) { return ((max_kv_len + 63
 // 6 us longer until then, and its longest item decides when there are few.  So this form takes what fits on the chip about at once, two
 // workgroups per CU, four heads per workgroup (whose row tiles are half as long, and read the keys twice as often) somewhat less.  us on
 // either side, bf16, without the store: 16 heads over 8 kv heads of 128, two prompts of 270 rows 20.5 -> 14.5, one of 3000 67 -> 60, of 4000
-// (512 workgroups) 92 -> 82, ten of 406 (488) 32 -> 30, two of 2330 (592) 66 -> 68,
+// (512 workgroups) 92 -> 82, ten of 406 (488) 32 -> 30, two of 2330 (592) 66 -> 68, nine of 463 (592) 30 -> 33,
 // seven of 965 (900) 51 -> 56; 32 heads, one of 1500 (384) 38.6 -> 35.7, four of 875 (904) 42 -> 51.  At head_dim
 // 64 the other form is this kernel over its banded order, which pays for packed batches as soon as their tiles differ (3500 rows,
-// 448 workgroups: 30 us, here 33) and costs cached ones its padding (1000 rows behind as many 26 -> 24).
+// 448 workgroups: 30 us, here 33) and costs cached ones its padding (1000 rows behind as many 26 -> 24).  What stays there though it is within
+// these bounds, us there and here: two sequences in place of one or of several from 420 workgroups to two per CU (3650 rows of 16 heads 53.4 /
+// 54.7); 32 heads of 64 at 321 to 400 (1244 rows of up to 724 keys 21.0 / 22.0: no place of its bands is empty); a few rows at head_dim 64,
+// where placing the bands costs nothing (23 rows 8.8 / 9.5; from 5 sequences of 32 heads and 10 of 16 on 12.3 / 11.0); 200 workgroups with more
+// than 7000 keys, whose ranges the other form cuts (121 / 128).
 // Which range: a tile takes a workgroup 0.9 us (0.8 at head_dim 64), workgroups of 0.6 of the longest sequence's tiles each fill 256 CUs;
 // a range brings every row's fp32 partial result into memory and back, about 0.7 of the ranges are there on average.  Batches of more
 // than 192 workgroups gain nothing that the partial results do not cost (1500 rows behind 1500, 32 heads, 376 workgroups: whole 72, two
@@ -449,10 +453,15 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
   if (!ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype)) return 0;
   const int group = num_heads / num_kv_heads, bm = rows_of_tile(group);
   const int64_t wgs = (total_q_tokens / bm + num_seqs) * ((int64_t)num_heads * bm / 128), tiles = (max_kv_len + 63) / 64;
-  const int limit = head_dim == 64 ? (block_size > 0 ? 768 : tiles >= 16 ? 384 : 0) : group % 4 != 0 ? (tiles >= 16 ? 512 : 640) : tiles >= 12 ? 384 : 320;
+  const bool four = group % 4 == 0;
+  const int limit = head_dim == 64 ? (block_size > 0 ? 768 : tiles >= 16 && !four ? 384 : 0)
+                    : !four        ? (tiles >= 16 ? 512 : tiles >= 7 ? 580 : 640)
+                                   : tiles >= 12 ? 384 : 300;
   if (wgs > limit) return 0;
+  if (!four && num_seqs == 2 && wgs > 420 && wgs < 500) return 0;
+  if (four && head_dim == 64 && tiles >= 7 && tiles < 16 && wgs > 320 && wgs <= 400) return 0;
   int64_t p = (tiles + 1) / 2 * 2;
-  if (wgs > 192) return (int)p;
+  if (wgs > 192) return four && head_dim == 128 && tiles > 112 ? 0 : (int)p;
   const float per_tile = head_dim == 64 ? 0.8f : 0.9f, per_range = 0.3f + 0.7f * 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f;
   float best = 3.f;
   for (int64_t x = 6; x < tiles; x += 2) {
@@ -464,7 +473,7 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
       p = x;
     }
   }
-  return (int)p;
+  return head_dim == 64 && p >= tiles && wgs < (four ? 48 : 80) ? 0 : (int)p;
 }
 
 extern "C" size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim, int range_tiles) {
