@@ -13,6 +13,8 @@ Additions with no counterpart in the reference: the INT8 KV-cache operators
 """
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 import torch.nn as nn
 
@@ -221,16 +223,25 @@ def flash_attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, c
     return output
 
 
+@lru_cache(maxsize=256)
+def _prefill_ranges_plan(lib, num_seqs, total, max_seqlen, num_heads, num_kv_heads, head_dim, block_size, code):
+    """(key tiles per range, workspace bytes) of a batch of these sizes, (0, 0): not over ranges.  Every layer of a step asks again."""
+    tiles = lib.mvllm_prefill_ranges_plan(num_seqs, total, max_seqlen, num_heads, num_kv_heads, head_dim, block_size, code)
+    return tiles, lib.mvllm_prefill_ranges_workspace_bytes(total, max_seqlen, num_heads, head_dim, tiles) if tiles else 0
+
+
 def _prefill_ranges(lib, output, q, k, v, block_tables, cu_seqlens_q, cu_seqlens_k, num_seqs, max_seqlen, scale, num_heads,
                     num_kv_heads, head_dim, block_size, num_blocks, sink) -> bool:
     """Runs the call over key ranges if the library's plan says so."""
     code = _C.dtype_code(q.dtype)
-    tiles = lib.mvllm_prefill_ranges_plan(num_seqs, q.shape[0], max_seqlen, num_heads, num_kv_heads, head_dim, block_size, code)
-    need = lib.mvllm_prefill_ranges_workspace_bytes(q.shape[0], max_seqlen, num_heads, head_dim, tiles) if tiles else 0
-    if not tiles or need > STAGED_PREFILL_MAX_BYTES or not scale > 0 or any(t.data_ptr() % 16 for t in (output, q, k, v)):
+    tiles, need = _prefill_ranges_plan(lib, num_seqs, q.shape[0], max_seqlen, num_heads, num_kv_heads, head_dim, block_size, code)
+    if not tiles or need > STAGED_PREFILL_MAX_BYTES or not scale > 0:
+        return False
+    o_at, q_at, k_at, v_at = output.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr()
+    if (o_at | q_at | k_at | v_at) % 16:
         return False
     workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None      # none: one range
-    st = lib.mvllm_prefill_ranges(_ptr(output), _ptr(q), _ptr(k), _ptr(v), 0 if block_tables is None else _ptr(block_tables),
+    st = lib.mvllm_prefill_ranges(o_at, q_at, k_at, v_at, 0 if block_tables is None else _ptr(block_tables),
                                   0 if block_tables is None else block_tables.shape[1], _ptr(cu_seqlens_q),
                                   0 if cu_seqlens_k is None else _ptr(cu_seqlens_k), num_seqs, q.shape[0], max_seqlen, num_heads,
                                   num_kv_heads, head_dim, block_size, num_blocks, float(scale),
