@@ -101,7 +101,7 @@ class RaggedStep:
 
 BLOCK_ROWS = 64                # rows per block of a recurrence's block form: segments are whole blocks
 FILL_WORKGROUPS = 512          # segments are made shorter until there are this many workgroups ...
-# ... but not shorter than this, and portions below two of them stay whole: the states' own pass, two launches and their way through
+# ... but not shorter than this, and portions of a few of them stay whole (see _segments): the states' own pass, two launches and their way through
 # memory have to pay.  One portion of 700 rows, 16 heads of 128 x 256: 43 us (256: 55, 64: 40), 2000 rows, 8 heads: 50 (60, 57), 200
 # rows in two segments 36 against 31 whole.
 MIN_SEGMENT_ROWS = 128
@@ -114,10 +114,15 @@ def _segments(lens, cu, units):
     length = total
     if long_entries and units and len(long_entries) * units < FILL_WORKGROUPS // 2:
         length = max(-(-total * units // (FILL_WORKGROUPS * BLOCK_ROWS)) * BLOCK_ROWS, MIN_SEGMENT_ROWS)
+    # the rows from which cutting pays: its two more launches take the longer the more there is to combine.  us whole and cut, memory of 128 x 256:
+    # 8 heads, one portion of 256 rows 34.5 / 35.4, of 300 37 / 35.5; two of 256 35 / 38.5, of 384 44 / 41; eight of 256 42 / 55, of 384 54 / 61, of
+    # 512 69 / 67.5
+    busy = len(long_entries) * (units or 0)
+    least = MIN_SEGMENT_ROWS * (4 if busy <= 16 else 5 if busy <= 64 else 7) // 2
     out = []
     for e in long_entries:
         n, at = int(lens[e]), int(cu[e])
-        pieces = max(-(-n // length), 1) if n >= 2 * MIN_SEGMENT_ROWS else 1
+        pieces = max(-(-n // length), 1) if n > least else 1
         size = -(-n // (pieces * BLOCK_ROWS)) * BLOCK_ROWS
         cuts = list(range(0, n, size)) + [n]
         for i, (lo, hi) in enumerate(zip(cuts, cuts[1:])):
