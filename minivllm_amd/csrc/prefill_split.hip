@@ -428,7 +428,7 @@ static bool ranges_shape_ok(int num_seqs, int64_t total_q, int max_kv_len, int n
   return total_q <= ((int64_t)1 << 24);
 }
 static int rows_of_tile(int group) { return 32 * (group % 4 == 0 ? 1 : group % 2 == 0 ? 2 : 4); }
-static int ranges_of(int max_kv_len, int range_tiles) { return ((max_kv_len + 63) / 64 + range_tiles - 1) / range_tiles; }
+static int64_t ranges_of(int64_t max_kv_len, int64_t range_tiles) { return ((max_kv_len + 63) / 64 + range_tiles - 1) / range_tiles; }
 
 // The range for a batch of these sizes, at least every sequence's tiles where none is cut; 0: the other kernels.
 // Which kernel: the two-group kernel holds one workgroup per CU and runs faster once it has started (906 TFLOP/s against 680), but takes
@@ -452,7 +452,7 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
                                          int head_dim, int block_size, int dtype) {
   if (!ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype)) return 0;
   const int group = num_heads / num_kv_heads, bm = rows_of_tile(group);
-  const int64_t wgs = (total_q_tokens / bm + num_seqs) * ((int64_t)num_heads * bm / 128), tiles = (max_kv_len + 63) / 64;
+  const int64_t wgs = (total_q_tokens / bm + num_seqs) * ((int64_t)num_heads * bm / 128), tiles = ranges_of(max_kv_len, 1);
   const bool four = group % 4 == 0;
   const int limit = head_dim == 64 ? (block_size > 0 ? 768 : tiles >= 16 && !four ? 384 : 0)
                     : !four        ? (tiles >= 16 ? 512 : tiles >= 7 ? 580 : 640)
@@ -464,9 +464,9 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
   if (wgs > 192) return four && head_dim == 128 && tiles > 112 ? 0 : (int)p;
   const float per_tile = head_dim == 64 ? 0.8f : 0.9f, per_range = 0.3f + 0.7f * 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f;
   float best = 3.f;
-  for (int64_t x = 6; x < tiles; x += 2) {
-    const int64_t n = (tiles + x - 1) / x;
-    if (n > kMaxRanges) continue;
+  for (int64_t most = kMaxRanges; most > 1; --most) {       // the shortest range that gives so many
+    const int64_t even = ((tiles + most - 1) / most + 1) / 2 * 2, x = even < 6 ? 6 : even, n = (tiles + x - 1) / x;
+    if (x >= tiles) continue;
     const float gain = per_tile * ((float)tiles - fmaxf((float)x, 0.6f * (float)(wgs * tiles) / 256.f)) - 4.f - per_range * (float)n;
     if (gain > best) {
       best = gain;
@@ -478,7 +478,7 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
 
 extern "C" size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim, int range_tiles) {
   if (total_q_tokens <= 0 || max_kv_len <= 0 || num_heads <= 0 || head_dim <= 0 || range_tiles <= 0) return 0;
-  const int ranges = ranges_of(max_kv_len, range_tiles);
+  const int64_t ranges = ranges_of(max_kv_len, range_tiles);
   return ranges < 2 ? 0 : (size_t)ranges * total_q_tokens * num_heads * (head_dim + 1) * sizeof(float);
 }
 
@@ -496,8 +496,8 @@ extern "C" int mvllm_prefill_ranges(void* out, const void* q, const void* k, con
   if (!out || !q || !k || !v || !cu_seqlens_q || (paged && (!block_tables || !cu_seqlens_k))) return MVLLM_ERR_NULL_POINTER;
   if (range_tiles % 2 != 0 || !ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype))
     return MVLLM_ERR_UNSUPPORTED;
-  const int ranges = ranges_of(max_kv_len, range_tiles);
-  if (ranges > kMaxRanges) return MVLLM_ERR_UNSUPPORTED;
+  if (ranges_of(max_kv_len, range_tiles) > kMaxRanges) return MVLLM_ERR_UNSUPPORTED;
+  const int ranges = (int)ranges_of(max_kv_len, range_tiles);
   if (!aligned16(q) || !aligned16(out) || !aligned16(k) || !aligned16(v)) return MVLLM_ERR_MISALIGNED;
   if (ranges > 1 && (!workspace || !aligned16(workspace)) ||
       workspace_bytes < mvllm_prefill_ranges_workspace_bytes(total_q_tokens, max_kv_len, num_heads, head_dim, range_tiles))

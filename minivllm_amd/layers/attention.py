@@ -207,7 +207,8 @@ def flash_attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, c
     num_seqs = cu_seqlens.shape[0] - 1
     _warn_if_generic("prefill", num_heads, num_kv_heads, head_dim, 0, q.dtype, False)
     lib = _C.load()
-    if max_seqlen is not None and _prefill_ranges(lib, output, q, k, v, None, cu_seqlens, None, num_seqs, int(max_seqlen), scale,
+    # (a bound may be loose, up to the model's longest sequence: ranges that nobody reaches would still cost a merge)
+    if max_seqlen is not None and _prefill_ranges(lib, output, q, k, v, None, cu_seqlens, None, num_seqs, min(int(max_seqlen), total), scale,
                                                   num_heads, num_kv_heads, head_dim, 0, 0, sink):
         return output
     if sink is not None:
@@ -311,8 +312,8 @@ def flash_attention_prefill_paged(q: torch.Tensor, k_cache: torch.Tensor, v_cach
             return output
     if max_seqlen_k is not None and int(max_seqlen_k) > 0 and q.dtype != torch.float32:
         if key_splits is None and _prefill_ranges(lib, output, q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, num_seqs,
-                                                  int(max_seqlen_k), scale, num_heads, num_kv_heads, head_dim, block_size,
-                                                  k_cache.shape[0], sink):
+                                                  min(int(max_seqlen_k), block_tables.shape[1] * block_size), scale, num_heads,
+                                                  num_kv_heads, head_dim, block_size, k_cache.shape[0], sink):
             return output
         code = _C.dtype_code(q.dtype)
         splits = key_splits

@@ -68,6 +68,17 @@ def test_host_only_entry_points():
     assert lib.mvllm_paged_decode_workspace_bytes(256, 32, 128, 2048, 16) == 256 * 32 * 32 * 130 * 4
 
 
+def test_prefill_ranges_take_any_bound():
+    """A bound of the keys that is no bound at all is still one: counts do not overflow, the range grows with it."""
+    lib = _lib().load()
+    for keys in (4096, 2 ** 20, 2 ** 31 - 64, 2 ** 31 - 1):
+        tiles, per = -(-keys // 64), lib.mvllm_prefill_ranges_plan(10, 500, keys, 16, 8, 128, 0, 1)
+        ranges = -(-tiles // per)
+        assert per % 2 == 0 and 2 <= ranges <= 64
+        assert lib.mvllm_prefill_ranges_workspace_bytes(500, keys, 16, 128, per) == ranges * 500 * 16 * 129 * 4
+        assert lib.mvllm_prefill_ranges_workspace_bytes(500, keys, 16, 128, 6) == -(-tiles // 6) * 500 * 16 * 129 * 4
+
+
 def test_prefill_split_plan_is_host_arithmetic():
     """When a paged prefill is cut over its keys: few query tiles, at least 4096 keys, a shape the split form takes;
     and the workspace holds the ranges' tables, partial results and denominators."""

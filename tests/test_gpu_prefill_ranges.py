@@ -60,6 +60,22 @@ def test_prefill_over_key_ranges_sinks_and_empty_sequences(lengths):
     assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
 
 
+@pytest.mark.parametrize("bound", [300, 32768, 2 ** 31 - 1, 2 ** 40])
+def test_loose_bounds_cost_no_ranges(monkeypatch, bound):
+    """The keys of a batch bound the caller's own bound: packed rows, or the places of the block tables."""
+    c, asked, plan = make_paged_prefill_case(9, [300, 120], [200, 0], 8, 4, 128, 16, dtype=torch.bfloat16), [], attention._prefill_ranges_plan
+    monkeypatch.setattr(attention, "_prefill_ranges_plan", lambda *a: asked.append(a[3]) or plan(*a))
+    on = {n: c[n].to(DEV) for n in ("q", "k", "v", "q_new", "k_cache", "v_cache", "block_tables", "cu_q", "cu_k")}
+    got = attention.flash_attention_prefill(on["q"], on["k"], on["v"], on["cu_k"], 128 ** -0.5, 8, 4, 128, max_seqlen=bound)
+    paged = attention.flash_attention_prefill_paged(on["q_new"], on["k_cache"], on["v_cache"], on["block_tables"], on["cu_q"], on["cu_k"],
+                                                    128 ** -0.5, 8, 4, 128, 16, min(bound, 2 ** 31 - 1))
+    assert asked == [min(bound, 420), min(bound, 16 * c["block_tables"].shape[1])]
+    want = attention.flash_attention_prefill(on["q"], on["k"], on["v"], on["cu_k"], 128 ** -0.5, 8, 4, 128)
+    for a, b in ((got, want), (paged.cpu(), want.cpu()[c["new_rows"]])):
+        mx, mean = error_stats(a.cpu(), b.cpu().float())
+        assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
+
+
 def test_prefill_ranges_plan_and_rejections():
     lib = _C.load()
     bf, f32 = _C.dtype_code(torch.bfloat16), _C.dtype_code(torch.float32)
