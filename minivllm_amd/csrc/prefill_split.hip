@@ -430,19 +430,41 @@ static bool ranges_shape_ok(int num_seqs, int64_t total_q, int max_kv_len, int n
 static int rows_of_tile(int group) { return 32 * (group % 4 == 0 ? 1 : group % 2 == 0 ? 2 : 4); }
 static int64_t ranges_of(int64_t max_kv_len, int64_t range_tiles) { return ((max_kv_len + 63) / 64 + range_tiles - 1) / range_tiles; }
 
+// The busiest CU of a batch of equal sequences, in longest tiles: workgroup i of `wgs`, heaviest first within a sequence, lands on CU i
+// mod 256 and costs 1 - fresh (place in its sequence), `fresh` being the share of the keys that the rows bring themselves.
+static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
+  const float of_seq = (float)wgs / (float)num_seqs;
+  float most = 1.f;
+  for (int64_t cu = 0; cu + 256 < wgs && cu < 256; ++cu) {
+    float sum = 0.f;
+    for (int64_t i = cu; i < wgs; i += 256) sum += 1.f - fresh * (fmodf((float)i, of_seq) / of_seq);
+    most = fmaxf(most, sum);
+  }
+  return most;
+}
+
 // The range for a batch of these sizes, at least every sequence's tiles where none is cut; 0: the other kernels.
 // Which kernel: the two-group kernel holds one workgroup per CU and runs faster once it has started (906 TFLOP/s against 680), but takes
 // 6 us longer until then, and its longest item decides when there are few.  So this form takes what fits on the chip about at once, two
 // workgroups per CU, four heads per workgroup (whose row tiles are half as long, and read the keys twice as often) somewhat less.  us on
 // either side, bf16, without the store: 16 heads over 8 kv heads of 128, two prompts of 270 rows 20.5 -> 14.5, one of 3000 67 -> 60, of 4000
 // (512 workgroups) 92 -> 82, ten of 406 (488) 32 -> 30, two of 2330 (592) 66 -> 68, nine of 463 (592) 30 -> 33,
-// seven of 965 (900) 51 -> 56; 32 heads, one of 1500 (384) 38.6 -> 35.7, four of 875 (904) 42 -> 51.  At head_dim
-// 64 the other form is this kernel over its banded order, which pays for packed batches as soon as their tiles differ (3500 rows,
-// 448 workgroups: 30 us, here 33) and costs cached ones its padding (1000 rows behind as many 26 -> 24).  What stays there though it is within
-// these bounds, us there and here: two sequences in place of one or of several from 420 workgroups to two per CU (3650 rows of 16 heads 53.4 /
-// 54.7); 32 heads of 64 at 321 to 400 (1244 rows of up to 724 keys 21.0 / 22.0: no place of its bands is empty); a few rows at head_dim 64,
-// where placing the bands costs nothing (23 rows 8.8 / 9.5; from 5 sequences of 32 heads and 10 of 16 on 12.3 / 11.0); 200 workgroups with more
-// than 7000 keys, whose ranges the other form cuts (121 / 128).
+// seven of 965 (900) 51 -> 56; 32 heads, one of 1500 (384) 38.6 -> 35.7, four of 875 (904) 42 -> 51.
+// The two workgroups of a CU are the i-th and the (i + 256)-th.  Of a single sequence that is a heavy and a light one; of several equal
+// ones it can be two of the heaviest, and the longer the tiles, the less the later start of the other kernel counts.  us there and here, and
+// busiest_cu: two prompts of 1496 (384 workgroups) 36.6 / 34.8 1.67, of 1656 (424) 38.8 / 40.2 1.79, of 1976 (504) 47.3 / 51.8 1.98, three of 976
+// (384) 28.2 / 30.6 2.0, of 1296 (504) 36.6 / 34.5 1.52; behind cached halves three of 794 rows (320) 42.7 / 40.6 1.80, four of
+// 588 (320) 34.3 / 36.6 1.90; behind 95 %, nine of 128 (32 heads, 360) 59 / 71 2.0.  Uneven ones meet by chance: 3300 rows of two
+// (60 and 40 %) 44.2 / 38.3, of three 43.9 / 34.6.  Cached batches do not tell whether they are even and count as if.  (Above 112 tiles the
+// other form cuts its keys too, and loses on either side of the line.)
+// At head_dim 64 the other form is this kernel over its banded order, 256 rows of a sequence at a time, the heaviest first: it pays for
+// packed batches as soon as their tiles differ (3500 rows, 448 workgroups: 30 us, here 33).  Cached ones pay its empty places, which fill the
+// chip's 512 the sooner, and gain from its order where they have more than one workgroup per CU and still fit: us there and here, 32
+// heads, four of 418 rows (512 places) of 758 keys 17.3 / 19.1, of 1142 23.5 / 25.0, of 518 (768) 26.5 / 20.2 and 38.3 / 30.3; of 118 (256 and
+// 240 workgroups) 15.2 / 14.9; eight of 93 (512 and 192) 19.1 / 15.8; from 30 tiles on a start counts less: 37.5 / 37.3.
+// A few rows at head_dim 64 stay there, where placing the bands costs nothing (23 rows 8.8 / 9.5; from 5 sequences of 32 heads and 10 of 16
+// on 12.3 / 11.0), and so do 200 workgroups with more than 7000 keys, whose ranges the other form cuts (four heads of 128 121 / 128, of 64
+// 88 / 97, two of 64 80 / 96).
 // Which range: a tile takes a workgroup 0.9 us (0.8 at head_dim 64), workgroups of 0.6 of the longest sequence's tiles each fill 256 CUs;
 // a range brings every row's fp32 partial result into memory and back, about 0.7 of the ranges are there on average.  Batches of more
 // than 192 workgroups gain nothing that the partial results do not cost (1500 rows behind 1500, 32 heads, 376 workgroups: whole 72, two
@@ -452,20 +474,27 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
                                          int head_dim, int block_size, int dtype) {
   if (!ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype)) return 0;
   const int group = num_heads / num_kv_heads, bm = rows_of_tile(group);
-  const int64_t wgs = (total_q_tokens / bm + num_seqs) * ((int64_t)num_heads * bm / 128), tiles = ranges_of(max_kv_len, 1);
-  const bool four = group % 4 == 0;
-  const int limit = head_dim == 64 ? (block_size > 0 ? 768 : tiles >= 16 && !four ? 384 : 0)
+  const int64_t slices = (int64_t)num_heads * bm / 128, wgs = (total_q_tokens / bm + num_seqs) * slices, tiles = ranges_of(max_kv_len, 1);
+  const bool four = group % 4 == 0, paged = block_size > 0;
+  const int limit = head_dim == 64 ? (paged ? 768 : tiles >= 16 && !four ? 384 : 0)
                     : !four        ? (tiles >= 16 ? 512 : tiles >= 7 ? 580 : 640)
                                    : tiles >= 12 ? 384 : 300;
   if (wgs > limit) return 0;
-  if (!four && num_seqs == 2 && wgs > 420 && wgs < 500) return 0;
-  if (four && head_dim == 64 && tiles >= 7 && tiles < 16 && wgs > 320 && wgs <= 400) return 0;
+  // were all sequences as long as their mean: workgroups that have rows, the other form's places (10 % of the rows more, for those that are longer)
+  const int64_t even = num_seqs * ((total_q_tokens + (int64_t)num_seqs * bm - 1) / ((int64_t)num_seqs * bm)) * slices;
+  const int64_t places = num_seqs * ((total_q_tokens * 11 / 10 + (int64_t)num_seqs * 256 - 1) / ((int64_t)num_seqs * 256)) * (256 / bm) * slices;
+  const float fresh = fminf(1.f, (float)total_q_tokens / ((float)num_seqs * (float)max_kv_len));
+  if (head_dim == 64) {
+    if (paged && num_seqs <= 8 && even > 256 && places <= 512 && tiles < 30) return 0;
+  } else if (num_seqs > 1 && even > 272 && tiles >= 16 && (paged ? tiles <= 112 : fresh >= 0.87f)) {
+    if (busiest_cu(even, num_seqs, fresh) > (paged ? 1.85f : 1.75f)) return 0;
+  }
   int64_t p = (tiles + 1) / 2 * 2;
-  if (wgs > 192) return four && head_dim == 128 && tiles > 112 ? 0 : (int)p;
+  if (wgs > 192) return (four || head_dim == 64) && tiles > 112 ? 0 : (int)p;
   const float per_tile = head_dim == 64 ? 0.8f : 0.9f, per_range = 0.3f + 0.7f * 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f;
   float best = 3.f;
   for (int64_t most = kMaxRanges; most > 1; --most) {       // the shortest range that gives so many
-    const int64_t even = ((tiles + most - 1) / most + 1) / 2 * 2, x = even < 6 ? 6 : even, n = (tiles + x - 1) / x;
+    const int64_t even_tiles = ((tiles + most - 1) / most + 1) / 2 * 2, x = even_tiles < 6 ? 6 : even_tiles, n = (tiles + x - 1) / x;
     if (x >= tiles) continue;
     const float gain = per_tile * ((float)tiles - fmaxf((float)x, 0.6f * (float)(wgs * tiles) / 256.f)) - 4.f - per_range * (float)n;
     if (gain > best) {

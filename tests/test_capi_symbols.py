@@ -79,6 +79,22 @@ def test_prefill_ranges_take_any_bound():
         assert lib.mvllm_prefill_ranges_workspace_bytes(500, keys, 16, 128, 6) == -(-tiles // 6) * 500 * 16 * 129 * 4
 
 
+def test_prefill_ranges_plan_looks_at_the_busiest_cu():
+    """Equal sequences whose heavy row tiles meet on a CU stay with the other kernels, whatever their number; uneven ones, a single one and
+    those that fit side by side go over."""
+    plan = _lib().load().mvllm_prefill_ranges_plan
+    heads, packed, paged = (16, 8, 128), (0, 1), (16, 1)
+    assert plan(2, 2992, 1496, *heads, *packed) == 24 and plan(2, 3312, 1656, *heads, *packed) == 0    # 1.67 and 1.79 of the longest tile
+    assert plan(3, 2928, 976, *heads, *packed) == 0 and plan(3, 3888, 1296, *heads, *packed) == 22     # 2.0 and 1.52
+    assert plan(2, 3311, 1987, *heads, *packed) == 32 and plan(1, 3376, 3376, *heads, *packed) == 54   # uneven, one
+    assert plan(5, 3120, 624, *heads, *packed) == 10                                                   # short: the start counts
+    assert plan(3, 2382, 1588, *heads, *paged) == 26 and plan(4, 2352, 1176, *heads, *paged) == 0      # 1.80 and 1.90
+    four = (32, 8, 64)
+    assert plan(4, 1672, 758, *four, *paged) == 0 and plan(4, 2072, 758, *four, *paged) == 12          # 512 and 768 places of the other form
+    assert plan(4, 472, 758, *four, *paged) == 12 and plan(8, 744, 758, *four, *paged) == 12           # one workgroup per CU
+    assert plan(4, 1672, 1910, *four, *paged) == 30                                                    # long
+
+
 def test_prefill_split_plan_is_host_arithmetic():
     """When a paged prefill is cut over its keys: few query tiles, at least 4096 keys, a shape the split form takes;
     and the workspace holds the ranges' tables, partial results and denominators."""
