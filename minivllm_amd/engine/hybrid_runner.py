@@ -45,7 +45,7 @@ class HybridModelRunner(ModelRunner):
     def forward_step(self, seqs, layer_outputs=None):
         """Run every sequence's scheduled tokens; returns (hidden rows, the step)."""
         step = ragged_step(seqs, self.model.windows, self.block_size, self.device, self.model.memory_units,
-                           self.model.latent_views)
+                           self.model.latent_views, self.model.memory_coarse)
         set_context(step.multi_rows > 0, ragged=step)
         try:
             hidden = self.model(step.input_ids, step.positions, layer_outputs)

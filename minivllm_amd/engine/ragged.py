@@ -101,24 +101,37 @@ class RaggedStep:
 
 BLOCK_ROWS = 64                # rows per block of a recurrence's block form: segments are whole blocks
 FILL_WORKGROUPS = 512          # segments are made shorter until there are this many workgroups ...
-# ... but not shorter than this, and portions of a few of them stay whole (see _segments): the states' own pass, two launches and their way through
-# memory have to pay.  One portion of 700 rows, 16 heads of 128 x 256: 43 us (256: 55, 64: 40), 2000 rows, 8 heads: 50 (60, 57), 200
+# ... but not shorter than this or twice this, and portions of a few of them stay whole (see _segments): the states' own pass, two launches and
+# their way through memory have to pay.  One portion of 700 rows, 16 heads of 128 x 256: 43 us (256: 55, 64: 40), 2000 rows, 8 heads: 50 (60, 57), 200
 # rows in two segments 36 against 31 whole.
 MIN_SEGMENT_ROWS = 128
+MAX_CHAIN = 40                 # segments of a portion at the shorter length: their states are combined one after the other
 
 
-def _segments(lens, cu, units):
-    """[entry, first row, rows, flags (1 first, 2 last, 4 only)] of every long entry."""
+def _segments(lens, cu, units, coarse=False):
+    """[entry, first row, rows, flags (1 first, 2 last, 4 only)] of every long entry.
+
+    ``coarse``: memories with keys of more than 128 dims, whose workgroups have a CU to themselves, and those without gates, whose
+    blocks take less beside what a segment costs: segments of less than 256 rows only while a CU has one workgroup at most.  us at
+    128 and 256 rows: decay memory of 8 heads of 256 x 256, 4 x 512 rows (256 workgroups) 64 / 84, 4 x 1024 (512) 123 / 96, one portion of
+    2000 64 / 84, 8 x 450 130 / 94; of 16 heads of 128 x 128, 4 x 1024 65 / 62; mLSTM of 8 heads of 256 x 512, one portion of 2000 132 / 109, of 4
+    of 256 x 256, 8000 151 / 116.  mLSTM up to 128 dims, two workgroups to a CU: 8 heads of 128 x 256, 4 x 1024 rows 61 / 72; 4 of 64 x 256, 8 x
+    1024 45 / 56, one portion of 5000 rows, a chain of 40 segments, 54 / 58, but of 8000, a chain of 63, 75 / 66 (8 of 64 x 64, 6000 rows, 47, 74 / 71)."""
     long_entries = [e for e, n in enumerate(lens) if n >= LONG_ROWS]
     total = int(sum(lens[e] for e in long_entries))
     length = total
     if long_entries and units and len(long_entries) * units < FILL_WORKGROUPS // 2:
-        length = max(-(-total * units // (FILL_WORKGROUPS * BLOCK_ROWS)) * BLOCK_ROWS, MIN_SEGMENT_ROWS)
+        longest = max(int(lens[e]) for e in long_entries)
+        many = total * units > FILL_WORKGROUPS // 2 * MIN_SEGMENT_ROWS if coarse else longest > MAX_CHAIN * MIN_SEGMENT_ROWS
+        length = -(-total * units // (FILL_WORKGROUPS * BLOCK_ROWS)) * BLOCK_ROWS
+        if length <= MIN_SEGMENT_ROWS:
+            length = MIN_SEGMENT_ROWS * (2 if many else 1)
     # the rows from which cutting pays: its two more launches take the longer the more there is to combine.  us whole and cut, memory of 128 x 256:
     # 8 heads, one portion of 256 rows 34.5 / 35.4, of 300 37 / 35.5; two of 256 35 / 38.5, of 384 44 / 41; eight of 256 42 / 55, of 384 54 / 61, of
-    # 512 69 / 67.5
+    # 512 69 / 67.5.  Coarse ones, two portions of 300 rows: decay memory of 16 heads of 128 x 128 35.6 / 32.2, of 8 of 256 x 256 57.5 / 51.6, eight of
+    # 4 of 256 x 64 93 / 61
     busy = len(long_entries) * (units or 0)
-    least = MIN_SEGMENT_ROWS * (4 if busy <= 16 else 5 if busy <= 64 else 7) // 2
+    least = MIN_SEGMENT_ROWS * (4 if busy <= (32 if coarse else 16) else 5 if busy <= 64 else 7) // 2
     out = []
     for e in long_entries:
         n, at = int(lens[e]), int(cu[e])
@@ -271,7 +284,7 @@ def _ring_arrays(items, window, index, block_size, cu, num_short):
     return out, dict(absorbed=absorbed, num_long=cu_q[-1], num_keys=cu_k[-1])
 
 
-def ragged_arrays(seqs, windows, block_size, memory_units=0, latent=False):
+def ragged_arrays(seqs, windows, block_size, memory_units=0, latent=False, memory_coarse=False):
     """Host side of a step over ``seqs``: each runs its tokens [num_computed_tokens, + num_scheduled_tokens).  Returns
     (arrays, window arrays, window counts, facts), everything in numpy; the sequences' convolution banks flip for entries
     of more than one token."""
@@ -300,7 +313,7 @@ def ragged_arrays(seqs, windows, block_size, memory_units=0, latent=False):
     for e, i in enumerate(order):
         starts[i] = int(cu[e])
     singles = int((lens == 1).sum())
-    segments = _segments(lens, cu, memory_units) if memory_units else []
+    segments = _segments(lens, cu, memory_units, memory_coarse) if memory_units else []
     if segments:
         arrays["segments"] = np.asarray(segments, dtype=np.int32)
     facts = dict(num_tokens=int(cu[-1]), num_entries=len(items), num_single=singles, multi_rows=int(cu[-1]) - singles,
@@ -308,10 +321,10 @@ def ragged_arrays(seqs, windows, block_size, memory_units=0, latent=False):
     return arrays, [a for a, _ in per_window], [c for _, c in per_window], facts
 
 
-def ragged_step(seqs, windows, block_size, device, memory_units=0, latent=False) -> RaggedStep:
+def ragged_step(seqs, windows, block_size, device, memory_units=0, latent=False, memory_coarse=False) -> RaggedStep:
     """The step's device tensors: one copy per integer type, every tensor a 16-byte aligned slice of it.  ``latent``: the
     views of windows that are plain numbers are LatentSteps."""
-    arrays, window_arrays, counts, facts = ragged_arrays(seqs, windows, block_size, memory_units, latent)
+    arrays, window_arrays, counts, facts = ragged_arrays(seqs, windows, block_size, memory_units, latent, memory_coarse)
     named = [((None, k), a) for k, a in arrays.items()]
     for g, wa in enumerate(window_arrays):
         named += [((g, k), a) for k, a in wa.items()]

@@ -124,7 +124,7 @@ class FevosunLayer(nn.Module):
 
 class FevosunForCausalLM(nn.Module):
     latent_views = False                                # its windows are sliding ones (engine/windows.py)
-    memory_units = 0                                    # no recurrence
+    memory_units, memory_coarse = 0, False              # no recurrence
 
     def __init__(self, config: dict, block_size: int, dtype: torch.dtype, device: torch.device):
         super().__init__()

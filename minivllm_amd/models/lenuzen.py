@@ -89,7 +89,7 @@ class LenuzenLayer(nn.Module):
 
 class LenuzenForCausalLM(nn.Module):
     latent_views = False                                # its windows are sliding ones (engine/windows.py) and chunks
-    memory_units = 0                                    # no recurrence
+    memory_units, memory_coarse = 0, False              # no recurrence
 
     def __init__(self, config: dict, block_size: int, dtype: torch.dtype, device: torch.device):
         super().__init__()

@@ -127,6 +127,7 @@ class NiridraForCausalLM(nn.Module):
         # workgroups per segment of the block form of the memories (0: no such layer): how far portions are cut
         self.memory_units = min((e["mixer"]["heads"] * -(-e["mixer"]["vdim"] // 128) for e in layers if e["type"] == "lightning"),
                                 default=0)
+        self.memory_coarse = True                                        # no gates
         bigram = config["embedding"].get("bigram")
         self.hashing = (bigram["buckets"], bigram["mul_prev"], bigram["mul_cur"]) if bigram else None
 

@@ -157,6 +157,7 @@ class SokevikForCausalLM(nn.Module):
         # workgroups per segment of the block form of the matrix memory (0: no such layer): how far portions are cut
         self.memory_units = min((e["mixer"]["heads"] * -(-e["mixer"]["vdim"] // 128) for e in layers if e["type"] == "mlstm"),
                                 default=0)
+        self.memory_coarse = any(e["mixer"]["dim"] > 128 for e in layers if e["type"] == "mlstm")
         max_position, tables = config.get("max_position", 4096), {}
 
         def table(base, dims, scaling):

@@ -180,6 +180,31 @@ def _brute_force(seqs, window, bs, index):
     return rows
 
 
+@pytest.mark.parametrize("lens,units,coarse,rows", [
+    ([256], 16, False, [[256]]), ([257], 16, False, [[128, 128, 1]]),                         # from the rows on from which cutting pays ...
+    ([300] * 2, 16, False, [[300]] * 2), ([321] * 2, 16, False, [[128, 128, 65]] * 2),         # ... more of them beside others
+    ([448] * 5, 16, False, [[448]] * 5), ([449] * 5, 16, False, [[128, 128, 128, 65]] * 5),
+    ([1024] * 4, 16, False, [[128] * 8] * 4), ([1024] * 4, 16, True, [[256] * 4] * 4),         # two workgroups to a CU, or one
+    ([512] * 4, 16, True, [[128] * 4] * 4), ([520] * 4, 16, True, [[192, 192, 136]] * 4),
+    ([300] * 2, 16, True, [[128, 128, 44]] * 2), ([300] * 3, 16, True, [[300]] * 3),
+    ([5120], 8, False, [[128] * 40]), ([5124], 8, False, [[256] * 20 + [4]]),                  # a chain of 40 segments at most
+    ([4160], 16, True, [[192] * 21 + [128]]),                                                  # longer ones to fill the chip: as they come
+    ([8000], 4, True, [[128] * 62 + [64]]),                                                    # (not where workgroups take long)
+    ([1024] * 16, 16, False, [[1024]] * 16), ([40, 300, 33], 0, False, [[40], [300], [33]]),   # the chip is full; nobody asks
+])
+def test_segments_of_portions(lens, units, coarse, rows):
+    """How far long portions are cut: edges of the shortest segment, of the portions that stay whole and of the two rules for them."""
+    from minivllm_amd.engine.ragged import _segments
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    got = _segments(np.asarray(lens), cu, units, coarse)
+    for e, want in enumerate(rows):
+        mine = [s for s in got if s[0] == e]
+        assert [s[2] for s in mine] == want
+        assert [s[1] for s in mine] == [cu[e] + sum(want[:i]) for i in range(len(want))]
+        assert [s[3] for s in mine] == ([7] if len(want) == 1 else [1] + [0] * (len(want) - 2) + [2])
+    assert len(got) == sum(len(w) for w in rows)
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_ragged_arrays_against_row_by_row(seed):
     rng = random.Random(seed)
