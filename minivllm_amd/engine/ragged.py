@@ -113,7 +113,7 @@ def _segments(lens, cu, units, coarse=False):
 
     ``coarse``: memories with keys of more than 128 dims, whose workgroups have a CU to themselves, and those without gates, whose
     blocks take less beside what a segment costs: segments of less than 256 rows only while a CU has one workgroup at most.  us at
-    128 and 256 rows: decay memory of 8 heads of 256 x 256, 4 x 512 rows (256 workgroups) 64 / 84, 4 x 1024 (512) 123 / 96, one portion of
+    128 and 256 rows: decay memory of 8 heads of 256 x 256, 2 x 1024 rows (256 workgroups) 64 / 84, 4 x 1024 (512) 123 / 96, one portion of
     2000 64 / 84, 8 x 450 130 / 94; of 16 heads of 128 x 128, 4 x 1024 65 / 62; mLSTM of 8 heads of 256 x 512, one portion of 2000 132 / 109, of 4
     of 256 x 256, 8000 151 / 116.  mLSTM up to 128 dims, two workgroups to a CU: 8 heads of 128 x 256, 4 x 1024 rows 61 / 72; 4 of 64 x 256, 8 x
     1024 45 / 56, one portion of 5000 rows, a chain of 40 segments, 54 / 58, but of 8000, a chain of 63, 75 / 66 (8 of 64 x 64, 6000 rows, 47, 74 / 71)."""
