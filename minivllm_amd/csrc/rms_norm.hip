@@ -108,17 +108,26 @@ static int launch_norm(void* out, void* residual_out, const void* x, const void*
                        int64_t rows, int hidden, int64_t x_stride, int64_t res_stride, hipStream_t s) {
   const int chunks = (hidden + 511) / 512;
   const int per_group = chunks > 2 ? 1 : kNormThreads / 64;
-  const dim3 grid((unsigned)((rows + per_group - 1) / per_group)), block(kNormThreads);
-#define MVLLM_LAUNCH_N(C, W)                                                                                      \
-  add_rms_norm_kernel<T, C, W><<<grid, block, 0, s>>>((T*)out, (T*)residual_out, (const T*)x, (const T*)residual, \
-                                                      gamma, eps, rows, hidden, x_stride, res_stride)
-  if (chunks <= 1) MVLLM_LAUNCH_N(1, 1);
-  else if (chunks <= 2) MVLLM_LAUNCH_N(2, 1);
-  else if (chunks <= 4) MVLLM_LAUNCH_N(1, 4);
-  else if (chunks <= 8) MVLLM_LAUNCH_N(2, 4);
-  else MVLLM_LAUNCH_N(4, 4);
+  constexpr int64_t kMostGroups = (((int64_t)1 << 32) - 1) / kNormThreads;      // a launch counts its threads in 32 bits
+  const int64_t most = kMostGroups * per_group;
+  for (int64_t row0 = 0; row0 < rows; row0 += most) {
+    const int64_t n = rows - row0 < most ? rows - row0 : most;
+    const dim3 grid((unsigned)((n + per_group - 1) / per_group)), block(kNormThreads);
+    T* o = (T*)out + row0 * hidden;
+    T* ro = residual_out ? (T*)residual_out + row0 * hidden : nullptr;
+    const T* xr = (const T*)x + row0 * x_stride;
+    const T* rr = residual ? (const T*)residual + row0 * res_stride : nullptr;
+#define MVLLM_LAUNCH_N(C, W) add_rms_norm_kernel<T, C, W><<<grid, block, 0, s>>>(o, ro, xr, rr, gamma, eps, n, hidden, x_stride, res_stride)
+    if (chunks <= 1) MVLLM_LAUNCH_N(1, 1);
+    else if (chunks <= 2) MVLLM_LAUNCH_N(2, 1);
+    else if (chunks <= 4) MVLLM_LAUNCH_N(1, 4);
+    else if (chunks <= 8) MVLLM_LAUNCH_N(2, 4);
+    else MVLLM_LAUNCH_N(4, 4);
 #undef MVLLM_LAUNCH_N
-  return launch_status();
+    const int status = launch_status();
+    if (status != MVLLM_OK) return status;
+  }
+  return MVLLM_OK;
 }
 
 }  // namespace mvllm

@@ -44,6 +44,19 @@ def test_add_rms_norm(dtype, rows, hidden, with_residual):
     _close(got_y, want_y, dtype)
 
 
+def test_add_rms_norm_more_rows_than_a_launch_counts():
+    """2^32 threads and some more: rows on both sides of the end of the first launch, which holds 2^24 - 1 rows of more than 1024 numbers."""
+    rows, hidden, first = 2 ** 24 + 2, 1032, 2 ** 24 - 1
+    x = torch.empty(rows, hidden, dtype=torch.bfloat16, device=DEV)
+    at = torch.tensor([0, first - 1, first, first + 1, rows - 1], device=DEV)
+    some = torch.randn(len(at), hidden, generator=torch.Generator().manual_seed(3)).bfloat16()
+    x[at], gamma = some.to(DEV), torch.linspace(0.5, 1.5, hidden)
+    got = add_rms_norm(x, gamma.to(DEV), 1e-6)[at]
+    del x
+    torch.cuda.empty_cache()
+    _close(got, oracle.add_rms_norm_oracle(some, gamma, 1e-6), torch.bfloat16)
+
+
 def test_add_rms_norm_strided_rows_and_errors():
     g = torch.Generator().manual_seed(2)
     wide = torch.randn(9, 3 * 512, generator=g).to(torch.bfloat16)
