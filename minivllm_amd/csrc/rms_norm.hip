@@ -11,7 +11,7 @@
 // row is read once and written once (16-byte accesses).  Up to 1024 numbers a row takes one wave; longer ones four, because a wave with
 // 32 numbers or more per lane to take through the norm is what few rows wait for, and holds too many registers to have enough rows
 // under way where there are many (us with one wave and with four: 61 rows of 4096 6.6 / 3.1, 1024 rows 8.8 / 6.5, 8192 rows 44.7 / 39.6;
-// 8192 rows of 8192 135 / 103 = 5.2 TB/s).
+// 8192 rows of 8192 135 / 103 = 5.2 TB/s).  Many rows just above 1024: see kManyRows.
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -103,11 +103,19 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
   }
 }
 
+// ... but not where half the threads of four waves would have no element and rows enough are there to fill the chip: a row just above 1024
+// numbers stays in one wave (with a residual twice the loads are under way, and fewer of them idle).  us in four and in one, 3072 /
+// 8192 / 65536 rows: of 1032 numbers 5.2 / 9.4 / 55.7 and 5.1 / 8.2 / 45.6, of 1280 5.2 / 9.5 / 69.8 and 4.9 / 8.5 / 61.8, of 1536 5.4 / 9.9 / 74 and
+// 5.2 / 9.1 / 72 but 16.6 and 16.7 at 16384; with a residual 1032 6.9 / 14.2 / 110 and 6.7 / 13.5 / 110, 1152 6.9 / 13.7 / 109 and 6.8 / 13.9 / 111.
+// 2048 rows of 1280 in four 4.3, in one 4.5.
+constexpr int64_t kManyRows = 3072;
+
 template <typename T>
 static int launch_norm(void* out, void* residual_out, const void* x, const void* residual, const float* gamma, float eps,
                        int64_t rows, int hidden, int64_t x_stride, int64_t res_stride, hipStream_t s) {
   const int chunks = (hidden + 511) / 512;
-  const int per_group = chunks > 2 ? 1 : kNormThreads / 64;
+  const bool one_wave = chunks <= 2 || (rows >= kManyRows && hidden <= (residual ? 1088 : 1280));
+  const int per_group = one_wave ? kNormThreads / 64 : 1;
   constexpr int64_t kMostGroups = (((int64_t)1 << 32) - 1) / kNormThreads;      // a launch counts its threads in 32 bits
   const int64_t most = kMostGroups * per_group;
   for (int64_t row0 = 0; row0 < rows; row0 += most) {
@@ -120,6 +128,7 @@ static int launch_norm(void* out, void* residual_out, const void* x, const void*
 #define MVLLM_LAUNCH_N(C, W) add_rms_norm_kernel<T, C, W><<<grid, block, 0, s>>>(o, ro, xr, rr, gamma, eps, n, hidden, x_stride, res_stride)
     if (chunks <= 1) MVLLM_LAUNCH_N(1, 1);
     else if (chunks <= 2) MVLLM_LAUNCH_N(2, 1);
+    else if (one_wave) MVLLM_LAUNCH_N(3, 1);
     else if (chunks <= 4) MVLLM_LAUNCH_N(1, 4);
     else if (chunks <= 8) MVLLM_LAUNCH_N(2, 4);
     else MVLLM_LAUNCH_N(4, 4);

@@ -44,6 +44,23 @@ def test_add_rms_norm(dtype, rows, hidden, with_residual):
     _close(got_y, want_y, dtype)
 
 
+@pytest.mark.parametrize("rows", [3071, 3073])
+@pytest.mark.parametrize("hidden", [1032, 1088, 1096, 1280, 1288])
+@pytest.mark.parametrize("with_residual", [True, False])
+def test_add_rms_norm_one_wave_or_four(rows, hidden, with_residual):
+    """Both sides of the line between a wave and four per row, a last workgroup that is not full; the last rows against the oracle."""
+    g = torch.Generator().manual_seed(rows + hidden)
+    x, r = (torch.randn(rows, hidden, generator=g).bfloat16() for _ in range(2))
+    gamma = torch.rand(hidden, generator=g) + 0.5
+    got = add_rms_norm(x.to(DEV), gamma.to(DEV), 1e-6, r.to(DEV) if with_residual else None)
+    want = oracle.add_rms_norm_oracle(x[-70:], gamma, 1e-6, *([r[-70:]] if with_residual else []))
+    if with_residual:
+        assert torch.equal(got[1].cpu(), (x.float() + r.float()).bfloat16())
+        got, want = got[0], want[0]
+    _close(got[-70:], want, torch.bfloat16)
+    assert torch.isfinite(got).all()
+
+
 def test_add_rms_norm_more_rows_than_a_launch_counts():
     """2^32 threads and some more: rows on both sides of the end of the first launch, which holds 2^24 - 1 rows of more than 1024 numbers."""
     rows, hidden, first = 2 ** 24 + 2, 1032, 2 ** 24 - 1
