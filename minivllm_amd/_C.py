@@ -225,7 +225,10 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def current_stream_ptr(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of a tensor's device.  Asked on every call: without the Stream object around it (0.1 us, not 1.9, of the 10
+    that a small operator's call takes the host)."""
+    index = device.index if isinstance(device, torch.device) else None
+    return torch.cuda.current_stream(device).cuda_stream if index is None else torch._C._cuda_getCurrentRawStream(index)
 
 
 def require_cuda(*tensors) -> None:

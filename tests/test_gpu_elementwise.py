@@ -100,3 +100,26 @@ def test_silu_and_mul(dtype, rows, width):
     wide = torch.zeros(rows, 2 * width + 64, dtype=dtype)
     wide[:, : 2 * width] = x
     _close(silu_and_mul(wide.to(DEV)[:, : 2 * width]), want, dtype, ulps=2.0)
+
+
+def test_operators_run_on_the_current_stream():
+    """What the operators take for the current stream is torch's: default, inside a stream's block, on another thread, under capture."""
+    from concurrent.futures import ThreadPoolExecutor
+    from minivllm_amd import _C
+    device = torch.zeros(1, device=DEV).device
+    same = lambda: _C.current_stream_ptr(device) == torch.cuda.current_stream(device).cuda_stream
+    side = torch.cuda.Stream()
+    assert same() and _C.current_stream_ptr(torch.device("cuda")) == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side), ThreadPoolExecutor(1) as pool:
+        assert same() and _C.current_stream_ptr(device) == side.cuda_stream
+        assert pool.submit(same).result() and pool.submit(_C.current_stream_ptr, device).result() != side.cuda_stream
+    x, graph = torch.randn(4, 64, device=DEV), torch.cuda.CUDAGraph()
+    gamma = torch.ones(64, device=DEV)
+    add_rms_norm(x, gamma, 1e-6)
+    with torch.cuda.graph(graph):
+        assert same()
+        y = add_rms_norm(x, gamma, 1e-6)
+    x.copy_(torch.randn(4, 64, device=DEV))
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y, add_rms_norm(x, gamma, 1e-6))
