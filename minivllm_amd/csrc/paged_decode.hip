@@ -127,11 +127,12 @@ constexpr int kSplitManyWaves = 8;
 constexpr int kSplitMinGroups = 512;
 constexpr int kSplitMaxPart = 4096;
 constexpr int kSplitOnePartCtx = 512;
-// Tables of at most this many tokens (16-bit caches) are one partition from kSplitOnePartPairs (sequence, kv head) pairs on, and
-// below that cut into no less than kSplitNarrowPart tokens: us with partitions to fill the chip / so, 61 sequences of 64-1500 tokens
-// 51.5 / 37.6, 40 of 32-700 21.7 / 16.6, 32 of 500-2000 41.1 / 37.9 (16 of them 23.9 / 31.7); 1 of 2000 12.6 / 10.3, 4 of 1000-2000
-// 13.0 / 12.3, 8 of 100-1000 10.5 / 10.7.
-constexpr int kSplitNarrowCtx = 2048, kSplitNarrowPart = 256, kSplitOnePartPairs = 256;
+// Tables of at most this many tokens (16-bit caches) are one partition from kSplitOnePartPairs (sequence, kv head) pairs on; below that they
+// are cut into no less than 128 tokens while that gives at most kSplitMinGroups workgroups, else into no less than 256.  us with
+// partitions to fill the chip / of one: 61 sequences of 64-1500 tokens 51.5 / 37.6, 40 of 32-700 21.7 / 16.6, 32 of 500-2000 41.1 / 37.9 (16 of
+// them 23.9 / 31.7).  Parts of 64 / 128 / 256, 8 kv heads, tables of 2048: 1 of 300 7.1 / 7.5 / 8.4, of 1000 8.6 / 7.9 / 8.7, of 2000 11.4 / 9.2 / 9.0;
+// 4 of 300 8.6 / 8.0 / 8.9, of 600 9.9 / 8.9 / 9.4; 6 of 854-1455 (heads of 64; 192 tokens 10.5) 12.8 / 10.3 / 9.7; 8 of 1500-2000 21 / 17.0 / 14.3.
+constexpr int kSplitNarrowCtx = 2048, kSplitOnePartPairs = 256;
 inline bool split_wanted(int64_t max_ctx, int batch, int num_kv_heads, bool int8) {
   const int part = partition_tokens_for(max_ctx, batch);
   const int64_t parts = (max_ctx + part - 1) / part;
@@ -152,7 +153,8 @@ inline int split_partition_tokens(int64_t max_ctx, int batch, int num_kv_heads, 
   // the merge launch that several partitions need costs more than they save (16 sequences of 32-352 tokens:
   // 10.1 -> 8.0 us per call; from 1024-token tables on the finer split wins)
   const bool narrow = sixteen_bit && max_ctx <= kSplitNarrowCtx;
-  if (narrow && part < kSplitNarrowPart) part = kSplitNarrowPart;
+  const int64_t least = pairs * ((max_ctx + 127) / 128) <= kSplitMinGroups ? 128 : 256;
+  if (narrow && part < least) part = least;
   if (max_ctx <= kSplitOnePartCtx || (narrow && pairs >= kSplitOnePartPairs)) part = (max_ctx + 63) / 64 * 64;
   if (part > kSplitMaxPart) part = kSplitMaxPart;
   const int64_t floor_part = partition_tokens_for(max_ctx, batch);

@@ -122,6 +122,20 @@ def test_prefill_split_plan_is_host_arithmetic():
     assert lib.mvllm_prefill_paged_split_workspace_bytes(8, 128, 32768, 32, 8, 128, 256, bf16, 9) == 0   # 72 ranges
 
 
+def test_decode_plan_in_narrow_tables():
+    """(tokens per partition, partitions, waves) of 16-bit caches in tables of at most 2048 tokens: edges of every rule."""
+    import torch
+    from minivllm_amd.layers.attention import paged_decode_plan
+    _lib().load()
+    plan = lambda batch, tokens, kv=8, **kw: paged_decode_plan(batch, 4 * kv, kv, 128, tokens // 16, 16, **kw)
+    assert plan(1, 512) == (512, 1, 8) and plan(1, 528) == (128, 5, 8)                # one partition whatever the batch, or parts
+    assert plan(1, 2048) == (128, 16, 4) and plan(4, 2048) == (128, 16, 4)            # 512 workgroups at most ...
+    assert plan(5, 2048) == (256, 8, 4) and plan(8, 1024) == (128, 8, 4)              # ... from then on 256 tokens
+    assert plan(8, 1040) == (256, 5, 4) and plan(31, 2048) == (704, 3, 4)
+    assert plan(32, 2048) == (2048, 1, 8) and plan(33, 2048) == (2048, 1, 4)          # one from 256 pairs on; eight waves up to 256 workgroups
+    assert plan(1, 2048, int8_cache=True)[0] == 64 and plan(1, 2048, dtype=torch.float32)[0] == 64
+
+
 def test_decode_plan_is_host_arithmetic():
     """Which form a decode call takes, and that the split form never needs more workspace than is advertised."""
     import torch
