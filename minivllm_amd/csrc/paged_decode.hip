@@ -129,9 +129,12 @@ constexpr int kSplitMaxPart = 4096;
 constexpr int kSplitOnePartCtx = 512;
 // Tables of at most this many tokens (16-bit caches) are one partition from kSplitOnePartPairs (sequence, kv head) pairs on; below that they
 // are cut into no less than 128 tokens while that gives at most kSplitMinGroups workgroups, else into no less than 256.  us with
-// partitions to fill the chip / of one: 61 sequences of 64-1500 tokens 51.5 / 37.6, 40 of 32-700 21.7 / 16.6, 32 of 500-2000 41.1 / 37.9 (16 of
-// them 23.9 / 31.7).  Parts of 64 / 128 / 256, 8 kv heads, tables of 2048: 1 of 300 7.1 / 7.5 / 8.4, of 1000 8.6 / 7.9 / 8.7, of 2000 11.4 / 9.2 / 9.0;
+// partitions to fill the chip / of one, tables of 2048: 61 sequences of 64-1500 tokens 45 / 34, 40 of 32-700 20 / 14, 32 of 500-2000 41 / 38 (16 of
+// them 23.9 / 31.7).  In wider tables one partition gains as much where contexts are short (61 of 64-1500 in 4096 48 / 34), but a sequence may
+// be so much longer than the others that its workgroup is alone at the end: 48 of 100-3000, heads of 64, in 3072 39 / 48.5, in 4096 45 / 48.5.
+// Parts of 64 / 128 / 256, 8 kv heads, tables of 2048: 1 of 300 7.1 / 7.5 / 8.4, of 1000 8.6 / 7.9 / 8.7, of 2000 11.4 / 9.2 / 9.0;
 // 4 of 300 8.6 / 8.0 / 8.9, of 600 9.9 / 8.9 / 9.4; 6 of 854-1455 (heads of 64; 192 tokens 10.5) 12.8 / 10.3 / 9.7; 8 of 1500-2000 21 / 17.0 / 14.3.
+// (In wider tables partition_tokens_for's least is about as long.)
 constexpr int kSplitNarrowCtx = 2048, kSplitOnePartPairs = 256;
 inline bool split_wanted(int64_t max_ctx, int batch, int num_kv_heads, bool int8) {
   const int part = partition_tokens_for(max_ctx, batch);

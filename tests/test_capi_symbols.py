@@ -133,6 +133,7 @@ def test_decode_plan_in_narrow_tables():
     assert plan(5, 2048) == (256, 8, 4) and plan(8, 1024) == (128, 8, 4)              # ... from then on 256 tokens
     assert plan(8, 1040) == (256, 5, 4) and plan(31, 2048) == (704, 3, 4)
     assert plan(32, 2048) == (2048, 1, 8) and plan(33, 2048) == (2048, 1, 4)          # one from 256 pairs on; eight waves up to 256 workgroups
+    assert plan(31, 2064) == (704, 3, 4) and plan(33, 2064) == (1088, 2, 4)
     assert plan(1, 2048, int8_cache=True)[0] == 64 and plan(1, 2048, dtype=torch.float32)[0] == 64
 
 

@@ -90,6 +90,23 @@ def test_eight_waves_per_head(hq, hkv, d, bs, ctx_list):
     assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
 
 
+@pytest.mark.parametrize("batch,first,tokens,plan", [
+    (32, [2048, 1, 1025], 2048, (2048, 1, 8)), (33, [2048, 2047, 63], 2048, (2048, 1, 4)),         # whole sequences, eight waves and four
+    (33, [2060, 1088, 1089], 2064, (1088, 2, 4)), (31, [2048, 700, 705], 2048, (704, 3, 4)),       # cut: a table or a batch past the rule's end
+    (4, [2048, 128, 129, 1], 2048, (128, 16, 4)), (5, [2048, 256, 257], 2048, (256, 8, 4)),        # a few sequences
+])
+def test_partitions_of_narrow_tables(batch, first, tokens, plan):
+    hq, hkv, d, bs = 16, 8, 64, 16
+    case = make_paged_case(41, batch, 1, 1, hq, hkv, d, bs, dtype=torch.bfloat16, ctx_list=first + [17 + 5 * i for i in range(batch - len(first))])
+    q, kc, vc, tables, ctx = case
+    tables = torch.nn.functional.pad(tables, (0, tokens // bs - tables.shape[1]), value=-1)
+    assert paged_decode_plan(batch, hq, hkv, d, tables.shape[1], bs) == plan
+    scale = 1 / math.sqrt(d)
+    got = _run(q, kc, vc, tables, ctx, scale, hq, hkv, d, bs)
+    mx, mean = error_stats(got, _oracle32(*case, scale, hq, hkv, d, bs))
+    assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
+
+
 @pytest.mark.parametrize("dtype,hq,hkv,d,bs", [
     (torch.float32, 4, 2, 64, 4),       # generic kernel: fp32 with a block size of 4
     (torch.float32, 6, 2, 96, 16),      # fp32, head_dim 96
