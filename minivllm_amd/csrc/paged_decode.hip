@@ -132,6 +132,10 @@ constexpr int kSplitOnePartCtx = 512;
 // partitions to fill the chip / of one, tables of 2048: 61 sequences of 64-1500 tokens 45 / 34, 40 of 32-700 20 / 14, 32 of 500-2000 41 / 38 (16 of
 // them 23.9 / 31.7).  In wider tables one partition gains as much where contexts are short (61 of 64-1500 in 4096 48 / 34), but a sequence may
 // be so much longer than the others that its workgroup is alone at the end: 48 of 100-3000, heads of 64, in 3072 39 / 48.5, in 4096 45 / 48.5.
+// Below 112 dims that shows in these tables too, because a token takes a wave as long and the chip half the time: such workgroups have
+// eight waves (blocks of less than a tile, for which there is no such kernel, keep the partitions that fill the chip).  Heads of 64, two partitions / one of
+// four waves / of eight, tables of 2048: 36 of 16-2000 22.9 / 31.5 / 20.2, of 1500-2000 35.8 / 37.3 / 38.2, of 16-300 9.8 / 7.7 / 8.4, of 900-1000 30.6 /
+// 22.0 / 23.6; 63 of 16-2000 32.4 / 33.8 / 26.4, of 16-300 13.2 / 8.4 / 10.2.
 // Parts of 64 / 128 / 256, 8 kv heads, tables of 2048: 1 of 300 7.1 / 7.5 / 8.4, of 1000 8.6 / 7.9 / 8.7, of 2000 11.4 / 9.2 / 9.0;
 // 4 of 300 8.6 / 8.0 / 8.9, of 600 9.9 / 8.9 / 9.4; 6 of 854-1455 (heads of 64; 192 tokens 10.5) 12.8 / 10.3 / 9.7; 8 of 1500-2000 21 / 17.0 / 14.3.
 // (In wider tables partition_tokens_for's least is about as long.)
@@ -148,7 +152,12 @@ inline bool split_wanted(int64_t max_ctx, int batch, int num_kv_heads, bool int8
   if (int8) return few_groups || ((short_parts || narrow_table) && (int64_t)batch * num_kv_heads <= 512);
   return few_groups || short_parts || narrow_table;
 }
-inline int split_partition_tokens(int64_t max_ctx, int batch, int num_kv_heads, bool sixteen_bit) {
+constexpr int kSplitWideDim = 112;
+// whether a batch is taken whole for its number of pairs alone
+inline bool split_one_part(int64_t max_ctx, int64_t pairs, int head_dim, int block_size) {
+  return max_ctx <= kSplitNarrowCtx && pairs >= kSplitOnePartPairs && (head_dim >= kSplitWideDim || block_size % kTile == 0);
+}
+inline int split_partition_tokens(int64_t max_ctx, int batch, int num_kv_heads, bool sixteen_bit, int head_dim, int block_size) {
   const int64_t pairs = (int64_t)batch * num_kv_heads;
   const int64_t want_parts = (kSplitMinGroups + pairs - 1) / pairs;
   int64_t part = ((max_ctx + want_parts - 1) / want_parts + 63) / 64 * 64;
@@ -158,7 +167,7 @@ inline int split_partition_tokens(int64_t max_ctx, int batch, int num_kv_heads, 
   const bool narrow = sixteen_bit && max_ctx <= kSplitNarrowCtx;
   const int64_t least = pairs * ((max_ctx + 127) / 128) <= kSplitMinGroups ? 128 : 256;
   if (narrow && part < least) part = least;
-  if (max_ctx <= kSplitOnePartCtx || (narrow && pairs >= kSplitOnePartPairs)) part = (max_ctx + 63) / 64 * 64;
+  if (max_ctx <= kSplitOnePartCtx || (sixteen_bit && split_one_part(max_ctx, pairs, head_dim, block_size))) part = (max_ctx + 63) / 64 * 64;
   if (part > kSplitMaxPart) part = kSplitMaxPart;
   const int64_t floor_part = partition_tokens_for(max_ctx, batch);
   return (int)(part < floor_part ? floor_part : part);
@@ -1578,10 +1587,14 @@ static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, i
   const int64_t max_ctx = (int64_t)max_num_blocks * block_size;
   const bool split = fast_ok && split_wanted(max_ctx, batch, num_kv_heads, int8);
   DecodePlan plan;
-  plan.part_tokens = split ? split_partition_tokens(max_ctx, batch, num_kv_heads, !int8 && dtype != MVLLM_F32) : partition_tokens_for(max_ctx, batch);
+  const bool sixteen_bit = !int8 && dtype != MVLLM_F32;
+  plan.part_tokens = split ? split_partition_tokens(max_ctx, batch, num_kv_heads, sixteen_bit, head_dim, block_size) : partition_tokens_for(max_ctx, batch);
   plan.num_parts = (int)((max_ctx + plan.part_tokens - 1) / plan.part_tokens);
-  const bool many = !int8 && dtype != MVLLM_F32 && (head_dim == 128 || head_dim == 64) && block_size % kTile == 0 &&
-                    (int64_t)batch * num_kv_heads * plan.num_parts <= (plan.num_parts == 1 ? 256 : 64);
+  const int64_t pairs = (int64_t)batch * num_kv_heads;
+  const bool few = (head_dim == 128 || head_dim == 64) && pairs * plan.num_parts <= (plan.num_parts == 1 ? 256 : 64);
+  // (from kSplitMinGroups pairs on a sequence is one partition anyway: two workgroups per CU and more)
+  const bool narrow_dim = head_dim < kSplitWideDim && max_ctx > kSplitOnePartCtx && pairs < kSplitMinGroups && split_one_part(max_ctx, pairs, head_dim, block_size);
+  const bool many = sixteen_bit && block_size % kTile == 0 && (few || narrow_dim);
   plan.waves_per_head = !fast_ok ? 0 : !split ? 1 : many ? kSplitManyWaves : kSplitWaves;
   return plan;
 }
@@ -1607,7 +1620,7 @@ static int launch_decode(DecodeArgs a, bool int8, bool fast_ok, int waves, hipSt
     const dim3 grid((unsigned)a.num_parts, (unsigned)a.batch, groups);
     auto go = [&](auto DIM) {
       constexpr int D = decltype(DIM)::value;
-      if constexpr (IsSixteenBit<T>::value && (D == 64 || D == 128)) {
+      if constexpr (IsSixteenBit<T>::value && (D < kSplitWideDim || D == 128)) {
         if (waves == kSplitManyWaves) {
           decode_mfma_split_kernel<T, kSplitManyWaves, D><<<split_grid, dim3(64 * kSplitManyWaves), 0, stream>>>(a);
           launched = true;

@@ -133,6 +133,10 @@ def test_decode_plan_in_narrow_tables():
     assert plan(5, 2048) == (256, 8, 4) and plan(8, 1024) == (128, 8, 4)              # ... from then on 256 tokens
     assert plan(8, 1040) == (256, 5, 4) and plan(31, 2048) == (704, 3, 4)
     assert plan(32, 2048) == (2048, 1, 8) and plan(33, 2048) == (2048, 1, 4)          # one from 256 pairs on; eight waves up to 256 workgroups
+    thin = lambda batch, tokens, d, block=16: paged_decode_plan(batch, 32, 8, d, tokens // block, block)
+    assert thin(33, 2048, 64) == thin(63, 2048, 32) == thin(63, 2048, 104) == (2048, 1, 8)             # below 112 dims eight waves
+    assert thin(33, 2048, 112) == thin(64, 2048, 64) == (2048, 1, 4) and thin(33, 512, 64) == (512, 1, 4)
+    assert thin(33, 2048, 64, 8) == (1024, 2, 4) and thin(33, 2048, 128, 8) == (2048, 1, 4)            # blocks of less than a tile
     assert plan(31, 2064) == (704, 3, 4) and plan(33, 2064) == (1088, 2, 4)
     assert plan(1, 2048, int8_cache=True)[0] == 64 and plan(1, 2048, dtype=torch.float32)[0] == 64
 

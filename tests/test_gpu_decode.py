@@ -90,13 +90,16 @@ def test_eight_waves_per_head(hq, hkv, d, bs, ctx_list):
     assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
 
 
-@pytest.mark.parametrize("batch,first,tokens,plan", [
-    (32, [2048, 1, 1025], 2048, (2048, 1, 8)), (33, [2048, 2047, 63], 2048, (2048, 1, 4)),         # whole sequences, eight waves and four
-    (33, [2060, 1088, 1089], 2064, (1088, 2, 4)), (31, [2048, 700, 705], 2048, (704, 3, 4)),       # cut: a table or a batch past the rule's end
-    (4, [2048, 128, 129, 1], 2048, (128, 16, 4)), (5, [2048, 256, 257], 2048, (256, 8, 4)),        # a few sequences
+@pytest.mark.parametrize("batch,first,tokens,d,plan", [
+    (32, [2048, 1, 1025], 2048, 64, (2048, 1, 8)), (33, [2048, 2047, 63], 2048, 64, (2048, 1, 8)),     # whole sequences, eight waves ...
+    (33, [2048, 1, 129], 2048, 32, (2048, 1, 8)), (40, [1024, 1000, 15], 1024, 80, (1024, 1, 8)), (33, [520, 300], 528, 104, (576, 1, 8)),
+    (33, [2048, 2047, 63], 2048, 128, (2048, 1, 4)), (33, [2048, 1, 900], 2048, 112, (2048, 1, 4)),    # ... or four
+    (64, [2048, 63], 2048, 64, (2048, 1, 4)), (33, [512, 63], 512, 64, (512, 1, 4)),
+    (33, [2060, 1088, 1089], 2064, 64, (1088, 2, 4)), (31, [2048, 700, 705], 2048, 64, (704, 3, 4)),   # cut: a table or a batch past the rule's end
+    (4, [2048, 128, 129, 1], 2048, 64, (128, 16, 4)), (5, [2048, 256, 257], 2048, 64, (256, 8, 4)),    # a few sequences
 ])
-def test_partitions_of_narrow_tables(batch, first, tokens, plan):
-    hq, hkv, d, bs = 16, 8, 64, 16
+def test_partitions_of_narrow_tables(batch, first, tokens, d, plan):
+    hq, hkv, bs = 16, 8, 16
     case = make_paged_case(41, batch, 1, 1, hq, hkv, d, bs, dtype=torch.bfloat16, ctx_list=first + [17 + 5 * i for i in range(batch - len(first))])
     q, kc, vc, tables, ctx = case
     tables = torch.nn.functional.pad(tables, (0, tokens // bs - tables.shape[1]), value=-1)
