@@ -127,6 +127,14 @@ constexpr int kLargeTileRows = 384;      // rows per expert from which tiles are
 // ... up to which they are small: at 47 per expert (500 rows, top 6 of 64, width 2048) 76 + 42 us against 98 + 44 as tiles of 128, at
 // 65 121 + 73 against 100 + 48: experts of two tiles read their weights twice.
 constexpr int kSmallTileRows = 48;
+// An expert's last large tile is apart from the others up to here: it is short and brings the chip's last round to an end.  With more rows it takes
+// its time and would read the weights again, which the expert's other tiles have in the L2.  us as all that are not whole, up to 64 rows,
+// none apart: 64 experts, 400 rows each, 1536 x 2048 203 / 182 / 180, of 896 x 2240 288 / 254 / 255; 768 350 / 307 / 337 and 688 / 629 / 669; the 8192 rows of
+// a mixture, top 6 of 64, routed unevenly, 820 / 802 / 827.
+constexpr int kApartRows = 64;
+// ... where there are rounds enough: with few tiles all run at once, and an expert's do so on one XCD (8 experts of 600 rows, 320 x 1536, 33.9 us none
+// apart and 35.7).
+constexpr int kApartPairs = 8192;
 
 struct PlanArgs {
   const int32_t* ids;      // [pairs]
@@ -178,7 +186,7 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
     }
   }
   // inclusive sums over the experts: within a wave, then over the waves before it
-  const bool apart = a.tile_rows == 256 && n % 256 != 0;      // the last tile, not whole, goes behind all whole ones
+  const bool apart = a.tile_rows == 256 && n % 256 != 0 && n % 256 <= kApartRows && a.pairs >= kApartPairs;      // the last tile goes behind all others
   int sums[3] = {n, (n + a.tile_rows - 1) / a.tile_rows - apart, apart};
   const int lane = e & 63, wave = __builtin_amdgcn_readfirstlane(e >> 6);
   const bool some = 64 * wave < a.experts;
@@ -412,24 +420,35 @@ __global__ __launch_bounds__(256) void moe_linear_any_kernel(const ExpertLinearA
 
 // The tile of rows and of weights that a workgroup of the tiled products takes; false: none.  Each XCD has an eighth of the (row tile,
 // weight tile) pairs, to one: shares of whole row tiles left the last XCD a third of the others' work (66 tiles: seven of 9, one of 3).
-// Row tiles go in fours: workgroups of a four with the same weight tile follow one another.  Large tiles that are not whole, and so take
-// less time, come behind all whole ones, in turns over the XCDs: the chip's last round is made of short ones.  600 rows, top 6 of 64
-// with uneven routing, width 2048: 132 + 71 -> 101 + 62 us; 8192 rows with what follows at the large kernel: 387 + 239 -> 376 + 222.
+// A share's pairs go by row tiles, in fours: workgroups of a four with the same weight tile follow one another, and where shares are
+// whole row tiles, as with few experts, none of them is read by two XCDs.  Large tiles with few rows come behind all others (see kApartRows), shared evenly too: the chip's last round is made of
+// short ones.  600 rows, top 6 of 64 with uneven routing, width 2048: 132 + 71 -> 101 + 62 us.
 __device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, int& n_tile) {
   constexpr int kTogether = 4;
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  const int whole = a.num_tiles[0], rest = a.num_tiles[1], per = (whole * a.n_tiles + 7) / 8;
-  if (j < per) {
-    const int at = xcd * per + j;
-    if (at >= whole * a.n_tiles) return false;
-    const int first = at / (kTogether * a.n_tiles) * kTogether, in = at - first * a.n_tiles, together = min(kTogether, whole - first);
-    tile = first + in % together;
-    n_tile = in / together;
-    return true;
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, n = a.n_tiles;
+  const int whole = a.num_tiles[0], rest = a.num_tiles[1], per = (whole * n + 7) / 8;
+  if (j >= per) {
+    const int rest_per = (rest * n + 7) / 8, at = xcd * rest_per + j - per;
+    tile = whole + at / n;
+    n_tile = at % n;
+    return j - per < rest_per && at < rest * n;
   }
-  tile = whole + xcd + 8 * ((j - per) / a.n_tiles);
-  n_tile = (j - per) % a.n_tiles;
-  return tile < whole + rest;
+  const int low = xcd * per, high = min(low + per, whole * n);
+  if (low + j >= high) return false;
+  // the last weight tiles of a row tile that the XCD before began, row tiles of its own, the first weight tiles of one more
+  const int first_own = (low + n - 1) / n, begun = first_own * n - low, own = high / n - first_own, at = j - begun;
+  if (at < 0) {
+    tile = first_own - 1;
+    n_tile = n + at;
+  } else if (at < own * n) {
+    const int first = at / (kTogether * n) * kTogether, in = at - first * n, together = min(kTogether, own - first);
+    tile = first_own + first + in % together;
+    n_tile = in / together;
+  } else {
+    tile = first_own + own;
+    n_tile = at - own * n;
+  }
+  return true;
 }
 
 // Step of K that a workgroup starts with; it comes round to the ones before it at its end.  Rows a multiple of 4 KB long start in the same channel

@@ -542,6 +542,31 @@ def test_moe_linear_row_tile_edges(counts, n, k):
     assert row_rel(out, want) < 1e-2
 
 
+@pytest.mark.parametrize("n,k", [(336, 2048), (160, 4096), (272, 192)])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("counts", [[63, 65, 0, 1, 129, 2, 32, 5, 64], [128, 60, 129, 300, 0, 57, 100],
+                                    [256, 257, 320, 321, 640, 700, 1023, 449, 2048, 1088, 1, 1600], [384, 400, 448, 500]], ids=["64", "128", "256", "256-few"])
+def test_moe_linear_walks_and_shares(counts, n, k, glu):
+    """Rows a multiple of 4 KB, where experts and weight tiles begin K at different steps, in every form; the shares of the XCDs with weight tiles that
+    they do not divide, last tiles of up to 64 rows behind all others (from 8192 pairs on) and longer ones in order."""
+    g = gen(n + k)
+    experts, pairs = len(counts), sum(counts)
+    ids = torch.cat([torch.full((c,), i) for i, c in enumerate(counts)])[torch.randperm(pairs, generator=g)].int().view(-1, 1)
+    x = torch.randn(pairs, k, generator=g).bfloat16()
+    w = (torch.randn(experts, n // 32 * 32 * (2 if glu else 1), k, generator=g) * k ** -0.5).bfloat16()
+    plan = moe_plan(ids.to(DEV), experts)
+    out = moe_linear(x.to(DEV), w.to(DEV), ids.to(DEV), plan, 1, glu).cpu()[plan.place.cpu().long()]
+    want = torch.empty(out.shape, dtype=torch.float64)
+    for e in range(experts):
+        rows = (ids.view(-1) == e).nonzero().view(-1)
+        z = x[rows].double() @ w[e].double().T
+        if glu:                                            # gate and up rows in turns of 32
+            gate, up = z.view(len(rows), n // 32, 2, 32).unbind(2)
+            z = (torch.nn.functional.silu(gate) * up).reshape(len(rows), -1)
+        want[rows] = z
+    assert row_rel(out, want) < 1e-2
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("cfg", [moe(), moe(experts=12, top=5, groups=(3, 2), ff=72, shared=100), moe(experts=5, top=1, groups=None, shared=None),
                                  moe(experts=40, top=8, groups=(8, 3), ff=64, shared=16)], ids=["a", "b", "c", "d"])
