@@ -553,7 +553,7 @@ def test_moe_linear_walks_and_shares(counts, n, k, glu):
     experts, pairs = len(counts), sum(counts)
     ids = torch.cat([torch.full((c,), i) for i, c in enumerate(counts)])[torch.randperm(pairs, generator=g)].int().view(-1, 1)
     x = torch.randn(pairs, k, generator=g).bfloat16()
-    w = (torch.randn(experts, n // 32 * 32 * (2 if glu else 1), k, generator=g) * k ** -0.5).bfloat16()
+    w = (torch.randn(experts, n // 32 * 64 if glu else n, k, generator=g) * k ** -0.5).bfloat16()
     plan = moe_plan(ids.to(DEV), experts)
     out = moe_linear(x.to(DEV), w.to(DEV), ids.to(DEV), plan, 1, glu).cpu()[plan.place.cpu().long()]
     want = torch.empty(out.shape, dtype=torch.float64)
@@ -562,8 +562,8 @@ def test_moe_linear_walks_and_shares(counts, n, k, glu):
         z = x[rows].double() @ w[e].double().T
         if glu:                                            # gate and up rows in turns of 32
             gate, up = z.view(len(rows), n // 32, 2, 32).unbind(2)
-            z = (torch.nn.functional.silu(gate) * up).reshape(len(rows), -1)
-        want[rows] = z
+            z = torch.nn.functional.silu(gate) * up
+        want[rows] = z.reshape(len(rows), out.shape[1])
     assert row_rel(out, want) < 1e-2
 
 
