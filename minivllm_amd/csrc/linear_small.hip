@@ -6,7 +6,7 @@
 // operand's lanes are sixteen different rows).  Hence two kernels:
 //   linear_rows_kernel (very few rows): weights and x straight into registers, eight rows x 128 bytes per load.
 //   linear_ring_kernel (more rows): W and x through a ring of tiles in LDS, copied as whole 128-byte lines.
-// Both read a weight once.  A sum's order depends on (M, N, K) and, from kStreamBytes of weights on, on the column; a long K with few columns is cut into
+// Both read a weight once, but for few columns' ring, whose tiles of 16 rows are apart (rows_apart).  A sum's order depends on (M, N, K) and, from kStreamBytes of weights on, on the column; a long K with few columns is cut into
 // parts where the caller brings room for their sums (linear_split).
 // mvllm_norm_linear_small_m is the same product with the launches around it folded in: the residual add + RMSNorm in
 // front of the layer's first projections (src/myvllm/models/qwen3.py:197-212 through layers/layernorm.py:9-28) as
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(const LinearArgs a)
   }
 }
 
-// More rows: a workgroup owns 16 CT SC output columns and all MT * 16 rows.  SK waves split the 64 SK values of a stage
+// More rows: a workgroup owns 16 CT SC output columns and MT * 16 rows, all or (blockIdx.z) some of them.  SK waves split the 64 SK values of a stage
 // between them, SC such groups the columns; a stage is WB + XB blocks of 8 rows x 128 bytes per 64 values, copied into a ring of
 // S of them (buffer loads to LDS: eight lines a wave and copy, no registers, S - 1 stages under way; a row's eight pieces
 // trade places by the row's number, which spreads both the copies' and the reads' banks).  One barrier a stage: behind it
@@ -195,7 +195,9 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
   const uint32_t row_bytes = (uint32_t)a.K * 2u;
   const char* w0 = reinterpret_cast<const char*>(a.w) + (int64_t)first * row_bytes;
   const uint32_t w_bytes = (uint32_t)min(left, kSpan) * row_bytes;
-  const uint32_t x_bytes = ((uint32_t)(a.M - 1) * (uint32_t)a.x_row_stride + (uint32_t)a.K) * 2u;
+  const int m0 = 16 * MT * (int)blockIdx.z, rows = min(a.M - m0, 16 * MT);
+  const char* x0 = reinterpret_cast<const char*>(a.x) + (int64_t)m0 * a.x_row_stride * 2;
+  const uint32_t x_bytes = ((uint32_t)(rows - 1) * (uint32_t)a.x_row_stride + (uint32_t)a.K) * 2u;
   const int r8 = lane >> 3;
   const uint32_t piece = (uint32_t)(sk * 128 + (((lane & 7) ^ r8) << 4));
   uint32_t from[kCopies];                                  // rows past the last repeat it
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
     constexpr int i = decltype(I)::value;
     const int b = i * SC + sc;
     if constexpr (i < 2 * CT) from[i] = (uint32_t)min(8 * (GLU ? b >> 1 : b) + r8, left - 1) * row_bytes + piece;
-    else from[i] = (uint32_t)min(8 * (b - WB) + r8, a.M - 1) * (uint32_t)a.x_row_stride * 2u + piece;
+    else from[i] = (uint32_t)min(8 * (b - WB) + r8, rows - 1) * (uint32_t)a.x_row_stride * 2u + piece;
   });
   const int step0 = a.part_steps * (int)blockIdx.y, steps = min(a.K / (64 * SK) - step0, a.part_steps);    // of this workgroup's part of K
   // Rows a multiple of 4 KB long start in the same channel of the L2 and of the memory: workgroups that walk K in step would all read
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
   const uint32_t lds0 = lds_address(lds) + sk * kPanel + sc * 1024;
   auto copy = [&](int step, int buffer) __attribute__((always_inline)) {
     const bool live = step < steps;
-    const v4i x_rows = make_rsrc(reinterpret_cast<const char*>(a.x), live ? x_bytes : 0u);
+    const v4i x_rows = make_rsrc(x0, live ? x_bytes : 0u);
     const v4i w_rows = make_rsrc(w0, live ? w_bytes : 0u);
     const v4i up_rows = GLU ? make_rsrc(w0 + (int64_t)out_cols * row_bytes, live ? w_bytes : 0u) : w_rows;
     const uint32_t at = live ? (uint32_t)(step0 + (step < steps - turn ? step + turn : step + turn - steps)) * (SK * 128) : 0u, base = lds0 + buffer * kStage;
@@ -277,7 +279,7 @@ __global__ __launch_bounds__(64 * SK * SC) void linear_ring_kernel(const LinearA
       for (int r = 0; r < 4; ++r) u[r] = __shfl_xor(s[r], 32, 64);
       if (cls >= 2) continue;
     }
-    const int m = 16 * (mc / CT) + col, j = first + (GLU ? 8 : 16) * (c * CT + mc % CT) + 4 * cls;
+    const int m = m0 + 16 * (mc / CT) + col, j = first + (GLU ? 8 : 16) * (c * CT + mc % CT) + 4 * cls;
     if (!GLU && a.part) {
       if (m < a.M && j < a.N) *reinterpret_cast<float4*>(a.part + ((int64_t)blockIdx.y * a.M + m) * a.N + j) = make_float4(s[0], s[1], s[2], s[3]);
     } else {
@@ -473,6 +475,13 @@ static LinearSplit linear_split(int M, int N, int K) {
   return {columns, splits < 4 ? splits : 4};
 }
 
+// Few columns leave CUs without a workgroup, and each one with all the rows copies `rows + 16` rows of K values one stage after the other: the tiles of
+// 16 rows as workgroups of their own read the weights once each, from the L2 after the first, and copy 32 rows.  While they find a CU each: past
+// 256 the second round costs more than the rows.  us whole / apart: 49 x 512 x 14336 34.5 / 16.0, 64 x 512 x 4096 10.0 / 5.8, 17 x 2048 x 4096
+// (256 workgroups) 8.4 / 7.4, 64 x 1024 x 4096 gated (256) 10.7 / 6.8; 33 x 2048 x 14336 gated (384) 29.2 / 36.4, 17 x 2720 x 4096 (340)
+// 9.0 / 12.7.  A long K with 1024 columns on is cut into parts instead where the caller brings the room (64 x 1024 x 14336 15.7, apart 19.3).
+static bool rows_apart(int M, int N) { return (N + 15) / 16 * ((M + 15) / 16) <= 256; }
+
 template <typename T, bool GLU>
 static int launch_rows(const LinearArgs& a, hipStream_t stream) {
   // few columns: narrow tiles and more waves on a tile's K, to have more loads under way.  us at one row with 8 columns and 8 / 4 waves, 16 columns
@@ -497,7 +506,7 @@ static int launch_ring(LinearArgs a, hipStream_t stream) {
   const LinearSplit split = a.part ? linear_split(a.M, a.N, a.K) : LinearSplit{ring_columns(a.M, a.N), 1};
   const int columns = split.columns, steps = a.K / (columns == 16 ? 256 : 128);
   a.part_steps = (steps + split.splits - 1) / split.splits;
-  const dim3 grid((unsigned)((a.N + columns - 1) / columns), (unsigned)split.splits);
+  const dim3 grid((unsigned)((a.N + columns - 1) / columns), (unsigned)split.splits, (unsigned)((a.M + 16 * MT - 1) / (16 * MT)));
   constexpr int S = MT > 2 ? 3 : 4;
   switch (columns) {
     case 16:
@@ -531,7 +540,7 @@ static int launch_plain(const LinearArgs& a, hipStream_t stream) {
     }
     return MVLLM_OK;
   }
-  if (a.M <= 16) return launch_ring<T, 1, GLU>(a, stream);
+  if (a.M <= 16 || (!a.part && rows_apart(a.M, a.N))) return launch_ring<T, 1, GLU>(a, stream);
   if (a.M <= 32) return launch_ring<T, 2, GLU>(a, stream);
   if (a.M <= 48) return launch_ring<T, 3, GLU>(a, stream);
   return launch_ring<T, 4, GLU>(a, stream);

@@ -58,6 +58,27 @@ def test_linear_small_m_tile_edges(m, n, k):
     assert slack.max().item() <= 2e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n", [(17, 2048), (17, 2080), (33, 1344), (33, 1376), (64, 1024), (64, 1056), (49, 32), (48, 96)])
+@pytest.mark.parametrize("k", [512, 2560])
+def test_linear_small_m_tiles_of_rows_apart(dtype, m, n, k):
+    """Few columns: tiles of 16 rows as workgroups of their own, at both sides of the line (256 of them: the first of each pair of shapes) and
+    with a last tile of one row; strided rows, a plain, a gelu and a gated product."""
+    x, w, b = _case(600 + m, m, n, k, dtype, True, stride=k + 24)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    full = x.float() @ w.float().T + b.float()
+    for gelu in (False, True):
+        want = F.gelu(full, approximate="tanh") if gelu else full
+        err = (linear_small_m(x, w, b, gelu).float() - want).abs() - want.abs() * ulp
+        assert err.max().item() <= 2e-3
+    gate, up = full.to(dtype).float().chunk(2, 1)
+    want = F.silu(gate) * up
+    got = norm_linear_small_m(x.contiguous(), w, b, glu=True).float()
+    # as in the tile edges' test: a unit of the gate or of the up value that rounds the other way, and the two roundings behind them
+    slack = (got - want).abs() - 4 * ulp * (F.silu(gate).abs() + gate.abs() + 1) * (up.abs() + 1)
+    assert slack.max().item() <= 2e-3
+
+
 @pytest.mark.parametrize("m", [4, 17, 33, 64])
 @pytest.mark.parametrize("n,k", [(1360, 6656), (2032, 6656), (4112, 12800), (5440, 6144), (1024, 3072)])
 def test_linear_small_m_splits_of_k(m, n, k):
