@@ -79,6 +79,15 @@ def test_linear_small_m_tiles_of_rows_apart(dtype, m, n, k):
     assert slack.max().item() <= 2e-3
 
 
+@pytest.mark.parametrize("m", [1, 2, 3])
+@pytest.mark.parametrize("n,k", [(32, 512), (32, 1024), (1056, 1536), (2080, 512), (8192, 512), (8224, 1024)])
+def test_gated_product_of_few_rows_pairs_gate_and_up(m, n, k):
+    """One to three rows: the gated product is, bit for bit, silu_and_mul of the plain one (a column's sum has the same order in both), at every
+    number of waves and tiles and with last tiles that are not full."""
+    x, w, b = _case(800 + m, m, n, k, torch.bfloat16, True)
+    assert torch.equal(norm_linear_small_m(x, w, b, glu=True), silu_and_mul(linear_small_m(x, w, b)))
+
+
 @pytest.mark.parametrize("m", [4, 17, 33, 64])
 @pytest.mark.parametrize("n,k", [(1360, 6656), (2032, 6656), (4112, 12800), (5440, 6144), (1024, 3072)])
 def test_linear_small_m_splits_of_k(m, n, k):
