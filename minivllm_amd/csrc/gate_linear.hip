@@ -41,6 +41,10 @@ constexpr int kFewRows = 512;        // up to here K is split over sixteen waves
 // Up to here operands go straight into registers, whose call has less of a fixed part.  us so and through LDS: 8192 rows x 65, K 320 6.0 / 6.9,
 // 512 7.7 / 7.0, 1024 12.3 / 8.8; 30000 x 200, K 512 61 / 65, 1024 113 / 80; 32 x 65, K 512 3.0 / 2.9, 1024 3.8 / 3.2.
 constexpr int kShortK = 512;
+// Up to kFewRows the line also moves with the tile's rows and columns, as repeated rows cost the address unit nothing: registers while K times (rows + columns
+// of a tile) is no more.  us in registers / through LDS: 1 x 1, K 1024 2.4 / 2.9, 4096 3.6 / 4.1; 4 x 4, K 1536 3.0 / 3.2, 2048 3.4 / 3.3;
+// 8 x 8, K 1024 3.0 / 3.0, 2048 4.0 / 3.4; 16 x 8, K 576 2.75 / 2.8; 16 x 16, K 704 3.2 / 2.9; 4 x 2, K 2048 3.2 / 3.3, 3072 3.8 / 3.7, 4096 4.3 / 4.1.
+constexpr int64_t kRegisterLines = 16384;
 constexpr int kManyRows = 4096;      // from here 32 rows to a workgroup: they fill the CUs and read W half as often
 
 // Whole rows of x and W through LDS: a matrix operand's lanes are sixteen different rows, which a CU's address unit takes at 16 B per
@@ -240,7 +244,8 @@ extern "C" int mvllm_gate_linear(float* out, const void* x, int64_t x_row_stride
   const unsigned tiles = (unsigned)((rows + 15) / 16), columns = (unsigned)((N + 15) / 16);
   hipStream_t s = (hipStream_t)stream;
   const bool vec = K % 8 == 0 && x_row_stride % 8 == 0 && aligned16(x) && aligned16(w), full = vec && K % 64 == 0;
-  const bool ring = full && K > kShortK && std::max(32 * x_row_stride, 80 * (int64_t)K) * 2 < (int64_t)1 << 32;   // a descriptor's offsets
+  const bool wide = rows > kFewRows || (int64_t)K * (std::min((int)rows, 16) + std::min(N, 16)) > kRegisterLines;
+  const bool ring = full && wide && K > kShortK && std::max(32 * x_row_stride, 80 * (int64_t)K) * 2 < (int64_t)1 << 32;   // a descriptor's offsets
   if (dtype == MVLLM_F32) gate_linear_f32_kernel<<<dim3(tiles, columns), dim3(256), 0, s>>>(a);
   else if (!full) gate_linear_bf16_kernel<4, 1, false><<<dim3(tiles, columns), dim3(256), 0, s>>>(a, vec);
   else if (rows <= kFewRows && ring) gate_linear_ring_kernel<1, 1, 16, 1, 2><<<dim3(tiles, columns), dim3(1024), 0, s>>>(a);

@@ -356,6 +356,17 @@ def test_gate_linear(dtype, rows, n, k):
         assert got.dtype == torch.float32 and rel(got, want) < 2e-6      # also for bf16 inputs: fp32 from the product on
 
 
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 1024), (8, 8, 1024), (9, 8, 1024), (16, 8, 576), (16, 16, 576), (2, 1, 6976), (1, 17, 960), (512, 1, 576)])
+def test_gate_linear_of_a_part_of_the_rows_and_columns(rows, n, k):
+    """Few rows and columns go through registers, more through LDS, at both sides of the line: a sum has the same order in both (sixteen partial
+    sums up to 512 rows), so that a part of the rows and columns equals that part of a larger call to the bit."""
+    r = gen(k)
+    x, w = torch.randn(512, k, generator=r).bfloat16().to(DEV), torch.randn(max(n, 33), k, generator=r).bfloat16().to(DEV)
+    got, whole = gate_linear(x[:rows], w[:n], None, n, 0.0), gate_linear(x, w, None, len(w), 0.0)
+    assert torch.equal(got, whole[:rows, :n])
+    assert rel(got, x[:rows].cpu().double() @ w[:n].cpu().double().T) < 2e-6
+
+
 def _memory_case(seed, rows, heads, dim, vdim, dtype, forget=2.0, spread=2.0):
     r = gen(seed)
     col = heads * (2 * dim + vdim)
