@@ -457,11 +457,17 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
 // 588 (320) 34.3 / 36.6 1.90; behind 95 %, nine of 128 (32 heads, 360) 59 / 71 2.0.  Uneven ones meet by chance: 3300 rows of two
 // (60 and 40 %) 44.2 / 38.3, of three 43.9 / 34.6.  Cached batches do not tell whether they are even and count as if.  (Above 112 tiles the
 // other form cuts its keys too, and loses on either side of the line.)
+// An odd head group has row tiles of 128 here as there, so that nothing is gained from shorter ones: packed batches lose (us there and here, ten prompts of
+// 332, 12 heads over 4: 15.5 / 19.6; five of 764, 14 over 2: 22.7 / 28.7), but where the other form's places of 256 rows pass the chip's 512 and
+// these workgroups do not; cached ones gain what its empty places cost (seven of 40 to 70 rows behind as many, 40 over 8: 19.1 / 11.7; ten of
+// 163, 12 over 4, no empty places: 15.1 / 17.5) and where most keys are cached, so that tiles are alike (857 batches of random sizes behind 90 and 95 %:
+// 1.18 and 1.21 times as fast); few workgroups with few keys gain nothing (below 8 tiles 0.98).
 // At head_dim 64 the other form is this kernel over its banded order, 256 rows of a sequence at a time, the heaviest first: it pays for
-// packed batches as soon as their tiles differ (3500 rows, 448 workgroups: 30 us, here 33).  Cached ones pay its empty places, which fill the
-// chip's 512 the sooner, and gain from its order where they have more than one workgroup per CU and still fit: us there and here, 32
-// heads, four of 418 rows (512 places) of 758 keys 17.3 / 19.1, of 1142 23.5 / 25.0, of 518 (768) 26.5 / 20.2 and 38.3 / 30.3; of 118 (256 and
-// 240 workgroups) 15.2 / 14.9; eight of 93 (512 and 192) 19.1 / 15.8; from 30 tiles on a start counts less: 37.5 / 37.3.
+// packed batches as soon as their tiles differ (3500 rows, 448 workgroups: 30 us, here 33; equal ones of a busiest CU above 1.5, three of 1925, 8
+// heads, 27.7 / 35.2, of 1181, 12 heads over 4, 18.0 / 23.1).  Cached ones pay its empty places, which fill the
+// chip's 512 the sooner; up to there its order gains where the CUs differ and most keys are not cached: us there and here, two of 1852 rows
+// behind as many, 16 heads (480 workgroups of 512 places, busiest 1.97) 60.4 / 67.6, three of 1266, 16 over 2 (480, 1.8) 43.3 / 49.3; four of 418
+// of 758 keys, 32 heads (512 places) 17.3 / 19.1; beyond, of 518 of 958 (768) 26.5 / 20.2; eight of 93 of 168 (512 and 192) 19.1 / 15.8.
 // A few rows at head_dim 64 stay there, where placing the bands costs nothing (23 rows 8.8 / 9.5; from 5 sequences of 32 heads and 10 of 16
 // on 12.3 / 11.0), and so do 200 workgroups with more than 7000 keys, whose ranges the other form cuts (four heads of 128 121 / 128, of 64
 // 88 / 97, two of 64 80 / 96).
@@ -475,19 +481,24 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
   if (!ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype)) return 0;
   const int group = num_heads / num_kv_heads, bm = rows_of_tile(group);
   const int64_t slices = (int64_t)num_heads * bm / 128, wgs = (total_q_tokens / bm + num_seqs) * slices, tiles = ranges_of(max_kv_len, 1);
-  const bool four = group % 4 == 0, paged = block_size > 0;
+  const bool four = group % 4 == 0, odd = group % 2 != 0, paged = block_size > 0;
   const int limit = head_dim == 64 ? (paged ? 768 : tiles >= 16 && !four ? 384 : 0)
                     : !four        ? (tiles >= 16 ? 512 : tiles >= 7 ? 580 : 640)
                                    : tiles >= 12 ? 384 : 300;
   if (wgs > limit) return 0;
-  // were all sequences as long as their mean: workgroups that have rows, the other form's places (10 % of the rows more, for those that are longer)
+  // were all sequences as long as their mean: workgroups that have rows, the other form's places
   const int64_t even = num_seqs * ((total_q_tokens + (int64_t)num_seqs * bm - 1) / ((int64_t)num_seqs * bm)) * slices;
-  const int64_t places = num_seqs * ((total_q_tokens * 11 / 10 + (int64_t)num_seqs * 256 - 1) / ((int64_t)num_seqs * 256)) * (256 / bm) * slices;
+  const int64_t places = num_seqs * ((total_q_tokens + (int64_t)num_seqs * 256 - 1) / ((int64_t)num_seqs * 256)) * (256 / bm) * slices;
   const float fresh = fminf(1.f, (float)total_q_tokens / ((float)num_seqs * (float)max_kv_len));
+  const bool crowded = num_seqs > 1 && even > 272;
   if (head_dim == 64) {
-    if (paged && num_seqs <= 8 && even > 256 && places <= 512 && tiles < 30) return 0;
-  } else if (num_seqs > 1 && even > 272 && tiles >= 16 && (paged ? tiles <= 112 : fresh >= 0.87f)) {
-    if (busiest_cu(even, num_seqs, fresh) > (paged ? 1.85f : 1.75f)) return 0;
+    if (crowded && (paged ? fresh >= 0.3f && places <= 512 && 10 * places <= 13 * even : fresh >= 0.75f) &&
+        busiest_cu(even, num_seqs, fresh) > (paged ? 1.7f : 1.5f))
+      return 0;
+  } else {
+    if (odd && !paged && (places <= 512 || even > 512 || total_q_tokens <= (int64_t)bm * num_seqs)) return 0;
+    if (odd && paged && wgs > 192 && places <= 512 && 10 * places <= 11 * even && fresh >= 0.25f) return 0;
+    if (crowded && tiles >= 16 && (paged ? tiles <= 112 : fresh >= 0.87f) && busiest_cu(even, num_seqs, fresh) > (paged ? 1.85f : 1.75f)) return 0;
   }
   int64_t p = (tiles + 1) / 2 * 2;
   if (wgs > 192) return (four || head_dim == 64) && tiles > 112 ? 0 : (int)p;
@@ -502,7 +513,7 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
       p = x;
     }
   }
-  return head_dim == 64 && p >= tiles && wgs < (four ? 48 : 80) ? 0 : (int)p;
+  return p >= tiles && (head_dim == 64 ? wgs < (four ? 48 : 80) : odd && tiles < 8) ? 0 : (int)p;
 }
 
 extern "C" size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim, int range_tiles) {

@@ -95,6 +95,26 @@ def test_prefill_ranges_plan_looks_at_the_busiest_cu():
     assert plan(4, 1672, 1910, *four, *paged) == 30                                                    # long
 
 
+def test_prefill_ranges_plan_of_odd_head_groups():
+    """Row tiles of 128 in both forms: packed batches go over only where the other form's places pass the chip's 512, cached ones for its
+    empty places, for alike tiles or for keys cut into ranges."""
+    plan = _lib().load().mvllm_prefill_ranges_plan
+    packed, paged = (0, 1), (16, 1)
+    assert plan(10, 3320, 363, 12, 4, 128, *packed) == 0 and plan(5, 3820, 764, 14, 2, 128, *packed) == 0       # no more than 512 places
+    assert plan(3, 1200, 400, 40, 8, 128, *packed) == 0                                                        # 480 places
+    assert plan(4, 1120, 280, 40, 8, 128, *packed) == 6                                                        # 640 places, 480 workgroups
+    assert plan(9, 1152, 128, 40, 8, 128, *packed) == 0                                                        # short: empty places cost nothing
+    assert plan(1, 1000, 1000, 12, 4, 128, *packed) == 0
+    assert plan(7, 378, 138, 40, 8, 128, *paged) == 4 and plan(10, 1630, 325, 12, 4, 128, *paged) == 0          # empty places, none
+    assert plan(10, 1630, 1630, 12, 4, 128, *paged) == 26                                                      # most keys cached
+    assert plan(2, 60, 300, 12, 4, 128, *paged) == 0 and plan(2, 60, 500, 12, 4, 128, *paged) == 8              # few, 5 and 8 tiles of keys
+    assert 0 < plan(1, 100, 32768, 12, 4, 128, *paged) < 512
+    at64 = (8, 8, 64)
+    assert plan(3, 5775, 1925, *at64, *packed) == 0 and plan(3, 5000, 2600, *at64, *packed) == 42              # equal and uneven
+    assert plan(2, 3704, 3703, 16, 16, 64, *paged) == 0 and plan(2, 3704, 18500, 16, 16, 64, *paged) == 0      # 1.97; too many keys
+    assert plan(10, 4700, 948, 16, 16, 64, *paged) == 16                                                       # 640 places
+
+
 def test_prefill_split_plan_is_host_arithmetic():
     """When a paged prefill is cut over its keys: few query tiles, at least 4096 keys, a shape the split form takes;
     and the workspace holds the ranges' tables, partial results and denominators."""
