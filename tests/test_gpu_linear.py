@@ -88,6 +88,24 @@ def test_gated_product_of_few_rows_pairs_gate_and_up(m, n, k):
     assert torch.equal(norm_linear_small_m(x, w, b, glu=True), silu_and_mul(linear_small_m(x, w, b)))
 
 
+@pytest.mark.parametrize("m", [4, 16, 17, 33, 64])
+@pytest.mark.parametrize("n,k", [(3104, 2048), (1568, 4096), (4128, 2048), (4128, 4096), (12320, 2048), (24608, 2048)])
+def test_linear_small_m_walks_of_large_weights(m, n, k):
+    """Weights of 12 MiB and more with rows a multiple of 4 KB: column tiles begin K a quarter apart, in every tile width, whole and gated and with
+    tiles of rows apart; the last column tile is not full."""
+    assert n * k * 2 >= 12 << 20 and k % 2048 == 0
+    x, w, b = _case(900 + m, m, n, k, torch.bfloat16, True, stride=k + 24)
+    full = x.float() @ w.float().T + b.float()
+    err = (linear_small_m(x, w, b).float() - full).abs() - full.abs() * 2.0 ** -8
+    assert err.max().item() <= 2e-3
+    gate, up = full.bfloat16().float().chunk(2, 1)
+    want = F.silu(gate) * up
+    got = norm_linear_small_m(x.contiguous(), w, b, glu=True).float()
+    # as in the tile edges' test
+    slack = (got - want).abs() - 4 * 2.0 ** -8 * (F.silu(gate).abs() + gate.abs() + 1) * (up.abs() + 1)
+    assert slack.max().item() <= 2e-3
+
+
 @pytest.mark.parametrize("m", [4, 17, 33, 64])
 @pytest.mark.parametrize("n,k", [(1360, 6656), (2032, 6656), (4112, 12800), (5440, 6144), (1024, 3072)])
 def test_linear_small_m_splits_of_k(m, n, k):
