@@ -470,8 +470,9 @@ int mvllm_norm_linear_small_m(void* out, void* residual_out, const void* x, cons
 
 /*
  * Whether mvllm_linear_small_m (norm == 0 && glu == 0) or mvllm_norm_linear_small_m takes a shape, without a
- * launch: MVLLM_OK and in *waves (may be NULL) the number of parts K is cut into for this shape (with the norm: the fewest of 4, 8
- * or 16 whose 128 or 256 values each give 1024 parts in all), or MVLLM_ERR_UNSUPPORTED.  No counterpart
+ * launch: MVLLM_OK and in *waves (may be NULL) a number that only defines the set of shapes: of the parts of 128 or 256 values
+ * that K can be cut into, 4, 8 or 16, the fewest that give 1024 in all.  No kernel cuts K by it (the norm's has eight waves,
+ * mvllm_linear_small_m_split's parts are its own).  Otherwise MVLLM_ERR_UNSUPPORTED.  No counterpart
  * in the reference (its projections are library GEMMs of any shape).
  */
 int mvllm_linear_small_m_plan(int M, int N, int K, int norm, int glu, int dtype, int* waves);

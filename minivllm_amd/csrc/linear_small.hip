@@ -533,7 +533,7 @@ static int launch_ring(LinearArgs a, hipStream_t stream) {
 template <typename T, bool GLU>
 static int launch_plain(const LinearArgs& a, hipStream_t stream) {
   if (a.M <= kFewRows) return launch_rows<T, GLU>(a, stream);
-  if (((int64_t)(a.M - 1) * a.x_row_stride + a.K) * 2 > 0xffffffffll) {      // past a buffer descriptor's offsets: eight rows at a time
+  if (((int64_t)(a.M - 1) * a.x_row_stride + a.K) * 2 > 0xffffffffll) {      // past a buffer descriptor's offsets: kFewRows at a time
     LinearArgs part = a;
     for (int m = 0; m < a.M; m += kFewRows) {
       part.x = reinterpret_cast<const T*>(a.x) + (int64_t)m * a.x_row_stride;
