@@ -101,7 +101,7 @@ class RaggedStep:
 
 BLOCK_ROWS = 64                # rows per block of a recurrence's block form: segments are whole blocks
 FILL_WORKGROUPS = 512          # segments are made shorter until there are this many workgroups ...
-# ... but not shorter than this or twice this, and portions of a few of them stay whole (see _segments): the states' own pass, two launches and
+# ... but not shorter than this or twice this, and batches whose longest portion has a few of them stay whole (see _segments): the states' own pass, two launches and
 # their way through memory have to pay.  One portion of 700 rows, 16 heads of 128 x 256: 43 us (256: 55, 64: 40), 2000 rows, 8 heads: 50 (60, 57), 200
 # rows in two segments 36 against 31 whole.
 MIN_SEGMENT_ROWS = 128
@@ -119,23 +119,27 @@ def _segments(lens, cu, units, coarse=False):
     1024 45 / 56, one portion of 5000 rows, a chain of 40 segments, 54 / 58, but of 8000, a chain of 63, 75 / 66 (8 of 64 x 64, 6000 rows, 47, 74 / 71)."""
     long_entries = [e for e, n in enumerate(lens) if n >= LONG_ROWS]
     total = int(sum(lens[e] for e in long_entries))
+    longest = max((int(lens[e]) for e in long_entries), default=0)
     length = total
     if long_entries and units and len(long_entries) * units < FILL_WORKGROUPS // 2:
-        longest = max(int(lens[e]) for e in long_entries)
         many = total * units > FILL_WORKGROUPS // 2 * MIN_SEGMENT_ROWS if coarse else longest > MAX_CHAIN * MIN_SEGMENT_ROWS
         length = -(-total * units // (FILL_WORKGROUPS * BLOCK_ROWS)) * BLOCK_ROWS
         if length <= MIN_SEGMENT_ROWS:
             length = MIN_SEGMENT_ROWS * (2 if many else 1)
-    # the rows from which cutting pays: its two more launches take the longer the more there is to combine.  us whole and cut, memory of 128 x 256:
-    # 8 heads, one portion of 256 rows 34.5 / 35.4, of 300 37 / 35.5; two of 256 35 / 38.5, of 384 44 / 41; eight of 256 42 / 55, of 384 54 / 61, of
-    # 512 69 / 67.5.  Coarse ones, two portions of 300 rows: decay memory of 16 heads of 128 x 128 35.6 / 32.2, of 8 of 256 x 256 57.5 / 51.6, eight of
-    # 4 of 256 x 64 93 / 61
-    busy = len(long_entries) * (units or 0)
-    least = MIN_SEGMENT_ROWS * (4 if busy <= (32 if coarse else 16) else 5 if busy <= 64 else 7) // 2
+    # The longest portion's rows from which cutting pays, then for all portions: two more launches and the states' way through memory take the longer
+    # the more runs beside it, in workgroups of the longest one's length.  us whole and cut, memory of 128 x 256: 8 heads, one portion of 256 rows 34.5 / 35.4,
+    # of 300 37 / 35.5; two of 256 35 / 38.5, of 384 44 / 41; eight of 256 42 / 55, of 384 54 / 61, of 512 69 / 67.5.  Coarse ones lose more at few
+    # rows, where they have the CUs to themselves, and gain less at many: 8 heads of 256 x 256, one portion of 180 rows 36.7 / 43.2, four of 323 68 / 57, eight
+    # of 556 102 / 137; 16 heads of 128 x 128, two of 300 35.6 / 32.2.  In 3947 random batches of 13 sizes of memory the rule takes 1.005
+    # times the better of the two, cutting always 1.08.  (The longest decides for all: 313, 161 and 523 rows, 8 heads of 128 x 256, 52 all cut, 56 with the
+    # first two whole.)
+    beside = (units or 0) * total / max(longest, 1)
+    if longest <= (max(3 * BLOCK_ROWS, 150 + beside * beside / 25) if coarse else 224 + 2 * beside):
+        length = total
     out = []
     for e in long_entries:
         n, at = int(lens[e]), int(cu[e])
-        pieces = max(-(-n // length), 1) if n > least else 1
+        pieces = max(-(-n // length), 1)
         size = -(-n // (pieces * BLOCK_ROWS)) * BLOCK_ROWS
         cuts = list(range(0, n, size)) + [n]
         for i, (lo, hi) in enumerate(zip(cuts, cuts[1:])):

@@ -182,11 +182,14 @@ def _brute_force(seqs, window, bs, index):
 
 @pytest.mark.parametrize("lens,units,coarse,rows", [
     ([256], 16, False, [[256]]), ([257], 16, False, [[128, 128, 1]]),                         # from the rows on from which cutting pays ...
-    ([300] * 2, 16, False, [[300]] * 2), ([321] * 2, 16, False, [[128, 128, 65]] * 2),         # ... more of them beside others
-    ([448] * 5, 16, False, [[448]] * 5), ([449] * 5, 16, False, [[128, 128, 128, 65]] * 5),
+    ([288] * 2, 16, False, [[288]] * 2), ([289] * 2, 16, False, [[128, 128, 33]] * 2),         # ... more of them beside others
+    ([384] * 5, 16, False, [[384]] * 5), ([385] * 5, 16, False, [[128, 128, 128, 1]] * 5),
+    ([313, 161, 523], 16, False, [[128, 128, 57], [128, 33], [128] * 4 + [11]]),               # the longest one decides for all
+    ([192], 16, True, [[192]]), ([163, 213, 163], 4, True, [[128, 35], [128, 85], [128, 35]]),
+    ([314] * 4, 16, True, [[128, 128, 58]] * 4),
     ([1024] * 4, 16, False, [[128] * 8] * 4), ([1024] * 4, 16, True, [[256] * 4] * 4),         # two workgroups to a CU, or one
     ([512] * 4, 16, True, [[128] * 4] * 4), ([520] * 4, 16, True, [[192, 192, 136]] * 4),
-    ([300] * 2, 16, True, [[128, 128, 44]] * 2), ([300] * 3, 16, True, [[300]] * 3),
+    ([300] * 2, 16, True, [[128, 128, 44]] * 2), ([313] * 4, 16, True, [[313]] * 4),
     ([5120], 8, False, [[128] * 40]), ([5124], 8, False, [[256] * 20 + [4]]),                  # a chain of 40 segments at most
     ([4160], 16, True, [[192] * 21 + [128]]),                                                  # longer ones to fill the chip: as they come
     ([8000], 4, True, [[128] * 62 + [64]]),                                                    # (not where workgroups take long)
