@@ -467,7 +467,8 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
 // heads, 27.7 / 35.2, of 1181, 12 heads over 4, 18.0 / 23.1).  Cached ones pay its empty places, which fill the
 // chip's 512 the sooner; up to there its order gains where the CUs differ and most keys are not cached: us there and here, two of 1852 rows
 // behind as many, 16 heads (480 workgroups of 512 places, busiest 1.97) 60.4 / 67.6, three of 1266, 16 over 2 (480, 1.8) 43.3 / 49.3; four of 418
-// of 758 keys, 32 heads (512 places) 17.3 / 19.1; beyond, of 518 of 958 (768) 26.5 / 20.2; eight of 93 of 168 (512 and 192) 19.1 / 15.8.
+// of 758 keys, 32 heads (512 places) 17.3 / 19.1, of 350 (352 of 512) 21.4 / 23.3; with tiles of 64 or 128 rows a third of the places empty ends
+// that (1.03 times as fast here in 40 random batches); beyond, of 518 of 958 (768) 26.5 / 20.2; eight of 93 of 168 (512 and 192) 19.1 / 15.8.
 // A few rows at head_dim 64 stay there, where placing the bands costs nothing (23 rows 8.8 / 9.5; from 5 sequences of 32 heads and 10 of 16
 // on 12.3 / 11.0), and so do 200 workgroups with more than 7000 keys, whose ranges the other form cuts (four heads of 128 121 / 128, of 64
 // 88 / 97, two of 64 80 / 96).
@@ -492,7 +493,7 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
   const float fresh = fminf(1.f, (float)total_q_tokens / ((float)num_seqs * (float)max_kv_len));
   const bool crowded = num_seqs > 1 && even > 272;
   if (head_dim == 64) {
-    if (crowded && (paged ? fresh >= 0.3f && places <= 512 && 10 * places <= 13 * even : fresh >= 0.75f) &&
+    if (crowded && (paged ? fresh >= 0.3f && places <= 512 && (four || 10 * places <= 13 * even) : fresh >= 0.75f) &&
         busiest_cu(even, num_seqs, fresh) > (paged ? 1.7f : 1.5f))
       return 0;
   } else {

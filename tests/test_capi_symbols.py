@@ -111,6 +111,7 @@ def test_prefill_ranges_plan_of_odd_head_groups():
     assert plan(10, 1630, 1630, 12, 4, 128, *paged) == 26                                                      # most keys cached
     assert plan(2, 60, 300, 12, 4, 128, *paged) == 0 and plan(2, 60, 500, 12, 4, 128, *paged) == 8              # few, 5 and 8 tiles of keys
     assert 0 < plan(1, 100, 32768, 12, 4, 128, *paged) < 512
+    assert plan(4, 1397, 700, 32, 8, 64, *paged) == 0 and plan(4, 1397, 1400, 32, 8, 64, *paged) == 22          # four heads: 352 of 512 places
     at64 = (8, 8, 64)
     assert plan(3, 5775, 1925, *at64, *packed) == 0 and plan(3, 5000, 2600, *at64, *packed) == 42              # equal and uneven
     assert plan(2, 3704, 3703, 16, 16, 64, *paged) == 0 and plan(2, 3704, 18500, 16, 16, 64, *paged) == 0      # 1.97; too many keys
