@@ -972,8 +972,8 @@ __device__ __forceinline__ uint2 load8_stream(const void* p) {
   return make_uint2(x.x, x.y);
 }
 
-// W as in decode_mfma_item: 1 = the wave walks its partition, > 1 = W waves of the workgroup share it.
-template <typename T, int NCH, int W, int D>
+// W as in decode_mfma_item: 1 = the wave walks its partition, > 1 = W waves of the workgroup share it.  kRows: K in whole rows through LDS.
+template <typename T, int NCH, int W, int D, bool kRows>
 __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b, int p, int slice, int w) {
   static_assert(NCH == 1, "one chunk of up to 16 heads");
   static_assert(D == 128 || D == 64, "one or two 64-dim steps");
@@ -1017,10 +1017,9 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
   const int64_t row = (int64_t)a.num_kv_heads * D;          // bytes per token row
   const char* kc = reinterpret_cast<const char*>(a.k_cache) + (int64_t)g * D;
   const char* vc = reinterpret_cast<const char*>(a.v_cache) + (int64_t)g * D;
-  // W == 1, a stream of many tiles: K arrives in whole rows, D / 16 lanes each, and goes through LDS into the first product's operands;
-  // in the operands' own order, token lane%16 and bytes 16*q4 (+64 j), a load's lanes are 16 bytes of 16 rows, and 128 sequences of
-  // 256-16384 tokens took 240 us instead of 230
-  constexpr bool kRows = W == 1;
+  // kRows: K arrives in whole rows, D / 16 lanes each, and goes through LDS into the first product's operands; in the operands' own
+  // order, token lane%16 and bytes 16*q4 (+64 j), a load's lanes are 16 bytes of 16 rows (see int8_rows_pay)
+  static_assert(!kRows || (W == 1 && D == 128), "one wave per kv head, two loads per tile");
   constexpr int kChunks = D / 16, kRowsPer = 64 / kChunks;   // 16-byte chunks of a row, rows of a load
   const int k_lane_off = kRows ? lane / kChunks * (int)row + lane % kChunks * 16 : col * (int)row + q4 * 16;
   const int64_t k_step = kRows ? (int64_t)kRowsPer * row : 64;
@@ -1300,17 +1299,17 @@ __global__ __launch_bounds__(64 * W, D > 128 ? 1 : kDecodeWavesPerEu) void decod
   const int p = (int)((blockIdx.y + (unsigned)b) % (unsigned)a.num_parts);
   decode_mfma_item<T, W, D, SUB>(a, b, p, g, threadIdx.x >> 6);
 }
-template <typename T, int NCH, int D>
+template <typename T, int NCH, int D, bool kRows>
 __global__ __launch_bounds__(kDecodeI8Threads, kDecodeI8WavesPerEu) void decode_mfma_int8_kernel(const DecodeArgs a) {
   int b, p, hg;
   if (!decode_item<true>(a, b, p, hg)) return;
-  decode_mfma_int8_item<T, NCH, 1, D>(a, b, p, hg * (blockDim.x >> 6) + (threadIdx.x >> 6), 0);
+  decode_mfma_int8_item<T, NCH, 1, D, kRows>(a, b, p, hg * (blockDim.x >> 6) + (threadIdx.x >> 6), 0);
 }
 template <typename T, int W, int D>
 __global__ __launch_bounds__(64 * W, kDecodeI8WavesPerEu) void decode_mfma_int8_split_kernel(const DecodeArgs a) {
   const int g = blockIdx.x, b = blockIdx.z;
   const int p = (int)((blockIdx.y + (unsigned)b) % (unsigned)a.num_parts);
-  decode_mfma_int8_item<T, 1, W, D>(a, b, p, g, threadIdx.x >> 6);
+  decode_mfma_int8_item<T, 1, W, D, false>(a, b, p, g, threadIdx.x >> 6);
 }
 
 // ---------------------------------------------------------------------------
@@ -1599,6 +1598,12 @@ static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, i
   return plan;
 }
 
+// INT8 keys of 128 dims in whole rows through LDS, or as operands straight from memory: rows cost the address unit a quarter, and a longer way from a
+// load to its product, which a wave with the SIMD to itself waits for: from more than two waves per SIMD on.  us, rows / operands, 8 kv heads: 5
+// sequences of 30000 tokens (1200 waves) 101 / 94, 8 (1920) 105 / 99, 10 (2400) 118 / 119, 16 222 / 226; 128 of 1000 to 13700 366 / 374, of 4096 209 / 205.
+// (64 dims, one load per tile: 5 of 30000 95.7 / 92.2, 16 181 / 171, 128 of 4096 161 / 155, 24 of 17000 equal: never.)
+static bool int8_rows_pay(int64_t waves) { return waves > 2048; }
+
 template <typename T> struct IsSixteenBit { static constexpr bool value = true; };
 template <> struct IsSixteenBit<float> { static constexpr bool value = false; };
 
@@ -1651,8 +1656,9 @@ static int launch_decode(DecodeArgs a, bool int8, bool fast_ok, int waves, hipSt
       const dim3 grid((unsigned)a.num_parts, groups, (unsigned)a.batch);
       if (split && a.head_dim == 64) decode_mfma_int8_split_kernel<T, kSplitWaves, 64><<<split_grid, split_block, 0, stream>>>(a);
       else if (split) decode_mfma_int8_split_kernel<T, kSplitWaves, 128><<<split_grid, split_block, 0, stream>>>(a);
-      else if (a.head_dim == 64) decode_mfma_int8_kernel<T, 1, 64><<<grid, block, 0, stream>>>(a);
-      else decode_mfma_int8_kernel<T, 1, 128><<<grid, block, 0, stream>>>(a);
+      else if (a.head_dim == 64) decode_mfma_int8_kernel<T, 1, 64, false><<<grid, block, 0, stream>>>(a);
+      else if (int8_rows_pay((int64_t)a.num_parts * a.batch * slices)) decode_mfma_int8_kernel<T, 1, 128, true><<<grid, block, 0, stream>>>(a);
+      else decode_mfma_int8_kernel<T, 1, 128, false><<<grid, block, 0, stream>>>(a);
       launched = true;
     }
   }

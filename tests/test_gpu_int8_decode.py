@@ -176,3 +176,19 @@ def test_config4_full_size_on_its_own_plan():
     sv *= 2
     got2 = paged_attention_decode_int8(q, ck, cv, sk, sv, td, cd, scale, hq, hkv, d, bs).cpu()
     assert (got2.float() - 2 * got.float()).abs().max() <= 2e-2 + 2.0 ** -7 * got.float().abs().max()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq", [32, 8])
+def test_int8_keys_as_operands_or_in_rows(dtype, hq):
+    """Long tables: a batch of up to 2048 waves takes its keys as operands, a larger one in rows through LDS; same products in the same
+    order, so the sequences of the smaller batch come out the same to the bit.  Contexts end at and beside tile and partition edges."""
+    hkv, d, bs, scale = 8, 128, 16, 128 ** -0.5
+    lens = [32768, 30001, 1, 17, 1024, 1025, 5007, 2048, 16]
+    case = _quantised_case(67, 0, 0, 0, hq, hkv, d, bs, dtype, ctx_list=lens)
+    few, many = (paged_decode_plan(n, hq, hkv, d, 2048, bs, int8_cache=True) for n in (8, 9))
+    assert few == many and few[1] * 8 * hkv == 2048 and few[2] == 1            # one wave per kv head and partition
+    whole = _check(case, hq, hkv, d, bs, scale)
+    q, ck, cv, sk, sv, tables, ctx = case
+    got = paged_attention_decode_int8(q[:8].to(DEV), ck, cv, sk, sv, tables[:8].to(DEV), ctx[:8].to(DEV), scale, hq, hkv, d, bs).cpu()
+    assert torch.equal(got, whole[:8])
