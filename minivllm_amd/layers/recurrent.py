@@ -12,6 +12,7 @@ from dataclasses import dataclass
 import torch
 
 from minivllm_amd import _C
+from minivllm_amd.engine.ragged import BLOCK_ROWS
 
 __all__ = ["DecayMemoryState", "MlstmState", "decay_memory", "gate_linear", "gated_row_norm", "mlstm"]
 
@@ -62,10 +63,12 @@ def chunked_output_takes(segments: int, rows: int, heads: int, dim: int, vdim: i
 
     A workgroup holds all columns of a head, so heads up to 128 x 256, but not those up to 128 columns, of which half its waves
     would have none.  It takes longer per block of rows than two workgroups of the other form (9.5 us against 8), which have twice as
-    many CUs while there are few of them, and saves a launch and the sums' way through memory.  Heads of 128 x 256: 64 segments of
-    200 rows and heads 40 us against 36, 128 of them 44 against 48, 8 x 16 of 1024 rows 145 against 159, 32 of 100 rows 21 against 25."""
+    many CUs while there are few of them, and saves a launch and the sums' way through memory.  us this form / the other, captured, heads of
+    128 x 256: 64 segments of 200 rows and heads 40 / 36, 128 of them 44 / 48, 8 x 16 of 1024 rows 145 / 159; 96 of 100 rows 23.7 / 25.0, 80 of
+    100 and of 190 23.2 / 22.9 and 32.6 / 33.7; 8 of 64, one block, 13.1 / 13.2 (and 12.4 / 20.2 where the launches are not captured and the host
+    is the bound), 8 of 72 21.7 / 19.1 (20.7 / 20.2), 8 of 150 29.9 / 25.0.  Of 64 x 256: 8 of 100 rows 17.6 / 15.5 but 16.8 / 20.4 not captured."""
     fits = dim <= 128 and 128 < vdim <= 256 and gate % 8 == 0 and weight.data_ptr() % 16 == 0
-    return fits and (segments * heads >= 96 or rows <= 128 * segments)
+    return fits and (segments * heads >= 96 or rows <= (100 if dim <= 64 else BLOCK_ROWS) * segments)
 
 
 def mlstm(step, proj: torch.Tensor, gates: torch.Tensor, gate_col: int, weight: torch.Tensor, state: MlstmState,

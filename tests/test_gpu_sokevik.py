@@ -478,6 +478,18 @@ def test_mlstm_whole_heads(monkeypatch, heads, dim, vdim):
     test_mlstm_segments_side_by_side(monkeypatch, heads, dim, vdim)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 256), (3, 24, 136), (2, 72, 144)])
+def test_mlstm_whole_heads_whatever_runs_beside(monkeypatch, heads, dim, vdim):
+    """The same with every portion of long entries in that form: a few workgroups would take it only for portions of one block."""
+    from minivllm_amd.layers import recurrent
+    takes = recurrent.chunked_output_takes
+    assert takes(1, 64, 1, 128, 256, 0, torch.ones(4)) and not takes(1, 65, 1, 128, 256, 0, torch.ones(4))
+    assert takes(2, 200, 1, 64, 256, 0, torch.ones(4)) and not takes(2, 201, 1, 64, 256, 0, torch.ones(4))
+    assert takes(6, 9999, 16, 128, 256, 0, torch.ones(4)) and not takes(5, 9999, 16, 128, 256, 0, torch.ones(4))
+    monkeypatch.setattr(recurrent, "chunked_output_takes", lambda segments, *rest: takes(10 ** 6, *rest))
+    test_mlstm_whole_heads(monkeypatch, heads, dim, vdim)
+
+
 # ---- the model ----
 _runners: dict = {}
 
