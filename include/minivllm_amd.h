@@ -594,6 +594,9 @@ int mvllm_gate_linear(float* out, const void* x, int64_t x_row_stride, const voi
  *   mvllm_mlstm_chunked_workspace_bytes.
  * mvllm_mlstm_chunked_output: the same for dim <= 128 and vdim <= 256 with mvllm_mlstm_output behind it, in one pass: out's rows
  *   of these entries (16-byte aligned, like weight), m_state[slot].  gate: rows proj_row_stride apart, 8-byte aligned.
+ * mvllm_mlstm_chunked_output_parts: the same without a workspace for portions (segments that are the only one of their entry, flags 7):
+ *   the rows of those that start at position 0 are shared by up to `parts` workgroups per head (1 to 16), each of which
+ *   works out the state in front of its own rows by itself.  The results are those of one part but for roundings of fp32.
  */
 int mvllm_mlstm_recurrent(float* num, float* den, float* m_next, const void* proj, int64_t proj_row_stride,
                           const float* gates, float* s_state, float* n_state, const float* m_state,
@@ -610,6 +613,11 @@ int mvllm_mlstm_chunked_output(void* out, const float* weight, const void* gate,
                                const int32_t* cu_seqlens, const int32_t* slots, const int64_t* positions,
                                const int32_t* segments, int num_segments, int split, int num_heads, int dim, int vdim,
                                float q_scale, float floor, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+int mvllm_mlstm_chunked_output_parts(void* out, const float* weight, const void* gate, float eps, const void* proj,
+                                     int64_t proj_row_stride, const float* gates, float* s_state, float* n_state,
+                                     float* m_state, const int32_t* cu_seqlens, const int32_t* slots,
+                                     const int64_t* positions, const int32_t* portions, int num_portions, int parts,
+                                     int num_heads, int dim, int vdim, float q_scale, float floor, int dtype, void* stream);
 int mvllm_mlstm_output(void* out, const float* num, const float* den, const float* weight, const void* gate,
                        int64_t gate_row_stride, float eps, const float* m_next, float* m_state,
                        const int32_t* cu_seqlens, const int32_t* row_entry, const int32_t* slots, int64_t rows,

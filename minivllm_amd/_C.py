@@ -104,6 +104,8 @@ SIGNATURES = {
                                                                                             c_void_p, c_size_t, c_void_p]),
     "mvllm_mlstm_chunked_output": (c_int, [c_void_p] * 3 + [c_float, c_void_p, c_int64] + [c_void_p] * 8 + [c_int] * 5 +
                                    [c_float, c_float, c_int, c_void_p, c_size_t, c_void_p]),
+    "mvllm_mlstm_chunked_output_parts": (c_int, [c_void_p] * 3 + [c_float, c_void_p, c_int64] + [c_void_p] * 8 + [c_int] * 5 +
+                                         [c_float, c_float, c_int, c_void_p]),
     "mvllm_stream_embed_norm": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_float, c_void_p] + [c_int64] * 3 +
                                 [c_void_p] * 9 + [c_float, c_int64, c_int, c_int, c_int, c_void_p]),
     "mvllm_stream_norm": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,

@@ -25,6 +25,9 @@
 namespace mvllm {
 
 constexpr int kBlock = 64;           // rows per block
+constexpr int kMaxParts = 16;        // workgroups that share a head's rows, at most: more bring less than 1 %
+// What passing over a block takes of a block's time: 2.5 of 6.1 us where few workgroups run, of 8.3 where they fill the chip (whose clock falls).
+constexpr float kPassOver = 0.3f;
 
 struct MemoryChunkArgs {
   float* num;                // [T, H, vdim]
@@ -54,6 +57,8 @@ struct MemoryChunkArgs {
   const bf16_t* gate;        // [T, proj_stride]: H * vdim pre-activations per row
   float* m_out;              // [slots, H]: m_state
   float eps;
+  int parts;                 // workgroups that share the rows of a head ...
+  float least;               // ... and what each of them takes at least, as a share of the rows
 };
 
 // eight packed values through z * sigmoid(z), rounded again
@@ -98,11 +103,15 @@ template <typename F> __device__ __forceinline__ float wave_scan(float x, float 
 }
 
 // kOut (with gates, vdim <= 256, eight waves: whole heads): the results go through the norm and the output gate here, out = rms(num / den)
-// weight sigmoid(gate), and the sums never leave the chip.  8 x 1024 rows, 16 heads of 128 x 256: 155 us where the sums' pass took 119
-// and their norm 56 (two times 134 MB).  The vector unit bounds it: two waves per SIMD issue 16 of a block's 20 thousand cycles, a
-// quarter of them for norm and gate (116 us without), and 128 workgroups leave half the CUs idle; segments to fill them cost as much as
-// they bring (158 us), since their states are a pass of their own.  Scores are 16 x 16 tiles so that all waves have some (143 without
-// them), the normaliser and n are spread over all threads.
+// weight sigmoid(gate), and the sums never leave the chip.  8 x 1024 rows, 16 heads of 128 x 256: 139 us in one part where the sums' pass
+// took 119 and their norm 56 (two times 134 MB).  The vector unit bounds it: two waves per SIMD issue 11 of a block's 15 thousand
+// cycles, a quarter of them for norm and gate.  Scores are 16 x 16 tiles so that all waves have some, the normaliser and n are spread
+// over all threads; norm and gate take sixteen lanes per row, so that the scalars and sums of four rows are worked out at once
+// (143 with a row per wave).
+// parts > 1: several workgroups share the rows of a head, each of which works out the state in front of its part by itself: passing over
+// a block takes 0.3 of its time (2.5 us; bound by the chain write, barrier, weights, products), no state goes through memory, and
+// it is one launch.  The same 8 x 1024 rows, 128 workgroups on 256 CUs as they are, 105 us in two parts; segments, whose states are
+// a pass of their own, 158.  8 heads, one portion of 305 rows: 32.3 whole, 23.8 in four parts.
 template <int DIMP, int kWaves, bool kStateOnly, bool kGates, bool kOut>
 __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk_kernel(const MemoryChunkArgs a) {
   constexpr int kThreads = 64 * kWaves;
@@ -120,13 +129,43 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
   constexpr int kORow = VT + 8;
   __shared__ __attribute__((aligned(16))) float os[kOut ? kBlock * kORow : 4];
   __shared__ float sc_den[kOut ? kBlock : 1];
+  __shared__ __attribute__((aligned(16))) float out_w[kOut ? VT : 4];
   static_assert(!kOut || (kGates && !kStateOnly && kWaves == 8), "whole heads, with gates");
 
-  const int seg = blockIdx.x, h = blockIdx.y, tile = blockIdx.z;
-  const int entry = a.segments[4 * seg], row0 = a.segments[4 * seg + 1], rows = a.segments[4 * seg + 2];
+  const int seg = blockIdx.x, h = blockIdx.y, tile = kOut ? 0 : blockIdx.z;
+  const int entry = a.segments[4 * seg], row0 = a.segments[4 * seg + 1];
+  int rows = a.segments[4 * seg + 2];
   const int flags = a.segments[4 * seg + 3];
   const int slot = a.slot[entry];
   if (rows <= 0 || slot < 0 || (kStateOnly && (flags & 2))) return;     // the last segment's contribution is not needed
+  int begin = 0;                                    // rows in front of the workgroup's own
+  bool last = (flags & 2) != 0;
+  if constexpr (kOut) if (a.parts > 1) {
+    // Only entries that start from nothing are shared: a slot's state would be read by all parts and replaced by the last one.
+    const int z = blockIdx.z;
+    if (!(flags & 4) || a.positions[row0] != 0) {
+      if (z > 0) return;
+    } else {
+      // Every part takes as many blocks as it has time for behind the ones it passes over; lane l tries l / 32 of a block's time more
+      // than the least, the first that comes to the last block decides.
+      const int blocks = (rows + kBlock - 1) / kBlock;
+      const float time = a.least * (float)blocks + (float)(threadIdx.x & 63) * (1.f / 32.f);
+      int at = 0, from = 0, to = 0;
+      for (int i = 0; i < a.parts; ++i) {
+        from = i == z ? at : from;
+        at = min(at + max((int)(time - kPassOver * (float)at), 0), blocks);
+        to = i == z ? at : to;
+      }
+      const unsigned long long there = __ballot(at == blocks);
+      const int decides = __builtin_amdgcn_readfirstlane(there != 0ull ? __ffsll(there) - 1 : 0);
+      const int b0 = there != 0ull ? __builtin_amdgcn_readlane(from, decides) : z == 0 ? 0 : blocks;       // (none: the first part takes all)
+      const int b1 = there != 0ull ? __builtin_amdgcn_readlane(to, decides) : blocks;
+      if (b0 >= b1) return;
+      last = b1 == blocks;
+      begin = b0 * kBlock;
+      rows = min(b1 * kBlock, rows);
+    }
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5, i16 = lane & 15, half = (lane >> 4) & 1;
   const int dim = a.dim, vdim = a.vdim, H = a.heads;
@@ -167,11 +206,11 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
       __builtin_amdgcn_sched_barrier(0);
     });
   }
-  const int out_c = 4 * lane;                       // kOut: this lane's columns of a row
-  float4 out_w = make_float4(0.f, 0.f, 0.f, 0.f);
-  uint2 gr[kOut ? kBlock / kWaves : 1];             // ... its part of the output gate, of rows kBlock / kWaves * wave + i
+  // kOut, norm and gate: sixteen lanes per row, so that four rows' sums and scalars are worked out at once
+  constexpr int kTurns = kBlock / (4 * kWaves);     // rows of a lane: kBlock / kWaves * wave + 4 turn + lane / 16 ...
+  const int out_c = 4 * i16;                        // ... its columns: out_c + 64 j + 0 .. 3
+  uint2 gr[kOut ? kTurns * 4 : 1];                  // ... their part of the output gate
   if constexpr (kOut) {
-    if (out_c < vdim) out_w = *reinterpret_cast<const float4*>(a.weight + (int64_t)h * vdim + out_c);
     // of the scores' 16 x 16 tiles past the diagonal the products read two
     for (int i = tid; i < 2 * 16 * 16; i += kThreads) {
       const int t = 32 * (i >> 8) + ((i >> 4) & 15), x = 32 * (i >> 8) + 16 + (i & 15);
@@ -193,7 +232,7 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
   const uint32_t pitch_in = (uint32_t)a.proj_stride * 2u;
   const uint32_t q_first = q_d < dim ? (uint32_t)q_r * pitch_in + (uint32_t)q_d * 2u : 0x80000000u;
   const uint32_t v_first = tile * VT + v_d < vdim ? (uint32_t)v_r * pitch_in + (uint32_t)v_d * 2u : 0x80000000u;
-  auto fetch = [&](int at) __attribute__((always_inline)) {
+  auto fetch = [&](int at, auto WITH_Q) __attribute__((always_inline)) {
     const int64_t base = (int64_t)(row0 + at) * a.proj_stride;
     const uint32_t reach = (uint32_t)(min(kBlock, rows - at) - 1) * pitch_in;
     auto rows_of = [&](const bf16_t* p, int cols) {
@@ -202,7 +241,7 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
     uint32_t q_off = q_first, v_off = v_first;
     asm volatile("" : "+v"(q_off), "+v"(v_off));    // (offsets of all loads kept across the loop would not fit the registers)
     const auto k_rows = rows_of(kg, dim), v_rows = rows_of(vg, vdim - tile * VT);
-    if constexpr (!kStateOnly) {
+    if constexpr (!kStateOnly && decltype(WITH_Q)::value) {
       const auto q_rows = rows_of(qg, dim);
 #pragma unroll
       for (int i = 0; i < kQLoads; ++i) qr[i] = load16(q_rows, q_off + (uint32_t)(i * kQStep) * pitch_in);
@@ -218,10 +257,158 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
       gate_f = live ? g[H + h] : 0.f;
     }
   };
-  fetch(0);
+  constexpr std::true_type with_q{};
+
+  if constexpr (kOut) {
+    if (begin > 0) {
+      // The state behind the rows in front of the part, without their outputs: two buffers (the other one where the outputs are
+      // later), one barrier per block.
+      static_assert(sizeof(os) >= kBlock * (kQRow + kVRow) * 2 + kBlock * 4 + sizeof(n_part), "the second buffer lies in os");
+      uint16_t* const k_other = reinterpret_cast<uint16_t*>(os);
+      uint16_t* const v_other = k_other + kBlock * kQRow;
+      float* const w_other = reinterpret_cast<float*>(v_other + kBlock * kVRow);
+      float* const part_other = w_other + kBlock;
+      constexpr int kPairs = DIMP / 2, kShares = kThreads / kPairs;
+      // S and n are kept as exp(-behind) times themselves, so that a block's decay joins its rows' weights and they are scaled only when
+      // it has come to 2^-20
+      float behind = 0.f;
+      auto advance_n = [&](const float* part, float scale) __attribute__((always_inline)) {
+        if (tid >= DIMP) return;
+        float x = 0.f;
+#pragma unroll
+        for (int i = 0; i < kShares; ++i) x += part[2 * (i * kPairs) + tid];
+        n_lds[tid] = fmaf(scale, n_lds[tid], x);
+      };
+      auto scale_s = [&](float scale) __attribute__((always_inline)) {
+#pragma unroll
+        for (int td = 0; td < kTD; ++td)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[td][r] *= scale;
+      };
+      // two blocks on their way
+      uint4 k_in[2][kQLoads], v_in[2][kVLoads];
+      float i_in[2], f_in[2];
+      auto send = [&](int at, auto SET) __attribute__((always_inline)) {
+        constexpr int set = decltype(SET)::value;
+        const int64_t base = (int64_t)(row0 + at) * a.proj_stride;
+        const bool some = at < begin;               // (whole blocks all of them)
+        uint32_t q_off = q_first, v_off = v_first;
+        asm volatile("" : "+v"(q_off), "+v"(v_off));
+        const auto k_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(kg + base), 0, some ? (kBlock - 1) * pitch_in + (uint32_t)dim * 2u : 0u, 0x00020000);
+        const auto v_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(vg + base), 0, some ? (kBlock - 1) * pitch_in + (uint32_t)vdim * 2u : 0u, 0x00020000);
+        const float* g = a.gates + (int64_t)(row0 + (some ? at : 0) + lane) * 2 * H;
+        i_in[set] = g[h];
+        f_in[set] = g[H + h];
+#pragma unroll
+        for (int i = 0; i < kQLoads; ++i) k_in[set][i] = load16(k_rows, q_off + (uint32_t)(i * kQStep) * pitch_in);
+#pragma unroll
+        for (int i = 0; i < kVLoads; ++i) v_in[set][i] = load16(v_rows, v_off + (uint32_t)(i * kVStep) * pitch_in);
+      };
+      constexpr std::integral_constant<int, 0> c0{};
+      constexpr std::integral_constant<int, 1> c1{};
+      float scale_before = 1.f;
+      auto advance = [&](int at, auto OTHER) __attribute__((always_inline)) {          // one block, in the other buffer
+        constexpr int other = decltype(OTHER)::value;
+        uint16_t* const k = other ? k_other : ks;
+        uint16_t* const v = other ? v_other : vs;
+        float* const w = other ? w_other : sc_w;
+        float* const part = other ? part_other : n_part;
+        const float F = wave_scan(f_in[other], 0.f, [](float x, float y) { return x + y; });
+        const float av = i_in[other] - F;
+        const float M_last = fmaxf(m, wave_max_in_registers(av));
+        const float F_last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(F), 63));
+        behind += m - M_last;
+        float scale = 1.f;
+        if (behind < -13.8f) {                      // (the same for all)
+          scale = __expf(behind);
+          behind = 0.f;
+        }
+        if (wave == 0) w[lane] = __expf(av - M_last - behind);
+        m = F_last + M_last;
+#pragma unroll
+        for (int i = 0; i < kQLoads; ++i) *reinterpret_cast<uint4*>(&k[(q_r + i * kQStep) * kQRow + q_d]) = k_in[other][i];
+#pragma unroll
+        for (int i = 0; i < kVLoads; ++i) *reinterpret_cast<uint4*>(&v[(v_r + i * kVStep) * kVRow + v_d]) = v_in[other][i];
+        __syncthreads();
+        if (at > 0) advance_n(other ? n_part : part_other, scale_before);
+        send(at + 2 * kBlock, OTHER);
+        __builtin_amdgcn_sched_barrier(0);
+        Split8 wv[4];
+        const uint16_t* vp = &v[(4 * hi + (i16 >> 2)) * kVRow + 32 * wave + 16 * half + 4 * (i16 & 3)];
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+          const v4s x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(vp + 16 * st * kVRow));
+          const v4s x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(vp + (16 * st + 8) * kVRow));
+          const uint2 y0 = __builtin_bit_cast(uint2, x0), y1 = __builtin_bit_cast(uint2, x1);
+          const uint32_t two[4] = {y0.x, y0.y, y1.x, y1.y};
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float g = w[16 * st + 8 * (e >> 2) + 4 * hi + (e & 3)];
+            x[e] = g * (e & 1 ? hi_to_float<bf16_t>(two[e >> 1]) : lo_to_float<bf16_t>(two[e >> 1]));
+          }
+          wv[st] = split8(x);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (scale != 1.f) scale_s(scale);
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<kTD>([&](auto TD) {
+          constexpr int td = decltype(TD)::value;
+          const uint16_t* p = &k[(4 * hi + (i16 >> 2)) * kQRow + 32 * td + 16 * half + 4 * (i16 & 3)];
+#pragma unroll
+          for (int st = 0; st < 4; ++st) {
+            const v4s x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p + 16 * st * kQRow));
+            const v4s x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p + (16 * st + 8) * kQRow));
+            const uint2 y0 = __builtin_bit_cast(uint2, x0), y1 = __builtin_bit_cast(uint2, x1);
+            const uint4 kf = make_uint4(y0.x, y0.y, y1.x, y1.y);
+            s[td] = mfma32x32x16<bf16_t>(kf, wv[st].hi, s[td]);
+            s[td] = mfma32x32x16<bf16_t>(kf, wv[st].lo, s[td]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        {
+          const int pair = tid % kPairs, share = tid / kPairs;
+          float x0 = 0.f, x1 = 0.f;
+#pragma unroll
+          for (int i = 0; i < kBlock / kShares; ++i) {
+            const int t = share + i * kShares;
+            const uint32_t two = *reinterpret_cast<const uint32_t*>(&k[t * kQRow + 2 * pair]);
+            x0 = fmaf(w[t], lo_to_float<bf16_t>(two), x0);
+            x1 = fmaf(w[t], hi_to_float<bf16_t>(two), x1);
+          }
+          part[2 * (share * kPairs + pair)] = x0;
+          part[2 * (share * kPairs + pair) + 1] = x1;
+        }
+        scale_before = scale;
+      };
+      // (an odd block first: a loop that could end between its two would hold S in two places)
+      int at = 0;
+      if (begin / kBlock % 2 != 0) {
+        send(0, c1);
+        send(kBlock, c0);
+        advance(0, c1);
+        at = kBlock;
+      } else {
+        send(0, c0);
+        send(kBlock, c1);
+      }
+      for (; at < begin; at += 2 * kBlock) {
+        advance(at, c0);
+        advance(at + kBlock, c1);
+      }
+      __syncthreads();
+      advance_n(part_other, scale_before);
+      const float rest = __expf(behind);
+      scale_s(rest);
+      if (tid < DIMP) n_lds[tid] *= rest;
+    }
+  }
+  if constexpr (kOut)
+    if (tid < VT) out_w[tid] = tid < vdim ? a.weight[(int64_t)h * vdim + tid] : 0.f;
+  fetch(begin, with_q);
 
   float f_total = 0.f;                              // kStateOnly: sum of the log forget gates so far
-  for (int at = 0; at < rows; at += kBlock) {
+  for (int at = begin; at < rows; at += kBlock) {
     // ---- registers -> LDS; the block's scalars ----
     if constexpr (!kGates) {
       if (a.silu) {
@@ -275,12 +462,15 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
       asm volatile("" : "+s"(pitch));
       const auto g_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(a.gate + (int64_t)(row0 + at) * a.proj_stride + (int64_t)h * vdim), 0,
                                                             (uint32_t)(min(kBlock, rows - at) - 1) * pitch + (uint32_t)vdim * 2u, 0x00020000);
-      const uint32_t g_first = out_c < vdim ? (uint32_t)(kBlock / kWaves * wave) * pitch + (uint32_t)out_c * 2u : 0x80000000u;
+      uint32_t g_first = (uint32_t)(kBlock / kWaves * wave + (lane >> 4)) * pitch + (uint32_t)out_c * 2u;
+      asm volatile("" : "+v"(g_first));
 #pragma unroll
-      for (int i = 0; i < kBlock / kWaves; ++i)
-        gr[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(g_rows, g_first + (uint32_t)i * pitch, 0, 0));
+      for (int i = 0; i < 4 * kTurns; ++i) {        // (columns past vdim: whatever lies there, not used)
+        const uint32_t at_g = g_first + (uint32_t)(4 * (i >> 2)) * pitch + 128u * (i & 3);
+        gr[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(g_rows, at_g, 0, 0));
+      }
     }
-    if (at + kBlock < rows) fetch(at + kBlock);     // the next block's rows, on their way during this one
+    if (at + kBlock < rows) fetch(at + kBlock, with_q);     // the next block's rows, on their way during this one
 
     // kOut: what the normaliser and n take of this block before the scores are there
     constexpr int kPer = kThreads / kBlock;         // threads per row
@@ -452,17 +642,24 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
     }
     if constexpr (!kStateOnly) {
       __syncthreads();                              // the weighted scores are complete
-#pragma unroll
-      for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-        for (int st = 0; st < 2 * (rt + 1); ++st) {
-          const int at_p = (32 * rt + l32) * kPRow + 16 * st + 4 * hi;
-          const uint2 h0 = *reinterpret_cast<const uint2*>(&ph[at_p]), h1 = *reinterpret_cast<const uint2*>(&ph[at_p + 8]);
-          const uint2 l0 = *reinterpret_cast<const uint2*>(&pl[at_p]), l1 = *reinterpret_cast<const uint2*>(&pl[at_p + 8]);
-          o[rt] = mfma32x32x16<bf16_t>(make_uint4(h0.x, h0.y, h1.x, h1.y), vf[st], o[rt]);
-          o[rt] = mfma32x32x16<bf16_t>(make_uint4(l0.x, l0.y, l1.x, l1.y), vf[st], o[rt]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+      // the weighted scores' operands one step ahead of the products
+      uint4 p_hi[2], p_lo[2];
+      auto p_frag = [&](auto STEP) __attribute__((always_inline)) {
+        constexpr int step = decltype(STEP)::value, rt = step < 2 ? 0 : 1, st = step < 2 ? step : step - 2;
+        const int at_p = (32 * rt + l32) * kPRow + 16 * st + 4 * hi;
+        const uint2 h0 = *reinterpret_cast<const uint2*>(&ph[at_p]), h1 = *reinterpret_cast<const uint2*>(&ph[at_p + 8]);
+        const uint2 l0 = *reinterpret_cast<const uint2*>(&pl[at_p]), l1 = *reinterpret_cast<const uint2*>(&pl[at_p + 8]);
+        p_hi[step & 1] = make_uint4(h0.x, h0.y, h1.x, h1.y);
+        p_lo[step & 1] = make_uint4(l0.x, l0.y, l1.x, l1.y);
+      };
+      p_frag(std::integral_constant<int, 0>{});
+      static_for<6>([&](auto STEP) {
+        constexpr int step = decltype(STEP)::value, rt = step < 2 ? 0 : 1, st = step < 2 ? step : step - 2;
+        if constexpr (step < 5) p_frag(std::integral_constant<int, step + 1>{});
+        o[rt] = mfma32x32x16<bf16_t>(p_hi[step & 1], vf[st], o[rt]);
+        o[rt] = mfma32x32x16<bf16_t>(p_lo[step & 1], vf[st], o[rt]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
       if constexpr (kOut) {
         float* p = &os[4 * hi * kORow + 32 * wave + l32];
 #pragma unroll
@@ -538,27 +735,39 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
       asm volatile("" : "+s"(pitch));
       const auto out = __builtin_amdgcn_make_buffer_rsrc(a.out + ((int64_t)(row0 + at) * H + h) * vdim, 0,
                                                          (uint32_t)(min(kBlock, rows - at) - 1) * pitch + (uint32_t)vdim * 2u, 0x00020000);
-      const uint32_t out_first = out_c < vdim ? (uint32_t)first * pitch + (uint32_t)out_c * 2u : 0x80000000u;
+      uint32_t out_first = (uint32_t)(first + (lane >> 4)) * pitch + (uint32_t)out_c * 2u;
+      asm volatile("" : "+v"(out_first));
 #pragma unroll
-      for (int i = 0; i < kBlock / kWaves; ++i) {
-        const float inv_den = __builtin_amdgcn_rcpf(sc_den[first + i]);
-        const float4 num = *reinterpret_cast<const float4*>(&os[(first + i) * kORow + out_c]);
-        const float x[4] = {num.x * inv_den, num.y * inv_den, num.z * inv_den, num.w * inv_den};
-        const float ss = four_rows_sum(row16_sum(x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3]));
-        const float sc = __builtin_amdgcn_rsqf(ss * inv_vdim + a.eps);
-        const float y[4] = {x[0] * sc * out_w.x, x[1] * sc * out_w.y, x[2] * sc * out_w.z, x[3] * sc * out_w.w};
-        const float z[4] = {lo_to_float<bf16_t>(gr[i].x), hi_to_float<bf16_t>(gr[i].x), lo_to_float<bf16_t>(gr[i].y), hi_to_float<bf16_t>(gr[i].y)};
-        float o4[4];
+      for (int turn = 0; turn < kTurns; ++turn) {
+        const int row = first + 4 * turn + (lane >> 4);
+        const float inv_den = __builtin_amdgcn_rcpf(sc_den[row]);
+        float x[4][4], ss = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o4[e] = y[e] * __builtin_amdgcn_rcpf(1.0f + __expf(-z[e]));
-        const uint2 packed = make_uint2(pack2<bf16_t>(o4[0], o4[1]), pack2<bf16_t>(o4[2], o4[3]));
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, packed), out, out_first + (uint32_t)i * pitch, 0, 2 /* nt */);
+        for (int j = 0; j < 4; ++j) {
+          const float4 num = *reinterpret_cast<const float4*>(&os[row * kORow + out_c + 64 * j]);
+          x[j][0] = num.x * inv_den; x[j][1] = num.y * inv_den; x[j][2] = num.z * inv_den; x[j][3] = num.w * inv_den;
+          ss += (x[j][0] * x[j][0] + x[j][1] * x[j][1]) + (x[j][2] * x[j][2] + x[j][3] * x[j][3]);
+        }
+        const float sc = __builtin_amdgcn_rsqf(row16_sum(ss) * inv_vdim + a.eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float4 w4 = *reinterpret_cast<const float4*>(&out_w[out_c + 64 * j]);
+          const uint2 g2 = gr[4 * turn + j];
+          const float wt[4] = {w4.x, w4.y, w4.z, w4.w};
+          const float z[4] = {lo_to_float<bf16_t>(g2.x), hi_to_float<bf16_t>(g2.x), lo_to_float<bf16_t>(g2.y), hi_to_float<bf16_t>(g2.y)};
+          float o4[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o4[e] = x[j][e] * sc * wt[e] * __builtin_amdgcn_rcpf(1.0f + __expf(-z[e]));
+          const uint2 packed = make_uint2(pack2<bf16_t>(o4[0], o4[1]), pack2<bf16_t>(o4[2], o4[3]));
+          const uint32_t at_out = out_c + 64 * j < vdim ? out_first + (uint32_t)(4 * turn) * pitch + 128u * j : 0x80000000u;
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, packed), out, at_out, 0, 2 /* nt */);
+        }
       }
     }
   }
 
   // ---- the state behind the segment: contribution -> workspace (kStateOnly), the last one -> the slot ----
-  if (!kStateOnly && !(flags & 2)) return;
+  if (!kStateOnly && !last) return;
   float* s_out = kStateOnly ? a.ws_s + ((int64_t)seg * H + h) * dim * vdim : a.s_state + ((int64_t)slot * H + h) * dim * vdim;
   const auto state = __builtin_amdgcn_make_buffer_rsrc(s_out, 0, s_bytes, 0x00020000);
   uint32_t s_pitch = (uint32_t)vdim * 4u;
@@ -678,7 +887,7 @@ static int launch_chunked(const MemoryChunkArgs& a, bool split, hipStream_t s) {
     status = launch_status();
     if (status != 0) return status;
   }
-  if constexpr (kOut) memory_chunk_kernel<DIMP, 8, false, true, true><<<dim3(grid.x, grid.y), dim3(512), 0, s>>>(a);
+  if constexpr (kOut) memory_chunk_kernel<DIMP, 8, false, true, true><<<dim3(grid.x, grid.y, (unsigned)(a.parts > 1 ? a.parts : 1)), dim3(512), 0, s>>>(a);
   else memory_chunk_kernel<DIMP, kWaves, false, kGates, false><<<grid, block, 0, s>>>(a);
   return launch_status();
 }

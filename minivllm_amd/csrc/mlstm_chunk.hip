@@ -1,6 +1,8 @@
 // The mLSTM recurrence of mlstm.hip in blocks of 64 rows on the matrix unit (memory_chunk.h).
 #include "memory_chunk.h"
 
+#include <cmath>
+
 using namespace mvllm;
 
 static int64_t chunk_ws_floats(int num_segments, int num_heads, int dim, int vdim) {
@@ -57,12 +59,11 @@ extern "C" int mvllm_mlstm_chunked(float* num, float* den, float* m_next, const 
   return launch_chunked_sizes<true>(a, split != 0, (hipStream_t)stream);
 }
 
-extern "C" int mvllm_mlstm_chunked_output(void* out, const float* weight, const void* gate, float eps, const void* proj,
-                                          int64_t proj_row_stride, const float* gates, float* s_state, float* n_state,
-                                          float* m_state, const int32_t* cu_seqlens, const int32_t* slots,
-                                          const int64_t* positions, const int32_t* segments, int num_segments, int split,
-                                          int num_heads, int dim, int vdim, float q_scale, float floor, int dtype,
-                                          void* workspace, size_t workspace_bytes, void* stream) {
+static int chunked_output(void* out, const float* weight, const void* gate, float eps, const void* proj, int64_t proj_row_stride,
+                          const float* gates, float* s_state, float* n_state, float* m_state, const int32_t* cu_seqlens,
+                          const int32_t* slots, const int64_t* positions, const int32_t* segments, int num_segments, int split, int parts,
+                          int num_heads, int dim, int vdim, float q_scale, float floor, int dtype, void* workspace, size_t workspace_bytes,
+                          void* stream) {
   MemoryChunkArgs a;
   const int status = chunk_args(a, proj, proj_row_stride, gates, s_state, n_state, m_state, cu_seqlens, slots, positions, segments,
                                 num_segments, split, num_heads, dim, vdim, q_scale, floor, dtype, workspace, workspace_bytes);
@@ -72,6 +73,28 @@ extern "C" int mvllm_mlstm_chunked_output(void* out, const float* weight, const 
   if (!out || !weight || !gate) return MVLLM_ERR_NULL_POINTER;
   if (!aligned16(out) || !aligned16(weight) || (reinterpret_cast<uintptr_t>(gate) & 7u) != 0) return MVLLM_ERR_MISALIGNED;
   a.out = reinterpret_cast<bf16_t*>(out); a.weight = weight; a.gate = reinterpret_cast<const bf16_t*>(gate); a.m_out = m_state; a.eps = eps;
+  a.parts = parts;
+  a.least = (float)(kPassOver / (1.0 - pow(1.0 - kPassOver, parts)));
   hipStream_t s = (hipStream_t)stream;
   return dim <= 64 ? launch_chunked<64, 4, true, true>(a, split != 0, s) : launch_chunked<128, 4, true, true>(a, split != 0, s);
+}
+
+extern "C" int mvllm_mlstm_chunked_output(void* out, const float* weight, const void* gate, float eps, const void* proj,
+                                          int64_t proj_row_stride, const float* gates, float* s_state, float* n_state,
+                                          float* m_state, const int32_t* cu_seqlens, const int32_t* slots,
+                                          const int64_t* positions, const int32_t* segments, int num_segments, int split,
+                                          int num_heads, int dim, int vdim, float q_scale, float floor, int dtype,
+                                          void* workspace, size_t workspace_bytes, void* stream) {
+  return chunked_output(out, weight, gate, eps, proj, proj_row_stride, gates, s_state, n_state, m_state, cu_seqlens, slots, positions,
+                        segments, num_segments, split, 1, num_heads, dim, vdim, q_scale, floor, dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mvllm_mlstm_chunked_output_parts(void* out, const float* weight, const void* gate, float eps, const void* proj,
+                                                int64_t proj_row_stride, const float* gates, float* s_state, float* n_state,
+                                                float* m_state, const int32_t* cu_seqlens, const int32_t* slots,
+                                                const int64_t* positions, const int32_t* portions, int num_portions, int parts,
+                                                int num_heads, int dim, int vdim, float q_scale, float floor, int dtype, void* stream) {
+  if (parts < 1 || parts > kMaxParts) return MVLLM_ERR_BAD_SHAPE;
+  return chunked_output(out, weight, gate, eps, proj, proj_row_stride, gates, s_state, n_state, m_state, cu_seqlens, slots, positions,
+                        portions, num_portions, 0, parts, num_heads, dim, vdim, q_scale, floor, dtype, nullptr, 0, stream);
 }

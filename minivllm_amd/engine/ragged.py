@@ -94,6 +94,8 @@ class RaggedStep:
     short_rows: Optional[int] = None                  # ... and their rows
     segments: Optional[torch.Tensor] = None           # int32 [n, 4] of long entries: entry, first row, rows, flags
     split: bool = False                               # some long entry has more than one segment
+    portions: Optional[torch.Tensor] = None           # the long entries as segments of one piece each (None: ``segments`` are)
+    fresh_rows: tuple = ()                            # rows of every long entry, if all of them start at position 0
     order: list = field(default_factory=list)         # entry e of the packing is sequence order[e] of the caller
     starts: list = field(default_factory=list)        # first packed row of the caller's sequence i
     scratch: dict = field(default_factory=dict)       # what layers of one step share
@@ -318,10 +320,18 @@ def ragged_arrays(seqs, windows, block_size, memory_units=0, latent=False, memor
         starts[i] = int(cu[e])
     singles = int((lens == 1).sum())
     segments = _segments(lens, cu, memory_units, memory_coarse) if memory_units else []
+    split = any(not s[3] & 4 for s in segments)
+    long_rows, fresh_rows = lens[num_short:].tolist(), ()
     if segments:
         arrays["segments"] = np.asarray(segments, dtype=np.int32)
+        if all(p == 0 for p, _, _ in items[num_short:]):
+            fresh_rows = tuple(long_rows)
+            if split:
+                arrays["portions"] = portions = np.full((len(long_rows), 4), 7, dtype=np.int32)
+                portions[:, 0] = np.arange(num_short, len(items))
+                portions[:, 1], portions[:, 2] = cu[num_short:-1], long_rows
     facts = dict(num_tokens=int(cu[-1]), num_entries=len(items), num_single=singles, multi_rows=int(cu[-1]) - singles,
-                 num_short=num_short, short_rows=int(cu[num_short]), split=any(not s[3] & 4 for s in segments), order=order, starts=starts)
+                 num_short=num_short, short_rows=int(cu[num_short]), split=split, fresh_rows=fresh_rows, order=order, starts=starts)
     return arrays, [a for a, _ in per_window], [c for _, c in per_window], facts
 
 

@@ -58,17 +58,49 @@ def chunked_takes(proj: torch.Tensor, dim: int, vdim: int) -> bool:
             and proj.shape[1] % 8 == 0 and (proj.shape[0] == 1 or proj.stride(0) % 8 == 0))
 
 
+MAX_PARTS = 16            # csrc/memory_chunk.h: kMaxParts
+PASS_OVER = 0.3           # ... kPassOver
+CUS = 256
+
+
+def chunked_output_fits(dim: int, vdim: int, gate: int, weight: torch.Tensor) -> bool:
+    """Whether the block form's own norm and gate take this layer: whole heads of up to 128 x 256, but not those up to 128 columns, of
+    which half a workgroup's waves would have none."""
+    return dim <= 128 and 128 < vdim <= 256 and gate % 8 == 0 and weight.data_ptr() % 16 == 0
+
+
+def chunked_output_parts(fresh_rows: tuple, split: bool, heads: int, vdim: int) -> int:
+    """How many workgroups share the rows of a head of portions that start from nothing (``fresh_rows``; none if one of them does not).
+
+    A workgroup passes over the blocks in front of its own part, updating the state alone, at 0.3 of a block's time: with enough of them
+    a portion of n blocks takes 0.3 n blocks' time instead of n, in one launch, as long as all run at once.  us in one part and
+    shared, captured, heads of 128 x 256: 8 x 16 of 1024 rows 142 / 105 (2 parts), of 256 41 / 33.5; 8 heads, one portion of 128 17.6 / 16.2,
+    of 305 32 / 24.  Where the step's segments are cut (``split``), those cost two more passes and three launches but then go on side by
+    side however long a portion is: 34 us and the more, the more blocks there are in all.  us in segments and shared: 7 x 8 of
+    1000 rows 83 / 64.5, 4 x 16 of 1000 91.5 / 66, 2 x 16 of 800 54 / 45, 8 of 512 35.3 / 31.3, 4 x 8 of 1500 68.6 / 73, 8 of
+    1024 43.5 / 51.  (Fewer columns, less state to combine: of 128 x 136, 4 x 8 of 1500 61.8 / 72, 2 x 16 of 800 48 / 45.)"""
+    groups = heads * len(fresh_rows)
+    blocks = max((-(-n // BLOCK_ROWS) for n in fresh_rows), default=0)
+    parts = min(MAX_PARTS, CUS // max(groups, 1), blocks)
+    if parts < 2:
+        return 1
+    if split:
+        shared = 10.5 + 8.2 * PASS_OVER / (1 - (1 - PASS_OVER) ** parts) * blocks
+        segments = 32 + 0.053 * (0.5 + vdim / 512) * heads * sum(-(-n // BLOCK_ROWS) for n in fresh_rows)
+        if shared >= segments:
+            return 1
+    return parts
+
+
 def chunked_output_takes(segments: int, rows: int, heads: int, dim: int, vdim: int, gate: int, weight: torch.Tensor) -> bool:
     """Whether ``rows`` of long entries in ``segments`` go through the norm and the output gate in the block form's own pass.
 
-    A workgroup holds all columns of a head, so heads up to 128 x 256, but not those up to 128 columns, of which half its waves
-    would have none.  It takes longer per block of rows than two workgroups of the other form (9.5 us against 8), which have twice as
+    A workgroup holds all columns of a head.  It takes longer per block of rows than two workgroups of the other form (9.5 us against 8), which have twice as
     many CUs while there are few of them, and saves a launch and the sums' way through memory.  us this form / the other, captured, heads of
     128 x 256: 64 segments of 200 rows and heads 40 / 36, 128 of them 44 / 48, 8 x 16 of 1024 rows 145 / 159; 96 of 100 rows 23.7 / 25.0, 80 of
     100 and of 190 23.2 / 22.9 and 32.6 / 33.7; 8 of 64, one block, 13.1 / 13.2 (and 12.4 / 20.2 where the launches are not captured and the host
     is the bound), 8 of 72 21.7 / 19.1 (20.7 / 20.2), 8 of 150 29.9 / 25.0.  Of 64 x 256: 8 of 100 rows 17.6 / 15.5 but 16.8 / 20.4 not captured."""
-    fits = dim <= 128 and 128 < vdim <= 256 and gate % 8 == 0 and weight.data_ptr() % 16 == 0
-    return fits and (segments * heads >= 96 or rows <= (100 if dim <= 64 else BLOCK_ROWS) * segments)
+    return chunked_output_fits(dim, vdim, gate, weight) and (segments * heads >= 96 or rows <= (100 if dim <= 64 else BLOCK_ROWS) * segments)
 
 
 def mlstm(step, proj: torch.Tensor, gates: torch.Tensor, gate_col: int, weight: torch.Tensor, state: MlstmState,
@@ -96,8 +128,11 @@ def mlstm(step, proj: torch.Tensor, gates: torch.Tensor, gate_col: int, weight: 
     lib = _C.load()
     scale = dim ** -0.5
     blocks = step.segments is not None and chunked_takes(proj, dim, vdim)
-    # rows of long entries straight to their outputs
-    whole = blocks and step.short_rows is not None and \
+    # rows of long entries straight to their outputs, in several parts of a head's rows or in segments
+    parts = 1
+    if blocks and step.short_rows is not None and chunked_output_fits(dim, vdim, gate, weight):
+        parts = chunked_output_parts(step.fresh_rows, step.split, heads, vdim)
+    whole = parts > 1 or blocks and step.short_rows is not None and \
         chunked_output_takes(step.segments.shape[0], rows - step.short_rows, heads, dim, vdim, gate, weight)
     plain = step.short_rows if whole else rows                # rows whose norm and gate are a pass of their own
     state_of = (_ptr(state.s), _ptr(state.n), _ptr(state.m), _ptr(step.cu_seqlens), _ptr(step.state_slots), _ptr(step.positions))
@@ -115,7 +150,12 @@ def mlstm(step, proj: torch.Tensor, gates: torch.Tensor, gate_col: int, weight: 
         nbytes = lib.mvllm_mlstm_chunked_workspace_bytes(count, heads, dim, vdim) if step.split else 0
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
         tail = (_ptr(step.segments), count, int(step.split), heads, dim, vdim, scale, DEN_FLOOR, code, _ptr(ws), nbytes, stream)
-        if whole:
+        if parts > 1:
+            portions = step.segments if step.portions is None else step.portions
+            _C.check(lib.mvllm_mlstm_chunked_output_parts(
+                _ptr(out), _ptr(weight), gate, float(eps), _ptr(proj), stride, _ptr(gates), *state_of, _ptr(portions), portions.shape[0],
+                parts, heads, dim, vdim, scale, DEN_FLOOR, code, stream), "mlstm_chunked_output_parts")
+        elif whole:
             _C.check(lib.mvllm_mlstm_chunked_output(_ptr(out), _ptr(weight), gate, float(eps), _ptr(proj), stride, _ptr(gates),
                                                     *state_of, *tail), "mlstm_chunked_output")
         else:

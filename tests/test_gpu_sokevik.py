@@ -490,6 +490,50 @@ def test_mlstm_whole_heads_whatever_runs_beside(monkeypatch, heads, dim, vdim):
     test_mlstm_whole_heads(monkeypatch, heads, dim, vdim)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 256), (3, 24, 136), (2, 72, 144)])
+@pytest.mark.parametrize("parts", [2, 3, 16])
+def test_mlstm_rows_of_a_head_in_parts(monkeypatch, parts, heads, dim, vdim):
+    """Heads whose rows several workgroups share: an odd and an even number of blocks to pass over, one row past a block, fewer blocks than
+    parts, gates that forget everything and nothing, short entries beside them; and portions that go on from a state, which are not
+    shared.  Against the recurrence, as the other forms; the state against that of one part: sums of fp32 products in
+    the same order, with the blocks' decays multiplied at other places (2^-24 each, at most 16 blocks of 64 rows: 1e-5)."""
+    from minivllm_amd.layers import recurrent
+    lengths = [1, 40, 64, 65, 129, 20, 333, 960]
+    forget = [3.0, -30.0, 8.0, 3.0, 0.0, 3.0, -1.0, 5.0]
+    cases = [_memory_case(70 + i, n, heads, dim, vdim, torch.bfloat16, f, 1.0) for i, (n, f) in enumerate(zip(lengths, forget))]
+    weight, col = cases[0][2], cases[0][3]
+    states = []
+    for count in (1, parts):
+        monkeypatch.setattr(recurrent, "chunked_output_parts", lambda *_, count=count: count)
+        monkeypatch.setattr(recurrent, "chunked_output_takes", lambda *_: True)
+        m, seqs = manager([], 1, 16, len(lengths)), []
+        for n in lengths:
+            s = Sequence([1] * n, block_size=16)
+            m.allocate(s)
+            s.num_computed_tokens, s.num_scheduled_tokens = 0, n
+            seqs.append(s)
+        state = MlstmState.allocate(len(lengths), heads, dim, vdim, DEV)
+        for t in (state.s, state.n, state.m):
+            t.fill_(float("nan"))
+        step = ragged_step(seqs, [], 16, DEV, 1)
+        assert step.split and step.portions[:, 2].tolist() == [n for n in lengths if n >= 33] == list(step.fresh_rows)
+        if count == 1:                                               # in one piece, as the parts
+            step.segments, step.split = step.portions, False
+        proj, gates = (torch.cat([cases[i][j] for i in step.order]).to(DEV) for j in (0, 1))
+        out = mlstm(step, proj, gates, col, weight.to(DEV), state, 1e-4).cpu()
+        for i, n in enumerate(lengths):
+            want = _memory_reference(cases[i][0], cases[i][1], weight, heads, dim, vdim, 1e-4)
+            got = out[step.starts[i]:step.starts[i] + n]
+            assert rel(got, want) < 4e-3, (count, i)
+            per_row = (got.double() - want).pow(2).mean(-1).sqrt() / want.pow(2).mean(-1).sqrt()
+            assert per_row.max() < 2e-2, (count, i, int(per_row.argmax()))
+        states.append([t.cpu() for t in (state.s, state.n, state.m)])
+    for one, shared in zip(*states):
+        assert rel(shared, one.double()) < 1e-5
+    # a state to go on from: one part, whatever is asked for
+    test_mlstm_portions(torch.bfloat16, heads, dim, vdim, [100, 200])
+
+
 # ---- the model ----
 _runners: dict = {}
 

@@ -208,6 +208,34 @@ def test_segments_of_portions(lens, units, coarse, rows):
     assert len(got) == sum(len(w) for w in rows)
 
 
+@pytest.mark.parametrize("rows,split,heads,vdim,parts", [
+    ((), False, 8, 256, 1), ((64,), False, 8, 256, 1), ((65,), False, 8, 256, 2), ((2000,) * 8, False, 16, 256, 2),      # one block; two; all CUs twice
+    ((2000,) * 9, False, 16, 256, 1), ((70,), False, 1, 256, 2), ((5000,), False, 1, 256, 16), ((1000, 70), False, 1, 256, 16),
+    ((1000,) * 7, True, 8, 256, 4), ((512,), True, 8, 256, 8), ((1024,), True, 8, 256, 1), ((800,) * 2, True, 16, 256, 8),
+    ((1500,) * 4, True, 8, 256, 1), ((1500,) * 4, True, 8, 136, 1), ((2500, 1500, 500), True, 16, 256, 1),               # segments go on side by side
+])
+def test_parts_of_a_heads_rows(rows, split, heads, vdim, parts):
+    from minivllm_amd.layers.recurrent import chunked_output_parts
+    assert chunked_output_parts(rows, split, heads, vdim) == parts
+
+
+@pytest.mark.parametrize("computed,segments", [((0, 0), True), ((0, 5), False)])
+def test_portions_that_start_from_nothing(computed, segments):
+    """Whole portions stand beside the segments only where all long ones start at position 0."""
+    m = manager([], 400, 16, 8)
+    seqs = []
+    for p, n in zip(computed, (700, 40)):
+        s = Sequence([1] * (p + n), block_size=16)
+        m.allocate(s)
+        s.num_computed_tokens, s.num_scheduled_tokens = p, n
+        seqs.append(s)
+    arrays, _, _, facts = ragged_arrays(seqs, [], 16, memory_units=3)
+    assert facts["split"] and facts["fresh_rows"] == ((700, 40) if segments else ())
+    assert ("portions" in arrays) == segments
+    if segments:
+        assert arrays["portions"].tolist() == [[0, 0, 700, 7], [1, 700, 40, 7]]
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_ragged_arrays_against_row_by_row(seed):
     rng = random.Random(seed)
