@@ -321,6 +321,19 @@ int mvllm_prefill_ranges(void* out, const void* q, const void* k, const void* v,
                          size_t workspace_bytes, void* stream);
 
 /*
+ * The same for fp32 tensors (packed or over an fp32 cache; block_size a multiple of 16), in ranges of `range_tiles` tiles of 32 keys.
+ */
+int mvllm_prefill_f32_ranges_plan(int num_seqs, int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads,
+                                  int head_dim, int block_size);
+size_t mvllm_prefill_f32_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim,
+                                                int range_tiles);
+int mvllm_prefill_f32_ranges(float* out, const float* q, const float* k, const float* v, const int32_t* block_tables,
+                             int max_num_blocks, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int num_seqs,
+                             int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads, int head_dim,
+                             int block_size, int64_t num_blocks, float scale, const float* sink, int range_tiles,
+                             void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * The caller's per-layer chain between the QKV projection and the attention kernels, fused:
  *   q = rms_norm(q); k = rms_norm(k)      src/myvllm/models/qwen3.py:104-106, layers/layernorm.py:9-17
  *   q, k = rotary_emb(positions, q, k)    qwen3.py:108, layers/rotary_embedding.py:4-23, 77-83

@@ -25,7 +25,11 @@ constexpr int kF32Keys = 32;            // keys per tile
 
 typedef float v16f32 __attribute__((ext_vector_type(16)));
 
-template <int D, int HPW, bool PAGED>
+// RANGES: workgroup y walks the key tiles [y range_tiles, (y + 1) range_tiles) of its rows, the last one all that are left; a row tile
+// with several writes their results and log sums to part and lse (see PrefillArgs), others go straight to out.  A matrix unit that has one wave takes
+// 2.8 us per tile of 32 keys at head_dim 64 (64 products of 64 clocks) however empty the chip is: three prompts of 78 rows behind 1480
+// keys, 16 heads over 8, 48 workgroups: 136 us whole, 40 in ranges.
+template <int D, int HPW, bool PAGED, bool RANGES>
 __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const PrefillArgs a) {
   static_assert(D == 128 || D == 64, "head_dim 128 or 64");
   constexpr int kRowB = D * 4;                  // bytes per tile row
@@ -51,7 +55,10 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
   const unsigned round = slot / kXcdChunk;
   const unsigned item = (round * 8 + ((xcd + round) & 7)) * kXcdChunk + slot % kXcdChunk;
   int item_y, seq_start, seq_len, row0, seq_index;
-  if (a.num_seqs <= 64) {
+  if constexpr (RANGES) {                                            // slices fastest, nothing padded (prefill_mfma.h)
+    item_y = (int)(id % (unsigned)a.heads_y);
+    if (!locate_tile(a.cu_seqlens, a.num_seqs, tiles_x - 1 - (int)(id / (unsigned)a.heads_y), BM, seq_start, seq_len, row0, seq_index)) return;
+  } else if (a.num_seqs <= 64) {
     if (!locate_banded<BM>(a.cu_seqlens, a.num_seqs, item, a.heads_y, a.band_bits, a.band_shift, seq_start, seq_len, row0, seq_index, item_y)) return;
   } else {
     if (item >= (unsigned)tiles_x * (unsigned)a.heads_y) return;
@@ -78,7 +85,13 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
   const int pos0 = cached + r0;                                       // position of that row among the keys
   const int j_last = min(pos0 + kWaveRows - 1, kv_len - 1) / kF32Keys;   // last tile any row of the wave sees
   const int wg_last = min(row0 + BM, seq_len) - 1;
-  const int ntiles = (cached + wg_last) / kF32Keys + 1;               // tiles the workgroup walks
+  int ntiles = (cached + wg_last) / kF32Keys + 1;                     // tiles the workgroup walks: [t0, ntiles)
+  const int t0 = RANGES ? (int)blockIdx.y * a.range_tiles : 0;
+  const bool in_ranges = RANGES && gridDim.y > 1 && ntiles > a.range_tiles;
+  if constexpr (RANGES) {
+    if (t0 >= ntiles) return;
+    if (blockIdx.y + 1 < gridDim.y) ntiles = min(ntiles, t0 + a.range_tiles);
+  }
   const int l32 = lane & 31;
   const int hi = lane >> 5;
   const int qrow = r0 + l32;                                          // query row of this lane
@@ -133,7 +146,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
       dma16_to_lds<2 * kTileBytes + i * 1024>(rv, src_off[i], base);
     });
   };
-  issue_tile(0, 0);
+  issue_tile(t0, t0 & 1);
 
   // ---- Q: this lane's row, dims 2 s + hi, times scale * log2 e ----
   float qf[kSteps];
@@ -160,7 +173,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
   const int k_row_off = l32 * kRowB;
   const int k_swz = swz(l32);
 
-  for (int j = 0; j < ntiles; ++j) {
+  for (int j = t0; j < ntiles; ++j) {
     dma_wait_all();
     __syncthreads();                             // tile j has landed; everybody is done with tile j - 1
     if (j + 1 < ntiles) issue_tile(j + 1, (j + 1) & 1);
@@ -198,13 +211,15 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
     for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
     mx = max_with_lane_xor32(mx);
     const float m_new = fmaxf(m, mx);
-    const float alpha = fast_exp2(m - m_new);    // m = -inf at the first tile: 0
+    // m = -inf at the first tile: 0.  A range may begin behind what a row sees: its maximum stays -inf, and its weights are zeros.
+    const float m_ref = RANGES && m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = fast_exp2(m - m_ref);
     m = m_new;
     l *= alpha;
     float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = fast_exp2(s[r] - m_new);
+      s[r] = fast_exp2(s[r] - m_ref);
       sum += s[r];
     }
     l += sum;
@@ -232,8 +247,16 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
   // ---- output: lane (row l32, hi) holds dims 32 t + 8 (r / 4) + 4 hi + r % 4 ----
   const float row_sum = sum_with_lane_xor32(l);   // (every lane takes part in the exchange)
   if (active && qrow < seq_len) {
-    const float inv = 1.f / (a.sink != nullptr ? add_sink(row_sum, m, a.sink[h]) : row_sum);
-    float* dst = reinterpret_cast<float*>(a.out) + ((int64_t)(seq_start + qrow) * a.num_heads + h) * D;
+    int64_t at = (int64_t)(seq_start + qrow) * a.num_heads + h;
+    float inv = 1.f / (a.sink != nullptr && !in_ranges ? add_sink(row_sum, m, a.sink[h]) : row_sum);
+    float* dst = reinterpret_cast<float*>(a.out);
+    if (RANGES && in_ranges) {
+      at += (int64_t)blockIdx.y * a.total_tokens * a.num_heads;
+      inv = row_sum > 0.f ? inv : 0.f;             // (no keys)
+      dst = a.part;
+      if (hi == 0) a.lse[at] = row_sum > 0.f ? log2f(row_sum) + m : -INFINITY;
+    }
+    dst += at * D;
 #pragma unroll
     for (int t = 0; t < kTD; ++t)
 #pragma unroll
@@ -243,13 +266,13 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
   }
 }
 
-template <int D, bool PAGED>
-int launch_f32_as(const PrefillArgs& a, hipStream_t stream) {
+template <int D, bool PAGED, bool RANGES>
+int launch_f32_as(const PrefillArgs& a, hipStream_t stream, int ranges = 1) {
   const int group = a.num_heads / a.num_kv_heads;
   const int hpw = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
   const int bm = kWaveRows * (kPfWaves / hpw);
   PrefillArgs b = a;
-  b.band_shift = band_shift_for(a.total_tokens, a.num_seqs, bm, PAGED);
+  b.band_shift = RANGES ? 0 : band_shift_for(a.total_tokens, a.num_seqs, bm, PAGED);
   b.tiles_x = a.num_seqs <= 64 ? (int)(a.total_tokens / bm + ((int64_t)a.num_seqs << b.band_shift))
                                : (int)(a.total_tokens / bm + a.num_seqs);
   b.heads_y = a.num_kv_heads * (group / hpw);
@@ -257,10 +280,10 @@ int launch_f32_as(const PrefillArgs& a, hipStream_t stream) {
   while (((int64_t)1 << b.band_bits) <= a.total_tokens / (bm << b.band_shift) + 1) ++b.band_bits;
   const int64_t items = (int64_t)b.tiles_x * b.heads_y;
   const int64_t span = 8 * (int64_t)kXcdChunk;
-  const dim3 grid((unsigned)((items + span - 1) / span * span)), block(64 * kPfWaves);
-  if (hpw == 4) prefill_f32_kernel<D, 4, PAGED><<<grid, block, 0, stream>>>(b);
-  else if (hpw == 2) prefill_f32_kernel<D, 2, PAGED><<<grid, block, 0, stream>>>(b);
-  else prefill_f32_kernel<D, 1, PAGED><<<grid, block, 0, stream>>>(b);
+  const dim3 grid(RANGES ? (unsigned)items : (unsigned)((items + span - 1) / span * span), (unsigned)ranges), block(64 * kPfWaves);
+  if (hpw == 4) prefill_f32_kernel<D, 4, PAGED, RANGES><<<grid, block, 0, stream>>>(b);
+  else if (hpw == 2) prefill_f32_kernel<D, 2, PAGED, RANGES><<<grid, block, 0, stream>>>(b);
+  else prefill_f32_kernel<D, 1, PAGED, RANGES><<<grid, block, 0, stream>>>(b);
   return launch_status();
 }
 
@@ -268,9 +291,14 @@ int launch_f32_as(const PrefillArgs& a, hipStream_t stream) {
 
 // fp32 q / k / v (and fp32 paged cache), head_dim 128 or 64; paged: block_size a multiple of 16
 int launch_prefill_f32(const PrefillArgs& a, bool paged, hipStream_t stream) {
-  if (a.head_dim == 128) return paged ? launch_f32_as<128, true>(a, stream) : launch_f32_as<128, false>(a, stream);
-  if (a.head_dim == 64) return paged ? launch_f32_as<64, true>(a, stream) : launch_f32_as<64, false>(a, stream);
+  if (a.head_dim == 128) return paged ? launch_f32_as<128, true, false>(a, stream) : launch_f32_as<128, false, false>(a, stream);
+  if (a.head_dim == 64) return paged ? launch_f32_as<64, true, false>(a, stream) : launch_f32_as<64, false, false>(a, stream);
   return MVLLM_ERR_UNSUPPORTED;
+}
+
+int launch_prefill_f32_ranges(const PrefillArgs& a, bool paged, int ranges, hipStream_t s) {
+  if (a.head_dim == 128) return paged ? launch_f32_as<128, true, true>(a, s, ranges) : launch_f32_as<128, false, true>(a, s, ranges);
+  return paged ? launch_f32_as<64, true, true>(a, s, ranges) : launch_f32_as<64, false, true>(a, s, ranges);
 }
 
 }  // namespace mvllm

@@ -827,6 +827,8 @@ int launch_prefill_paged_int8(const PrefillArgs& a, int dtype, hipStream_t strea
 int launch_prefill_ranges(const PrefillArgs& a, int dtype, bool paged, int ranges, hipStream_t stream);
 // fp32 tensors, head_dim 128 or 64, packed or over a paged fp32 cache (prefill_f32.hip)
 int launch_prefill_f32(const PrefillArgs& a, bool paged, hipStream_t stream);
+// ... over ranges of their 32-key tiles side by side
+int launch_prefill_f32_ranges(const PrefillArgs& a, bool paged, int ranges, hipStream_t stream);
 // every other multiple of 8 from 32 to 120, and 256 (prefill_other_dims.hip, prefill_half_step_dims.hip); 16-bit element types only
 bool prefill_mfma_other_dim(int head_dim);
 int launch_prefill_mfma_other(const PrefillArgs& a, int dtype, bool paged, hipStream_t stream);

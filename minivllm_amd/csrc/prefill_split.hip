@@ -175,7 +175,7 @@ struct RangeMergeArgs {
   const float* sink;
   int num_seqs, ranges, range_tiles, rows_per_tile, total_q, num_heads;
 };
-template <typename T, int D>
+template <typename T, int D, int kKeys = 64>
 __global__ __launch_bounds__(256) void range_merge_kernel(const RangeMergeArgs a) {
   constexpr int kHeads = 256 / D, kLanes = D / 4;  // heads of a wave, lanes of a head
   const int lane = threadIdx.x & 63, t = blockIdx.x;
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256) void range_merge_kernel(const RangeMergeArgs a
   const int start = __builtin_amdgcn_readlane(lo, s), len = __builtin_amdgcn_readlane(end, s) - start;
   const int kv = a.cu_seqlens_k ? a.cu_seqlens_k[s + 1] - a.cu_seqlens_k[s] : len, cached = max(kv - len, 0);
   const int last = min((t - start) / a.rows_per_tile * a.rows_per_tile + a.rows_per_tile, len) - 1;
-  const int tiles = min((cached + last) / 64, (kv - 1) / 64) + 1;
+  const int tiles = min((cached + last) / kKeys, (kv - 1) / kKeys) + 1;
   if (tiles <= a.range_tiles) return;
   const int n = min((tiles + a.range_tiles - 1) / a.range_tiles, a.ranges);
   const int h = (blockIdx.y * 4 + (threadIdx.x >> 6)) * kHeads + lane / kLanes, c = 4 * (lane % kLanes);
@@ -224,8 +224,11 @@ __global__ __launch_bounds__(256) void range_merge_kernel(const RangeMergeArgs a
   }
   if (a.sink != nullptr) den = add_sink(den, top, a.sink[h]);
   const float inv = 1.f / den;
-  *reinterpret_cast<uint2*>(reinterpret_cast<T*>(a.out) + at * D + c) =
-      make_uint2(pack2<T>(acc.x * inv, acc.y * inv), pack2<T>(acc.z * inv, acc.w * inv));
+  if constexpr (std::is_same_v<T, float>)
+    *reinterpret_cast<float4*>(reinterpret_cast<float*>(a.out) + at * D + c) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+  else
+    *reinterpret_cast<uint2*>(reinterpret_cast<T*>(a.out) + at * D + c) =
+        make_uint2(pack2<T>(acc.x * inv, acc.y * inv), pack2<T>(acc.z * inv, acc.w * inv));
 }
 
 int gcd_int(int x, int y) {
@@ -567,5 +570,108 @@ extern "C" int mvllm_prefill_ranges(void* out, const void* q, const void* k, con
     if (head_dim == 128) range_merge_kernel<f16_t, 128><<<grid, dim3(256), 0, s>>>(m);
     else range_merge_kernel<f16_t, 64><<<grid, dim3(256), 0, s>>>(m);
   }
+  return launch_status();
+}
+
+// ---- the same for fp32 (prefill_f32.hip), whose tiles are 32 keys ----
+
+static bool f32_ranges_shape_ok(int num_seqs, int64_t total_q, int max_kv_len, int num_heads, int num_kv_heads, int head_dim, int block_size) {
+  if (num_seqs <= 0 || num_seqs > 64 || total_q <= 0 || max_kv_len <= 0 || num_heads <= 0 || num_kv_heads <= 0 || block_size < 0) return false;
+  if (num_heads % num_kv_heads != 0 || num_heads > 65535 || (head_dim != 128 && head_dim != 64) || block_size % 16 != 0) return false;
+  if ((int64_t)num_kv_heads * head_dim * 4 * 64 >= ((int64_t)1 << 31) || (int64_t)block_size * num_kv_heads * head_dim * 4 >= ((int64_t)1 << 31)) return false;
+  return total_q <= ((int64_t)1 << 24);
+}
+static int64_t f32_ranges_of(int64_t max_kv_len, int64_t range_tiles) { return ((max_kv_len + 31) / 32 + range_tiles - 1) / range_tiles; }
+
+// The range for a batch of these sizes, all tiles where none is cut; 0: the kernel over whole rows.  A tile of 32 keys takes a workgroup 2.6 us
+// at head_dim 64, 5.5 at 128, alone on its CU or in turns with another one, so what counts is how many tiles the busiest CU gets: `even` workgroups of equal
+// sequences, the share of the longest one's tiles that they have on average, and 0.3 of a workgroup more where there are more than CUs or where
+// the order has places without rows among them, two of which can meet.  The other order's places (256 rows of a sequence at a time) leave half of
+// them empty from 128 rows per sequence down: 12 prompts of 60 rows behind 1100, 16 heads over 8 of 64 (96 workgroups of 384 places) 174 us there, 107 in this
+// order uncut and 54 in 8 ranges; 16 of 100 behind 1900, 32 heads (512 workgroups) 425 and 300.  A merge is a launch (4 us) and
+// the partial results' way through memory.  us whole and as planned, dims 64: 3 of 78 rows behind 1480, 16 heads 136 / 40; 20 behind 500
+// 50 / 16; 40 behind 4000 331 / 30; one of 400, nothing cached, 36 / 23; 860 behind 860, 32 heads 148 / 115; two of 800 68 / 52, 32 heads
+// 93, stay; 2000 behind 2000 (504 workgroups) 494 / 470; dims 128: 3 of 78 behind 1480 311 / 79, one of 2000 306 / 232.
+extern "C" int mvllm_prefill_f32_ranges_plan(int num_seqs, int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads,
+                                             int head_dim, int block_size) {
+  if (!f32_ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size)) return 0;
+  const int bm = rows_of_tile(num_heads / num_kv_heads);
+  const int64_t slices = (int64_t)num_heads * bm / 128, tiles = f32_ranges_of(max_kv_len, 1), rows = (total_q_tokens + num_seqs - 1) / num_seqs;
+  const int64_t even = num_seqs * ((rows + bm - 1) / bm) * slices, slots = (total_q_tokens / bm + num_seqs) * slices;
+  const int64_t places = num_seqs * ((rows + 255) / 256) * (256 / bm) * slices;
+  const float fresh = fminf(1.f, (float)total_q_tokens / ((float)num_seqs * (float)max_kv_len)), share = 1.f - 0.5f * fresh;
+  const float tile = head_dim == 64 ? 2.6f : 5.5f, of_cus = (float)even / 256.f;
+  const bool gaps = 10 * slots > 11 * even, padded = block_size > 0 && places > 256 && 2 * even <= places;
+  auto busiest = [&](int64_t n) {                           // of n ranges, in ranges
+    const bool meet = gaps && slots * n > 256;
+    if (of_cus * (share * (float)n + 0.5f * fresh) <= 1.f && !meet) return 1.f;
+    return fmaxf(1.f, 0.95f * share * of_cus * (float)n + (meet ? 0.6f : 0.3f));
+  };
+  const float whole = tile * (float)tiles * fmaxf(1.f, share * of_cus + (even > 256 ? 0.3f : 0.f)) * (padded ? 1.4f : 1.f);
+  const float per_range = 0.3f + 0.7f * 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f;
+  float best = 0.93f * whole - 1.f;
+  int64_t p = 0;
+  if (padded && tile * (float)tiles * busiest(1) < best) {
+    best = tile * (float)tiles * busiest(1);
+    p = tiles;
+  }
+  if (padded && even > 256) return (int)p;
+  for (int64_t most = tiles < kMaxRanges ? tiles : kMaxRanges; most > 1; --most) {
+    const int64_t x = (tiles + most - 1) / most, n = (tiles + x - 1) / x;
+    if (x < 2 || x >= tiles) continue;
+    const float us = tile * (float)x * busiest(n) + 4.f + per_range * (float)n;
+    if (us < best) {
+      best = us;
+      p = x;
+    }
+  }
+  return (int)p;
+}
+
+extern "C" size_t mvllm_prefill_f32_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim,
+                                                           int range_tiles) {
+  if (total_q_tokens <= 0 || max_kv_len <= 0 || num_heads <= 0 || head_dim <= 0 || range_tiles <= 0) return 0;
+  const int64_t ranges = f32_ranges_of(max_kv_len, range_tiles);
+  return ranges < 2 ? 0 : (size_t)ranges * total_q_tokens * num_heads * (head_dim + 1) * sizeof(float);
+}
+
+extern "C" int mvllm_prefill_f32_ranges(float* out, const float* q, const float* k, const float* v, const int32_t* block_tables,
+                                        int max_num_blocks, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int num_seqs,
+                                        int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads, int head_dim,
+                                        int block_size, int64_t num_blocks, float scale, const float* sink, int range_tiles,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+  const bool paged = block_size > 0;
+  if (num_seqs < 0 || total_q_tokens < 0 || max_kv_len < 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || block_size < 0 ||
+      num_blocks < 0 || max_num_blocks < 0 || num_heads % num_kv_heads != 0 || !(scale > 0.f) || range_tiles <= 0)
+    return MVLLM_ERR_BAD_SHAPE;
+  if (num_seqs == 0 || total_q_tokens == 0) return MVLLM_OK;
+  if (!out || !q || !k || !v || !cu_seqlens_q || (paged && (!block_tables || !cu_seqlens_k))) return MVLLM_ERR_NULL_POINTER;
+  if (!f32_ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size) ||
+      f32_ranges_of(max_kv_len, range_tiles) > kMaxRanges)
+    return MVLLM_ERR_UNSUPPORTED;
+  const int ranges = (int)f32_ranges_of(max_kv_len, range_tiles);
+  if (!aligned16(q) || !aligned16(out) || !aligned16(k) || !aligned16(v)) return MVLLM_ERR_MISALIGNED;
+  if ((ranges > 1 && (!workspace || !aligned16(workspace))) ||
+      workspace_bytes < mvllm_prefill_f32_ranges_workspace_bytes(total_q_tokens, max_kv_len, num_heads, head_dim, range_tiles))
+    return MVLLM_ERR_WORKSPACE;
+  hipStream_t s = (hipStream_t)stream;
+  PrefillArgs a = {};
+  a.out = out; a.q = q; a.k = k; a.v = v; a.cu_seqlens = cu_seqlens_q; a.total_tokens = total_q_tokens; a.num_seqs = num_seqs;
+  a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.head_dim = head_dim; a.scale_log2 = scale * kLog2e;
+  a.cu_seqlens_k = paged ? cu_seqlens_k : nullptr; a.block_tables = paged ? block_tables : nullptr; a.max_num_blocks = max_num_blocks;
+  a.block_size = block_size; a.num_blocks = num_blocks; a.sink = sink;
+  a.range_tiles = range_tiles;
+  a.part = reinterpret_cast<float*>(workspace);
+  a.lse = ranges > 1 ? a.part + (int64_t)ranges * total_q_tokens * num_heads * head_dim : nullptr;
+  const int status = launch_prefill_f32_ranges(a, paged, ranges, s);
+  if (status != MVLLM_OK || ranges == 1) return status;
+  RangeMergeArgs m;
+  m.out = out; m.part = a.part; m.lse = a.lse; m.cu_seqlens_q = cu_seqlens_q; m.cu_seqlens_k = a.cu_seqlens_k; m.sink = sink;
+  m.num_seqs = num_seqs; m.ranges = ranges; m.range_tiles = range_tiles; m.rows_per_tile = rows_of_tile(num_heads / num_kv_heads);
+  m.total_q = (int)total_q_tokens; m.num_heads = num_heads;
+  const int per = 4 * (256 / head_dim);
+  const dim3 grid((unsigned)total_q_tokens, (unsigned)((num_heads + per - 1) / per));
+  if (head_dim == 128) range_merge_kernel<float, 128, 32><<<grid, dim3(256), 0, s>>>(m);
+  else range_merge_kernel<float, 64, 32><<<grid, dim3(256), 0, s>>>(m);
   return launch_status();
 }

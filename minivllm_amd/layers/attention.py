@@ -224,9 +224,15 @@ def flash_attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, c
     return output
 
 
+_F32 = _C.dtype_code(torch.float32)
+
+
 @lru_cache(maxsize=256)
 def _prefill_ranges_plan(lib, num_seqs, total, max_seqlen, num_heads, num_kv_heads, head_dim, block_size, code):
     """(key tiles per range, workspace bytes) of a batch of these sizes, (0, 0): not over ranges.  Every layer of a step asks again."""
+    if code == _F32:
+        tiles = lib.mvllm_prefill_f32_ranges_plan(num_seqs, total, max_seqlen, num_heads, num_kv_heads, head_dim, block_size)
+        return tiles, lib.mvllm_prefill_f32_ranges_workspace_bytes(total, max_seqlen, num_heads, head_dim, tiles) if tiles else 0
     tiles = lib.mvllm_prefill_ranges_plan(num_seqs, total, max_seqlen, num_heads, num_kv_heads, head_dim, block_size, code)
     return tiles, lib.mvllm_prefill_ranges_workspace_bytes(total, max_seqlen, num_heads, head_dim, tiles) if tiles else 0
 
@@ -242,12 +248,11 @@ def _prefill_ranges(lib, output, q, k, v, block_tables, cu_seqlens_q, cu_seqlens
     if (o_at | q_at | k_at | v_at) % 16:
         return False
     workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None      # none: one range
-    st = lib.mvllm_prefill_ranges(o_at, q_at, k_at, v_at, 0 if block_tables is None else _ptr(block_tables),
-                                  0 if block_tables is None else block_tables.shape[1], _ptr(cu_seqlens_q),
-                                  0 if cu_seqlens_k is None else _ptr(cu_seqlens_k), num_seqs, q.shape[0], max_seqlen, num_heads,
-                                  num_kv_heads, head_dim, block_size, num_blocks, float(scale),
-                                  0 if sink is None else _sink_ptr(sink, num_heads), code, tiles, 0 if workspace is None else _ptr(workspace), need,
-                                  _C.current_stream_ptr(q.device))
+    head = (o_at, q_at, k_at, v_at, 0 if block_tables is None else _ptr(block_tables), 0 if block_tables is None else block_tables.shape[1],
+            _ptr(cu_seqlens_q), 0 if cu_seqlens_k is None else _ptr(cu_seqlens_k), num_seqs, q.shape[0], max_seqlen, num_heads,
+            num_kv_heads, head_dim, block_size, num_blocks, float(scale), 0 if sink is None else _sink_ptr(sink, num_heads))
+    tail = (tiles, 0 if workspace is None else _ptr(workspace), need, _C.current_stream_ptr(q.device))
+    st = lib.mvllm_prefill_f32_ranges(*head, *tail) if code == _F32 else lib.mvllm_prefill_ranges(*head, code, *tail)
     _C.check(st, "prefill over key ranges")
     return True
 
@@ -310,7 +315,7 @@ def flash_attention_prefill_paged(q: torch.Tensor, k_cache: torch.Tensor, v_cach
                                                 _C.current_stream_ptr(q.device))
             _C.check(st, "flash_attention_prefill_paged (staged)")
             return output
-    if max_seqlen_k is not None and int(max_seqlen_k) > 0 and q.dtype != torch.float32:
+    if max_seqlen_k is not None and int(max_seqlen_k) > 0 and (q.dtype != torch.float32 or key_splits is None and block_size % 16 == 0):
         if key_splits is None and _prefill_ranges(lib, output, q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, num_seqs,
                                                   min(int(max_seqlen_k), block_tables.shape[1] * block_size), scale, num_heads,
                                                   num_kv_heads, head_dim, block_size, k_cache.shape[0], sink):

@@ -87,3 +87,49 @@ def test_prefill_ranges_plan_and_rejections():
     assert plan(1, 100, 4000, 16, 8, 80, 16, bf) == 0 and plan(1, 100, 4000, 16, 8, 128, 8, bf) == 0
     assert lib.mvllm_prefill_ranges_workspace_bytes(100, 640, 16, 128, 10) == 0
     assert lib.mvllm_prefill_ranges_workspace_bytes(100, 641, 16, 128, 10) == 2 * 100 * 16 * 129 * 4
+
+
+@pytest.mark.parametrize("hq,hkv,d,bs,lengths,cached,tiles", [
+    (8, 2, 128, 16, [64, 65, 63, 1], [32, 50, 62, 0], 1),              # a last tile that ends a range, starts one, falls short of it
+    (8, 4, 64, 32, [160, 700], [96, 690], 3),                          # a range that only the later of two row tiles reaches
+    (5, 5, 64, 48, [600, 300, 64], [470, 10, 63], 4),                  # one head per workgroup, row tiles over several waves
+    (4, 2, 128, 256, [1000, 30], [0, 7], 5),                           # nothing cached: every row tile its own number of ranges
+    (8, 2, 64, 16, [2040], [2030], 1),                                 # 64 ranges
+    (16, 8, 64, 16, [500, 200], [400, 150], 16),                       # whole: one range
+])
+@pytest.mark.parametrize("paged", [True, False])
+def test_fp32_prefill_over_key_ranges(hq, hkv, d, bs, lengths, cached, tiles, paged, monkeypatch):
+    """fp32: against the oracle in 64 bits, 4e-6 of the results' root mean square (sums of up to 2000 fp32 products, weights by exp2 to 2^-21);
+    rows that see nothing of a range, a bound that is too low, a sink against the kernel over whole rows."""
+    c = make_paged_prefill_case(61, lengths, cached, hq, hkv, d, bs, dtype=torch.float32)
+    want = oracle.prefill_paged_oracle(c["q_new"].double(), torch.nan_to_num(c["k_cache"].double()), torch.nan_to_num(c["v_cache"].double()),
+                                       c["block_tables"], c["cu_q"], c["cu_k"], 1 / math.sqrt(d), hq, hkv, d, bs).double()
+    monkeypatch.setattr(attention, "_prefill_ranges_plan", lambda lib, s, t, keys, hq, hkv, d, bs, code: (
+        tiles, lib.mvllm_prefill_f32_ranges_workspace_bytes(t, keys, hq, d, tiles)))
+    for bound in (max(lengths), max(1, max(lengths) - 150)):
+        got = _run(c, hq, hkv, d, bs, tiles, bound, paged)
+        got = got if paged else got[c["new_rows"]]
+        assert torch.isfinite(got).all() and ((got.double() - want).norm() / want.norm()).item() <= 4e-6, bound
+    if not paged:
+        sink = torch.randn(hq, generator=torch.Generator().manual_seed(1)).to(DEV)
+        got = _run(c, hq, hkv, d, bs, tiles, max(lengths), False, sink)
+        whole = attention.flash_attention_prefill(*(c[n].to(DEV) for n in ("q", "k", "v", "cu_k")), d ** -0.5, hq, hkv, d, sink=sink).cpu()
+        assert ((got - whole).norm() / whole.norm()).item() <= 2e-6
+
+
+def test_fp32_ranges_plan_and_rejections():
+    lib = _C.load()
+    plan = lib.mvllm_prefill_f32_ranges_plan
+    assert plan(3, 234, 1558, 16, 8, 64, 16) == 10                       # few rows behind many keys
+    assert plan(12, 720, 1160, 16, 8, 64, 16) in (4, 5, 6) and plan(16, 1600, 2000, 32, 8, 64, 16) == 63      # places without rows in the other order
+    assert plan(8, 1200, 150, 16, 8, 64, 0) == 0 and plan(8, 2400, 600, 32, 8, 64, 16) == 0      # short; the chip is full
+    assert plan(65, 650, 4000, 16, 8, 64, 16) == 0 and plan(1, 100, 4000, 16, 8, 80, 16) == 0 and plan(1, 100, 4000, 16, 8, 64, 8) == 0
+    keys = 2 ** 31 - 1                                                   # a bound that is none
+    per = plan(1, 100, keys, 16, 8, 64, 16)
+    assert -(-(-(-keys // 32)) // per) <= 64
+    bad = lambda *a: lib.mvllm_prefill_f32_ranges(*a)
+    q = torch.zeros(64, 8, 64, device=DEV)
+    cu = torch.tensor([0, 64], dtype=torch.int32, device=DEV)
+    p = q.data_ptr()
+    args = lambda tiles, nbytes, dim=64, ws=p: (p, p, p, p, 0, 0, cu.data_ptr(), 0, 1, 64, 64, 8, 8, dim, 0, 0, 1.0, 0, tiles, ws, nbytes, 0)
+    assert bad(*args(1, 0)) == -5 and bad(*args(1, 1 << 20, ws=0)) == -5 and bad(*args(0, 1 << 20)) == -3 and bad(*args(1, 1 << 20, dim=80)) == -4
