@@ -13,6 +13,7 @@ import torch
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libminivllm_amd.so")
 _lib = None
 _partial = None      # path of a library that holds some of the entry points only (use_library)
+calls = None         # once the library is loaded: csrc/calls.cpp, where it has been built (a partial library's checkout may be without)
 
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
@@ -210,7 +211,16 @@ def load():
         fn.restype = restype
         fn.argtypes = argtypes
     _lib = lib
+    _bind_calls(lib)
     return lib
+
+
+def _bind_calls(lib):
+    global calls
+    if os.path.exists(os.path.join(os.path.dirname(_LIB_PATH), "_calls.so")):
+        from minivllm_amd import _calls
+        _calls.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES if hasattr(lib, name)})
+        calls = _calls
 
 
 def check(status: int, what: str) -> None:

@@ -20,6 +20,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libminivllm_amd.so")
 PROBE_LIB_PATH = os.path.join(PKG_DIR, "libmvllm_probe.so")      # measurement support for bench.py, not an operator
 PROBE_SOURCES = ["mfma_probe.hip"]
+CALLS_PATH = os.path.join(PKG_DIR, "_calls.so")                  # the attention operators' way to the library (csrc/calls.cpp)
 SOURCES = ["capi.hip", "store_kvcache.hip", "paged_decode.hip", "prefill_varlen.hip", "prefill_other_dims.hip", "prefill_half_step_dims.hip", "prefill_pingpong.hip", "prefill_staged.hip", "prefill_split.hip", "prefill_ranges.hip", "prefill_f32.hip", "qk_norm_rope_store.hip", "sampler.hip",
            "rms_norm.hip", "activation.hip", "linear_small.hip", "norm_conv.hip", "head_rope.hip", "gate_linear.hip", "mlstm.hip", "mlstm_chunk.hip",
            "decay_memory.hip", "latent.hip", "moe.hip", "stream_norm.hip", "ring_rows.hip", "window_prefill.hip",
@@ -72,6 +73,25 @@ def _link(lib, members, verbose):
     os.replace(part, lib)
 
 
+def _build_calls(verbose):
+    import sysconfig
+
+    import torch
+    home = os.path.dirname(torch.__file__)
+    part = f"{CALLS_PATH}.{os.getpid()}"
+    include = [os.path.join(os.path.dirname(PKG_DIR), "include"), os.path.join(home, "include"),
+               os.path.join(home, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-I" + i for i in include),
+           os.path.join(CSRC, "calls.cpp"), "-o", part, "-L" + os.path.join(home, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for calls.cpp:\n{res.stderr}")
+    os.replace(part, CALLS_PATH)
+
+
 def build_library(verbose: bool = True, jobs: int = 8) -> str:
     # the long ones first, so that no job is left compiling alone at the end
     order = sorted(SOURCES + PROBE_SOURCES, key=lambda src: -os.path.getsize(os.path.join(CSRC, src)))
@@ -82,9 +102,11 @@ def build_library(verbose: bool = True, jobs: int = 8) -> str:
         probe_decode = pool.submit(_compile, "paged_decode.hip", verbose, ("-DMVLLM_DECODE_LOADS_ONLY=1",), "_loads_only")
         # ... and the two-group prefill kernel with its per-tile clock stamps
         probe_prefill = pool.submit(_compile, "prefill_pingpong.hip", verbose, ("-DMVLLM_PP_TIMELINE=1",), "_timeline")
+        calls = pool.submit(_build_calls, verbose)
         running.update({src: pool.submit(_compile, src, verbose) for src in order[3:]})
         objs = {src: job.result() for src, job in running.items()}
         probes = [probe_decode.result(), probe_prefill.result()]
+        calls.result()
     _link(LIB_PATH, [objs[s] for s in SOURCES], verbose)
     _link(PROBE_LIB_PATH, [objs[s] for s in PROBE_SOURCES] + probes, verbose)
     return LIB_PATH

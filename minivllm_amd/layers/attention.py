@@ -122,6 +122,8 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
     (num_blocks, block_size, num_kv_heads, head_dim); slot_mapping:
     (num_tokens,) flat slot per token, -1 = skip.  Reference: attention.py:67-108.
     """
+    if _C.calls is not None and _C.calls.store(key, value, k_cache, v_cache, slot_mapping):
+        return
     num_tokens, num_kv_heads, head_dim = key.shape
     assert k_cache.shape == v_cache.shape, "K and V cache shapes must match"
     assert slot_mapping.numel() == num_tokens, "Slot mapping size must match number of tokens"
@@ -188,6 +190,11 @@ def flash_attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, c
     which a batch too small to fill the chip has its keys cut into ranges that are walked side by side.
     No device->host synchronisation happens here.
     """
+    if _C.calls is not None and sink is None and out is None:
+        done = _C.calls.prefill(q, k, v, cu_seqlens, scale, num_heads, num_kv_heads, head_dim, max_seqlen, _prefill_ranges_plan, _C.load(),
+                                STAGED_PREFILL_MAX_BYTES)
+        if done is not None:
+            return done
     _C.require_cuda(q, k, v, cu_seqlens)
     if q.dim() != 3 or tuple(q.shape[1:]) != (num_heads, head_dim):
         raise ValueError(f"q must be (total_tokens, {num_heads}, {head_dim}), got {tuple(q.shape)}")
@@ -280,6 +287,11 @@ def flash_attention_prefill_paged(q: torch.Tensor, k_cache: torch.Tensor, v_cach
     ``sink`` and ``out`` as in ``flash_attention_prefill`` (with a sink, block sizes that are not a multiple of 16 stay on
     the generic kernel).
     """
+    if _C.calls is not None and max_seqlen_k is not None and key_splits is None and sink is None and out is None:
+        done = _C.calls.prefill_paged(q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, scale, num_heads, num_kv_heads, head_dim,
+                                      block_size, max_seqlen_k, _prefill_ranges_plan, _C.load(), STAGED_PREFILL_MAX_BYTES)
+        if done is not None:
+            return done
     _C.require_cuda(q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k)
     if q.dim() != 3 or tuple(q.shape[1:]) != (num_heads, head_dim):
         raise ValueError(f"q must be (total_tokens, {num_heads}, {head_dim}), got {tuple(q.shape)}")
@@ -494,6 +506,11 @@ def paged_attention_decode(query: torch.Tensor, k_cache: torch.Tensor, v_cache: 
     partials; without it, or when it is too small, a per-device buffer of this module is used.  ``sink`` and ``out`` as in
     ``flash_attention_prefill``.
     """
+    if _C.calls is not None and sink is None and out is None:
+        done = _C.calls.decode(query, k_cache, v_cache, None, None, block_tables, context_lens, scale, num_heads, num_kv_heads, head_dim,
+                               block_size, workspace, _workspaces.get(query.device.index))
+        if done is not None:
+            return done
     _C.require_cuda(query, k_cache, v_cache, block_tables, context_lens)
     if k_cache.dtype != query.dtype or v_cache.dtype != query.dtype:
         raise ValueError(f"query {query.dtype} and cache {k_cache.dtype} dtypes differ")
@@ -531,6 +548,11 @@ def paged_attention_decode_int8(query: torch.Tensor, k_cache: torch.Tensor, v_ca
                                 workspace: torch.Tensor | None = None) -> torch.Tensor:
     """Paged decode over an int8 cache written by ``store_kvcache_int8`` (``workspace`` as in
     ``paged_attention_decode``)."""
+    if _C.calls is not None:
+        done = _C.calls.decode(query, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens, scale, num_heads, num_kv_heads, head_dim,
+                               block_size, workspace, _workspaces.get(query.device.index))
+        if done is not None:
+            return done
     _C.require_cuda(query, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens)
     if k_cache.dtype != torch.int8 or v_cache.dtype != torch.int8:
         raise ValueError("int8 caches expected")

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass
+from functools import lru_cache
 
 import torch
 
@@ -69,6 +70,7 @@ def chunked_output_fits(dim: int, vdim: int, gate: int, weight: torch.Tensor) ->
     return dim <= 128 and 128 < vdim <= 256 and gate % 8 == 0 and weight.data_ptr() % 16 == 0
 
 
+@lru_cache(maxsize=256)
 def chunked_output_parts(fresh_rows: tuple, split: bool, heads: int, vdim: int) -> int:
     """How many workgroups share the rows of a head of portions that start from nothing (``fresh_rows``; none if one of them does not).
 

@@ -162,6 +162,8 @@ def window_prefill(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, cu_q: to
     (None: the keys), into out (T, H, dim).  Query i of an entry stands at key (keys - queries) + i and sees ``window`` keys up to it
     (0: all); ``slopes`` times the distance is taken off a score, ``temperature`` = (coef, every) makes scores grow with
     ``positions``, ``gate`` (T, H, dim), or (T, H) for one number per head, multiplies the result with its sigmoid."""
+    if _C.calls is not None and _C.calls.window_prefill(out, q, k, cu_q, cu_k, scale, window, k2, v, gate, slopes, positions, *temperature):
+        return
     _C.require_cuda(out, q, k, cu_q, cu_k, k2, v, gate, slopes, positions)
     t, heads = q.shape[:2]
     keys, groups, dim = k.shape

@@ -1,0 +1,29 @@
+"""The native way to the attention operators (csrc/calls.cpp) on the CPU: it takes nothing that is not a plain tensor on a GPU, and says so."""
+import pytest
+import torch
+
+from minivllm_amd import _C
+
+
+@pytest.fixture(scope="module")
+def calls():
+    _C.load()
+    if _C.calls is None:
+        pytest.skip("csrc/calls.cpp has not been built")
+    return _C.calls
+
+
+def test_calls_decline_what_is_not_theirs(calls):
+    x, i, cache = torch.zeros(3, 2, 64), torch.zeros(3, dtype=torch.int64), torch.zeros(2, 16, 2, 64)
+    cu = torch.tensor([0, 3], dtype=torch.int32)
+    plan = lambda *a: pytest.fail("asked for a plan")
+    for q in (x, None, 3, "x", x.half(), torch.nn.Parameter(x)):
+        assert calls.store(q, x, cache, cache, i) is False
+        assert calls.decode(q, cache, cache, None, None, cu[None], i, 1.0, 2, 2, 64, 16, None, None) is None
+        assert calls.prefill(q, x, x, cu, 1.0, 2, 2, 64, None, plan, None, 1 << 30) is None
+        assert calls.prefill_paged(q, cache, cache, cu[None], cu, cu, 1.0, 2, 2, 64, 16, 3, plan, None, 1 << 30) is None
+        assert calls.window_prefill(q, q, x, cu, cu, 1.0, 0, None, x, None, None, None, 0.0, 0) is False
+    assert calls.store() is False and calls.store(x) is False and calls.decode(x) is None and calls.prefill() is None
+    assert calls.prefill_paged(x) is None and calls.window_prefill(x) is False                 # numbers of arguments
+    with pytest.raises(TypeError):
+        calls.bind([1])

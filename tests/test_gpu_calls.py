@@ -1,0 +1,186 @@
+"""The native way to the attention operators (csrc/calls.cpp): the same results, bit for bit, as the longer way, which everything else takes."""
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from minivllm_amd import _C
+from minivllm_amd.layers import attention
+from minivllm_amd.layers.window import window_prefill
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+class Counted:
+    """Passes calls on and counts those that were taken."""
+
+    def __init__(self):
+        self.calls, self.taken = _C.calls, 0
+
+    def __getattr__(self, name):
+        def call(*a):
+            got = getattr(self.calls, name)(*a)
+            self.taken += got is not None and got is not False
+            return got
+        return call
+
+
+@pytest.fixture
+def counted(monkeypatch):
+    _C.load()
+    assert _C.calls is not None
+    counted = Counted()
+    monkeypatch.setattr(_C, "calls", counted)
+    return counted
+
+
+def both(counted, monkeypatch, f, taken):
+    """f() with the native way and without it; how many of its calls were taken."""
+    counted.taken = 0
+    a = f()
+    assert counted.taken == taken
+    with monkeypatch.context() as m:
+        m.setattr(_C, "calls", None)
+        b = f()
+    assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride()
+    assert torch.equal(a, b)
+    return a
+
+
+def normal(*shape, dtype=torch.bfloat16):
+    return torch.randn(*shape, device=DEV, generator=torch.Generator(DEV).manual_seed(sum(shape))).to(dtype)
+
+
+def paged(lengths, block, kv, dim, dtype, int8=False):
+    tables = torch.full((len(lengths), max(-(-n // block) for n in lengths) + 1), -1, dtype=torch.int32)
+    at = 0
+    for b, n in enumerate(lengths):
+        need = -(-n // block)
+        tables[b, :need] = torch.arange(at, at + need)
+        at += need
+    caches = [normal(at, block, kv, dim, dtype=torch.float32) for _ in range(2)]
+    if int8:
+        return tables.to(DEV), [(c * 40).round().clamp(-127, 127).to(torch.int8) for c in caches], [torch.rand(at, block, kv, device=DEV) + 0.01 for _ in range(2)]
+    return tables.to(DEV), [c.to(dtype) for c in caches], []
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lengths,block", [([5], 16), ([300, 1, 77], 16), ([2500, 3000], 256)])
+def test_decode(counted, monkeypatch, dtype, lengths, block):
+    tables, (k, v), _ = paged(lengths, block, 2, 64, dtype)
+    q = normal(len(lengths), 8, 64, dtype=dtype)
+    for lens in (torch.tensor(lengths, device=DEV), torch.tensor(lengths, dtype=torch.int32, device=DEV)):
+        args = (q, k, v, tables, lens, 0.125, 8, 2, 64, block)
+        attention.paged_attention_decode(*args)                          # (the device's workspace has its size)
+        both(counted, monkeypatch, lambda: attention.paged_attention_decode(*args), 1)
+    need = attention.decode_workspace_bytes(len(lengths), 8, 64, tables.shape[1], block)
+    own = torch.empty(need + 16, dtype=torch.uint8, device=DEV)
+    both(counted, monkeypatch, lambda: attention.paged_attention_decode(*args, workspace=own), 1)
+    # converted, or turned down
+    wide = normal(len(lengths), 8, 128, dtype=dtype)[..., :64]
+    both(counted, monkeypatch, lambda: attention.paged_attention_decode(wide, *args[1:]), 0)
+    both(counted, monkeypatch, lambda: attention.paged_attention_decode(*args[:3], tables.long(), *args[4:]), 0)
+    for wrong in ((q, k, v, tables, lens, 0.125, 8, 2, 64, block * 2), (q, k, v[:, :, :1], *args[3:]), (q, k.double(), *args[2:]),
+                  (q, k, v, tables, lens[:0], *args[5:]), (q, k, v, tables, lens, 0.125, 4, 2, 64, block)):
+        with pytest.raises(ValueError):
+            attention.paged_attention_decode(*wrong)
+    assert counted.taken == 0
+
+
+@pytest.mark.parametrize("lengths,block", [([5], 16), ([300, 1, 77], 32)])
+def test_decode_int8(counted, monkeypatch, lengths, block):
+    tables, (k, v), (ks, vs) = paged(lengths, block, 2, 128, None, int8=True)
+    args = (normal(len(lengths), 4, 128), k, v, ks, vs, tables, torch.tensor(lengths, device=DEV), 0.1, 4, 2, 128, block)
+    attention.paged_attention_decode_int8(*args)
+    both(counted, monkeypatch, lambda: attention.paged_attention_decode_int8(*args), 1)
+    for wrong in ((*args[:3], ks.half(), *args[4:]), (*args[:4], vs[:, :1], *args[5:]), (args[0], k.float(), *args[2:])):
+        with pytest.raises(ValueError):
+            attention.paged_attention_decode_int8(*wrong)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lengths", [[1], [40, 7], [900, 300]])
+def test_prefill_and_store(counted, monkeypatch, dtype, lengths):
+    rows, scale = sum(lengths), 0.125
+    q, k, v = normal(rows, 8, 64, dtype=dtype), normal(rows, 2, 64, dtype=dtype), normal(rows + 1, 2, 64, dtype=dtype)[1:]
+    cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    for most in (max(lengths), 10 ** 6, None):
+        both(counted, monkeypatch, lambda: attention.flash_attention_prefill(q, k, v, cu, scale, 8, 2, 64, max_seqlen=most), 1)
+    both(counted, monkeypatch, lambda: attention.flash_attention_prefill(q, k, v, cu.long(), scale, 8, 2, 64, max_seqlen=max(lengths)), 0)
+    both(counted, monkeypatch, lambda: attention.flash_attention_prefill(normal(rows, 2, 8, 64, dtype=dtype)[:, 0], k, v, cu, scale, 8, 2, 64),
+         int(rows == 1))                                                   # (one row is dense)
+    both(counted, monkeypatch, lambda: attention.flash_attention_prefill(q, k, v, cu, scale, 8, 2, 64, sink=torch.zeros(8, device=DEV)), 0)
+    for wrong in ((q, k[:-1], v, cu), (q, k, v.double(), cu), (q[:, :4], k, v, cu)):
+        with pytest.raises(ValueError):
+            attention.flash_attention_prefill(*wrong, scale, 8, 2, 64)
+
+    def stored(slots, key=k):
+        caches = [torch.zeros(rows // 16 + 2, 16, 2, 64, dtype=dtype, device=DEV) for _ in range(2)]
+        attention.store_kvcache(key, v, *caches, slots, 16)
+        return torch.cat(caches)
+
+    slots = torch.randperm(rows, generator=torch.Generator().manual_seed(1)).to(DEV)
+    slots[0] = -1
+    both(counted, monkeypatch, lambda: stored(slots), 1)
+    both(counted, monkeypatch, lambda: stored(slots.int()), 0)
+    both(counted, monkeypatch, lambda: stored(slots, normal(rows, 4, 64, dtype=dtype)[:, ::2]), 0)
+    with pytest.raises((ValueError, AssertionError)):
+        stored(slots[:-1])
+
+
+@pytest.mark.parametrize("dtype,lengths,cached", [(torch.bfloat16, [200, 90], [150, 0]), (torch.float32, [700, 40], [640, 20]), (torch.bfloat16, [3000] * 8, [0] * 8),
+                                                  (torch.float16, [9000], [5800])])                               # (its keys are split)
+def test_prefill_over_a_prefix(counted, monkeypatch, dtype, lengths, cached):
+    tables, (k, v), _ = paged(lengths, 16, 2, 64, dtype)
+    new = [n - c for n, c in zip(lengths, cached)]
+    cu = lambda x: torch.tensor([0, *torch.tensor(x).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    args = (normal(sum(new), 8, 64, dtype=dtype), k, v, tables, cu(new), cu(lengths), 0.125, 8, 2, 64, 16)
+    both(counted, monkeypatch, lambda: attention.flash_attention_prefill_paged(*args, max_seqlen_k=max(lengths)), int(max(lengths) < 5000))
+    both(counted, monkeypatch, lambda: attention.flash_attention_prefill_paged(*args), 0)
+    both(counted, monkeypatch, lambda: attention.flash_attention_prefill_paged(*args, max_seqlen_k=max(lengths), key_splits=2 * (dtype != torch.float32)), 0)
+    if max(lengths) == 700:                                                # no room for partial results
+        monkeypatch.setattr(attention, "STAGED_PREFILL_MAX_BYTES", 16)
+        both(counted, monkeypatch, lambda: attention.flash_attention_prefill_paged(*args, max_seqlen_k=max(lengths)), 0)
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_windows(counted, monkeypatch, shared):
+    rows = 150
+    q, k, v = normal(rows, 8, 96)[..., :64], normal(rows, 2, 64), normal(rows, 3, 64)[:, :2]
+    cu = torch.tensor([0, 70, rows], dtype=torch.int32, device=DEV)
+    options = dict(slopes=torch.rand(8, device=DEV), positions=torch.arange(rows, device=DEV), temperature=(0.1, 16), gate=normal(rows, 8, 64)) if shared \
+        else dict(v=v, gate=normal(rows, 8))
+
+    def run(*change, **more):
+        out = torch.zeros(rows, 8, 64, dtype=torch.bfloat16, device=DEV)
+        window_prefill(out, *(change or (q, k, cu, cu, 0.125, 33)), **{**options, **more})
+        return out
+
+    both(counted, monkeypatch, run, 1)
+    both(counted, monkeypatch, lambda: run(gate=None), 1)
+    for change, more in (((q, k, cu.long(), cu, 0.125, 33), {}), ((q, k, cu, cu[:2], 0.125, 33), {}), ((q[:, :, :32], k, cu, cu, 0.125, 33), {}),
+                         ((), dict(gate=normal(rows, 4))), ((), dict(slopes=torch.rand(7, device=DEV)))):
+        with pytest.raises(ValueError):
+            run(*change, **more)
+
+
+def test_subclasses_and_modes_go_the_longer_way(counted):
+    """What wants to see torch's operators, or is not a plain tensor, is left to them."""
+    class Mine(torch.Tensor):
+        pass
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names = getattr(self, "names", []) + [str(func)]
+            return func(*args, **(kwargs or {}))
+
+    q, k = normal(40, 8, 64), normal(40, 2, 64)
+    cu = torch.tensor([0, 40], dtype=torch.int32, device=DEV)
+    want = attention.flash_attention_prefill(q, k, k, cu, 0.125, 8, 2, 64)
+    assert counted.taken == 1
+    got = attention.flash_attention_prefill(q.as_subclass(Mine), k, k, cu, 0.125, 8, 2, 64)
+    assert type(got) is Mine and torch.equal(got.as_subclass(torch.Tensor), want)
+    with Seen() as seen:
+        assert torch.equal(attention.flash_attention_prefill(q, k, k, cu, 0.125, 8, 2, 64), want)
+    assert counted.taken == 1 and any("empty_like" in n for n in seen.names)
+    assert attention.flash_attention_prefill(torch.nn.Parameter(q), k, k, cu, 0.125, 8, 2, 64).requires_grad is False and counted.taken == 2
