@@ -142,9 +142,11 @@ struct PlanArgs {
   int32_t* sorted_pair;    // [pairs]: pair at a sorted place
   int32_t* place;          // [pairs]: sorted place of a pair
   int32_t* row_start;      // [E + 1]
-  int32_t* tile_expert;    // [max tiles]
-  int32_t* tile_row;       // [max tiles]: first sorted row
-  int32_t* num_tiles;      // [2] those in order, those behind them (see find_tile)
+  struct Tiles {
+    int32_t* expert;       // [max tiles]
+    int32_t* row;          // [max tiles]: first sorted row
+    int32_t* num;          // [2] those in order, those behind them (see find_tile)
+  } tiles[2];              // of tile_rows; and, where that is 128, of 256
   int pairs, experts, blocks, tile_rows;
 };
 
@@ -164,7 +166,8 @@ __global__ __launch_bounds__(256) void moe_count_kernel(const PlanArgs a) {
 // A chain of latencies, not bytes: the counts of the blocks, sums over the experts, places.  With the counts' loads one by one and the sums in ten rounds
 // with two barriers each 14 us at 49152 pairs of 64 experts, so 5.9; 1800 pairs 5.1 and 3.5.
 __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
-  __shared__ int32_t total[kMaxExperts + 1], tiles[kMaxExperts + 1], parts[kMaxExperts + 1], cursor[kMaxExperts], of_wave[3][16];
+  constexpr int kSums = 5;                          // rows; of either tiling the tiles in order and those behind them
+  __shared__ int32_t sum_to[kSums][kMaxExperts + 1], cursor[kMaxExperts], of_wave[kSums][16];
   const int e = threadIdx.x;
   int n = 0, mine = 0;
   if (a.blocks == 1) {                              // counted here
@@ -186,32 +189,33 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
     }
   }
   // inclusive sums over the experts: within a wave, then over the waves before it
-  const bool apart = a.tile_rows == 256 && n % 256 != 0 && n % 256 <= kApartRows && a.pairs >= kApartPairs;      // the last tile goes behind all others
-  int sums[3] = {n, (n + a.tile_rows - 1) / a.tile_rows - apart, apart};
+  const bool large = a.tile_rows == 256, both = a.tile_rows == 128;
+  const bool apart = (large || both) && n % 256 != 0 && n % 256 <= kApartRows && a.pairs >= kApartPairs;      // the last tile of 256 goes behind all others
+  int sums[kSums] = {n, (n + a.tile_rows - 1) / a.tile_rows - (large && apart), large && apart, both ? (n + 255) / 256 - apart : 0, both && apart};
   const int lane = e & 63, wave = __builtin_amdgcn_readfirstlane(e >> 6);
   const bool some = 64 * wave < a.experts;
   if (some) {
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1)
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
+      for (int i = 0; i < kSums; ++i) {
         const int before = __shfl_up(sums[i], o, 64);
         sums[i] += lane >= o ? before : 0;
       }
     if (lane == 63)
-      for (int i = 0; i < 3; ++i) of_wave[i][wave] = sums[i];
+      for (int i = 0; i < kSums; ++i) of_wave[i][wave] = sums[i];
   }
   __syncthreads();
   if (some) {
     for (int w = 0; w < wave; ++w)
 #pragma unroll
-      for (int i = 0; i < 3; ++i) sums[i] += of_wave[i][w];
-    total[e + 1] = sums[0];
-    tiles[e + 1] = sums[1];
-    parts[e + 1] = sums[2];
+      for (int i = 0; i < kSums; ++i) sums[i] += of_wave[i][w];
+#pragma unroll
+    for (int i = 0; i < kSums; ++i) sum_to[i][e + 1] = sums[i];
   }
-  if (e == 0) total[0] = tiles[0] = parts[0] = 0;
+  if (e < kSums) sum_to[e][0] = 0;
   __syncthreads();
+  const int32_t* total = sum_to[0];
   if (e < a.experts) cursor[e] = total[e] + mine;
   __syncthreads();
   const int end = min((int)(blockIdx.x + 1) * kPlanPairs, a.pairs);
@@ -227,19 +231,24 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
   }
   if (blockIdx.x == 0 && e < a.experts) {
     a.row_start[e] = total[e];
-    if (e == a.experts - 1) {
-      a.row_start[e + 1] = total[e + 1];
-      a.num_tiles[0] = tiles[e + 1];
-      a.num_tiles[1] = parts[e + 1];
-    }
-    for (int t = tiles[e]; t < tiles[e + 1]; ++t) {
-      a.tile_expert[t] = e;
-      a.tile_row[t] = total[e] + (t - tiles[e]) * a.tile_rows;
-    }
-    if (apart) {
-      const int t = tiles[a.experts] + parts[e];
-      a.tile_expert[t] = e;
-      a.tile_row[t] = total[e + 1] - n % 256;
+    if (e == a.experts - 1) a.row_start[e + 1] = total[e + 1];
+    for (int i = 0; i < 1 + both; ++i) {
+      const PlanArgs::Tiles& t = a.tiles[i];
+      const int32_t *tiles = sum_to[1 + 2 * i], *parts = sum_to[2 + 2 * i];
+      const int rows = i == 0 ? a.tile_rows : 256;
+      if (e == a.experts - 1) {
+        t.num[0] = tiles[e + 1];
+        t.num[1] = parts[e + 1];
+      }
+      for (int k = tiles[e]; k < tiles[e + 1]; ++k) {
+        t.expert[k] = e;
+        t.row[k] = total[e] + (k - tiles[e]) * rows;
+      }
+      if (parts[e + 1] > parts[e]) {
+        const int k = tiles[a.experts] + parts[e];
+        t.expert[k] = e;
+        t.row[k] = total[e + 1] - n % 256;
+      }
     }
   }
 }
@@ -746,7 +755,18 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
 static int tile_rows(int64_t pairs, int experts) {
   return pairs >= kLargeTileRows * (int64_t)experts ? 256 : pairs > kSmallTileRows * (int64_t)experts ? 128 : 64;
 }
-static int64_t max_tiles(int64_t pairs, int experts) { return (pairs + tile_rows(pairs, experts) - 1) / tile_rows(pairs, experts) + experts; }
+static int64_t max_tiles(int64_t pairs, int experts, int rows) { return (pairs + rows - 1) / rows + experts; }
+// Whether a product of N outputs runs on the tiles of 256 rows of a plan that has both.  With 48 to 384 rows per expert a large tile has one to four of its
+// blocks of 64 rows; it reads every weight once for the expert's rows and half as much of LDS per flop, but has a CU to itself and 12 us of
+// start and end, so that few of them leave CUs idle or a short last round: they pay from two and a half rounds on, or one and a half of
+// longer ones, where N fills them.  us of both products as 128 and 256 rows, top 4 routed unevenly: 64 experts of 2560 x 4096 and 4096
+// x 1280, 80 rows each 510 / 470, 200 776 / 621; of 1536 x 2048, 56 146 / 144, 160 200 / 177; 128 of 1536 x 2048, 80 310 / 284;
+// but 32 of 1536 x 2048, 80 73 / 82, 64 of 2048 x 1024, 120 121 / 144, 64 of 640 x 1536, 120 59 / 73, 8 of 1536 x 2048, 160 41 / 65.
+static bool large_tiles_pay(int64_t pairs, int experts, int N) {
+  const int64_t wide = (N + 255) / 256, rows = pairs / 256 + experts / 2, tiles = wide * (rows > experts ? rows : experts);
+  if (8 * (256 * wide - N) > N) return false;
+  return tiles >= 640 || (tiles >= 384 && pairs >= 144 * (int64_t)experts);
+}
 static int plan_blocks(int64_t pairs) { return (int)((pairs + kPlanPairs - 1) / kPlanPairs); }
 
 }  // namespace mvllm
@@ -792,7 +812,9 @@ extern "C" int mvllm_moe_route_softmax(int32_t* ids, float* weights, const float
 
 extern "C" size_t mvllm_moe_plan_bytes(int64_t pairs, int experts) {
   if (pairs <= 0 || experts <= 0) return 0;
-  return (size_t)(2 * pairs + experts + 1 + 2 * max_tiles(pairs, experts) + 2 + (int64_t)plan_blocks(pairs) * experts + 4) * sizeof(int32_t);
+  const int rows = tile_rows(pairs, experts);
+  const int64_t tiles = 2 * max_tiles(pairs, experts, rows) + 2 + (rows == 128 ? 2 * max_tiles(pairs, experts, 256) + 2 : 0);
+  return (size_t)(2 * pairs + experts + 1 + tiles + (int64_t)plan_blocks(pairs) * experts + 4) * sizeof(int32_t);
 }
 
 // the parts of a plan, in order
@@ -802,12 +824,15 @@ static PlanArgs plan_parts_of(void* plan, const int32_t* ids, int64_t pairs, int
   a.place = reinterpret_cast<int32_t*>(plan);
   a.sorted_pair = a.place + pairs;
   a.row_start = a.sorted_pair + pairs;
-  a.tile_expert = a.row_start + experts + 1;
-  a.tile_row = a.tile_expert + max_tiles(pairs, experts);
-  a.num_tiles = a.tile_row + max_tiles(pairs, experts);
-  a.hist = a.num_tiles + 2;
   a.pairs = (int)pairs; a.experts = experts; a.blocks = plan_blocks(pairs);
   a.tile_rows = tile_rows(pairs, experts);
+  int32_t* at = a.row_start + experts + 1;
+  for (int i = 0; i < 2; ++i) {
+    const int64_t most = i == 0 ? max_tiles(pairs, experts, a.tile_rows) : a.tile_rows == 128 ? max_tiles(pairs, experts, 256) : 0;
+    a.tiles[i] = {at, at + most, at + 2 * most};
+    at += most > 0 ? 2 * most + 2 : 0;
+  }
+  a.hist = at;
   return a;
 }
 
@@ -859,12 +884,14 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
     return launch_status();
   }
   const PlanArgs p = plan_parts_of(plan, ids, pairs, experts);
-  a.sorted_pair = p.sorted_pair; a.row_start = p.row_start; a.tile_expert = p.tile_expert; a.tile_row = p.tile_row;
-  a.num_tiles = p.num_tiles;
+  a.sorted_pair = p.sorted_pair; a.row_start = p.row_start;
   if (dtype == MVLLM_BF16) {
-    a.max_tiles = (int)max_tiles(pairs, experts);
-    a.n_tiles = p.tile_rows == 256 ? (N + 255) / 256 : (N + 127) / 128;
-    if (p.tile_rows == 256 && out_row_stride % 8 != 0) return MVLLM_ERR_UNSUPPORTED;
+    const bool second = p.tile_rows == 128 && out_row_stride % 8 == 0 && large_tiles_pay(pairs, experts, N);
+    const int rows = second ? 256 : p.tile_rows;
+    a.tile_expert = p.tiles[second].expert; a.tile_row = p.tiles[second].row; a.num_tiles = p.tiles[second].num;
+    a.max_tiles = (int)max_tiles(pairs, experts, rows);
+    a.n_tiles = rows == 256 ? (N + 255) / 256 : (N + 127) / 128;
+    if (rows == 256 && out_row_stride % 8 != 0) return MVLLM_ERR_UNSUPPORTED;
     const int64_t x_rows = per_token ? (pairs + per_token - 1) / per_token : pairs, x_bytes = ((x_rows - 1) * x_row_stride + K) * 2;
     if (x_bytes >= (int64_t)1 << 32 || (int64_t)N * K * 2 >= (int64_t)1 << 31) return MVLLM_ERR_UNSUPPORTED;
     a.x_bytes = (uint32_t)x_bytes;
@@ -872,8 +899,8 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
     if (blocks > 0x7fffffff) return MVLLM_ERR_BAD_SHAPE;
     with_glu(glu, [&](auto G) {
       constexpr int kGlu = decltype(G)::value;
-      if (p.tile_rows == 256) moe_linear_large_kernel<kGlu><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
-      else if (p.tile_rows == 128) moe_linear_many_kernel<kGlu, 4><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      if (rows == 256) moe_linear_large_kernel<kGlu><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      else if (rows == 128) moe_linear_many_kernel<kGlu, 4><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
       else moe_linear_many_kernel<kGlu, 2><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
     });
   } else {

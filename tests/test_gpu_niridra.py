@@ -11,6 +11,7 @@ from minivllm_amd.engine import ragged
 from minivllm_amd.engine.hybrid_runner import HybridModelRunner
 from minivllm_amd.engine.ragged import ragged_step
 from minivllm_amd.engine.sequence import Sequence
+from minivllm_amd import _C
 from minivllm_amd.layers.experts import ExpertOutput, SparseExperts, interleave_gate_up, moe_linear, moe_plan, moe_route
 from minivllm_amd.layers.fused import stream_embed_norm, stream_norm
 from minivllm_amd.layers.latent import head_linear, latent_decode, latent_norm_store, latent_width
@@ -565,6 +566,40 @@ def test_moe_linear_walks_and_shares(counts, n, k, glu):
             z = torch.nn.functional.silu(gate) * up
         want[rows] = z.reshape(len(rows), out.shape[1])
     assert row_rel(out, want) < 1e-2
+
+
+@pytest.mark.parametrize("n,k", [(2560, 128), (2304, 64)])           # products on tiles of 256 rows, and (2304: 576 tiles) on those of 128
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("more", [0, 120])
+def test_moe_linear_both_tilings_of_a_plan(n, k, glu, more):
+    """Plans between small and large tiles have both: experts without rows, of every number of 64-row parts, past a large tile by a few rows (behind all
+    others from 8192 pairs on) and by more; an output whose rows are no multiple of 16 bytes stays on the smaller ones."""
+    counts = [0, 1, 63, 64, 65, 127, 128, 129, 192, 193, 255, 256, 257, 300, 320, 321] * 4
+    counts = [c + (more if i % 5 == 0 else 0) - (c > 200 and more == 0 and 100) for i, c in enumerate(counts)]
+    g, experts, pairs = gen(n + k), len(counts), sum(counts)
+    assert 48 * experts < pairs < 384 * experts and (pairs >= 8192)
+    ids = torch.cat([torch.full((c,), i) for i, c in enumerate(counts)])[torch.randperm(pairs, generator=g)].int().view(-1, 1)
+    x = torch.randn(pairs, k, generator=g).bfloat16()
+    w = (torch.randn(experts, n, k, generator=g) * k ** -0.5).bfloat16()
+    xd, wd, idd = x.to(DEV), w.to(DEV), ids.to(DEV)
+    plan = moe_plan(idd, experts)
+    place = plan.place.cpu().long()
+    out = moe_linear(xd, wd, idd, plan, 1, glu)
+    want = torch.empty(out.shape, dtype=torch.float64)
+    for e in range(experts):
+        rows = (ids.view(-1) == e).nonzero().view(-1)
+        z = x[rows].double() @ w[e].double().T
+        if glu:
+            gate, up = z.view(len(rows), n // 64, 2, 32).unbind(2)
+            z = torch.nn.functional.silu(gate) * up
+        want[rows] = z.reshape(len(rows), out.shape[1])
+    assert row_rel(out.cpu()[place], want) < 1e-2
+    stride = out.shape[1] + 4
+    odd = torch.full((pairs, stride), float("nan"), dtype=torch.bfloat16, device=DEV)
+    st = _C.load().mvllm_moe_linear(odd.data_ptr(), stride, xd.data_ptr(), k, wd.data_ptr(), idd.data_ptr(), plan.data.data_ptr(), pairs, experts, n, k, 1,
+                                    int(glu), 1, _C.current_stream_ptr(odd.device))
+    assert st == 0
+    assert row_rel(odd[:, :out.shape[1]].cpu()[place], want) < 1e-2 and torch.isnan(odd[:, out.shape[1]:]).all()
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
