@@ -140,6 +140,14 @@ constexpr int kSplitOnePartCtx = 512;
 // 4 of 300 8.6 / 8.0 / 8.9, of 600 9.9 / 8.9 / 9.4; 6 of 854-1455 (heads of 64; 192 tokens 10.5) 12.8 / 10.3 / 9.7; 8 of 1500-2000 21 / 17.0 / 14.3.
 // (In wider tables partition_tokens_for's least is about as long.)
 constexpr int kSplitNarrowCtx = 2048, kSplitOnePartPairs = 256;
+// Tables of kSplitFineCtx tokens and more that take a merge anyway: 4, 8 or 16 partitions, the fewest that give kSplitFineGroups workgroups and none
+// shorter than kSplitFinePart tokens.  A CU holds several workgroups, and sequences differ: with one round of long partitions the CUs that got the
+// longest sequences decide (24 sequences of 576-8566 INT8 tokens, 576 workgroups: CUs busy half the time).  us, one round / finer, 8 kv heads:
+// 23 of up to 4054 in full tables 66 / 52, 46 of 7549 203 / 173, 17 of 14057 182 / 137, 9 of 19713 heads of 64 116 / 84, INT8 26 of 17625 110 / 84, 43 of
+// 7784 heads of 64 108 / 64; all as long as the table 24 of 8191 164 / 142; contexts of a quarter of the table 24 of 4071 in 8192 74 / 52, of an
+// eighth 20.7 / 21.7; fp32, 45 of up to 6000 271 / 184.  Finer still costs even batches (partials, start-up): INT8, 20 of 4999 50 / 52 / 61 with 4 / 8 / 20 partitions.
+// A batch whose partitions are exactly kSplitMinGroups workgroups, an even round, keeps them: 16 of 8191 in 8192 85 / 86, heads of 64 49 / 54 (16 of 512 to 8094 57 / 37).
+constexpr int kSplitFineCtx = 2304, kSplitFineParts = 16, kSplitFinePart = 512, kSplitFineGroups = 1536;
 inline bool split_wanted(int64_t max_ctx, int batch, int num_kv_heads, bool int8) {
   const int part = partition_tokens_for(max_ctx, batch);
   const int64_t parts = (max_ctx + part - 1) / part;
@@ -170,7 +178,16 @@ inline int split_partition_tokens(int64_t max_ctx, int batch, int num_kv_heads, 
   if (max_ctx <= kSplitOnePartCtx || (sixteen_bit && split_one_part(max_ctx, pairs, head_dim, block_size))) part = (max_ctx + 63) / 64 * 64;
   if (part > kSplitMaxPart) part = kSplitMaxPart;
   const int64_t floor_part = partition_tokens_for(max_ctx, batch);
-  return (int)(part < floor_part ? floor_part : part);
+  part = part < floor_part ? floor_part : part;
+  const int64_t parts = (max_ctx + part - 1) / part;
+  if (max_ctx >= kSplitFineCtx && parts > 1 && pairs * parts != kSplitMinGroups)
+    for (int64_t n = 4; n <= kSplitFineParts; n *= 2) {
+      const int64_t finer = ((max_ctx + n - 1) / n + 63) / 64 * 64;
+      if (finer < kSplitFinePart) break;
+      if (finer < part && finer >= floor_part) part = finer;
+      if (n * pairs >= kSplitFineGroups) break;
+    }
+  return (int)part;
 }
 
 __device__ __forceinline__ int64_t load_ctx(const DecodeArgs& a, int b) {

@@ -282,6 +282,24 @@ def test_both_grid_forms_vs_oracle(dtype, hq, hkv, bs, d, form):
     assert torch.count_nonzero(got[3]) == 0
 
 
+@pytest.mark.parametrize("batch,first,tokens,d,dtype,plan", [
+    (24, [8192, 1024, 1025, 1], 8192, 128, torch.bfloat16, (1024, 8, 4)), (9, [4160, 512, 575, 513], 4160, 64, torch.float16, (576, 8, 4)),   # finer
+    (31, [2304, 576, 577], 2304, 128, torch.bfloat16, (576, 4, 4)), (31, [2288, 763, 705], 2288, 128, torch.bfloat16, (768, 3, 4)),   # from 2304 tokens on
+    (33, [8200, 4100, 2112, 2113], 8208, 128, torch.bfloat16, (1088, 8, 4)), (49, [4096, 17, 1024], 4096, 64, torch.float32, (1024, 4, 4)),
+    (16, [8192, 2048, 2049], 8192, 64, torch.bfloat16, (2048, 4, 4)),                                                     # an even round stays
+])
+def test_partitions_of_wide_tables(batch, first, tokens, d, dtype, plan):
+    hq, hkv, bs = 16, 8, 16
+    case = make_paged_case(43, batch, 1, 1, hq, hkv, d, bs, dtype=dtype, ctx_list=first + [17 + 9 * i for i in range(batch - len(first))])
+    q, kc, vc, tables, ctx = case
+    tables = torch.nn.functional.pad(tables, (0, tokens // bs - tables.shape[1]), value=-1)
+    assert paged_decode_plan(batch, hq, hkv, d, tables.shape[1], bs, dtype) == plan
+    scale = 1 / math.sqrt(d)
+    got = _run(q, kc, vc, tables, ctx, scale, hq, hkv, d, bs)
+    mx, mean = error_stats(got, _oracle32(*case, scale, hq, hkv, d, bs))
+    assert mx <= (MAX_ABS_32 if dtype == torch.float32 else MAX_ABS_16) and mean <= MEAN_ABS_16, (mx, mean)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,bs,d", [(16, 8, 16, 256), (8, 1, 32, 256), (5, 5, 48, 256), (16, 8, 16, 32), (12, 2, 256, 32),
                                          (32, 8, 16, 96), (6, 6, 48, 96), (12, 1, 256, 96), (32, 8, 16, 80), (5, 5, 48, 112),
