@@ -83,6 +83,7 @@ template <typename T> __device__ __forceinline__ uint4 dequant8_biased(uint32_t 
 // a sequence's tiles costs such prompts nothing.
 // Every lane of the calling wave must be active; all lanes return the same values.
 constexpr int kBandRows = 256;          // rows per band of the heaviest-first item order (a multiple of 128)
+constexpr int kBandLevelsWalked = 8;    // levels among which the item's is found one by one
 constexpr int kShortPromptRows = 192;   // mean rows per sequence up to which bands are single tiles
 // log2 of the row tiles per band for a batch of these static sizes (bm: rows per workgroup, a power of two <= kBandRows)
 // (packed: the rows are also the keys.  Over a cached prefix few rows may stand behind many keys, which the tiles of a
@@ -112,21 +113,40 @@ __device__ __forceinline__ bool locate_banded(const int32_t* __restrict__ cu, in
     const int trial = top | (1 << bit);
     if (__ballot(nb >= trial) != 0ull) top = trial;
   }
-  // walk the levels down from the top one until the item's level is found
-  unsigned base = 0;
-  int b = top - 1;
+  // The item's level, the highest with more items there and above than the item's number: walked down from the top where there are few levels, else
+  // bit by bit too, by sums over the sequences (a sum costs as much as two steps; two prompts of 7600 tokens, 30 levels, in windows of 512:
+  // 122 us walked, 117 so; 16 prompts of 248, one level: 22.2, 22.4).
+  const unsigned unit = (unsigned)heads_y << band_shift;
   unsigned long long mask = 0ull;
-  unsigned per_y = 0;
-  for (; b >= 0; --b) {
+  unsigned count = 0, base = 0;
+  int b = top - 1;
+  if (top > kBandLevelsWalked) {
+    auto bands_from = [&](int at) __attribute__((always_inline)) { return (unsigned)__builtin_amdgcn_readlane(wave_prefix_sum(max(nb - at, 0)), 63); };
+    unsigned bands = bands_from(0);
+    if (item >= bands * unit) return false;     // past the last item: grid padding
+    b = 0;
+    for (int bit = 31 - __builtin_clz((unsigned)top); bit >= 0; --bit) {
+      const unsigned above = bands_from(b | (1 << bit));
+      if (item < above * unit) {
+        b |= 1 << bit;
+        bands = above;
+      }
+    }
     mask = __ballot(nb > b);
-    per_y = (unsigned)__popcll(mask) << band_shift;
-    const unsigned items = per_y * (unsigned)heads_y;
-    if (item - base < items) break;
-    base += items;
+    count = (unsigned)__popcll(mask);
+    base = (bands - count) * unit;
+  } else {
+    for (; b >= 0; --b) {
+      mask = __ballot(nb > b);
+      count = (unsigned)__popcll(mask);
+      if (item - base < count * unit) break;
+      base += count * unit;
+    }
+    if (b < 0) return false;                    // past the last item: grid padding
   }
-  if (b < 0) return false;                      // past the last item: grid padding
+  const unsigned per_y = count << band_shift;
   const unsigned idx = item - base;
-  item_y = (int)(idx / per_y);
+  item_y = (count & (count - 1)) == 0 ? (int)(idx >> __builtin_ctz(per_y)) : (int)(idx / per_y);
   const unsigned rem = idx - (unsigned)item_y * per_y;
   const int q = (int)(rem >> band_shift), r = (int)(rem & (unsigned)(R - 1));
   // the q-th sequence of this level = the lane whose bit is set with q set bits below it
@@ -134,9 +154,9 @@ __device__ __forceinline__ bool locate_banded(const int32_t* __restrict__ cu, in
   const unsigned long long pick = __ballot(((mask >> lane) & 1ull) != 0ull && below == q);
   const int owner = __ffsll((long long)pick) - 1;
   const int t = (b << band_shift) + (R - 1 - r);   // row tile inside the sequence, last tile of the band first
-  if (t >= __shfl(n, owner, 64)) return false;  // the band's padding
-  seq_start = __shfl(lo, owner, 64);
-  seq_len = __shfl(len, owner, 64);
+  if (t >= __builtin_amdgcn_readlane(n, owner)) return false;  // the band's padding
+  seq_start = __builtin_amdgcn_readlane(lo, owner);
+  seq_len = __builtin_amdgcn_readlane(len, owner);
   row0 = t * BM;
   seq_index = owner;
   return true;
@@ -195,7 +215,11 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   // a long sequence over all XCDs instead of always handing them to the same one
   const unsigned round = slot / kXcdChunk;
   const unsigned item = (round * 8 + ((xcd + round) & 7)) * kXcdChunk + slot % kXcdChunk;
-  int item_y, seq_start, seq_len, row0, seq_index;
+  int item_y, seq_start, seq_len, row0, seq_index, keys = 0;
+  if constexpr (PAGED) {                             // every lane a sequence's keys, on their way together with its rows
+    const int s = threadIdx.x & 63;
+    if (s < a.num_seqs && a.num_seqs <= 64) keys = a.cu_seqlens_k[s + 1] - a.cu_seqlens_k[s];
+  }
   if constexpr (RANGES) {
     // slices fastest: with a multiple of eight of them all that reads the keys of one is on one XCD; nothing is padded, which would
     // count once per range (in the other order 195 rows behind 3700 keys in 11 ranges took 92 us, 4000 workgroups without work among them;
@@ -220,7 +244,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   seq_index = __builtin_amdgcn_readfirstlane(seq_index);
   // Keys of the sequence: its own rows, or in paged mode the cached prefix plus them (query row r sits at
   // position cached + r and sees keys 0 .. cached + r).
-  const int kv_len = PAGED ? a.cu_seqlens_k[seq_index + 1] - a.cu_seqlens_k[seq_index] : seq_len;
+  const int kv_len = !PAGED ? seq_len : a.num_seqs <= 64 ? __builtin_amdgcn_readlane(keys, seq_index) : a.cu_seqlens_k[seq_index + 1] - a.cu_seqlens_k[seq_index];
   const int cached = !PAGED ? 0 : a.q_pos != nullptr ? a.q_pos[seq_index] : max(kv_len - seq_len, 0);
   if (PAGED && a.q_pos != nullptr && kv_len <= 0) return;   // a key range that is empty (uniform over the workgroup)
 

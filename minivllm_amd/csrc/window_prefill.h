@@ -91,23 +91,31 @@ __global__ __launch_bounds__(256, KS1 > 8 ? 1 : 2) void window_prefill_kernel(co
   const unsigned id = blockIdx.x, slot = id >> 3, xcd = id & 7, round = slot / kXcdChunk;
   const unsigned item = (round * 8 + ((xcd + round) & 7)) * kXcdChunk + slot % kXcdChunk;
   const int BM = kWinRows * (4 / a.hpw);
-  int seq_start, seq_len, row0, seq, item_y;
+  int seq_start, seq_len, row0, seq, item_y, k_lo = 0, k_hi = 0;
   if (a.num_seqs <= 64) {
+    const int s = threadIdx.x & 63;                  // every lane a sequence's keys, on their way together with its rows
+    if (s < a.num_seqs) {
+      k_lo = a.cu_k[s];
+      k_hi = a.cu_k[s + 1];
+    }
     const bool found = a.hpw == 4 ? locate_banded<kWinRows>(a.cu_q, a.num_seqs, item, a.heads_y, a.band_bits, a.band_shift, seq_start, seq_len, row0, seq, item_y)
                      : a.hpw == 2 ? locate_banded<2 * kWinRows>(a.cu_q, a.num_seqs, item, a.heads_y, a.band_bits, a.band_shift, seq_start, seq_len, row0, seq, item_y)
                                   : locate_banded<4 * kWinRows>(a.cu_q, a.num_seqs, item, a.heads_y, a.band_bits, a.band_shift, seq_start, seq_len, row0, seq, item_y);
     if (!found) return;
+    k_lo = __builtin_amdgcn_readlane(k_lo, seq);
+    k_hi = __builtin_amdgcn_readlane(k_hi, seq);
   } else {
     if (item >= (unsigned)a.tiles_x * (unsigned)a.heads_y) return;
     item_y = (int)(item / (unsigned)a.tiles_x);
     if (!locate_tile(a.cu_q, a.num_seqs, a.tiles_x - 1 - (int)(item % (unsigned)a.tiles_x), BM, seq_start, seq_len, row0, seq)) return;
+    k_lo = a.cu_k[seq];
+    k_hi = a.cu_k[seq + 1];
   }
   item_y = __builtin_amdgcn_readfirstlane(item_y);
   seq_start = __builtin_amdgcn_readfirstlane(seq_start);
   seq_len = __builtin_amdgcn_readfirstlane(seq_len);
   row0 = __builtin_amdgcn_readfirstlane(row0);
-  seq = __builtin_amdgcn_readfirstlane(seq);
-  const int k_start = a.cu_k[seq], kv_len = a.cu_k[seq + 1] - k_start, cached = kv_len - seq_len;
+  const int k_start = __builtin_amdgcn_readfirstlane(k_lo), kv_len = __builtin_amdgcn_readfirstlane(k_hi) - k_start, cached = kv_len - seq_len;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
   const int group = a.heads / a.kv_heads, slices = group / a.hpw;

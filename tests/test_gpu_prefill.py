@@ -184,6 +184,31 @@ def test_prefill_item_order_covers_every_tile(hq, hkv, num_seqs):
     assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
 
 
+@pytest.mark.parametrize("by_ranges", [False, True])                # heaviest-first bands, or prefix sums over the sequences' tiles
+@pytest.mark.parametrize("num_seqs", [1, 2, 3, 15, 16, 17, 31, 32, 33, 47, 63, 64])
+def test_prefill_finds_rows_at_every_count_of_sequences(num_seqs, by_ranges):
+    """Counts beside the sixteen lanes that a prefix sum takes at a time, equal and ragged lengths, empty ones among them and a last one that
+    ends the batch: the rows a workgroup takes come from sums over the lanes, so a wrong step leaves rows untouched or doubled."""
+    hq, hkv, d = 4, 2, 64
+    lengths = [(0, 1, 64, 65, 33, 129, 64)[i % 7] if num_seqs % 2 else 65 for i in range(num_seqs)]
+    lengths[num_seqs // 2], lengths[-1] = 300, 513
+    q, k, v, cu = make_varlen_case(59 + num_seqs, lengths, hq, hkv, d, dtype=torch.bfloat16)
+    scale = 1 / math.sqrt(d)
+    from minivllm_amd import _C
+    out = torch.full_like(q, float("nan")).to(DEV)
+    qd, kd, vd, cud = (t.to(DEV) for t in (q, k, v, cu))
+    head = (out.data_ptr(), qd.data_ptr(), kd.data_ptr(), vd.data_ptr())
+    code, stream = _C.dtype_code(q.dtype), _C.current_stream_ptr(out.device)
+    if by_ranges:                                                   # one range: no workspace
+        st = _C.load().mvllm_prefill_ranges(*head, 0, 0, cud.data_ptr(), 0, num_seqs, q.shape[0], 513, hq, hkv, d, 0, 0, scale, 0, code, 10, 0, 0, stream)
+    else:
+        st = _C.load().mvllm_prefill_varlen(*head, cud.data_ptr(), num_seqs, q.shape[0], hq, hkv, d, scale, code, stream)
+    torch.cuda.synchronize()
+    assert st == 0
+    mx, mean = error_stats(out.cpu(), _oracle32(q, k, v, cu, scale, hq, hkv, d))
+    assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
+
+
 @pytest.mark.parametrize("hq,hkv,dtype", [(32, 8, torch.bfloat16), (64, 8, torch.bfloat16), (24, 2, torch.bfloat16),
                                           (8, 2, torch.bfloat16), (12, 3, torch.bfloat16), (4, 1, torch.bfloat16),
                                           (16, 8, torch.bfloat16), (16, 8, torch.float16), (12, 2, torch.bfloat16),
