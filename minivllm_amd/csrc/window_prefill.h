@@ -348,22 +348,42 @@ __global__ __launch_bounds__(256, KS1 > 8 ? 1 : 2) void window_prefill_kernel(co
     });
   };
 
-  int buffer = 0;
-  for (int j = wg_first; j <= wg_last; ++j, buffer ^= 1) {
+  // The wave's tiles in runs of one kind, a loop each: others' tiles, tiles that the window's first key may cross, whole ones, tiles that the causal limit
+  // may cross, others'.  In one loop with a branch for each kind the compiler gave the accumulators a set of registers on either path, and every
+  // tile moved all of them twice (64 double moves among 200 vector instructions at 128 dims).  us so / in runs: 9000 rows, windows of 2048, 32 heads of
+  // 128 238 / 222, of 64 140 / 126, values that are the keys 231 / 205 and 146 / 128, 16 heads of 256 350 / 282, 192 267 / 225; in
+  // windows of 256 79 / 77, 49 / 42, 77 / 66, 50 / 44, 127 / 111, 92 / 85.
+  // (The large heads take every tile as one that may be crossed: one copy of the step, whose registers then stay put.)
+  const int end = active ? j_last + 1 : wg_first;
+  const int first = active ? j_first : wg_first;
+  const int whole_from = KS1 > 8 ? end : min(max(first, pos0 + kWinRows - 1 - W < 0 ? 0 : (pos0 + kWinRows - 1 - W) / kWinKeys + 1), end);
+  const int whole_end = max(whole_from, min((pos0 + 1) / kWinKeys, end));
+  int j = wg_first;
+  auto arrived = [&]() __attribute__((always_inline)) {
     dma_wait_all();
     __syncthreads();                                 // tile j is there; nobody reads the other buffer any more
-    const bool more = j < wg_last;
-    if (!active || j < j_first || j > j_last) {      // other waves' tile: this wave's share of the next copy only
-      if (more) {
-        const Source s = source(j + 1, true);
-        static_for<kCopies>([&](auto C) { copy(s, C, buffer ^ 1); });
-      }
-      continue;
+  };
+  auto others_until = [&](int until) __attribute__((always_inline)) {      // this wave's share of the next copy only
+    for (; j < until; ++j) {
+      arrived();
+      if (j == wg_last) continue;
+      const Source s = source(j + 1, true);
+      static_for<kCopies>([&](auto C) { copy(s, C, ((j - wg_first) & 1) ^ 1); });
     }
-    const bool whole = j * kWinKeys > pos0 + kWinRows - 1 - W && j * kWinKeys + kWinKeys - 1 <= pos0;
-    if (KS1 <= 8 && whole) tile_step(j, std::false_type{}, buffer, more);
-    else tile_step(j, std::true_type{}, buffer, more);      // (the large heads: one copy of the step, whose registers then stay put)
+  };
+  auto tiles_until = [&](int until, auto MASKED) __attribute__((always_inline)) {
+    for (; j < until; ++j) {
+      arrived();
+      tile_step(j, MASKED, (j - wg_first) & 1, j < wg_last);
+    }
+  };
+  others_until(first);
+  tiles_until(whole_from, std::true_type{});
+  if constexpr (KS1 <= 8) {
+    tiles_until(whole_end, std::false_type{});
+    tiles_until(end, std::true_type{});
   }
+  others_until(wg_last + 1);
 
   // ---- normalise, turn through LDS, store whole rows ----
   dma_wait_all();

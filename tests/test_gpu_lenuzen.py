@@ -229,6 +229,23 @@ def test_window_prefill_of_keys_and_values(dtype, window, heads, groups, dim):
             assert rel(out[a], want) < tol(dtype, 3e-6, 1.5e-2), e
 
 
+@pytest.mark.parametrize("dim,heads", [(64, 4), (128, 2), (256, 1)])
+@pytest.mark.parametrize("window", [32, 33, 63, 65, 94, 95, 96, 97, 127, 128, 129, 159, 160, 192, 193])
+def test_window_prefill_tiles_in_runs(window, dim, heads):
+    """A wave walks its 64-key tiles in runs (those the window's first key crosses, whole ones, those the causal limit crosses), any of
+    which may be empty, and passes those that only other waves of its workgroup need: windows beside multiples of 32, pasts and
+    lengths beside the tiles' borders, one to four query heads, so four to one row tiles, of a workgroup."""
+    dtype, g, lens, pasts = torch.bfloat16, gen(3 * dim + window), [1, 32, 63, 65, 129, 300], [64, 0, 1, 95, 33, 31]
+    rows, keys = sum(lens), sum(lens) + sum(pasts)
+    q, k, v = rand(g, rows, heads, dim, dtype=dtype, scale=2.0), rand(g, keys, 1, dim, dtype=dtype), rand(g, keys, 1, dim, dtype=dtype)
+    cu_q, cu_k = prefix_sums(lens), prefix_sums([a + b for a, b in zip(lens, pasts)])
+    out = torch.full((rows, heads, dim), float("nan"), dtype=dtype, device=DEV)
+    window_prefill(out, on(q), on(k), on(cu_q), on(cu_k), dim ** -0.5, window, v=on(v))
+    for e in range(len(lens)):
+        a, b = slice(int(cu_q[e]), int(cu_q[e + 1])), slice(int(cu_k[e]), int(cu_k[e + 1]))
+        assert rel(out[a], window_reference(q[a], k[b], v[b], dim ** -0.5, window)) < 1.5e-2, e
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("window", [5, 64, 97])
 def test_window_edges_in_prompts(dtype, window):
