@@ -55,6 +55,8 @@ constexpr unsigned kXcdChunk = 32;      // consecutive work items handed to one 
 constexpr int kPfWaves = 4;             // waves per workgroup: 4, so that two workgroups share a CU
 constexpr int kBN = 64;                 // K/V rows per LDS tile
 constexpr int kWaveRows = 32;           // query rows per wave
+template <int N> struct TileBuffer { static constexpr int value = N; static constexpr uint32_t at = 0; };   // one of a tile's two buffers, ...
+struct EitherBuffer { static constexpr int value = -1; uint32_t at; };                                       // ... or known at run time, by its offset
 
 // Eight int8 codes (two dwords, biased by +128 so that the unsigned byte conversions apply) times one scale, rounded
 // once to the element type: fma(u, scale, -128 scale) is the exactly rounded (u - 128) * scale = code * scale.
@@ -371,8 +373,8 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
     constexpr int c = decltype(C)::value;
     constexpr bool is_k = c < kCopies;
     constexpr int i = is_k ? c : c - kCopies;
-    constexpr int imm = (is_k ? 0 : 2 * kTileBytes) + decltype(BUF)::value * kTileBytes + i * 1024;
-    dma16_to_lds<imm>(is_k ? t.k : t.v, is_k ? k_src_off[i] : v_src_off[i], lds_wave_base);
+    constexpr int buf = decltype(BUF)::value, imm = (is_k ? 0 : 2 * kTileBytes) + (buf > 0 ? kTileBytes : 0) + i * 1024;
+    dma16_to_lds<imm>(is_k ? t.k : t.v, is_k ? k_src_off[i] : v_src_off[i], lds_wave_base + BUF.at);
   };
   auto issue_tile = [&](int j, int buf) {                        // whole tile at once, buffer chosen at run time
     const TileSrc t = tile_src(j, true);
@@ -492,7 +494,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   auto v_off = [&](int td) __attribute__((always_inline)) { return v_off_[td & 3] + (td >> 2) * 256; };
 
   // One K/V tile: scores, softmax, P.V.  Compile-time parameters: BUF, the buffer index (so that all LDS
-  // addresses are register + constant); DIAG, set for the wave's last tile, the one the causal diagonal runs
+  // addresses are register + constant) or EitherBuffer; DIAG, set for the wave's last tile, the one the causal diagonal runs
   // through (the only one that is masked); NH, the number of 32-row halves of the tile that are computed at
   // all: 1 when the wave's rows are the upper half of the 64-row block, so that the diagonal tile's second
   // half is masked entirely.
@@ -500,7 +502,10 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
     constexpr int buf = decltype(BUF)::value;
     constexpr bool diag = decltype(DIAG)::value;
     constexpr int NH = decltype(NHALF)::value;
-    using NEXT_BUF = std::integral_constant<int, buf ^ 1>;
+    const auto next_buf = [&]() __attribute__((always_inline)) {
+      if constexpr (buf < 0) return EitherBuffer{(uint32_t)kTileBytes - BUF.at};
+      else return TileBuffer<buf ^ 1>{};
+    }();
     TileSrc next;
     if constexpr (!I8) next = tile_src(j + 1, prefetch);      // INT8: the codes of the next tile are already on their way
 
@@ -508,7 +513,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
     // The two 32-row halves of the tile form two independent accumulator chains that are issued
     // alternately, so no MFMA waits for the result of the one before it.
     v16f s[NH];
-    const char* kb = &lds.k[buf][0];
+    const char* kb = &lds.k[buf < 0 ? 0 : buf][0] + BUF.at;
     {
       // K fragments are read one step ahead of the MFMAs that use them.  The reads of step ks + 1 stand in front
       // of step ks's copy instruction on purpose: the copy is an asm statement, which no LDS read is moved
@@ -531,7 +536,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
           }
 #pragma unroll
           for (int tk = 0; tk < NH; ++tk) s[tk] = mfma32x32x16<T>(kf[ks % 3][tk], qf[ks], ks == 0 ? neg_m : s[tk]);
-          if constexpr (!I8 && ks < 2 * kCopies) issue_copy(next, NEXT_BUF{}, KS);
+          if constexpr (!I8 && ks < 2 * kCopies) issue_copy(next, next_buf, KS);
         });
       } else {
         uint4 kf[2][NH];
@@ -547,15 +552,15 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
           }
 #pragma unroll
           for (int tk = 0; tk < NH; ++tk) s[tk] = mfma32x32x16<T>(kf[ks & 1][tk], qf[ks], ks == 0 ? neg_m : s[tk]);
-          if constexpr (!I8 && ks < 2 * kCopies) issue_copy(next, NEXT_BUF{}, KS);    // copies of the next tile, K first
+          if constexpr (!I8 && ks < 2 * kCopies) issue_copy(next, next_buf, KS);    // copies of the next tile, K first
         });
       }
       // fewer steps than copy instructions (head dims below the layout's): the rest of the copies follow here
       if constexpr (!I8 && kKS < 2 * kCopies)
-        static_for<2 * kCopies - kKS>([&](auto C) { issue_copy(next, NEXT_BUF{}, std::integral_constant<int, kKS + decltype(C)::value>{}); });
+        static_for<2 * kCopies - kKS>([&](auto C) { issue_copy(next, next_buf, std::integral_constant<int, kKS + decltype(C)::value>{}); });
     }
     // head_dim 256: the V^T fragments of the tile's first 16 keys set out now and arrive during the softmax
-    const char* vb = &lds.v[buf][0];
+    const char* vb = &lds.v[buf < 0 ? 0 : buf][0] + BUF.at;
     auto v_frags = [&](int step, uint4 (&af)[kTD]) __attribute__((always_inline)) {
 #pragma unroll
       for (int td = 0; td < kTD; ++td) {
@@ -689,8 +694,8 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   // Tile j lives in buffer j % 2.  The main loop is unrolled by two so that the buffer index is a compile-time
   // constant inside tile_step.  A wave's tiles are n_full complete ones and then those the causal diagonal runs
   // through: one when the rows start at a multiple of 32 keys (always, without a cached prefix), else up to two.
-  using B0 = std::integral_constant<int, 0>;
-  using B1 = std::integral_constant<int, 1>;
+  using B0 = TileBuffer<0>;
+  using B1 = TileBuffer<1>;
   using H1 = std::integral_constant<int, 1>;
   using H2 = std::integral_constant<int, 2>;
   auto full_step = [&](int j, auto BUF) {
@@ -698,12 +703,15 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
     __syncthreads();                   // ... and everybody else's; tile j-1 is no longer read
     tile_step(j, BUF, std::false_type{}, H2{}, j + 1 < ntiles);
   };
-  auto diag_step = [&](int j, auto BUF) {
+  // Of the last tile the second 32 keys are skipped where no row of the wave reaches them.  The diagonal's tiles are a loop of whole ones and a half one
+  // behind it, of either buffer.  As one loop with four copies of the step, for the half and the buffer, the compiler moved all accumulators twice per
+  // tile and kept 17 to 26 registers of the kernels of 128 dims in memory, and short calls waited for twice the code: us so / now, 16 heads of 128 over
+  // 8, 13 prompts of up to 104 tokens behind as many 13.8 / 12.7, 8 of 433 23.2 / 20.9, 7 of 240 15.1 / 13.8; 32 heads, 8 of 77 11.8 / 10.4.
+  const int whole_end = j_last + (pos0 + kWaveRows - 1 < j_last * kBN + 32 ? 0 : 1);
+  auto diag_step = [&](int j, auto NHALF) {
     dma_wait_all();
     __syncthreads();
-    // no row of the wave reaches the second 32 keys of the tile: skip that half
-    if (pos0 + kWaveRows - 1 < j * kBN + 32) tile_step(j, BUF, std::true_type{}, H1{}, j + 1 < ntiles);
-    else tile_step(j, BUF, std::true_type{}, H2{}, j + 1 < ntiles);
+    tile_step(j, EitherBuffer{(uint32_t)(j & 1) * kTileBytes}, std::true_type{}, NHALF, j + 1 < ntiles);
   };
   int j = t0;
   if constexpr (I8) {
@@ -721,10 +729,14 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
         stage(j);
         tile_step(j, B0{}, std::false_type{}, H2{}, false);
       }
-      for (; j <= j_last; ++j) {
+      for (; j < whole_end; ++j) {
         stage(j);
-        if (pos0 + kWaveRows - 1 < j * kBN + 32) tile_step(j, B0{}, std::true_type{}, H1{}, false);
-        else tile_step(j, B0{}, std::true_type{}, H2{}, false);
+        tile_step(j, B0{}, std::true_type{}, H2{}, false);
+      }
+      if (j <= j_last) {
+        stage(j);
+        tile_step(j, B0{}, std::true_type{}, H1{}, false);
+        ++j;
       }
     }
     for (; j < ntiles; ++j) stage(j);
@@ -738,9 +750,10 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
       full_step(j, B0{});
       ++j;
     }
-    for (; j <= j_last; ++j) {
-      if (j & 1) diag_step(j, B1{});
-      else diag_step(j, B0{});
+    for (; j < whole_end; ++j) diag_step(j, H2{});
+    if (j <= j_last) {
+      diag_step(j, H1{});
+      ++j;
     }
   }
   // Tiles that only other waves of the workgroup still compute on (their rows are further down): keep copying

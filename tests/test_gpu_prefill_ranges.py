@@ -49,6 +49,21 @@ def test_prefill_over_key_ranges(hq, hkv, d, bs, lengths, cached, tiles, paged, 
         assert torch.isfinite(got.float()).all() and mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (bound, mx, mean)
 
 
+@pytest.mark.parametrize("new", [1, 31, 32, 33, 65, 100])
+@pytest.mark.parametrize("hq,hkv,d,tiles", [(8, 2, 128, 4), (4, 2, 64, 2), (3, 3, 128, 4)])
+def test_the_diagonal_at_every_place_of_a_tile(hq, hkv, d, tiles, new):
+    """A wave's last tiles, one or two with the causal limit in them, the last of them whole or its first half: in the first or the second of the
+    two buffers, first tile of a range or not, behind prefixes beside every multiple of 32 up to three tiles."""
+    cached = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 192]
+    c = make_paged_prefill_case(83 + new, [n + new for n in cached], cached, hq, hkv, d, 16, dtype=torch.bfloat16)
+    want = oracle.prefill_paged_oracle(c["q_new"].float(), torch.nan_to_num(c["k_cache"].float()), torch.nan_to_num(c["v_cache"].float()),
+                                       c["block_tables"], c["cu_q"], c["cu_k"], 1 / math.sqrt(d), hq, hkv, d, 16)
+    for paged in (True, False):
+        got = _run(c, hq, hkv, d, 16, tiles, max(cached) + new, paged)
+        mx, mean = error_stats(got if paged else got[c["new_rows"]], want)
+        assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (paged, mx, mean)
+
+
 @pytest.mark.parametrize("lengths", [[0, 300, 0, 77], [200]])
 def test_prefill_over_key_ranges_sinks_and_empty_sequences(lengths):
     """Against the kernel without ranges: the sink counts once, sequences without tokens have no rows."""
