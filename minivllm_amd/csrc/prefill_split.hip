@@ -449,17 +449,20 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
 // The range for a batch of these sizes, at least every sequence's tiles where none is cut; 0: the other kernels.
 // Which kernel: the two-group kernel holds one workgroup per CU and runs faster once it has started (906 TFLOP/s against 680), but takes
 // 6 us longer until then, and its longest item decides when there are few.  So this form takes what fits on the chip about at once, two
-// workgroups per CU, four heads per workgroup (whose row tiles are half as long, and read the keys twice as often) somewhat less.  us on
-// either side, bf16, without the store: 16 heads over 8 kv heads of 128, two prompts of 270 rows 20.5 -> 14.5, one of 3000 67 -> 60, of 4000
-// (512 workgroups) 92 -> 82, ten of 406 (488) 32 -> 30, two of 2330 (592) 66 -> 68, nine of 463 (592) 30 -> 33,
-// seven of 965 (900) 51 -> 56; 32 heads, one of 1500 (384) 38.6 -> 35.7, four of 875 (904) 42 -> 51.
+// workgroups per CU, and somewhat more where its many short row tiles meet the other's long ones: short prompts, and one prompt, whose tiles are all
+// different.  us on either side, bf16: 16 heads over 8 kv heads of 128, two prompts of 270 rows 20.5 / 13, one of 3600 (456 workgroups) 84 / 73, of 5800
+// (728) 152 / 146, 16 of 370 (736) 33 / 29, 13 of 430 (816) 39 / 35, but seven of 760 (680) 37 / 40, two of 2500 (640) 73 / 75; 11 of 900 behind half (664)
+// 58 / 52, seven of 1600 (728) 83 / 83.  32 heads: nine of 120 16.2 / 13.9, 13 of 150 (576) 21.5 / 17.7, one of 1800 46.6 / 41.8, of 2500 (616) 67 / 63, five of
+// 530 (680) 30 / 30, six of 600 (896) 37 / 40; nine of 580 behind up to half (544) 37 / 30, four of 1900 (608) 66 / 60, one of 2270 (568) 147 / 166.
 // The two workgroups of a CU are the i-th and the (i + 256)-th.  Of a single sequence that is a heavy and a light one; of several equal
-// ones it can be two of the heaviest, and the longer the tiles, the less the later start of the other kernel counts.  us there and here, and
-// busiest_cu: two prompts of 1496 (384 workgroups) 36.6 / 34.8 1.67, of 1656 (424) 38.8 / 40.2 1.79, of 1976 (504) 47.3 / 51.8 1.98, three of 976
+// ones it can be two of the heaviest, and the longer the tiles, the less the later start of the other kernel counts.  us there and here (before
+// the one-group kernel's diagonal tiles became one loop, which took up to a tenth off short prompts here), and busiest_cu: two prompts of 1496 (384 workgroups) 36.6 / 34.8 1.67, of 1656 (424) 38.8 / 40.2 1.79, of 1976 (504) 47.3 / 51.8 1.98, three of 976
 // (384) 28.2 / 30.6 2.0, of 1296 (504) 36.6 / 34.5 1.52; behind cached halves three of 794 rows (320) 42.7 / 40.6 1.80, four of
 // 588 (320) 34.3 / 36.6 1.90; behind 95 %, nine of 128 (32 heads, 360) 59 / 71 2.0.  Uneven ones meet by chance: 3300 rows of two
-// (60 and 40 %) 44.2 / 38.3, of three 43.9 / 34.6.  Cached batches do not tell whether they are even and count as if.  (Above 112 tiles the
-// other form cuts its keys too, and loses on either side of the line.)
+// (60 and 40 %) 44.2 / 38.3, of three 43.9 / 34.6.  Cached batches do not tell whether they are even and count as if.  With four heads per workgroup
+// row tiles are half as long and equal sequences cost less: two prompts of 960 (496) 33.5 / 34.3, of 1040 34.9 / 36.7, three of 500 (392) 23.3 / 24.0, nine of
+// 233 (576, busiest 3) 21.1 / 23.0, but four of 680 (648, 2.2) 30.0 / 29.9, seven of 370 (624, 2.7) 25.4 / 24.0; behind halves only two of them lose (of 1630
+// 52 / 54; four of 1100 56 / 51).  (Above 112 tiles the other form cuts its keys too, and loses on either side of the line.)
 // An odd head group has row tiles of 128 here as there, so that nothing is gained from shorter ones: packed batches lose (us there and here, ten prompts of
 // 332, 12 heads over 4: 15.5 / 19.6; five of 764, 14 over 2: 22.7 / 28.7), but where the other form's places of 256 rows pass the chip's 512 and
 // these workgroups do not; cached ones gain what its empty places cost (seven of 40 to 70 rows behind as many, 40 over 8: 19.1 / 11.7; ten of
@@ -472,6 +475,9 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
 // behind as many, 16 heads (480 workgroups of 512 places, busiest 1.97) 60.4 / 67.6, three of 1266, 16 over 2 (480, 1.8) 43.3 / 49.3; four of 418
 // of 758 keys, 32 heads (512 places) 17.3 / 19.1, of 350 (352 of 512) 21.4 / 23.3; with tiles of 64 or 128 rows a third of the places empty ends
 // that (1.03 times as fast here in 40 random batches); beyond, of 518 of 958 (768) 26.5 / 20.2; eight of 93 of 168 (512 and 192) 19.1 / 15.8.
+// With four heads per workgroup a band is eight tiles: packed batches of 400 to 600 workgroups gain where it has empty places (nine of 244 16.8 / 13.5, five
+// of 190 15.0 / 14.3, three of 600 19.7 / 17.7; two of 960, none empty, 19.4 / 23.0) or is one sequence (of 1800 30.2 / 28.3), cached ones up to 1400 (16 of
+// 170 behind as many 27.8 / 22.2, three of 1600 behind up to half 107 / 98; none empty: eight of 500 47 / 50).
 // A few rows at head_dim 64 stay there, where placing the bands costs nothing (23 rows 8.8 / 9.5; from 5 sequences of 32 heads and 10 of 16
 // on 12.3 / 11.0), and so do 200 workgroups with more than 7000 keys, whose ranges the other form cuts (four heads of 128 121 / 128, of 64
 // 88 / 97, two of 64 80 / 96).
@@ -486,23 +492,29 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
   const int group = num_heads / num_kv_heads, bm = rows_of_tile(group);
   const int64_t slices = (int64_t)num_heads * bm / 128, wgs = (total_q_tokens / bm + num_seqs) * slices, tiles = ranges_of(max_kv_len, 1);
   const bool four = group % 4 == 0, odd = group % 2 != 0, paged = block_size > 0;
-  const int limit = head_dim == 64 ? (paged ? 768 : tiles >= 16 && !four ? 384 : 0)
-                    : !four        ? (tiles >= 16 ? 512 : tiles >= 7 ? 580 : 640)
-                                   : tiles >= 12 ? 384 : 300;
-  if (wgs > limit) return 0;
   // were all sequences as long as their mean: workgroups that have rows, the other form's places
   const int64_t even = num_seqs * ((total_q_tokens + (int64_t)num_seqs * bm - 1) / ((int64_t)num_seqs * bm)) * slices;
   const int64_t places = num_seqs * ((total_q_tokens + (int64_t)num_seqs * 256 - 1) / ((int64_t)num_seqs * 256)) * (256 / bm) * slices;
+  const bool packed64 = num_seqs == 1 ? even >= 384 && even <= 640 : num_seqs >= 3 && places > 512 && even >= 400 && even <= 600;
+  const int64_t limit = head_dim == 64 ? (paged  ? (four && places > even ? 1400 : 768)
+                                          : four ? (packed64 ? wgs : 0)
+                                                 : tiles >= 16 ? 384 : 0)
+                        : four  ? (paged && num_seqs == 1 ? 384 : 640)
+                        : odd   ? (tiles >= 16 ? 512 : tiles >= 7 ? 580 : 640)
+                        : paged ? (tiles >= 16 ? 512 : 780)
+                                : (num_seqs == 1 ? 740 : tiles >= 16 ? 512 : tiles > 7 ? 580 : 980);
+  if (wgs > limit) return 0;
   const float fresh = fminf(1.f, (float)total_q_tokens / ((float)num_seqs * (float)max_kv_len));
   const bool crowded = num_seqs > 1 && even > 272;
   if (head_dim == 64) {
-    if (crowded && (paged ? fresh >= 0.3f && places <= 512 && (four || 10 * places <= 13 * even) : fresh >= 0.75f) &&
+    if (crowded && (paged ? fresh >= 0.3f && places <= 512 && (four || 10 * places <= 13 * even) : !four && fresh >= 0.75f) &&
         busiest_cu(even, num_seqs, fresh) > (paged ? 1.7f : 1.5f))
       return 0;
   } else {
     if (odd && !paged && (places <= 512 || even > 512 || total_q_tokens <= (int64_t)bm * num_seqs)) return 0;
     if (odd && paged && wgs > 192 && places <= 512 && 10 * places <= 11 * even && fresh >= 0.25f) return 0;
-    if (crowded && tiles >= 16 && (paged ? tiles <= 112 : fresh >= 0.87f) && busiest_cu(even, num_seqs, fresh) > (paged ? 1.85f : 1.75f)) return 0;
+    if (crowded && tiles >= 16 && (paged ? tiles <= 112 && !(four && fresh >= 0.3f && num_seqs > 2) : fresh >= 0.87f) && busiest_cu(even, num_seqs, fresh) > (paged ? 1.85f : 1.75f)) return 0;
+    if (four && crowded && !paged && fresh >= 0.87f && busiest_cu(even, num_seqs, fresh) > (num_seqs <= 3 ? 1.87f : 2.9f)) return 0;
   }
   int64_t p = (tiles + 1) / 2 * 2;
   if (wgs > 192) return (four || head_dim == 64) && tiles > 112 ? 0 : (int)p;

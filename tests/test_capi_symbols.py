@@ -118,6 +118,26 @@ def test_prefill_ranges_plan_of_odd_head_groups():
     assert plan(10, 4700, 948, 16, 16, 64, *paged) == 16                                                       # 640 places
 
 
+def test_prefill_ranges_plan_at_its_limits():
+    """Which batches go over key ranges, on either side of each limit; all of them whole (one range of all tiles, an even number)."""
+    plan = _lib().load().mvllm_prefill_ranges_plan
+    packed, paged, four, two = (0, 1), (16, 1), (32, 8, 128), (16, 8, 128)
+    assert plan(9, 1080, 120, *four, *packed) == 2 and plan(13, 1950, 150, *four, *packed) == 4                # four heads: up to 640 workgroups
+    assert plan(7, 2300, 370, *four, *packed) == 6 and plan(7, 2400, 370, *four, *packed) == 0                 # 616 and 656
+    assert plan(2, 1920, 960, *four, *packed) == 0 and plan(2, 1700, 960, *four, *packed) == 16                # 1.95 of the longest tile and 1.82
+    assert plan(9, 2097, 233, *four, *packed) == 0                                                            # 3 of it
+    assert plan(4, 2200, 1100, *four, *paged) == 18 and plan(2, 1627, 1631, *four, *paged) == 0                # behind halves: not two of them
+    assert plan(1, 1500, 3000, *four, *paged) == 48 and plan(1, 1600, 3200, *four, *paged) == 0                # 384 and 408 of one sequence
+    assert plan(4, 700, 3600, *four, *paged) == 58 and plan(8, 1200, 4000, *four, *paged) == 0                 # most keys cached: equal ones stay
+    assert plan(1, 5800, 5800, *two, *packed) == 92 and plan(1, 6000, 6000, *two, *packed) == 0                # two heads: one sequence
+    assert plan(16, 5900, 370, *two, *packed) == 6 and plan(16, 6900, 440, *two, *packed) == 0                 # 16 short ones
+    assert plan(11, 4800, 900, *two, *paged) == 16 and plan(11, 5700, 900, *two, *paged) == 0                  # 688 and 800
+    at64 = (32, 8, 64)
+    assert plan(9, 1954, 334, *at64, *packed) == 6 and plan(3, 1344, 450, *at64, *packed) == 0                 # places without rows, none
+    assert plan(2, 1800, 960, *at64, *packed) == 0 and plan(1, 1800, 1800, *at64, *packed) == 30               # two, one
+    assert plan(16, 2720, 340, *at64, *paged) == 6 and plan(8, 4096, 1024, *at64, *paged) == 0                 # beyond 768 workgroups the same
+
+
 def test_prefill_split_plan_is_host_arithmetic():
     """When a paged prefill is cut over its keys: few query tiles, at least 4096 keys, a shape the split form takes;
     and the workspace holds the ranges' tables, partial results and denominators."""
