@@ -3,7 +3,7 @@
 // operator accepts without a conversion (dense tensors of the expected types on a GPU) and says None, or False where there is no result, to
 // everything else: then the operator goes its longer way (layers/attention.py, layers/window.py), which converts, warns or refuses.
 // What a small call takes the host, most of which was attribute look-ups of tensors, us the longer way and this one: decode 10.5 / 4.5, prefill
-// with its store 19.7 / 11.0, over a cached prefix 23.0 / 11.2, a window's prompts 15.2 / 5.0; a launch takes 3 of them.
+// with its store 19.7 / 11.0 (8.0 in one launch), over a cached prefix 23.0 / 11.2, a window's prompts 15.2 / 5.0; a launch takes 3 of them.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -33,6 +33,7 @@ struct Library {
   decltype(&mvllm_prefill_varlen) prefill;
   decltype(&mvllm_prefill_ranges) prefill_ranges;
   decltype(&mvllm_prefill_f32_ranges) prefill_f32_ranges;
+  decltype(&mvllm_prefill_ranges_store) prefill_store;
   decltype(&mvllm_prefill_paged) prefill_paged;
   decltype(&mvllm_prefill_paged_split_plan) split_plan;
   decltype(&mvllm_window_prefill) window_prefill;
@@ -205,10 +206,16 @@ bool ranges_of(PyObject* plan, PyObject* library, const int64_t (&sizes)[8], int
   return true;
 }
 
-// over key ranges into out; MVLLM_ERR_UNSUPPORTED: not taken
+// where the rows of k and v are stored
+struct Rows {
+  const at::Tensor *k_cache, *v_cache, *slots;
+  int64_t num_slots;
+};
+
+// over key ranges into out, the rows of k and v stored in the same launch where `to` says so; MVLLM_ERR_UNSUPPORTED: not taken
 int over_ranges(const at::Tensor& out, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor* tables, const at::Tensor& cu_q,
                 const at::Tensor* cu_k, int64_t max_keys, int heads, int kv_heads, int dim, int block, double scale, int code, int64_t tiles,
-                int64_t need, int64_t limit) {
+                int64_t need, int64_t limit, const Rows* to = nullptr) {
   if (tiles <= 0 || tiles > INT32_MAX || need < 0 || need > limit || !(scale > 0) || !aligned16(out) || !aligned16(q) || !aligned16(k) || !aligned16(v))
     return MVLLM_ERR_UNSUPPORTED;
   at::Tensor space;
@@ -217,6 +224,12 @@ int over_ranges(const at::Tensor& out, const at::Tensor& q, const at::Tensor& k,
   const int32_t *table = tables ? at_of<int32_t>(*tables) : nullptr, *keys = cu_k ? at_of<int32_t>(*cu_k) : nullptr;
   const int width = tables ? (int)tables->size(1) : 0, seqs = (int)cu_q.size(0) - 1;
   const int64_t blocks = tables ? k.size(0) : 0;
+  if (to)
+    return run([&] {
+      return lib.prefill_store(out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), to->k_cache->data_ptr(), to->v_cache->data_ptr(),
+                               at_of<int64_t>(*to->slots), to->num_slots, at_of<int32_t>(cu_q), seqs, q.size(0), (int)max_keys, heads, kv_heads, dim,
+                               (float)scale, code, (int)tiles, ws, (size_t)need, stream);
+    });
   return run([&] {
     return code == MVLLM_F32 ? lib.prefill_f32_ranges(at_of<float>(out), at_of<float>(q), at_of<float>(k), at_of<float>(v), table, width,
                                                       at_of<int32_t>(cu_q), keys, seqs, q.size(0), (int)max_keys, heads, kv_heads, dim, block,
@@ -227,10 +240,18 @@ int over_ranges(const at::Tensor& out, const at::Tensor& q, const at::Tensor& k,
   });
 }
 
+// whether the memory of two dense tensors meets
+bool meet(const at::Tensor& x, const at::Tensor& y) {
+  const char *x0 = at_of<char>(x), *y0 = at_of<char>(y);
+  return x0 < y0 + y.nbytes() && y0 < x0 + x.nbytes();
+}
+
 // prefill(q, k, v, cu_seqlens, scale, heads, kv_heads, head_dim, max_seqlen or None, plan, library, bytes at most) -> result
+// With (..., k_cache, v_cache, slots) behind them k and v are stored as well: beside the attention where that goes over key ranges, else in front of it.
 PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 12 || !lib.prefill || !ordinary()) return none();
+  const bool store = n == 15;
+  if ((n != 12 && !store) || !lib.prefill || !ordinary() || (store && (!lib.store || !lib.prefill_store))) return none();
   const at::Tensor *q = dense(a[0]), *k = dense(a[1]), *v = dense(a[2]), *cu = dense(a[3], at::kInt);
   double scale;
   int heads, kv_heads, dim;
@@ -245,16 +266,33 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
       q->size(2) != dim || !has_shape(*k, {rows, kv_heads, dim}) || v->sizes() != k->sizes() || k->scalar_type() != q->scalar_type() ||
       v->scalar_type() != q->scalar_type())
     return none();
+  const at::Tensor *k_cache = store ? dense(a[12], q->scalar_type()) : nullptr, *v_cache = store ? dense(a[13], q->scalar_type()) : nullptr;
+  const at::Tensor* slots = store ? dense(a[14], at::kLong) : nullptr;
+  if (store && (!k_cache || !v_cache || !slots || k_cache->dim() != 4 || v_cache->sizes() != k_cache->sizes() || k_cache->size(2) != kv_heads ||
+                k_cache->size(3) != dim || slots->numel() != rows))
+    return none();
+  const int64_t num_slots = store ? k_cache->size(0) * k_cache->size(1) : 0;
+  bool apart = store;                     // beside each other only where neither reads what the other writes
+  for (const at::Tensor* c : {k_cache, v_cache})
+    for (const at::Tensor* t : {q, k, v, cu}) apart = apart && !meet(*c, *t);
   int kernel = 0;                         // (shapes without a tiled kernel are warned of)
   if (lib.prefill_plan(heads, kv_heads, dim, 0, code, 0, &kernel) != MVLLM_OK || kernel <= 0) return none();
   int64_t tiles = 0, need = 0;
   longest = std::min(longest, rows);
   if (bound && !ranges_of(a[9], a[10], {cu->size(0) - 1, rows, longest, heads, kv_heads, dim, 0, code}, tiles, need)) return nullptr;
   at::Tensor out = at::empty_like(*q);
-  int status = tiles > 0 ? over_ranges(out, *q, *k, *v, nullptr, *cu, nullptr, longest, heads, kv_heads, dim, 0, scale, code, tiles, need, limit)
+  void* stream = stream_of(*q);
+  const bool beside = tiles > 0 && apart && aligned16(*k_cache) && aligned16(*v_cache);
+  if (store && !beside && run([&] {
+        return lib.store(k->data_ptr(), v->data_ptr(), k_cache->data_ptr(), v_cache->data_ptr(), at_of<int64_t>(*slots), rows, num_slots, kv_heads, dim,
+                         code, stream);
+      }) != MVLLM_OK)
+    return none();
+  const Rows to = {k_cache, v_cache, slots, num_slots};
+  int status = tiles > 0 ? over_ranges(out, *q, *k, *v, nullptr, *cu, nullptr, longest, heads, kv_heads, dim, 0, scale, code, tiles, need, limit,
+                                       beside ? &to : nullptr)
                          : MVLLM_ERR_UNSUPPORTED;
   if (tiles <= 0) {
-    void* stream = stream_of(*q);
     status = run([&] {
       return lib.prefill(out.data_ptr(), q->data_ptr(), k->data_ptr(), v->data_ptr(), at_of<int32_t>(*cu), (int)cu->size(0) - 1, rows, heads,
                          kv_heads, dim, (float)scale, code, stream);
@@ -386,6 +424,7 @@ PyObject* bind(PyObject*, PyObject* of) {
   set("mvllm_prefill_varlen", lib.prefill);
   set("mvllm_prefill_ranges", lib.prefill_ranges);
   set("mvllm_prefill_f32_ranges", lib.prefill_f32_ranges);
+  set("mvllm_prefill_ranges_store", lib.prefill_store);
   set("mvllm_prefill_paged", lib.prefill_paged);
   set("mvllm_prefill_paged_split_plan", lib.split_plan);
   set("mvllm_window_prefill", lib.window_prefill);

@@ -21,6 +21,7 @@ def test_calls_decline_what_is_not_theirs(calls):
         assert calls.store(q, x, cache, cache, i) is False
         assert calls.decode(q, cache, cache, None, None, cu[None], i, 1.0, 2, 2, 64, 16, None, None) is None
         assert calls.prefill(q, x, x, cu, 1.0, 2, 2, 64, None, plan, None, 1 << 30) is None
+        assert calls.prefill(q, x, x, cu, 1.0, 2, 2, 64, None, plan, None, 1 << 30, x, x, cu) is None
         assert calls.prefill_paged(q, cache, cache, cu[None], cu, cu, 1.0, 2, 2, 64, 16, 3, plan, None, 1 << 30) is None
         assert calls.window_prefill(q, q, x, cu, cu, 1.0, 0, None, x, None, None, None, 0.0, 0) is False
     assert calls.store() is False and calls.store(x) is False and calls.decode(x) is None and calls.prefill() is None

@@ -6,6 +6,7 @@ from torch.utils._python_dispatch import TorchDispatchMode
 from minivllm_amd import _C
 from minivllm_amd.layers import attention
 from minivllm_amd.layers.window import window_prefill
+from minivllm_amd.utils import reset_context, set_context
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -126,6 +127,40 @@ def test_prefill_and_store(counted, monkeypatch, dtype, lengths):
     both(counted, monkeypatch, lambda: stored(slots, normal(rows, 4, 64, dtype=dtype)[:, ::2]), 0)
     with pytest.raises((ValueError, AssertionError)):
         stored(slots[:-1])
+
+
+@pytest.mark.parametrize("dtype,heads,kv,dim", [(torch.bfloat16, 8, 2, 64), (torch.float16, 6, 3, 128), (torch.float32, 8, 8, 64), (torch.float32, 2, 1, 128),
+                                                (torch.bfloat16, 4, 1, 64), (torch.bfloat16, 4, 2, 96), (torch.bfloat16, 32, 8, 128)])
+@pytest.mark.parametrize("lengths", [[1], [0, 31, 0], [129, 7], [700, 300, 40], [1900]])
+def test_layer_stores_beside_its_prompts(counted, monkeypatch, dtype, heads, kv, dim, lengths):
+    """Rows without a slot, slots past the cache, rows that end within a workgroup's portion, several ranges; odd units per row; shapes that no ranges take."""
+    rows = sum(lengths)
+    q, k, v = normal(rows, heads, dim, dtype=dtype), normal(rows, kv, dim, dtype=dtype), normal(rows + 1, kv, dim, dtype=dtype)[1:]
+    cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    slots = torch.randperm(rows + 5, generator=torch.Generator().manual_seed(rows))[:rows]
+    slots[rows // 2], slots[rows // 3] = -1, 10 ** 12
+    slots = slots.to(DEV)
+    layer = attention.Attention(heads, dim, num_kv_heads=kv, block_size=16)
+
+    def forward(key=k, at=slots, most=max(lengths), caches=None):
+        layer.k_cache, layer.v_cache = caches or [torch.zeros(rows // 16 + 1, 16, kv, dim, dtype=dtype, device=DEV) for _ in range(2)]
+        set_context(True, cu_seqlens_q=cu, max_seqlen_q=most, slot_mapping=at)
+        try:
+            out = layer(q, key, v)
+        finally:
+            reset_context()
+        return torch.cat([t.flatten() for t in (out, layer.k_cache, layer.v_cache)])
+
+    for most in (max(lengths), 0):
+        got = both(counted, monkeypatch, lambda: forward(most=most), 1)
+    want = [torch.zeros(rows // 16 + 1, 16, kv, dim, dtype=dtype, device=DEV) for _ in range(2)]
+    there = (slots >= 0) & (slots < want[0].shape[0] * 16)
+    for cache, x in zip(want, (k, v)):
+        cache.view(-1, kv, dim)[slots[there]] = x[there]
+    assert torch.equal(got[rows * heads * dim:], torch.cat([t.flatten() for t in want]))
+    both(counted, monkeypatch, lambda: forward(at=slots.int()), 1)         # (the attention alone)
+    off = lambda: torch.zeros((rows // 16 + 1) * 16 * kv * dim + 1, dtype=dtype, device=DEV)[1:].view(-1, 16, kv, dim)
+    both(counted, monkeypatch, lambda: forward(caches=[off(), off()]), 1)  # caches off 16 bytes: one after the other
 
 
 @pytest.mark.parametrize("dtype,lengths,cached", [(torch.bfloat16, [200, 90], [150, 0]), (torch.float32, [700, 40], [640, 20]), (torch.bfloat16, [3000] * 8, [0] * 8),
