@@ -334,13 +334,14 @@ int mvllm_prefill_f32_ranges(float* out, const float* q, const float* k, const f
                              void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * mvllm_store_kvcache and mvllm_prefill_ranges (fp32: mvllm_prefill_f32_ranges) of a packed batch in one launch: the rows of k and v go to the
- * caches while the attention runs.  Caches are 16-byte aligned and are not q, k, v or out.  MVLLM_ERR_UNSUPPORTED (nothing has run): the two calls.
+ * mvllm_store_kvcache and the attention of a packed batch in one launch: the rows of k and v go to the caches while mvllm_prefill_varlen's kernels run
+ * (range_tiles 0), or those of mvllm_prefill_ranges and mvllm_prefill_f32_ranges.  Caches are 16-byte aligned and meet none of q, k, v
+ * and out.  MVLLM_ERR_UNSUPPORTED (nothing has run): the two calls.
  */
-int mvllm_prefill_ranges_store(void* out, const void* q, const void* k, const void* v, void* k_cache, void* v_cache,
-                               const int64_t* slot_mapping, int64_t num_slots, const int32_t* cu_seqlens, int num_seqs,
-                               int64_t total_tokens, int max_seqlen, int num_heads, int num_kv_heads, int head_dim, float scale,
-                               int dtype, int range_tiles, void* workspace, size_t workspace_bytes, void* stream);
+int mvllm_prefill_store(void* out, const void* q, const void* k, const void* v, void* k_cache, void* v_cache,
+                        const int64_t* slot_mapping, int64_t num_slots, const int32_t* cu_seqlens, int num_seqs,
+                        int64_t total_tokens, int max_seqlen, int num_heads, int num_kv_heads, int head_dim, float scale,
+                        int dtype, int range_tiles, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * The caller's per-layer chain between the QKV projection and the attention kernels, fused:

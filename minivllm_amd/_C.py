@@ -41,7 +41,7 @@ SIGNATURES = {
     "mvllm_prefill_f32_ranges_workspace_bytes": (c_size_t, [c_int64] + [c_int] * 4),
     "mvllm_prefill_f32_ranges": (c_int, [c_void_p] * 5 + [c_int, c_void_p, c_void_p, c_int, c_int64] + [c_int] * 5 +
                                  [c_int64, c_float, c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
-    "mvllm_prefill_ranges_store": (c_int, [c_void_p] * 7 + [c_int64, c_void_p, c_int, c_int64] + [c_int] * 4 + [c_float, c_int, c_int, c_void_p,
+    "mvllm_prefill_store": (c_int, [c_void_p] * 7 + [c_int64, c_void_p, c_int, c_int64] + [c_int] * 4 + [c_float, c_int, c_int, c_void_p,
                                                                                                               c_size_t, c_void_p]),
     "mvllm_prefill_varlen": (c_int, [c_void_p] * 5 + [c_int, c_int64, c_int, c_int, c_int, c_float, c_int,
                                                        c_void_p]),

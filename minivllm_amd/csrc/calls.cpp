@@ -33,7 +33,7 @@ struct Library {
   decltype(&mvllm_prefill_varlen) prefill;
   decltype(&mvllm_prefill_ranges) prefill_ranges;
   decltype(&mvllm_prefill_f32_ranges) prefill_f32_ranges;
-  decltype(&mvllm_prefill_ranges_store) prefill_store;
+  decltype(&mvllm_prefill_store) prefill_store;
   decltype(&mvllm_prefill_paged) prefill_paged;
   decltype(&mvllm_prefill_paged_split_plan) split_plan;
   decltype(&mvllm_window_prefill) window_prefill;
@@ -247,7 +247,7 @@ bool meet(const at::Tensor& x, const at::Tensor& y) {
 }
 
 // prefill(q, k, v, cu_seqlens, scale, heads, kv_heads, head_dim, max_seqlen or None, plan, library, bytes at most) -> result
-// With (..., k_cache, v_cache, slots) behind them k and v are stored as well: beside the attention where that goes over key ranges, else in front of it.
+// With (..., k_cache, v_cache, slots) behind them k and v are stored as well: beside the attention where its kernel takes that, else in front of it.
 PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   const bool store = n == 15;
@@ -282,22 +282,27 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (bound && !ranges_of(a[9], a[10], {cu->size(0) - 1, rows, longest, heads, kv_heads, dim, 0, code}, tiles, need)) return nullptr;
   at::Tensor out = at::empty_like(*q);
   void* stream = stream_of(*q);
-  const bool beside = tiles > 0 && apart && aligned16(*k_cache) && aligned16(*v_cache);
-  if (store && !beside && run([&] {
+  const Rows to = {k_cache, v_cache, slots, num_slots};
+  auto attend = [&](const Rows* beside) {
+    if (tiles > 0)
+      return over_ranges(out, *q, *k, *v, nullptr, *cu, nullptr, longest, heads, kv_heads, dim, 0, scale, code, tiles, need, limit, beside);
+    return run([&] {
+      return beside ? lib.prefill_store(out.data_ptr(), q->data_ptr(), k->data_ptr(), v->data_ptr(), k_cache->data_ptr(), v_cache->data_ptr(),
+                                        at_of<int64_t>(*slots), num_slots, at_of<int32_t>(*cu), (int)cu->size(0) - 1, rows, (int)longest, heads, kv_heads,
+                                        dim, (float)scale, code, 0, nullptr, 0, stream)
+                    : lib.prefill(out.data_ptr(), q->data_ptr(), k->data_ptr(), v->data_ptr(), at_of<int32_t>(*cu), (int)cu->size(0) - 1, rows,
+                                  heads, kv_heads, dim, (float)scale, code, stream);
+    });
+  };
+  int status = MVLLM_ERR_UNSUPPORTED;
+  if (apart && aligned16(*k_cache) && aligned16(*v_cache)) status = attend(&to);
+  if (status == MVLLM_OK) return THPVariable_Wrap(std::move(out));
+  if (store && run([&] {
         return lib.store(k->data_ptr(), v->data_ptr(), k_cache->data_ptr(), v_cache->data_ptr(), at_of<int64_t>(*slots), rows, num_slots, kv_heads, dim,
                          code, stream);
       }) != MVLLM_OK)
     return none();
-  const Rows to = {k_cache, v_cache, slots, num_slots};
-  int status = tiles > 0 ? over_ranges(out, *q, *k, *v, nullptr, *cu, nullptr, longest, heads, kv_heads, dim, 0, scale, code, tiles, need, limit,
-                                       beside ? &to : nullptr)
-                         : MVLLM_ERR_UNSUPPORTED;
-  if (tiles <= 0) {
-    status = run([&] {
-      return lib.prefill(out.data_ptr(), q->data_ptr(), k->data_ptr(), v->data_ptr(), at_of<int32_t>(*cu), (int)cu->size(0) - 1, rows, heads,
-                         kv_heads, dim, (float)scale, code, stream);
-    });
-  }
+  status = attend(nullptr);
   return status == MVLLM_OK ? THPVariable_Wrap(std::move(out)) : none();
   END_HANDLE_TH_ERRORS
 }
@@ -424,7 +429,7 @@ PyObject* bind(PyObject*, PyObject* of) {
   set("mvllm_prefill_varlen", lib.prefill);
   set("mvllm_prefill_ranges", lib.prefill_ranges);
   set("mvllm_prefill_f32_ranges", lib.prefill_f32_ranges);
-  set("mvllm_prefill_ranges_store", lib.prefill_store);
+  set("mvllm_prefill_store", lib.prefill_store);
   set("mvllm_prefill_paged", lib.prefill_paged);
   set("mvllm_prefill_paged_split_plan", lib.split_plan);
   set("mvllm_window_prefill", lib.window_prefill);

@@ -265,6 +265,16 @@ bool prefill_rows16_takes(int head_dim, int dtype, bool int8_cache);
 // Varlen causal prefill in the two-group form (prefill_pingpong.hip): one persistent 8-wave workgroup per CU whose two
 // wave groups alternate between the matrix unit and the softmax.  Launched from the prefill entry point for the batches
 // it takes; everything else stays on prefill_mfma_kernel.
+// The rows of k and v of a packed prefill that go to a paged cache in its launch (store_beside, prefill_tiles.h); without a cache there are none.
+struct StoreBeside {
+  unsigned first = 0;            // the workgroups from here on copy; set by the launcher
+  unsigned row_units = 0, units = 0;      // 16-byte units per token row, and of all rows
+  const void *key = nullptr, *value = nullptr;
+  void *k_cache = nullptr, *v_cache = nullptr;
+  const int64_t* slots = nullptr;
+  int64_t num_slots = 0;
+};
+
 struct PrefillPpArgs {
   void* out;
   const void* q;
@@ -296,6 +306,7 @@ struct PrefillPpArgs {
   unsigned long long* timeline;
   int timeline_entries;
   int timeline_block;
+  StoreBeside store;      // packed batches
 };
 // block_size: 0 for the packed entry point
 bool prefill_pp_takes(int num_seqs, int num_heads, int num_kv_heads, int head_dim, int dtype, int block_size);

@@ -55,9 +55,9 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
   const unsigned round = slot / kXcdChunk;
   const unsigned item = (round * 8 + ((xcd + round) & 7)) * kXcdChunk + slot % kXcdChunk;
   int item_y, seq_start, seq_len, row0, seq_index;
-  if constexpr (RANGES && !PAGED)
-    if (id >= a.items) {
-      store_beside(a, (id - a.items) * gridDim.y + blockIdx.y, (gridDim.x - a.items) * gridDim.y);
+  if constexpr (!PAGED)
+    if (id >= a.store.first) {
+      store_beside<64 * kPfWaves>(a.store);
       return;
     }
   if constexpr (RANGES) {                                            // slices fastest, nothing padded (prefill_mfma.h)
@@ -285,8 +285,9 @@ int launch_f32_as(const PrefillArgs& a, hipStream_t stream, int ranges = 1) {
   while (((int64_t)1 << b.band_bits) <= a.total_tokens / (bm << b.band_shift) + 1) ++b.band_bits;
   const int64_t items = (int64_t)b.tiles_x * b.heads_y;
   const int64_t span = 8 * (int64_t)kXcdChunk;
-  b.items = (unsigned)items;
-  const dim3 grid(RANGES ? (unsigned)items + store_groups(a, ranges) : (unsigned)((items + span - 1) / span * span), (unsigned)ranges), block(64 * kPfWaves);
+  dim3 grid(RANGES ? (unsigned)items : (unsigned)((items + span - 1) / span * span), (unsigned)ranges);
+  if (!PAGED) add_store_groups(b.store, grid);
+  const dim3 block(64 * kPfWaves);
   if (hpw == 4) prefill_f32_kernel<D, 4, PAGED, RANGES><<<grid, block, 0, stream>>>(b);
   else if (hpw == 2) prefill_f32_kernel<D, 2, PAGED, RANGES><<<grid, block, 0, stream>>>(b);
   else prefill_f32_kernel<D, 1, PAGED, RANGES><<<grid, block, 0, stream>>>(b);

@@ -49,55 +49,8 @@ struct PrefillArgs {
   // [ranges, total_tokens, num_heads] as above (-inf: no keys), others go straight to out.
   int range_tiles = 0;
   float* part = nullptr;
-  // Key ranges of packed batches: workgroups from `items` on copy the new rows of k and v to the paged cache (store_beside); without a
-  // cache there are none.
-  unsigned items = 0;
-  int row_units = 0;             // 16-byte units per token row
-  uint4* k_store = nullptr;
-  uint4* v_store = nullptr;
-  const int64_t* slots = nullptr;
-  int64_t num_slots = 0;
+  StoreBeside store;             // packed batches
 };
-
-constexpr int kStoreUnits = 1024, kStoreGroups = 256;      // units of K, and of V, that a workgroup copies at a time; workgroups at most
-
-// The cache store of a packed batch as workgroups of the attention's own launch, behind its items: nothing here reads the cache, so neither waits for the
-// other.  As a launch of its own the copy of a short batch's rows is 2.5 us of launch and 1 of copying, and as much again of the host's
-// time, in front of a kernel that leaves most CUs idle.  us with the store in front / beside, bf16, 8 kv heads of 128: 7 prompts of 60 to 151,
-// 32 heads, 12.4 / 8.4; 3 of 165 to 1036 24.0 / 20.2, one of 1800 40.2 / 36.9; 16 heads, 13 of 60 to 500 20.5 / 15.3, two of 900 to 1500 31.4 / 26.7;
-// fp32, heads of 64, one of 400 26.1 / 22.6.
-// Workgroups of the kernel's 256 threads, 32 KB each; more than kStoreGroups would queue for the places that the kernel's LDS leaves (two per CU).
-__device__ __forceinline__ void store_beside(const PrefillArgs& a, unsigned block, unsigned blocks) {
-  typedef uint32_t unit __attribute__((ext_vector_type(4)));
-  const unsigned units = (unsigned)a.row_units, all = (unsigned)a.total_tokens * units;      // (below 2^30, which the host has checked)
-  const unit *key = reinterpret_cast<const unit*>(a.k), *value = reinterpret_cast<const unit*>(a.v);
-  unit *to_k = reinterpret_cast<unit*>(a.k_store), *to_v = reinterpret_cast<unit*>(a.v_store);
-  for (unsigned first = block * kStoreUnits + threadIdx.x; first < all; first += blocks * kStoreUnits) {
-    unit k[4], v[4];
-    int64_t to[4];
-    static_for<4>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      const unsigned i = first + kStoreUnits / 4 * j, in = i < all ? i : all - 1, row = in / units;
-      const int64_t slot = a.slots[row];
-      to[j] = i < all && slot >= 0 && slot < a.num_slots ? slot * units + (in - row * units) : -1;
-      k[j] = key[in];
-      v[j] = value[in];
-    });
-    static_for<4>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      if (to[j] >= 0) {
-        to_k[to[j]] = k[j];
-        to_v[to[j]] = v[j];
-      }
-    });
-  }
-}
-// workgroups of a range that do so, of a launch of `ranges` ranges
-inline unsigned store_groups(const PrefillArgs& a, int ranges) {
-  if (a.k_store == nullptr) return 0;
-  const int64_t all = (a.total_tokens * a.row_units + kStoreUnits - 1) / kStoreUnits, n = all < kStoreGroups ? all : kStoreGroups;
-  return (unsigned)((n + ranges - 1) / ranges);
-}
 
 constexpr unsigned kXcdChunk = 32;      // consecutive work items handed to one XCD
 constexpr int kPfWaves = 4;             // waves per workgroup: 4, so that two workgroups share a CU
@@ -270,9 +223,9 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
     const int s = threadIdx.x & 63;
     if (s < a.num_seqs && a.num_seqs <= 64) keys = a.cu_seqlens_k[s + 1] - a.cu_seqlens_k[s];
   }
-  if constexpr (RANGES && !PAGED)
-    if (id >= a.items) {
-      store_beside(a, (id - a.items) * gridDim.y + blockIdx.y, (gridDim.x - a.items) * gridDim.y);
+  if constexpr (!PAGED)
+    if (id >= a.store.first) {
+      store_beside<64 * kPfWaves>(a.store);
       return;
     }
   if constexpr (RANGES) {
@@ -896,8 +849,8 @@ static int launch_prefill_mfma_as(const PrefillArgs& a, hipStream_t stream, int 
   while (((int64_t)1 << b.band_bits) <= a.total_tokens / (bm << b.band_shift) + 1) ++b.band_bits;
   const int64_t items = (int64_t)b.tiles_x * b.heads_y;
   const int64_t span = 8 * (int64_t)kXcdChunk;
-  b.items = (unsigned)items;
-  dim3 grid(RANGES ? (unsigned)items + store_groups(a, ranges) : (unsigned)((items + span - 1) / span * span), (unsigned)ranges);
+  dim3 grid(RANGES ? (unsigned)items : (unsigned)((items + span - 1) / span * span), (unsigned)ranges);
+  if (!PAGED) add_store_groups(b.store, grid);
   const dim3 block(64 * kPfWaves);
   if (hpw == 4) prefill_mfma_kernel<T, 4, PAGED, D, I8, DD, RANGES><<<grid, block, 0, stream>>>(b);
   else if (hpw == 2) prefill_mfma_kernel<T, 2, PAGED, D, I8, DD, RANGES><<<grid, block, 0, stream>>>(b);
@@ -910,6 +863,10 @@ static int launch_prefill_mfma(const PrefillArgs& a, hipStream_t stream) {
                           : launch_prefill_mfma_as<T, PAGED, I8, 128, 128>(a, stream);
 }
 
+// mvllm_prefill_varlen(_sink), and with the rows' store beside it (prefill_varlen.hip)
+int run_prefill_varlen(void* out, const void* q, const void* k, const void* v, const int32_t* cu_seqlens, int num_seqs, int64_t total_tokens,
+                       int num_heads, int num_kv_heads, int head_dim, float scale, const float* sink, int dtype, const StoreBeside& store,
+                       void* stream);
 // the paged form over a 16-bit cache, head_dim 64 or 128, bf16 / fp16 (prefill_varlen.hip)
 int launch_prefill_paged_16bit(const PrefillArgs& a, int dtype, hipStream_t stream);
 // the paged form over an INT8 cache (codes + fp32 scales), head_dim 64 or 128, bf16 / fp16 queries (prefill_varlen.hip)

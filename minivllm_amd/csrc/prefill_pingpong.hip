@@ -884,6 +884,11 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
 template <typename T, int D, bool PAGED, int HPI>
 __global__ __launch_bounds__(64 * kPpWaves, 1) void prefill_pp_kernel(const PrefillPpArgs a) {
   __shared__ __attribute__((aligned(1024))) PpLds<D> lds;
+  if constexpr (!PAGED)
+    if (blockIdx.x >= a.store.first) {                // the CUs whose last items are done copy the rows meanwhile
+      store_beside<64 * kPpWaves>(a.store);
+      return;
+    }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (wave < 4) pp_run<T, D, 0, PAGED, HPI>(a, lds, wave);
   else pp_run<T, D, 1, PAGED, HPI>(a, lds, wave);
@@ -938,7 +943,9 @@ int launch_prefill_pp(const PrefillPpArgs& args, int dtype, hipStream_t stream) 
   const int64_t most_keys = paged ? (int64_t)a.max_num_blocks * a.block_size + a.total_tokens : a.total_tokens;
   a.level_bits = 1;
   while (((int64_t)1 << a.level_bits) <= most_keys / 64 + 4) ++a.level_bits;
-  const dim3 g(grid), b(64 * kPpWaves);
+  dim3 g(grid);
+  if (!paged) add_store_groups(a.store, g);
+  const dim3 b(64 * kPpWaves);
   if (dtype == MVLLM_BF16) launch_prefill_pp_as<bf16_t>(a, paged, hpi, g, b, stream);
   else launch_prefill_pp_as<f16_t>(a, paged, hpi, g, b, stream);
   return launch_status();

@@ -538,25 +538,10 @@ extern "C" size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, i
   return ranges < 2 ? 0 : (size_t)ranges * total_q_tokens * num_heads * (head_dim + 1) * sizeof(float);
 }
 
-// the paged cache that a packed batch's new rows go to in the same launch (store_beside); none: no store
-struct StoreTo {
-  void *k_cache, *v_cache;
-  const int64_t* slots;
-  int64_t num_slots;
-};
-static int add_store(PrefillArgs& a, const StoreTo& to, int element_bytes) {
-  if (to.k_cache == nullptr) return MVLLM_OK;
-  a.row_units = (int)((int64_t)a.num_kv_heads * a.head_dim * element_bytes / 16);
-  if (a.total_tokens * a.row_units >= ((int64_t)1 << 30)) return MVLLM_ERR_UNSUPPORTED;      // (positions in store_beside are 32 bits)
-  a.k_store = reinterpret_cast<uint4*>(to.k_cache); a.v_store = reinterpret_cast<uint4*>(to.v_cache);
-  a.slots = to.slots; a.num_slots = to.num_slots;
-  return MVLLM_OK;
-}
-
 static int run_ranges(void* out, const void* q, const void* k, const void* v, const int32_t* block_tables, int max_num_blocks,
                       const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int num_seqs, int64_t total_q_tokens, int max_kv_len,
                       int num_heads, int num_kv_heads, int head_dim, int block_size, int64_t num_blocks, float scale, const float* sink,
-                      int dtype, int range_tiles, void* workspace, size_t workspace_bytes, const StoreTo& store, void* stream) {
+                      int dtype, int range_tiles, void* workspace, size_t workspace_bytes, const StoreBeside& store, void* stream) {
   if (dtype_size(dtype) == 0) return MVLLM_ERR_BAD_DTYPE;
   const bool paged = block_size > 0;
   if (num_seqs < 0 || total_q_tokens < 0 || max_kv_len < 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || block_size < 0 ||
@@ -581,9 +566,8 @@ static int run_ranges(void* out, const void* q, const void* k, const void* v, co
   a.range_tiles = range_tiles;
   a.part = reinterpret_cast<float*>(workspace);
   a.lse = ranges > 1 ? a.part + (int64_t)ranges * total_q_tokens * num_heads * head_dim : nullptr;
-  int status = add_store(a, store, 2);
-  if (status != MVLLM_OK) return status;
-  status = launch_prefill_ranges(a, dtype, paged, ranges, s);
+  a.store = store;
+  const int status = launch_prefill_ranges(a, dtype, paged, ranges, s);
   if (status != MVLLM_OK || ranges == 1) return status;
   RangeMergeArgs m;
   m.out = out; m.part = a.part; m.lse = a.lse; m.cu_seqlens_q = cu_seqlens_q; m.cu_seqlens_k = a.cu_seqlens_k; m.sink = sink;
@@ -607,7 +591,7 @@ extern "C" int mvllm_prefill_ranges(void* out, const void* q, const void* k, con
                                     int64_t num_blocks, float scale, const float* sink, int dtype, int range_tiles, void* workspace,
                                     size_t workspace_bytes, void* stream) {
   return run_ranges(out, q, k, v, block_tables, max_num_blocks, cu_seqlens_q, cu_seqlens_k, num_seqs, total_q_tokens, max_kv_len, num_heads,
-                    num_kv_heads, head_dim, block_size, num_blocks, scale, sink, dtype, range_tiles, workspace, workspace_bytes, StoreTo{}, stream);
+                    num_kv_heads, head_dim, block_size, num_blocks, scale, sink, dtype, range_tiles, workspace, workspace_bytes, StoreBeside{}, stream);
 }
 
 // ---- the same for fp32 (prefill_f32.hip), whose tiles are 32 keys ----
@@ -675,7 +659,7 @@ extern "C" size_t mvllm_prefill_f32_ranges_workspace_bytes(int64_t total_q_token
 static int run_f32_ranges(float* out, const float* q, const float* k, const float* v, const int32_t* block_tables, int max_num_blocks,
                           const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int num_seqs, int64_t total_q_tokens, int max_kv_len,
                           int num_heads, int num_kv_heads, int head_dim, int block_size, int64_t num_blocks, float scale, const float* sink,
-                          int range_tiles, void* workspace, size_t workspace_bytes, const StoreTo& store, void* stream) {
+                          int range_tiles, void* workspace, size_t workspace_bytes, const StoreBeside& store, void* stream) {
   const bool paged = block_size > 0;
   if (num_seqs < 0 || total_q_tokens < 0 || max_kv_len < 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || block_size < 0 ||
       num_blocks < 0 || max_num_blocks < 0 || num_heads % num_kv_heads != 0 || !(scale > 0.f) || range_tiles <= 0)
@@ -699,9 +683,8 @@ static int run_f32_ranges(float* out, const float* q, const float* k, const floa
   a.range_tiles = range_tiles;
   a.part = reinterpret_cast<float*>(workspace);
   a.lse = ranges > 1 ? a.part + (int64_t)ranges * total_q_tokens * num_heads * head_dim : nullptr;
-  int status = add_store(a, store, 4);
-  if (status != MVLLM_OK) return status;
-  status = launch_prefill_f32_ranges(a, paged, ranges, s);
+  a.store = store;
+  const int status = launch_prefill_f32_ranges(a, paged, ranges, s);
   if (status != MVLLM_OK || ranges == 1) return status;
   RangeMergeArgs m;
   m.out = out; m.part = a.part; m.lse = a.lse; m.cu_seqlens_q = cu_seqlens_q; m.cu_seqlens_k = a.cu_seqlens_k; m.sink = sink;
@@ -720,19 +703,23 @@ extern "C" int mvllm_prefill_f32_ranges(float* out, const float* q, const float*
                                         int block_size, int64_t num_blocks, float scale, const float* sink, int range_tiles,
                                         void* workspace, size_t workspace_bytes, void* stream) {
   return run_f32_ranges(out, q, k, v, block_tables, max_num_blocks, cu_seqlens_q, cu_seqlens_k, num_seqs, total_q_tokens, max_kv_len, num_heads,
-                        num_kv_heads, head_dim, block_size, num_blocks, scale, sink, range_tiles, workspace, workspace_bytes, StoreTo{}, stream);
+                        num_kv_heads, head_dim, block_size, num_blocks, scale, sink, range_tiles, workspace, workspace_bytes, StoreBeside{}, stream);
 }
 
-extern "C" int mvllm_prefill_ranges_store(void* out, const void* q, const void* k, const void* v, void* k_cache, void* v_cache,
-                                          const int64_t* slot_mapping, int64_t num_slots, const int32_t* cu_seqlens, int num_seqs,
-                                          int64_t total_tokens, int max_seqlen, int num_heads, int num_kv_heads, int head_dim, float scale,
-                                          int dtype, int range_tiles, void* workspace, size_t workspace_bytes, void* stream) {
+extern "C" int mvllm_prefill_store(void* out, const void* q, const void* k, const void* v, void* k_cache, void* v_cache,
+                                   const int64_t* slot_mapping, int64_t num_slots, const int32_t* cu_seqlens, int num_seqs,
+                                   int64_t total_tokens, int max_seqlen, int num_heads, int num_kv_heads, int head_dim, float scale,
+                                   int dtype, int range_tiles, void* workspace, size_t workspace_bytes, void* stream) {
   if (dtype_size(dtype) == 0) return MVLLM_ERR_BAD_DTYPE;
-  if (num_slots < 0) return MVLLM_ERR_BAD_SHAPE;
-  if (num_seqs == 0) return MVLLM_ERR_UNSUPPORTED;          // (there may be rows to store all the same)
+  if (num_slots < 0 || total_tokens < 0 || num_kv_heads <= 0 || head_dim <= 0) return MVLLM_ERR_BAD_SHAPE;
+  if (num_seqs == 0 || total_tokens > ((int64_t)1 << 30)) return MVLLM_ERR_UNSUPPORTED;          // (no sequences: there may be rows to store all the same)
   if (!k_cache || !v_cache || !slot_mapping) return MVLLM_ERR_NULL_POINTER;
   if (!aligned16(k_cache) || !aligned16(v_cache)) return MVLLM_ERR_MISALIGNED;
-  const StoreTo to = {k_cache, v_cache, slot_mapping, num_slots};
+  StoreBeside to;
+  if (!store_to(to, k, v, k_cache, v_cache, slot_mapping, num_slots, total_tokens, (int64_t)num_kv_heads * head_dim * dtype_size(dtype)))
+    return MVLLM_ERR_UNSUPPORTED;
+  if (range_tiles == 0)
+    return run_prefill_varlen(out, q, k, v, cu_seqlens, num_seqs, total_tokens, num_heads, num_kv_heads, head_dim, scale, nullptr, dtype, to, stream);
   return dtype == MVLLM_F32
              ? run_f32_ranges((float*)out, (const float*)q, (const float*)k, (const float*)v, nullptr, 0, cu_seqlens, nullptr, num_seqs, total_tokens,
                               max_seqlen, num_heads, num_kv_heads, head_dim, 0, 0, scale, nullptr, range_tiles, workspace, workspace_bytes, to, stream)

@@ -116,4 +116,53 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
+// The cache store of a packed batch as workgroups of the attention's own launch, behind its items: nothing there reads the cache, so neither waits for the
+// other.  As a launch of its own the copy of a short batch's rows is 2.5 us of launch and 1 of copying, and as much again of the host's
+// time, in front of a kernel that leaves most CUs idle.  us with the store in front / beside, bf16, 8 kv heads of 128: 7 prompts of 60 to 151,
+// 32 heads, 12.4 / 8.4; 3 of 165 to 1036 24.0 / 20.2, one of 1800 40.2 / 36.9; 16 heads, 13 of 60 to 500 20.5 / 15.3, two of 900 to 1500 31.4 / 26.7;
+// heads of 64, 16 of 250 20.2 / 16.4; fp32 one of 400 26.1 / 22.6, 8 of 18 to 305 27.6 / 23.4.  The two-group kernel has every CU to
+// itself until its first workgroups are done: two of 2500, 16 heads 69.4 / 62.7, 32 heads, 4 of 1200 to 1800 83.9 / 79.3, 16 of 64 to 2048 143.8 / 143.2.
+// Workgroups of the attention kernel's kThreads threads, 32 or 64 KB each; more than kStoreGroups would queue for the places that its LDS leaves.
+constexpr unsigned kStoreGroups = 256;
+template <int kThreads> __device__ __forceinline__ void store_beside(const StoreBeside& a) {
+  typedef uint32_t unit __attribute__((ext_vector_type(4)));
+  const unit *key = reinterpret_cast<const unit*>(a.key), *value = reinterpret_cast<const unit*>(a.value);
+  unit *to_k = reinterpret_cast<unit*>(a.k_cache), *to_v = reinterpret_cast<unit*>(a.v_cache);
+  const unsigned block = (blockIdx.x - a.first) * gridDim.y + blockIdx.y, blocks = (gridDim.x - a.first) * gridDim.y;
+  for (unsigned at = block * 4 * kThreads + threadIdx.x; at < a.units; at += blocks * 4 * kThreads) {      // (units are below 2^30)
+    unit k[4], v[4];
+    int64_t to[4];
+    static_for<4>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      const unsigned i = at + kThreads * j, in = i < a.units ? i : a.units - 1, row = in / a.row_units;
+      const int64_t slot = a.slots[row];
+      to[j] = i < a.units && slot >= 0 && slot < a.num_slots ? slot * a.row_units + (in - row * a.row_units) : -1;
+      k[j] = key[in];
+      v[j] = value[in];
+    });
+    static_for<4>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      if (to[j] >= 0) {
+        to_k[to[j]] = k[j];
+        to_v[to[j]] = v[j];
+      }
+    });
+  }
+}
+// behind a grid of items, (x, ranges)
+inline void add_store_groups(StoreBeside& a, dim3& grid) {
+  a.first = grid.x;
+  if (a.k_cache == nullptr) return;
+  const unsigned all = (a.units + 1023) / 1024, n = all < kStoreGroups ? all : kStoreGroups;
+  grid.x += (n + grid.y - 1) / grid.y;
+}
+// false: more rows than 32-bit positions reach, or rows that are not whole units
+inline bool store_to(StoreBeside& a, const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* slots, int64_t num_slots,
+                     int64_t tokens, int64_t row_bytes) {
+  if (row_bytes % 16 != 0 || row_bytes / 16 >= ((int64_t)1 << 30) || tokens * (row_bytes / 16) >= ((int64_t)1 << 30)) return false;
+  a.row_units = (unsigned)(row_bytes / 16); a.units = (unsigned)(tokens * (row_bytes / 16));
+  a.key = k; a.value = v; a.k_cache = k_cache; a.v_cache = v_cache; a.slots = slots; a.num_slots = num_slots;
+  return true;
+}
+
 }  // namespace mvllm

@@ -180,9 +180,10 @@ extern "C" int mvllm_prefill_plan(int num_heads, int num_kv_heads, int head_dim,
   return MVLLM_OK;
 }
 
-static int prefill_varlen_entry(void* out, const void* q, const void* k, const void* v, const int32_t* cu_seqlens,
-                                int num_seqs, int64_t total_tokens, int num_heads, int num_kv_heads, int head_dim,
-                                float scale, const float* sink, int dtype, void* stream) {
+namespace mvllm {
+int run_prefill_varlen(void* out, const void* q, const void* k, const void* v, const int32_t* cu_seqlens, int num_seqs, int64_t total_tokens,
+                       int num_heads, int num_kv_heads, int head_dim, float scale, const float* sink, int dtype, const StoreBeside& store,
+                       void* stream) {
   if (dtype_size(dtype) == 0) return MVLLM_ERR_BAD_DTYPE;
   if (num_seqs < 0 || total_tokens < 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0)
     return MVLLM_ERR_BAD_SHAPE;
@@ -201,6 +202,8 @@ static int prefill_varlen_entry(void* out, const void* q, const void* k, const v
   const bool aligned = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out);
   const int kind = aligned ? prefill_kernel_for(num_heads, num_kv_heads, head_dim, 0, dtype, false, false) : 0;
   const bool mfma_ok = kind == 2;
+  if (store.k_cache != nullptr && !mfma_ok) return MVLLM_ERR_UNSUPPORTED;        // (the other kernels have no workgroups for it)
+  a.store = store;
   if (mfma_ok && dtype == MVLLM_F32) return launch_prefill_f32(a, false, (hipStream_t)stream);
   if (mfma_ok && !sink && scale > 0.f && prefill_pp_takes(num_seqs, num_heads, num_kv_heads, head_dim, dtype, 0)) {
     PrefillPpArgs p;
@@ -209,6 +212,7 @@ static int prefill_varlen_entry(void* out, const void* q, const void* k, const v
     p.slices = 0; p.n_teams = 0; p.team_size = 0; p.level_bits = 0; p.spt_magic = 0; p.chunks_magic = 0;
     p.cu_seqlens_k = nullptr; p.block_tables = nullptr; p.max_num_blocks = 0; p.block_size = 0; p.num_blocks = 0; p.block_magic = 0; p.block_bytes = 0; p.num_blocks32 = 0;
     p.timeline = nullptr; p.timeline_entries = 0; p.timeline_block = 0;
+    p.store = store;
     return launch_prefill_pp(p, dtype, (hipStream_t)stream);
   }
   // fp32, and 16-bit head dims 32, 80, 96, 112 and 256: 16-row tiles on the decode kernel's tile arithmetic (paged_decode.hip)
@@ -223,21 +227,22 @@ static int prefill_varlen_entry(void* out, const void* q, const void* k, const v
   }
   return prefill_dispatch<false>(a, dtype, mfma_ok, (hipStream_t)stream);
 }
+}  // namespace mvllm
 
 extern "C" int mvllm_prefill_varlen(void* out, const void* q, const void* k, const void* v,
                                     const int32_t* cu_seqlens, int num_seqs, int64_t total_tokens,
                                     int num_heads, int num_kv_heads, int head_dim, float scale, int dtype,
                                     void* stream) {
-  return prefill_varlen_entry(out, q, k, v, cu_seqlens, num_seqs, total_tokens, num_heads, num_kv_heads, head_dim, scale,
-                              nullptr, dtype, stream);
+  return run_prefill_varlen(out, q, k, v, cu_seqlens, num_seqs, total_tokens, num_heads, num_kv_heads, head_dim, scale, nullptr, dtype,
+                            StoreBeside{}, stream);
 }
 
 extern "C" int mvllm_prefill_varlen_sink(void* out, const void* q, const void* k, const void* v,
                                          const int32_t* cu_seqlens, int num_seqs, int64_t total_tokens,
                                          int num_heads, int num_kv_heads, int head_dim, float scale,
                                          const float* sink, int dtype, void* stream) {
-  return prefill_varlen_entry(out, q, k, v, cu_seqlens, num_seqs, total_tokens, num_heads, num_kv_heads, head_dim, scale,
-                              sink, dtype, stream);
+  return run_prefill_varlen(out, q, k, v, cu_seqlens, num_seqs, total_tokens, num_heads, num_kv_heads, head_dim, scale, sink, dtype,
+                            StoreBeside{}, stream);
 }
 
 static int prefill_paged_entry(void* out, const void* q, const void* k_cache, const void* v_cache,

@@ -630,7 +630,7 @@ class Attention(nn.Module):
 
         if k_cache.numel() > 0 and v_cache.numel() > 0 and context.slot_mapping is not None:
             if context.is_prefill and context.block_tables is None and not int8 and q.dim() == 3 and _C.calls is not None:
-                # packed prompts: their attention reads k and v themselves, so that store and attention may run beside each other
+                # packed prompts: their attention reads k and v themselves, so that the store runs beside it
                 o = _C.calls.prefill(q, k, v, context.cu_seqlens_q, self.scale / (self.head_dim ** 0.5), self.num_heads, self.num_kv_heads,
                                      self.head_dim, context.max_seqlen_q or None, _prefill_ranges_plan, _C.load(), STAGED_PREFILL_MAX_BYTES,
                                      k_cache, v_cache, context.slot_mapping)

@@ -131,9 +131,9 @@ def test_prefill_and_store(counted, monkeypatch, dtype, lengths):
 
 @pytest.mark.parametrize("dtype,heads,kv,dim", [(torch.bfloat16, 8, 2, 64), (torch.float16, 6, 3, 128), (torch.float32, 8, 8, 64), (torch.float32, 2, 1, 128),
                                                 (torch.bfloat16, 4, 1, 64), (torch.bfloat16, 4, 2, 96), (torch.bfloat16, 32, 8, 128)])
-@pytest.mark.parametrize("lengths", [[1], [0, 31, 0], [129, 7], [700, 300, 40], [1900]])
+@pytest.mark.parametrize("lengths", [[1], [0, 31, 0], [129, 7], [700, 300, 40], [1900], [2000, 1500, 1400]])
 def test_layer_stores_beside_its_prompts(counted, monkeypatch, dtype, heads, kv, dim, lengths):
-    """Rows without a slot, slots past the cache, rows that end within a workgroup's portion, several ranges; odd units per row; shapes that no ranges take."""
+    """Rows without a slot, slots past the cache, rows that end within a workgroup's portion, several ranges, kernels over whole rows, the two-group kernel."""
     rows = sum(lengths)
     q, k, v = normal(rows, heads, dim, dtype=dtype), normal(rows, kv, dim, dtype=dtype), normal(rows + 1, kv, dim, dtype=dtype)[1:]
     cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
