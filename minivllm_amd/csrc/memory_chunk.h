@@ -46,6 +46,7 @@ struct MemoryChunkArgs {
   float* ws_n;               // [num_segments, H, dim]
   float* ws_m;               // [num_segments, H]: maximum
   float* ws_f;               // [num_segments, H]: sum of the log forget gates
+  float* ws_front;           // [num_segments, H]: maximum in front of the segment
   int64_t proj_stride;
   int num_segments, heads, dim, vdim;
   float q_scale, floor;
@@ -189,7 +190,7 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
       if constexpr (kGates) n_in = a.n_state + ((int64_t)slot * H + h) * dim;
     }
   } else {
-    m = kGates ? a.ws_m[(int64_t)seg * H + h] : 0.f;
+    m = kGates ? a.ws_front[(int64_t)seg * H + h] : 0.f;
     s_in = a.ws_s + ((int64_t)seg * H + h) * dim * vdim;
     if constexpr (kGates) n_in = a.ws_n + ((int64_t)seg * H + h) * dim;
   }
@@ -795,7 +796,9 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
   }
 }
 
-// Contributions of an entry's segments -> the state in front of each of them, in place.  Workgroup = (first segment of an
+// Contributions of an entry's segments -> the state in front of each of them, in place, and with gates the maximum there, which has a place of its own
+// because the contributions' own maxima are read by every slice (put there by a launch of its own behind this one, 3 us more: 4 prompts of 1102 to
+// 1748, 8 heads 70.6 / 67.6, two of 176 to 2390 46.2 / 43.4).  Workgroup = (first segment of an
 // entry, slice of the elements of S and n; head).  Slices run fastest: with segments there, the one workgroup in
 // num_segments that has work would always fall to the same XCD.  A thread owns four consecutive elements; the
 // contributions of kAhead segments are loaded together, before the states that replace them are stored.
@@ -837,6 +840,7 @@ __global__ __launch_bounds__(256) void memory_combine_kernel(const MemoryChunkAr
 #pragma unroll
     for (int j = 0; j < kAhead; ++j) {
       *reinterpret_cast<float4*>(ws + (base + j) * pitch) = x;
+      if (kGates && at == 0) a.ws_front[(int64_t)(base + j) * H + h] = m;
       if (last[j]) return;
       float m_new = 0.f, keep = 1.f, add = 1.f;
       if constexpr (kGates) {
@@ -854,22 +858,6 @@ __global__ __launch_bounds__(256) void memory_combine_kernel(const MemoryChunkAr
     }
   }
 }
-// The maxima in front of the segments: after the kernel above, which still needs the contributions' own.
-static __global__ __launch_bounds__(64) void memory_combine_max_kernel(const MemoryChunkArgs a) {
-  const int seg0 = blockIdx.x, h = blockIdx.y * 64 + threadIdx.x;
-  const int flags0 = a.segments[4 * seg0 + 3];
-  if (!(flags0 & 1) || (flags0 & 4) || h >= a.heads) return;
-  const int slot = a.slot[a.segments[4 * seg0]];
-  if (slot < 0) return;
-  float m = a.positions[a.segments[4 * seg0 + 1]] == 0 ? 0.f : a.m_state[(int64_t)slot * a.heads + h];
-  for (int seg = seg0; seg < a.num_segments; ++seg) {
-    float* p = a.ws_m + (int64_t)seg * a.heads + h;
-    const float own = *p;
-    *p = m;
-    if (a.segments[4 * seg + 3] & 2) break;
-    m = fmaxf(a.ws_f[(int64_t)seg * a.heads + h] + m, own);
-  }
-}
 
 template <int DIMP, int kWaves, bool kGates, bool kOut>
 static int launch_chunked(const MemoryChunkArgs& a, bool split, hipStream_t s) {
@@ -882,8 +870,6 @@ static int launch_chunked(const MemoryChunkArgs& a, bool split, hipStream_t s) {
     const int slices = (a.dim * a.vdim + (kGates ? a.dim : 0) + kCombineElements - 1) / kCombineElements;
     if ((int64_t)slices * a.num_segments >= 1 << 24) return MVLLM_ERR_BAD_SHAPE;
     memory_combine_kernel<kGates><<<dim3((unsigned)(slices * a.num_segments), (unsigned)a.heads), dim3(256), 0, s>>>(a, slices);
-    if constexpr (kGates)
-      memory_combine_max_kernel<<<dim3((unsigned)a.num_segments, (unsigned)((a.heads + 63) / 64)), dim3(64), 0, s>>>(a);
     status = launch_status();
     if (status != 0) return status;
   }

@@ -6,7 +6,7 @@
 using namespace mvllm;
 
 static int64_t chunk_ws_floats(int num_segments, int num_heads, int dim, int vdim) {
-  return (int64_t)num_segments * num_heads * ((int64_t)dim * vdim + dim + 2) + 16;
+  return (int64_t)num_segments * num_heads * ((int64_t)dim * vdim + dim + 3) + 16;
 }
 
 extern "C" size_t mvllm_mlstm_chunked_workspace_bytes(int num_segments, int num_heads, int dim, int vdim) {
@@ -41,6 +41,7 @@ static int chunk_args(MemoryChunkArgs& a, const void* proj, int64_t proj_row_str
   a.ws_n = split ? a.ws_s + units * dim * vdim : nullptr;
   a.ws_m = split ? a.ws_n + units * dim : nullptr;
   a.ws_f = split ? a.ws_m + units : nullptr;
+  a.ws_front = split ? a.ws_f + units : nullptr;
   return MVLLM_OK;
 }
 

@@ -77,8 +77,8 @@ def chunked_output_parts(fresh_rows: tuple, split: bool, heads: int, vdim: int) 
     A workgroup passes over the blocks in front of its own part, updating the state alone, at 0.3 of a block's time: with enough of them
     a portion of n blocks takes 0.3 n blocks' time instead of n, in one launch, as long as all run at once.  us in one part and
     shared, captured, heads of 128 x 256: 8 x 16 of 1024 rows 142 / 105 (2 parts), of 256 41 / 33.5; 8 heads, one portion of 128 17.6 / 16.2,
-    of 305 32 / 24.  Where the step's segments are cut (``split``), those cost two more passes and three launches but then go on side by
-    side however long a portion is: 34 us and the more, the more blocks there are in all.  us in segments and shared: 7 x 8 of
+    of 305 32 / 24.  Where the step's segments are cut (``split``), those cost two more passes, each a launch, but then go on side by
+    side however long a portion is: 31 us and the more, the more blocks there are in all.  us in segments (3 more than now) and shared: 7 x 8 of
     1000 rows 83 / 64.5, 4 x 16 of 1000 91.5 / 66, 2 x 16 of 800 54 / 45, 8 of 512 35.3 / 31.3, 4 x 8 of 1500 68.6 / 73, 8 of
     1024 43.5 / 51.  (Fewer columns, less state to combine: of 128 x 136, 4 x 8 of 1500 61.8 / 72, 2 x 16 of 800 48 / 45.)"""
     groups = heads * len(fresh_rows)
@@ -88,7 +88,7 @@ def chunked_output_parts(fresh_rows: tuple, split: bool, heads: int, vdim: int) 
         return 1
     if split:
         shared = 10.5 + 8.2 * PASS_OVER / (1 - (1 - PASS_OVER) ** parts) * blocks
-        segments = 32 + 0.053 * (0.5 + vdim / 512) * heads * sum(-(-n // BLOCK_ROWS) for n in fresh_rows)
+        segments = 29 + 0.053 * (0.5 + vdim / 512) * heads * sum(-(-n // BLOCK_ROWS) for n in fresh_rows)
         if shared >= segments:
             return 1
     return parts
