@@ -88,9 +88,20 @@ template <typename T16, int N> struct VecN {
 // value after a round trip through the element type
 template <typename T> __device__ __forceinline__ float rounded(float x) { return to_float(from_float<T>(x)); }
 
+// Sums over xor-neighbours, widest first; up to 8 lanes apart through the vector unit's own lane moves, a tenth of the way through the LDS' permutes.
 template <int GROUP> __device__ __forceinline__ float group_sum(float x) {
+  auto moved = [&](float old, auto CTRL, auto BANKS) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), decltype(CTRL)::value, 0xf, decltype(BANKS)::value, false));
+  };
+  using c = std::integral_constant<int, 0xf>;
 #pragma unroll
-  for (int o = GROUP / 2; o > 0; o >>= 1) x = x + __shfl_xor(x, o, 64);
+  for (int o = GROUP / 2; o > 8; o >>= 1) x = x + __shfl_xor(x, o, 64);
+  if constexpr (GROUP > 8) x = x + moved(0.f, std::integral_constant<int, 0x128>{}, c{});                    // rotated by 8 of 16
+  if constexpr (GROUP > 4)                                                                                  // from 4 lanes on, and 4 lanes before
+    x = x + moved(moved(0.f, std::integral_constant<int, 0x104>{}, std::integral_constant<int, 0x5>{}), std::integral_constant<int, 0x114>{},
+                  std::integral_constant<int, 0xa>{});
+  if constexpr (GROUP > 2) x = x + moved(0.f, std::integral_constant<int, 0x4e>{}, c{});
+  if constexpr (GROUP > 1) x = x + moved(0.f, std::integral_constant<int, 0xb1>{}, c{});
   return x;
 }
 template <int GROUP> __device__ __forceinline__ float group_max(float x) {
@@ -119,18 +130,22 @@ __device__ __forceinline__ void store_codes(int8_t* dst, const float (&x)[N], fl
 constexpr int kFusedThreads = 256;
 
 // EPL = elements per lane and half: 8 when head_dim is a multiple of 16 (16-byte accesses), else 4.
+// A decode step's few rows are a chain of latencies, so everything is asked for at the start, whether a vector needs it or not (v needs neither gamma
+// nor angles): two trips to memory, the position and the angles it points to.  With each load where it was used there were four or
+// five, and the division of the item's number took 64 bits.  us before / now, captured steps of 8 layers of 1024: 1 row 228.0 / 222.7, 16 rows 304.5 / 293.7,
+// 40 rows 494.9 / 485.0; 16384 tokens of 32 + 2 x 8 heads of 128 74.4 / 70.4, 8192 of 16 + 2 x 8 28.6 / 26.9.
 template <typename T, int GROUP, int EPL, bool INT8>
 __global__ __launch_bounds__(kFusedThreads) void qk_norm_rope_store_kernel(const FusedArgs a) {
   constexpr int kVecPerBlock = kFusedThreads / GROUP;
   const int j = threadIdx.x % GROUP;
   const int per_token = a.num_heads + 2 * a.num_kv_heads;
-  const int64_t item = (int64_t)blockIdx.x * kVecPerBlock + threadIdx.x / GROUP;
-  if (item >= a.num_tokens * per_token) return;          // whole groups leave together
-  const int64_t t = item / per_token;
+  const int64_t item = (int64_t)blockIdx.x * kVecPerBlock + threadIdx.x / GROUP, items = a.num_tokens * per_token;
+  if (item >= items) return;                             // whole groups leave together
+  const int64_t t = items <= 0xffffffffll ? (int64_t)((uint32_t)item / (uint32_t)per_token) : item / per_token;
   const int i = (int)(item - t * per_token);
   const int D = a.head_dim, half = D >> 1;
   const bool lane_live = 2 * EPL * j < D;                // GROUP may exceed the lanes a vector needs
-  const int e1 = EPL * j, e2 = half + EPL * j;
+  const int e1 = lane_live ? EPL * j : 0, e2 = half + e1;      // (the others read the first lane's)
 
   const int kind = i < a.num_heads ? 0 : (i < a.num_heads + a.num_kv_heads ? 1 : 2);   // q, k, v
   const int h = kind == 0 ? i : (kind == 1 ? i - a.num_heads : i - a.num_heads - a.num_kv_heads);
@@ -139,13 +154,19 @@ __global__ __launch_bounds__(kFusedThreads) void qk_norm_rope_store_kernel(const
                              : reinterpret_cast<const T*>(a.v) + t * a.v_stride;
   src += (int64_t)h * D;
 
-  float x1[EPL], x2[EPL];
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) x1[e] = x2[e] = 0.f;
-  if (lane_live) {
-    VecN<T, EPL>::load(src + e1, x1);
-    VecN<T, EPL>::load(src + e2, x2);
-  }
+  int64_t pos = a.positions[t];
+  const int64_t slot = (a.slot_mapping ? a.slot_mapping : a.positions)[t];
+  float x1[EPL], x2[EPL], g1[EPL], g2[EPL], c[EPL], s[EPL];
+  VecN<T, EPL>::load(src + e1, x1);
+  VecN<T, EPL>::load(src + e2, x2);
+  const float* gamma = a.gamma ? a.gamma : a.cos_sin;    // (a row of angles is as long)
+  VecN<float, EPL>::load(gamma + e1, g1);
+  VecN<float, EPL>::load(gamma + e2, g2);
+  pos = pos < 0 ? 0 : (pos >= a.max_position ? a.max_position - 1 : pos);
+  VecN<float, EPL>::load(a.cos_sin + pos * D + e1, c);
+  VecN<float, EPL>::load(a.cos_sin + pos * D + e2, s);
+
+  asm volatile("" ::: "memory");                         // (the compiler would move the loads to where they are used)
 
   if (kind != 2) {
     if (a.gamma) {
@@ -155,33 +176,21 @@ __global__ __launch_bounds__(kFusedThreads) void qk_norm_rope_store_kernel(const
       for (int e = 0; e < EPL; ++e) ss = ss + x1[e] * x1[e];
 #pragma unroll
       for (int e = 0; e < EPL; ++e) ss = ss + x2[e] * x2[e];
-      ss = group_sum<GROUP>(ss);
+      ss = group_sum<GROUP>(lane_live ? ss : 0.f);
       const SharedDivisor denom(sqrtf(ss / (float)D + a.eps));
-      if (lane_live) {
-        float g1[EPL], g2[EPL];
-        VecN<float, EPL>::load(a.gamma + e1, g1);
-        VecN<float, EPL>::load(a.gamma + e2, g2);
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-          x1[e] = rounded<T>(denom.divide(x1[e]) * g1[e]);
-          x2[e] = rounded<T>(denom.divide(x2[e]) * g2[e]);
-        }
+      for (int e = 0; e < EPL; ++e) {
+        x1[e] = rounded<T>(denom.divide(x1[e]) * g1[e]);
+        x2[e] = rounded<T>(denom.divide(x2[e]) * g2[e]);
       }
     }
     // out1 = x1 cos - x2 sin, out2 = x1 sin + x2 cos  (rotary_embedding.py:14-22)
-    if (lane_live) {
-      int64_t pos = a.positions[t];
-      pos = pos < 0 ? 0 : (pos >= a.max_position ? a.max_position - 1 : pos);
-      float c[EPL], s[EPL];
-      VecN<float, EPL>::load(a.cos_sin + pos * D + e1, c);
-      VecN<float, EPL>::load(a.cos_sin + pos * D + e2, s);
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        const float o1 = x1[e] * c[e] - x2[e] * s[e];
-        const float o2 = x1[e] * s[e] + x2[e] * c[e];
-        x1[e] = rounded<T>(o1);
-        x2[e] = rounded<T>(o2);
-      }
+    for (int e = 0; e < EPL; ++e) {
+      const float o1 = x1[e] * c[e] - x2[e] * s[e];
+      const float o2 = x1[e] * s[e] + x2[e] * c[e];
+      x1[e] = rounded<T>(o1);
+      x2[e] = rounded<T>(o2);
     }
   }
 
@@ -195,16 +204,13 @@ __global__ __launch_bounds__(kFusedThreads) void qk_norm_rope_store_kernel(const
     VecN<T, EPL>::store(dst + e1, x1);
     VecN<T, EPL>::store(dst + e2, x2);
   }
-  if (kind == 0 || !a.slot_mapping) return;
-
   // cache write, same slot arithmetic and skip rule as store_kvcache (attention.py:25-64)
-  const int64_t slot = a.slot_mapping[t];
-  if (slot < 0 || slot >= a.num_slots) return;
+  if (kind == 0 || !a.slot_mapping || slot < 0 || slot >= a.num_slots) return;
   const int64_t vec = slot * a.num_kv_heads + h;
   if constexpr (INT8) {
     float amax = 0.f;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) amax = fmaxf(amax, fmaxf(fabsf(x1[e]), fabsf(x2[e])));
+    for (int e = 0; e < EPL; ++e) amax = fmaxf(amax, fmaxf(fabsf(x1[e]), fabsf(x2[e])));      // (lanes past the vector hold the first one's)
     amax = group_max<GROUP>(amax);
     const float scale = amax / 127.0f;
     const bool live = scale > 0.f;
