@@ -165,8 +165,11 @@ __global__ __launch_bounds__(256) void moe_count_kernel(const PlanArgs a) {
 
 // A chain of latencies, not bytes: the counts of the blocks, sums over the experts, places.  With the counts' loads one by one and the sums in ten rounds
 // with two barriers each 14 us at 49152 pairs of 64 experts, so 5.9; 1800 pairs 5.1 and 3.5.
+// kRows: a.tile_rows.  It has no more sums than its tiles need: five of them for every plan took a small one 0.5 us.
+template <int kRows>
 __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
-  constexpr int kSums = 5;                          // rows; of either tiling the tiles in order and those behind them
+  constexpr bool large = kRows == 256, both = kRows == 128;
+  constexpr int kSums = both ? 4 : large ? 3 : 2;   // rows; tiles in order; of the tiling of 256 rows, those and the ones behind them
   __shared__ int32_t sum_to[kSums][kMaxExperts + 1], cursor[kMaxExperts], of_wave[kSums][16];
   const int e = threadIdx.x;
   int n = 0, mine = 0;
@@ -189,9 +192,12 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
     }
   }
   // inclusive sums over the experts: within a wave, then over the waves before it
-  const bool large = a.tile_rows == 256, both = a.tile_rows == 128;
   const bool apart = (large || both) && n % 256 != 0 && n % 256 <= kApartRows && a.pairs >= kApartPairs;      // the last tile of 256 goes behind all others
-  int sums[kSums] = {n, (n + a.tile_rows - 1) / a.tile_rows - (large && apart), large && apart, both ? (n + 255) / 256 - apart : 0, both && apart};
+  int sums[kSums];
+  sums[0] = n;
+  sums[1] = (n + kRows - 1) / kRows - (large && apart);
+  if constexpr (both) sums[2] = (n + 255) / 256 - apart;
+  if constexpr (large || both) sums[kSums - 1] = apart;
   const int lane = e & 63, wave = __builtin_amdgcn_readfirstlane(e >> 6);
   const bool some = 64 * wave < a.experts;
   if (some) {
@@ -232,19 +238,21 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const PlanArgs a) {
   if (blockIdx.x == 0 && e < a.experts) {
     a.row_start[e] = total[e];
     if (e == a.experts - 1) a.row_start[e + 1] = total[e + 1];
+#pragma unroll
     for (int i = 0; i < 1 + both; ++i) {
       const PlanArgs::Tiles& t = a.tiles[i];
-      const int32_t *tiles = sum_to[1 + 2 * i], *parts = sum_to[2 + 2 * i];
-      const int rows = i == 0 ? a.tile_rows : 256;
+      const bool wide = large || i == 1;
+      const int32_t *tiles = sum_to[1 + i], *parts = sum_to[kSums - 1];      // (parts: of the wide tiling alone)
+      const int rows = i == 0 ? kRows : 256;
       if (e == a.experts - 1) {
         t.num[0] = tiles[e + 1];
-        t.num[1] = parts[e + 1];
+        t.num[1] = wide ? parts[e + 1] : 0;
       }
       for (int k = tiles[e]; k < tiles[e + 1]; ++k) {
         t.expert[k] = e;
         t.row[k] = total[e] + (k - tiles[e]) * rows;
       }
-      if (parts[e + 1] > parts[e]) {
+      if (wide && parts[e + 1] > parts[e]) {
         const int k = tiles[a.experts] + parts[e];
         t.expert[k] = e;
         t.row[k] = total[e + 1] - n % 256;
@@ -845,7 +853,10 @@ extern "C" int mvllm_moe_plan(void* plan, size_t plan_bytes, const int32_t* ids,
   const PlanArgs a = plan_parts_of(plan, ids, pairs, experts);
   hipStream_t s = (hipStream_t)stream;
   if (a.blocks > 1) moe_count_kernel<<<dim3((unsigned)a.blocks), dim3(256), 0, s>>>(a);
-  moe_place_kernel<<<dim3((unsigned)a.blocks), dim3(1024), 0, s>>>(a);
+  const dim3 grid((unsigned)a.blocks), block(1024);
+  if (a.tile_rows == 64) moe_place_kernel<64><<<grid, block, 0, s>>>(a);
+  else if (a.tile_rows == 128) moe_place_kernel<128><<<grid, block, 0, s>>>(a);
+  else moe_place_kernel<256><<<grid, block, 0, s>>>(a);
   return launch_status();
 }
 

@@ -85,6 +85,13 @@ def test_fused_outputs_and_store(dtype, hq, hkv, d, norm):
     assert torch.equal(vc.cpu().view(torch.uint8), ref_v.view(torch.uint8))
 
 
+@pytest.mark.parametrize("d", [16, 24, 40, 72, 136, 264, 320, 512])
+@pytest.mark.parametrize("norm", [True, False])
+def test_sums_over_every_number_of_lanes(d, norm):
+    """2 to 64 lanes of 4 elements and 2 to 32 of 8 per vector, and lanes past the vector's end."""
+    test_fused_outputs_and_store(torch.bfloat16, 3, 2, d, norm)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (2, 1, 96)])
 def test_fused_int8_cache_bit_exact(dtype, hq, hkv, d):
