@@ -140,12 +140,12 @@ PyObject* store(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// decode(query, k_cache, v_cache, k_scale or None, v_scale or None, block_tables, context_lens, scale, heads, kv_heads, head_dim, block_size,
-//        workspace or None, the device's workspace or None) -> result
-PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
+// decode(query, k_cache, v_cache, None, None, block_tables, context_lens, scale, heads, kv_heads, head_dim, block_size, workspace or None,
+//        the device's workspace or None) -> result
+// decode_int8(query, k_cache, v_cache, k_scale, v_scale, ...): which of the two it is says the operator, not what it was given as scales
+template <bool int8> PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 14 || !lib.decode || !ordinary()) return none();
-  const bool int8 = a[3] != Py_None;
+  if (n != 14 || !lib.decode || !ordinary() || (!int8 && (a[3] != Py_None || a[4] != Py_None))) return none();
   const at::Tensor *q = dense(a[0]), *k = dense(a[1]), *v = dense(a[2]), *tables = dense(a[5], at::kInt), *lens = dense(a[6]);
   const at::Tensor *ks = int8 ? dense(a[3], at::kFloat) : nullptr, *vs = int8 ? dense(a[4], at::kFloat) : nullptr;
   double scale;
@@ -441,7 +441,8 @@ PyObject* bind(PyObject*, PyObject* of) {
 
 PyMethodDef methods[] = {{"bind", bind, METH_O, nullptr},
                          {"store", (PyCFunction)(void*)store, METH_FASTCALL, nullptr},
-                         {"decode", (PyCFunction)(void*)decode, METH_FASTCALL, nullptr},
+                         {"decode", (PyCFunction)(void*)decode<false>, METH_FASTCALL, nullptr},
+                         {"decode_int8", (PyCFunction)(void*)decode<true>, METH_FASTCALL, nullptr},
                          {"prefill", (PyCFunction)(void*)prefill, METH_FASTCALL, nullptr},
                          {"prefill_paged", (PyCFunction)(void*)prefill_paged, METH_FASTCALL, nullptr},
                          {"window_prefill", (PyCFunction)(void*)window_prefill, METH_FASTCALL, nullptr},

@@ -549,8 +549,8 @@ def paged_attention_decode_int8(query: torch.Tensor, k_cache: torch.Tensor, v_ca
     """Paged decode over an int8 cache written by ``store_kvcache_int8`` (``workspace`` as in
     ``paged_attention_decode``)."""
     if _C.calls is not None:
-        done = _C.calls.decode(query, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens, scale, num_heads, num_kv_heads, head_dim,
-                               block_size, workspace, _workspaces.get(query.device.index))
+        done = _C.calls.decode_int8(query, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens, scale, num_heads, num_kv_heads,
+                                    head_dim, block_size, workspace, _workspaces.get(query.device.index))
         if done is not None:
             return done
     _C.require_cuda(query, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens)

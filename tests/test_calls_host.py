@@ -20,11 +20,12 @@ def test_calls_decline_what_is_not_theirs(calls):
     for q in (x, None, 3, "x", x.half(), torch.nn.Parameter(x)):
         assert calls.store(q, x, cache, cache, i) is False
         assert calls.decode(q, cache, cache, None, None, cu[None], i, 1.0, 2, 2, 64, 16, None, None) is None
+        assert calls.decode_int8(q, cache, cache, None, None, cu[None], i, 1.0, 2, 2, 64, 16, None, None) is None
         assert calls.prefill(q, x, x, cu, 1.0, 2, 2, 64, None, plan, None, 1 << 30) is None
         assert calls.prefill(q, x, x, cu, 1.0, 2, 2, 64, None, plan, None, 1 << 30, x, x, cu) is None
         assert calls.prefill_paged(q, cache, cache, cu[None], cu, cu, 1.0, 2, 2, 64, 16, 3, plan, None, 1 << 30) is None
         assert calls.window_prefill(q, q, x, cu, cu, 1.0, 0, None, x, None, None, None, 0.0, 0) is False
-    assert calls.store() is False and calls.store(x) is False and calls.decode(x) is None and calls.prefill() is None
+    assert calls.store() is False and calls.store(x) is False and calls.decode(x) is None and calls.decode_int8(x) is None and calls.prefill() is None
     assert calls.prefill_paged(x) is None and calls.window_prefill(x) is False                 # numbers of arguments
     with pytest.raises(TypeError):
         calls.bind([1])

@@ -99,6 +99,20 @@ def test_decode_int8(counted, monkeypatch, lengths, block):
             attention.paged_attention_decode_int8(*wrong)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.int8])
+def test_decode_int8_without_scales_is_refused(counted, dtype):
+    """What is missing does not make the call one of the other operator's, whose caches would fit."""
+    tables, (k, v), scales = paged([40, 17], 16, 2, 128, dtype, int8=dtype == torch.int8)
+    ks, vs = scales or [torch.ones(k.shape[:3], device=DEV) for _ in range(2)]
+    q, rest = normal(2, 4, 128, dtype=torch.bfloat16 if dtype == torch.int8 else dtype), (tables, torch.tensor([40, 17], device=DEV), 0.1, 4, 2, 128, 16)
+    for given in ((None, None), (ks, None), (None, vs)):
+        with pytest.raises((ValueError, AttributeError)):
+            attention.paged_attention_decode_int8(q, k, v, *given, *rest)
+        assert counted.calls.decode_int8(q, k, v, *given, *rest, None, None) is None
+        assert given == (None, None) or counted.calls.decode(q, k, v, *given, *rest, None, None) is None
+    assert counted.taken == 0
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("lengths", [[1], [40, 7], [900, 300]])
 def test_prefill_and_store(counted, monkeypatch, dtype, lengths):
