@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 import torch
 
@@ -197,7 +198,7 @@ def use_library(path: str) -> None:
 
 def load():
     """Load the shared library once; raise if it has not been built."""
-    global _lib
+    global _lib, calls
     if _lib is not None:
         return _lib
     path = _partial or _LIB_PATH
@@ -212,17 +213,23 @@ def load():
         fn = getattr(lib, name)      # AttributeError if the symbol is missing
         fn.restype = restype
         fn.argtypes = argtypes
-    _lib = lib
-    _bind_calls(lib)
+    calls = _bind_calls(lib)
+    _lib = lib                       # last: whoever finds the library finds the calls as they stay
     return lib
 
 
 def _bind_calls(lib):
-    global calls
-    if os.path.exists(os.path.join(os.path.dirname(_LIB_PATH), "_calls.so")):
+    """csrc/calls.cpp with its entry points from ``lib``; None where it has not been built or cannot be used here (a module for
+    another torch or Python): then the operators go their longer way, every time alike."""
+    if not os.path.exists(os.path.join(os.path.dirname(_LIB_PATH), "_calls.so")):
+        return None
+    try:
         from minivllm_amd import _calls
-        _calls.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES if hasattr(lib, name)})
-        calls = _calls
+    except ImportError as error:
+        warnings.warn(f"minivllm_amd: _calls.so cannot be used ({error}); attention operators take longer on the host", RuntimeWarning, stacklevel=3)
+        return None
+    _calls.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES if hasattr(lib, name)})
+    return _calls
 
 
 def check(status: int, what: str) -> None:

@@ -29,3 +29,22 @@ def test_calls_decline_what_is_not_theirs(calls):
     assert calls.prefill_paged(x) is None and calls.window_prefill(x) is False                 # numbers of arguments
     with pytest.raises(TypeError):
         calls.bind([1])
+
+
+def _loaded_again(monkeypatch):
+    """The binding as it is before the library is first asked for."""
+    for name in ("_lib", "calls"):
+        monkeypatch.setattr(_C, name, None)
+
+
+def test_a_module_that_cannot_be_imported_is_declined_every_time(calls, monkeypatch):
+    import sys
+
+    import minivllm_amd
+    _loaded_again(monkeypatch)
+    monkeypatch.setitem(sys.modules, "minivllm_amd._calls", None)          # as one built for another torch or Python
+    monkeypatch.delattr(minivllm_amd, "_calls")
+    with pytest.warns(RuntimeWarning, match="_calls"):
+        first = _C.load()
+    assert first.mvllm_version() >= 1000 and _C.calls is None
+    assert _C.load() is first and _C.calls is None
