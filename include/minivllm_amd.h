@@ -47,6 +47,9 @@ enum mvllm_status {
 /* ABI version: major*1000 + minor. */
 int mvllm_version(void);
 
+/* Digest of this header and of csrc/calls.cpp as the library was built ("": not by the package's own build).  HOST pointer. */
+const char* mvllm_calls_digest(void);
+
 /* Static, human-readable text for a status returned by this library
  * (negative codes only; positive codes are hipError_t). HOST pointer. */
 const char* mvllm_status_string(int status);

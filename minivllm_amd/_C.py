@@ -25,6 +25,7 @@ c_uint64 = ctypes.c_uint64
 # name -> (restype, argtypes); mirrors include/minivllm_amd.h one to one
 SIGNATURES = {
     "mvllm_version": (c_int, []),
+    "mvllm_calls_digest": (ctypes.c_char_p, []),
     "mvllm_status_string": (ctypes.c_char_p, [c_int]),
     "mvllm_store_kvcache": (c_int, [c_void_p] * 5 + [c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
     "mvllm_store_kvcache_int8": (c_int, [c_void_p] * 7 + [c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
@@ -220,16 +221,18 @@ def load():
 
 def _bind_calls(lib):
     """csrc/calls.cpp with its entry points from ``lib``; None where it has not been built or cannot be used here (a module for
-    another torch or Python): then the operators go their longer way, every time alike."""
+    another torch, Python or library): then the operators go their longer way, every time alike."""
     if not os.path.exists(os.path.join(os.path.dirname(_LIB_PATH), "_calls.so")):
         return None
     try:
         from minivllm_amd import _calls
-    except ImportError as error:
-        warnings.warn(f"minivllm_amd: _calls.so cannot be used ({error}); attention operators take longer on the host", RuntimeWarning, stacklevel=3)
-        return None
-    _calls.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES if hasattr(lib, name)})
-    return _calls
+        if _calls.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES if hasattr(lib, name)}):
+            return _calls
+        error = "it was built from other sources than the library"
+    except ImportError as e:
+        error = e
+    warnings.warn(f"minivllm_amd: _calls.so cannot be used ({error}); attention operators take longer on the host", RuntimeWarning, stacklevel=3)
+    return None
 
 
 def check(status: int, what: str) -> None:

@@ -46,7 +46,18 @@ def _hipcc() -> str:
     return exe
 
 
+def calls_digest() -> str:
+    """Of what csrc/calls.cpp calls the library as: compiled into both, so that neither is used with another build's."""
+    digest = hashlib.sha1()
+    for path in (os.path.join(os.path.dirname(PKG_DIR), "include", "minivllm_amd.h"), os.path.join(CSRC, "calls.cpp")):
+        with open(path, "rb") as f:
+            digest.update(f.read())
+    return digest.hexdigest()
+
+
 def _compile(src, verbose, extra=(), suffix=""):
+    if src == "capi.hip":
+        extra = (*extra, f'-DMVLLM_CALLS_DIGEST="{calls_digest()}"')
     obj_dir = os.path.join(PKG_DIR, "build")
     os.makedirs(obj_dir, exist_ok=True)
     obj = os.path.join(obj_dir, src.replace(".hip", suffix + ".o"))
@@ -82,7 +93,7 @@ def _build_calls(verbose):
     include = [os.path.join(os.path.dirname(PKG_DIR), "include"), os.path.join(home, "include"),
                os.path.join(home, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-I" + i for i in include),
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DMVLLM_CALLS_DIGEST="{calls_digest()}"', *("-I" + i for i in include),
            os.path.join(CSRC, "calls.cpp"), "-o", part, "-L" + os.path.join(home, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10_hip", "-lc10"]
     if verbose:
         print(" ".join(cmd), flush=True)

@@ -410,11 +410,25 @@ PyObject* window_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind({name: address}) of the loaded library's entry points; those that are missing stay unused
+// What the addresses are called as is this file's, compiled with a header: only a library built with the same two is called.
+#ifndef MVLLM_CALLS_DIGEST
+#define MVLLM_CALLS_DIGEST ""
+#endif
+bool same_build(PyObject* of) {
+  PyObject* at = PyDict_GetItemString(of, "mvllm_calls_digest");
+  auto digest = at ? reinterpret_cast<decltype(&mvllm_calls_digest)>(PyLong_AsVoidPtr(at)) : nullptr;
+  return digest && MVLLM_CALLS_DIGEST[0] != 0 && std::strcmp(digest(), MVLLM_CALLS_DIGEST) == 0;
+}
+
+// bind({name: address}) of the loaded library's entry points, those that are missing stay unused -> whether it is this module's library
 PyObject* bind(PyObject*, PyObject* of) {
   if (!PyDict_Check(of)) {
     PyErr_SetString(PyExc_TypeError, "a dict of addresses");
     return nullptr;
+  }
+  if (!same_build(of)) {
+    if (PyErr_Occurred()) return nullptr;
+    return no();
   }
   auto set = [&](const char* name, auto& f) {
     PyObject* at = PyDict_GetItemString(of, name);
@@ -436,7 +450,7 @@ PyObject* bind(PyObject*, PyObject* of) {
   if (!lib.decode_int8 || !lib.decode_bytes || !lib.decode_plan) lib.decode = nullptr;
   if (!lib.prefill_plan || !lib.prefill_ranges || !lib.prefill_f32_ranges || !lib.split_plan) lib.prefill = nullptr, lib.prefill_paged = nullptr;
   if (PyErr_Occurred()) return nullptr;
-  Py_RETURN_NONE;
+  Py_RETURN_TRUE;
 }
 
 PyMethodDef methods[] = {{"bind", bind, METH_O, nullptr},

@@ -3,6 +3,11 @@
 
 extern "C" int mvllm_version(void) { return 1 * 1000 + 7; }
 
+#ifndef MVLLM_CALLS_DIGEST
+#define MVLLM_CALLS_DIGEST ""
+#endif
+extern "C" const char* mvllm_calls_digest(void) { return MVLLM_CALLS_DIGEST; }
+
 extern "C" const char* mvllm_status_string(int status) {
   switch (status) {
     case MVLLM_OK: return "ok";

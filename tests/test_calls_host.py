@@ -1,8 +1,11 @@
 """The native way to the attention operators (csrc/calls.cpp) on the CPU: it takes nothing that is not a plain tensor on a GPU, and says so."""
+import ctypes
+import types
+
 import pytest
 import torch
 
-from minivllm_amd import _C
+from minivllm_amd import _build, _C
 
 
 @pytest.fixture(scope="module")
@@ -48,3 +51,19 @@ def test_a_module_that_cannot_be_imported_is_declined_every_time(calls, monkeypa
         first = _C.load()
     assert first.mvllm_version() >= 1000 and _C.calls is None
     assert _C.load() is first and _C.calls is None
+
+
+def test_a_module_of_another_build_is_declined(calls, monkeypatch):
+    """The library's and the module's digests of the header and of calls.cpp: others, or none, and nothing is bound."""
+    lib = _C.load()
+    assert lib.mvllm_calls_digest().decode() == _build.calls_digest()
+    names = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _C.SIGNATURES}
+    for text in (b"", b"another", _build.calls_digest()[:-1].encode()):
+        held = ctypes.create_string_buffer(text)
+        digest = ctypes.CFUNCTYPE(ctypes.c_void_p)(lambda: ctypes.addressof(held))
+        assert calls.bind({**names, "mvllm_calls_digest": ctypes.cast(digest, ctypes.c_void_p).value}) is False
+    del names["mvllm_calls_digest"]
+    assert calls.bind(names) is False
+    with pytest.warns(RuntimeWarning, match="_calls"):
+        assert _C._bind_calls(types.SimpleNamespace(mvllm_calls_digest=digest)) is None
+    assert _C._bind_calls(lib) is calls
