@@ -67,3 +67,36 @@ def test_a_module_of_another_build_is_declined(calls, monkeypatch):
     with pytest.warns(RuntimeWarning, match="_calls"):
         assert _C._bind_calls(types.SimpleNamespace(mvllm_calls_digest=digest)) is None
     assert _C._bind_calls(lib) is calls
+
+
+def test_a_build_that_fails_leaves_the_module_that_was_there(tmp_path, monkeypatch):
+    """A kernel that does not compile, or a link that fails: neither file is replaced.  A module that does not compile: the library is
+    there without one."""
+    here = tmp_path / "_calls.so"
+    here.write_text("before")
+    monkeypatch.setattr(_build, "CALLS_PATH", str(here))
+
+    def run(**steps):
+        def built(_):
+            (tmp_path / "part").write_text("built")
+            return str(tmp_path / "part")
+        for name, step in {"_compile": lambda src, *a: src, "_link": lambda *a: None, "_build_calls": built, **steps}.items():
+            monkeypatch.setattr(_build, name, step)
+        return _build.build_library(verbose=False, jobs=2)
+
+    def broken(*a):
+        raise RuntimeError("broken")
+
+    compile_calls = _build._build_calls
+    for name in ("_compile", "_link"):
+        with pytest.raises(RuntimeError, match="broken"):
+            run(**{name: broken})
+        assert here.read_text() == "before"
+    assert run() == _build.LIB_PATH and here.read_text() == "built"
+    monkeypatch.setenv("CXX", "false")
+    with pytest.warns(RuntimeWarning, match="calls.cpp"):
+        run(_build_calls=compile_calls)
+    assert not here.exists()
+    monkeypatch.setenv("CXX", str(tmp_path / "there is none"))
+    with pytest.warns(RuntimeWarning, match="calls.cpp"):
+        run(_build_calls=compile_calls)
