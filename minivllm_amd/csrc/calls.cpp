@@ -140,12 +140,11 @@ PyObject* store(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// decode(query, k_cache, v_cache, None, None, block_tables, context_lens, scale, heads, kv_heads, head_dim, block_size, workspace or None,
-//        the device's workspace or None) -> result
+// decode(query, k_cache, v_cache, None, None, block_tables, context_lens, scale, heads, kv_heads, head_dim, block_size, workspace or None) -> result
 // decode_int8(query, k_cache, v_cache, k_scale, v_scale, ...): which of the two it is says the operator, not what it was given as scales
 template <bool int8> PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 14 || !lib.decode || !ordinary() || (!int8 && (a[3] != Py_None || a[4] != Py_None))) return none();
+  if (n != 13 || !lib.decode || !ordinary() || (!int8 && (a[3] != Py_None || a[4] != Py_None))) return none();
   const at::Tensor *q = dense(a[0]), *k = dense(a[1]), *v = dense(a[2]), *tables = dense(a[5], at::kInt), *lens = dense(a[6]);
   const at::Tensor *ks = int8 ? dense(a[3], at::kFloat) : nullptr, *vs = int8 ? dense(a[4], at::kFloat) : nullptr;
   double scale;
@@ -166,16 +165,11 @@ template <bool int8> PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t 
   int part_tokens, parts, waves = 0;      // (shapes without a tiled kernel are warned of)
   if (lib.decode_plan(1, heads, kv_heads, dim, 1, block, code, int8, &part_tokens, &parts, &waves) != MVLLM_OK || waves == 0) return none();
   const size_t need = lib.decode_bytes((int)batch, heads, dim, most, block);
-  const at::Tensor* space = nullptr;
-  if (need > 0) {
-    for (int i = 12; i < 14 && !space; ++i) {
-      if (a[i] == Py_None) continue;
-      const at::Tensor* t = dense(a[i], at::kByte);
-      if (!t) return none();
-      if ((size_t)t->numel() >= need) space = t;
-    }
-    if (!space) return none();
-  }
+  // the caller's workspace where it is one and large enough, else one of this call's, on its stream like the result
+  const at::Tensor* space = need > 0 && a[12] != Py_None ? dense(a[12], at::kByte) : nullptr;
+  if (need > 0 && a[12] != Py_None && !space) return none();
+  at::Tensor own;
+  if (need > 0 && (!space || (size_t)space->numel() < need)) space = &(own = at::empty({(int64_t)need}, q->options().dtype(at::kByte)));
   at::Tensor out = at::empty_like(*q);
   void *stream = stream_of(*q), *ws = space ? space->data_ptr() : nullptr;
   const size_t bytes = space ? (size_t)space->numel() : 0;

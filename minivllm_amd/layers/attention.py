@@ -29,26 +29,16 @@ __all__ = [
     "prefill_plan", "Attention",
 ]
 
-_workspaces: dict = {}   # device index -> uint8 tensor reused by decode calls on that device that bring no workspace
-_retired: list = []      # outgrown workspaces: kept alive, because a captured hipGraph may hold their address
-
 
 def _decode_workspace(device: torch.device, nbytes: int, own: torch.Tensor | None = None):
     """Split-K scratch for paged decode.  ``own`` (a caller-owned uint8 tensor, e.g. the model runner's, sized
-    before its graphs were captured) is used when it is large enough; otherwise one buffer per device, grown on
-    demand and never freed: a buffer that has been handed out may be referenced by a captured graph."""
+    before its graphs were captured) is used when it is large enough; otherwise a tensor of this call's, on its stream like the
+    result: calls on other streams and threads have their own, and a captured graph's is in the graph's pool."""
     if nbytes == 0:
         return None
     if own is not None and own.numel() >= nbytes:
         return own
-    key = device.index if device.index is not None else torch.cuda.current_device()
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        if ws is not None:
-            _retired.append(ws)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+    return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
 
 def decode_workspace_bytes(batch: int, num_heads: int, head_dim: int, max_num_blocks: int, block_size: int) -> int:
@@ -503,12 +493,12 @@ def paged_attention_decode(query: torch.Tensor, k_cache: torch.Tensor, v_cache: 
     block_tables int32 (batch, max_num_blocks), -1 padded; context_lens int32 or
     int64 (batch,).  Returns a tensor like query; rows with context_len 0 are zeros.
     ``workspace`` (optional, not in the reference): a uint8 device tensor the caller owns for the split-K
-    partials; without it, or when it is too small, a per-device buffer of this module is used.  ``sink`` and ``out`` as in
+    partials; without it, or when it is too small, the call allocates its own.  ``sink`` and ``out`` as in
     ``flash_attention_prefill``.
     """
     if _C.calls is not None and sink is None and out is None:
         done = _C.calls.decode(query, k_cache, v_cache, None, None, block_tables, context_lens, scale, num_heads, num_kv_heads, head_dim,
-                               block_size, workspace, _workspaces.get(query.device.index))
+                               block_size, workspace)
         if done is not None:
             return done
     _C.require_cuda(query, k_cache, v_cache, block_tables, context_lens)
@@ -550,7 +540,7 @@ def paged_attention_decode_int8(query: torch.Tensor, k_cache: torch.Tensor, v_ca
     ``paged_attention_decode``)."""
     if _C.calls is not None:
         done = _C.calls.decode_int8(query, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens, scale, num_heads, num_kv_heads,
-                                    head_dim, block_size, workspace, _workspaces.get(query.device.index))
+                                    head_dim, block_size, workspace)
         if done is not None:
             return done
     _C.require_cuda(query, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens)

@@ -22,8 +22,8 @@ def test_calls_decline_what_is_not_theirs(calls):
     plan = lambda *a: pytest.fail("asked for a plan")
     for q in (x, None, 3, "x", x.half(), torch.nn.Parameter(x)):
         assert calls.store(q, x, cache, cache, i) is False
-        assert calls.decode(q, cache, cache, None, None, cu[None], i, 1.0, 2, 2, 64, 16, None, None) is None
-        assert calls.decode_int8(q, cache, cache, None, None, cu[None], i, 1.0, 2, 2, 64, 16, None, None) is None
+        assert calls.decode(q, cache, cache, None, None, cu[None], i, 1.0, 2, 2, 64, 16, None) is None
+        assert calls.decode_int8(q, cache, cache, None, None, cu[None], i, 1.0, 2, 2, 64, 16, None) is None
         assert calls.prefill(q, x, x, cu, 1.0, 2, 2, 64, None, plan, None, 1 << 30) is None
         assert calls.prefill(q, x, x, cu, 1.0, 2, 2, 64, None, plan, None, 1 << 30, x, x, cu) is None
         assert calls.prefill_paged(q, cache, cache, cu[None], cu, cu, 1.0, 2, 2, 64, 16, 3, plan, None, 1 << 30) is None
@@ -100,3 +100,29 @@ def test_a_build_that_fails_leaves_the_module_that_was_there(tmp_path, monkeypat
     monkeypatch.setenv("CXX", str(tmp_path / "there is none"))
     with pytest.warns(RuntimeWarning, match="calls.cpp"):
         run(_build_calls=compile_calls)
+
+
+def test_decodes_that_overlap_have_a_workspace_each(monkeypatch):
+    """Another thread's decode, on a stream of its own, while the first one's kernels may still run: its partial results lie elsewhere."""
+    from minivllm_amd.layers import attention
+    places = []
+
+    def kernels(*args):
+        places.append((args[-3], args[-2]))
+        if len(places) == 1:
+            decode()
+        return 0
+
+    lib = types.SimpleNamespace(mvllm_paged_decode=kernels, mvllm_paged_decode_int8=kernels, mvllm_paged_decode_workspace_bytes=lambda *sizes: 1 << 20)
+    for name, to in {"calls": None, "load": lambda: lib, "require_cuda": lambda *t: None, "current_stream_ptr": lambda d: 0}.items():
+        monkeypatch.setattr(_C, name, to)
+    monkeypatch.setattr(attention, "_warn_if_generic", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    q, cache, codes, scales = torch.zeros(2, 4, 64), torch.zeros(4, 16, 2, 64), torch.zeros(4, 16, 2, 64, dtype=torch.int8), torch.ones(4, 16, 2)
+    tables, rest = torch.zeros(2, 2, dtype=torch.int32), (torch.tensor([20, 30]), 1.0, 4, 2, 64, 16)
+    for decode in (lambda: attention.paged_attention_decode(q, cache, cache, tables, *rest),
+                   lambda: attention.paged_attention_decode_int8(q, codes, codes, scales, scales, tables, *rest)):
+        places.clear()
+        decode()
+        (first, n), (second, m) = places
+        assert n >= 1 << 20 and m >= 1 << 20 and (first + n <= second or second + m <= first)

@@ -72,7 +72,6 @@ def test_decode(counted, monkeypatch, dtype, lengths, block):
     q = normal(len(lengths), 8, 64, dtype=dtype)
     for lens in (torch.tensor(lengths, device=DEV), torch.tensor(lengths, dtype=torch.int32, device=DEV)):
         args = (q, k, v, tables, lens, 0.125, 8, 2, 64, block)
-        attention.paged_attention_decode(*args)                          # (the device's workspace has its size)
         both(counted, monkeypatch, lambda: attention.paged_attention_decode(*args), 1)
     need = attention.decode_workspace_bytes(len(lengths), 8, 64, tables.shape[1], block)
     own = torch.empty(need + 16, dtype=torch.uint8, device=DEV)
@@ -88,11 +87,40 @@ def test_decode(counted, monkeypatch, dtype, lengths, block):
     assert counted.taken == 0
 
 
+def test_decodes_on_two_streams_without_a_workspace(counted):
+    """Partial results of calls that run side by side do not meet; captured calls keep theirs in the graph's pool."""
+    cases, streams = [], [torch.cuda.Stream() for _ in range(2)]
+    for lengths, heads in (([9000, 4000, 7000], 8), ([6000, 8500], 4)):
+        tables, (k, v), _ = paged(lengths, 16, 2, 64, torch.bfloat16)
+        args = (normal(len(lengths), heads, 64), k, v, tables, torch.tensor(lengths, device=DEV), 0.125, heads, 2, 64, 16)
+        own = torch.empty(attention.decode_workspace_bytes(len(lengths), heads, 64, tables.shape[1], 16), dtype=torch.uint8, device=DEV)
+        cases.append((args, attention.paged_attention_decode(*args, workspace=own)))
+    assert all(attention.paged_decode_plan(*(c[0][0].shape[0], c[0][6], 2, 64, c[0][3].shape[1], 16))[1] > 1 for c in cases)
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(20):
+        for i, stream in enumerate(streams):
+            with torch.cuda.stream(stream):
+                got[i].append(attention.paged_attention_decode(*cases[i][0]))
+    torch.cuda.synchronize()
+    for results, (_, want) in zip(got, cases):
+        assert all(torch.equal(r, want) for r in results)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = attention.paged_attention_decode(*cases[0][0])
+    for _ in range(3):
+        captured.zero_()
+        graph.replay()
+        other = attention.paged_attention_decode(*cases[1][0])
+        torch.cuda.synchronize()
+        assert torch.equal(captured, cases[0][1]) and torch.equal(other, cases[1][1])
+    assert counted.taken == 2 + 40 + 1 + 3
+
+
 @pytest.mark.parametrize("lengths,block", [([5], 16), ([300, 1, 77], 32)])
 def test_decode_int8(counted, monkeypatch, lengths, block):
     tables, (k, v), (ks, vs) = paged(lengths, block, 2, 128, None, int8=True)
     args = (normal(len(lengths), 4, 128), k, v, ks, vs, tables, torch.tensor(lengths, device=DEV), 0.1, 4, 2, 128, block)
-    attention.paged_attention_decode_int8(*args)
     both(counted, monkeypatch, lambda: attention.paged_attention_decode_int8(*args), 1)
     for wrong in ((*args[:3], ks.half(), *args[4:]), (*args[:4], vs[:, :1], *args[5:]), (args[0], k.float(), *args[2:])):
         with pytest.raises(ValueError):
@@ -108,8 +136,8 @@ def test_decode_int8_without_scales_is_refused(counted, dtype):
     for given in ((None, None), (ks, None), (None, vs)):
         with pytest.raises((ValueError, AttributeError)):
             attention.paged_attention_decode_int8(q, k, v, *given, *rest)
-        assert counted.calls.decode_int8(q, k, v, *given, *rest, None, None) is None
-        assert given == (None, None) or counted.calls.decode(q, k, v, *given, *rest, None, None) is None
+        assert counted.calls.decode_int8(q, k, v, *given, *rest, None) is None
+        assert given == (None, None) or counted.calls.decode(q, k, v, *given, *rest, None) is None
     assert counted.taken == 0
 
 
