@@ -90,7 +90,8 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_f32_kernel(const Pre
   const int pos0 = cached + r0;                                       // position of that row among the keys
   const int j_last = min(pos0 + kWaveRows - 1, kv_len - 1) / kF32Keys;   // last tile any row of the wave sees
   const int wg_last = min(row0 + BM, seq_len) - 1;
-  int ntiles = (cached + wg_last) / kF32Keys + 1;                     // tiles the workgroup walks: [t0, ntiles)
+  // tiles the workgroup walks: [t0, ntiles); with fewer keys than rows those that have keys, as the merge counts them
+  int ntiles = min((cached + wg_last) / kF32Keys, (kv_len - 1) / kF32Keys) + 1;
   const int t0 = RANGES ? (int)blockIdx.y * a.range_tiles : 0;
   const bool in_ranges = RANGES && gridDim.y > 1 && ntiles > a.range_tiles;
   if constexpr (RANGES) {

@@ -148,3 +148,19 @@ def test_fp32_ranges_plan_and_rejections():
     p = q.data_ptr()
     args = lambda tiles, nbytes, dim=64, ws=p: (p, p, p, p, 0, 0, cu.data_ptr(), 0, 1, 64, 64, 8, 8, dim, 0, 0, 1.0, 0, tiles, ws, nbytes, 0)
     assert bad(*args(1, 0)) == -5 and bad(*args(1, 1 << 20, ws=0)) == -5 and bad(*args(0, 1 << 20)) == -3 and bad(*args(1, 1 << 20, dim=80)) == -4
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (4, 2, 128), (3, 3, 64)])
+@pytest.mark.parametrize("tiles", [1, 2, 4])
+def test_fp32_ranges_with_fewer_keys_than_rows(hq, hkv, d, tiles, monkeypatch):
+    """Paged sequences of more rows than keys: kernel and merge take the same row tiles for cut ones, and every row is written."""
+    keys, rows = [64, 33, 200, 0, 300, 128], [300, 70, 65, 33, 310, 129]
+    c = make_paged_prefill_case(29, keys, [0] * len(keys), hq, hkv, d, 16, dtype=torch.float32)
+    c["q_new"] = torch.randn(sum(rows), hq, d, generator=torch.Generator().manual_seed(3))
+    c["cu_q"] = torch.tensor([0, *torch.tensor(rows).cumsum(0).tolist()], dtype=torch.int32)
+    monkeypatch.setattr(attention, "_prefill_ranges_plan", lambda lib, s, t, k, hq, hkv, d, bs, code: (
+        tiles, lib.mvllm_prefill_f32_ranges_workspace_bytes(t, k, hq, d, tiles)))
+    got = _run(c, hq, hkv, d, 16, tiles, max(keys), True)
+    whole = attention.flash_attention_prefill_paged(*(c[n].to(DEV) for n in ("q_new", "k_cache", "v_cache", "block_tables", "cu_q", "cu_k")),
+                                                    d ** -0.5, hq, hkv, d, 16).cpu()
+    assert torch.isfinite(got).all() and ((got - whole).norm() / whole.norm()).item() <= 2e-6
