@@ -146,7 +146,9 @@ constexpr int kSplitNarrowCtx = 2048, kSplitOnePartPairs = 256;
 // 23 of up to 4054 in full tables 66 / 52, 46 of 7549 203 / 173, 17 of 14057 182 / 137, 9 of 19713 heads of 64 116 / 84, INT8 26 of 17625 110 / 84, 43 of
 // 7784 heads of 64 108 / 64; all as long as the table 24 of 8191 164 / 142; contexts of a quarter of the table 24 of 4071 in 8192 74 / 52, of an
 // eighth 20.7 / 21.7; fp32, 45 of up to 6000 271 / 184.  Finer still costs even batches (partials, start-up): INT8, 20 of 4999 50 / 52 / 61 with 4 / 8 / 20 partitions.
-// A batch whose partitions are exactly kSplitMinGroups workgroups, an even round, keeps them: 16 of 8191 in 8192 85 / 86, heads of 64 49 / 54 (16 of 512 to 8094 57 / 37).
+// Long partitions that are one even round (16 sequences of 8 kv heads in 4, 512 workgroups) are no exception.  us, long / finer, contexts spread over the
+// logarithm of a sixteenth of the table to all of it: 8 in 16384 57 / 50, 16 in 8192 55 / 35, in 16384 105 / 68, 32 in 4096 56 / 42, heads of 64 39 / 29, 40 / 24, 71 /
+// 37, 39 / 22, INT8 51 / 41, 52 / 39, 93 / 49, 49 / 31; all as long as the table 82 / 90, 82 / 85, 175 / 179, 82 / 84, 47 / 56, 47 / 51, 87 / 93, 47 / 50, 58 / 69, 59 / 65, 107 / 117, 57 / 63.
 constexpr int kSplitFineCtx = 2304, kSplitFineParts = 16, kSplitFinePart = 512, kSplitFineGroups = 1536;
 inline bool split_wanted(int64_t max_ctx, int batch, int num_kv_heads, bool int8) {
   const int part = partition_tokens_for(max_ctx, batch);
@@ -180,7 +182,7 @@ inline int split_partition_tokens(int64_t max_ctx, int batch, int num_kv_heads, 
   const int64_t floor_part = partition_tokens_for(max_ctx, batch);
   part = part < floor_part ? floor_part : part;
   const int64_t parts = (max_ctx + part - 1) / part;
-  if (max_ctx >= kSplitFineCtx && parts > 1 && pairs * parts != kSplitMinGroups)
+  if (max_ctx >= kSplitFineCtx && parts > 1)
     for (int64_t n = 4; n <= kSplitFineParts; n *= 2) {
       const int64_t finer = ((max_ctx + n - 1) / n + 63) / 64 * 64;
       if (finer < kSplitFinePart) break;

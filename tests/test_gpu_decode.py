@@ -286,7 +286,8 @@ def test_both_grid_forms_vs_oracle(dtype, hq, hkv, bs, d, form):
     (24, [8192, 1024, 1025, 1], 8192, 128, torch.bfloat16, (1024, 8, 4)), (9, [4160, 512, 575, 513], 4160, 64, torch.float16, (576, 8, 4)),   # finer
     (31, [2304, 576, 577], 2304, 128, torch.bfloat16, (576, 4, 4)), (31, [2288, 763, 705], 2288, 128, torch.bfloat16, (768, 3, 4)),   # from 2304 tokens on
     (33, [8200, 4100, 2112, 2113], 8208, 128, torch.bfloat16, (1088, 8, 4)), (49, [4096, 17, 1024], 4096, 64, torch.float32, (1024, 4, 4)),
-    (16, [8192, 2048, 2049], 8192, 64, torch.bfloat16, (2048, 4, 4)),                                                     # an even round stays
+    (16, [8192, 2048, 2049], 8192, 64, torch.bfloat16, (512, 16, 4)), (15, [8192, 512], 8192, 64, torch.bfloat16, (512, 16, 4)),      # an even round, and not
+    (32, [4096, 2049], 4096, 128, torch.bfloat16, (512, 8, 4)), (33, [4096, 513], 4096, 128, torch.bfloat16, (512, 8, 4)),
 ])
 def test_partitions_of_wide_tables(batch, first, tokens, d, dtype, plan):
     hq, hkv, bs = 16, 8, 16
