@@ -1,13 +1,13 @@
 #!/usr/bin/env python3
 """Benchmark of the paged-attention hot path on one MI355X.
 
-Prints ONE JSON line.  The headline (`metric`/`value`) is BASELINE.json config 3:
-paged-attention decode, batch 256, context lengths log-uniform in [128, 32768],
-32 query heads / 8 KV heads / head_dim 128, bf16 cache, block_size 16, reported
+Prints ONE JSON line.  The headline (`metric`/`value`) is paged-attention decode, batch 256, context lengths log-uniform
+in [128, 32768], 32 query heads / 8 KV heads / head_dim 128, bf16 cache, block_size 16, reported
 as algorithmic HBM GB/s.  A "step" is one decode call over the whole batch with
-all inputs resident in HBM.  `extra` carries the other measured workloads
-(decode at block_size 256, varlen prefill TFLOP/s and store_kvcache GB/s on
-config 2, the INT8 cache path of config 4, the engine generate loop of config 5).  `cpu_baseline` times the CPU oracle's naive decode on a bounded
+all inputs resident in HBM.  `extra` holds the other measured workloads
+(decode at block_size 256, varlen prefill TFLOP/s and store_kvcache GB/s on a ragged batch of prompts, the INT8 cache
+path, the engine's generate loop); where they make the line long they are written to a file (`--extra`), the line names it
+in `extra_file`, and `summary` has the figures of each.  `cpu_baseline` times the CPU oracle's naive decode on a bounded
 subset of the same batch on the host cores.
 """
 from __future__ import annotations
@@ -17,6 +17,7 @@ import json
 import math
 import os
 import sys
+import tempfile
 import time
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
@@ -29,6 +30,7 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, published
 # 2708744 KiB x 2.0 (copy-kernel calibration) fetched + 22855 KiB written.
 DECODE_TRAFFIC_BYTES_DEFAULT = int(2708744 * 2.0 * 1024 + 22855 * 1024)
 MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16, published
+MAX_LINE = 4000                # characters of the JSON line: records keep the last few thousand of an output, warnings included
 
 
 def parse_args():
@@ -43,6 +45,8 @@ def parse_args():
     ap.add_argument("--calib-copy", action="store_true",
                     help="also launch three 1 GiB device copies (reads 1 GiB, writes 1 GiB each) so a rocprofv3 "
                          "--pmc run can scale FETCH_SIZE / WRITE_SIZE against a kernel of known traffic")
+    ap.add_argument("--extra", default=os.path.join(tempfile.gettempdir(), "minivllm_amd_bench_extra.json"), metavar="FILE",
+                    help="where the other workloads' figures go when the line would be longer than %d characters with them" % MAX_LINE)
     return ap.parse_args()
 
 
@@ -1665,6 +1669,16 @@ def summary_of(line):
     return out
 
 
+def line_of(line, path):
+    """The JSON line, its `extra` in the file ``path`` where it is long."""
+    text = json.dumps(line)
+    if len(text) <= MAX_LINE:
+        return text
+    with open(path, "w") as f:
+        json.dump(line["extra"], f, indent=1)
+    return json.dumps({k: v for k, v in (*line.items(), ("extra_file", path)) if k != "extra"})
+
+
 def main():
     args = parse_args()
     if args.gpus != 1:
@@ -1770,8 +1784,8 @@ def main():
         "cpu_baseline": cpu,
         "extra": extra,
     }
-    line["summary"] = summary_of(line)     # last on purpose: a record that keeps only the end of the line keeps this
-    print(json.dumps(line))
+    line["summary"] = summary_of(line)
+    print(line_of(line, args.extra))
 
 
 if __name__ == "__main__":

@@ -73,3 +73,18 @@ def test_bench_refuses_more_than_one_gpu_and_a_machine_without_one():
         r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--steps", "1", "--warmup", "0"],
                            capture_output=True, text=True)
         assert r.returncode != 0 and "no GPU" in (r.stdout + r.stderr)
+
+
+def test_bench_line_stays_short(tmp_path):
+    """A record keeps the end of the output: with long figures of the other workloads the line names a file that has them."""
+    import json
+
+    import bench
+    file = tmp_path / "extra.json"
+    line = {"metric": "m", "value": 1.0, "extra": {"a": {"ms": 1.5}}, "summary": {"decode_gbs": 6000}}
+    assert json.loads(bench.line_of(line, str(file))) == line and not file.exists()
+    line["extra"]["probe"] = ["x" * 100] * 50
+    text = bench.line_of(line, str(file))
+    assert len(text) < bench.MAX_LINE and "\n" not in text
+    assert json.loads(text) == {"metric": "m", "value": 1.0, "summary": {"decode_gbs": 6000}, "extra_file": str(file)}
+    assert json.loads(file.read_text()) == line["extra"]
