@@ -248,7 +248,7 @@ def cpu_prefill_baseline(q, k, v, cu, lengths, scale, hq, hkv, d, flops, gpu_fn)
 
 
 def bench_prefill_store(args, which, want_cpu=False):
-    """16 prompts L~U[64,2048], Hq32/Hkv8/D128 bf16; store into a block-256 paged cache."""
+    """A ragged batch of 16 prompts L~U[64,2048], Hq32/Hkv8/D128 bf16; store into a block-256 paged cache."""
     import torch
     from helpers import make_slot_mapping
     from minivllm_amd.layers.attention import flash_attention_prefill, store_kvcache
@@ -297,7 +297,7 @@ def bench_prefill_store(args, which, want_cpu=False):
         }
         del q16
     if "prefill_long" in which:
-        # the same kernel away from config 2's short prompts: 4 prompts of 8192 tokens (the start and end of a
+        # the same kernel away from short prompts: 4 prompts of 8192 tokens (the start and end of a
         # workgroup's life are a small share of its 128 key tiles)
         long_lengths = [8192] * 4
         scale = 1.0 / math.sqrt(d)
@@ -409,7 +409,7 @@ def bench_prefill_store(args, which, want_cpu=False):
 
 
 def bench_int8(args, want_cpu=True, want_probe=False):
-    """B 128, ctx U[256,16384], Hq32/Hkv8/D128; K/V ~ N(0,1) with 1 % outliers at 8 sigma are
+    """INT8 cache, B 128, ctx U[256,16384], Hq32/Hkv8/D128; K/V ~ N(0,1) with 1 % outliers at 8 sigma are
     quantised by store_kvcache_int8 into a block-16 int8 cache, then decoded with in-kernel dequantisation."""
     import torch
     from minivllm_amd.layers.attention import paged_attention_decode_int8, store_kvcache_int8
@@ -484,7 +484,7 @@ def bench_int8(args, want_cpu=True, want_probe=False):
 
 
 def bench_fused_qk(args):
-    """The caller's chain in front of the attention kernels on the prefill batch of config 2 (same lengths):
+    """The caller's chain in front of the attention kernels on the prefill batch (same lengths):
     q/k RMSNorm + rotary embedding + store into a block-256 bf16 cache, as one HIP launch reading the packed QKV
     projection output, against the same chain as separate modules (torch ops + store_kvcache)."""
     import torch
@@ -532,7 +532,7 @@ def bench_fused_qk(args):
 
 
 def bench_sampler(args):
-    """One sampling step of config 5's decode batch: 64 rows of bf16 logits over the 151 936-token vocabulary,
+    """One sampling step of a decode batch: 64 rows of bf16 logits over the 151 936-token vocabulary,
     as one HIP launch against the module chain (fp32 softmax, exponential_, divide, argmax)."""
     import torch
     from minivllm_amd.layers.basic import Sampler
@@ -549,7 +549,7 @@ def bench_sampler(args):
     nbytes = batch * vocab * 2 + batch * 12
     out = {"workload": "sampler: 64 x 151936 bf16 logits, T 0.6", "algorithmic_bytes": nbytes,
            "event_ms_per_step": fused_ms, "gbs": nbytes / (fused_ms * 1e-3) / 1e9, "unfused_modules_event_ms": modules_ms}
-    # the LM head in front of it, config 5's: (rows, 1024) x (151936, 1024)^T, as the library GEMM + the sampler
+    # the LM head in front of it: (rows, 1024) x (151936, 1024)^T, as the library GEMM + the sampler
     # launch and as one pass over the weights that never writes the logits
     import torch.nn.functional as F
     from minivllm_amd.layers.fused import lm_head_sample, lm_head_sample_workspace_bytes
@@ -879,7 +879,7 @@ def bench_prefill_timeline(args):
 
 
 def bench_engine(args, max_num_sequences, graph):
-    """random-init Qwen3-style decoder (hidden 1024, 8 layers, Hq16/Hkv8/D128, FFN 3072,
+    """The engine, random-init Qwen3-style decoder (hidden 1024, 8 layers, Hq16/Hkv8/D128, FFN 3072,
     vocab 151936, bf16), 60 prompts of random ids with lengths U[32,96], 256 new tokens each, T 0.6."""
     import torch
     from minivllm_amd.engine.llm_engine import LLMEngine

@@ -1490,7 +1490,7 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(const DecodeArgs a) 
 
 // The same merge for head dims 32, 64, 128 and 256: D / 4 lanes per head with 16-byte loads, and the partials of
 // eight partitions requested before the first is merged (the loop above waits for every partition in turn; a
-// sequence of config 3 has up to 16 of them).  Same arithmetic in
+// sequence of 32768 tokens has up to 16 of them).  Same arithmetic in
 // the same order, so the result is the same bit for bit.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void decode_reduce_vec_kernel(const DecodeArgs a) {

@@ -167,7 +167,7 @@ CONFIG5 = dict(vocab_size=151936, hidden_size=1024, num_layers=8, num_heads=16, 
 
 
 def test_config5_full_shape():
-    """BASELINE.json config 5 at its own shape (llm_engine.py:71-88 driven as main.py:15-41 does): Qwen3-style
+    """The engine benchmark at its own shape (llm_engine.py:71-88 driven as main.py:15-41 does): Qwen3-style
     decoder 8 x 1024, 16 query / 8 kv heads of 128 dims, vocabulary 151 936, blocks of 256 tokens, 60 prompts of
     32-96 random ids, 256 new tokens each at temperature 0.6.  Checked: the run completes with every id in range;
     the hipGraph decode run and an eager run on the captured shapes (the batch padded to its bucket, the block

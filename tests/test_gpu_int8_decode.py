@@ -3,7 +3,7 @@
 The INT8 format is defined by this build (the reference has none): the oracle dequantises code*scale in
 fp32 and runs the naive decode.  Tolerance: mean-abs 2e-3 and |err| <= 2e-2 + |want| * 2^-8 elementwise; the
 second term is the rounding of the 16-bit output itself, which matters here because the 8-sigma outliers of
-config 4 make single outputs as large as 30 (one bf16 ulp at 16..32 is 0.125)."""
+the INT8 workload make single outputs as large as 30 (one bf16 ulp at 16..32 is 0.125)."""
 import math
 
 import pytest
@@ -90,7 +90,7 @@ def test_int8_zero_context_and_missing_blocks():
 
 
 def test_config4_subset():
-    """BASELINE.json config 4 shape (B 128 is cut to 24 sequences here, ctx U[256,16384]) on the fast path."""
+    """The INT8 workload's shape (B 128 is cut to 24 sequences here, ctx U[256,16384]) on the fast path."""
     hq, hkv, d, bs = 32, 8, 128, 16
     case = _quantised_case(65, 24, 256, 16384, hq, hkv, d, bs)
     _check(case, hq, hkv, d, bs, 1 / math.sqrt(d))
@@ -126,7 +126,7 @@ def test_int8_both_grid_forms(hq, hkv, bs, d, form):
 
 
 def test_config4_full_size_on_its_own_plan():
-    """BASELINE.json config 4 in full: B 128, ctx U[256,16384], Hq32/Hkv8/D128, block 16, N(0,1) inputs with 1 % of
+    """The INT8 workload in full: B 128, ctx U[256,16384], Hq32/Hkv8/D128, block 16, N(0,1) inputs with 1 % of
     the entries at 8 sigma, INT8 store then INT8 decode.  At this size the host picks the one-wave-per-head kernel
     with 16 partitions of 1024 tokens and the merge kernel (a smaller batch would take the other form).  The cache
     (2.2 GB of codes) is written on the device by the INT8 store in chunks; the oracle runs on picked sequences."""

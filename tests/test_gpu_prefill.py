@@ -245,7 +245,7 @@ def test_two_group_prefill_deals_every_item_once(hq, hkv, dtype, num_seqs):
 
 
 def test_config2_full_size():
-    """16 prompts L U[64,2048], Hq32/Hkv8/D128 bf16; store into block-256 cache; the last
+    """A ragged batch of 16 prompts L U[64,2048], Hq32/Hkv8/D128 bf16; store into block-256 cache; the last
     row of each prompt must agree with a paged decode of that token over the stored cache."""
     hq, hkv, d, bs = 32, 8, 128, 256
     g = torch.Generator().manual_seed(53)
