@@ -450,42 +450,42 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
 // Which kernel: the two-group kernel holds one workgroup per CU and runs faster once it has started (906 TFLOP/s against 680), but takes
 // 6 us longer until then, and its longest item decides when there are few.  So this form takes what fits on the chip about at once, two
 // workgroups per CU, and somewhat more where its many short row tiles meet the other's long ones: short prompts, and one prompt, whose tiles are all
-// different.  us on either side, bf16: 16 heads over 8 kv heads of 128, two prompts of 270 rows 20.5 / 13, one of 3600 (456 workgroups) 84 / 73, of 5800
-// (728) 152 / 146, 16 of 370 (736) 33 / 29, 13 of 430 (816) 39 / 35, but seven of 760 (680) 37 / 40, two of 2500 (640) 73 / 75; 11 of 900 behind half (664)
-// 58 / 52, seven of 1600 (728) 83 / 83.  32 heads: nine of 120 16.2 / 13.9, 13 of 150 (576) 21.5 / 17.7, one of 1800 46.6 / 41.8, of 2500 (616) 67 / 63, five of
-// 530 (680) 30 / 30, six of 600 (896) 37 / 40; nine of 580 behind up to half (544) 37 / 30, four of 1900 (608) 66 / 60, one of 2270 (568) 147 / 166.
+// different.  All figures here are us there / here, bf16, captured layers with their store (beside packed prompts in either launch, in front of cached
+// ones).  16 heads over 8 kv heads of 128: two prompts of 270 rows 16.0 / 9.8, one of 3600 (456 workgroups) 78 / 66, of 5800 (728) 142 / 135, 16 of 370 (864)
+// 30.6 / 27.1, 13 of 430 (800) 31.6 / 26.7, but seven of 760 (720) 32.0 / 34.1, two of 2500 (640) 65 / 66; behind as many, 11 of 420 (664) 56 / 51, seven of 800
+// (752) 80 / 82.  32 heads: nine of 120 (336) 11.3 / 10.2, 13 of 150 (584) 17.5 / 13.4, one of 1800 42 / 36, of 2500 (632) 62 / 58; of the limit's other side five of
+// 530 (696) 25.8 / 24.4, six of 600 (944) 33.1 / 31.0, nine of 290 behind as many (720) 43.4 / 43.3, but four of 950 behind as many (976) 95 / 104, one of 2270 (568) 145 / 163.
 // The two workgroups of a CU are the i-th and the (i + 256)-th.  Of a single sequence that is a heavy and a light one; of several equal
-// ones it can be two of the heaviest, and the longer the tiles, the less the later start of the other kernel counts.  us there and here (before
-// the one-group kernel's diagonal tiles became one loop, which took up to a tenth off short prompts here), and busiest_cu: two prompts of 1496 (384 workgroups) 36.6 / 34.8 1.67, of 1656 (424) 38.8 / 40.2 1.79, of 1976 (504) 47.3 / 51.8 1.98, three of 976
-// (384) 28.2 / 30.6 2.0, of 1296 (504) 36.6 / 34.5 1.52; behind cached halves three of 794 rows (320) 42.7 / 40.6 1.80, four of
-// 588 (320) 34.3 / 36.6 1.90; behind 95 %, nine of 128 (32 heads, 360) 59 / 71 2.0.  Uneven ones meet by chance: 3300 rows of two
-// (60 and 40 %) 44.2 / 38.3, of three 43.9 / 34.6.  Cached batches do not tell whether they are even and count as if.  With four heads per workgroup
-// row tiles are half as long and equal sequences cost less: two prompts of 960 (496) 33.5 / 34.3, of 1040 34.9 / 36.7, three of 500 (392) 23.3 / 24.0, nine of
-// 233 (576, busiest 3) 21.1 / 23.0, but four of 680 (648, 2.2) 30.0 / 29.9, seven of 370 (624, 2.7) 25.4 / 24.0; behind halves only two of them lose (of 1630
-// 52 / 54; four of 1100 56 / 51).  (Above 112 tiles the other form cuts its keys too, and loses on either side of the line.)
-// An odd head group has row tiles of 128 here as there, so that nothing is gained from shorter ones: packed batches lose (us there and here, ten prompts of
-// 332, 12 heads over 4: 15.5 / 19.6; five of 764, 14 over 2: 22.7 / 28.7), but where the other form's places of 256 rows pass the chip's 512 and
-// these workgroups do not; cached ones gain what its empty places cost (seven of 40 to 70 rows behind as many, 40 over 8: 19.1 / 11.7; ten of
-// 163, 12 over 4, no empty places: 15.1 / 17.5) and where most keys are cached, so that tiles are alike (857 batches of random sizes behind 90 and 95 %:
-// 1.18 and 1.21 times as fast); few workgroups with few keys gain nothing (below 8 tiles 0.98).
+// ones it can be two of the heaviest, and the longer the tiles, the less the later start of the other kernel counts.  us, and busiest_cu: two prompts of
+// 1496 (384 workgroups) 37.5 / 33.1 1.67, of 1656 (424) 40.5 / 38.8 1.79, of 1976 (504) 49.6 / 51.4 1.98, three of 976 (384) 28.3 / 28.2 2.0, of 1296 (504) 38.0 /
+// 33.0 1.52; behind as many three of 794 rows (320) 51 / 47 1.80, four of 588 (320) 42.5 / 42.1 1.90; behind 95 %, nine of 128 (32 heads, 360)
+// 64 / 74 2.0: the line lies a little low, by 4 % of one and nothing of the others.  Uneven ones meet by chance: 3300 rows of two (60 and 40 %) 46 / 36, of
+// three 38 / 32.  Cached batches do not tell whether they are even and count as if.  With four heads per workgroup row tiles are half as long and equal
+// sequences cost less: two prompts of 960 (496) 27.1 / 28.2, of 1040 30.5 / 31.1, three of 500 (392) 18.2 / 18.6, nine of 233 (592, busiest 3) 17.7 / 18.0, four of 680
+// (712) 27.4 / 27.9, seven of 370 (696) 21.2 / 22.7; behind as many only two of them lose (of 815 51 / 52; four of 550 54 / 51).  (Above 112 tiles the other form
+// cuts its keys too, and loses on either side of the line.)
+// An odd head group has row tiles of 128 here as there, so that nothing is gained from shorter ones: packed batches lose (ten prompts of
+// 332, 12 heads over 4: 15.9 / 16.6; five of 764, 14 over 2: 20.5 / 24.8; three of 400, 40 over 8, 480 places: 16.0 / 16.3), but where the other form's places of 256
+// rows pass the chip's 512 and these workgroups do not (four of 280 19.5 / 14.0); cached ones gain what its empty places cost (seven of 55 rows behind as many, 40
+// over 8: 19.7 / 14.9; ten of 163, 12 over 4, no empty places: 18.9 / 22.5) and where most keys are cached, so that tiles are alike (in the mean of 857 batches of
+// random sizes, 1.2 times as fast; not ten of 163 behind 1467: 40 / 44); few workgroups with few keys gain nothing (two of 30 behind 270 13.4 / 13.3).
 // At head_dim 64 the other form is this kernel over its banded order, 256 rows of a sequence at a time, the heaviest first: it pays for
-// packed batches as soon as their tiles differ (3500 rows, 448 workgroups: 30 us, here 33; equal ones of a busiest CU above 1.5, three of 1925, 8
-// heads, 27.7 / 35.2, of 1181, 12 heads over 4, 18.0 / 23.1).  Cached ones pay its empty places, which fill the
-// chip's 512 the sooner; up to there its order gains where the CUs differ and most keys are not cached: us there and here, two of 1852 rows
-// behind as many, 16 heads (480 workgroups of 512 places, busiest 1.97) 60.4 / 67.6, three of 1266, 16 over 2 (480, 1.8) 43.3 / 49.3; four of 418
-// of 758 keys, 32 heads (512 places) 17.3 / 19.1, of 350 (352 of 512) 21.4 / 23.3; with tiles of 64 or 128 rows a third of the places empty ends
-// that (1.03 times as fast here in 40 random batches); beyond, of 518 of 958 (768) 26.5 / 20.2; eight of 93 of 168 (512 and 192) 19.1 / 15.8.
-// With four heads per workgroup a band is eight tiles: packed batches of 400 to 600 workgroups gain where it has empty places (nine of 244 16.8 / 13.5, five
-// of 190 15.0 / 14.3, three of 600 19.7 / 17.7; two of 960, none empty, 19.4 / 23.0) or is one sequence (of 1800 30.2 / 28.3), cached ones up to 1400 (16 of
-// 170 behind as many 27.8 / 22.2, three of 1600 behind up to half 107 / 98; none empty: eight of 500 47 / 50).
-// A few rows at head_dim 64 stay there, where placing the bands costs nothing (23 rows 8.8 / 9.5; from 5 sequences of 32 heads and 10 of 16
-// on 12.3 / 11.0), and so do 200 workgroups with more than 7000 keys, whose ranges the other form cuts (four heads of 128 121 / 128, of 64
-// 88 / 97, two of 64 80 / 96).
+// packed batches as soon as their tiles differ (3500 rows, 440 workgroups: 43.9 / 42.8; equal ones of a busiest CU above 1.5, three of 1925, 8
+// heads, 26.0 / 34.7, of 1181, 12 heads over 4, 17.6 / 22.5).  Cached ones pay its empty places, which fill the
+// chip's 512 the sooner; up to there its order gains where the CUs differ and most keys are not cached: two of 1852 rows
+// behind as many, 16 heads (480 workgroups of 512 places, busiest 1.97) 69 / 76, three of 1266, 16 over 2 (480, 1.8) 48 / 52; four of 418
+// of 758 keys, 32 heads (512 places) 21.7 / 22.0, of 350 (352 of 512) 20.3 / 22.6; with tiles of 64 or 128 rows a third of the places empty ends
+// that (1.03 times as fast here in 40 random batches); beyond, of 518 of 958 (768) 29.0 / 27.3; eight of 93 of 168 (512 and 192) 12.6 / 11.1.
+// With four heads per workgroup a band is eight tiles: packed batches of 400 to 600 workgroups gain where it has empty places (nine of 244 12.0 / 11.8,
+// three of 600 15.9 / 14.5; two of 960, none empty, 16.0 / 19.8) or is one sequence (of 1800 24.2 / 23.8), cached ones up to 1400 (16 of
+// 170 behind as many 27.7 / 22.2, three of 1600 behind 800 90 / 84; none empty: eight of 500 46 / 48).
+// A few rows at head_dim 64 stay there, where placing the bands costs nothing (23 rows 4.8 / 4.8; five sequences of them, 32 heads, 5.2 / 4.9), and so do 200
+// workgroups with more than 7000 keys, whose ranges the other form cuts (800 behind 7600, 32 heads of 128 141 / 144, of 64 94 / 109).
 // Which range: a tile takes a workgroup 0.9 us (0.8 at head_dim 64), workgroups of 0.6 of the longest sequence's tiles each fill 256 CUs;
 // a range brings every row's fp32 partial result into memory and back, about 0.7 of the ranges are there on average.  Batches of more
 // than 192 workgroups gain nothing that the partial results do not cost (1500 rows behind 1500, 32 heads, 376 workgroups: whole 72, two
-// ranges 86).  Measured, whole -> ranges: 343 rows behind 6500, 16 heads 64 -> 35; 870 behind 7800 50 -> 40; 132 behind 32768, 32
-// heads: 104, two-group kernel with split keys 155.
+// ranges 86).  The other kernels, split keys where they take them, / ranges: 343 rows behind 6500, 16 heads 50 / 43; 870 behind 7800 107 / 81; 132 of
+// 32768, 32 heads 150 / 102.
 extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads,
                                          int head_dim, int block_size, int dtype) {
   if (!ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype)) return 0;
