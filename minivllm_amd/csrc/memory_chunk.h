@@ -26,7 +26,8 @@ namespace mvllm {
 
 constexpr int kBlock = 64;           // rows per block
 constexpr int kMaxParts = 16;        // workgroups that share a head's rows, at most: more bring less than 1 %
-// What passing over a block takes of a block's time: 2.5 of 6.1 us where few workgroups run, of 8.3 where they fill the chip (whose clock falls).
+// What passing over a block takes of a block's time: 2.5 us of 8.3 where workgroups fill the chip (whose clock falls), 0.3.  Of 6.1 where few run, 0.4: the
+// parts of a single prompt are shared out by the same 0.3, so that its later ones end somewhat after the first.  layers/recurrent.py has both numbers too.
 constexpr float kPassOver = 0.3f;
 
 struct MemoryChunkArgs {

@@ -392,3 +392,14 @@ def test_preemption_starts_over():
     seqs, prefill = sch.schedule()                                # both need a third block: the later one goes back
     assert not prefill and seqs == [a] and b.state_slot < 0 and b.num_computed_tokens == 0 and list(sch.waiting) == [b]
     assert len(b) == 33
+
+
+def test_shared_rows_are_planned_with_the_kernels_numbers():
+    """layers/recurrent.py plans the parts of a head's rows that csrc/memory_chunk.h shares out."""
+    import re
+    from pathlib import Path
+
+    from minivllm_amd.layers import recurrent
+    text = (Path(recurrent.__file__).parents[1] / "csrc" / "memory_chunk.h").read_text()
+    number = lambda name: float(re.search(rf"constexpr \w+ {name} = ([0-9.]+)f?;", text).group(1))
+    assert (number("kMaxParts"), number("kPassOver"), number("kBlock")) == (recurrent.MAX_PARTS, recurrent.PASS_OVER, recurrent.BLOCK_ROWS)
