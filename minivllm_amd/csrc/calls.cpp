@@ -7,6 +7,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -163,8 +164,9 @@ template <bool int8> PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t 
   if (int8 && (!has_shape(*ks, {k->size(0), block, kv_heads}) || vs->sizes() != ks->sizes())) return none();
   const int most = (int)tables->size(1);
   int part_tokens, parts, waves = 0;      // (shapes without a tiled kernel are warned of)
-  if (lib.decode_plan(1, heads, kv_heads, dim, 1, block, code, int8, &part_tokens, &parts, &waves) != MVLLM_OK || waves == 0) return none();
-  const size_t need = lib.decode_bytes((int)batch, heads, dim, most, block);
+  if (lib.decode_plan((int)batch, heads, kv_heads, dim, std::max(most, 1), block, code, int8, &part_tokens, &parts, &waves) != MVLLM_OK || waves == 0)
+    return none();
+  const size_t need = parts > 1 ? lib.decode_bytes((int)batch, heads, dim, most, block) : 0;
   // the caller's workspace where it is one and large enough, else one of this call's, on its stream like the result
   const at::Tensor* space = need > 0 && a[12] != Py_None ? dense(a[12], at::kByte) : nullptr;
   if (need > 0 && a[12] != Py_None && !space) return none();
