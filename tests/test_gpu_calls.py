@@ -261,3 +261,76 @@ def test_subclasses_and_modes_go_the_longer_way(counted):
         assert torch.equal(attention.flash_attention_prefill(q, k, k, cu, 0.125, 8, 2, 64), want)
     assert counted.taken == 1 and any("empty_like" in n for n in seen.names)
     assert attention.flash_attention_prefill(torch.nn.Parameter(q), k, k, cu, 0.125, 8, 2, 64).requires_grad is False and counted.taken == 2
+
+
+def _changed(t, rows):
+    """A tensor that an operator converts or refuses: other types, device, layout, and of data other shapes, ``rows`` where the host knows their number."""
+    yield from (None, t.cpu(), t.double(), t.to(torch.int32), torch.stack([t, t], -1)[..., 0])
+    if t.dim() > 1:
+        yield from (t.unsqueeze(0), t[..., :-1], t[..., :-1].contiguous(), t[:, :-1].contiguous())
+        if rows:
+            yield t[:-1]
+        if t.is_floating_point():
+            yield t.half()
+
+
+def _operators():
+    bf = dict(dtype=torch.bfloat16)
+    tables, (k, v), _ = paged([40, 17], 16, 2, 64, torch.bfloat16)
+    _, (k8, v8), (ks, vs) = paged([40, 17], 16, 2, 64, None, int8=True)
+    lens, cu, cu_k = torch.tensor([40, 17], device=DEV), torch.tensor([0, 30, 39], dtype=torch.int32, device=DEV), torch.tensor([0, 40, 57], dtype=torch.int32, device=DEV)
+    q, new_k, new_v, slots = normal(39, 4, 64, **bf), normal(39, 2, 64, **bf), normal(39, 2, 64, **bf) + 1, torch.arange(39, device=DEV)
+    rest = (0.125, 4, 2, 64)
+
+    def stored(*args):
+        caches = [torch.zeros(4, 16, 2, 64, device=DEV, **bf) for _ in range(2)]
+        attention.store_kvcache(*args[:2], *caches, args[2], 16)
+        return torch.stack(caches)
+
+    def layer(*args):
+        a = attention.Attention(4, 64, num_kv_heads=2, block_size=16)
+        a.k_cache, a.v_cache = [torch.zeros(4, 16, 2, 64, device=DEV, **bf) for _ in range(2)]
+        set_context(True, cu_seqlens_q=args[3], max_seqlen_q=30, slot_mapping=args[4])
+        try:
+            return torch.cat([t.flatten() for t in (a(*args[:3]), a.k_cache, a.v_cache)])
+        finally:
+            reset_context()
+
+    def window(*args):
+        out = torch.zeros(39, 4, 64, device=DEV, **bf)
+        window_prefill(out, *args[:4], 0.125, 20, v=args[4])
+        return out
+
+    return {
+        "store": (stored, (new_k, new_v, slots)),
+        "decode": (lambda *a: attention.paged_attention_decode(*a, *rest, 16), (q[:2], k, v, tables, lens)),
+        "decode_int8": (lambda *a: attention.paged_attention_decode_int8(*a, *rest, 16), (q[:2], k8, v8, ks, vs, tables, lens)),
+        "prefill": (lambda *a: attention.flash_attention_prefill(*a, *rest, max_seqlen=30), (q, new_k, new_v, cu)),
+        "prefill_paged": (lambda *a: attention.flash_attention_prefill_paged(*a, *rest, 16, max_seqlen_k=40), (q, k, v, tables, cu, cu_k)),
+        "layer": (layer, (q, new_k, new_v, cu, slots)),
+        "window": (window, (q, new_k, cu, cu, new_v)),
+    }
+
+
+@pytest.mark.parametrize("name", ["store", "decode", "decode_int8", "prefill", "prefill_paged", "layer", "window"])
+def test_both_ways_take_and_refuse_the_same(counted, monkeypatch, name):
+    """Every argument changed by itself: what one way converts or refuses, and with which error, so does the other."""
+    def outcome(f, args):
+        try:
+            return f(*args)
+        except Exception as e:
+            return type(e)
+
+    f, args = _operators()[name]
+    both(counted, monkeypatch, lambda: f(*args), 1)
+    refused = 0
+    for i in range(len(args)):
+        for j, other in enumerate(_changed(args[i], name not in ("prefill_paged", "window"))):
+            changed = (*args[:i], other, *args[i + 1:])
+            a = outcome(f, changed)
+            with monkeypatch.context() as m:
+                m.setattr(_C, "calls", None)
+                b = outcome(f, changed)
+            refused += isinstance(a, type)
+            assert (a is b) if isinstance(a, type) or isinstance(b, type) else torch.equal(a, b), (i, j, a, b)
+    assert refused > len(args)
