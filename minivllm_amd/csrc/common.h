@@ -262,9 +262,6 @@ int launch_prefill_rows16(const PrefillRowsArgs& a, int head_dim, int dtype, hip
 // shapes that kernel is built for: fp32 and INT8 caches with 64 or 128 dims per head, 16-bit also with 32, 80, 96, 112 and 256
 bool prefill_rows16_takes(int head_dim, int dtype, bool int8_cache);
 
-// Varlen causal prefill in the two-group form (prefill_pingpong.hip): one persistent 8-wave workgroup per CU whose two
-// wave groups alternate between the matrix unit and the softmax.  Launched from the prefill entry point for the batches
-// it takes; everything else stays on prefill_mfma_kernel.
 // The rows of k and v of a packed prefill that go to a paged cache in its launch (store_beside, prefill_tiles.h); without a cache there are none.
 struct StoreBeside {
   unsigned first = 0;            // the workgroups from here on copy; set by the launcher
@@ -275,6 +272,9 @@ struct StoreBeside {
   int64_t num_slots = 0;
 };
 
+// Varlen causal prefill in the two-group form (prefill_pingpong.hip): one persistent 8-wave workgroup per CU whose two
+// wave groups alternate between the matrix unit and the softmax.  Launched from the prefill entry point for the batches
+// it takes; everything else stays on prefill_mfma_kernel.
 struct PrefillPpArgs {
   void* out;
   const void* q;
