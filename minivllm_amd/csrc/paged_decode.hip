@@ -7,8 +7,9 @@
 //   workgroup owns kv head g and all Hq/Hkv query heads that share it (16 of them at a time where a kv head has more:
 //   head_slice), so the waves of one workgroup stream contiguous pieces of the [token, Hkv, D] rows.
 //   A wave walks its partition in tiles of 16 tokens, both products on the matrix unit:
-//     S[16 tok x 16 head]  = K_tile (A operand, straight from global in MFMA
-//                            layout) x Q^T (B operand, column n = head n)
+//     S[16 tok x 16 head]  = K_tile (A operand, loaded in whole rows and put
+//                            into MFMA layout by way of LDS: KeyRows)
+//                            x Q^T (B operand, column n = head n)
 //     online softmax       per lane over its four tokens, base-2, lazy rescale with one
 //                            maximum per head shared by the lanes that hold it
 //     O[16 head x 128]    += P (the scores' own layout, packed to 16 bit) x V; V rows are
@@ -260,6 +261,18 @@ struct TileIO {
     for (int j = 0; j < kSteps; ++j)
       t.k[j] = has_dims(j, cls) ? *reinterpret_cast<const uint4*>(kp + 32 * j) : make_uint4(0u, 0u, 0u, 0u);
   }
+  // K in whole rows: load j is rows kRowsPer j .. of the tile, D / 8 lanes each
+  static constexpr int kChunks = D / 8, kRowsPer = 64 / (D / 8 < 64 ? D / 8 : 64), kRowLoads = (D == 64 || D == 128) ? kTile / kRowsPer : 1;
+  template <bool STREAM>
+  static __device__ __forceinline__ void load_k_rows(KVTile<T, D>& t, const T* kp, int64_t row) {
+#pragma unroll
+    for (int j = 0; j < kRowLoads; ++j) {
+      const T* from = kp + j * kRowsPer * row;
+      t.k[j] = STREAM ? load16_stream(from) : *reinterpret_cast<const uint4*>(from);
+    }
+  }
+  // place of chunk c of the tile's row r in the wave's LDS: the sixteen rows' same chunk are in different banks
+  static __device__ __forceinline__ int row_place(int r, int c) { return (r * kChunks + (c ^ ((D == 128 ? r : r >> 1) & (kChunks - 1)))) * 16; }
   template <bool STREAM>
   static __device__ __forceinline__ void load_v(KVTile<T, D>& t, int i, const T* vp, bool own) {
 #pragma unroll
@@ -353,7 +366,7 @@ __device__ __forceinline__ void finish_head(HEAD& hd, const DecodeArgs& a, int b
 
 // One wave = one kv head of one (sequence, partition); both products run on the matrix unit.
 //   S[token][head] = K Q^T   v_mfma 16x16x32: A = 16 tokens x 32 dims (lane l: token l%16, dims 8*(l/16).. of each
-//                    32-dim step, 16 B straight from the cache row), B = the query heads of the group as columns
+//                    32-dim step, 16 B of the cache row: KeyRows), B = the query heads of the group as columns
 //                    (column n = head n, zero past the group), four steps for 128 dims.  Lane l then holds
 //                    S[token 4*(l/16)+i][head l%16], i < 4.
 //   softmax          per lane over its four tokens; the running maximum m of a head is kept identical in the four
@@ -426,8 +439,10 @@ struct DecodeHead {
 
   // one tile of 16 tokens starting at token t0 of the sequence; tokens at or past part_end do not count
   // (col_end: prefill only, where column n is a query row: tokens at or past it do not count for this lane's column)
+  // kRows: t.k holds whole rows, which become the first product's operands in k_lds (the wave's own: no barrier, the LDS keeps a wave's order)
+  template <bool kRows = false>
   __device__ __forceinline__ void consume(const KVTile<T, D>& t, int part_end, float scale_log2, int lane,
-                                          int col_end = 0x7fffffff) {
+                                          int col_end = 0x7fffffff, char* k_lds = nullptr) {
     if constexpr (MVLLM_DECODE_LOADS_ONLY) {      // the loads of the tile and nothing else: the access pattern's ceiling
       uint32_t x = 0;
 #pragma unroll
@@ -441,8 +456,18 @@ struct DecodeHead {
     const int tok_base = t.t0 + 4 * cls;
     const bool partial = (!t.ok) || (t.t0 + kTile > part_end);
     v4f s = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (kRows) {
+      using IO = TileIO<T, D>;
 #pragma unroll
-    for (int j = 0; j < kSteps; ++j) s = mfma16x16x32<T>(t.k[j], qf[j], s);
+      for (int j = 0; j < IO::kRowLoads; ++j)
+        *reinterpret_cast<uint4*>(k_lds + IO::row_place(IO::kRowsPer * j + lane / IO::kChunks, lane % IO::kChunks)) = t.k[j];
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j)
+        s = mfma16x16x32<T>(*reinterpret_cast<const uint4*>(k_lds + IO::row_place(lane & 15, cls + 4 * j)), qf[j], s);
+    } else {
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j) s = mfma16x16x32<T>(t.k[j], qf[j], s);
+    }
     float s2[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) s2[i] = s[i] * scale_log2;
@@ -549,8 +574,9 @@ struct DecodeHead<float, D> {
     load_q(reinterpret_cast<const float*>(a.q) + ((int64_t)b * a.num_heads + head0 + (live ? col : 0)) * D, live, lane);
   }
 
+  template <bool kRows = false>
   __device__ __forceinline__ void consume(const KVTile<float, D>& t, int part_end, float scale_log2, int lane,
-                                          int col_end = 0x7fffffff) {
+                                          int col_end = 0x7fffffff, char* = nullptr) {
     const int cls = lane >> 4;
     const int tok_base = t.t0 + 4 * cls;
     const bool partial = (!t.ok) || (t.t0 + kTile > part_end);
@@ -636,10 +662,10 @@ struct DecodeHead<float, D> {
 // then share the log-sum-exp merge and the output, four dims of a head per thread.  (One wave folding the others' accumulators into
 // its own, 16 heads whether live or not, was a chain of 0.3 us per wave.)  Every wave of the workgroup must call this.
 template <int W, typename HEAD>
-__device__ __forceinline__ void finish_waves(HEAD& hd, const DecodeArgs& a, int b, int p, int head0, int group, bool direct, int w, int lane) {
+__device__ __forceinline__ void finish_waves(HEAD& hd, const DecodeArgs& a, int b, int p, int head0, int group, bool direct, int w, int lane,
+                                             float (&rows)[W][16][HEAD::kDim]) {
   using T = typename HEAD::Elem;
   constexpr int D = HEAD::kDim;
-  __shared__ __attribute__((aligned(16))) float rows[W][16][D];
   __shared__ float2 ml[W][16];
   hd.l += __shfl_xor(hd.l, 16, 64);                 // the four token classes
   hd.l += __shfl_xor(hd.l, 32, 64);
@@ -687,6 +713,27 @@ __device__ __forceinline__ void finish_waves(HEAD& hd, const DecodeArgs& a, int 
   }
 }
 
+// The wave of its workgroup, in a scalar register, so that what a wave walks, its tiles' addresses and its branches are the scalar unit's: as lanes' values
+// they were loops under masks, 64-bit products in the vector unit and 32 registers cleared per tile.  us before / now: 3 sequences of 302 tokens 6.41 / 6.23,
+// one of 3000, heads of 64, 10.17 / 9.89, 44 of 1159 to 2310 35.6 / 35.0; where memory bounds it the same.
+__device__ __forceinline__ int this_wave() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// 16-bit keys in whole rows through LDS, or as operands straight from memory (other head dims, blocks of less than a tile).  The address unit of a CU
+// takes a 16-byte load of a wave at 64 B per clock where four neighbouring lanes share 64 bytes, and at 16 B where its lanes are sixteen
+// rows, as an operand's are: keys took it four times as long as values, and a CU with a few hundred tokens to itself had no other bound (1
+// sequence of 512 tokens in one workgroup per head: 1.35 us per tile and wave).  Rows go through a wave's own 4 KB of LDS (the accumulators' room of the merge
+// where there is one), a row's chunks trading places by its number.  Caches cold, 8 kv heads, operands / rows: 252 batches of 1 to 256 sequences in tables of
+// 512 to 16384 1.044 times as fast on average (heads of 64 1.02); one of 511 7.9 / 6.9 us, 64 of 64 to 2047 1.05 to 1.09, 24 to 40 full tables 1.04 to
+// 1.08, one wave per head, full tables 1.01, lengths spread 1.02 to 1.14.  Three waves per SIMD (168 registers, one spilled) instead of two: 1.025.
+// kStreamKeys: keys past the caches, as values (they are read once), where the waves of a head share it: 61 sequences of a decode step 558 / 571 us,
+// 16 of a smaller one 286 / 298, whose weights the caches hold; one wave per head, full tables 0.97 to 0.99 of the speed without; heads of 64 0.94 to 1.07.
+// Waves of eight at 64 dims, tables of up to 512: 0.98 to 1.00 with rows, so not there.
+template <typename T, int W, int D, bool SUB>
+struct KeyRows {
+  static constexpr bool kRows = sizeof(T) == 2 && !SUB && (D == 128 || (D == 64 && W != kSplitManyWaves));
+  static constexpr bool kStreamKeys = W > 1 && D == 128;
+};
+
 // W = 1: the wave walks all tiles of its partition.  W > 1 (the workgroup is W waves on one kv head): wave w takes
 // tiles w, w + W, ... and the partial results meet in LDS (finish_waves), so a short context costs a few tiles
 // of latency per wave and no second launch.
@@ -733,7 +780,9 @@ __device__ __forceinline__ void decode_mfma_item(const DecodeArgs& a, int b, int
   const T* vc = reinterpret_cast<const T*>(a.v_cache) + (int64_t)g * D;
 
   using IO = TileIO<T, D>;
-  const int k_lane_off = col * (int)row + cls * IO::kKLane;        // token lane%16, first dim of class lane/16
+  constexpr bool kRows = KeyRows<T, W, D, SUB>::kRows;
+  // token lane%16, first dim of class lane/16; or the lane's chunk of a row
+  const int k_lane_off = kRows ? lane / (D / 8) * (int)row + lane % (D / 8) * 8 : col * (int)row + cls * IO::kKLane;
   const int v_lane_off = 4 * cls * (int)row + col * IO::kVLane;    // token 4*(lane/16), first dim of column lane%16
 
   auto load_tile = [&](KVTile<T, D>& t, int tile) {
@@ -783,10 +832,10 @@ __device__ __forceinline__ void decode_mfma_item(const DecodeArgs& a, int b, int
       const T* kp = kc + base + k_lane_off;
       const T* vp = vc + base + v_lane_off;
       // V is read once, in whole 256-byte rows per instruction: non-temporal loads stream it past the caches.
-      // K is read in the MFMA operand layout, 64 bytes of a row per instruction, so the second half of each
-      // 128-byte line has to survive in cache until the next instruction: ordinary loads (the hint costs 7 %
-      // there).
-      IO::load_k(t, kp, lane >> 4);
+      // K in the MFMA operand layout is 64 bytes of a row per instruction, so the second half of each 128-byte line
+      // has to survive in cache until the next instruction: ordinary loads (the hint costs 7 % there).
+      if constexpr (kRows) IO::template load_k_rows<KeyRows<T, W, D, SUB>::kStreamKeys>(t, kp, row);
+      else IO::load_k(t, kp, lane >> 4);
 #pragma unroll
       for (int i = 0; i < 4; ++i) IO::template load_v<true>(t, i, vp + (int64_t)i * row, IO::owns(col));
     } else {
@@ -804,17 +853,22 @@ __device__ __forceinline__ void decode_mfma_item(const DecodeArgs& a, int b, int
   // Tiles in pairs (ta, tb: one consumed while the other is in flight), the odd one after the loop.  A single
   // loop exit keeps the accumulators in one set of registers (an exit between the two halves made the compiler
   // hold two: 184 VGPRs instead of 154, one wave per SIMD less).
+  // a wave's keys on their way into operands; W > 1: and its rows of the merge
+  constexpr int kKeyBytes = kTile * D * (int)sizeof(T), kWaves = W > 1 ? W : kRows ? kDecodeWpb : 1;
+  __shared__ __attribute__((aligned(16))) float meet[kWaves][16][W > 1 ? D : kRows ? D / 2 : 4];
+  static_assert(!kRows || sizeof(meet[0]) >= kKeyBytes, "a tile's keys");
+  char* k_lds = reinterpret_cast<char*>(meet[kWaves > 1 ? this_wave() : 0]);
   KVTile<T, D> ta, tb;
   if (ntiles > 0) load_tile(ta, 0);
   int tile = 0;
   for (; tile + 1 < ntiles; tile += 2) {
     load_tile(tb, tile + 1);
-    head.consume(ta, part_end, a.scale_log2, lane);
+    head.template consume<kRows>(ta, part_end, a.scale_log2, lane, 0x7fffffff, k_lds);
     if (tile + 2 < ntiles) load_tile(ta, tile + 2);
-    head.consume(tb, part_end, a.scale_log2, lane);
+    head.template consume<kRows>(tb, part_end, a.scale_log2, lane, 0x7fffffff, k_lds);
   }
-  if (tile < ntiles) head.consume(ta, part_end, a.scale_log2, lane);
-  if constexpr (W > 1) finish_waves<W>(head, a, b, p, hs.head0, group, direct, w, lane);
+  if (tile < ntiles) head.template consume<kRows>(ta, part_end, a.scale_log2, lane, 0x7fffffff, k_lds);
+  if constexpr (W > 1) finish_waves<W>(head, a, b, p, hs.head0, group, direct, w, lane, meet);
   else head.finish(a, b, p, hs.head0, group, direct, lane);
 }
 
@@ -1299,11 +1353,6 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
   if (!direct && lane < group && lane < 16) *reinterpret_cast<float2*>(a.ws_ml + (slot + lane) * 2) = make_float2(m, l);
 }
 
-// The wave of its workgroup, in a scalar register, so that what a wave walks, its tiles' addresses and its branches are the scalar unit's: as lanes' values
-// they were loops under masks, 64-bit products in the vector unit and 32 registers cleared per tile.  us before / now: 3 sequences of 302 tokens 6.41 / 6.23,
-// one of 3000, heads of 64, 10.17 / 9.89, 44 of 1159 to 2310 35.6 / 35.0; where memory bounds it the same.
-__device__ __forceinline__ int this_wave() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
-
 // ---------------------------------------------------------------------------
 // Kernels of the fast path: one workgroup per (partition, sequence, group of kv heads); the partition index is
 // an upper bound, and a workgroup whose partition lies past its sequence's context returns at once.
@@ -1319,7 +1368,8 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512, D > 128 ? 1 : kDecodeWavesPerE
 template <typename T, int W, int D, bool SUB = false>
 __global__ __launch_bounds__(64 * W, D > 128 ? 1 : kDecodeWavesPerEu) void decode_mfma_split_kernel(const DecodeArgs a) {
   // kv head fastest: the workgroups of one (sequence, partition) start together and read the same token rows
-  const int g = blockIdx.x, b = blockIdx.z;
+  const int b = blockIdx.z;
+  const int g = blockIdx.x;
   const int p = (int)((blockIdx.y + (unsigned)b) % (unsigned)a.num_parts);
   decode_mfma_item<T, W, D, SUB>(a, b, p, g, this_wave());
 }

@@ -90,6 +90,30 @@ def test_eight_waves_per_head(hq, hkv, d, bs, ctx_list):
     assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("waves,batch,blocks", [(8, 20, 2), (4, 64, 2), (1, 64, 1024)])
+def test_every_key_meets_its_own_value(waves, batch, blocks, d, dtype):
+    """Keys of +-1 and queries that are four times one of them: that token's weight is 1 and each other's below e^-24 (asserted), so
+    that the result is its value, bit for bit, wherever in a tile it lies."""
+    hkv, group, bs = 8, 2, 16
+    assert paged_decode_plan(batch, hkv * group, hkv, d, blocks, bs, dtype)[2] == waves
+    g = torch.Generator().manual_seed(5)
+    kc = (torch.randint(0, 2, (2 * batch, bs, hkv, d), generator=g) * 2 - 1).to(dtype)
+    vc = torch.randn(2 * batch, bs, hkv, d, generator=g).to(dtype)
+    tables = torch.full((batch, blocks), -1, dtype=torch.int32)
+    tables[:, :2] = torch.randperm(2 * batch, generator=g).view(batch, 2).to(torch.int32)
+    rows = [c[tables[:, :2].long()].reshape(batch, 2 * bs, hkv, d) for c in (kc, vc)]
+    ctx = torch.tensor([2 * bs - b % 5 for b in range(batch)])
+    at = torch.arange(batch) % 28                                  # the token that is meant
+    keys, values = (t[torch.arange(batch), at] for t in rows)
+    others = torch.einsum("bthd,bhd->bth", rows[0].float(), keys.float())
+    others[torch.arange(batch), at] = 0
+    assert others.max() * 4 < 4 * d - 24
+    got = _run((4 * keys).repeat_interleave(group, 1), kc, vc, tables, ctx, 1.0, hkv * group, hkv, d, bs)
+    assert torch.equal(got.cpu(), values.repeat_interleave(group, 1))
+
+
 @pytest.mark.parametrize("batch,first,tokens,d,plan", [
     (32, [2048, 1, 1025], 2048, 64, (2048, 1, 8)), (33, [2048, 2047, 63], 2048, 64, (2048, 1, 8)),     # whole sequences, eight waves ...
     (33, [2048, 1, 129], 2048, 32, (2048, 1, 8)), (40, [1024, 1000, 15], 1024, 80, (1024, 1, 8)), (33, [520, 300], 528, 104, (576, 1, 8)),
