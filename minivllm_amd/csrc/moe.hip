@@ -278,6 +278,8 @@ struct ExpertLinearArgs {
   int max_tiles, n_tiles;
   uint32_t x_bytes;            // (many) what x holds
   float alpha, limit, shift;   // of kClampedGlu
+  int groups;                  // (large) workgroups per XCD
+  uint32_t token_factor;       // (large) (2^32 - 1) / per_token
 };
 
 enum { kNoGlu = 0, kSiluGlu = 1, kClampedGlu = 2 };
@@ -440,20 +442,11 @@ __global__ __launch_bounds__(256) void moe_linear_any_kernel(const ExpertLinearA
 // A share's pairs go by row tiles, in fours: workgroups of a four with the same weight tile follow one another, and where shares are
 // whole row tiles, as with few experts, none of them is read by two XCDs.  Large tiles with few rows come behind all others (see kApartRows), shared evenly too: the chip's last round is made of
 // short ones.  600 rows, top 6 of 64 with uneven routing, width 2048: 132 + 71 -> 101 + 62 us.
-__device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, int& n_tile) {
+// at: a place among an XCD's (row tile, weight tile) pairs, which begin with pair `low` of all and end before `high`
+__device__ __forceinline__ void pair_at(int n, int low, int high, int place, int& tile, int& n_tile) {
   constexpr int kTogether = 4;
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, n = a.n_tiles;
-  const int whole = a.num_tiles[0], rest = a.num_tiles[1], per = (whole * n + 7) / 8;
-  if (j >= per) {
-    const int rest_per = (rest * n + 7) / 8, at = xcd * rest_per + j - per;
-    tile = whole + at / n;
-    n_tile = at % n;
-    return j - per < rest_per && at < rest * n;
-  }
-  const int low = xcd * per, high = min(low + per, whole * n);
-  if (low + j >= high) return false;
   // the last weight tiles of a row tile that the XCD before began, row tiles of its own, the first weight tiles of one more
-  const int first_own = (low + n - 1) / n, begun = first_own * n - low, own = high / n - first_own, at = j - begun;
+  const int first_own = (low + n - 1) / n, begun = first_own * n - low, own = high / n - first_own, at = place - begun;
   if (at < 0) {
     tile = first_own - 1;
     n_tile = n + at;
@@ -465,6 +458,19 @@ __device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, 
     tile = first_own + own;
     n_tile = at - own * n;
   }
+}
+__device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, int& n_tile) {
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, n = a.n_tiles;
+  const int whole = a.num_tiles[0], rest = a.num_tiles[1], per = (whole * n + 7) / 8;
+  if (j >= per) {
+    const int rest_per = (rest * n + 7) / 8, at = xcd * rest_per + j - per;
+    tile = whole + at / n;
+    n_tile = at % n;
+    return j - per < rest_per && at < rest * n;
+  }
+  const int low = xcd * per, high = min(low + per, whole * n);
+  if (low + j >= high) return false;
+  pair_at(n, low, high, j, tile, n_tile);
   return true;
 }
 
@@ -594,31 +600,83 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
 // registers; per flop it reads half as much of LDS as with 64 x 64).  The operands of a 16-wide step are read during the
 // products of the one before; a step's last products hide the barrier, after which the next step's operands are there and
 // more copies start: x, which other workgroups of the XCD read too, one step ahead in two buffers, the weights, which come
-// from memory, two steps ahead in three.  Together they fill the LDS.
+// from memory, two steps ahead in three.  Together they fill the LDS.  What x waits for bounds a step: its copies right behind a barrier that is as early as
+// the last reads allow (4096 wide, random numbers, 8 rounds of tiles: 1176 TFLOP/s with the barrier at the fourth product and copies from the eighth, 1235
+// from the fourth, 1276 so; a barrier in the sixteen before for the copies and one for the reads: 1272).  Then comes power: the same product of zeros 1340 to 1670.
+// A workgroup stays on its CU and takes every a.groups-th tile of its XCD, because the way into a tile was as long as six to eight steps of K: its number,
+// expert and rows (one load for the other, 5 us under load), the first copies (3.5), and behind the steps the stores (4.5).  The tile behind is
+// known and its rows' places are loaded a tile ahead, its first copies run beside the stores, and these go through LDS, since a lane's runs of eight outputs
+// in 32 rows took the address unit four times as long as whole rows do.  us: 65536 rows, 2048 x 768 268 -> 229, 2048 x 2048 498 -> 472; both
+// products of 8192 rows, top 6 of 64, routed unevenly, 1536 x 2048 with the gate 359 -> 337, 2048 x 768 238 -> 219.
+constexpr int kLargeGroups = 32;                    // workgroups per XCD: its CUs
 template <int kGlu>
 __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLinearArgs a) {
   constexpr int kTile = 256, kK = 64, kStage = kTile * kK * 2;       // bytes of one operand's step
   __shared__ __attribute__((aligned(16))) char lds[5 * kStage];      // weights three times, x twice
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
-  int tile, n_tile;
-  if (!find_tile(a, tile, n_tile)) return;
-  const int e = a.tile_expert[tile], row0 = a.tile_row[tile], row_end = min(row0 + kTile, a.row_start[e + 1]);
-  const int n0 = n_tile * kTile;
+  // ---- this workgroup's tiles: every a.groups-th of its XCD's.  Where they leave a last round of no more than half the workgroups, its tiles are
+  // taken in halves of 128 rows; tiles of few rows come behind them ----
+  const int n_tiles = a.n_tiles, whole = a.num_tiles[0], rest = a.num_tiles[1], xcd = blockIdx.x & 7;
+  const int per = (whole * n_tiles + 7) / 8, rest_per = (rest * n_tiles + 7) / 8;
+  const int low = min(xcd * per, whole * n_tiles), high = min(low + per, whole * n_tiles);
+  const int rest_low = min(xcd * rest_per, rest * n_tiles), rest_high = min(rest_low + rest_per, rest * n_tiles);
+  const int last = (high - low) % a.groups, halved = 2 * last <= a.groups ? last : 0, full = high - low - halved;
+  const int places = full + 2 * halved + rest_high - rest_low;
+  struct Tile { int e, row0, rows, n_tile; };
+  auto find = [&](int j, Tile& t) __attribute__((always_inline)) {
+    int tile, half = 0;
+    if (j < full + 2 * halved) {
+      const int over = j - full;
+      if (over >= 0) half = over & 1;
+      pair_at(n_tiles, low, high, over < 0 ? j : full + (over >> 1), tile, t.n_tile);
+      t.rows = over < 0 ? kTile : kTile / 2;
+    } else {
+      const int at = rest_low + j - full - 2 * halved;
+      tile = whole + at / n_tiles;
+      t.n_tile = at % n_tiles;
+      t.rows = kTile;
+    }
+    t.e = a.tile_expert[tile];
+    t.row0 = a.tile_row[tile] + half * (kTile / 2);
+  };
+  int j = blockIdx.x >> 3;
+  Tile now{}, next{};
+  if (j >= places) return;
+  find(j, now);
+  j += a.groups;
+  if (j < places) find(j, next);
 
-  const v4i w_rows = make_rsrc(reinterpret_cast<const char*>(a.w) + (int64_t)e * a.N * a.K * 2, (uint32_t)((int64_t)a.N * a.K * 2));
   const v4i x_rows = make_rsrc(reinterpret_cast<const char*>(a.x), a.x_bytes);
-  uint32_t from_w[8], from_x[8];
+  const int total = a.row_start[a.experts], steps = a.K / kK;
+  // the rows of x that this thread copies: those of the sorted rows row0 + (256 i + tid) / 8.  Past the tile's end they are the next
+  // expert's, whose results are not stored.
+  auto pairs_of = [&](const Tile& t, uint32_t (&pair)[8]) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int c = 256 * i + tid, r = c >> 3, p = (c & 7) ^ ((r >> 1) & 7);
-    from_w[i] = (uint32_t)(min(n0 + r, a.N - 1) * a.K + 8 * p) * 2u;
-    const int at = min(row0 + r, row_end - 1);
-    const uint32_t xr = (uint32_t)(a.per_token ? a.sorted_pair[at] / a.per_token : at);
-    from_x[i] = (xr * (uint32_t)a.x_stride + 8u * p) * 2u;
-  }
+    for (int i = 0; i < 8; ++i) {
+      const int at = min(t.row0 + ((256 * i + tid) >> 3), total - 1);
+      pair[i] = (uint32_t)(a.per_token ? a.sorted_pair[at] : at);
+    }
+  };
+  uint32_t from_w[8], from_x[8], pair[8];
+  v4i w_rows;
+  int turn;
+  auto places_of = [&](const Tile& t) __attribute__((always_inline)) {
+    w_rows = make_rsrc(reinterpret_cast<const char*>(a.w) + (int64_t)t.e * a.N * a.K * 2, (uint32_t)((int64_t)a.N * a.K * 2));
+    turn = first_step(a, t.e, t.n_tile, steps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int c = 256 * i + tid, r = c >> 3, p = (c & 7) ^ ((r >> 1) & 7);
+      from_w[i] = (uint32_t)(min(t.n_tile * kTile + r, a.N - 1) * a.K + 8 * p) * 2u;
+      uint32_t row = pair[i];
+      if (a.per_token) {                            // pair / per_token: the quotient of the rounded factor is that or one less
+        row = __umulhi(pair[i], a.token_factor);
+        row += pair[i] - row * (uint32_t)a.per_token >= (uint32_t)a.per_token;
+      }
+      from_x[i] = (row * (uint32_t)a.x_stride + 8u * p) * 2u;
+    }
+  };
   constexpr int kX = 3 * kStage;                    // where x begins
   const uint32_t lds_wave = lds_address(lds) + 1024 * wave;
-  const int steps = a.K / kK, turn = first_step(a, e, n_tile, steps);
   auto k_of = [&](int step) __attribute__((always_inline)) { return (uint32_t)(step < steps - turn ? step + turn : step + turn - steps) * (2 * kK); };
   // copy i of eight of a step's operand; past the last step nothing is read (the buffer is not used again)
   auto copy_w = [&](auto I, int step, uint32_t buffer) __attribute__((always_inline)) {
@@ -631,16 +689,17 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
     rows[2] = step < steps ? rows[2] : 0;
     dma16_to_lds_at<4096 * decltype(I)::value>(rows, from_x[decltype(I)::value], k_of(step), lds_wave + kX + (step & 1) * kStage);
   };
+  auto copy_first = [&](int blocks) __attribute__((always_inline)) {       // the first step's operands, then the second's weights
+    static_for<8>([&](auto I) { copy_w(I, 0, 0); });
+    static_for<8>([&](auto I) {
+      if (decltype(I)::value < 2 * blocks) copy_x(I, 0);
+    });
+    static_for<8>([&](auto I) { copy_w(I, 1, kStage); });
+  };
   const int wn = wave & 1, wm = wave >> 1;
   const int sw = (l32 >> 1) & 7;
   const char* frag = lds + l32 * 128;
   v16f acc[4][4];
-#pragma unroll
-  for (int n = 0; n < 4; ++n)
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[n][m][r] = 0.f;
   uint4 wf[2][4], xf[2][4];
   // where this lane's operands of the four 16-wide steps lie in a buffer
   uint32_t place[4];
@@ -654,6 +713,7 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
   // time than its rows do.
   auto run = [&](auto BLOCKS) __attribute__((always_inline)) {
     constexpr int kBlocks = decltype(BLOCKS)::value, kProducts = 4 * kBlocks, kPer = kBlocks == 1 ? 2 : 1;
+    constexpr int kBarrier = kBlocks == 4 ? 1 : kBlocks - 1;         // the product of the last sixteen with the step's barrier, before the next step's reads
     // The products of a 16-wide step one by one; after each of them one of the next step's reads (every kEvery-th from product
     // kFirst on, those that are needed first come first) and whatever `also` does: the matrix unit must not wait for a queue of
     // reads or copies.
@@ -679,12 +739,7 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
     constexpr std::integral_constant<int, kBlocks == 4 ? 2 : 1> spread{};
     auto nothing = [](auto) {};
 
-    static_for<8>([&](auto I) {
-      copy_w(I, 0, 0);
-      if constexpr (decltype(I)::value < 2 * kBlocks) copy_x(I, 0);
-      copy_w(I, 1, kStage);
-    });
-    dma_wait_all();
+    dma_wait_all();                                 // the first copies; what the tile before stored
     __syncthreads();
     static_for<2 * kBlocks>([&](auto I) { copy_x(I, 1); });
 #pragma unroll
@@ -711,51 +766,97 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
       // ahead follows into its buffer.  What may be in flight until then are the eight copies of weights from above.
       products(c1, BLOCKS, c1, w_frag + w_next + place[0], x_frag + ((step & 1) ^ 1) * kStage + place[0], [&](auto I) {
         constexpr int i = decltype(I)::value;
-        if constexpr (i == kBlocks - 1) {
+        if constexpr (i == kBarrier) {
           dma_wait_but<8>();
           workgroup_barrier();
         }
-        if constexpr (i >= 2 * kBlocks) copy_x(std::integral_constant<int, i - 2 * kBlocks>{}, step + 2);
+        if constexpr (i > kBarrier && i <= kBarrier + 2 * kBlocks) copy_x(std::integral_constant<int, i - kBarrier - 1>{}, step + 2);
       });
       w_at = w_next;
     }
     dma_wait_all();                                 // (copies past the last step)
   };
-  switch ((row_end - row0 + 63) / 64) {
-    case 1: run(c1); break;
-    case 2: run(std::integral_constant<int, 2>{}); break;
-    case 3: run(std::integral_constant<int, 3>{}); break;
-    default: run(std::integral_constant<int, 4>{});
-  }
-  // ---- lane: row l32 of a block, weight rows 8 (r / 4) + 4 hi + r % 4; halves of the wave trade runs of four, so that a lane
-  // stores eight outputs in a row.  Gated units of all blocks at once, also of those without rows: one block after the other each waits for its own
-  // exponentials (8 experts of 1500 rows, 320 x 1536, 36.6 us so and 35.9; 700 of 1216 x 896 26.3 and 25.7) ----
+  pairs_of(now, pair);
+  places_of(now);
+  // (a second half without rows is one block whose results are not stored)
+  int row_end = min(now.row0 + now.rows, a.row_start[now.e + 1]), blocks = max((row_end - now.row0 + 63) / 64, 1);
+  copy_first(blocks);
+  for (;;) {
+    const bool more = j < places;
+    int next_end = 0;
+    Tile after{};
+    if (more) {                                     // what the boundary behind this tile needs, here already
+      pairs_of(next, pair);
+      next_end = min(next.row0 + next.rows, a.row_start[next.e + 1]);
+      j += a.groups;
+      if (j < places) find(j, after);
+    }
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    if (!kGlu && row0 + 32 * (wm + 2 * m) >= row_end) break;
-    if constexpr (kGlu == kClampedGlu)
-      if (m == 3) {                                 // not all sums into the other registers at once: there is one too many
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][m][r] = 0.f;
+    switch (blocks) {
+      case 1: run(c1); break;
+      case 2: run(std::integral_constant<int, 2>{}); break;
+      case 3: run(std::integral_constant<int, 3>{}); break;
+      default: run(std::integral_constant<int, 4>{});
+    }
+    workgroup_barrier();                            // the last step's operands have been read
+    const Tile of = now;
+    const int end = row_end;
+    if (more) {
+      now = next;
+      next = after;
+      row_end = next_end;
+      blocks = max((row_end - now.row0 + 63) / 64, 1);
+      places_of(now);
+      copy_first(blocks);
+    }
+    // ---- lane: row l32 of a block, weight rows 8 (r / 4) + 4 hi + r % 4; halves of the wave trade runs of four, so that a lane has eight outputs
+    // in a row, and a block's rows go through LDS, the wave's 8 KB of the third weights' or of the second x buffer, which the next tile's first copies
+    // leave alone, so that a store's lanes are whole rows ----
+    constexpr int kChunks = kGlu ? 8 : 16, kRowsPer = 64 / kChunks;        // 16-byte chunks of a wave's output row; rows of a store
+    auto place_of = [&](int row, int chunk) __attribute__((always_inline)) {
+      return row * (16 * kChunks) + ((chunk ^ ((kGlu ? row >> 1 : row) & (kChunks - 1))) << 4);
+    };
+    const int out_cols = kGlu ? a.N / 2 : a.N, col0 = (of.n_tile * kTile + wn * 128) / (kGlu ? 2 : 1);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      if (of.row0 + 32 * (wm + 2 * m) >= end) break;
+      char* const own = lds + (m & 1 ? 4 : 2) * kStage + 8192 * wave;
+      if constexpr (kGlu != kNoGlu) {                // a block's sums leave their registers only now
 #pragma unroll
         for (int n = 0; n < 4; ++n) asm volatile("" : "+a"(acc[n][m]));
       }
-    const int row = row0 + 32 * (wm + 2 * m) + l32;
-    bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (int64_t)min(row, row_end - 1) * a.out_stride;
 #pragma unroll
-    for (int n = 0; n < (kGlu ? 2 : 4); ++n) {
+      for (int n = 0; n < (kGlu ? 2 : 4); ++n) {
 #pragma unroll
-      for (int r = 0; r < 16; r += 8) {
-        float o[8];
+        for (int r = 0; r < 16; r += 8) {
+          float o[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if constexpr (kGlu) o[i] = glu_of<kGlu>(a, acc[2 * n][m][r + i], acc[2 * n + 1][m][r + i]);
-          else o[i] = acc[n][m][r + i];
+          for (int i = 0; i < 8; ++i) {
+            if constexpr (kGlu) o[i] = glu_of<kGlu>(a, acc[2 * n][m][r + i], acc[2 * n + 1][m][r + i]);
+            else o[i] = acc[n][m][r + i];
+          }
+          const auto x = __builtin_amdgcn_permlane32_swap(pack2<bf16_t>(o[0], o[1]), pack2<bf16_t>(o[4], o[5]), false, false);
+          const auto y = __builtin_amdgcn_permlane32_swap(pack2<bf16_t>(o[2], o[3]), pack2<bf16_t>(o[6], o[7]), false, false);
+          *reinterpret_cast<uint4*>(own + place_of(l32, 4 * n + (r >> 2) + hi)) = make_uint4(x[0], y[0], x[1], y[1]);
         }
-        const auto x = __builtin_amdgcn_permlane32_swap(pack2<bf16_t>(o[0], o[1]), pack2<bf16_t>(o[4], o[5]), false, false);
-        const auto y = __builtin_amdgcn_permlane32_swap(pack2<bf16_t>(o[2], o[3]), pack2<bf16_t>(o[6], o[7]), false, false);
-        const int col = (kGlu ? (n0 + wn * 128) / 2 : n0 + wn * 128) + 32 * n + 2 * r + 8 * hi;
-        if (row < row_end && col < (kGlu ? a.N / 2 : a.N)) *reinterpret_cast<uint4*>(out + col) = make_uint4(x[0], y[0], x[1], y[1]);
       }
+      __builtin_amdgcn_wave_barrier();
+      const int chunk = lane % kChunks, col = col0 + 8 * chunk;
+      const int row = of.row0 + 32 * (wm + 2 * m) + lane / kChunks;
+      bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (int64_t)row * a.out_stride + col;
+#pragma unroll
+      for (int i = 0; i < 32 / kRowsPer; ++i) {
+        const uint4 v = *reinterpret_cast<const uint4*>(own + place_of(kRowsPer * i + lane / kChunks, chunk));
+        if (row + kRowsPer * i < end && col < out_cols) *reinterpret_cast<uint4*>(out + (int64_t)(kRowsPer * i) * a.out_stride) = v;
+      }
+      __builtin_amdgcn_wave_barrier();
     }
+    if (!more) break;
   }
 }
 
@@ -908,9 +1009,11 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
     a.x_bytes = (uint32_t)x_bytes;
     const int64_t blocks = 8 * (((int64_t)a.max_tiles * a.n_tiles + 7) / 8 + 1 + a.n_tiles);
     if (blocks > 0x7fffffff) return MVLLM_ERR_BAD_SHAPE;
+    a.groups = (int)(blocks / 8 < kLargeGroups ? blocks / 8 : kLargeGroups);
+    a.token_factor = 0xffffffffu / (uint32_t)(per_token ? per_token : 1);
     with_glu(glu, [&](auto G) {
       constexpr int kGlu = decltype(G)::value;
-      if (rows == 256) moe_linear_large_kernel<kGlu><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      if (rows == 256) moe_linear_large_kernel<kGlu><<<dim3(8u * (unsigned)a.groups), dim3(256), 0, s>>>(a);
       else if (rows == 128) moe_linear_many_kernel<kGlu, 4><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
       else moe_linear_many_kernel<kGlu, 2><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
     });

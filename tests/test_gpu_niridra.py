@@ -568,6 +568,37 @@ def test_moe_linear_walks_and_shares(counts, n, k, glu):
     assert row_rel(out, want) < 1e-2
 
 
+@pytest.mark.parametrize("counts,n,k,top", [
+    ([1024] * 10, 2048, 64, 1),                                       # 320 tiles, 40 per XCD: one round, eight tiles of the second in halves
+    ([1000] * 10 + [64, 1, 0, 300, 128, 640], 2048, 192, 3),          # the same with tiles that are not whole, halves without rows, few rows behind them
+    ([300, 520, 20, 700] * 20, 1040, 128, 7),                         # last weight tile of 16 outputs; rows are pair / 7
+])
+@pytest.mark.parametrize("glu", [False, True])
+def test_moe_linear_rounds_of_large_tiles(counts, n, k, top, glu):
+    """More tiles of 256 rows than CUs, so that workgroups go from one to the next: every row against the product in float32, whose sums of at most 192
+    numbers differ by less than a rounding to 16 bits (2^-9 of the value), the gated ones by those of its factors."""
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    pairs = sum(counts) // top * top
+    ids = torch.cat([torch.full((c,), i, device=DEV) for i, c in enumerate(counts)])[torch.randperm(sum(counts), generator=g, device=DEV)]
+    ids = ids[:pairs].int().view(-1, top).contiguous()
+    x = torch.randn(pairs // top, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(len(counts), n // 64 * 64 if glu else n, k, generator=g, device=DEV) * k ** -0.5).bfloat16()
+    plan = moe_plan(ids, len(counts))
+    out = moe_linear(x, w, ids, plan, top, glu)[plan.place.long()].float()
+    again = moe_linear(x, w, ids, plan, top, glu)[plan.place.long()].float()
+    assert torch.equal(out, again)
+    want = torch.empty_like(out)
+    for e in range(len(counts)):
+        rows = (ids.view(-1) == e).nonzero().view(-1)
+        z = x[rows // top].float() @ w[e].float().T
+        if glu:
+            gate, up = z.view(len(rows), w.shape[1] // 64, 2, 32).unbind(2)
+            z = (torch.nn.functional.silu(gate) * up).reshape(len(rows), w.shape[1] // 2)
+        want[rows] = z
+    worst = (out - want).abs().amax(1) / want.abs().amax(1)
+    assert worst.max() < 2 ** -8, worst.max()
+
+
 @pytest.mark.parametrize("n,k", [(2560, 128), (2304, 64)])           # products on tiles of 256 rows, and (2304: 576 tiles) on those of 128
 @pytest.mark.parametrize("glu", [False, True])
 @pytest.mark.parametrize("more", [0, 120])
