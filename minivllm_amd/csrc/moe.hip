@@ -866,15 +866,15 @@ static int tile_rows(int64_t pairs, int experts) {
 }
 static int64_t max_tiles(int64_t pairs, int experts, int rows) { return (pairs + rows - 1) / rows + experts; }
 // Whether a product of N outputs runs on the tiles of 256 rows of a plan that has both.  With 48 to 384 rows per expert a large tile has one to four of its
-// blocks of 64 rows; it reads every weight once for the expert's rows and half as much of LDS per flop, but has a CU to itself and 12 us of
-// start and end, so that few of them leave CUs idle or a short last round: they pay from two and a half rounds on, or one and a half of
-// longer ones, where N fills them.  us of both products as 128 and 256 rows, top 4 routed unevenly: 64 experts of 2560 x 4096 and 4096
-// x 1280, 80 rows each 510 / 470, 200 776 / 621; of 1536 x 2048, 56 146 / 144, 160 200 / 177; 128 of 1536 x 2048, 80 310 / 284;
-// but 32 of 1536 x 2048, 80 73 / 82, 64 of 2048 x 1024, 120 121 / 144, 64 of 640 x 1536, 120 59 / 73, 8 of 1536 x 2048, 160 41 / 65.
+// blocks of 64 rows; it reads every weight once for the expert's rows and half as much of LDS per flop, but has a CU to itself: it pays where there is one
+// for each CU and N fills it.  us as 128 and 256 rows, weights from memory, top 4 routed unevenly: 64 experts of 1536 x 2048 with the gate (384 tiles and
+// more), 50 rows each 88 / 84, 80 87 / 94, 120 111 / 102, 340 193 / 169, of 2048 x 768 49 / 46, 57 / 50, 62 / 61, 128 / 99, of 2560 x 4096 271 / 258, 278 /
+// 295, 344 / 319, 646 / 528; 32 of 2048 x 1024 (256 tiles) 41 / 31, 45 / 45, 46 / 49, 82 / 62; but 32 of 1536 x 2048 (192) 41 / 46, 47 / 45, of 640 x 1536
+// 27 / 29, 25 / 32, 26 / 35, 8 of 1536 x 2048 (48) 23 / 25, 340 rows each 29 / 41.
 static bool large_tiles_pay(int64_t pairs, int experts, int N) {
   const int64_t wide = (N + 255) / 256, rows = pairs / 256 + experts / 2, tiles = wide * (rows > experts ? rows : experts);
   if (8 * (256 * wide - N) > N) return false;
-  return tiles >= 640 || (tiles >= 384 && pairs >= 144 * (int64_t)experts);
+  return tiles >= 256;
 }
 static int plan_blocks(int64_t pairs) { return (int)((pairs + kPlanPairs - 1) / kPlanPairs); }
 
