@@ -30,6 +30,30 @@ template <> struct Chunk<bf16_t, 4> {
     store8_stream(p, *reinterpret_cast<const uint2*>(r));
   }
 };
+template <> struct Chunk<float, 8> {
+  static __device__ __forceinline__ void load(const float* p, float* v) {
+    Chunk<float, 4>::load(p, v);
+    Chunk<float, 4>::load(p + 4, v + 4);
+  }
+  static __device__ __forceinline__ void store(float* p, const float* v) {
+    Chunk<float, 4>::store(p, v);
+    Chunk<float, 4>::store(p + 4, v + 4);
+  }
+};
+template <> struct Chunk<bf16_t, 8> {                // (of rows that are read once)
+  static __device__ __forceinline__ void load(const bf16_t* p, float* v) {
+    const uint4 w = load16_stream(p);
+    v[0] = lo_to_float<bf16_t>(w.x); v[1] = hi_to_float<bf16_t>(w.x);
+    v[2] = lo_to_float<bf16_t>(w.y); v[3] = hi_to_float<bf16_t>(w.y);
+    v[4] = lo_to_float<bf16_t>(w.z); v[5] = hi_to_float<bf16_t>(w.z);
+    v[6] = lo_to_float<bf16_t>(w.w); v[7] = hi_to_float<bf16_t>(w.w);
+  }
+  static __device__ __forceinline__ void store(bf16_t* p, const float* v) {
+    bf16_t r[8];
+    for (int i = 0; i < 8; ++i) r[i] = from_float<bf16_t>(v[i]);
+    store16_stream(p, *reinterpret_cast<const uint4*>(r));
+  }
+};
 template <typename T> struct Chunk<T, 1> {
   static __device__ __forceinline__ void load(const T* p, float* v) { v[0] = to_float(*p); }
   static __device__ __forceinline__ void store(T* p, const float* v) { *p = from_float<T>(v[0]); }

@@ -240,6 +240,30 @@ def test_decay_memory_segments_side_by_side(monkeypatch, heads, dim, vdim):
         assert rel(torch.cat(outs[i]), memory_reference(cases[i], heads, dim, vdim, decay)) < 5e-3, i
 
 
+@pytest.mark.parametrize("width", [8, 520, 2048, 2056, 8192, 8200])       # up to 8192 in chunks of eight, where rows are multiples of 16 bytes
+@pytest.mark.parametrize("top", [1, 2, 3, 4, 7, 9])
+@pytest.mark.parametrize("rows,odd", [(5, 0), (5, 4), (530, 0)])
+def test_stream_norm_of_a_mixture_in_wide_chunks(width, top, rows, odd):
+    """Two streams, a shared row behind a gate, choices that hand their input on (their places are -1); the streams are fp32 sums, so 4e-6, the output
+    rounds to 16 bits, 4e-3."""
+    g = gen(width + top)
+    x, y, own = torch.randn(rows, 2, width, generator=g), torch.randn(rows, width, generator=g).bfloat16(), torch.randn(rows, width, generator=g).bfloat16()
+    parts, weights = torch.randn(rows * top, width + odd, generator=g).bfloat16(), torch.rand(rows, top, generator=g)
+    ids = torch.randint(-1, 3, (rows, top), generator=g).int()
+    live = ids.view(-1) >= 0
+    place = torch.full((rows * top,), -1)
+    place[live] = torch.randperm(rows * top, generator=g)[:int(live.sum())]
+    gate, out_w, mix, in_w, scale, gain = (torch.randn(n, generator=g) for n in (rows, 2, 4, 2, width, width))
+    each = torch.where(live[:, None], parts[place.clamp(min=0), :width].double(), own.double().repeat_interleave(top, 0)).view(rows, top, width)
+    total = torch.sigmoid(gate.double())[:, None] * y.double() + (weights.double()[..., None] * each).sum(1)
+    new = torch.einsum("st,nsw->ntw", mix.view(2, 2).double(), x.double()) + out_w.double()[None, :, None] * (scale.double() * total)[:, None]
+    u = (in_w.double()[None, :, None] * new).sum(1)
+    on = lambda t: t.to(DEV)
+    out = ExpertOutput(on(parts)[:, :width], on(weights), on(place.int()), on(y), on(gate), on(ids), on(own))
+    h, mine = stream_norm(on(x), out, on(out_w), on(mix.view(2, 2)), on(gain), 1e-3, on(in_w), on(scale))
+    assert rel(mine, new) < 4e-6 and rel(h, ref.rms(u, 1e-3) * gain.double()) < 4e-3
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("width", [36, 97, 640, 4096, 5000])
 @pytest.mark.parametrize("rows", [3, 600])
