@@ -446,6 +446,30 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
   return most;
 }
 
+// The range of a cached batch, which is even.  A workgroup alone on its CU waits a tile's trip to memory, 0.85 us, so that the longest sequence's chain
+// decides until the CUs have several; `on_cu` is what a CU has in tiles, sequences of log-uniform lengths assumed, the more of them the further
+// below the longest.  A merge takes 1.6 us and each range its partial results' way.  Fitted to 356 random batches, caches cold, and tried on 368 others: on
+// average 1.4 % behind the best range of each (3.8 % before, where a range was at least 6 tiles and batches of more than 192 workgroups were whole).  us
+// before / now, heads of 128: 12 of 755 rows in all, 95 % cached, 32 heads, up to 50 tiles 72.2 / 54; of 572, 37 tiles 55.4 / 38.9; three of 145, 16 tiles 23.2 /
+// 17.9; the worst, nine of 12 tiles, 104 workgroups, 1.19 times as long.  From 193 workgroups on equal ones gain nothing (1500 rows behind 1500, 376
+// workgroups: 72 whole, 86 in two), and few sequences may be equal.
+static int64_t cached_range(int64_t wgs, int64_t tiles, int num_seqs, float fresh, int head_dim, float part_us) {
+  const float on_cu = 1.29f * powf((float)num_seqs, -0.4f) * (1.f - 0.29f * fresh) * (float)(wgs * tiles) / 256.f, per_tile = head_dim == 64 ? 0.58f : 0.85f;
+  auto chain = [&](float x) { return fmaxf(x, on_cu) + 0.7f * fminf(x, on_cu); };
+  int64_t p = (tiles + 1) / 2 * 2;
+  float best = 0.8f;
+  for (int64_t most = kMaxRanges; most > 1; --most) {       // the shortest range that gives so many
+    const int64_t even_tiles = ((tiles + most - 1) / most + 1) / 2 * 2, x = even_tiles < 4 ? 4 : even_tiles, n = (tiles + x - 1) / x;
+    if (x >= tiles) continue;
+    const float gain = per_tile * (chain((float)tiles) - chain((float)x)) - 1.6f - (0.6f + 0.81f * part_us) * (float)n;
+    if (gain > best) {
+      best = gain;
+      p = x;
+    }
+  }
+  return p;
+}
+
 // The range for a batch of these sizes, at least every sequence's tiles where none is cut; 0: the other kernels.
 // Which kernel: the two-group kernel holds one workgroup per CU and runs faster once it has started (906 TFLOP/s against 680), but takes
 // 6 us longer until then, and its longest item decides when there are few.  So this form takes what fits on the chip about at once, two
@@ -481,7 +505,7 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
 // 170 behind as many 27.7 / 22.2, three of 1600 behind 800 90 / 84; none empty: eight of 500 46 / 48).
 // A few rows at head_dim 64 stay there, where placing the bands costs nothing (23 rows 4.8 / 4.8; five sequences of them, 32 heads, 5.2 / 4.9), and so do 200
 // workgroups with more than 7000 keys, whose ranges the other form cuts (800 behind 7600, 32 heads of 128 141 / 144, of 64 94 / 109).
-// Which range: a tile takes a workgroup 0.9 us (0.8 at head_dim 64), workgroups of 0.6 of the longest sequence's tiles each fill 256 CUs;
+// Which range, packed (cached: cached_range): a tile takes a workgroup 0.9 us (0.8 at head_dim 64), workgroups of 0.6 of the longest sequence's tiles each fill 256 CUs;
 // a range brings every row's fp32 partial result into memory and back, about 0.7 of the ranges are there on average.  Batches of more
 // than 192 workgroups gain nothing that the partial results do not cost (1500 rows behind 1500, 32 heads, 376 workgroups: whole 72, two
 // ranges 86).  The other kernels, split keys where they take them, / ranges: 343 rows behind 6500, 16 heads 50 / 43; 870 behind 7800 107 / 81; 132 of
@@ -517,10 +541,12 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
     if (four && crowded && !paged && fresh >= 0.87f && busiest_cu(even, num_seqs, fresh) > (num_seqs <= 3 ? 1.87f : 2.9f)) return 0;
   }
   int64_t p = (tiles + 1) / 2 * 2;
+  if (paged && (wgs <= 192 || num_seqs >= 5))
+    p = cached_range(wgs, tiles, num_seqs, fresh, head_dim, 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f);
   if (wgs > 192) return (four || head_dim == 64) && tiles > 112 ? 0 : (int)p;
   const float per_tile = head_dim == 64 ? 0.8f : 0.9f, per_range = 0.3f + 0.7f * 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f;
   float best = 3.f;
-  for (int64_t most = kMaxRanges; most > 1; --most) {       // the shortest range that gives so many
+  for (int64_t most = kMaxRanges; !paged && most > 1; --most) {       // the shortest range that gives so many
     const int64_t even_tiles = ((tiles + most - 1) / most + 1) / 2 * 2, x = even_tiles < 6 ? 6 : even_tiles, n = (tiles + x - 1) / x;
     if (x >= tiles) continue;
     const float gain = per_tile * ((float)tiles - fmaxf((float)x, 0.6f * (float)(wgs * tiles) / 256.f)) - 4.f - per_range * (float)n;
