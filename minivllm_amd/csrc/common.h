@@ -275,6 +275,14 @@ struct StoreBeside {
 // Varlen causal prefill in the two-group form (prefill_pingpong.hip): one persistent 8-wave workgroup per CU whose two
 // wave groups alternate between the matrix unit and the softmax.  Launched from the prefill entry point for the batches
 // it takes; everything else stays on prefill_mfma_kernel.
+// Windows (launch_prefill_pp_window): where rows and heads lie, all in bytes; query row r of a sequence with n queries and m keys sits at key m - n + r and
+// sees the `window` keys up to it.
+struct PpWindow {
+  const void* gate;         // [total_q rows, heads] 16-bit numbers, the result times their sigmoid, or null
+  int64_t q_head, k_head, v_head, out_head;
+  int q_row, k_row, v_row, out_row, gate_row;
+  int window;
+};
 struct PrefillPpArgs {
   void* out;
   const void* q;
@@ -307,9 +315,13 @@ struct PrefillPpArgs {
   int timeline_entries;
   int timeline_block;
   StoreBeside store;      // packed batches
+  PpWindow win;           // windows: keys of a sequence at cu_seqlens_k
 };
 // block_size: 0 for the packed entry point
 bool prefill_pp_takes(int num_seqs, int num_heads, int num_kv_heads, int head_dim, int dtype, int block_size);
 int launch_prefill_pp(const PrefillPpArgs& a, int dtype, hipStream_t stream);
+// Windows over packed keys: bf16, shapes as prefill_pp_takes, rows of 16-byte multiples, windows of kPpLeastWindow keys at least.
+constexpr int kPpLeastWindow = 256;
+int launch_prefill_pp_window(const PrefillPpArgs& a, hipStream_t stream);
 
 }  // namespace mvllm

@@ -77,6 +77,7 @@ struct PpItems {
 };
 struct PpItem {
   int seq_start, seq_len, rb;   // the sequence's query rows; the item's 64-row block of them
+  int first;          // windows: index of the item's first key tile
   int nt;             // index of the item's last key tile ( = rb without a cached prefix)
   int kvh, h0;        // kv head; first of the item's four query heads
   int seq, cached;    // paged mode: the sequence's row in the block table, its cached tokens
@@ -98,9 +99,16 @@ __device__ __forceinline__ unsigned div_small(unsigned x, unsigned d, unsigned m
 // 64 GRP + 32 ((w % 4) / 2) ...; the block's last key tile is then the index of its second 64-row step, the
 // diagonal crosses its last two tiles (three over a prefix in general position), and the waves of its first 64 rows
 // compute a last tile they see nothing of.
-template <typename T, int D, int GRP, bool PAGED, int HPI>
+//
+// WIN: sliding windows over packed keys (PpWindow).  Positions as over a cached prefix, keys of a sequence at cu_seqlens_k; an item's tiles begin with
+// the one that holds its first row's first key, and up to the one that holds its last row's, a row may have seen nothing yet.  Those and the
+// tiles of the causal limit are taken with both masks and look at their maximum (a row's first keys set it, wherever it lies); the
+// ones between are ordinary ones.
+template <typename T, int D, int GRP, bool PAGED, int HPI, bool WIN>
 __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, const int wave) {
   static_assert(HPI == 4 || HPI == 2, "items of four or of two query heads");
+  static_assert(!WIN || !PAGED, "windows: packed keys");
+  constexpr bool kBehind = PAGED || WIN;       // queries may lie behind cached keys
   constexpr int kTPB = 4 / HPI;                // 64-row steps (and diagonal key tiles) per item
   constexpr int kRPI = 64 * kTPB;              // query rows per item
   constexpr int kRowB = D * 2;
@@ -136,12 +144,13 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
 #define TCOUNT(items, tiles) do {} while (0)
 #endif
   // ---- the batch, one sequence per lane ----
-  int lo = 0, len = 0, cached = 0, kv_len = 0;
+  int lo = 0, len = 0, cached = 0, kv_len = 0, k_lo = 0;
   if (lane < a.num_seqs) {
     lo = a.cu_seqlens[lane];
     len = a.cu_seqlens[lane + 1] - lo;
-    if (PAGED) {
-      kv_len = a.cu_seqlens_k[lane + 1] - a.cu_seqlens_k[lane];
+    if (kBehind) {
+      k_lo = a.cu_seqlens_k[lane];
+      kv_len = a.cu_seqlens_k[lane + 1] - k_lo;
       cached = kv_len > len ? kv_len - len : 0;
     }
   }
@@ -151,9 +160,16 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
   const int lvl0 = (cached + kRPI - 1) >> 6;
   const int lvl_end = nb > 0 ? lvl0 + kTPB * (nb - 1) + 1 : 0;
   int top = 0;                                 // one past the highest level in the batch
-  for (int bit = a.level_bits - 1; bit >= 0; --bit) {
-    const int trial = top | (1 << bit);
-    if (__ballot(lvl_end >= trial) != 0ull) top = trial;
+  if constexpr (WIN) {                         // (the host does not know how many keys there are)
+    top = lvl_end;
+#pragma unroll
+    for (int step = 1; step < 64; step <<= 1) top = max(top, __shfl_xor(top, step, 64));
+    top = __builtin_amdgcn_readfirstlane(top);
+  } else {
+    for (int bit = a.level_bits - 1; bit >= 0; --bit) {
+      const int trial = top | (1 << bit);
+      if (__ballot(lvl_end >= trial) != 0ull) top = trial;
+    }
   }
 
   // ---- which items are this workgroup's ----
@@ -186,6 +202,14 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     const unsigned R = round * TS + (backwards ? TS - 1u - t : t);
     unsigned long long mask = 0ull;
     unsigned cnt = 0;
+    if constexpr (WIN) {                       // one sequence: one item per slice and level, so the item's level follows
+      if (a.num_seqs == 1 && walk.level >= 0) {
+        const unsigned levels = div_small(R - walk.base, spt, a.spt_magic);
+        walk.base += levels * spt;
+        walk.level -= (int)levels * kTPB;
+        if (walk.level < __builtin_amdgcn_readfirstlane(lvl0)) walk.level = -1;
+      }
+    }
     while (walk.level >= 0) {
       mask = __ballot(walk.level < lvl_end && walk.level >= lvl0 && (kTPB == 1 || ((walk.level - lvl0) & (kTPB - 1)) == 0));
       cnt = (unsigned)__popcll(mask);
@@ -215,7 +239,7 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     kept_len = lane == at ? seq_len : kept_len;
     kept_rb = lane == at ? walk.level : kept_rb;     // -1: no such item
     kept_heads = lane == at ? heads : kept_heads;
-    if (PAGED) kept_seq = lane == at ? seq : kept_seq;
+    if (kBehind) kept_seq = lane == at ? seq : kept_seq;
     ++produced;
   };
   auto item_at = [&](int k) {
@@ -230,11 +254,13 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     it.h0 = heads & 0xffff;
     it.valid = it.nt >= 0;
     it.seq = 0; it.cached = 0;
-    if (PAGED) {
+    if (kBehind) {
       it.seq = __builtin_amdgcn_readlane(kept_seq, at);
       it.cached = __builtin_amdgcn_readlane(cached, it.seq);
     }
     it.rb = (it.nt - ((it.cached + kRPI - 1) >> 6)) / kTPB;
+    it.first = 0;
+    if constexpr (WIN) it.first = max(it.cached + kRPI * it.rb - a.win.window + 1, 0) >> 6;
     return it;
   };
 
@@ -244,13 +270,13 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
   PpItem nxt = item_at(ci++);
   int di = 0;
   PpItem dit = cur;                            // item the copy cursor is in
-  int dj = 0;                                  // ... and its tile there
+  int dj = WIN ? dit.first : 0;                // ... and its tile there
 
   const T* qg = reinterpret_cast<const T*>(a.q);
   const char* kg = reinterpret_cast<const char*>(a.k);
   const char* vg = reinterpret_cast<const char*>(a.v);
-  const int kv_row_bytes = a.num_kv_heads * kRowB;
-  const int q_row_bytes = a.num_heads * kRowB;
+  const int kv_row_bytes = !WIN ? a.num_kv_heads * kRowB : GRP == 0 ? a.win.k_row : a.win.v_row;
+  const int q_row_bytes = WIN ? a.win.q_row : a.num_heads * kRowB, out_row_bytes = WIN ? a.win.out_row : q_row_bytes;
   const int total_rows = (int)a.total_tokens;
 
   // ---- copies ----
@@ -298,6 +324,10 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     d_head_off = dit.kvh * kRowB;
     if constexpr (PAGED) {
       d_kv_len = dit.valid ? __builtin_amdgcn_readlane(kv_len, dit.seq) : 0;
+    } else if constexpr (WIN) {                // (rows left: of the sequence)
+      const int seq = dit.valid ? dit.seq : 0, first = kPpBN * dit.first;
+      d_off = (int64_t)(__builtin_amdgcn_readlane(k_lo, seq) + first) * kv_row_bytes + (int64_t)dit.kvh * (GRP == 0 ? a.win.k_head : a.win.v_head);
+      d_rows_left = dit.valid ? __builtin_amdgcn_readlane(kv_len, seq) - first : 0;
     } else {
       d_off = (int64_t)dit.seq_start * kv_row_bytes + d_head_off;
       d_rows_left = dit.valid ? total_rows - dit.seq_start : 0;
@@ -315,6 +345,8 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       const uint32_t size = ok ? (uint32_t)(valid - 1) * (uint32_t)kv_row_bytes + (uint32_t)kRowB : 0u;
       const int64_t start = ok ? (int64_t)d_phys * a.block_bytes + d_in_off : 0;
       r = make_rsrc(copy_src + start, size);
+    } else if constexpr (WIN) {
+      r = make_rsrc(copy_src + d_off, d_rows_left > 0 ? (uint32_t)(min(d_rows_left, kPpBN) - 1) * (uint32_t)kv_row_bytes + (uint32_t)kRowB : 0u);
     } else {
       const uint32_t size = d_rows_left <= 0        ? 0u
                             : d_rows_left > rows_4g ? 0xffffffffu
@@ -331,7 +363,7 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     if (dit.valid) {
       if (++dj > dit.nt) {
         dit = item_at(++di);
-        dj = 0;
+        dj = WIN ? dit.first : 0;
         enter_item();
       } else if constexpr (!PAGED) {
         d_off += (int64_t)kPpBN * kv_row_bytes;      // the next 64 rows of the same sequence and head
@@ -360,9 +392,10 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     const int rows_left = total_rows - row;
     const int rows_4g = (int)(0xffffffffu / (uint32_t)q_row_bytes);
     const uint32_t size = rows_left <= 0 ? 0u
+                          : WIN ? (uint32_t)(min(rows_left, 32) - 1) * (uint32_t)q_row_bytes + (uint32_t)kRowB
                           : rows_left > rows_4g ? 0xffffffffu
                                                 : (uint32_t)rows_left * (uint32_t)q_row_bytes - (uint32_t)(h * kRowB);
-    const v4i r = make_rsrc(reinterpret_cast<const char*>(qg) + (int64_t)row * q_row_bytes + (int64_t)h * kRowB, size);
+    const v4i r = make_rsrc(reinterpret_cast<const char*>(qg) + (int64_t)row * q_row_bytes + (int64_t)h * (WIN ? a.win.q_head : (int64_t)kRowB), size);
     int lane_q = lane;
     asm volatile("" : "+v"(lane_q));              // the eight source offsets are computed per item, not kept in registers
     const int qrow = lane_q >> 4, qchunk = lane_q & 15;
@@ -487,14 +520,14 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     // The descriptor ends with the head's part of the sequence's last row, so the stores of rows past it are dropped
     // by the bounds check: all eight are always issued, as the wait counts assume.
     const int rows = seq_len - r0 < 32 ? seq_len - r0 : 32;
-    const uint32_t size = rows > 0 ? (uint32_t)(rows - 1) * (uint32_t)q_row_bytes + (uint32_t)kRowB : 0u;
-    char* base = reinterpret_cast<char*>(out) + (int64_t)(seq_start + r0) * q_row_bytes + (int64_t)(h0 + wh) * kRowB;
-    const uint32_t off0 = (uint32_t)(orow * q_row_bytes + 16 * ochunk);
+    const uint32_t size = rows > 0 ? (uint32_t)(rows - 1) * (uint32_t)out_row_bytes + (uint32_t)kRowB : 0u;
+    char* base = reinterpret_cast<char*>(out) + (int64_t)(seq_start + r0) * out_row_bytes + (int64_t)(h0 + wh) * (WIN ? a.win.out_head : (int64_t)kRowB);
+    const uint32_t off0 = (uint32_t)(orow * out_row_bytes + 16 * ochunk);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int row = 4 * i + orow;
       const uint4 w = *reinterpret_cast<const uint4*>(ot + row * kRowB + ((ochunk ^ kswz(row)) << 4));
-      store16_buffer(base, size, off0 + (uint32_t)(4 * i) * (uint32_t)q_row_bytes, w);
+      store16_buffer(base, size, off0 + (uint32_t)(4 * i) * (uint32_t)out_row_bytes, w);
     }
   };
   // The barrier that ends a softmax interval publishes the copy step issued in the wave's previous softmax interval:
@@ -503,7 +536,9 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
   // whatever the sequence's length, so the count is exact) must have completed.  (Letting the previous interval's
   // stores and Q copies stay in flight as well was measured and is slower.)
   auto wait_copies = [&](int later) {
-    if (later == 4) vm_wait<4>();
+    if (WIN && later == 13) vm_wait<13>();
+    else if (WIN && later == 21) vm_wait<21>();
+    else if (later == 4) vm_wait<4>();
     else if (later == 12) vm_wait<12>();
     else if (later == 20) vm_wait<20>();
     else vm_wait<0>();
@@ -549,6 +584,17 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       for (int r = 0; r < 16; ++r)
         if (32 * tk + 8 * (r >> 2) + (r & 3) > lim) s[tk][r] = -INFINITY;
   };
+  // ... and against the window's lower end, which tiles up to window_low() may hold
+  auto window_low = [&]() { return (cur.cached + kRPI * (cur.rb + 1) - 1 - a.win.window) >> 6; };
+  auto mask_window = [&](int j) {
+    int lim = cur.cached + kPpBN * (kTPB * cur.rb - j) + row_off + l32 - 4 * hi;
+    asm volatile("" : "+v"(lim));
+#pragma unroll
+    for (int tk = 0; tk < 2; ++tk)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)               // 0 <= distance < window
+        if ((unsigned)(lim - (32 * tk + 8 * (r >> 2) + (r & 3))) >= (unsigned)a.win.window) s[tk][r] = -INFINITY;
+  };
   auto tile_max = [&]() {                        // maximum of the lane's row over the tile, relative to the running one
     const float mx0 = fmaxf(s[0][15], s[1][15]);
     float mx = mx0, mx1 = mx0;
@@ -588,6 +634,26 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
         pf[2 * tk + st] = p;
       }
     return sum;
+  };
+  // Windows: the lane's row's gate, asked for in the item's first softmax interval.  It counts as one vector memory instruction in front of that
+  // interval's copy step; the compiler, which does not see the copies, sees the eight output stores behind it and waits for all but eight.
+  uint32_t gate_bits = 0;
+  bool empty = false;                            // windows: the lane's row has seen no key yet
+  auto load_gate = [&]() {
+    if constexpr (WIN) {
+      const int row = cur.rb * kRPI + row_off, rows = cur.seq_len - row < 32 ? cur.seq_len - row : 32;
+      char* base = reinterpret_cast<char*>(const_cast<void*>(a.win.gate)) + (int64_t)(cur.seq_start + row) * a.win.gate_row + 2 * (cur.h0 + wh);
+      const uint32_t size = a.win.gate && rows > 0 ? (uint32_t)(rows - 1) * (uint32_t)a.win.gate_row + 2u : 0u;
+      gate_bits = __builtin_amdgcn_raw_buffer_load_b16(__builtin_amdgcn_make_buffer_rsrc(base, 0, (int)size, 0x00020000), l32 * a.win.gate_row, 0, 0);
+    }
+  };
+  auto row_factor = [&]() {                      // what an output row is multiplied with
+    const float inv = __builtin_amdgcn_rcpf(sum_with_lane_xor32(l));
+    if constexpr (WIN) {
+      const float sig = __builtin_amdgcn_rcpf(1.f + __expf(-lo_to_float<T>(gate_bits)));
+      return a.win.gate ? inv * sig : inv;
+    }
+    return inv;
   };
   auto set_neg_m = [&](float v) {
 #pragma unroll
@@ -682,7 +748,7 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       if (last) {                                // a single tile: no other work to hide these behind
         vm_wait<0>();
         load_q();
-        inv = __builtin_amdgcn_rcpf(sum_with_lane_xor32(l));
+        inv = row_factor();
         static_for<4>([&](auto TD) { stage_out(TD, inv); });
       }
     }
@@ -691,7 +757,7 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       // them
       vm_wait<4>();
       read_q();
-      inv = __builtin_amdgcn_rcpf(sum_with_lane_xor32(l));
+      inv = row_factor();
       scale_q(I0{});
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -749,7 +815,14 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     TSTAMP();
     if constexpr (decltype(INSIDE)::value) copy_step_inside();
     else copy_step();
-    if constexpr (PAGED || HPI != 4) {
+    if constexpr (WIN && HPI == 4) {
+      if constexpr (decltype(LAST)::value) {
+        if ((cur.cached & 63) != 0) mask_tile(j);
+        else mask_diagonal();
+      } else if constexpr (decltype(MASKED)::value) {
+        mask_tile(j);
+      }
+    } else if constexpr (PAGED || HPI != 4) {
       if constexpr (decltype(LAST)::value) mask_tile(j);
       else if constexpr (decltype(MASKED)::value) {
         if (HPI != 4 || (cur.cached & 63) != 0) mask_tile(j);
@@ -786,23 +859,60 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     TSTAMP();
   };
 
+  // Windows: the same for a tile in which a row may see its first key.
+  auto early_tile = [&](int j, uint4 (&vf0)[kTD], uint4 (&vf1)[kTD]) {
+    TSTAMP();
+    copy_step();
+    if (j <= window_low()) mask_window(j);
+    const float mx = tile_max();
+    const float d = empty ? (mx == -INFINITY ? 0.f : mx) : mx > 8.f ? mx : 0.f;
+    if (__any(d != 0.f)) {                       // a row's first keys set its maximum, wherever that lies
+      const float alpha = empty ? 1.f : fast_exp2(-d);
+      l *= alpha;
+#pragma unroll
+      for (int td = 0; td < kTD; ++td)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[td][r] *= alpha;
+      set_neg_m(neg_m[0] - d);
+    }
+    empty = empty && mx == -INFINITY;
+    l += weights(std::true_type{}, d);
+    pin_weights();
+    TSTAMP();
+    v_frags(c_slot, std::integral_constant<int, 0>{}, vf0);
+    v_frags(c_slot, std::integral_constant<int, 1>{}, vf1);
+    vm_wait<4>();
+    pp_barrier();
+    TSTAMP();
+  };
+
   while (true) {
     // ======== first tile of an item ========
-    const bool single = cur.nt == 0;
-    int trail = 0;                               // vector memory instructions behind this interval's copy step
+    const bool single = cur.nt == (WIN ? cur.first : 0);
+    int trail = 0;                               // vector memory instructions behind this interval's copy step (windows: and one in front of it)
     TSTAMP();
+    if constexpr (WIN) {
+      load_gate();
+      trail = 1;
+    }
     copy_step();
     // tiles at the item's end that the diagonal may cross (items of four heads without a prefix: the last one, by
     // mask_diagonal)
-    const int masked_tail = kTPB + (PAGED && (cur.cached & 63) != 0 ? 1 : 0);
-    if constexpr (PAGED || HPI != 4) {
+    const int masked_tail = kTPB + (kBehind && (cur.cached & 63) != 0 ? 1 : 0);
+    if constexpr (WIN) {
+      if (cur.first <= window_low() || cur.first > cur.nt - masked_tail) mask_window(cur.first);
+    } else if constexpr (PAGED || HPI != 4) {
       if (cur.nt < masked_tail) mask_tile(0);
     } else if (single) {
       mask_diagonal();
     }
-    const float mx_first = tile_max();           // neg_m is zero here: the tile's maximum itself
+    float mx_first = tile_max();                 // neg_m is zero here: the tile's maximum itself
+    if constexpr (WIN) {
+      empty = mx_first == -INFINITY;
+      mx_first = empty ? 0.f : mx_first;
+    }
     // the item before this one leaves (its output was staged in the slot during the interval before) ...
-    if (have_prev) {
+    if (WIN || have_prev) {                      // (windows: in front of the first item nothing, as eight stores that are dropped)
       write_out(p_seq_start, p_seq_len, p_rb, p_h0);
       trail += 8;
     }
@@ -825,7 +935,27 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     bool more = matrix_interval(std::true_type{}, std::false_type{}, single, vf0, vf1);
     if (!single) {
       // ======== the item's other tiles ========
-      if constexpr (HPI == 4) {
+      if constexpr (WIN) {
+        // tiles in which a row may see its first key; ordinary ones; those of the causal limit
+        const int seen = (cur.cached + kRPI * (cur.rb + 1) - a.win.window) >> 6, plain_end = cur.nt - masked_tail + 1;
+        int j = cur.first + 1;
+        for (; j <= seen; ++j) {                 // (before those of the causal limit: kPpLeastWindow)
+          early_tile(j, vf0, vf1);
+          matrix_interval(std::false_type{}, std::false_type{}, false, vf0, vf1);
+        }
+        for (; j < cur.nt - 2 && j < plain_end; ++j) {       // the copy cursor stays inside this item
+          later_tile(std::false_type{}, std::false_type{}, std::true_type{}, j, vf0, vf1);
+          matrix_interval(std::false_type{}, std::false_type{}, false, vf0, vf1);
+        }
+        for (; j < plain_end; ++j) {
+          later_tile(std::false_type{}, std::false_type{}, std::false_type{}, j, vf0, vf1);
+          matrix_interval(std::false_type{}, std::false_type{}, false, vf0, vf1);
+        }
+        for (; j < cur.nt; ++j) {
+          later_tile(std::false_type{}, std::true_type{}, std::false_type{}, j, vf0, vf1);
+          matrix_interval(std::false_type{}, std::false_type{}, false, vf0, vf1);
+        }
+      } else if constexpr (HPI == 4) {
         const int plain_end = PAGED ? cur.nt - 1 : cur.nt;
         int j = 1;
         for (; j < cur.nt - 2; ++j) {              // the copy cursor stays inside this item
@@ -860,7 +990,7 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       later_tile(std::true_type{}, std::true_type{}, std::false_type{}, cur.nt, vf0, vf1);
       more = matrix_interval(std::false_type{}, std::true_type{}, false, vf0, vf1);
     }
-    TCOUNT(1, cur.nt + 1);
+    TCOUNT(1, cur.nt - (WIN ? cur.first : 0) + 1);
     p_seq_start = cur.seq_start; p_seq_len = cur.seq_len; p_rb = cur.rb; p_h0 = cur.h0;
     have_prev = true;
     if (!more) break;
@@ -890,8 +1020,15 @@ __global__ __launch_bounds__(64 * kPpWaves, 1) void prefill_pp_kernel(const Pref
       return;
     }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (wave < 4) pp_run<T, D, 0, PAGED, HPI>(a, lds, wave);
-  else pp_run<T, D, 1, PAGED, HPI>(a, lds, wave);
+  if (wave < 4) pp_run<T, D, 0, PAGED, HPI, false>(a, lds, wave);
+  else pp_run<T, D, 1, PAGED, HPI, false>(a, lds, wave);
+}
+template <typename T, int D, int HPI>
+__global__ __launch_bounds__(64 * kPpWaves, 1) void window_pp_kernel(const PrefillPpArgs a) {
+  __shared__ __attribute__((aligned(1024))) PpLds<D> lds;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wave < 4) pp_run<T, D, 0, false, HPI, true>(a, lds, wave);
+  else pp_run<T, D, 1, false, HPI, true>(a, lds, wave);
 }
 
 template <typename T>
@@ -913,10 +1050,11 @@ bool prefill_pp_takes(int num_seqs, int num_heads, int num_kv_heads, int head_di
   return group % 2 == 0 && (int64_t)num_heads * head_dim * 2 * 64 < ((int64_t)1 << 31);
 }
 
-int launch_prefill_pp(const PrefillPpArgs& args, int dtype, hipStream_t stream) {
-  PrefillPpArgs a = args;
+static int pp_heads(int group) { return group % 4 == 0 ? 4 : 2; }      // query heads per item
+// The workgroups and what of an item's place is worked out here.
+static int pp_grid(PrefillPpArgs& a) {
   const int group = a.num_heads / a.num_kv_heads;
-  const int hpi = group % 4 == 0 ? 4 : 2;             // query heads per item
+  const int hpi = pp_heads(group);
   a.slices = a.num_kv_heads * (group / hpi);
   int n_teams = 8;
   while (a.slices % n_teams != 0) n_teams >>= 1;      // gcd(8, slices)
@@ -933,8 +1071,14 @@ int launch_prefill_pp(const PrefillPpArgs& args, int dtype, hipStream_t stream) 
   auto magic = [](int d) { return d <= 1 ? 0u : (unsigned)(((uint64_t)1 << 32) / (uint64_t)d + 1u); };
   a.spt_magic = magic(a.slices / n_teams);
   a.chunks_magic = magic(group / hpi);
+  return grid;
+}
+
+int launch_prefill_pp(const PrefillPpArgs& args, int dtype, hipStream_t stream) {
+  PrefillPpArgs a = args;
+  const int grid = pp_grid(a), hpi = pp_heads(a.num_heads / a.num_kv_heads);
   const bool paged = a.block_tables != nullptr;
-  a.block_magic = magic(a.block_size);
+  a.block_magic = a.block_size <= 1 ? 0u : (unsigned)(((uint64_t)1 << 32) / (uint64_t)a.block_size + 1u);
   a.block_bytes = a.block_size * a.num_kv_heads * 128 * 2;
   a.num_blocks32 = a.num_blocks > 0x7fffffff ? 0x7fffffff : (int)a.num_blocks;
   // levels: one past the last key tile of the longest possible sequence (paged: as wide as its block-table row).  An
@@ -948,6 +1092,16 @@ int launch_prefill_pp(const PrefillPpArgs& args, int dtype, hipStream_t stream) 
   const dim3 b(64 * kPpWaves);
   if (dtype == MVLLM_BF16) launch_prefill_pp_as<bf16_t>(a, paged, hpi, g, b, stream);
   else launch_prefill_pp_as<f16_t>(a, paged, hpi, g, b, stream);
+  return launch_status();
+}
+
+// bf16 (the caller has looked at shapes, strides and alignment).  Windows of kPpLeastWindow keys and more: an item's tiles in which a row may see its first
+// key are none of the causal limit's.
+int launch_prefill_pp_window(const PrefillPpArgs& args, hipStream_t stream) {
+  PrefillPpArgs a = args;
+  const dim3 g(pp_grid(a)), b(64 * kPpWaves);
+  if (pp_heads(a.num_heads / a.num_kv_heads) == 4) window_pp_kernel<bf16_t, 128, 4><<<g, b, 0, stream>>>(a);
+  else window_pp_kernel<bf16_t, 128, 2><<<g, b, 0, stream>>>(a);
   return launch_status();
 }
 

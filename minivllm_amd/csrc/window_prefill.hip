@@ -96,6 +96,38 @@ static int launch_shared(const WindowPrefillArgs& a, hipStream_t s) {
   }
 }
 
+__attribute__((weak)) bool prefill_pp_takes(int, int, int, int, int, int) { return false; }
+__attribute__((weak)) int launch_prefill_pp_window(const PrefillPpArgs&, hipStream_t) { return MVLLM_ERR_UNSUPPORTED; }
+
+// Heads with values of their own on the two-group kernel (prefill_pingpong.hip), or kNoTiles: head_dim 128, an even number of query heads per kv head, at
+// most 64 sequences, no gate or one number per head, and batches that keep its 256 workgroups busy.  An item there (four heads by 64 rows, two by
+// 128) costs five tiles of its own beside those of its window, where the other kernel's waves share a CU's LDS and read every tile whole: us there / here, four
+// heads per kv head (32 over 8), windows of 256 / 1024 / 2048: eight prompts of 300 (304 items) 28.9 / 19.5, 1000 of them (1032) 73 / 59, 100 / 78, 100 / 78, five
+// of 708 to 3170 (980) 79 / 64, 121 / 101, 152 / 121, one of 8000 (1000) 74 / 61, 149 / 132, 245 / 212, three of 2174 rows (272) 1.31 / 1.34 / 1.09 times as
+// fast, two of 1000 (258) 22.1 / 20.3, 30.6 / 30.3, 30.8 / 30.7; but one of 1000 (128) 15.4 / 17.9, 25.2 / 28.0, two of 1780 rows (224) 1.03 / 0.97 / 0.92.  Two heads
+// (16 over 8): eight of 1000 (532) 43 / 41, 55 / 47, 55 / 48, one of 8000 (504) 45 / 44, 85 / 77, 137 / 120, but five of 9637 rows (616) 0.88 / 0.96 / 1.04, two of
+// 9584 (600) 0.78 / 0.93 / 0.99, one of 3000 (191) 22.5 / 22.8, 42 / 37, 51 / 53, two of 3000 (383) 37 / 43, 65 / 67, 89 / 72.
+static bool two_group_pays(const WindowPrefillArgs& a) {
+  const int group = a.heads / a.kv_heads, heads = group % 4 == 0 ? 4 : 2;
+  const int64_t items = (a.total_q * heads / 256 + a.num_seqs / 2) * (a.heads / heads);
+  return heads == 4 ? items >= 256 && (a.window == 0 || a.window >= kPpLeastWindow) : items >= 448 && (a.window == 0 || a.window >= 2048);
+}
+static int launch_two_group(const WindowPrefillArgs& a, hipStream_t s) {
+  constexpr int64_t kMostRow = (int64_t)1 << 24;     // bytes of a row: 64 of them in 31 bits
+  const int64_t rows[] = {a.q_row, a.k_row, a.v_row, a.out_row, a.gate ? a.gate_row : 0};
+  if (!two_group_pays(a) || a.k2 || a.slopes || a.temp_every > 0.f || (a.gate && a.gate_head != 1) || !prefill_pp_takes(a.num_seqs, a.heads, a.kv_heads, a.dim, MVLLM_BF16, 0)) return kNoTiles;
+  for (int64_t x : rows)
+    if (2 * x > kMostRow) return kNoTiles;
+  PrefillPpArgs p = {};
+  p.out = a.out; p.q = a.q; p.k = a.k; p.v = a.v; p.cu_seqlens = a.cu_q; p.cu_seqlens_k = a.cu_k; p.total_tokens = a.total_q;
+  p.num_seqs = a.num_seqs; p.num_heads = a.heads; p.num_kv_heads = a.kv_heads; p.scale_log2 = a.scale_log2;
+  p.win.gate = a.gate; p.win.gate_row = a.gate ? (int)(2 * a.gate_row) : 0;
+  p.win.q_row = (int)(2 * a.q_row); p.win.k_row = (int)(2 * a.k_row); p.win.v_row = (int)(2 * a.v_row); p.win.out_row = (int)(2 * a.out_row);
+  p.win.q_head = 2 * a.q_head; p.win.k_head = 2 * a.k_head; p.win.v_head = 2 * a.v_head; p.win.out_head = 2 * a.out_head;
+  p.win.window = a.window > 0 ? a.window : 0x3fffffff;
+  return launch_prefill_pp_window(p, s);
+}
+
 __attribute__((weak)) int launch_window_prefill_parts(const WindowPrefillArgs&, hipStream_t) { return kNoTiles; }
 __attribute__((weak)) int launch_window_prefill_heads(const WindowPrefillArgs&, hipStream_t) { return kNoTiles; }
 
@@ -133,7 +165,9 @@ extern "C" int mvllm_window_prefill(void* out, int64_t out_row_stride, int64_t o
   bool tiles = dtype == MVLLM_BF16 && aligned16(out) && aligned16(q) && aligned16(k) && aligned16(k2) && aligned16(v) && (one_gate || aligned16(gate)) &&
                k_row_stride < (1 << 24) && k2_row_stride < (1 << 24) && v_row_stride < (1 << 24) && (v || !k2) && !(v && slopes);
   for (int64_t x : strides) tiles = tiles && x % 8 == 0;
-  const int st = !tiles ? kNoTiles : k2 ? launch_window_prefill_parts(a, s) : v ? launch_window_prefill_heads(a, s) : launch_shared(a, s);
+  int st = tiles && v ? launch_two_group(a, s) : kNoTiles;
+  if (st != kNoTiles) return st;
+  st = !tiles ? kNoTiles : k2 ? launch_window_prefill_parts(a, s) : v ? launch_window_prefill_heads(a, s) : launch_shared(a, s);
   if (st != kNoTiles) return st;
   return dtype == MVLLM_F32 ? launch_any<float>(a, s) : launch_any<bf16_t>(a, s);
 }

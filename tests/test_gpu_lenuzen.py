@@ -229,6 +229,48 @@ def test_window_prefill_of_keys_and_values(dtype, window, heads, groups, dim):
             assert rel(out[a], want) < tol(dtype, 3e-6, 1.5e-2), e
 
 
+def window_reference_on_gpu(q, k, v, scale, window, gate):
+    n, m, group = q.shape[0], k.shape[0], q.shape[1] // k.shape[1]
+    away = torch.arange(m - n, m, device=DEV)[:, None] - torch.arange(m, device=DEV)[None]
+    see, out = (away >= 0) & ((away < window) if window else True), []
+    for h in range(q.shape[1]):
+        s = (q[:, h].double() @ k[:, h // group].double().T * scale).masked_fill(~see, float("-inf"))
+        out.append(torch.softmax(s, -1) @ v[:, h // group].double())
+    out = torch.stack(out, 1)
+    return out if gate is None else out * torch.sigmoid(gate.double())[..., None]
+
+
+@pytest.mark.parametrize("heads,groups,window", [(64, 2, w) for w in (0, 256, 257, 320, 511, 512, 1000)] + [(60, 2, w) for w in (0, 2048, 2111)])
+@pytest.mark.parametrize("shift", [0, -128, 128])
+@pytest.mark.parametrize("gated", [True, False])
+def test_window_prefill_of_many_heads(heads, groups, window, shift, gated):
+    """Batches for the kernel with two groups of waves (at least 256 items of four heads by 64 rows, or 448 of two by 128): portions and pasts of any
+    length, the window's end anywhere in a tile, rows that see nothing of their item's first tiles.  ``shift`` moves all scores of a row by 16 * shift *
+    scale (181 to either side), which the softmax does not see: a row's maximum has to come from its own first keys."""
+    dim, g = 128, gen(heads + window + shift)
+    lens, pasts = [1, 63, 700, 64, 65, 131, 128, 400], [0, 5, 64, 300, 2200, 0, 1000, 2300]
+    rows, keys = sum(lens), sum(lens) + sum(pasts)
+    q, kv, gate = rand(g, rows, heads, dim, dtype=torch.bfloat16, scale=2.0), rand(g, keys, groups, 2 * dim, dtype=torch.bfloat16), rand(g, rows, heads, dtype=torch.bfloat16)
+    q[..., 0], kv[..., 0] = 16.0, float(shift)
+    cu_q, cu_k = prefix_sums(lens), prefix_sums([a + b for a, b in zip(lens, pasts)])
+    view, both, gates = inside(q), on(kv), inside(gate, 3, 5) if gated else None
+    out = torch.full((rows, heads, dim), float("nan"), dtype=torch.bfloat16, device=DEV)
+    window_prefill(out, view, both[..., :dim], on(cu_q), on(cu_k), dim ** -0.5, window, v=both[..., dim:], gate=gates)
+    for e in range(len(lens)):
+        a, b = slice(int(cu_q[e]), int(cu_q[e + 1])), slice(int(cu_k[e]), int(cu_k[e + 1]))
+        want = window_reference_on_gpu(view[a], both[b, :, :dim], both[b, :, dim:], dim ** -0.5, window, gates[a] if gated else None)
+        assert rel(out[a].cpu(), want.cpu()) < 1.5e-2, e
+
+
+@pytest.mark.parametrize("window,n,past", [(256, 1100, 0), (700, 1030, 333), (0, 1024, 64)])
+def test_window_prefill_of_many_heads_one_prompt(window, n, past):
+    g, heads, dim = gen(window), 64, 128
+    q, k, v = (rand(g, rows, h, dim, dtype=torch.bfloat16, scale=2.0).to(DEV) for rows, h in ((n, heads), (n + past, 2), (n + past, 2)))
+    out = torch.full((n, heads, dim), float("nan"), dtype=torch.bfloat16, device=DEV)
+    window_prefill(out, q, k, on(prefix_sums([n])), on(prefix_sums([n + past])), dim ** -0.5, window, v=v)
+    assert rel(out.cpu(), window_reference_on_gpu(q, k, v, dim ** -0.5, window, None).cpu()) < 1.5e-2
+
+
 @pytest.mark.parametrize("dim,heads", [(64, 4), (128, 2), (256, 1)])
 @pytest.mark.parametrize("window", [32, 33, 63, 65, 94, 95, 96, 97, 127, 128, 129, 159, 160, 192, 193])
 def test_window_prefill_tiles_in_runs(window, dim, heads):
