@@ -723,15 +723,16 @@ __device__ __forceinline__ int this_wave() { return __builtin_amdgcn_readfirstla
 // rows, as an operand's are: keys took it four times as long as values, and a CU with a few hundred tokens to itself had no other bound (1
 // sequence of 512 tokens in one workgroup per head: 1.35 us per tile and wave).  Rows go through a wave's own 4 KB of LDS (the accumulators' room of the merge
 // where there is one), a row's chunks trading places by its number.  Caches cold, 8 kv heads, operands / rows: 252 batches of 1 to 256 sequences in tables of
-// 512 to 16384 1.044 times as fast on average (heads of 64 1.02); one of 511 7.9 / 6.9 us, 64 of 64 to 2047 1.05 to 1.09, 24 to 40 full tables 1.04 to
+// 512 to 16384 1.044 times as fast on average; one of 511 7.9 / 6.9 us, 64 of 64 to 2047 1.05 to 1.09, 24 to 40 full tables 1.04 to
 // 1.08, one wave per head, full tables 1.01, lengths spread 1.02 to 1.14.  Three waves per SIMD (168 registers, one spilled) instead of two: 1.025.
 // kStreamKeys: keys past the caches, as values (they are read once), where the waves of a head share it: 61 sequences of a decode step 558 / 571 us,
-// 16 of a smaller one 286 / 298, whose weights the caches hold; one wave per head, full tables 0.97 to 0.99 of the speed without; heads of 64 0.94 to 1.07.
-// Waves of eight at 64 dims, tables of up to 512: 0.98 to 1.00 with rows, so not there.
+// 16 of a smaller one 286 / 298, whose weights the caches hold; one wave per head, full tables 0.97 to 0.99 of the speed without.
+// Heads of 64, whose operands are half as many loads: one wave per head 1.01 to 1.05; where waves share one a row's longer way shows instead (one sequence of
+// 15000 in caches just read 17.9 / 19.4, tables of up to 512 0.98 to 1.00, 200 full ones 1.02), so not there.
 template <typename T, int W, int D, bool SUB>
 struct KeyRows {
-  static constexpr bool kRows = sizeof(T) == 2 && !SUB && (D == 128 || (D == 64 && W != kSplitManyWaves));
-  static constexpr bool kStreamKeys = W > 1 && D == 128;
+  static constexpr bool kRows = sizeof(T) == 2 && !SUB && (D == 128 || (D == 64 && W == 1));
+  static constexpr bool kStreamKeys = W > 1;
 };
 
 // W = 1: the wave walks all tiles of its partition.  W > 1 (the workgroup is W waves on one kv head): wave w takes
