@@ -495,6 +495,20 @@ int mvllm_norm_linear_small_m(void* out, void* residual_out, const void* x, cons
                               int64_t x_row_stride, int M, int N, int K, int glu, int dtype, void* stream);
 
 /*
+ * mvllm_linear_small_m with the residual add + RMSNorm behind it (src/myvllm/models/qwen3.py:118, 197-212, 306-312), in two launches: the product in
+ * parts of K, left as fp32 sums in the workspace, and the norm, which adds them up:
+ *   h = (x W^T + bias, rounded) + residual, rounded; residual_out = h; out = h / sqrt(mean(h^2) + eps) * gamma
+ * with the roundings of the two calls.  residual, residual_out and out dense [M, N]; residual_out may be residual, and out x.
+ * mvllm_linear_add_rms_norm_bytes says how much workspace a shape takes, 0 where it is not built (or would not pay): then MVLLM_ERR_UNSUPPORTED, and
+ * the caller runs the two calls.  The workspace is 16-byte aligned and free again after the call's work on the stream; too little:
+ * MVLLM_ERR_WORKSPACE.
+ */
+size_t mvllm_linear_add_rms_norm_bytes(int M, int N, int K, int64_t x_row_stride);
+int mvllm_linear_add_rms_norm(void* out, void* residual_out, const void* x, const void* w, const void* bias, const void* residual,
+                              const float* gamma, float eps, int64_t x_row_stride, int M, int N, int K, int dtype, void* workspace,
+                              size_t workspace_bytes, void* stream);
+
+/*
  * Whether mvllm_linear_small_m (norm == 0 && glu == 0) or mvllm_norm_linear_small_m takes a shape, without a
  * launch: MVLLM_OK and in *waves (may be NULL) a number that only defines the set of shapes: of the parts of 128 or 256 values
  * that K can be cut into, 4, 8 or 16, the fewest that give 1024 in all.  No kernel cuts K by it (the norm's has eight waves,

@@ -83,6 +83,8 @@ SIGNATURES = {
                                                             c_int, c_int, c_void_p]),
     "mvllm_linear_small_m_split_bytes": (c_size_t, [c_int, c_int, c_int, c_int64]),
     "mvllm_linear_small_m_split": (c_int, [c_void_p] * 4 + [c_int64] + [c_int] * 5 + [c_void_p, c_size_t, c_void_p]),
+    "mvllm_linear_add_rms_norm_bytes": (c_size_t, [c_int, c_int, c_int, c_int64]),
+    "mvllm_linear_add_rms_norm": (c_int, [c_void_p] * 7 + [c_float, c_int64] + [c_int] * 4 + [c_void_p, c_size_t, c_void_p]),
     "mvllm_linear_small_m_plan": (c_int, [c_int] * 6 + [ctypes.POINTER(c_int)]),
     "mvllm_qk_norm_rope_store": (c_int, [c_void_p] * 6 + [c_int64] * 3 + [c_void_p, c_float, c_void_p, c_int64,
                                                            c_void_p, c_void_p] + [c_void_p] * 4 +

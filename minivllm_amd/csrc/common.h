@@ -324,4 +324,9 @@ int launch_prefill_pp(const PrefillPpArgs& a, int dtype, hipStream_t stream);
 constexpr int kPpLeastWindow = 256;
 int launch_prefill_pp_window(const PrefillPpArgs& a, hipStream_t stream);
 
+// rms_norm.hip: norm(sum of `splits` parts [splits, rows, hidden], 2 to 4 of them, + bias + residual) * gamma and the sum with the residual, both dense, of
+// a 16-bit type; hidden a multiple of 4, at most 8192.
+int launch_parts_norm(void* out, void* residual_out, const float* part, int splits, const void* bias, const void* residual, const float* gamma,
+                      float eps, int rows, int hidden, int dtype, hipStream_t stream);
+
 }  // namespace mvllm

@@ -11,12 +11,14 @@
 // mvllm_norm_linear_small_m is the same product with the launches around it folded in: the residual add + RMSNorm in
 // front of the layer's first projections (src/myvllm/models/qwen3.py:197-212 through layers/layernorm.py:9-28) as
 // the kernel's prologue (linear_norm_kernel), and SiluAndMul behind the gate/up projection (layers/activation.py:15-18) as
-// its epilogue, each rounding where the separate launch rounds.
+// its epilogue, each rounding where the separate launch rounds.  mvllm_linear_add_rms_norm is the product in parts of K with that norm behind it.
 #include "prefill_tiles.h"
 
 #pragma clang fp contract(off)
 
 namespace mvllm {
+
+struct LinearSplit { int columns, splits; };               // of K; splits 1: whole, with ring_columns
 
 struct LinearArgs {
   void* out;
@@ -34,6 +36,8 @@ struct LinearArgs {
   int gelu;               // plain product only: the result through the tanh form of gelu
   int part_steps;         // steps of the ring in a part of K
   float* part;            // plain product only: partial sums [gridDim.y, M, N] of the splits of K, or null
+  LinearSplit split;      // with part
+  bool leave_parts;       // the next launch adds the parts up
 };
 
 // silu(g) * u with the roundings of the two tensor operations (activation.hip): silu in fp32 rounded to T, then the
@@ -468,7 +472,6 @@ static int ring_columns(int M, int N) {
 // 2048 x 6144 10.0 / 13.9 / 18.0 and 8.6 / 9.7 / 11.7, 1024 x 6144 9.2 / 13.3 / 17.2 and 6.8 / 8.5 / 9.6.  No gain: 4 to 24 rows of 2736 to 4096
 // columns and K of 6144 to 8192 (3072 x 8192 at 16 rows 13.8 and 14.8), 4096 x 4096 (13.6 and 13.2 at 64 rows), more columns
 // (6144 x 4096 18.5 and 18.3), 1024 x 3072 up to 32 rows (5.4 and 6.2 at 16; 9.0 and 7.4 at 64).
-struct LinearSplit { int columns, splits; };               // splits 1: whole
 static LinearSplit linear_split(int M, int N, int K) {
   constexpr int kTiles = 256 / 3;                           // at most so many, for three splits of each over 256 CUs
   if (M <= kFewRows || N < 1024 || N > 64 * kTiles) return {0, 1};
@@ -477,6 +480,25 @@ static LinearSplit linear_split(int M, int N, int K) {
   const int columns = N <= 16 * kTiles ? 16 : N <= 32 * kTiles ? 32 : 64;
   const int splits = 256 / ((N + columns - 1) / columns);
   return {columns, splits < 4 ? splits : 4};
+}
+
+// The same where the residual norm follows and its launch adds the parts up (parts_norm_kernel): it reads 4 bytes a part instead of two, and has
+// less to wait for than the norm alone, a thread for four numbers.  So parts pay nearly everywhere: two to four of them, with the narrowest
+// tile of which 256 CUs have a workgroup each, but at least two stages in a part.  us with the norm at 4 / 17 / 40 / 61 rows, apart (linear_split's
+// where it takes the shape) and now: 1024 x 2048 6.8 / 7.0 / 7.2 / 7.4 and 5.4 / 5.9 / 6.1 / 6.6, 1024 x 3072 7.4 / 7.3 / 9.8 / 10.4 and 5.7 / 6.2 / 6.5 / 7.1,
+// 2048 x 2048 6.8 / 7.0 / 8.2 / 9.0 and 6.1 / 6.6 / 7.1 / 7.8, 2048 x 6144 10.5 / 11.3 / 12.8 / 14.1 and 8.3 / 9.1 / 10.5 / 11.8, 2560 x 2560 8.7 / 9.7 / 11.7 / 12.8
+// and 7.3 / 7.7 / 8.8 / 10.2, 4096 x 4096 10.9 / 12.0 / 14.3 / 16.3 and 10.2 / 11.0 / 12.5 / 14.0, 4096 x 12288 23.5 / 23.4 / 25.7 / 28.4 and 20.7 / 21.5 / 23.5 / 25.9,
+// 5120 x 5120 19.1 / 18.1 / 21.6 / 25.5 and 13.8 / 14.8 / 16.9 / 19.0, 7168 x 2048 12.2 / 12.2 / 13.9 / 15.1 and 10.7 / 11.3 / 12.7 / 14.3; least: 4096 x 1024
+// 7.1 / 7.6 / 8.0 / 8.5 and 6.7 / 7.0 / 7.7 / 8.3, 2048 x 1024 5.9 / 6.0 / 6.9 / 7.3 and 5.6 / 6.0 / 6.7 / 7.2.  Past that none: 8192 x 4096 17.9 / 17.2 / 19.9 / 22.0
+// and 17.7 / 18.4 / 19.8 / 21.3.  Up to 4096 columns two parts of 32 or four of 64 fill the chip: 4096 x 2048 7.7 / 8.3 / 9.4 / 10.4 and 8.0 / 8.7 / 10.0 / 11.3, 3072 x 3072
+// 8.3 / 8.9 / 10.3 / 11.5 and 8.4 / 9.1 / 10.2 / 11.5, 4096 x 12288 21.8 / 21.7 / 25.1 / 29.0 and as above.
+static LinearSplit linear_norm_split(int M, int N, int K) {
+  if (M <= kFewRows || N < 512 || N > 7168 || K < (N > 4096 ? 2048 : 1024)) return {0, 1};
+  if (N <= 1024) return {K < 2048 ? 32 : 16, 4};
+  if (N <= 2048) return {32, 4};
+  if (N <= 2720) return {32, 3};
+  if (N <= 4096) return K < 4096 ? LinearSplit{32, 2} : LinearSplit{64, 4};
+  return {64, N <= 5440 ? 3 : 2};
 }
 
 // Few columns leave CUs without a workgroup, and each one with all the rows copies `rows + 16` rows of K values one stage after the other: the tiles of
@@ -507,7 +529,7 @@ static int launch_rows(const LinearArgs& a, hipStream_t stream) {
 template <typename T, int MT, bool GLU>
 static int launch_ring(LinearArgs a, hipStream_t stream) {
   const bool stream_weights = (int64_t)a.N * a.K * 2 >= kStreamBytes;
-  const LinearSplit split = a.part ? linear_split(a.M, a.N, a.K) : LinearSplit{ring_columns(a.M, a.N), 1};
+  const LinearSplit split = a.part ? a.split : LinearSplit{ring_columns(a.M, a.N), 1};
   const int columns = split.columns, steps = a.K / (columns == 16 ? 256 : 128);
   a.part_steps = (steps + split.splits - 1) / split.splits;
   const dim3 grid((unsigned)((a.N + columns - 1) / columns), (unsigned)split.splits, (unsigned)((a.M + 16 * MT - 1) / (16 * MT)));
@@ -525,7 +547,7 @@ static int launch_ring(LinearArgs a, hipStream_t stream) {
     default: linear_ring_kernel<T, MT, 3, 2, 2, 4, true, GLU><<<grid, dim3(256), 0, stream>>>(a);
   }
   const int status = launch_status();
-  if (status != MVLLM_OK || !a.part) return status;
+  if (status != MVLLM_OK || !a.part || a.leave_parts) return status;
   linear_sum_kernel<T><<<dim3((unsigned)(((int64_t)a.M * a.N / 4 + 255) / 256)), dim3(256), 0, stream>>>(a, split.splits);
   return launch_status();
 }
@@ -618,6 +640,7 @@ static int linear_plain(void* out, const void* x, const void* w, const void* bia
   LinearArgs a{};
   a.out = out; a.x = x; a.w = w; a.bias = bias; a.x_row_stride = x_row_stride; a.M = M; a.N = N; a.K = K;
   a.gelu = gelu; a.part = part;
+  if (part) a.split = linear_split(M, N, K);
   return dtype == MVLLM_BF16 ? launch_linear_fused<bf16_t>(a, false, (hipStream_t)stream)
                              : launch_linear_fused<f16_t>(a, false, (hipStream_t)stream);
 }
@@ -676,4 +699,29 @@ extern "C" int mvllm_norm_linear_small_m(void* out, void* residual_out, const vo
   a.row_tiles = norm_row_tiles(M);
   return dtype == MVLLM_BF16 ? launch_linear_fused<bf16_t>(a, glu != 0, (hipStream_t)stream)
                              : launch_linear_fused<f16_t>(a, glu != 0, (hipStream_t)stream);
+}
+
+extern "C" size_t mvllm_linear_add_rms_norm_bytes(int M, int N, int K, int64_t x_row_stride) {
+  if (M <= 0 || M > 64 || N <= 0 || N % 16 != 0 || K <= 0 || K % 512 != 0 || ((int64_t)(M - 1) * x_row_stride + K) * 2 > 0xffffffffll) return 0;
+  const int splits = linear_norm_split(M, N, K).splits;
+  return splits < 2 ? 0 : (size_t)splits * M * N * sizeof(float);
+}
+
+extern "C" int mvllm_linear_add_rms_norm(void* out, void* residual_out, const void* x, const void* w, const void* bias, const void* residual,
+                                         const float* gamma, float eps, int64_t x_row_stride, int M, int N, int K, int dtype, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
+  const int bad = linear_check(out, x, w, bias, x_row_stride, M, N, K, dtype);
+  if (bad || M == 0) return bad;
+  if (!residual_out || !residual || !gamma) return MVLLM_ERR_NULL_POINTER;
+  if (!aligned16(out) || !aligned16(residual_out) || !aligned16(residual) || !aligned16(gamma)) return MVLLM_ERR_MISALIGNED;
+  const size_t need = mvllm_linear_add_rms_norm_bytes(M, N, K, x_row_stride);
+  if (need == 0) return MVLLM_ERR_UNSUPPORTED;
+  if (!workspace || !aligned16(workspace) || workspace_bytes < need) return MVLLM_ERR_WORKSPACE;
+  LinearArgs a{};
+  a.x = x; a.w = w; a.x_row_stride = x_row_stride; a.M = M; a.N = N; a.K = K;
+  a.part = reinterpret_cast<float*>(workspace); a.split = linear_norm_split(M, N, K); a.leave_parts = true;
+  const int status = dtype == MVLLM_BF16 ? launch_linear_fused<bf16_t>(a, false, (hipStream_t)stream)
+                                         : launch_linear_fused<f16_t>(a, false, (hipStream_t)stream);
+  if (status != MVLLM_OK) return status;
+  return launch_parts_norm(out, residual_out, a.part, a.split.splits, bias, residual, gamma, eps, M, N, dtype, (hipStream_t)stream);
 }

@@ -139,6 +139,95 @@ static int launch_norm(void* out, void* residual_out, const void* x, const void*
   return MVLLM_OK;
 }
 
+// The norm behind a projection whose K was cut into parts (linear_small.hip): the row is the sum of the parts, plus the bias, rounded to T, and goes on as
+// above, so that neither the sums nor the rounded product need a launch and a pass of their own.  A workgroup per row, a
+// thread per four numbers of it, all S parts' loads under way at once: few rows wait for one memory latency, not for bandwidth.
+struct PartsNorm {
+  void* out;
+  void* residual_out;
+  const float* part;                                   // [S, gridDim.x, hidden]
+  const void* bias;                                    // [hidden] or null
+  const void* residual;                                // [rows, hidden] dense
+  const float* gamma;
+  float eps;
+  int hidden;
+};
+
+template <typename T, int S, int CHUNKS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void parts_norm_kernel(const PartsNorm a) {
+  __shared__ float sums[WAVES];
+  const int64_t at = (int64_t)blockIdx.x * a.hidden, size = (int64_t)gridDim.x * a.hidden;
+  const T* residual = reinterpret_cast<const T*>(a.residual) + at;
+  const T* bias = reinterpret_cast<const T*>(a.bias);
+  float4 p[CHUNKS][S], gam[CHUNKS];
+  uint2 res[CHUNKS];
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int e0 = 4 * (threadIdx.x + 64 * WAVES * c);
+    if (e0 >= a.hidden) continue;
+#pragma unroll
+    for (int i = 0; i < S; ++i) p[c][i] = *reinterpret_cast<const float4*>(a.part + i * size + at + e0);
+    res[c] = *reinterpret_cast<const uint2*>(residual + e0);
+    gam[c] = *reinterpret_cast<const float4*>(a.gamma + e0);
+  }
+  float v[CHUNKS][4], ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int e0 = 4 * (threadIdx.x + 64 * WAVES * c);
+    if (e0 >= a.hidden) continue;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < S; ++i) { s[0] += p[c][i].x; s[1] += p[c][i].y; s[2] += p[c][i].z; s[3] += p[c][i].w; }
+    const float r[4] = {lo_to_float<T>(res[c].x), hi_to_float<T>(res[c].x), lo_to_float<T>(res[c].y), hi_to_float<T>(res[c].y)};
+    T h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (bias) s[e] += to_float(bias[e0 + e]);
+      h[e] = from_float<T>(to_float(from_float<T>(s[e])) + r[e]);
+      v[c][e] = to_float(h[e]);
+      ss = ss + v[c][e] * v[c][e];
+    }
+    *reinterpret_cast<uint2*>(reinterpret_cast<T*>(a.residual_out) + at + e0) = *reinterpret_cast<const uint2*>(h);
+  }
+  ss = four_rows_sum(row16_sum(ss));
+  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  ss = sums[0];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) ss = ss + sums[w];
+  const SharedDivisor denom(sqrtf(ss / (float)a.hidden + a.eps));
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int e0 = 4 * (threadIdx.x + 64 * WAVES * c);
+    if (e0 >= a.hidden) continue;
+    const T y[4] = {from_float<T>(denom.divide(v[c][0]) * gam[c].x), from_float<T>(denom.divide(v[c][1]) * gam[c].y),
+                    from_float<T>(denom.divide(v[c][2]) * gam[c].z), from_float<T>(denom.divide(v[c][3]) * gam[c].w)};
+    *reinterpret_cast<uint2*>(reinterpret_cast<T*>(a.out) + at + e0) = *reinterpret_cast<const uint2*>(y);
+  }
+}
+
+template <typename T, int S>
+static int launch_parts(const PartsNorm& a, int rows, hipStream_t stream) {
+  const dim3 grid((unsigned)rows);
+  if (a.hidden <= 1024) parts_norm_kernel<T, S, 1, 4><<<grid, dim3(256), 0, stream>>>(a);
+  else if (a.hidden <= 2048) parts_norm_kernel<T, S, 1, 8><<<grid, dim3(512), 0, stream>>>(a);
+  else if (a.hidden <= 4096) parts_norm_kernel<T, S, 1, 16><<<grid, dim3(1024), 0, stream>>>(a);
+  else parts_norm_kernel<T, S, 2, 16><<<grid, dim3(1024), 0, stream>>>(a);
+  return launch_status();
+}
+
+int launch_parts_norm(void* out, void* residual_out, const float* part, int splits, const void* bias, const void* residual, const float* gamma,
+                      float eps, int rows, int hidden, int dtype, hipStream_t stream) {
+  const PartsNorm a{out, residual_out, part, bias, residual, gamma, eps, hidden};
+  const bool bf = dtype == MVLLM_BF16;
+  switch (splits) {
+    case 2: return bf ? launch_parts<bf16_t, 2>(a, rows, stream) : launch_parts<f16_t, 2>(a, rows, stream);
+    case 3: return bf ? launch_parts<bf16_t, 3>(a, rows, stream) : launch_parts<f16_t, 3>(a, rows, stream);
+    case 4: return bf ? launch_parts<bf16_t, 4>(a, rows, stream) : launch_parts<f16_t, 4>(a, rows, stream);
+    default: return MVLLM_ERR_UNSUPPORTED;
+  }
+}
+
 }  // namespace mvllm
 
 using namespace mvllm;

@@ -18,7 +18,7 @@ import torch
 
 from minivllm_amd import _C
 
-__all__ = ["qk_norm_rope_store", "sample_tokens", "sample_tokens_into", "decode_advance", "add_rms_norm", "silu_and_mul", "linear_small_m", "linear_small_m_takes", "norm_linear_small_m", "norm_linear_small_m_pays", "norm_linear_small_m_takes",
+__all__ = ["qk_norm_rope_store", "sample_tokens", "sample_tokens_into", "decode_advance", "add_rms_norm", "silu_and_mul", "linear_small_m", "linear_small_m_takes", "norm_linear_small_m", "norm_linear_small_m_pays", "norm_linear_small_m_takes", "linear_add_rms_norm", "linear_add_rms_norm_takes",
            "lm_head_sample", "lm_head_sample_takes", "lm_head_sample_workspace_bytes", "norm_conv", "head_rope_store",
            "head_unrotate_gate", "chunk_decode_step", "stream_embed_norm", "stream_norm", "gated_unit", "gelu_tanh", "post_norm",
            "embed_rows"]
@@ -381,6 +381,45 @@ def norm_linear_small_m(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tenso
                                              _C.dtype_code(x.dtype), _C.current_stream_ptr(x.device))
     _C.check(st, "norm_linear_small_m")
     return (out, res_out) if want_residual else out
+
+
+def linear_add_rms_norm_takes(x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, max_rows: int = 64) -> bool:
+    """Whether ``linear_add_rms_norm`` is built for this call, and pays: 4 to 64 rows, bf16 / fp16 on the GPU, K a multiple of 512 from
+    1024 on, 512 to 7168 outputs (a multiple of 16), a dense residual."""
+    return (linear_small_m_takes(x, weight, max_rows) and residual.dtype == x.dtype and residual.is_contiguous()
+            and tuple(residual.shape) == (x.shape[0], weight.shape[0]) and x.shape[1] == weight.shape[1] and residual.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0
+            and _C.load().mvllm_linear_add_rms_norm_bytes(x.shape[0], weight.shape[0], weight.shape[1], x.stride(0)) > 0)
+
+
+def linear_add_rms_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, residual: torch.Tensor, gamma: torch.Tensor,
+                        eps: float):
+    """``add_rms_norm(linear_small_m(x, weight, bias), gamma, eps, residual)`` for the few rows of a decode step, with those calls' roundings: the
+    product in parts of K, whose sums the norm's launch adds up.  gamma float32 (N,).  Returns (norm, sum with the residual), (M, N) both."""
+    _C.require_cuda(x, weight, bias, residual, gamma)
+    if x.dim() != 2 or weight.dim() != 2 or weight.shape[1] != x.shape[1]:
+        raise ValueError(f"x (M, K) and weight (N, K) expected, got {tuple(x.shape)} and {tuple(weight.shape)}")
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.dtype != x.dtype or residual.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
+        raise ValueError("x, weight, bias and residual must share one dtype")
+    if not weight.is_contiguous() or x.stride(1) != 1:
+        raise ValueError("weight must be contiguous and the rows of x dense")
+    if tuple(residual.shape) != (m, n) or not residual.is_contiguous():
+        raise ValueError("residual must be a contiguous (M, N) tensor")
+    if bias is not None and (tuple(bias.shape) != (n,) or not bias.is_contiguous()):
+        raise ValueError("bias must be contiguous of shape (N,)")
+    if gamma.dtype != torch.float32 or tuple(gamma.shape) != (n,) or not gamma.is_contiguous():
+        raise ValueError("gamma must be contiguous float32 of shape (N,)")
+    out, total = torch.empty_like(residual), torch.empty_like(residual)
+    lib = _C.load()
+    stride = x.stride(0) if m > 1 else k
+    need = lib.mvllm_linear_add_rms_norm_bytes(m, n, k, stride)
+    workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+    st = lib.mvllm_linear_add_rms_norm(_ptr(out), _ptr(total), _ptr(x), _ptr(weight), _ptr(bias), _ptr(residual), _ptr(gamma), float(eps), stride,
+                                       m, n, k, _C.dtype_code(x.dtype), _ptr(workspace), need, _C.current_stream_ptr(x.device))
+    _C.check(st, "linear_add_rms_norm")
+    return out, total
 
 
 def lm_head_sample_takes(hidden: torch.Tensor, weight: torch.Tensor, batch: int | None = None) -> bool:

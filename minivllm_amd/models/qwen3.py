@@ -15,7 +15,7 @@ import torch.nn.functional as F
 
 from minivllm_amd.layers.attention import Attention
 from minivllm_amd.layers.basic import Linear, RMSNorm, RotaryEmbedding, SiluAndMul
-from minivllm_amd.layers.fused import norm_linear_small_m, norm_linear_small_m_pays, norm_linear_small_m_takes
+from minivllm_amd.layers.fused import linear_add_rms_norm, linear_add_rms_norm_takes, norm_linear_small_m, norm_linear_small_m_pays, norm_linear_small_m_takes
 from minivllm_amd.utils.context import get_context
 
 
@@ -38,6 +38,10 @@ class Qwen3Attention(nn.Module):
 
     def forward_qkv(self, qkv, positions):
         """Everything after the QKV projection (whose output a caller may have produced fused with the norm)."""
+        return self.output_projection(self.attend(qkv, positions))
+
+    def attend(self, qkv, positions):
+        """``forward_qkv`` without the output projection."""
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
         if self.fused_qk:
             # views of the projection output, no copies; norm + rotation + cache store in one launch
@@ -45,16 +49,15 @@ class Qwen3Attention(nn.Module):
             k = k.unflatten(-1, (self.num_kv_heads, self.head_dim))
             v = v.unflatten(-1, (self.num_kv_heads, self.head_dim))
             gamma = None if self.qkv_bias else self.rms_norm.weight_fp32()
-            o = self.attention.forward_fused(q, k, v, positions, self.rotary_emb.cos_sin_cache, gamma,
-                                             self.rms_norm.eps)
-            return self.output_projection(o)
+            return self.attention.forward_fused(q, k, v, positions, self.rotary_emb.cos_sin_cache, gamma,
+                                                self.rms_norm.eps)
         q = q.reshape(-1, self.num_heads, self.head_dim)
         k = k.reshape(-1, self.num_kv_heads, self.head_dim)
         v = v.reshape(-1, self.num_kv_heads, self.head_dim)
         if not self.qkv_bias:
             q, k = self.rms_norm(q), self.rms_norm(k)
         q, k = self.rotary_emb(positions, q, k)
-        return self.output_projection(self.attention(q, k, v))
+        return self.attention(q, k, v)
 
 
 class Qwen3MLP(nn.Module):
@@ -66,11 +69,15 @@ class Qwen3MLP(nn.Module):
         self.small_rows, self.fused = small_rows, fused
 
     def forward(self, x):
+        return self.gate_down(self.gated(x))
+
+    def gated(self, x):
+        """``forward`` without the last projection."""
         # a decode step's rows: SiluAndMul as the epilogue of the gate/up projection (one launch instead of two)
         if (self.small_rows and self.fused and x.dim() == 2 and x.shape[0] <= self.small_rows and x.is_contiguous()
                 and norm_linear_small_m_takes(x, self.gate_up.weight, self.small_rows, norm=False, glu=True)):
-            return self.gate_down(norm_linear_small_m(x, self.gate_up.weight, self.gate_up.bias, glu=True))
-        return self.gate_down(self.activation(self.gate_up(x)))
+            return norm_linear_small_m(x, self.gate_up.weight, self.gate_up.bias, glu=True)
+        return self.activation(self.gate_up(x))
 
 
 class Qwen3DecoderLayer(nn.Module):
@@ -90,7 +97,11 @@ class Qwen3DecoderLayer(nn.Module):
         return (self.norm_rows and self.fused_elementwise and x.dim() == 2 and x.shape[0] <= self.norm_rows and x.is_contiguous()
                 and norm_linear_small_m_pays(x.shape[0], weight) and norm_linear_small_m_takes(x, weight, self.norm_rows, glu=glu))
 
-    def forward(self, x, residual, positions):
+    def forward(self, x, residual, positions, step=None):
+        """``step`` (normed, behind), for few rows: whether the input norm has been applied to x already, and the norm that follows the layer and may be
+        applied here, or None; whether it has been is then a third result."""
+        if step is not None:
+            return self._few_rows(x, residual, positions, *step)
         attn, mlp, norm = self.self_attn, self.mlp, self.input_layernorm
         proj = attn.qkv_projection
         if self._norm_in_product(x, proj.weight):
@@ -112,6 +123,39 @@ class Qwen3DecoderLayer(nn.Module):
             return mlp.gate_down(act), residual
         x, residual = norm(x, residual)
         return mlp(x), residual
+
+    def _project_norm(self, proj, x, residual, norm):
+        """``norm(proj(x), residual)`` where the norm can join the projection, else the projection and ``residual`` as it is; and which."""
+        if norm is not None and norm.fused and proj.small_rows and linear_add_rms_norm_takes(x, proj.weight, residual, proj.small_rows):
+            return *linear_add_rms_norm(x, proj.weight, proj.bias, residual, norm.weight_fp32(), norm.eps), True
+        return proj(x), residual, False
+
+    def _few_rows(self, x, residual, positions, normed, behind):
+        """A decode step's rows: each norm in the launches of the projection behind it where that is faster, else in those of the one before."""
+        attn, mlp, norm = self.self_attn, self.mlp, self.input_layernorm
+        proj = attn.qkv_projection
+        if normed:
+            qkv = proj(x)
+        elif residual is None:
+            residual = x
+            if self._norm_in_product(x, proj.weight):
+                qkv = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps)
+            else:
+                qkv = proj(norm(x))
+        elif self._norm_in_product(x, proj.weight):
+            qkv, residual = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps, residual, True)
+        else:
+            x, residual = norm(x, residual)
+            qkv = proj(x)
+        norm, inside = self.post_attention_layernorm, self._norm_in_product(x, mlp.gate_up.weight, glu=True)
+        x, residual, normed = self._project_norm(attn.output_projection, attn.attend(qkv, positions), residual, None if inside else norm)
+        if inside:
+            x, residual = norm_linear_small_m(x, mlp.gate_up.weight, mlp.gate_up.bias, norm.weight_fp32(), norm.eps, residual, True, glu=True)
+        else:
+            if not normed:
+                x, residual = norm(x, residual)
+            x = mlp.gated(x)
+        return self._project_norm(mlp.gate_down, x, residual, behind)
 
 
 class Qwen3ForCausalLM(nn.Module):
@@ -136,6 +180,7 @@ class Qwen3ForCausalLM(nn.Module):
         self.lm_head_weight = self.embedding_layer.weight if tie_word_embeddings else nn.Parameter(
             torch.empty(vocab_size, hidden_size))
         self.max_position = max_position
+        self.small_rows, self.joined_norms = small_rows, fused_elementwise
 
     def reset_parameters(self, seed: int = 0, std: float = 0.02):
         g = torch.Generator(device="cpu").manual_seed(seed)
@@ -152,11 +197,17 @@ class Qwen3ForCausalLM(nn.Module):
         # a decode step's few rows by plain indexing: the embedding operator's small-batch kernel takes 11 us for 16
         # rows, the gather 4
         x = self.embedding_layer.weight[input_ids] if input_ids.numel() <= 256 else self.embedding_layer(input_ids)
-        residual = None
-        for layer in self.layer_stack:
-            x, residual = layer(x, residual, positions)
-        x, _ = self.final_layernorm(x, residual)
-        return x
+        residual, normed, layers = None, False, list(self.layer_stack)
+        if not self.joined_norms or not x.is_cuda or x.shape[0] > self.small_rows:
+            for layer in layers:
+                x, residual = layer(x, residual, positions)
+        else:
+            for layer, after in zip(layers, [*layers[1:], None]):
+                behind = self.final_layernorm if after is None else after.input_layernorm
+                if after is not None and after._norm_in_product(x, after.self_attn.qkv_projection.weight):
+                    behind = None
+                x, residual, normed = layer(x, residual, positions, (normed, behind))
+        return x if normed else self.final_layernorm(x, residual)[0]
 
     def compute_logits(self, hidden):
         context = get_context()

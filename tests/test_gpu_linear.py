@@ -7,7 +7,7 @@ import torch.nn.functional as F
 
 from minivllm_amd import _C
 from minivllm_amd.layers.basic import Linear
-from minivllm_amd.layers.fused import (add_rms_norm, decode_advance, linear_small_m, linear_small_m_takes,
+from minivllm_amd.layers.fused import (add_rms_norm, decode_advance, linear_add_rms_norm, linear_add_rms_norm_takes, linear_small_m, linear_small_m_takes,
                                        norm_linear_small_m, norm_linear_small_m_takes, silu_and_mul)
 
 pytestmark = pytest.mark.gpu
@@ -252,3 +252,35 @@ def test_norm_linear_last_columns(m, n, k, glu):
     assert torch.equal(got_res, want_res)
     worst = ((got.float() - want.float()).abs() / want.float().abs().amax(dim=1, keepdim=True)).max().item()
     assert worst <= (4 if glu else 2) * 2.0 ** -8, worst
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m", [4, 16, 17, 33, 61, 64])
+@pytest.mark.parametrize("n,k,bias,stride", [(512, 1024, True, None),          # 32 columns, parts of two stages
+                                             (784, 2560, False, 2584),         # 16, parts that differ in length, strided rows
+                                             (1024, 2048, False, None), (1040, 1024, False, None), (2048, 1536, True, None),
+                                             (2064, 1024, False, None),        # three parts of two or three stages, the last tile half full
+                                             (2736, 2048, False, 2056), (4096, 4096, True, None), (4112, 2560, False, None), (7168, 2048, False, None)])
+def test_linear_add_rms_norm(dtype, m, n, k, bias, stride):
+    """Every tile and number of parts of the product whose norm adds the parts up, at the edges of their ranges.  The sum with the residual is rounded
+    twice (product, sum); the norm divides by a root mean square that differs by less than those, and rounds once more."""
+    x, w, b = _case(900 + m, m, n, k, dtype, bias, stride=stride)
+    g = torch.Generator().manual_seed(m)
+    residual = torch.randn(m, n, generator=g).to(dtype).to(DEV)
+    gamma = (1 + 0.1 * torch.randn(n, generator=g)).to(DEV)
+    assert linear_add_rms_norm_takes(x, w, residual)
+    got, total = linear_add_rms_norm(x, w, b, residual, gamma, 1e-6)
+    product = x.float() @ w.float().T + (b.float() if bias else 0)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    want = product + residual.float()
+    assert ((total.float() - want).abs() - ulp * (product.abs() + want.abs()) * (1 + ulp)).max().item() <= 2e-3
+    # from the sums as they were stored: the same norm, and one that the separate launch computes
+    norm = total.float() / (total.float().pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * gamma
+    assert ((got.float() - norm).abs() - ulp * norm.abs()).max().item() <= 1e-4
+    assert not linear_add_rms_norm_takes(x[:3], w, residual[:3])
+
+
+@pytest.mark.parametrize("n,k", [(496, 1024), (512, 512), (4112, 1024), (7184, 2048)])
+def test_linear_add_rms_norm_leaves_the_rest(n, k):
+    x, w, _ = _case(7, 5, n, k, torch.bfloat16, False)
+    assert not linear_add_rms_norm_takes(x, w, torch.zeros(5, n, dtype=torch.bfloat16, device=DEV))
