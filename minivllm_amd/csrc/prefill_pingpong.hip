@@ -154,6 +154,19 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       cached = kv_len > len ? kv_len - len : 0;
     }
   }
+  if constexpr (WIN) {                         // rows in front of their sequence's first key see none: zeros, and the items are those of the other rows
+    const int keyless = max(len - max(kv_len, 0), 0);
+    for (unsigned long long some = __ballot(keyless > 0); some != 0ull; some &= some - 1) {
+      const int at = __ffsll((long long)some) - 1, rows = __builtin_amdgcn_readlane(keyless, at);
+      char* const base = reinterpret_cast<char*>(a.out) + (int64_t)__builtin_amdgcn_readlane(lo, at) * a.win.out_row;
+      for (int row = blockIdx.x; row < rows; row += gridDim.x)
+        for (int c = 64 * wave + lane; c < a.num_heads * (kRowB / 16); c += 64 * kPpWaves)
+          *reinterpret_cast<uint4*>(base + (int64_t)row * a.win.out_row + (c / (kRowB / 16)) * a.win.out_head + c % (kRowB / 16) * 16) = make_uint4(0u, 0u, 0u, 0u);
+      vm_wait<0>();                            // (the counts below begin at nothing)
+    }
+    lo += keyless;
+    len -= keyless;
+  }
   const int nb = (len + kRPI - 1) / kRPI;      // item blocks of the lane's sequence
   // An item's level is the index of its last key tile: block rb of a sequence with c cached tokens has level
   // (c + kRPI - 1) / 64 + kTPB rb, so the lane's sequence owns every kTPB-th level from lvl0 to lvl_end - 1.
@@ -648,10 +661,11 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     }
   };
   auto row_factor = [&]() {                      // what an output row is multiplied with
-    const float inv = __builtin_amdgcn_rcpf(sum_with_lane_xor32(l));
+    const float sum = sum_with_lane_xor32(l), inv = __builtin_amdgcn_rcpf(sum);
     if constexpr (WIN) {
+      const float own = sum > 0.f ? inv : 0.f;   // (no key with a weight: zeros)
       const float sig = __builtin_amdgcn_rcpf(1.f + __expf(-lo_to_float<T>(gate_bits)));
-      return a.win.gate ? inv * sig : inv;
+      return a.win.gate ? own * sig : own;
     }
     return inv;
   };

@@ -262,6 +262,27 @@ def test_window_prefill_of_many_heads(heads, groups, window, shift, gated):
         assert rel(out[a].cpu(), want.cpu()) < 1.5e-2, e
 
 
+@pytest.mark.parametrize("heads,groups,window", [(64, 2, 0), (64, 2, 300), (60, 2, 2048), (6, 3, 40)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_window_prefill_of_more_rows_than_keys(heads, groups, window, gated):
+    """Row i of an entry stands at key (keys - rows) + i also where that is in front of the first key: such rows are zeros, the others see the keys up to their
+    own.  On the kernel with two groups of waves (four heads and two at a time) and on the one for small batches."""
+    dim, g = 128, gen(heads + window)
+    lens, keys = [300, 700, 65, 400, 130, 64], [0, 630, 64, 900, 130, 1]
+    q, kv, gate = rand(g, sum(lens), heads, dim, dtype=torch.bfloat16, scale=2.0), rand(g, sum(keys), groups, 2 * dim, dtype=torch.bfloat16), rand(g, sum(lens), heads, dtype=torch.bfloat16)
+    cu_q, cu_k, both, gates = prefix_sums(lens), prefix_sums(keys), on(kv), on(gate) if gated else None
+    out = torch.full((sum(lens), heads, dim), float("nan"), dtype=torch.bfloat16, device=DEV)
+    window_prefill(out, on(q), both[..., :dim], on(cu_q), on(cu_k), dim ** -0.5, window, v=both[..., dim:], gate=gates)
+    for e, (n, m) in enumerate(zip(lens, keys)):
+        first, end = int(cu_q[e]), int(cu_q[e + 1])
+        start = end - min(n, m)                                    # the first row that has a key
+        assert not out[first:start].any(), e
+        if m:
+            b = slice(int(cu_k[e]), int(cu_k[e + 1]))
+            want = window_reference_on_gpu(on(q)[start:end], both[b, :, :dim], both[b, :, dim:], dim ** -0.5, window, gates[start:end] if gated else None)
+            assert rel(out[start:end].cpu(), want.cpu()) < 1.5e-2, e
+
+
 @pytest.mark.parametrize("window,n,past", [(256, 1100, 0), (700, 1030, 333), (0, 1024, 64)])
 def test_window_prefill_of_many_heads_one_prompt(window, n, past):
     g, heads, dim = gen(window), 64, 128
