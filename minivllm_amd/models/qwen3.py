@@ -12,11 +12,20 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from minivllm_amd.layers.attention import Attention
 from minivllm_amd.layers.basic import Linear, RMSNorm, RotaryEmbedding, SiluAndMul
 from minivllm_amd.layers.fused import linear_add_rms_norm, linear_add_rms_norm_takes, norm_linear_small_m, norm_linear_small_m_pays, norm_linear_small_m_takes
 from minivllm_amd.utils.context import get_context
+
+
+def _as_built(module, kind):
+    """Whether calling ``module`` is ``kind.forward`` and nothing else, so that its work may be done as a part of another launch: not where it was
+    replaced, or somebody hooked into it."""
+    return (type(module) is kind and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+            and not _has_any_global_hook())
 
 
 class Qwen3Attention(nn.Module):
@@ -75,6 +84,7 @@ class Qwen3MLP(nn.Module):
         """``forward`` without the last projection."""
         # a decode step's rows: SiluAndMul as the epilogue of the gate/up projection (one launch instead of two)
         if (self.small_rows and self.fused and x.dim() == 2 and x.shape[0] <= self.small_rows and x.is_contiguous()
+                and _as_built(self.gate_up, Linear) and _as_built(self.activation, SiluAndMul)
                 and norm_linear_small_m_takes(x, self.gate_up.weight, self.small_rows, norm=False, glu=True)):
             return norm_linear_small_m(x, self.gate_up.weight, self.gate_up.bias, glu=True)
         return self.activation(self.gate_up(x))
@@ -91,71 +101,58 @@ class Qwen3DecoderLayer(nn.Module):
         self.mlp = Qwen3MLP(hidden_size, intermediate_size, ffn_bias, fused_elementwise, small_rows)
         self.norm_rows, self.fused_elementwise = min(small_rows, norm_rows), fused_elementwise
 
-    def _norm_in_product(self, x, weight, glu=False):
+    def _norm_in_product(self, norm, proj, x, glu=False):
         """A decode step's few rows: the residual norm runs as the prologue of the projection behind it (and SiluAndMul as its
         epilogue) where that is faster than a launch of its own, with the same roundings."""
         return (self.norm_rows and self.fused_elementwise and x.dim() == 2 and x.shape[0] <= self.norm_rows and x.is_contiguous()
-                and norm_linear_small_m_pays(x.shape[0], weight) and norm_linear_small_m_takes(x, weight, self.norm_rows, glu=glu))
+                and _as_built(norm, RMSNorm) and _as_built(proj, Linear) and norm_linear_small_m_pays(x.shape[0], proj.weight)
+                and norm_linear_small_m_takes(x, proj.weight, self.norm_rows, glu=glu))
 
-    def forward(self, x, residual, positions, step=None):
-        """``step`` (normed, behind), for few rows: whether the input norm has been applied to x already, and the norm that follows the layer and may be
-        applied here, or None; whether it has been is then a third result."""
-        if step is not None:
-            return self._few_rows(x, residual, positions, *step)
-        attn, mlp, norm = self.self_attn, self.mlp, self.input_layernorm
-        proj = attn.qkv_projection
-        if self._norm_in_product(x, proj.weight):
-            if residual is None:
-                qkv, residual = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps), x
-            else:
-                qkv, residual = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps, residual, True)
-            x = attn.forward_qkv(qkv, positions)
-        else:
-            if residual is None:
-                residual = x
-                x = norm(x)
-            else:
-                x, residual = norm(x, residual)
-            x = attn(x, positions)
-        norm = self.post_attention_layernorm
-        if self._norm_in_product(x, mlp.gate_up.weight, glu=True):
-            act, residual = norm_linear_small_m(x, mlp.gate_up.weight, mlp.gate_up.bias, norm.weight_fp32(), norm.eps, residual, True, glu=True)
-            return mlp.gate_down(act), residual
-        x, residual = norm(x, residual)
-        return mlp(x), residual
-
-    def _project_norm(self, proj, x, residual, norm):
-        """``norm(proj(x), residual)`` where the norm can join the projection, else the projection and ``residual`` as it is; and which."""
-        if norm is not None and norm.fused and proj.small_rows and linear_add_rms_norm_takes(x, proj.weight, residual, proj.small_rows):
+    def _project_norm(self, proj, x, residual, norm, into, glu=False):
+        """``norm(proj(x), residual)`` where the norm can join the projection and is not better off in ``into``, the projection behind it (None: unknown),
+        else the projection and ``residual`` as it is; and which."""
+        if (norm is not None and _as_built(proj, Linear) and proj.small_rows and _as_built(norm, RMSNorm) and norm.fused
+                and not (into is not None and self._norm_in_product(norm, into, residual, glu))
+                and linear_add_rms_norm_takes(x, proj.weight, residual, proj.small_rows)):
             return *linear_add_rms_norm(x, proj.weight, proj.bias, residual, norm.weight_fp32(), norm.eps), True
         return proj(x), residual, False
 
-    def _few_rows(self, x, residual, positions, normed, behind):
-        """A decode step's rows: each norm in the launches of the projection behind it where that is faster, else in those of the one before."""
+    def forward(self, x, residual, positions):
+        return self.walk(x, residual, positions)[:2]
+
+    def walk(self, x, residual, positions, normed=False, behind=None, into=None):
+        """``forward`` for a caller that knows its neighbours: ``normed``, x is behind the input norm already; ``behind``, the norm that follows the
+        layer and may be applied here, with ``into`` the projection that follows it.  The third result says whether it has been.  Modules that are not as
+        this file builds them are called as they are."""
         attn, mlp, norm = self.self_attn, self.mlp, self.input_layernorm
-        proj = attn.qkv_projection
+        own_attn, own_mlp = _as_built(attn, Qwen3Attention), _as_built(mlp, Qwen3MLP)
+        qkv = None
         if normed:
-            qkv = proj(x)
+            pass
+        elif own_attn and self._norm_in_product(norm, attn.qkv_projection, x):
+            proj = attn.qkv_projection
+            qkv = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps, residual, residual is not None)
+            qkv, residual = (qkv, x) if residual is None else qkv
         elif residual is None:
-            residual = x
-            if self._norm_in_product(x, proj.weight):
-                qkv = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps)
-            else:
-                qkv = proj(norm(x))
-        elif self._norm_in_product(x, proj.weight):
-            qkv, residual = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps, residual, True)
+            residual, x = x, norm(x)
         else:
             x, residual = norm(x, residual)
-            qkv = proj(x)
-        norm, inside = self.post_attention_layernorm, self._norm_in_product(x, mlp.gate_up.weight, glu=True)
-        x, residual, normed = self._project_norm(attn.output_projection, attn.attend(qkv, positions), residual, None if inside else norm)
-        if inside:
-            x, residual = norm_linear_small_m(x, mlp.gate_up.weight, mlp.gate_up.bias, norm.weight_fp32(), norm.eps, residual, True, glu=True)
+        norm, normed = self.post_attention_layernorm, False
+        if own_attn:
+            x = attn.attend(attn.qkv_projection(x) if qkv is None else qkv, positions)
+            x, residual, normed = self._project_norm(attn.output_projection, x, residual, norm, mlp.gate_up if own_mlp else None, glu=True)
+        else:
+            x = attn(x, positions)
+        if not normed and own_mlp and _as_built(mlp.activation, SiluAndMul) and self._norm_in_product(norm, mlp.gate_up, x, glu=True):
+            proj = mlp.gate_up
+            x, residual = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps, residual, True, glu=True)
         else:
             if not normed:
                 x, residual = norm(x, residual)
+            if not own_mlp:
+                return mlp(x), residual, False
             x = mlp.gated(x)
-        return self._project_norm(mlp.gate_down, x, residual, behind)
+        return self._project_norm(mlp.gate_down, x, residual, behind, into)
 
 
 class Qwen3ForCausalLM(nn.Module):
@@ -180,7 +177,6 @@ class Qwen3ForCausalLM(nn.Module):
         self.lm_head_weight = self.embedding_layer.weight if tie_word_embeddings else nn.Parameter(
             torch.empty(vocab_size, hidden_size))
         self.max_position = max_position
-        self.small_rows, self.joined_norms = small_rows, fused_elementwise
 
     def reset_parameters(self, seed: int = 0, std: float = 0.02):
         g = torch.Generator(device="cpu").manual_seed(seed)
@@ -198,15 +194,19 @@ class Qwen3ForCausalLM(nn.Module):
         # rows, the gather 4
         x = self.embedding_layer.weight[input_ids] if input_ids.numel() <= 256 else self.embedding_layer(input_ids)
         residual, normed, layers = None, False, list(self.layer_stack)
-        if not self.joined_norms or not x.is_cuda or x.shape[0] > self.small_rows:
-            for layer in layers:
+        own = [_as_built(layer, Qwen3DecoderLayer) for layer in layers]
+        for i, layer in enumerate(layers):
+            behind = into = None
+            if i + 1 == len(layers):
+                behind = self.final_layernorm
+            elif own[i + 1]:
+                behind, attn = layers[i + 1].input_layernorm, layers[i + 1].self_attn
+                into = attn.qkv_projection if _as_built(attn, Qwen3Attention) else None
+            if own[i]:
+                x, residual, normed = layer.walk(x, residual, positions, normed, behind, into)
+            else:
                 x, residual = layer(x, residual, positions)
-        else:
-            for layer, after in zip(layers, [*layers[1:], None]):
-                behind = self.final_layernorm if after is None else after.input_layernorm
-                if after is not None and after._norm_in_product(x, after.self_attn.qkv_projection.weight):
-                    behind = None
-                x, residual, normed = layer(x, residual, positions, (normed, behind))
+                normed = False
         return x if normed else self.final_layernorm(x, residual)[0]
 
     def compute_logits(self, hidden):
