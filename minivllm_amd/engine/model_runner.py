@@ -8,7 +8,8 @@ rms_norm_epsilon qkv_bias ffn_bias scale tie_word_embeddings max_position``; eng
 max_cached_blocks max_num_sequences max_num_batched_tokens dtype kv_cache_dtype seed``; ``linear_small_rows`` (default
 64): projections of at most that many rows, a decode step, run as the single-launch ``linear_small_m``, the gate/up
 projection with SiluAndMul as its epilogue (0: always the library GEMM); ``linear_norm_rows`` (default 32): up to that
-many rows, but no more than 16, the residual norms run as prologues of the projections behind them where that is faster (weights of at most 8 Mi numbers); ``fused_lm_head`` (default true): LM head and sampler as one pass
+many rows, but no more than 16, the residual norms run as prologues of the projections behind them where that is faster (weights of at most 8 Mi
+numbers); from 4 to ``linear_small_rows`` rows those that do not run with the output and down projections before them (0: as launches of their own); ``fused_lm_head`` (default true): LM head and sampler as one pass
 over the weights for at most 64 rows (``lm_head_sample``), otherwise the library GEMM and ``sample_tokens``.
 """
 from __future__ import annotations

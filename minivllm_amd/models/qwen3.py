@@ -111,7 +111,7 @@ class Qwen3DecoderLayer(nn.Module):
     def _project_norm(self, proj, x, residual, norm, into, glu=False):
         """``norm(proj(x), residual)`` where the norm can join the projection and is not better off in ``into``, the projection behind it (None: unknown),
         else the projection and ``residual`` as it is; and which."""
-        if (norm is not None and _as_built(proj, Linear) and proj.small_rows and _as_built(norm, RMSNorm) and norm.fused
+        if (norm is not None and self.norm_rows and _as_built(proj, Linear) and proj.small_rows and _as_built(norm, RMSNorm) and norm.fused
                 and not (into is not None and self._norm_in_product(norm, into, residual, glu))
                 and linear_add_rms_norm_takes(x, proj.weight, residual, proj.small_rows)):
             return *linear_add_rms_norm(x, proj.weight, proj.bias, residual, norm.weight_fp32(), norm.eps), True

@@ -94,6 +94,13 @@ def test_steps_are_the_chain_of_modules(joined, rows):
     assert torch.allclose(got, expected(model, ids), rtol=1e-4, atol=1e-4)       # (gamma in fp32)
 
 
+@pytest.mark.parametrize("rows", [2, 5, 30, 64])
+def test_no_norm_rows_no_joined_norms(joined, rows):
+    model, ids = decoder(norm_rows=0), torch.arange(rows)
+    got = model(ids, ids)
+    assert set(joined) == {"glu"} and torch.allclose(got, expected(model, ids), rtol=1e-4, atol=1e-4)
+
+
 def double(module, args, out):
     return 2 * out
 
