@@ -343,15 +343,15 @@ def norm_linear_small_m_takes(x: torch.Tensor, weight: torch.Tensor, max_rows: i
     return _PLAN_CACHE[key]
 
 
-def norm_linear_small_m_pays(rows: int, weight: torch.Tensor) -> bool:
-    """Whether the norm inside the product beats its own launch in front of it: every workgroup norms all rows again, which
+def norm_linear_small_m_pays(rows: int, weight: torch.Tensor, joins: bool = False) -> bool:
+    """Whether the norm inside the product beats its own launch in front of it or, with ``joins``, as part of the projection before it: every workgroup norms all rows again, which
     costs less than a launch up to 16 of them if a CU has one workgroup or two (us together / apart: 4096 x 1024 4.0 / 6.4 at one row,
-    5.5 / 6.7 at 16, 7.5 / 7.4 at 32; 6144 x 1024 gated 5.1 / 7.8, 6.6 / 7.6, 9.0 / 8.1; 4096 x 2048 5.8 / 7.4, 8.7 / 8.3; 12288 x 2048 15.5 / 13.3).  From
-    4 rows on the norm can join the projection before it instead (``linear_add_rms_norm``): worth more where K is long, less where
+    5.5 / 6.7 at 16, 7.5 / 7.4 at 32; 6144 x 1024 gated 5.1 / 7.8, 6.6 / 7.6, 9.0 / 8.1; 4096 x 2048 5.8 / 7.4, 8.7 / 8.3; 12288 x 2048 15.5 / 13.3).  The
+    projection before it (``linear_add_rms_norm``, from 4 rows on; a first layer has none) is worth more where K is long, less where
     it is short (us of a whole step, here / there: 8 layers of 1024 numbers 251 / 277 at 4 rows, 274 / 295 at 8, 361 / 370 at 16; of 2048
     363 / 360, 391 / 380, 473 / 452)."""
     n, k = weight.shape
-    return rows <= (16 if k <= 1024 else 3) and n * k <= (8 << 20)
+    return rows <= (3 if joins and k > 1024 else 16) and n * k <= (8 << 20)
 
 
 def norm_linear_small_m(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,

@@ -101,18 +101,18 @@ class Qwen3DecoderLayer(nn.Module):
         self.mlp = Qwen3MLP(hidden_size, intermediate_size, ffn_bias, fused_elementwise, small_rows)
         self.norm_rows, self.fused_elementwise = min(small_rows, norm_rows), fused_elementwise
 
-    def _norm_in_product(self, norm, proj, x, glu=False):
+    def _norm_in_product(self, norm, proj, x, glu=False, joins=False):
         """A decode step's few rows: the residual norm runs as the prologue of the projection behind it (and SiluAndMul as its
-        epilogue) where that is faster than a launch of its own, with the same roundings."""
+        epilogue) where that is faster than a launch of its own or, with ``joins``, than as part of the projection before it; the roundings are the same."""
         return (self.norm_rows and self.fused_elementwise and x.dim() == 2 and x.shape[0] <= self.norm_rows and x.is_contiguous()
-                and _as_built(norm, RMSNorm) and _as_built(proj, Linear) and norm_linear_small_m_pays(x.shape[0], proj.weight)
+                and _as_built(norm, RMSNorm) and _as_built(proj, Linear) and norm_linear_small_m_pays(x.shape[0], proj.weight, joins)
                 and norm_linear_small_m_takes(x, proj.weight, self.norm_rows, glu=glu))
 
     def _project_norm(self, proj, x, residual, norm, into, glu=False):
         """``norm(proj(x), residual)`` where the norm can join the projection and is not better off in ``into``, the projection behind it (None: unknown),
         else the projection and ``residual`` as it is; and which."""
         if (norm is not None and self.norm_rows and _as_built(proj, Linear) and proj.small_rows and _as_built(norm, RMSNorm) and norm.fused
-                and not (into is not None and self._norm_in_product(norm, into, residual, glu))
+                and not (into is not None and self._norm_in_product(norm, into, residual, glu, joins=True))
                 and linear_add_rms_norm_takes(x, proj.weight, residual, proj.small_rows)):
             return *linear_add_rms_norm(x, proj.weight, proj.bias, residual, norm.weight_fp32(), norm.eps), True
         return proj(x), residual, False

@@ -8,6 +8,7 @@ import torch.nn.functional as F
 import minivllm_amd.layers.basic as basic
 import minivllm_amd.models.qwen3 as qwen3
 from minivllm_amd.layers.basic import Linear
+from minivllm_amd.layers.fused import norm_linear_small_m_pays
 from minivllm_amd.models.qwen3 import Qwen3DecoderLayer, Qwen3ForCausalLM
 
 
@@ -92,6 +93,21 @@ def test_steps_are_the_chain_of_modules(joined, rows):
     got, ran = model(ids, torch.arange(rows)), set(joined)
     assert ran == ({"prologue", "join"} if 4 <= rows <= 6 else {"prologue"} if rows < 4 else {"join", "glu"} if rows <= 64 else set())
     assert torch.allclose(got, expected(model, ids), rtol=1e-4, atol=1e-4)       # (gamma in fp32)
+
+
+@pytest.mark.parametrize("rows,prologues,joins", [(3, 6, 0), (4, 1, 6), (16, 1, 6), (17, 0, 6)])
+def test_a_norm_without_a_projection_before_it(joined, monkeypatch, rows, prologues, joins):
+    """Long rows: the norms join the projections before them from 4 rows on.  The first has none and stays in the product behind it up to 16."""
+    monkeypatch.setattr(qwen3, "norm_linear_small_m_pays", lambda rows, w, joins=False: norm_linear_small_m_pays(rows, torch.empty(4096, 2048, device="meta"), joins))
+    model, ids = decoder(), torch.arange(rows)
+    got = model(ids, ids)
+    assert (joined.count("prologue"), joined.count("join")) == (prologues, joins) and torch.allclose(got, expected(model, ids), rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("n,k,rows,joins,pays", [(4096, 1024, 16, True, True), (4096, 1024, 17, True, False), (4096, 2048, 3, True, True), (4096, 2048, 4, True, False),
+                                                 (4096, 2048, 16, False, True), (4096, 2048, 17, False, False), (4112, 2048, 1, False, False)])
+def test_norm_in_product_rule(n, k, rows, joins, pays):
+    assert norm_linear_small_m_pays(rows, torch.empty(n, k, device="meta"), joins) == pays
 
 
 @pytest.mark.parametrize("rows", [2, 5, 30, 64])
