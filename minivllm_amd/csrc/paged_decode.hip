@@ -439,7 +439,8 @@ struct DecodeHead {
 
   // one tile of 16 tokens starting at token t0 of the sequence; tokens at or past part_end do not count
   // (col_end: prefill only, where column n is a query row: tokens at or past it do not count for this lane's column)
-  // kRows: t.k holds whole rows, which become the first product's operands in k_lds (the wave's own: no barrier, the LDS keeps a wave's order)
+  // kRows: t.k holds whole rows, which become the first product's operands in k_lds (the wave's own: the LDS keeps a wave's order, the compiler is told to by barriers that are no
+  // instruction, since lanes read what others wrote)
   template <bool kRows = false>
   __device__ __forceinline__ void consume(const KVTile<T, D>& t, int part_end, float scale_log2, int lane,
                                           int col_end = 0x7fffffff, char* k_lds = nullptr) {
@@ -461,9 +462,11 @@ struct DecodeHead {
 #pragma unroll
       for (int j = 0; j < IO::kRowLoads; ++j)
         *reinterpret_cast<uint4*>(k_lds + IO::row_place(IO::kRowsPer * j + lane / IO::kChunks, lane % IO::kChunks)) = t.k[j];
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int j = 0; j < kSteps; ++j)
         s = mfma16x16x32<T>(*reinterpret_cast<const uint4*>(k_lds + IO::row_place(lane & 15, cls + 4 * j)), qf[j], s);
+      __builtin_amdgcn_wave_barrier();
     } else {
 #pragma unroll
       for (int j = 0; j < kSteps; ++j) s = mfma16x16x32<T>(t.k[j], qf[j], s);
@@ -1182,7 +1185,7 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
   for (int e = 0; e < 8; ++e) o[e] = (v4f){0.f, 0.f, 0.f, 0.f};
 
   __shared__ __attribute__((aligned(16))) char k_tiles[kRows ? kDecodeI8Wpb : 1][kRows ? kTile * D : 16];
-  char* k_lds = k_tiles[kRows ? threadIdx.x >> 6 : 0];        // this wave's (no barrier: the LDS keeps a wave's order)
+  char* k_lds = k_tiles[kRows ? threadIdx.x >> 6 : 0];        // this wave's
   auto consume = [&](const KVTileI8& t) {
     if constexpr (MVLLM_DECODE_LOADS_ONLY) {
       uint32_t x = __float_as_uint(t.ks) ^ __float_as_uint(t.vs);
@@ -1215,6 +1218,7 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
         const int tok = kRowsPer * j + lane / kChunks;
         *reinterpret_cast<uint4*>(k_lds + (tok * kChunks + ((lane ^ tok) & (kChunks - 1))) * 16) = t.k[j];
       }
+      __builtin_amdgcn_wave_barrier();                  // (DecodeHead::consume)
     }
 #pragma unroll
     for (int j = 0; j < kSteps; ++j) {
@@ -1223,6 +1227,7 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
       shi = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qhi[j], shi, 0, 0, 0);
       slo = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qlo[j], slo, 0, 0, 0);
     }
+    if constexpr (kRows) __builtin_amdgcn_wave_barrier();
     float s2[4], t2[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
