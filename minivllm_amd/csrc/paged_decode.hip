@@ -728,22 +728,29 @@ __device__ __forceinline__ int this_wave() { return __builtin_amdgcn_readfirstla
 // where there is one), a row's chunks trading places by its number.  Caches cold, 8 kv heads, operands / rows: 252 batches of 1 to 256 sequences in tables of
 // 512 to 16384 1.044 times as fast on average; one of 511 7.9 / 6.9 us, 64 of 64 to 2047 1.05 to 1.09, 24 to 40 full tables 1.04 to
 // 1.08, one wave per head, full tables 1.01, lengths spread 1.02 to 1.14.  Three waves per SIMD (168 registers, one spilled) instead of two: 1.025.
-// kStreamKeys: keys past the caches, as values (they are read once), where the waves of a head share it: 61 sequences of a decode step 558 / 571 us,
-// 16 of a smaller one 286 / 298, whose weights the caches hold; one wave per head, full tables 0.97 to 0.99 of the speed without.
 // Heads of 64, whose operands are half as many loads: one wave per head 1.01 to 1.05; where waves share one a row's longer way shows instead (one sequence of
 // 15000 in caches just read 17.9 / 19.4, tables of up to 512 0.98 to 1.00, 200 full ones 1.02), so not there.
 template <typename T, int W, int D, bool SUB>
 struct KeyRows {
   static constexpr bool kRows = sizeof(T) == 2 && !SUB && (D == 128 || (D == 64 && W == 1));
-  static constexpr bool kStreamKeys = W > 1;
 };
+// Rows of keys past the caches, as values, where the waves of a head share it (STREAM; one wave per head, full tables 0.97 to 0.99 of the speed without).
+// us streamed / not: 61 sequences of a decode step 558 / 571, 16 of a smaller one 278 / 296, whose weights the caches hold.  That is for keys that are
+// read once.  More than 16 query heads per kv head are several workgroups on the same rows: heads 32 over 1, 64 full tables of 8192
+// 110 / 93, 128 over 2, 128 of 2048 231 / 203, 16 of up to 8192 33.6 / 32.0.  Sequences that begin with the same blocks read them together: 16 of 13000
+// tokens, all but 400 shared, 149 / 127, 32 of 6400 132 / 114, 16 of 3000 29.0 / 26.8; with up to 1600 shared 15.9 / 15.2, 81 / 77, 110 / 117 (operands from
+// memory, before there were rows: 129, 121, 28.6, 17.6, 110, 137).  The host does not see that, so tables wider than kStreamCtx are not streamed, at
+// the price of 3 % where nothing is shared there (16 full ones of 8192 95 / 100, up to 900 tokens in them 15.0 / 16.1, 32 spread over them 70 / 74; operands
+// 102, 17.8 and 68.5).
+constexpr int kStreamCtx = 2048;
+static bool stream_keys(const DecodeArgs& a) { return a.head_chunks <= 1 && (int64_t)a.max_num_blocks * a.block_size <= kStreamCtx; }
 
 // W = 1: the wave walks all tiles of its partition.  W > 1 (the workgroup is W waves on one kv head): wave w takes
 // tiles w, w + W, ... and the partial results meet in LDS (finish_waves), so a short context costs a few tiles
 // of latency per wave and no second launch.
 // SUB: blocks of 1, 2, 4 or 8 tokens.  A 16-token tile then spans several blocks, and every lane looks up the blocks
 // of its own tokens (one for its K row, up to four for its V rows) in the block-table window.
-template <typename T, int W, int D, bool SUB = false>
+template <typename T, int W, int D, bool SUB = false, bool STREAM = false>
 __device__ __forceinline__ void decode_mfma_item(const DecodeArgs& a, int b, int p, int slice, int w) {
   const int lane = threadIdx.x & 63;
   const HeadSlice hs = head_slice(a, slice);
@@ -838,7 +845,7 @@ __device__ __forceinline__ void decode_mfma_item(const DecodeArgs& a, int b, int
       // V is read once, in whole 256-byte rows per instruction: non-temporal loads stream it past the caches.
       // K in the MFMA operand layout is 64 bytes of a row per instruction, so the second half of each 128-byte line
       // has to survive in cache until the next instruction: ordinary loads (the hint costs 7 % there).
-      if constexpr (kRows) IO::template load_k_rows<KeyRows<T, W, D, SUB>::kStreamKeys>(t, kp, row);
+      if constexpr (kRows) IO::template load_k_rows<STREAM>(t, kp, row);
       else IO::load_k(t, kp, lane >> 4);
 #pragma unroll
       for (int i = 0; i < 4; ++i) IO::template load_v<true>(t, i, vp + (int64_t)i * row, IO::owns(col));
@@ -1371,13 +1378,13 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512, D > 128 ? 1 : kDecodeWavesPerE
   decode_mfma_item<T, 1, D, SUB>(a, b, p, hg * (blockDim.x >> 6) + this_wave(), 0);
 }
 // Small batches: one workgroup of W waves per (partition, sequence, kv head), the waves splitting the tiles.
-template <typename T, int W, int D, bool SUB = false>
+template <typename T, int W, int D, bool SUB = false, bool STREAM = false>
 __global__ __launch_bounds__(64 * W, D > 128 ? 1 : kDecodeWavesPerEu) void decode_mfma_split_kernel(const DecodeArgs a) {
   // kv head fastest: the workgroups of one (sequence, partition) start together and read the same token rows
   const int b = blockIdx.z;
   const int g = blockIdx.x;
   const int p = (int)((blockIdx.y + (unsigned)b) % (unsigned)a.num_parts);
-  decode_mfma_item<T, W, D, SUB>(a, b, p, g, this_wave());
+  decode_mfma_item<T, W, D, SUB, STREAM>(a, b, p, g, this_wave());
 }
 template <typename T, int NCH, int D, bool kRows>
 __global__ __launch_bounds__(kDecodeI8Threads, kDecodeI8WavesPerEu) void decode_mfma_int8_kernel(const DecodeArgs a) {
@@ -1705,6 +1712,14 @@ static int launch_decode(DecodeArgs a, bool int8, bool fast_ok, int waves, hipSt
     const dim3 grid((unsigned)a.num_parts, (unsigned)a.batch, groups);
     auto go = [&](auto DIM) {
       constexpr int D = decltype(DIM)::value;
+      if constexpr (IsSixteenBit<T>::value && D == 128) {
+        if (split && stream_keys(a)) {
+          if (waves == kSplitManyWaves) decode_mfma_split_kernel<T, kSplitManyWaves, D, false, true><<<split_grid, dim3(64 * kSplitManyWaves), 0, stream>>>(a);
+          else decode_mfma_split_kernel<T, kSplitWaves, D, false, true><<<split_grid, split_block, 0, stream>>>(a);
+          launched = true;
+          return;
+        }
+      }
       if constexpr (IsSixteenBit<T>::value && (D < kSplitWideDim || D == 128)) {
         if (waves == kSplitManyWaves) {
           decode_mfma_split_kernel<T, kSplitManyWaves, D><<<split_grid, dim3(64 * kSplitManyWaves), 0, stream>>>(a);

@@ -92,11 +92,12 @@ def test_eight_waves_per_head(hq, hkv, d, bs, ctx_list):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("waves,batch,blocks", [(8, 20, 2), (4, 64, 2), (1, 64, 1024)])
-def test_every_key_meets_its_own_value(waves, batch, blocks, d, dtype):
+@pytest.mark.parametrize("waves,batch,blocks,group", [(8, 20, 2, 2), (4, 64, 2, 2), (1, 64, 1024, 2), (4, 20, 256, 2),       # tables that are streamed; one wave; wide ones
+                                                      (8, 10, 2, 20), (4, 64, 2, 20)])                                    # several workgroups read the same keys
+def test_every_key_meets_its_own_value(waves, batch, blocks, group, d, dtype):
     """Keys of +-1 and queries that are four times one of them: that token's weight is 1 and each other's below e^-24 (asserted), so
     that the result is its value, bit for bit, wherever in a tile it lies."""
-    hkv, group, bs = 8, 2, 16
+    hkv, bs = 8, 16
     assert paged_decode_plan(batch, hkv * group, hkv, d, blocks, bs, dtype)[2] == waves
     g = torch.Generator().manual_seed(5)
     kc = (torch.randint(0, 2, (2 * batch, bs, hkv, d), generator=g) * 2 - 1).to(dtype)
