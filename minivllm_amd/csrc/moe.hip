@@ -608,19 +608,25 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
 // known and its rows' places are loaded a tile ahead, its first copies run beside the stores, and these go through LDS, since a lane's runs of eight outputs
 // in 32 rows took the address unit four times as long as whole rows do.  us: 65536 rows, 2048 x 768 268 -> 229, 2048 x 2048 498 -> 472; both
 // products of 8192 rows, top 6 of 64, routed unevenly, 1536 x 2048 with the gate 359 -> 337, 2048 x 768 238 -> 219.
-constexpr int kLargeGroups = 32;                    // workgroups per XCD: its CUs
+// With K of 4096 and more and two and a half rounds, the way into a tile is little of it and uneven tiles are more: there every tile has a workgroup of its
+// own again and goes where a CU is free.  us, 64 experts of 2560 x 4096 with the gate, 60 / 160 / 200 / 300 rows each, strided 294 / 366 / 381 / 500, so 278 / 342 /
+// 378 / 475, of 3072 x 4096 340 / 449 / 499 / 617 and 335 / 433 / 495 / 601 (a round and a quarter, 32 experts of 2560 x 4096, 80 rows 159 and 166).
+// Halves: tiles of the last round in halves gain a quarter of a tile (64 experts of 1536 x 2048 with the gate, 132 rows each 113 / 104 without / with), but where
+// tiles of few rows were to fill that round they come one round later: 156 rows 116 / 126, 180 120 / 131.
+constexpr int kLargeGroups = 32;                    // workgroups per XCD that go on to another tile: its CUs
 template <int kGlu>
 __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLinearArgs a) {
   constexpr int kTile = 256, kK = 64, kStage = kTile * kK * 2;       // bytes of one operand's step
   __shared__ __attribute__((aligned(16))) char lds[5 * kStage];      // weights three times, x twice
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
   // ---- this workgroup's tiles: every a.groups-th of its XCD's.  Where they leave a last round of no more than half the workgroups, its tiles are
-  // taken in halves of 128 rows; tiles of few rows come behind them ----
+  // taken in halves of 128 rows, unless these push the tiles of few rows, which come behind them, into one round more ----
   const int n_tiles = a.n_tiles, whole = a.num_tiles[0], rest = a.num_tiles[1], xcd = blockIdx.x & 7;
   const int per = (whole * n_tiles + 7) / 8, rest_per = (rest * n_tiles + 7) / 8;
   const int low = min(xcd * per, whole * n_tiles), high = min(low + per, whole * n_tiles);
   const int rest_low = min(xcd * rest_per, rest * n_tiles), rest_high = min(rest_low + rest_per, rest * n_tiles);
-  const int last = (high - low) % a.groups, halved = 2 * last <= a.groups ? last : 0, full = high - low - halved;
+  const int last = (high - low) % kLargeGroups, behind = last + rest_high - rest_low;
+  const int halved = 2 * last <= kLargeGroups && (behind + last - 1) / kLargeGroups == (behind - 1) / kLargeGroups ? last : 0, full = high - low - halved;
   const int places = full + 2 * halved + rest_high - rest_low;
   struct Tile { int e, row0, rows, n_tile; };
   auto find = [&](int j, Tile& t) __attribute__((always_inline)) {
@@ -865,16 +871,21 @@ static int tile_rows(int64_t pairs, int experts) {
   return pairs >= kLargeTileRows * (int64_t)experts ? 256 : pairs > kSmallTileRows * (int64_t)experts ? 128 : 64;
 }
 static int64_t max_tiles(int64_t pairs, int experts, int rows) { return (pairs + rows - 1) / rows + experts; }
+// Tiles of 256 rows and weight rows to be expected.
+static int64_t large_tiles(int64_t pairs, int experts, int N) {
+  const int64_t rows = pairs / 256 + experts / 2;
+  return (N + 255) / 256 * (rows > experts ? rows : experts);
+}
 // Whether a product of N outputs runs on the tiles of 256 rows of a plan that has both.  With 48 to 384 rows per expert a large tile has one to four of its
 // blocks of 64 rows; it reads every weight once for the expert's rows and half as much of LDS per flop, but has a CU to itself: it pays where there is one
-// for each CU and N fills it.  us as 128 and 256 rows, weights from memory, top 4 routed unevenly: 64 experts of 1536 x 2048 with the gate (384 tiles and
-// more), 50 rows each 88 / 84, 80 87 / 94, 120 111 / 102, 340 193 / 169, of 2048 x 768 49 / 46, 57 / 50, 62 / 61, 128 / 99, of 2560 x 4096 271 / 258, 278 /
-// 295, 344 / 319, 646 / 528; 32 of 2048 x 1024 (256 tiles) 41 / 31, 45 / 45, 46 / 49, 82 / 62; but 32 of 1536 x 2048 (192) 41 / 46, 47 / 45, of 640 x 1536
-// 27 / 29, 25 / 32, 26 / 35, 8 of 1536 x 2048 (48) 23 / 25, 340 rows each 29 / 41.
+// for each CU and N fills it.  us as 128 and 256 rows, weights from memory, top 4 routed unevenly, 50 / 80 / 120 / 340 rows each: 64 experts of 1536 x 2048 with
+// the gate (384 tiles and more) 98 99 125 208 / 94 101 105 168, of 2048 x 768 57 59 71 132 / 55 60 61 96, of 2560 x 4096 282 331 365 722 / 268 295 313 531; 32 of
+// 2048 x 1024 (256 tiles) 42 44 48 87 / 36 50 50 62.  370 batches of 16 to 128 experts, 49 to 1500 rows each, from 256 tiles on: 0.944 of the time that the rule before took,
+// 640 tiles or 384 of many rows; what loses has a few rows more than a block on average (70 to 115 rows; worst 32 of 3072 x 1024 with the gate, 76 rows 56 / 61,
+// 64 of 1024 x 2048, 95 rows 86 / 90).  Below: 32 of 1536 x 2048 (192) 48 49 75 111 / 48 53 51 85, 16 of 1024 x 2048 (64 tiles), 56 rows 33 / 33.
 static bool large_tiles_pay(int64_t pairs, int experts, int N) {
-  const int64_t wide = (N + 255) / 256, rows = pairs / 256 + experts / 2, tiles = wide * (rows > experts ? rows : experts);
-  if (8 * (256 * wide - N) > N) return false;
-  return tiles >= 256;
+  if (8 * (256 * ((N + 255) / 256) - N) > N) return false;
+  return large_tiles(pairs, experts, N) >= 256;
 }
 static int plan_blocks(int64_t pairs) { return (int)((pairs + kPlanPairs - 1) / kPlanPairs); }
 
@@ -1009,7 +1020,8 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
     a.x_bytes = (uint32_t)x_bytes;
     const int64_t blocks = 8 * (((int64_t)a.max_tiles * a.n_tiles + 7) / 8 + 1 + a.n_tiles);
     if (blocks > 0x7fffffff) return MVLLM_ERR_BAD_SHAPE;
-    a.groups = (int)(blocks / 8 < kLargeGroups ? blocks / 8 : kLargeGroups);
+    const bool own = K >= 4096 && large_tiles(pairs, experts, N) >= 640;         // (moe_linear_large_kernel)
+    a.groups = (int)(own || blocks / 8 < kLargeGroups ? blocks / 8 : kLargeGroups);
     a.token_factor = 0xffffffffu / (uint32_t)(per_token ? per_token : 1);
     with_glu(glu, [&](auto G) {
       constexpr int kGlu = decltype(G)::value;

@@ -596,11 +596,14 @@ def test_moe_linear_walks_and_shares(counts, n, k, glu):
     ([1024] * 10, 2048, 64, 1),                                       # 320 tiles, 40 per XCD: one round, eight tiles of the second in halves
     ([1000] * 10 + [64, 1, 0, 300, 128, 640], 2048, 192, 3),          # the same with tiles that are not whole, halves without rows, few rows behind them
     ([300, 520, 20, 700] * 20, 1040, 128, 7),                         # last weight tile of 16 outputs; rows are pair / 7
+    ([1024] * 10 + [20] * 20, 2048, 64, 1),                           # 40 tiles per XCD and 20 of few rows, which halves would push into a third round
+    ([1024] * 10 + [20] * 30, 2048, 64, 1),                           # the same with 30, which need that round anyway
+    ([4096] * 9 + [4000, 40], 1024, 4096, 1),                         # long K: a workgroup for every tile
 ])
 @pytest.mark.parametrize("glu", [False, True])
 def test_moe_linear_rounds_of_large_tiles(counts, n, k, top, glu):
-    """More tiles of 256 rows than CUs, so that workgroups go from one to the next: every row against the product in float32, whose sums of at most 192
-    numbers differ by less than a rounding to 16 bits (2^-9 of the value), the gated ones by those of its factors."""
+    """More tiles of 256 rows than CUs, so that workgroups go from one to the next: every row against the product in float32, whose sums
+    differ by less than a rounding to 16 bits (2^-9 of the value), the gated ones by those of its factors."""
     g = torch.Generator(device=DEV).manual_seed(n + k)
     pairs = sum(counts) // top * top
     ids = torch.cat([torch.full((c,), i, device=DEV) for i, c in enumerate(counts)])[torch.randperm(sum(counts), generator=g, device=DEV)]
