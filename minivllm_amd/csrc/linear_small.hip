@@ -484,7 +484,8 @@ static LinearSplit linear_split(int M, int N, int K) {
 
 // The same where the residual norm follows and its launch adds the parts up (parts_norm_kernel): it reads 4 bytes a part instead of two, and has
 // less to wait for than the norm alone, a thread for four numbers.  So parts pay nearly everywhere: two to four of them, with the narrowest
-// tile of which 256 CUs have a workgroup each, but at least two stages in a part.  us with the norm at 4 / 17 / 40 / 61 rows, apart (linear_split's
+// tile of which 256 CUs have a workgroup each, of at least two stages but for a last part (K of 2560, up to 1024 columns: 3, 3, 3
+// and 1).  us with the norm at 4 / 17 / 40 / 61 rows, apart (linear_split's
 // where it takes the shape) and now: 1024 x 2048 6.8 / 7.0 / 7.2 / 7.4 and 5.4 / 5.9 / 6.1 / 6.6, 1024 x 3072 7.4 / 7.3 / 9.8 / 10.4 and 5.7 / 6.2 / 6.5 / 7.1,
 // 2048 x 2048 6.8 / 7.0 / 8.2 / 9.0 and 6.1 / 6.6 / 7.1 / 7.8, 2048 x 6144 10.5 / 11.3 / 12.8 / 14.1 and 8.3 / 9.1 / 10.5 / 11.8, 2560 x 2560 8.7 / 9.7 / 11.7 / 12.8
 // and 7.3 / 7.7 / 8.8 / 10.2, 4096 x 4096 10.9 / 12.0 / 14.3 / 16.3 and 10.2 / 11.0 / 12.5 / 14.0, 4096 x 12288 23.5 / 23.4 / 25.7 / 28.4 and 20.7 / 21.5 / 23.5 / 25.9,

@@ -17,7 +17,7 @@
 //                            and two byte permutes per product turn them into the B operand.
 //   See DecodeHead for the operand layouts.
 // The kernel is HBM-bound: a kernel that only issues the same loads (no arithmetic) reaches
-// 6.25 TB/s on this access pattern, this one about 6.05.
+// 6.10 to 6.14 TB/s on this access pattern, this one 6.09 to 6.11 (256 sequences of 128 to 32768 tokens, the merge included).
 #include <atomic>
 #include <type_traits>
 #include "common.h"

@@ -449,9 +449,11 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
 // The range of a cached batch, which is even.  A workgroup alone on its CU waits a tile's trip to memory, 0.85 us, so that the longest sequence's chain
 // decides until the CUs have several; `on_cu` is what a CU has in tiles, sequences of log-uniform lengths assumed, the more of them the further
 // below the longest.  A merge takes 1.6 us and each range its partial results' way.  Fitted to 356 random batches, caches cold, and tried on 368 others: on
-// average 1.4 % behind the best range of each (3.8 % before, where a range was at least 6 tiles and batches of more than 192 workgroups were whole).  us
+// average 1.4 % behind the best range of each (3.8 % before, where a range was at least 6 tiles and batches of more than 192 workgroups were whole).  1086
+// batches, 1 to 16 sequences, took 0.977 of the time before, 192 of them less than 0.95, 14 more than 1.05 (five of 240 rows in all, 20 tiles, 16 heads 19.9 / 23.3;
+// two of 554, 87 tiles 72.6 / 84; four of 480, 72 tiles, heads of 64 27.7 / 32).  us
 // before / now, heads of 128: 12 of 755 rows in all, 95 % cached, 32 heads, up to 50 tiles 72.2 / 54; of 572, 37 tiles 55.4 / 38.9; three of 145, 16 tiles 23.2 /
-// 17.9; the worst, nine of 12 tiles, 104 workgroups, 1.19 times as long.  From 193 workgroups on equal ones gain nothing (1500 rows behind 1500, 376
+// 17.9; furthest behind the best, nine of 12 tiles, 104 workgroups, 1.19 times as long.  From 193 workgroups on equal ones gain nothing (1500 rows behind 1500, 376
 // workgroups: 72 whole, 86 in two), and few sequences may be equal.
 static int64_t cached_range(int64_t wgs, int64_t tiles, int num_seqs, float fresh, int head_dim, float part_us) {
   const float on_cu = 1.29f * powf((float)num_seqs, -0.4f) * (1.f - 0.29f * fresh) * (float)(wgs * tiles) / 256.f, per_tile = head_dim == 64 ? 0.58f : 0.85f;

@@ -388,7 +388,7 @@ def norm_linear_small_m(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tenso
 
 def linear_add_rms_norm_takes(x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, max_rows: int = 64) -> bool:
     """Whether ``linear_add_rms_norm`` is built for this call, and pays: 4 to 64 rows, bf16 / fp16 on the GPU, K a multiple of 512 from
-    1024 on, 512 to 7168 outputs (a multiple of 16), a dense residual."""
+    1024 on (from 2048 on with more than 4096 outputs), 512 to 7168 outputs (a multiple of 16), a dense residual."""
     return (linear_small_m_takes(x, weight, max_rows) and residual.dtype == x.dtype and residual.is_contiguous()
             and tuple(residual.shape) == (x.shape[0], weight.shape[0]) and x.shape[1] == weight.shape[1] and residual.data_ptr() % 16 == 0
             and weight.data_ptr() % 16 == 0

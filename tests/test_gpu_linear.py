@@ -280,6 +280,21 @@ def test_linear_add_rms_norm(dtype, m, n, k, bias, stride):
     assert not linear_add_rms_norm_takes(x[:3], w, residual[:3])
 
 
+@pytest.mark.parametrize("m", [4, 17, 61])
+@pytest.mark.parametrize("n,k", [(1024, 1024), (2048, 2048), (2560, 2560), (5120, 5120)])
+def test_linear_add_rms_norm_in_place(m, n, k):
+    """The sum with the residual in the residual's place, and the norm in that of x: what the call writes elsewhere otherwise, bit for bit."""
+    x, w, b = _case(40 + m, m, n, k, torch.bfloat16, True)
+    residual, gamma = torch.randn(m, n, device=DEV).bfloat16(), torch.rand(n, device=DEV) + 0.5
+    want, total = linear_add_rms_norm(x, w, b, residual, gamma, 1e-6)
+    lib = _C.load()
+    need = lib.mvllm_linear_add_rms_norm_bytes(m, n, k, k)
+    workspace = torch.empty(need, dtype=torch.uint8, device=DEV)
+    st = lib.mvllm_linear_add_rms_norm(x.data_ptr(), residual.data_ptr(), x.data_ptr(), w.data_ptr(), b.data_ptr(), residual.data_ptr(), gamma.data_ptr(), 1e-6, k, m, n, k,
+                                       _C.dtype_code(x.dtype), workspace.data_ptr(), need, _C.current_stream_ptr(x.device))
+    assert st == 0 and torch.equal(x, want) and torch.equal(residual, total)
+
+
 @pytest.mark.parametrize("n,k", [(496, 1024), (512, 512), (4112, 1024), (7184, 2048)])
 def test_linear_add_rms_norm_leaves_the_rest(n, k):
     x, w, _ = _case(7, 5, n, k, torch.bfloat16, False)

@@ -626,7 +626,7 @@ def test_moe_linear_rounds_of_large_tiles(counts, n, k, top, glu):
     assert worst.max() < 2 ** -8, worst.max()
 
 
-@pytest.mark.parametrize("n,k", [(2560, 128), (2304, 64)])           # products on tiles of 256 rows; those whose rows are no multiple of 16 bytes on those of 128
+@pytest.mark.parametrize("n,k", [(2560, 128), (2304, 64), (768, 64)])      # products on tiles of 256 rows; those of 768 outputs (192 tiles), and those whose rows are no multiple of 16 bytes, on those of 128
 @pytest.mark.parametrize("glu", [False, True])
 @pytest.mark.parametrize("more", [0, 120])
 def test_moe_linear_both_tilings_of_a_plan(n, k, glu, more):
