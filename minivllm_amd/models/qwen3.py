@@ -22,10 +22,13 @@ from minivllm_amd.utils.context import get_context
 
 def _as_built(module, kind):
     """Whether calling ``module`` is ``kind.forward`` and nothing else, so that its work may be done as a part of another launch: not where it was
-    replaced, or somebody hooked into it."""
-    return (type(module) is kind and "forward" not in module.__dict__
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
-            and not _has_any_global_hook())
+    replaced, or somebody hooked into it (hooks on all modules: ``_has_any_global_hook``).  A step asks this of every module it passes by: 0.3 us each."""
+    own = module.__dict__
+    return type(module) is kind and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own)
+
+
+# a norm between two projections: nobody has looked yet, it has been applied with the one before, it is to run in the one behind
+_OPEN, _NORMED, _INSIDE = range(3)
 
 
 class Qwen3Attention(nn.Module):
@@ -84,7 +87,7 @@ class Qwen3MLP(nn.Module):
         """``forward`` without the last projection."""
         # a decode step's rows: SiluAndMul as the epilogue of the gate/up projection (one launch instead of two)
         if (self.small_rows and self.fused and x.dim() == 2 and x.shape[0] <= self.small_rows and x.is_contiguous()
-                and _as_built(self.gate_up, Linear) and _as_built(self.activation, SiluAndMul)
+                and _as_built(self.gate_up, Linear) and _as_built(self.activation, SiluAndMul) and not _has_any_global_hook()
                 and norm_linear_small_m_takes(x, self.gate_up.weight, self.small_rows, norm=False, glu=True)):
             return norm_linear_small_m(x, self.gate_up.weight, self.gate_up.bias, glu=True)
         return self.activation(self.gate_up(x))
@@ -104,32 +107,39 @@ class Qwen3DecoderLayer(nn.Module):
     def _norm_in_product(self, norm, proj, x, glu=False, joins=False):
         """A decode step's few rows: the residual norm runs as the prologue of the projection behind it (and SiluAndMul as its
         epilogue) where that is faster than a launch of its own or, with ``joins``, than as part of the projection before it; the roundings are the same."""
-        return (self.norm_rows and self.fused_elementwise and x.dim() == 2 and x.shape[0] <= self.norm_rows and x.is_contiguous()
-                and _as_built(norm, RMSNorm) and _as_built(proj, Linear) and norm_linear_small_m_pays(x.shape[0], proj.weight, joins)
-                and norm_linear_small_m_takes(x, proj.weight, self.norm_rows, glu=glu))
+        if not (self.norm_rows and self.fused_elementwise and x.dim() == 2 and x.shape[0] <= self.norm_rows and x.is_contiguous()
+                and _as_built(norm, RMSNorm) and _as_built(proj, Linear)):
+            return False
+        weight = proj.weight
+        return norm_linear_small_m_pays(x.shape[0], weight, joins) and norm_linear_small_m_takes(x, weight, self.norm_rows, glu=glu)
 
     def _project_norm(self, proj, x, residual, norm, into, glu=False):
         """``norm(proj(x), residual)`` where the norm can join the projection and is not better off in ``into``, the projection behind it (None: unknown),
         else the projection and ``residual`` as it is; and which."""
-        if (norm is not None and self.norm_rows and _as_built(proj, Linear) and proj.small_rows and _as_built(norm, RMSNorm) and norm.fused
-                and not (into is not None and self._norm_in_product(norm, into, residual, glu, joins=True))
+        if norm is None or not _as_built(proj, Linear):
+            return proj(x), residual, _OPEN
+        if into is not None and self._norm_in_product(norm, into, residual, glu, joins=True):
+            return proj(x), residual, _INSIDE
+        if (self.norm_rows and proj.small_rows and norm.fused and _as_built(norm, RMSNorm)
                 and linear_add_rms_norm_takes(x, proj.weight, residual, proj.small_rows)):
-            return *linear_add_rms_norm(x, proj.weight, proj.bias, residual, norm.weight_fp32(), norm.eps), True
-        return proj(x), residual, False
+            return *linear_add_rms_norm(x, proj.weight, proj.bias, residual, norm.weight_fp32(), norm.eps), _NORMED
+        return proj(x), residual, _OPEN
 
     def forward(self, x, residual, positions):
         return self.walk(x, residual, positions)[:2]
 
-    def walk(self, x, residual, positions, normed=False, behind=None, into=None):
-        """``forward`` for a caller that knows its neighbours: ``normed``, x is behind the input norm already; ``behind``, the norm that follows the
-        layer and may be applied here, with ``into`` the projection that follows it.  The third result says whether it has been.  Modules that are not as
+    def walk(self, x, residual, positions, state=_OPEN, behind=None, into=None):
+        """``forward`` for a caller that knows its neighbours: ``state`` of the input norm; ``behind``, the norm that follows the
+        layer and may be applied here, with ``into`` the projection that follows it.  The third result is that norm's state.  Modules that are not as
         this file builds them are called as they are."""
         attn, mlp, norm = self.self_attn, self.mlp, self.input_layernorm
-        own_attn, own_mlp = _as_built(attn, Qwen3Attention), _as_built(mlp, Qwen3MLP)
+        free = not _has_any_global_hook()
+        own_attn = free and _as_built(attn, Qwen3Attention)
+        own_mlp = free and _as_built(mlp, Qwen3MLP) and _as_built(mlp.activation, SiluAndMul)
         qkv = None
-        if normed:
+        if state == _NORMED:
             pass
-        elif own_attn and self._norm_in_product(norm, attn.qkv_projection, x):
+        elif own_attn and (state == _INSIDE or self._norm_in_product(norm, attn.qkv_projection, x)):
             proj = attn.qkv_projection
             qkv = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps, residual, residual is not None)
             qkv, residual = (qkv, x) if residual is None else qkv
@@ -137,20 +147,20 @@ class Qwen3DecoderLayer(nn.Module):
             residual, x = x, norm(x)
         else:
             x, residual = norm(x, residual)
-        norm, normed = self.post_attention_layernorm, False
+        norm, state = self.post_attention_layernorm, _OPEN
         if own_attn:
             x = attn.attend(attn.qkv_projection(x) if qkv is None else qkv, positions)
-            x, residual, normed = self._project_norm(attn.output_projection, x, residual, norm, mlp.gate_up if own_mlp else None, glu=True)
+            x, residual, state = self._project_norm(attn.output_projection, x, residual, norm, mlp.gate_up if own_mlp else None, glu=True)
         else:
             x = attn(x, positions)
-        if not normed and own_mlp and _as_built(mlp.activation, SiluAndMul) and self._norm_in_product(norm, mlp.gate_up, x, glu=True):
+        if state != _NORMED and own_mlp and (state == _INSIDE or self._norm_in_product(norm, mlp.gate_up, x, glu=True)):
             proj = mlp.gate_up
             x, residual = norm_linear_small_m(x, proj.weight, proj.bias, norm.weight_fp32(), norm.eps, residual, True, glu=True)
         else:
-            if not normed:
+            if state != _NORMED:
                 x, residual = norm(x, residual)
             if not own_mlp:
-                return mlp(x), residual, False
+                return mlp(x), residual, _OPEN
             x = mlp.gated(x)
         return self._project_norm(mlp.gate_down, x, residual, behind, into)
 
@@ -193,21 +203,22 @@ class Qwen3ForCausalLM(nn.Module):
         # a decode step's few rows by plain indexing: the embedding operator's small-batch kernel takes 11 us for 16
         # rows, the gather 4
         x = self.embedding_layer.weight[input_ids] if input_ids.numel() <= 256 else self.embedding_layer(input_ids)
-        residual, normed, layers = None, False, list(self.layer_stack)
-        own = [_as_built(layer, Qwen3DecoderLayer) for layer in layers]
+        residual, state, layers = None, _OPEN, list(self.layer_stack)
+        free = not _has_any_global_hook()
+        own = [free and _as_built(layer, Qwen3DecoderLayer) for layer in layers]
         for i, layer in enumerate(layers):
             behind = into = None
             if i + 1 == len(layers):
-                behind = self.final_layernorm
+                behind = self.final_layernorm if free else None
             elif own[i + 1]:
                 behind, attn = layers[i + 1].input_layernorm, layers[i + 1].self_attn
                 into = attn.qkv_projection if _as_built(attn, Qwen3Attention) else None
             if own[i]:
-                x, residual, normed = layer.walk(x, residual, positions, normed, behind, into)
+                x, residual, state = layer.walk(x, residual, positions, state, behind, into)
             else:
                 x, residual = layer(x, residual, positions)
-                normed = False
-        return x if normed else self.final_layernorm(x, residual)[0]
+                state = _OPEN
+        return x if state == _NORMED else self.final_layernorm(x, residual)[0]
 
     def compute_logits(self, hidden):
         context = get_context()
