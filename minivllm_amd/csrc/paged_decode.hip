@@ -738,11 +738,12 @@ struct KeyRows {
 // us streamed / not: 61 sequences of a decode step 558 / 571, 16 of a smaller one 278 / 296, whose weights the caches hold.  That is for keys that are
 // read once.  More than 16 query heads per kv head are several workgroups on the same rows: heads 32 over 1, 64 full tables of 8192
 // 110 / 93, 128 over 2, 128 of 2048 231 / 203, 16 of up to 8192 33.6 / 32.0.  Sequences that begin with the same blocks read them together: 16 of 13000
-// tokens, all but 400 shared, 149 / 127, 32 of 6400 132 / 114, 16 of 3000 29.0 / 26.8; with up to 1600 shared 15.9 / 15.2, 81 / 77, 110 / 117 (operands from
-// memory, before there were rows: 129, 121, 28.6, 17.6, 110, 137).  The host does not see that, so tables wider than kStreamCtx are not streamed, at
-// the price of 3 % where nothing is shared there (16 full ones of 8192 95 / 100, up to 900 tokens in them 15.0 / 16.1, 32 spread over them 70 / 74; operands
-// 102, 17.8 and 68.5).
-constexpr int kStreamCtx = 2048;
+// tokens, all but 400 shared, 149 / 127, 32 of 6400 132 / 114 (operands from memory, before there were rows: 129, 121).  The host does not see that, so
+// tables wider than kStreamCtx are not streamed, at the price of 3 % where nothing is shared there (16 full ones of 8192 95 / 100, up to 900 tokens in them
+// 15.0 / 16.1, 32 spread over them 70 / 74; operands 102, 17.8 and 68.5).  In tables of 4096 the two are about even: fronts of 3000 tokens, 16 sequences 29.0 /
+// 26.8, 32 48.9 / 44.1 (operands 28.6, 47.3), nothing shared, 61 full ones 172 / 179, 32 spread 37.2 / 40.3; below, with up to 1600 shared, 15.9 / 15.2,
+// 81 / 77, 110 / 117 (17.6, 110, 137).
+constexpr int kStreamCtx = 4096;
 static bool stream_keys(const DecodeArgs& a) { return a.head_chunks <= 1 && (int64_t)a.max_num_blocks * a.block_size <= kStreamCtx; }
 
 // W = 1: the wave walks all tiles of its partition.  W > 1 (the workgroup is W waves on one kv head): wave w takes

@@ -92,7 +92,7 @@ def test_eight_waves_per_head(hq, hkv, d, bs, ctx_list):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("waves,batch,blocks,group", [(8, 20, 2, 2), (4, 64, 2, 2), (1, 64, 1024, 2), (4, 20, 256, 2),       # tables that are streamed; one wave; wide ones
+@pytest.mark.parametrize("waves,batch,blocks,group", [(8, 20, 2, 2), (4, 64, 2, 2), (1, 64, 1024, 2), (4, 20, 512, 2),       # tables that are streamed; one wave; wide ones
                                                       (8, 10, 2, 20), (4, 64, 2, 20)])                                    # several workgroups read the same keys
 def test_every_key_meets_its_own_value(waves, batch, blocks, group, d, dtype):
     """Keys of +-1 and queries that are four times one of them: that token's weight is 1 and each other's below e^-24 (asserted), so
