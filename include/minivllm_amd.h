@@ -748,6 +748,15 @@ int mvllm_moe_plan(void* plan, size_t plan_bytes, const int32_t* ids, int64_t pa
 int mvllm_moe_linear(void* out, int64_t out_row_stride, const void* x, int64_t x_row_stride, const void* w,
                      const int32_t* ids, void* plan, int64_t pairs, int experts, int N, int K, int per_token, int glu,
                      int dtype, void* stream);
+/*
+ * mvllm_moe_linear_shared: ... and in the same launch shared_out row r = shared_x row r through shared_w [shared_N, shared_K]
+ *   for shared_rows rows, with glu silu(gate) * up of weights whose gate rows all come before the up rows (an expert that
+ *   every row goes through).  With a plan, bf16; shared_K % 64 == 0, shared_N % 16 == 0 (glu: 64), row strides multiples of 8.
+ */
+int mvllm_moe_linear_shared(void* out, int64_t out_row_stride, const void* x, int64_t x_row_stride, const void* w,
+                            const int32_t* ids, void* plan, int64_t pairs, int experts, int N, int K, int per_token, int glu,
+                            void* shared_out, int64_t shared_out_row_stride, const void* shared_x, int64_t shared_x_row_stride,
+                            const void* shared_w, int shared_rows, int shared_N, int shared_K, int dtype, void* stream);
 
 /*
  * ... and for models whose router is a softmax and whose experts have a clamped gate:

@@ -137,6 +137,8 @@ SIGNATURES = {
     "mvllm_moe_plan_bytes": (c_size_t, [c_int64, c_int]),
     "mvllm_moe_plan": (c_int, [c_void_p, c_size_t, c_void_p, c_int64, c_int, c_void_p]),
     "mvllm_moe_linear": (c_int, [c_void_p, c_int64, c_void_p, c_int64] + [c_void_p] * 3 + [c_int64] + [c_int] * 6 + [c_void_p]),
+    "mvllm_moe_linear_shared": (c_int, [c_void_p, c_int64, c_void_p, c_int64] + [c_void_p] * 3 + [c_int64] + [c_int] * 5 +
+                                [c_void_p, c_int64, c_void_p, c_int64, c_void_p] + [c_int] * 4 + [c_void_p]),
     "mvllm_mlstm_output": (c_int, [c_void_p] * 5 + [c_int64, c_float] + [c_void_p] * 5 + [c_int64, c_int, c_int, c_int,
                                                                                       c_void_p]),
     "mvllm_moe_route_softmax": (c_int, [c_void_p] * 3 + [c_int64, c_void_p, c_int64] + [c_int] * 4 + [c_void_p]),

@@ -8,6 +8,7 @@
 //               32, so that both halves of an output are in one lane
 // Products, by the number of rows: very few (no plan; a workgroup finds its expert's rows itself, its waves share K), many (bf16: tiles of 64 x 128,
 // 128 x 128 or 256 x 256 on the matrix unit over sorted rows), any (fp32, over sorted rows).
+#include "expert_tiles.h"
 #include "prefill_tiles.h"
 
 #pragma clang fp contract(off)
@@ -280,9 +281,28 @@ struct ExpertLinearArgs {
   float alpha, limit, shift;   // of kClampedGlu
   int groups;                  // (large) workgroups per XCD
   uint32_t token_factor;       // (large) (2^32 - 1) / per_token
+  // The product of an expert that all rows go through, as more tiles of the same launch: row r of x to row r of out.  On its own it took two or three
+  // launches that leave CUs idle at their ends, and the activation between them went through memory as twice as many numbers.  us of a mixture and the norm
+  // behind it, apart / so: 2048 wide, top 6 of 64 experts of 768 and 1536 shared, 3 rows 57 / 55, 100 137 / 120, 300 168 / 145, 1000 236 / 203, 8192 742 / 710;
+  // 4096 wide, top 8 of 64 of 1280 and 2048 shared, 32 rows 328 / 317, 1000 621 / 572.
+  struct Shared {
+    const bf16_t* x;           // [rows, x_stride]
+    const bf16_t* w;           // [N, K], with a gate all its rows before all of up's
+    bf16_t* out;               // [rows, out_stride]
+    int64_t x_stride, out_stride;
+    int rows, N, K;            // (no rows: there is none)
+    int row_tiles, n_tiles, blocks;     // (many) blocks: of the grid, in front of the others, a multiple of eight
+    int units;                 // (large) what a tile takes, in tiles of the experts
+    uint32_t x_bytes;
+  } shared;
 };
 
 enum { kNoGlu = 0, kSiluGlu = 1, kClampedGlu = 2 };
+
+// The row of the shared expert's weights for row r of a product's tiles, in which gate and up rows come in turns of 32.
+template <int kGlu> __device__ __forceinline__ int shared_row(const ExpertLinearArgs& a, int r) {
+  return kGlu != kNoGlu ? (r >> 6 << 5) + (r & 31) + ((r >> 5 & 1) != 0 ? a.shared.N / 2 : 0) : r;
+}
 
 // silu(g) * u, or with g' = min(g, limit) and u' = u within +-limit: g' sigmoid(alpha g') (u' + shift)
 template <int kGlu> __device__ __forceinline__ float glu_of(const ExpertLinearArgs& a, float g, float u) {
@@ -442,25 +462,8 @@ __global__ __launch_bounds__(256) void moe_linear_any_kernel(const ExpertLinearA
 // A share's pairs go by row tiles, in fours: workgroups of a four with the same weight tile follow one another, and where shares are
 // whole row tiles, as with few experts, none of them is read by two XCDs.  Large tiles with few rows come behind all others (see kApartRows), shared evenly too: the chip's last round is made of
 // short ones.  600 rows, top 6 of 64 with uneven routing, width 2048: 132 + 71 -> 101 + 62 us.
-// at: a place among an XCD's (row tile, weight tile) pairs, which begin with pair `low` of all and end before `high`
-__device__ __forceinline__ void pair_at(int n, int low, int high, int place, int& tile, int& n_tile) {
-  constexpr int kTogether = 4;
-  // the last weight tiles of a row tile that the XCD before began, row tiles of its own, the first weight tiles of one more
-  const int first_own = (low + n - 1) / n, begun = first_own * n - low, own = high / n - first_own, at = place - begun;
-  if (at < 0) {
-    tile = first_own - 1;
-    n_tile = n + at;
-  } else if (at < own * n) {
-    const int first = at / (kTogether * n) * kTogether, in = at - first * n, together = min(kTogether, own - first);
-    tile = first_own + first + in % together;
-    n_tile = in / together;
-  } else {
-    tile = first_own + own;
-    n_tile = at - own * n;
-  }
-}
-__device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, int& n_tile) {
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, n = a.n_tiles;
+__device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int block, int& tile, int& n_tile) {
+  const int xcd = block & 7, j = block >> 3, n = a.n_tiles;
   const int whole = a.num_tiles[0], rest = a.num_tiles[1], per = (whole * n + 7) / 8;
   if (j >= per) {
     const int rest_per = (rest * n + 7) / 8, at = xcd * rest_per + j - per;
@@ -479,8 +482,8 @@ __device__ __forceinline__ bool find_tile(const ExpertLinearArgs& a, int& tile, 
 // everybody.  Four groups of experts start a quarter of K apart and the weight tiles of an expert a step apart: x stays shared, and the
 // order of a sum depends on expert and column alone.  us from the first step on and so: 300 rows, top 6 of 64 experts of 1536 x 2048 84 / 68, 600
 // rows 115 / 94, 8192 rows 354 / 336; of 2560 x 4096, 8192 rows 1390 / 1345, 32 rows 211 / 209.  Other rows (K of 768 and 1280): no difference.
-__device__ __forceinline__ int first_step(const ExpertLinearArgs& a, int e, int n_tile, int steps) {
-  return a.K % 2048 == 0 ? ((e & 3) * (steps >> 2) + n_tile) % steps : 0;
+__device__ __forceinline__ int first_step(int K, int e, int n_tile, int steps) {
+  return K % 2048 == 0 ? ((e & 3) * (steps >> 2) + n_tile) % steps : 0;
 }
 
 // many: 128 weight rows x 32 kRows sorted rows per workgroup, four waves on v_mfma_f32_32x32x16_bf16.  Weights are the row
@@ -500,28 +503,44 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
   __shared__ __attribute__((aligned(16))) char lds[kStages * kStage];     // [buffer][weights, x]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
   // ---- which tile ----
-  int tile, n_tile;
-  if (!find_tile(a, tile, n_tile)) return;
-  const int e = a.tile_expert[tile], row0 = a.tile_row[tile], row_end = min(row0 + 32 * kRows, a.row_start[e + 1]);
-  const int n0 = n_tile * kTile;
+  int n_tile, e, row0, row_end;
+  const bool shared = kGlu != kClampedGlu && (int)blockIdx.x < a.shared.blocks;
+  if (shared) {                                     // an XCD has all row tiles of some weight tiles: they are read once
+    const int at = (int)(blockIdx.x & 7) * (a.shared.blocks >> 3) + (int)(blockIdx.x >> 3);
+    n_tile = at / a.shared.row_tiles;
+    if (n_tile >= a.shared.n_tiles) return;
+    e = 0;
+    row0 = at % a.shared.row_tiles * (32 * kRows);
+    row_end = min(row0 + 32 * kRows, a.shared.rows);
+  } else {
+    int tile;
+    if (!find_tile(a, (int)blockIdx.x - a.shared.blocks, tile, n_tile)) return;
+    e = a.tile_expert[tile];
+    row0 = a.tile_row[tile];
+    row_end = min(row0 + 32 * kRows, a.row_start[e + 1]);
+  }
+  const int n0 = n_tile * kTile, N = shared ? a.shared.N : a.N, K = shared ? a.shared.K : a.K;
 
   // ---- copies: chunks of either operand per thread and step ----
-  const v4i w_rows = make_rsrc(reinterpret_cast<const char*>(a.w) + (int64_t)e * a.N * a.K * 2, (uint32_t)((int64_t)a.N * a.K * 2));
-  const v4i x_rows = make_rsrc(reinterpret_cast<const char*>(a.x), a.x_bytes);
+  const v4i w_rows = make_rsrc(shared ? reinterpret_cast<const char*>(a.shared.w) : reinterpret_cast<const char*>(a.w) + (int64_t)e * N * K * 2,
+                               (uint32_t)((int64_t)N * K * 2));
+  const v4i x_rows = make_rsrc(shared ? reinterpret_cast<const char*>(a.shared.x) : reinterpret_cast<const char*>(a.x), shared ? a.shared.x_bytes : a.x_bytes);
+  const uint32_t x_stride = shared ? (uint32_t)a.shared.x_stride : (uint32_t)a.x_stride;
   uint32_t from_w[4], from_x[kRows];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int c = 256 * i + tid, r = c >> 3, p = (c & 7) ^ ((r >> 1) & 7);
-    from_w[i] = (uint32_t)(min(n0 + r, a.N - 1) * a.K + 8 * p) * 2u;
+    const int row = min(n0 + r, N - 1);
+    from_w[i] = (uint32_t)((shared ? shared_row<kGlu>(a, row) : row) * K + 8 * p) * 2u;
   }
 #pragma unroll
   for (int i = 0; i < kRows; ++i) {
     const int c = 256 * i + tid, r = c >> 3, p = (c & 7) ^ ((r >> 1) & 7);
     const int at = min(row0 + r, row_end - 1);
-    const uint32_t xr = (uint32_t)(a.per_token ? a.sorted_pair[at] / a.per_token : at);
-    from_x[i] = (xr * (uint32_t)a.x_stride + 8u * p) * 2u;
+    const uint32_t xr = (uint32_t)(a.per_token && !shared ? a.sorted_pair[at] / a.per_token : at);
+    from_x[i] = (xr * x_stride + 8u * p) * 2u;
   }
-  const int steps = a.K / kK, turn = first_step(a, e, n_tile, steps);
+  const int steps = K / kK, turn = first_step(K, e, n_tile, steps);
   const uint32_t lds_wave = lds_address(lds) + 1024 * wave;
   auto copy = [&](int step, int buffer) __attribute__((always_inline)) {      // past the last step nothing is read, and the count stays
     v4i w = w_rows, x = x_rows;
@@ -570,11 +589,13 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
   }
   if (kStages > 2) dma_wait_all();                  // (copies past the last step)
   // ---- lane: row l32 of a block, weight rows 8 (r / 4) + 4 hi + r % 4 ----
+  bf16_t* const out_of = shared ? a.shared.out : reinterpret_cast<bf16_t*>(a.out);
+  const int64_t out_stride = shared ? a.shared.out_stride : a.out_stride;
 #pragma unroll
   for (int m = 0; m < kM; ++m) {
     const int row = row0 + (wm * kM + m) * 32 + l32;
     if (row >= row_end) continue;
-    bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (int64_t)row * a.out_stride;
+    bf16_t* out = out_of + (int64_t)row * out_stride;
 #pragma unroll
     for (int r = 0; r < 16; r += 4) {
       if constexpr (kGlu) {
@@ -582,12 +603,12 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
         float o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = glu_of<kGlu>(a, acc[0][m][r + i], acc[1][m][r + i]);
-        if (2 * col < a.N) *reinterpret_cast<uint2*>(out + col) = make_uint2(pack2<bf16_t>(o[0], o[1]), pack2<bf16_t>(o[2], o[3]));
+        if (2 * col < N) *reinterpret_cast<uint2*>(out + col) = make_uint2(pack2<bf16_t>(o[0], o[1]), pack2<bf16_t>(o[2], o[3]));
       } else {
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
           const int col = n0 + wn * 64 + 32 * n + 2 * r + 4 * hi;
-          if (col < a.N)
+          if (col < N)
             *reinterpret_cast<uint2*>(out + col) = make_uint2(pack2<bf16_t>(acc[n][m][r], acc[n][m][r + 1]),
                                                               pack2<bf16_t>(acc[n][m][r + 2], acc[n][m][r + 3]));
         }
@@ -614,72 +635,71 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
 // Halves: tiles of the last round in halves gain a quarter of a tile (64 experts of 1536 x 2048 with the gate, 132 rows each 113 / 104 without / with), but where
 // tiles of few rows were to fill that round they come one round later: 156 rows 116 / 126, 180 120 / 131.
 // (Halves that have no rows, of tiles of at most 128, are run all the same: without them 108 sizes took 0.98 to 1.07 of the time, 1.008 on average.)
-constexpr int kLargeGroups = 32;                    // workgroups per XCD that go on to another tile: its CUs
 template <int kGlu>
 __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLinearArgs a) {
   constexpr int kTile = 256, kK = 64, kStage = kTile * kK * 2;       // bytes of one operand's step
   __shared__ __attribute__((aligned(16))) char lds[5 * kStage];      // weights three times, x twice
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
-  // ---- this workgroup's tiles: every a.groups-th of its XCD's.  Where they leave a last round of no more than half the workgroups, its tiles are
-  // taken in halves of 128 rows, unless these push the tiles of few rows, which come behind them, into one round more ----
-  const int n_tiles = a.n_tiles, whole = a.num_tiles[0], rest = a.num_tiles[1], xcd = blockIdx.x & 7;
-  const int per = (whole * n_tiles + 7) / 8, rest_per = (rest * n_tiles + 7) / 8;
-  const int low = min(xcd * per, whole * n_tiles), high = min(low + per, whole * n_tiles);
-  const int rest_low = min(xcd * rest_per, rest * n_tiles), rest_high = min(rest_low + rest_per, rest * n_tiles);
-  const int last = (high - low) % kLargeGroups, behind = last + rest_high - rest_low;
-  const int halved = 2 * last <= kLargeGroups && (behind + last - 1) / kLargeGroups == (behind - 1) / kLargeGroups ? last : 0, full = high - low - halved;
-  const int places = full + 2 * halved + rest_high - rest_low;
-  struct Tile { int e, row0, rows, n_tile; };
+  // ---- this workgroup's tiles: every a.groups-th of its XCD's ----
+  const LargeShare share(a.n_tiles, a.num_tiles[0], a.num_tiles[1], kGlu == kClampedGlu ? 0 : a.shared.row_tiles, a.shared.n_tiles, a.shared.units,
+                         blockIdx.x & 7, a.groups);
+  struct Tile { int e, row0, rows, n_tile; };           // (e: a.experts for the shared one)
   auto find = [&](int j, Tile& t) __attribute__((always_inline)) {
-    int tile, half = 0;
-    if (j < full + 2 * halved) {
-      const int over = j - full;
-      if (over >= 0) half = over & 1;
-      pair_at(n_tiles, low, high, over < 0 ? j : full + (over >> 1), tile, t.n_tile);
-      t.rows = over < 0 ? kTile : kTile / 2;
+    TilePlace place;
+    if (!share.find(j, place)) return false;
+    t.n_tile = place.n_tile;
+    t.rows = place.half < 0 ? kTile : kTile / 2;
+    if (place.shared) {
+      t.e = a.experts;
+      t.row0 = place.tile * kTile;
     } else {
-      const int at = rest_low + j - full - 2 * halved;
-      tile = whole + at / n_tiles;
-      t.n_tile = at % n_tiles;
-      t.rows = kTile;
+      t.e = a.tile_expert[place.tile];
+      t.row0 = a.tile_row[place.tile] + (place.half > 0 ? kTile / 2 : 0);
     }
-    t.e = a.tile_expert[tile];
-    t.row0 = a.tile_row[tile] + half * (kTile / 2);
+    return true;
   };
+  auto is_shared = [&](const Tile& t) __attribute__((always_inline)) { return kGlu != kClampedGlu && t.e == a.experts; };
+  auto after_it = [&](const Tile& t) __attribute__((always_inline)) { return a.groups * (is_shared(t) ? a.shared.units : 1); };
+  auto end_of = [&](const Tile& t) __attribute__((always_inline)) { return min(t.row0 + t.rows, is_shared(t) ? a.shared.rows : a.row_start[t.e + 1]); };
   int j = blockIdx.x >> 3;
   Tile now{}, next{};
-  if (j >= places) return;
-  find(j, now);
-  j += a.groups;
-  if (j < places) find(j, next);
+  if (!find(j, now)) return;
+  j += after_it(now);
+  bool more = find(j, next);
 
-  const v4i x_rows = make_rsrc(reinterpret_cast<const char*>(a.x), a.x_bytes);
-  const int total = a.row_start[a.experts], steps = a.K / kK;
+  const int total = a.row_start[a.experts];
   // the rows of x that this thread copies: those of the sorted rows row0 + (256 i + tid) / 8.  Past the tile's end they are the next
   // expert's, whose results are not stored.
   auto pairs_of = [&](const Tile& t, uint32_t (&pair)[8]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int at = min(t.row0 + ((256 * i + tid) >> 3), total - 1);
-      pair[i] = (uint32_t)(a.per_token ? a.sorted_pair[at] : at);
+      const int at = min(t.row0 + ((256 * i + tid) >> 3), (is_shared(t) ? a.shared.rows : total) - 1);
+      pair[i] = (uint32_t)(a.per_token && !is_shared(t) ? a.sorted_pair[at] : at);
     }
   };
   uint32_t from_w[8], from_x[8], pair[8];
-  v4i w_rows;
-  int turn;
+  v4i w_rows, x_rows;
+  int steps, turn;
   auto places_of = [&](const Tile& t) __attribute__((always_inline)) {
-    w_rows = make_rsrc(reinterpret_cast<const char*>(a.w) + (int64_t)t.e * a.N * a.K * 2, (uint32_t)((int64_t)a.N * a.K * 2));
-    turn = first_step(a, t.e, t.n_tile, steps);
+    const bool shared = is_shared(t);
+    const int N = shared ? a.shared.N : a.N, K = shared ? a.shared.K : a.K;
+    w_rows = make_rsrc(shared ? reinterpret_cast<const char*>(a.shared.w) : reinterpret_cast<const char*>(a.w) + (int64_t)t.e * N * K * 2,
+                       (uint32_t)((int64_t)N * K * 2));
+    x_rows = make_rsrc(shared ? reinterpret_cast<const char*>(a.shared.x) : reinterpret_cast<const char*>(a.x), shared ? a.shared.x_bytes : a.x_bytes);
+    const uint32_t x_stride = shared ? (uint32_t)a.shared.x_stride : (uint32_t)a.x_stride;
+    steps = K / kK;
+    turn = first_step(K, t.e, t.n_tile, steps);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int c = 256 * i + tid, r = c >> 3, p = (c & 7) ^ ((r >> 1) & 7);
-      from_w[i] = (uint32_t)(min(t.n_tile * kTile + r, a.N - 1) * a.K + 8 * p) * 2u;
+      const int w_row = min(t.n_tile * kTile + r, N - 1);
+      from_w[i] = (uint32_t)((shared ? shared_row<kGlu>(a, w_row) : w_row) * K + 8 * p) * 2u;
       uint32_t row = pair[i];
-      if (a.per_token) {                            // pair / per_token: the quotient of the rounded factor is that or one less
+      if (a.per_token && !shared) {                            // pair / per_token: the quotient of the rounded factor is that or one less
         row = __umulhi(pair[i], a.token_factor);
         row += pair[i] - row * (uint32_t)a.per_token >= (uint32_t)a.per_token;
       }
-      from_x[i] = (row * (uint32_t)a.x_stride + 8u * p) * 2u;
+      from_x[i] = (row * x_stride + 8u * p) * 2u;
     }
   };
   constexpr int kX = 3 * kStage;                    // where x begins
@@ -786,17 +806,17 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
   pairs_of(now, pair);
   places_of(now);
   // (a second half without rows is one block whose results are not stored)
-  int row_end = min(now.row0 + now.rows, a.row_start[now.e + 1]), blocks = max((row_end - now.row0 + 63) / 64, 1);
+  int row_end = end_of(now), blocks = max((row_end - now.row0 + 63) / 64, 1);
   copy_first(blocks);
   for (;;) {
-    const bool more = j < places;
     int next_end = 0;
     Tile after{};
+    bool and_more = false;
     if (more) {                                     // what the boundary behind this tile needs, here already
       pairs_of(next, pair);
-      next_end = min(next.row0 + next.rows, a.row_start[next.e + 1]);
-      j += a.groups;
-      if (j < places) find(j, after);
+      next_end = end_of(next);
+      j += after_it(next);
+      and_more = find(j, after);
     }
 #pragma unroll
     for (int n = 0; n < 4; ++n)
@@ -828,7 +848,10 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
     auto place_of = [&](int row, int chunk) __attribute__((always_inline)) {
       return row * (16 * kChunks) + ((chunk ^ ((kGlu ? row >> 1 : row) & (kChunks - 1))) << 4);
     };
-    const int out_cols = kGlu ? a.N / 2 : a.N, col0 = (of.n_tile * kTile + wn * 128) / (kGlu ? 2 : 1);
+    const bool of_shared = is_shared(of);
+    bf16_t* const out_of = of_shared ? a.shared.out : reinterpret_cast<bf16_t*>(a.out);
+    const int64_t out_stride = of_shared ? a.shared.out_stride : a.out_stride;
+    const int of_N = of_shared ? a.shared.N : a.N, out_cols = kGlu ? of_N / 2 : of_N, col0 = (of.n_tile * kTile + wn * 128) / (kGlu ? 2 : 1);
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       if (of.row0 + 32 * (wm + 2 * m) >= end) break;
@@ -855,15 +878,16 @@ __global__ __launch_bounds__(256, 1) void moe_linear_large_kernel(const ExpertLi
       __builtin_amdgcn_wave_barrier();
       const int chunk = lane % kChunks, col = col0 + 8 * chunk;
       const int row = of.row0 + 32 * (wm + 2 * m) + lane / kChunks;
-      bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (int64_t)row * a.out_stride + col;
+      bf16_t* out = out_of + (int64_t)row * out_stride + col;
 #pragma unroll
       for (int i = 0; i < 32 / kRowsPer; ++i) {
         const uint4 v = *reinterpret_cast<const uint4*>(own + place_of(kRowsPer * i + lane / kChunks, chunk));
-        if (row + kRowsPer * i < end && col < out_cols) *reinterpret_cast<uint4*>(out + (int64_t)(kRowsPer * i) * a.out_stride) = v;
+        if (row + kRowsPer * i < end && col < out_cols) *reinterpret_cast<uint4*>(out + (int64_t)(kRowsPer * i) * out_stride) = v;
       }
       __builtin_amdgcn_wave_barrier();
     }
     if (!more) break;
+    more = and_more;
   }
 }
 
@@ -982,12 +1006,23 @@ template <typename F> static void with_glu(int glu, F f) {
 
 static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64_t x_row_stride, const void* w,
                          const int32_t* ids, void* plan, int64_t pairs, int experts, int N, int K, int per_token,
-                         int glu, float alpha, float limit, float shift, int dtype, void* stream) {
+                         int glu, float alpha, float limit, float shift, const ExpertLinearArgs::Shared& shared, int dtype, void* stream) {
   if (dtype_size(dtype) == 0) return MVLLM_ERR_BAD_DTYPE;
   if (pairs < 0 || experts <= 0 || N <= 0 || K <= 0 || per_token < 0 || x_row_stride < K || out_row_stride < (glu ? N / 2 : N)) return MVLLM_ERR_BAD_SHAPE;
   if (dtype == MVLLM_F16 || experts > kMaxExperts || pairs > (1 << 30) || K % 64 != 0 || N % (glu ? 64 : 16) != 0 || x_row_stride % 8 != 0 ||
       out_row_stride % 4 != 0)
     return MVLLM_ERR_UNSUPPORTED;
+  const int sh_N = shared.N, sh_K = shared.K;
+  if (shared.rows != 0) {
+    if (shared.rows < 0 || sh_N <= 0 || sh_K <= 0 || shared.x_stride < sh_K || shared.out_stride < (glu ? sh_N / 2 : sh_N)) return MVLLM_ERR_BAD_SHAPE;
+    if (dtype != MVLLM_BF16 || glu == kClampedGlu || sh_K % 64 != 0 || sh_N % (glu ? 64 : 16) != 0 || shared.x_stride % 8 != 0 || shared.out_stride % 8 != 0 ||
+        pairs == 0 || !plan)
+      return MVLLM_ERR_UNSUPPORTED;
+    const int64_t bytes = ((int64_t)(shared.rows - 1) * shared.x_stride + sh_K) * 2;
+    if (bytes >= (int64_t)1 << 32 || (int64_t)sh_N * sh_K * 2 >= (int64_t)1 << 31) return MVLLM_ERR_UNSUPPORTED;
+    if (!shared.x || !shared.w || !shared.out) return MVLLM_ERR_NULL_POINTER;
+    if (!aligned16(shared.x) || !aligned16(shared.w) || !aligned16(shared.out)) return MVLLM_ERR_MISALIGNED;
+  }
   if (pairs == 0) return MVLLM_OK;
   if (!out || !x || !w || (!plan && !ids)) return MVLLM_ERR_NULL_POINTER;
   if (!aligned16(out) || !aligned16(x) || !aligned16(w)) return MVLLM_ERR_MISALIGNED;
@@ -995,6 +1030,9 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
   ExpertLinearArgs a = {};
   a.out = out; a.x = x; a.w = w; a.ids = ids; a.x_stride = x_row_stride; a.out_stride = out_row_stride; a.pairs = (int)pairs;
   a.experts = experts; a.N = N; a.K = K; a.per_token = per_token; a.alpha = alpha; a.limit = limit; a.shift = shift;
+  a.shared = shared;
+  a.shared.units = 1;
+  if (shared.rows != 0) a.shared.x_bytes = (uint32_t)(((int64_t)(shared.rows - 1) * shared.x_stride + sh_K) * 2);
   hipStream_t s = (hipStream_t)stream;
   const int outputs = glu ? N / 2 : N;
   if (!plan) {
@@ -1019,10 +1057,18 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
     const int64_t x_rows = per_token ? (pairs + per_token - 1) / per_token : pairs, x_bytes = ((x_rows - 1) * x_row_stride + K) * 2;
     if (x_bytes >= (int64_t)1 << 32 || (int64_t)N * K * 2 >= (int64_t)1 << 31) return MVLLM_ERR_UNSUPPORTED;
     a.x_bytes = (uint32_t)x_bytes;
-    const int64_t blocks = 8 * (((int64_t)a.max_tiles * a.n_tiles + 7) / 8 + 1 + a.n_tiles);
+    if (shared.rows != 0) {
+      a.shared.row_tiles = (shared.rows + rows - 1) / rows;
+      a.shared.n_tiles = rows == 256 ? (sh_N + 255) / 256 : (sh_N + 127) / 128;
+      const int64_t tiles = 8 * (((int64_t)a.shared.row_tiles * a.shared.n_tiles + 7) / 8);
+      if (tiles > 0x3fffffff) return MVLLM_ERR_BAD_SHAPE;
+      a.shared.blocks = (int)tiles;
+    }
+    const int64_t blocks = 8 * (((int64_t)a.max_tiles * a.n_tiles + 7) / 8 + 1 + a.n_tiles) + a.shared.blocks;
     if (blocks > 0x7fffffff) return MVLLM_ERR_BAD_SHAPE;
     const bool own = K >= 4096 && large_tiles(pairs, experts, N) >= 640;         // (moe_linear_large_kernel)
     a.groups = (int)(own || blocks / 8 < kLargeGroups ? blocks / 8 : kLargeGroups);
+    if (shared.rows != 0 && a.groups == kLargeGroups) a.shared.units = sh_K > K ? (sh_K + K / 2) / K : 1;
     a.token_factor = 0xffffffffu / (uint32_t)(per_token ? per_token : 1);
     with_glu(glu, [&](auto G) {
       constexpr int kGlu = decltype(G)::value;
@@ -1042,12 +1088,23 @@ extern "C" int mvllm_moe_linear(void* out, int64_t out_row_stride, const void* x
                                 const int32_t* ids, void* plan, int64_t pairs, int experts, int N, int K, int per_token,
                                 int glu, int dtype, void* stream) {
   return expert_linear(out, out_row_stride, x, x_row_stride, w, ids, plan, pairs, experts, N, K, per_token, glu ? kSiluGlu : kNoGlu,
-                       0.f, 0.f, 0.f, dtype, stream);
+                       0.f, 0.f, 0.f, ExpertLinearArgs::Shared{}, dtype, stream);
+}
+
+extern "C" int mvllm_moe_linear_shared(void* out, int64_t out_row_stride, const void* x, int64_t x_row_stride, const void* w, const int32_t* ids,
+                                       void* plan, int64_t pairs, int experts, int N, int K, int per_token, int glu, void* shared_out,
+                                       int64_t shared_out_row_stride, const void* shared_x, int64_t shared_x_row_stride, const void* shared_w,
+                                       int shared_rows, int shared_N, int shared_K, int dtype, void* stream) {
+  ExpertLinearArgs::Shared shared = {};
+  shared.out = reinterpret_cast<bf16_t*>(shared_out); shared.x = reinterpret_cast<const bf16_t*>(shared_x); shared.w = reinterpret_cast<const bf16_t*>(shared_w);
+  shared.out_stride = shared_out_row_stride; shared.x_stride = shared_x_row_stride; shared.rows = shared_rows; shared.N = shared_N; shared.K = shared_K;
+  return expert_linear(out, out_row_stride, x, x_row_stride, w, ids, plan, pairs, experts, N, K, per_token, glu ? kSiluGlu : kNoGlu,
+                       0.f, 0.f, 0.f, shared, dtype, stream);
 }
 
 extern "C" int mvllm_moe_linear_clamped(void* out, int64_t out_row_stride, const void* x, int64_t x_row_stride, const void* w,
                                         const int32_t* ids, void* plan, int64_t pairs, int experts, int N, int K,
                                         int per_token, float alpha, float limit, float shift, int dtype, void* stream) {
   return expert_linear(out, out_row_stride, x, x_row_stride, w, ids, plan, pairs, experts, N, K, per_token, kClampedGlu, alpha, limit,
-                       shift, dtype, stream);
+                       shift, ExpertLinearArgs::Shared{}, dtype, stream);
 }

@@ -9,10 +9,12 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from minivllm_amd import _C
+from minivllm_amd.layers.basic import Linear, SiluAndMul
 from minivllm_amd.layers.recurrent import gate_linear
-from minivllm_amd.models.qwen3 import Qwen3MLP
+from minivllm_amd.models.qwen3 import Qwen3MLP, _as_built
 from minivllm_amd.utils.padding import pad_to, round_up
 
 __all__ = ["ExpertOutput", "ExpertPlan", "SparseExperts", "moe_route", "moe_route_softmax", "moe_plan", "moe_linear", "interleave_gate_up"]
@@ -96,12 +98,15 @@ def moe_plan(ids: torch.Tensor, experts: int) -> ExpertPlan:
 
 
 def moe_linear(x: torch.Tensor, weight: torch.Tensor, ids: torch.Tensor, plan: ExpertPlan | None = None, per_token: int = 0,
-               glu: bool | tuple = False) -> torch.Tensor:
+               glu: bool | tuple = False, shared: tuple | None = None):
     """Row p = x[row of p] W_e^T for every (token, choice) pair of ``ids`` (T, top), e its expert; with ``glu`` silu(gate) * up, with
     ``glu`` = (alpha, limit, shift) the clamped form of ``layers.fused.gated_unit``.  Pairs with negative ids have no row.
 
     With a plan rows are in its sorted order, without in the pairs'.  ``per_token`` > 0: pair p reads row p / per_token of x,
-    0: row p of x is row p's own (an earlier product's).  weight (E, N, K), with ``glu`` as ``interleave_gate_up`` makes it."""
+    0: row p of x is row p's own (an earlier product's).  weight (E, N, K), with ``glu`` as ``interleave_gate_up`` makes it.
+
+    ``shared``: (x, weight (N, K)) of an expert that all rows go through (bf16, with a plan; with ``glu`` True all gate rows before the up rows), in the same launch;
+    the result is then a pair."""
     _C.require_cuda(x, weight, ids)
     experts, n, k = weight.shape
     pairs = ids.numel()
@@ -115,6 +120,17 @@ def moe_linear(x: torch.Tensor, weight: torch.Tensor, ids: torch.Tensor, plan: E
     head = (_ptr(out), out.shape[1], _ptr(x), x.stride(0) if x.shape[0] > 1 else k, _ptr(weight), _ptr(ids),
             _ptr(plan.data if plan is not None else None), pairs, experts, n, k, per_token)
     tail = (_C.dtype_code(x.dtype), _C.current_stream_ptr(x.device))
+    if shared is not None:
+        xs, ws = shared
+        _C.require_cuda(xs, ws)
+        if (plan is None or isinstance(glu, tuple) or xs.dim() != 2 or ws.dim() != 2 or xs.shape[1] != ws.shape[1] or xs.stride(1) != 1 or xs.dtype != x.dtype
+                or ws.dtype != x.dtype or not ws.is_contiguous()):
+            raise ValueError("the shared product takes x (T, K) with dense rows and a contiguous weight (N, K) of the experts' dtype, a plan and no clamped gate")
+        t, (m, ks) = xs.shape[0], ws.shape
+        beside = torch.empty((t, m // 2 if glu else m), dtype=x.dtype, device=x.device)
+        st = _C.load().mvllm_moe_linear_shared(*head, int(glu), _ptr(beside), beside.shape[1], _ptr(xs), xs.stride(0) if t > 1 else ks, _ptr(ws), t, m, ks, *tail)
+        _C.check(st, "moe_linear")
+        return out, beside
     if isinstance(glu, tuple):
         st = _C.load().mvllm_moe_linear_clamped(*head, *(float(c) for c in glu), *tail)
     else:
@@ -176,6 +192,19 @@ class SparseExperts(nn.Module):
             self.shared.gate_up.weight = nn.Parameter(torch.cat([gate, up]), requires_grad=False)
             self.shared.gate_down.weight = nn.Parameter(pad_to(matrix(get("shared.down")), None, self.shared_ff), requires_grad=False)
 
+    def _shared_beside(self, h) -> bool:
+        """Whether the shared expert's products may be part of the experts' launches: not where it is not as built here, somebody hooked into it, or the
+        launches do not take its sizes."""
+        m = self.shared
+        if (m is None or self.glu is not True or h.dtype != torch.bfloat16 or h.dim() != 2 or h.shape[0] == 0 or _has_any_global_hook() or not _as_built(m, Qwen3MLP)
+                or not _as_built(m.gate_up, Linear) or not _as_built(m.gate_down, Linear) or not _as_built(m.activation, SiluAndMul)):
+            return False
+        if torch.is_grad_enabled() and h.requires_grad:
+            return False
+        up, down = m.gate_up.weight, m.gate_down.weight
+        return (m.gate_up.bias is None and m.gate_down.bias is None and up.dtype == down.dtype == h.dtype and up.is_contiguous() and down.is_contiguous()
+                and up.shape[0] == 2 * down.shape[1] and up.shape[1] == h.shape[1] and down.shape[1] % 64 == 0 and down.shape[0] % 16 == 0)
+
     def forward(self, h) -> ExpertOutput:
         logits = gate_linear(h, self.router, None, self.router.shape[0], 0.0)
         if self.softmax:
@@ -186,12 +215,17 @@ class SparseExperts(nn.Module):
         plan = None
         if h.dtype != torch.bfloat16 or pairs > FEW_PAIRS:
             plan = moe_plan(ids, self.experts)
-        act = moe_linear(h, self.gate_up, ids, plan, self.top, glu=self.glu)
-        parts = moe_linear(act, self.down, ids, plan)
+        shared = None
+        if plan is not None and self._shared_beside(h):
+            act, shared = moe_linear(h, self.gate_up, ids, plan, self.top, glu=True, shared=(h, self.shared.gate_up.weight))
+            parts, shared = moe_linear(act, self.down, ids, plan, shared=(shared, self.shared.gate_down.weight))
+        else:
+            act = moe_linear(h, self.gate_up, ids, plan, self.top, glu=self.glu)
+            parts = moe_linear(act, self.down, ids, plan)
         out = ExpertOutput(parts, weights, None if plan is None else plan.place)
         if self.identity:
             out.ids, out.inputs = ids, h
         if self.shared is not None:
-            out.shared = self.shared(h)
+            out.shared = self.shared(h) if shared is None else shared
             out.gate = logits[:, self.experts] if self.shared_gate else None
         return out

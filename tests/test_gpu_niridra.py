@@ -626,6 +626,58 @@ def test_moe_linear_rounds_of_large_tiles(counts, n, k, top, glu):
     assert worst.max() < 2 ** -8, worst.max()
 
 
+@pytest.mark.parametrize("rows,top,experts,n,k,sn,sk", [
+    (3, 2, 5, 128, 128, 64, 64),                                          # tiles of 64 rows; one tile of the shared expert
+    (130, 2, 6, 80, 192, 400, 320),                                       # ... three row tiles of it, its last weight tile of 16 outputs, more steps of K
+    (257, 1, 3, 336, 128, 144, 64),                                       # tiles of 128 rows
+    (300, 4, 16, 4096, 64, 720, 192),                                     # tiles of 256 rows of a plan with both, one for each workgroup
+    (1100, 1, 2, 3072, 64, 6400, 192),                                    # tiles of 256 rows, several for a workgroup, the shared ones in place of three
+    (2100, 1, 2, 3072, 192, 10304, 384),                                 # ... in whole rounds and a part of one
+    (700, 3, 40, 4096, 4096, 272, 2048),                                  # long K: a workgroup for every tile
+])
+@pytest.mark.parametrize("glu", [False, True])
+def test_moe_linear_shared(rows, top, experts, n, k, sn, sk, glu):
+    """An expert that all rows go through beside the others, in every form of the tiles: the others' results are as without it, bit for bit, its own are the
+    product in float32 to a rounding to 16 bits (2^-9 of the value; gated ones to those of its factors)."""
+    g = torch.Generator(device=DEV).manual_seed(n + k + sn)
+    normal = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).bfloat16()
+    ids = torch.randint(0, experts, (rows, top), generator=g, device=DEV).int()
+    x, xs, w, ws = normal(rows, k), normal(rows, sk + 8)[:, :sk], normal(experts, n // 64 * 64 if glu else n, k, std=k ** -0.5), normal(sn // 64 * 64 if glu else sn, sk, std=sk ** -0.5)
+    plan = moe_plan(ids, experts)
+    out, beside = moe_linear(x, w, ids, plan, top, glu, shared=(xs, ws))
+    assert torch.equal(out, moe_linear(x, w, ids, plan, top, glu))
+    want = xs.float() @ ws.float().T
+    if glu:
+        gate, up = want.chunk(2, 1)
+        want = torch.nn.functional.silu(gate) * up
+    worst = (beside.float() - want).abs().amax(1) / want.abs().amax(1)
+    assert beside.shape == want.shape and worst.max() < 2 ** -8, worst.max()
+    for bad in (dict(plan=None), dict(glu=(1.0, 7.0, 1.0)), dict(shared=(xs.float(), ws.float())), dict(shared=(xs[:, :-1], ws))):
+        with pytest.raises((ValueError, RuntimeError)):
+            moe_linear(x, w, ids, **{**dict(plan=plan, per_token=top, glu=glu, shared=(xs, ws)), **bad})
+
+
+def test_experts_call_a_shared_expert_that_is_not_as_built():
+    """A hook on the shared expert or one of its parts is called, one that was replaced is used."""
+    m = SparseExperts(128, 128, 4, 2, 64, shared_ff=64, small_rows=64)
+    weights = dict(router=(4, 128), **{"shared.sg": (1, 128), "shared.gate": (64, 128), "shared.up": (64, 128), "shared.down": (128, 64)}, gate=(64, 128), up=(64, 128),
+                   down=(128, 64))
+    g = torch.Generator(device=DEV).manual_seed(0)
+    m.load(lambda name: torch.zeros(4, device=DEV) if name == "correction" else
+           (torch.randn(weights.get(name) or weights[name.split(".")[1]], generator=g, device=DEV) / 11).bfloat16(), lambda t: t.contiguous())
+    h, calls = torch.randn(100, 128, generator=g, device=DEV).bfloat16(), []
+    with torch.no_grad():
+        plain = m(h).shared
+        assert torch.allclose(plain.float(), m.shared(h).float(), atol=2 ** -6)
+        for part in (m.shared, m.shared.gate_up, m.shared.activation, m.shared.gate_down):
+            handle = part.register_forward_hook(lambda *a: calls.append(1))
+            assert torch.allclose(plain.float(), m(h).shared.float(), atol=2 ** -6)
+            handle.remove()
+        assert len(calls) == 4
+        m.shared = torch.nn.Identity()
+        assert m(h).shared is h
+
+
 @pytest.mark.parametrize("n,k", [(2560, 128), (2304, 64), (768, 64)])      # products on tiles of 256 rows; those of 768 outputs (192 tiles), and those whose rows are no multiple of 16 bytes, on those of 128
 @pytest.mark.parametrize("glu", [False, True])
 @pytest.mark.parametrize("more", [0, 120])
