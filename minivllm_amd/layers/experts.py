@@ -19,7 +19,11 @@ from minivllm_amd.utils.padding import pad_to, round_up
 
 __all__ = ["ExpertOutput", "ExpertPlan", "SparseExperts", "moe_route", "moe_route_softmax", "moe_plan", "moe_linear", "interleave_gate_up"]
 
-FEW_PAIRS = 16             # (token, choice) pairs up to which the products run without a plan
+FEW_PAIRS = 16             # (token, choice) pairs up to which the products run without a plan ...
+# ... where the experts are small: without one every expert has workgroups that look for its rows, with one only those that have some have any, and the shared
+# expert is part of the launches.  us of a captured pass at one row, without / with: 8 experts of 256 x 512 13.6 / 17.6, 64 of them 20.8 / 19.4; 16 of 512 x
+# 1024 25.1 / 24.5, 64 32.0 / 25.6; 64 of 768 x 2048 54.6 / 40.0; 64 of 1280 x 4096 109 / 74, two rows 159 / 110; 8 of 14336 x 4096 216 / 175, eight rows 513 / 391.
+FEW_WEIGHTS = 4 << 20      # experts x width x ff
 
 
 def _ptr(t):
@@ -213,7 +217,7 @@ class SparseExperts(nn.Module):
             ids, weights = moe_route(logits, self.correction, self.experts, self.top, self.groups, self.keep)
         pairs = ids.numel()
         plan = None
-        if h.dtype != torch.bfloat16 or pairs > FEW_PAIRS:
+        if h.dtype != torch.bfloat16 or pairs > FEW_PAIRS or self.experts * self.ff * self.inputs > FEW_WEIGHTS:
             plan = moe_plan(ids, self.experts)
         shared = None
         if plan is not None and self._shared_beside(h):

@@ -678,6 +678,21 @@ def test_experts_call_a_shared_expert_that_is_not_as_built():
         assert m(h).shared is h
 
 
+@pytest.mark.parametrize("experts,sorted_pairs", [(8, False), (9, True)])
+def test_experts_of_one_row(experts, sorted_pairs):
+    """Few rows, on either side of the line from which their pairs are sorted too: as in a batch, whose products are those over sorted pairs."""
+    m, g = SparseExperts(1024, 1024, experts, 2, 512), torch.Generator(device=DEV).manual_seed(experts)
+    shape = dict(router=(experts, 1024), correction=(experts,), gate=(512, 1024), up=(512, 1024), down=(1024, 512))
+    m.load(lambda name: torch.randn(shape.get(name) or shape[name.split(".")[1]], generator=g, device=DEV).mul_(1024 ** -0.5).bfloat16(), lambda t: t.contiguous())
+    h = torch.randn(40, 1024, generator=g, device=DEV).bfloat16()
+    batch = m(h)
+    for n in (1, 2, 8):
+        out = m(h[:n])
+        assert (out.part_row is not None) == sorted_pairs and torch.equal(out.weights, batch.weights[:n])
+        place = out.part_row.long() if sorted_pairs else torch.arange(2 * n, device=DEV)
+        assert row_rel(out.parts[place], batch.parts[batch.part_row.long()[:2 * n]].cpu()) < 1e-2
+
+
 @pytest.mark.parametrize("n,k", [(2560, 128), (2304, 64), (768, 64)])      # products on tiles of 256 rows; those of 768 outputs (192 tiles), and those whose rows are no multiple of 16 bytes, on those of 128
 @pytest.mark.parametrize("glu", [False, True])
 @pytest.mark.parametrize("more", [0, 120])
