@@ -65,6 +65,9 @@ struct DecodeArgs {
   int block_size;
   int part_tokens;
   int num_parts;          // partitions per sequence in the grid / workspace
+  int spread;             // 0: partitions have part_tokens; else how many a sequence is to have: they have what part_tokens_of says ...
+  uint32_t spread_factor; // (2^32 / spread, rounded up)
+  int least;              // ... and no less than this
   float scale_log2;       // scale * log2(e)
   int head_chunks;        // MFMA kernels: slices of up to 16 query heads per kv head (1 unless a kv head has more than 16)
   const float* sink;      // [num_heads] or null: one more exp(sink) in a head's denominator (added where it is inverted)
@@ -200,6 +203,20 @@ __device__ __forceinline__ int64_t load_ctx(const DecodeArgs& a, int b) {
   if (c > cap) c = cap;   // tokens past the table contribute nothing
   if (c < 0) c = 0;
   return c;
+}
+
+// Tokens of a sequence's partitions.  Where waves share a head and there are several partitions of 256 tokens and more (heads of 64 and 128), a sequence that is
+// shorter than its table is shared out too, into shorter ones: the host knows only the table's width, and in partitions made for 2048 tokens 300 were one
+// workgroup's per head.  Tables of up to kSplitNarrowCtx: as many partitions as give kSplitMinGroups workgroups, two per CU (20 sequences of 900 to 1200 in all
+// four of the grid's, 640: 389 / 405).  No shorter than `least`: 128 where CUs would be idle else, 512 where memory is the bound anyway (16-bit heads of 128; 30 of 500 to 2000
+// 31.0 with 512 and 33.4 with 128, 20 of 100 to 16000 72.0 / 75.9), 256 for the others, whose tokens take a wave as long.  us of a decode step of eight
+// layers, tables of 2048, before / so: 12 sequences of 200-400 296 / 272, of 900-1200 329 / 310, 16 of 300-1500 358 / 327, 28 of them 422 / 406, of 30-60
+// as before; of a call, tables as wide as the longest context: 15 of 269-640 13.0 / 11.8, 7 of 100-4000 18.4 / 16.8, 23 of 200-4175 with heads of 64 28.7 / 23.7, INT8
+// 33.5 / 29.4, 12 of 1000-8000 with heads of 64 31.5 / 28.3, 20 of 100-16000 with heads of 64 INT8 52.7 / 49.4, 12 of 1000-8000 48.7 / 49.5.
+__device__ __forceinline__ int part_tokens_of(const DecodeArgs& a, int ctx) {
+  if (a.spread == 0) return a.part_tokens;
+  const int even = (int)__umulhi((uint32_t)(ctx + a.spread - 1), a.spread_factor);      // ctx / spread rounded up, or more
+  return min(max((even + 63) & ~63, a.least), a.part_tokens);
 }
 
 __device__ __forceinline__ float safe_exp2_diff(float m_old, float m_new) {
@@ -751,7 +768,7 @@ static bool stream_keys(const DecodeArgs& a) { return a.head_chunks <= 1 && (int
 // of latency per wave and no second launch.
 // SUB: blocks of 1, 2, 4 or 8 tokens.  A 16-token tile then spans several blocks, and every lane looks up the blocks
 // of its own tokens (one for its K row, up to four for its V rows) in the block-table window.
-template <typename T, int W, int D, bool SUB = false, bool STREAM = false>
+template <typename T, int W, int D, bool SUB = false, bool STREAM = false, bool SPREAD = false>
 __device__ __forceinline__ void decode_mfma_item(const DecodeArgs& a, int b, int p, int slice, int w) {
   const int lane = threadIdx.x & 63;
   const HeadSlice hs = head_slice(a, slice);
@@ -760,32 +777,56 @@ __device__ __forceinline__ void decode_mfma_item(const DecodeArgs& a, int b, int
   const int col = lane & 15;                           // head (first product), dim group (second product)
   const int cls = lane >> 4;                           // token class: tokens 4*cls .. 4*cls+3 of a tile
   const int bs = a.block_size;
-  const int part_start = p * a.part_tokens;
-  const int first = part_start + (W == 1 ? 0 : w * kTile);      // first token of this wave's first tile
   const int32_t* table = a.block_tables + (int64_t)b * a.max_num_blocks;
 
   // The query rows and the block-table window (lane i holds entry win_base + i of this sequence) do not depend
   // on the context length.  The split kernel, which is all latency, asks for them together with it; the
   // one-wave form first drops the workgroups whose partition lies past the context (most of a ragged batch).
+  // (Where the partitions' length depends on the context's, a table of up to 128 entries is asked for as a whole; wider ones wait for the length.)
   DecodeHead<T, D> head;
+  int part_tokens = a.part_tokens, part_start = p * part_tokens;
+  int first = part_start + (W == 1 ? 0 : w * kTile);            // first token of this wave's first tile
   int bi = first / bs;               // logical block of the next tile to load
-  int off = first - bi * bs;         // token offset inside that block
   int win_base = bi;
   int win;
-  auto prologue = [&]() __attribute__((always_inline)) {
+  auto window = [&]() __attribute__((always_inline)) { win = (win_base + lane < a.max_num_blocks) ? table[win_base + lane] : -1; };
+  const bool whole = SPREAD && a.max_num_blocks <= 128;
+  int win_64 = -1;                   // ... its entries from 64 on
+  if constexpr (W > 1) {
     head.start(a, b, hs.head0, group, lane);
-    win = (win_base + lane < a.max_num_blocks) ? table[win_base + lane] : -1;
-  };
-  if constexpr (W > 1) prologue();
+    if (whole) {
+      win_base = 0;
+      win_64 = 64 + lane < a.max_num_blocks ? table[64 + lane] : -1;
+    }
+    if (whole || !SPREAD) window();
+  }
 
   const int ctx = __builtin_amdgcn_readfirstlane((int)load_ctx(a, b));
+  if constexpr (SPREAD) {
+    part_tokens = part_tokens_of(a, ctx);
+    part_start = p * part_tokens;
+    first = part_start + w * kTile;
+    bi = first / bs;
+  }
+  int off = first - bi * bs;         // token offset inside that block
   // a sequence that fits one partition (or is empty) is finished here: partition 0 writes the output row
-  const bool direct = ctx <= a.part_tokens;
+  const bool direct = ctx <= part_tokens;
   if (part_start >= ctx && !(direct && p == 0)) return;
-  const int part_end = min(ctx, part_start + a.part_tokens);
+  const int part_end = min(ctx, part_start + part_tokens);
   const int tiles_all = part_end > part_start ? (part_end - part_start + kTile - 1) / kTile : 0;
   const int ntiles = W == 1 ? tiles_all : (tiles_all > w ? (tiles_all - w + W - 1) / W : 0);   // this wave's
-  if constexpr (W == 1) prologue();
+  if constexpr (W == 1) {
+    head.start(a, b, hs.head0, group, lane);
+    window();
+  } else if (whole) {
+    if (bi >= 64) {
+      win_base = 64;
+      win = win_64;
+    }
+  } else if constexpr (SPREAD) {
+    win_base = bi;
+    window();
+  }
 
   const int64_t row = (int64_t)a.num_kv_heads * D;       // elements per token row
   const T* kc = reinterpret_cast<const T*>(a.k_cache) + (int64_t)g * D;
@@ -1058,7 +1099,7 @@ __device__ __forceinline__ uint2 load8_stream(const void* p) {
 }
 
 // W as in decode_mfma_item: 1 = the wave walks its partition, > 1 = W waves of the workgroup share it.  kRows: K in whole rows through LDS.
-template <typename T, int NCH, int W, int D, bool kRows>
+template <typename T, int NCH, int W, int D, bool kRows, bool SPREAD = false>
 __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b, int p, int slice, int w) {
   static_assert(NCH == 1, "one chunk of up to 16 heads");
   static_assert(D == 128 || D == 64, "one or two 64-dim steps");
@@ -1071,23 +1112,47 @@ __device__ __forceinline__ void decode_mfma_int8_item(const DecodeArgs& a, int b
   const int q4 = lane >> 4;            // token class: tokens 4*q4 .. 4*q4+3 of a tile
   const int col = lane & 15;           // head (first product), dim group (second product)
   const int bs = a.block_size;
-  const int part_start = p * a.part_tokens;
-  const int first = part_start + (W == 1 ? 0 : w * kTile);      // first token of this wave's first tile
   const int32_t* table = a.block_tables + (int64_t)b * a.max_num_blocks;
+  int part_tokens = a.part_tokens, part_start = p * part_tokens;
+  int first = part_start + (W == 1 ? 0 : w * kTile);            // first token of this wave's first tile
   int bi = first / bs;
-  int off = first - bi * bs;
   int win_base = bi;
   int win;
-  if constexpr (W > 1) win = (win_base + lane < a.max_num_blocks) ? table[win_base + lane] : -1;   // before the context length
+  auto window = [&]() __attribute__((always_inline)) { win = (win_base + lane < a.max_num_blocks) ? table[win_base + lane] : -1; };
+  const bool whole = SPREAD && a.max_num_blocks <= 128;                                     // as in decode_mfma_item
+  int win_64 = -1;
+  if constexpr (W > 1) {
+    if (whole) {
+      win_base = 0;
+      win_64 = 64 + lane < a.max_num_blocks ? table[64 + lane] : -1;
+    }
+    if (whole || !SPREAD) window();
+  }
 
   const int ctx = __builtin_amdgcn_readfirstlane((int)load_ctx(a, b));
+  if constexpr (SPREAD) {
+    part_tokens = part_tokens_of(a, ctx);
+    part_start = p * part_tokens;
+    first = part_start + w * kTile;
+    bi = first / bs;
+  }
+  int off = first - bi * bs;
   // a sequence that fits one partition (or is empty) is finished here: partition 0 writes the output row
-  const bool direct = ctx <= a.part_tokens;
+  const bool direct = ctx <= part_tokens;
   if (part_start >= ctx && !(direct && p == 0)) return;
-  const int part_end = min(ctx, part_start + a.part_tokens);
+  const int part_end = min(ctx, part_start + part_tokens);
   const int tiles_all = part_end > part_start ? (part_end - part_start + kTile - 1) / kTile : 0;
   const int ntiles = W == 1 ? tiles_all : (tiles_all > w ? (tiles_all - w + W - 1) / W : 0);   // this wave's
-  if constexpr (W == 1) win = (win_base + lane < a.max_num_blocks) ? table[win_base + lane] : -1;
+  if constexpr (W == 1) window();
+  else if (whole) {
+    if (bi >= 64) {
+      win_base = 64;
+      win = win_64;
+    }
+  } else if constexpr (SPREAD) {
+    win_base = bi;
+    window();
+  }
 
   // the query's and the first tile's loads set out together: a workgroup's first keys arrive while the query becomes int8 (one after the
   // other the same batch took 251 us, not 240)
@@ -1379,13 +1444,13 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512, D > 128 ? 1 : kDecodeWavesPerE
   decode_mfma_item<T, 1, D, SUB>(a, b, p, hg * (blockDim.x >> 6) + this_wave(), 0);
 }
 // Small batches: one workgroup of W waves per (partition, sequence, kv head), the waves splitting the tiles.
-template <typename T, int W, int D, bool SUB = false, bool STREAM = false>
+template <typename T, int W, int D, bool SUB = false, bool STREAM = false, bool SPREAD = false>
 __global__ __launch_bounds__(64 * W, D > 128 ? 1 : kDecodeWavesPerEu) void decode_mfma_split_kernel(const DecodeArgs a) {
   // kv head fastest: the workgroups of one (sequence, partition) start together and read the same token rows
   const int b = blockIdx.z;
   const int g = blockIdx.x;
   const int p = (int)((blockIdx.y + (unsigned)b) % (unsigned)a.num_parts);
-  decode_mfma_item<T, W, D, SUB, STREAM>(a, b, p, g, this_wave());
+  decode_mfma_item<T, W, D, SUB, STREAM, SPREAD>(a, b, p, g, this_wave());
 }
 template <typename T, int NCH, int D, bool kRows>
 __global__ __launch_bounds__(kDecodeI8Threads, kDecodeI8WavesPerEu) void decode_mfma_int8_kernel(const DecodeArgs a) {
@@ -1393,11 +1458,11 @@ __global__ __launch_bounds__(kDecodeI8Threads, kDecodeI8WavesPerEu) void decode_
   if (!decode_item<true>(a, b, p, hg)) return;
   decode_mfma_int8_item<T, NCH, 1, D, kRows>(a, b, p, hg * (blockDim.x >> 6) + this_wave(), 0);
 }
-template <typename T, int W, int D>
+template <typename T, int W, int D, bool SPREAD>
 __global__ __launch_bounds__(64 * W, kDecodeI8WavesPerEu) void decode_mfma_int8_split_kernel(const DecodeArgs a) {
   const int g = blockIdx.x, b = blockIdx.z;
   const int p = (int)((blockIdx.y + (unsigned)b) % (unsigned)a.num_parts);
-  decode_mfma_int8_item<T, 1, W, D, false>(a, b, p, g, this_wave());
+  decode_mfma_int8_item<T, 1, W, D, false, SPREAD>(a, b, p, g, this_wave());
 }
 
 // ---------------------------------------------------------------------------
@@ -1515,7 +1580,8 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(const DecodeArgs a) 
   if (h >= a.num_heads) return;
   const int D = a.head_dim;
   const int ctx = (int)load_ctx(a, b);
-  int np = (ctx + a.part_tokens - 1) / a.part_tokens;
+  const int part_tokens = part_tokens_of(a, ctx);
+  int np = (ctx + part_tokens - 1) / part_tokens;
   if (np > a.num_parts) np = a.num_parts;
   if (np <= 1) return;                               // written directly by the partition-0 workgroup
   const int64_t slot0 = ((int64_t)b * a.num_parts) * a.num_heads + h;
@@ -1556,7 +1622,9 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(const DecodeArgs a) 
 // eight partitions requested before the first is merged (the loop above waits for every partition in turn; a
 // sequence of 32768 tokens has up to 16 of them).  Same arithmetic in
 // the same order, so the result is the same bit for bit.
-template <typename T, int D>
+// kAhead: the first partials are asked for before the context's length says how many there are, where most sequences have several (the wait for the
+// length is 0.5 of the merge's 4 to 5 us; where most have none it costs as much).
+template <typename T, int D, bool kAhead>
 __global__ __launch_bounds__(256) void decode_reduce_vec_kernel(const DecodeArgs a) {
   constexpr int kLanes = D / 4;                      // lanes per head
   constexpr int kBatch = 8;                          // partitions in flight (16: no faster, the short sequences' loads double)
@@ -1564,23 +1632,28 @@ __global__ __launch_bounds__(256) void decode_reduce_vec_kernel(const DecodeArgs
   const int li = (int)threadIdx.x % kLanes;
   const int b = blockIdx.y;
   if (h >= a.num_heads) return;
-  const int ctx = (int)load_ctx(a, b);
-  int np = (ctx + a.part_tokens - 1) / a.part_tokens;
-  if (np > a.num_parts) np = a.num_parts;
-  if (np <= 1) return;                               // written directly by the partition-0 workgroup
   const int64_t slot0 = ((int64_t)b * a.num_parts) * a.num_heads + h;
   const int64_t stride = a.num_heads;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  float mx = -INFINITY, lsum = 0.f;
-  for (int p0 = 0; p0 < np; p0 += kBatch) {
-    float2 ml[kBatch];
-    float4 part[kBatch];
+  float2 ml[kBatch];
+  float4 part[kBatch];
+  auto fetch = [&](int p0, int last) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const int64_t s = slot0 + (int64_t)min(p0 + i, np - 1) * stride;     // past the last: the last again, unused
+      const int64_t s = slot0 + (int64_t)min(p0 + i, last) * stride;       // past the last: the last again, unused
       ml[i] = *reinterpret_cast<const float2*>(a.ws_ml + s * 2);
       part[i] = *reinterpret_cast<const float4*>(a.ws_acc + s * D + 4 * li);
     }
+  };
+  if constexpr (kAhead) fetch(0, a.num_parts - 1);
+  const int ctx = (int)load_ctx(a, b);
+  const int part_tokens = kAhead || a.spread != 0 ? part_tokens_of(a, ctx) : a.part_tokens;
+  int np = (ctx + part_tokens - 1) / part_tokens;
+  if (np > a.num_parts) np = a.num_parts;
+  if (np <= 1) return;                               // written directly by the partition-0 workgroup
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  float mx = -INFINITY, lsum = 0.f;
+  for (int p0 = 0; p0 < np; p0 += kBatch) {
+    if (!kAhead || p0 > 0) fetch(p0, np - 1);
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       if (p0 + i < np) {
@@ -1612,10 +1685,13 @@ static void launch_decode_reduce(const DecodeArgs& a, hipStream_t stream) {
   const auto grid = [&](int lanes) { return dim3((unsigned)((a.num_heads + 256 / lanes - 1) / (256 / lanes)), (unsigned)a.batch); };
   // the 16-byte loads and 8- or 16-byte stores need the output rows aligned (the workspace is checked to be)
   const bool vec = (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0;
-  if (vec && a.head_dim == 128) decode_reduce_vec_kernel<T, 128><<<grid(32), block, 0, stream>>>(a);
-  else if (vec && a.head_dim == 64) decode_reduce_vec_kernel<T, 64><<<grid(16), block, 0, stream>>>(a);
-  else if (vec && a.head_dim == 256) decode_reduce_vec_kernel<T, 256><<<grid(64), block, 0, stream>>>(a);
-  else if (vec && a.head_dim == 32) decode_reduce_vec_kernel<T, 32><<<grid(8), block, 0, stream>>>(a);
+  const bool ahead = vec && a.spread != 0 && (int64_t)a.max_num_blocks * a.block_size > kSplitNarrowCtx;
+  if (ahead && a.head_dim == 128) decode_reduce_vec_kernel<T, 128, true><<<grid(32), block, 0, stream>>>(a);
+  else if (ahead && a.head_dim == 64) decode_reduce_vec_kernel<T, 64, true><<<grid(16), block, 0, stream>>>(a);
+  else if (vec && a.head_dim == 128) decode_reduce_vec_kernel<T, 128, false><<<grid(32), block, 0, stream>>>(a);
+  else if (vec && a.head_dim == 64) decode_reduce_vec_kernel<T, 64, false><<<grid(16), block, 0, stream>>>(a);
+  else if (vec && a.head_dim == 256) decode_reduce_vec_kernel<T, 256, false><<<grid(64), block, 0, stream>>>(a);
+  else if (vec && a.head_dim == 32) decode_reduce_vec_kernel<T, 32, false><<<grid(8), block, 0, stream>>>(a);
   else decode_reduce_kernel<T><<<dim3((unsigned)((a.num_heads + 3) / 4), (unsigned)a.batch), block, 0, stream>>>(a);
 }
 
@@ -1669,7 +1745,9 @@ static int head_chunks_of(int num_heads, int num_kv_heads) { return (num_heads /
 
 struct DecodePlan {
   int part_tokens, num_parts, waves_per_head;
+  int spread, least;      // how many partitions a sequence is to have, and of how many tokens at least (see part_tokens_of); 0: of part_tokens
 };
+constexpr int kSpreadFinePairs = 176;
 static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, int block_size, bool fast_ok, bool int8, int head_dim, int dtype) {
   const int64_t max_ctx = (int64_t)max_num_blocks * block_size;
   const bool split = fast_ok && split_wanted(max_ctx, batch, num_kv_heads, int8);
@@ -1683,6 +1761,12 @@ static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, i
   const bool narrow_dim = head_dim < kSplitWideDim && max_ctx > kSplitOnePartCtx && pairs < kSplitMinGroups && split_one_part(max_ctx, pairs, head_dim, block_size);
   const bool many = sixteen_bit && block_size % kTile == 0 && (few || narrow_dim);
   plan.waves_per_head = !fast_ok ? 0 : !split ? 1 : many ? kSplitManyWaves : kSplitWaves;
+  const bool heavy = sixteen_bit && head_dim == 128, wide = max_ctx > kSplitNarrowCtx;
+  plan.least = wide ? (pairs <= 64 ? 256 : 512) : !heavy ? 256 : pairs > kSpreadFinePairs ? 512 : 128;
+  plan.spread = wide || plan.num_parts * pairs <= kSplitMinGroups ? plan.num_parts : (int)(kSplitMinGroups / pairs);
+  if (plan.waves_per_head != kSplitWaves || dtype == MVLLM_F32 || (head_dim != 64 && head_dim != 128) || block_size % kTile != 0 || plan.num_parts == 1 ||
+      plan.part_tokens < 256 || plan.part_tokens <= plan.least || plan.spread < 2)
+    plan.spread = 0;
   return plan;
 }
 
@@ -1713,6 +1797,14 @@ static int launch_decode(DecodeArgs a, bool int8, bool fast_ok, int waves, hipSt
     const dim3 grid((unsigned)a.num_parts, (unsigned)a.batch, groups);
     auto go = [&](auto DIM) {
       constexpr int D = decltype(DIM)::value;
+      if constexpr (IsSixteenBit<T>::value && (D == 64 || D == 128)) {
+        if (split && a.spread != 0) {
+          if (D == 128 && stream_keys(a)) decode_mfma_split_kernel<T, kSplitWaves, D, false, D == 128, true><<<split_grid, split_block, 0, stream>>>(a);
+          else decode_mfma_split_kernel<T, kSplitWaves, D, false, false, true><<<split_grid, split_block, 0, stream>>>(a);
+          launched = true;
+          return;
+        }
+      }
       if constexpr (IsSixteenBit<T>::value && D == 128) {
         if (split && stream_keys(a)) {
           if (waves == kSplitManyWaves) decode_mfma_split_kernel<T, kSplitManyWaves, D, false, true><<<split_grid, dim3(64 * kSplitManyWaves), 0, stream>>>(a);
@@ -1750,8 +1842,10 @@ static int launch_decode(DecodeArgs a, bool int8, bool fast_ok, int waves, hipSt
   if constexpr (IsSixteenBit<T>::value) {           // the INT8 kernels take 16-bit queries
     if (fast_ok && int8) {
       const dim3 grid((unsigned)a.num_parts, groups, (unsigned)a.batch);
-      if (split && a.head_dim == 64) decode_mfma_int8_split_kernel<T, kSplitWaves, 64><<<split_grid, split_block, 0, stream>>>(a);
-      else if (split) decode_mfma_int8_split_kernel<T, kSplitWaves, 128><<<split_grid, split_block, 0, stream>>>(a);
+      if (split && a.head_dim == 64 && a.spread != 0) decode_mfma_int8_split_kernel<T, kSplitWaves, 64, true><<<split_grid, split_block, 0, stream>>>(a);
+      else if (split && a.head_dim == 64) decode_mfma_int8_split_kernel<T, kSplitWaves, 64, false><<<split_grid, split_block, 0, stream>>>(a);
+      else if (split && a.spread != 0) decode_mfma_int8_split_kernel<T, kSplitWaves, 128, true><<<split_grid, split_block, 0, stream>>>(a);
+      else if (split) decode_mfma_int8_split_kernel<T, kSplitWaves, 128, false><<<split_grid, split_block, 0, stream>>>(a);
       else if (a.head_dim == 64) decode_mfma_int8_kernel<T, 1, 64, false><<<grid, block, 0, stream>>>(a);
       else if (int8_rows_pay((int64_t)a.num_parts * a.batch * slices)) decode_mfma_int8_kernel<T, 1, 128, true><<<grid, block, 0, stream>>>(a);
       else decode_mfma_int8_kernel<T, 1, 128, false><<<grid, block, 0, stream>>>(a);
@@ -1815,6 +1909,9 @@ static int decode_entry(void* out, const void* q, const void* k_cache, const voi
   const DecodePlan plan = plan_decode(batch, num_kv_heads * a.head_chunks, max_num_blocks, block_size, fast_ok, int8, head_dim, dtype);
   a.part_tokens = plan.part_tokens;
   a.num_parts = plan.num_parts;
+  a.spread = plan.spread;
+  a.spread_factor = plan.spread == 0 ? 0u : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)plan.spread - 1) / (uint64_t)plan.spread);
+  a.least = plan.least;
   a.scale_log2 = scale * kLog2e;
   a.sink = sink;
   a.ws_acc = nullptr; a.ws_ml = nullptr;

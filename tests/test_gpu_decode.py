@@ -307,6 +307,27 @@ def test_both_grid_forms_vs_oracle(dtype, hq, hkv, bs, d, form):
     assert torch.count_nonzero(got[3]) == 0
 
 
+@pytest.mark.parametrize("batch,width,d,bs,dtype", [
+    (12, 2048, 128, 16, torch.bfloat16), (12, 2048, 64, 256, torch.float16),          # as many partitions as the grid has; tables of 128 entries and of 8
+    (20, 2016, 128, 48, torch.bfloat16), (24, 2048, 128, 16, torch.float16),          # fewer than that; partitions of at least 512 tokens
+    (9, 4096, 128, 16, torch.bfloat16), (20, 8192, 64, 32, torch.bfloat16)])          # wide tables
+def test_partitions_as_long_as_the_contexts_ask_for(batch, width, d, bs, dtype):
+    """Sequences of a call whose partitions follow their own lengths: at, in front of and past every length that one partition, a multiple of 64 tokens or
+    as many partitions as there are take, up to the table's."""
+    part, parts, waves = paged_decode_plan(batch, 16, 8, d, width // bs, bs, dtype)
+    assert parts > 1 and waves == 4 and part >= 256
+    edges = [1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 383, 384, 385, 511, 512, 513, 128 * parts, 128 * parts + 1, 256 * parts, 256 * parts + 1, 700, 1030, part * parts]
+    edges = [min(n, width) for n in edges] + [width - 1, width]
+    for at in range(0, len(edges), batch):
+        ctx_list = (edges[at:at + batch] + [0, 300] * batch)[:batch]
+        q, kc, vc, tables, ctx = make_paged_case(at + d, 0, 0, 0, 16, 8, d, bs, dtype=dtype, ctx_list=ctx_list)
+        got = _run(q, kc, vc, _pad_tables(tables, width, bs), ctx, d ** -0.5, 16, 8, d, bs)
+        live = ctx > 0
+        mx, mean = error_stats(got[live], _oracle32(q[live], kc, vc, tables[live], ctx[live], d ** -0.5, 16, 8, d, bs))
+        assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (ctx_list, mx, mean)
+        assert not got[~live].any()
+
+
 @pytest.mark.parametrize("batch,first,tokens,d,dtype,plan", [
     (24, [8192, 1024, 1025, 1], 8192, 128, torch.bfloat16, (1024, 8, 4)), (9, [4160, 512, 575, 513], 4160, 64, torch.float16, (576, 8, 4)),   # finer
     (31, [2304, 576, 577], 2304, 128, torch.bfloat16, (576, 4, 4)), (31, [2288, 763, 705], 2288, 128, torch.bfloat16, (768, 3, 4)),   # from 2304 tokens on

@@ -125,6 +125,25 @@ def test_int8_both_grid_forms(hq, hkv, bs, d, form):
     assert torch.isfinite(got).all() and excess <= 2e-2 and mean <= 2e-3, (mx, excess, mean)
 
 
+@pytest.mark.parametrize("batch,width,d,bs", [(12, 2048, 128, 16), (20, 2016, 64, 48), (9, 4096, 128, 16), (20, 8192, 64, 32)])
+def test_int8_partitions_as_long_as_the_contexts_ask_for(batch, width, d, bs):
+    """As test_partitions_as_long_as_the_contexts_ask_for of the 16-bit cache."""
+    part, parts, waves = paged_decode_plan(batch, 16, 8, d, width // bs, bs, torch.bfloat16, int8_cache=True)
+    assert parts > 1 and waves == 4 and part >= 256
+    edges = [1, 63, 64, 65, 255, 256, 257, 511, 512, 513, 256 * parts, 256 * parts + 1, 700, 1030, part * parts]
+    edges = [min(n, width) for n in edges] + [width - 1, width]
+    for at in range(0, len(edges), batch):
+        ctx_list = (edges[at:at + batch] + [129, 300] * batch)[:batch]
+        q, ck, cv, sk, sv, tables, ctx = _quantised_case(at + d, 0, 0, 0, 16, 8, d, bs, ctx_list=ctx_list)
+        wide = torch.full((batch, width // bs), -1, dtype=torch.int32)
+        wide[:, :tables.shape[1]] = tables
+        got = paged_attention_decode_int8(q.to(DEV), ck, cv, sk, sv, wide.to(DEV), ctx.to(DEV), d ** -0.5, 16, 8, d, bs).cpu()
+        want = oracle.decode_int8_oracle(q.float(), ck.cpu(), cv.cpu(), sk.cpu(), sv.cpu(), tables, ctx, d ** -0.5, 16, 8, d, bs)
+        mx, mean = error_stats(got, want)
+        excess = ((got.float() - want).abs() - half_step(want, got.dtype)).max().item()
+        assert torch.isfinite(got).all() and excess <= 2e-2 and mean <= 2e-3, (ctx_list, mx, excess, mean)
+
+
 def test_config4_full_size_on_its_own_plan():
     """The INT8 workload in full: B 128, ctx U[256,16384], Hq32/Hkv8/D128, block 16, N(0,1) inputs with 1 % of
     the entries at 8 sigma, INT8 store then INT8 decode.  At this size the host picks the one-wave-per-head kernel
