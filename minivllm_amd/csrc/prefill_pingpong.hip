@@ -63,18 +63,14 @@ __device__ __forceinline__ void store16_buffer(void* base, uint32_t bytes, uint3
   __builtin_amdgcn_raw_buffer_store_b128(w, __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, 0x00020000), (int)lane_off, 0, 2);
 }
 
-// 16 bytes per lane into LDS at m0_base + 16 * lane, from rsrc + lane_off.
+// 16 bytes per lane into LDS at lds_base + LDS_IMM + 16 * lane, from rsrc + lane_off.
+template <int LDS_IMM>
 __device__ __forceinline__ void dma16(v4i rsrc, uint32_t lane_off, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(lane_off), "s"(rsrc) : "m0", "memory");
+  asm volatile("s_add_u32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(lane_off), "s"(rsrc), "n"(LDS_IMM) : "scc", "m0", "memory");
 }
 
 }  // namespace
 
-// One team's item list, walked in rank order.  Wave-uniform.
-struct PpItems {
-  int level;          // level the walk has reached (-1: past the last item)
-  unsigned base;      // rank of that level's first item
-};
 struct PpItem {
   int seq_start, seq_len, rb;   // the sequence's query rows; the item's 64-row block of them
   int first;          // windows: index of the item's first key tile
@@ -144,13 +140,12 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
 #define TCOUNT(items, tiles) do {} while (0)
 #endif
   // ---- the batch, one sequence per lane ----
-  int lo = 0, len = 0, cached = 0, kv_len = 0, k_lo = 0;
+  int lo = 0, len = 0, cached = 0, kv_len = 0;
   if (lane < a.num_seqs) {
     lo = a.cu_seqlens[lane];
     len = a.cu_seqlens[lane + 1] - lo;
     if (kBehind) {
-      k_lo = a.cu_seqlens_k[lane];
-      kv_len = a.cu_seqlens_k[lane + 1] - k_lo;
+      kv_len = a.cu_seqlens_k[lane + 1] - a.cu_seqlens_k[lane];
       cached = kv_len > len ? kv_len - len : 0;
     }
   }
@@ -194,9 +189,12 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
   const unsigned spt = (unsigned)(a.slices / a.n_teams);                                  // slices per team
   const int group = a.num_heads / a.num_kv_heads;
   const int chunks = group / HPI;
-  // The workgroup's k-th item is rank k TS + (t or, in odd rounds, TS - 1 - t) of the team's list.  Locating an item
-  // costs a hundred-odd instructions per wave, and two cursors go through the same items (the copies run ahead of the
-  // arithmetic), so every item is located once and kept in lane (k mod 16) of four registers until both have passed.
+  // The workgroup's k-th item is rank k TS + (t or, in odd rounds, TS - 1 - t) of the team's list.  Items are located 32 at a time, one
+  // per lane, and kept in lane (k mod 64) of two registers: two cursors go through them (the copies run up to three items ahead of
+  // the arithmetic).  Located one by one at each item's end, they kept the other group waiting for 1000 to 1500 clocks of the 9000 that an
+  // item's end cost beyond its tiles.  With the first item's copies under way before the others are located, in one run, us before and now:
+  // 16 prompts of 64 to 2048 tokens, 32 / 8 heads, 133.3 and 130.4; of 500 to 600 68.1 and 65.9; one of 8000, 16 / 8 heads, 220.6 and 212.8; windows of
+  // 256 over 5 prompts of 700 to 4000 57.0 and 53.8; 39 batches 1.014 times as fast, between 0.992 and 1.060.
   // Ranks are dealt in rounds of TS, forwards and backwards in turn; the serpentine leaves the team's first
   // workgroups the most tiles (the first rounds, whose costs fall fastest, weigh most), so a last round that is not
   // full always runs backwards: its items, each worth three to four tiles of fixed cost, go to the workgroups that
@@ -206,81 +204,98 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
   for (int step = 1; step < 64; step <<= 1) team_items += __shfl_xor(team_items, step, 64);
   team_items = __builtin_amdgcn_readfirstlane(team_items) * (int)spt;
   const unsigned short_round = (unsigned)team_items % TS != 0u ? (unsigned)team_items / TS : 0xffffffffu;
-  PpItems walk = {top - 1, 0u};
-  int produced = 0;
-  int kept_start = 0, kept_len = 0, kept_rb = 0, kept_heads = 0, kept_seq = 0;   // kept_rb: the level; kept_seq: paged only
-  auto produce = [&]() {
-    const unsigned round = (unsigned)produced;
+  int located = 0;                             // items located so far
+  int kept_place = 0, kept_heads = 0;          // 64 level + sequence (negative: no such item); kv head, first query head
+  auto heads_of = [&](unsigned slice) {        // of the team's slices
+    const unsigned y = (unsigned)team + (unsigned)a.n_teams * slice, kvh = div_small(y, (unsigned)chunks, a.chunks_magic);
+    return (int)((kvh << 16) | (kvh * (unsigned)group + (y - kvh * (unsigned)chunks) * (unsigned)HPI));
+  };
+  auto locate = [&]() {                        // items located .. located + 31
+    const unsigned round = (unsigned)(located + (lane & 31));
     const bool backwards = (round & 1u) != 0u || round == short_round;
     const unsigned R = round * TS + (backwards ? TS - 1u - t : t);
-    unsigned long long mask = 0ull;
-    unsigned cnt = 0;
-    if constexpr (WIN) {                       // one sequence: one item per slice and level, so the item's level follows
-      if (a.num_seqs == 1 && walk.level >= 0) {
-        const unsigned levels = div_small(R - walk.base, spt, a.spt_magic);
-        walk.base += levels * spt;
-        walk.level -= (int)levels * kTPB;
-        if (walk.level < __builtin_amdgcn_readfirstlane(lvl0)) walk.level = -1;
+    int level = -1, owner = 0;
+    unsigned idx = 0;                          // the item's place inside its level: sequence-major, the team's slices of one sequence side by side
+    unsigned qth = 0;
+    // (the levels again from the lengths, not kept in registers between the calls)
+    int rows = len;
+    asm volatile("" : "+v"(rows));
+    const int lvl0 = kBehind ? (cached + kRPI - 1) >> 6 : (kRPI - 1) >> 6;
+    const int lvl_end = rows > 0 ? lvl0 + kTPB * ((rows + kRPI - 1) / kRPI - 1) + 1 : 0;
+    if (a.num_seqs == 1) {                     // (as for the first item)
+      const unsigned levels = R / spt;
+      const int lowest = __builtin_amdgcn_readfirstlane(lvl0);
+      idx = R - levels * spt;
+      level = top - 1 - (int)levels * kTPB;
+      if (level < lowest) level = -1;
+    } else {
+      const unsigned beyond = (unsigned)(located + 32) * TS;       // past the last of these ranks
+      unsigned base = 0;                       // rank of the level's first item
+      for (int at = top - 1; at >= 0 && base < beyond; --at) {
+        const unsigned items = (unsigned)__popcll(__ballot(at < lvl_end && at >= lvl0 && (kTPB == 1 || ((at - lvl0) & (kTPB - 1)) == 0))) * spt;
+        const bool here = R - base < items;    // (R < base: the difference is past any count)
+        level = here ? at : level;
+        idx = here ? R - base : idx;
+        base += items;
+      }
+      qth = div_small(idx, spt, a.spt_magic);
+      unsigned before = 0;                     // sequences of the level in front of s
+      for (int s = 0; s < a.num_seqs; ++s) {
+        const int from = __builtin_amdgcn_readlane(lvl0, s), to = __builtin_amdgcn_readlane(lvl_end, s);
+        const bool holds = level >= from && level < to && (kTPB == 1 || ((level - from) & (kTPB - 1)) == 0);
+        owner = holds && before == qth ? s : owner;
+        before += holds ? 1u : 0u;
       }
     }
-    while (walk.level >= 0) {
-      mask = __ballot(walk.level < lvl_end && walk.level >= lvl0 && (kTPB == 1 || ((walk.level - lvl0) & (kTPB - 1)) == 0));
-      cnt = (unsigned)__popcll(mask);
-      const unsigned items = cnt * spt;
-      if (R - walk.base < items) break;
-      walk.base += items;
-      --walk.level;
+    if (((lane ^ located) & 32) == 0) {
+      kept_place = level * 64 + owner;
+      kept_heads = heads_of(idx - qth * spt);
     }
-    int seq_start = 0, seq_len = 0, heads = 0, seq = 0;
-    if (walk.level >= 0) {
-      // inside a level: sequence-major, the team's slices of one sequence side by side
-      const unsigned idx = R - walk.base;
-      const unsigned qth = div_small(idx, spt, a.spt_magic);
-      const unsigned sl = idx - qth * spt;
-      const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-      const unsigned long long pick = __ballot(((mask >> lane) & 1ull) != 0ull && below == (int)qth);
-      const int owner = __ffsll((long long)pick) - 1;
-      seq_start = __builtin_amdgcn_readlane(lo, owner);
-      seq_len = __builtin_amdgcn_readlane(len, owner);
-      seq = owner;
-      const unsigned y = (unsigned)team + (unsigned)a.n_teams * sl;
-      const unsigned kvh = div_small(y, (unsigned)chunks, a.chunks_magic);
-      heads = (int)((kvh << 16) | (kvh * (unsigned)group + (y - kvh * (unsigned)chunks) * (unsigned)HPI));
-    }
-    const int at = produced & 15;
-    kept_start = lane == at ? seq_start : kept_start;
-    kept_len = lane == at ? seq_len : kept_len;
-    kept_rb = lane == at ? walk.level : kept_rb;     // -1: no such item
-    kept_heads = lane == at ? heads : kept_heads;
-    if (kBehind) kept_seq = lane == at ? seq : kept_seq;
-    ++produced;
+    located += 32;
   };
-  auto item_at = [&](int k) {
-    while (produced <= k) produce();
+  auto item_of = [&](int place, int heads) {
     PpItem it;
-    const int at = k & 15;
-    it.seq_start = __builtin_amdgcn_readlane(kept_start, at);
-    it.seq_len = __builtin_amdgcn_readlane(kept_len, at);
-    it.nt = __builtin_amdgcn_readlane(kept_rb, at);
-    const int heads = __builtin_amdgcn_readlane(kept_heads, at);
+    it.nt = place >> 6;
+    it.seq = place & 63;
+    it.seq_start = __builtin_amdgcn_readlane(lo, it.seq);
+    it.seq_len = __builtin_amdgcn_readlane(len, it.seq);
     it.kvh = (int)((unsigned)heads >> 16);
     it.h0 = heads & 0xffff;
     it.valid = it.nt >= 0;
-    it.seq = 0; it.cached = 0;
-    if (kBehind) {
-      it.seq = __builtin_amdgcn_readlane(kept_seq, at);
-      it.cached = __builtin_amdgcn_readlane(cached, it.seq);
-    }
+    it.cached = kBehind ? __builtin_amdgcn_readlane(cached, it.seq) : 0;
     it.rb = (it.nt - ((it.cached + kRPI - 1) >> 6)) / kTPB;
     it.first = 0;
     if constexpr (WIN) it.first = max(it.cached + kRPI * it.rb - a.win.window + 1, 0) >> 6;
     return it;
   };
+  auto item_at = [&](int k) { return item_of(__builtin_amdgcn_readlane(kept_place, k & 63), __builtin_amdgcn_readlane(kept_heads, k & 63)); };
 
-  int ci = 0;                                  // items handed to the arithmetic so far
-  PpItem cur = item_at(ci++);
+  // The first item alone, so that its copies set out; the others are located while those are on their way.
+  PpItem cur;
+  {
+    const unsigned R = short_round == 0u ? TS - 1u - t : t;
+    int level = top - 1, owner = 0;
+    unsigned idx = R, qth = 0;
+    if (a.num_seqs == 1) {                     // one item per slice and level, so the level follows
+      const unsigned levels = R / spt;
+      idx = R - levels * spt;
+      level = top - 1 - (int)levels * kTPB;
+      if (level < __builtin_amdgcn_readfirstlane(lvl0)) level = -1;
+    } else {
+      unsigned long long mask = 0ull;
+      for (; level >= 0; --level) {
+        mask = __ballot(level < lvl_end && level >= lvl0 && (kTPB == 1 || ((level - lvl0) & (kTPB - 1)) == 0));
+        const unsigned items = (unsigned)__popcll(mask) * spt;
+        if (idx < items) break;
+        idx -= items;
+      }
+      qth = div_small(idx, spt, a.spt_magic);
+      const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+      owner = max(__ffsll((long long)__ballot(((mask >> lane) & 1ull) != 0ull && below == (int)qth)) - 1, 0);
+    }
+    cur = item_of(level * 64 + owner, heads_of(idx - qth * spt));
+  }
   if (!cur.valid) return;                      // no item for this workgroup (all waves agree)
-  PpItem nxt = item_at(ci++);
   int di = 0;
   PpItem dit = cur;                            // item the copy cursor is in
   int dj = WIN ? dit.first : 0;                // ... and its tile there
@@ -339,8 +354,10 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       d_kv_len = dit.valid ? __builtin_amdgcn_readlane(kv_len, dit.seq) : 0;
     } else if constexpr (WIN) {                // (rows left: of the sequence)
       const int seq = dit.valid ? dit.seq : 0, first = kPpBN * dit.first;
-      d_off = (int64_t)(__builtin_amdgcn_readlane(k_lo, seq) + first) * kv_row_bytes + (int64_t)dit.kvh * (GRP == 0 ? a.win.k_head : a.win.v_head);
-      d_rows_left = dit.valid ? __builtin_amdgcn_readlane(kv_len, seq) - first : 0;
+      typedef const __attribute__((address_space(4))) int32_t* ConstStarts;         // (a scalar load, as for the table: once per item)
+      const int k_start = reinterpret_cast<ConstStarts>(reinterpret_cast<uintptr_t>(a.cu_seqlens_k))[__builtin_amdgcn_readfirstlane(seq)];
+      d_off = (int64_t)(k_start + first) * kv_row_bytes + (int64_t)dit.kvh * (GRP == 0 ? a.win.k_head : a.win.v_head);
+      d_rows_left = dit.valid ? dit.cached + dit.seq_len - first : 0;
     } else {
       d_off = (int64_t)dit.seq_start * kv_row_bytes + d_head_off;
       d_rows_left = dit.valid ? total_rows - dit.seq_start : 0;
@@ -367,8 +384,17 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       r = make_rsrc(copy_src + d_off, size);
     }
     const uint32_t dst = lds_copy0 + (uint32_t)(d_slot * kTileBytes);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dma16(r, src_off[i], dst + 1024u * i);
+    if constexpr (WIN) {                       // the other three from the first: registers are short here
+      int lane_c = lane;
+      asm volatile("" : "+v"(lane_c));
+      const uint32_t chunk = GRP == 0 ? (uint32_t)(((lane_c & 15) ^ (lane_c >> 4)) << 4) : 0u, row = src_off[0] - chunk;      // (V's swizzle is the same four rows on)
+      static_for<4>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        dma16<1024 * i>(r, row + (uint32_t)(4 * i * kv_row_bytes) + (GRP == 0 ? chunk ^ (uint32_t)(64 * i) : 0u), dst);
+      });
+    } else {
+      static_for<4>([&](auto I) { dma16<1024 * decltype(I)::value>(r, src_off[decltype(I)::value], dst); });
+    }
     d_slot = d_slot == kPpRing - 1 ? 0 : d_slot + 1;
   };
   auto copy_step = [&]() {
@@ -412,12 +438,14 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     int lane_q = lane;
     asm volatile("" : "+v"(lane_q));              // the eight source offsets are computed per item, not kept in registers
     const int qrow = lane_q >> 4, qchunk = lane_q & 15;
+    const uint32_t off = (uint32_t)(qrow * q_row_bytes), chunk = (uint32_t)((qchunk ^ qrow) << 4);       // row 4 i + qrow: its swizzle is 4 (i mod 4) ^ qrow
+    uint32_t from[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int rowi = 4 * i + qrow;
-      const uint32_t off = (uint32_t)(rowi * q_row_bytes + ((qchunk ^ kswz(rowi)) << 4));
-      dma16(r, off, lds_q + (uint32_t)(i * 1024));
-    }
+    for (int i = 0; i < 4; ++i) from[i] = off + (chunk ^ (uint32_t)(64 * i));
+    static_for<8>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      dma16<1024 * i>(r, from[i & 3] + (uint32_t)(4 * i * q_row_bytes), lds_q);
+    });
   };
 
   // ---- per-lane LDS offsets of the operand fragments (as in prefill_mfma_kernel) ----
@@ -525,7 +553,6 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
       }
   };
   auto write_out = [&](int seq_start, int seq_len, int rb, int h0) {
-    const char* ot = &lds.qo[wave][0];
     int lane_o = lane;
     asm volatile("" : "+v"(lane_o));
     const int orow = lane_o >> 4, ochunk = lane_o & 15;
@@ -536,12 +563,14 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     const uint32_t size = rows > 0 ? (uint32_t)(rows - 1) * (uint32_t)out_row_bytes + (uint32_t)kRowB : 0u;
     char* base = reinterpret_cast<char*>(out) + (int64_t)(seq_start + r0) * out_row_bytes + (int64_t)(h0 + wh) * (WIN ? a.win.out_head : (int64_t)kRowB);
     const uint32_t off0 = (uint32_t)(orow * out_row_bytes + 16 * ochunk);
+    const char* const row0 = &lds.qo[wave][0] + orow * kRowB;
+    const uint32_t chunk = (uint32_t)((ochunk ^ orow) << 4);       // (as in copy_q)
+    const char* from[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int row = 4 * i + orow;
-      const uint4 w = *reinterpret_cast<const uint4*>(ot + row * kRowB + ((ochunk ^ kswz(row)) << 4));
-      store16_buffer(base, size, off0 + (uint32_t)(4 * i) * (uint32_t)out_row_bytes, w);
-    }
+    for (int i = 0; i < 4; ++i) from[i] = row0 + (chunk ^ (uint32_t)(64 * i));
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      store16_buffer(base, size, off0 + (uint32_t)(4 * i * out_row_bytes), *reinterpret_cast<const uint4*>(from[i & 3] + 1024 * i));
   };
   // The barrier that ends a softmax interval publishes the copy step issued in the wave's previous softmax interval:
   // everything but the `later` vector memory instructions issued in this one (its copy step and, in an item's first
@@ -558,9 +587,19 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
   };
 
   // ---- start: the first item's Q rows and the first three copy steps ----
+  const bool inside = cur.nt - (WIN ? cur.first : 0) > 2;      // the cursor stays in the item
   copy_q(cur);
-  copy_step();
-  copy_step();
+  if (inside) {
+    copy_step_inside();
+    copy_step_inside();
+  }
+  locate();
+  int ci = 1;                                   // items handed to the arithmetic so far
+  PpItem nxt = item_at(ci++);
+  if (!inside) {
+    copy_step();
+    copy_step();
+  }
   vm_wait<0>();
   pp_barrier();
   load_q();
@@ -1009,6 +1048,7 @@ __device__ __forceinline__ void pp_run(const PrefillPpArgs& a, PpLds<D>& lds, co
     have_prev = true;
     if (!more) break;
     cur = nxt;
+    if (located < ci + 4) locate();              // (the copies' cursor is at item ci + 2 at most)
     nxt = item_at(ci++);
   }
   if (GRP == 0) pp_barrier();                   // group 1's last interval

@@ -244,6 +244,36 @@ def test_two_group_prefill_deals_every_item_once(hq, hkv, dtype, num_seqs):
     assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
 
 
+@pytest.mark.parametrize("num_seqs,window", [(64, 0), (3, 256), (1, 256)])
+def test_two_group_kernels_go_past_32_items_per_workgroup(num_seqs, window):
+    """Four heads and one kv head: every 64 rows are one item, and 8500 of them on the workgroups of 256 compute units are more than the 32 that
+    a workgroup locates at a time.  Half of the values say which sequence they belong to, so that a row without an item, or with another
+    sequence's keys, shows; the other half are random and checked in rows of the longest items, the shortest and between."""
+    from minivllm_amd.layers.window import window_prefill
+    rows, hq, d = 8500 * 64, 4, 128
+    lengths = [rows // num_seqs + (i * 37) % 64 - 32 for i in range(num_seqs)]
+    total, g = sum(lengths), torch.Generator(device=DEV).manual_seed(61)
+    q = torch.randn(total, hq, d, generator=g, device=DEV, dtype=torch.bfloat16)
+    k, v = (torch.randn(total, 1, d, generator=g, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    cu = torch.tensor([0, *lengths]).cumsum(0).to(torch.int32)
+    for s in range(num_seqs):
+        v[cu[s]:cu[s + 1], :, d // 2:] = s % 16 + 1
+    scale = 1 / math.sqrt(d)
+    if window:
+        out = torch.full_like(q, float("nan"))
+        window_prefill(out, q, k, cu.to(DEV), cu.to(DEV), scale, window, v=v)
+    else:
+        out = flash_attention_prefill(q, k, v, cu.to(DEV), scale, hq, 1, d)
+    for s in range(num_seqs):
+        a, b = int(cu[s]), int(cu[s + 1])
+        assert ((out[a:b, :, d // 2:].float() - (s % 16 + 1)).abs().amax() <= 16 * 2 ** -7).item(), s        # weights of 8 bits that sum up to 1
+        for row in (0, 63, 64, (b - a) // 2, b - a - 1):
+            first = max(row - window + 1, 0) if window else 0
+            keys, values = (t[a + first:a + row + 1, 0].double() for t in (k, v))
+            want = torch.softmax(q[a + row].double() @ keys.T * scale, -1) @ values
+            assert ((out[a + row].double() - want)[:, :d // 2].abs().max() <= MAX_ABS_16).item(), (s, row)
+
+
 def test_config2_full_size():
     """A ragged batch of 16 prompts L U[64,2048], Hq32/Hkv8/D128 bf16; store into block-256 cache; the last
     row of each prompt must agree with a paged decode of that token over the stored cache."""
