@@ -179,8 +179,11 @@ __device__ __forceinline__ bool locate_banded(const int32_t* __restrict__ cu, in
 // over ceil(DD / 16) steps and never reads them (kHalfStep below: the last step of DD = 16 n + 8), the second one
 // carries them through the output columns DD .. 32 ceil(DD / 32) - 1 of its last block, which are not stored.
 // RANGES: see PrefillArgs::range_tiles; head_dim 64 and 128, 16-bit keys and values.
-template <typename T, int HPW, bool PAGED, int D, bool I8 = false, int DD = D, bool RANGES = false>
-__global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_kernel(const PrefillArgs a) {
+// GROUPS: 2 (ranges only): eight waves; the second four walk the second half of the range's tiles, in buffers of their own.  The groups' sums meet in LDS
+// and each stores half of the dims (one group finishing all of them took 0.5 us longer).  pairs_pay in prefill_split.hip has when, and what it brings.
+template <typename T, int HPW, bool PAGED, int D, bool I8 = false, int DD = D, bool RANGES = false, int GROUPS = 1>
+__global__ __launch_bounds__(64 * kPfWaves * GROUPS, D == 256 ? 1 : 2) void prefill_mfma_kernel(const PrefillArgs a) {
+  static_assert(GROUPS == 1 || RANGES, "two groups: key ranges");
   static_assert(!I8 || PAGED, "INT8 caches are paged");
   static_assert(!RANGES || (!I8 && DD == D && D <= 128), "key ranges: plain layouts");
   static_assert(DD % 8 == 0 && DD <= D && (!I8 || DD == D), "head dims in steps of 8, INT8 only at 64 and 128");
@@ -206,7 +209,10 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   constexpr int ROWS_PER_WAVE = kBN / kPfWaves; // K/V tile rows one wave copies (4 per instruction)
   constexpr int BM = kWaveRows * ROW_TILES;     // query rows per workgroup
   struct Tiles { char k[2][kTileBytes]; char v[2][kTileBytes]; };     // double-buffered K and V tiles
-  __shared__ __attribute__((aligned(1024))) Tiles lds;
+  __shared__ __attribute__((aligned(1024))) Tiles lds_all[GROUPS];
+  Tiles& lds = lds_all[0];
+  const int pair = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * kPfWaves));       // the wave's group ...
+  const uint32_t lds_pair = (uint32_t)(pair * (int)sizeof(Tiles));                                         // ... and its buffers' place
 
   // Work item = (head slice y, query tile x), x fastest.  Workgroups are dealt to the 8 XCDs round-robin by
   // linear id; items are handed out in chunks of kXcdChunk consecutive items per XCD so that workgroups
@@ -225,7 +231,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   }
   if constexpr (!PAGED)
     if (id >= a.store.first) {
-      store_beside<64 * kPfWaves>(a.store);
+      store_beside<64 * kPfWaves * GROUPS>(a.store);
       return;
     }
   if constexpr (RANGES) {
@@ -257,7 +263,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   if (PAGED && a.q_pos != nullptr && kv_len <= 0) return;   // a key range that is empty (uniform over the workgroup)
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) - pair * kPfWaves;
   const int group = a.num_heads / a.num_kv_heads;
   const int chunks = group / HPW;                    // workgroups per kv head
   const int g = item_y / chunks;                     // kv head
@@ -270,15 +276,22 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   int j_last = min(pos0 + kWaveRows - 1, kv_len - 1) / kBN;         // last tile any row of the wave sees
   const int wg_last = min(row0 + BM, seq_len) - 1;
   int ntiles = min((cached + wg_last) / kBN, (kv_len - 1) / kBN) + 1;
-  // RANGES: this workgroup's tiles are [t0, ntiles), t0 even (tile j lies in buffer j % 2); the others belong to other workgroups
-  const int t0 = RANGES ? (int)blockIdx.y * a.range_tiles : 0;
+  // RANGES: this workgroup's tiles are [range0, ntiles), range0 even (tile j lies in buffer j % 2); the others belong to other workgroups
+  const int range0 = RANGES ? (int)blockIdx.y * a.range_tiles : 0;
+  int turns = 0;
   const bool in_ranges = RANGES && gridDim.y > 1 && ntiles > a.range_tiles;      // (one range: no partial results, whatever the bound)
   if constexpr (RANGES) {
-    if (t0 >= ntiles) return;
-    if (blockIdx.y + 1 < gridDim.y) ntiles = min(ntiles, t0 + a.range_tiles);
+    if (range0 >= ntiles) return;
+    if (blockIdx.y + 1 < gridDim.y) ntiles = min(ntiles, range0 + a.range_tiles);
+    if constexpr (GROUPS == 2) {
+      turns = (ntiles - range0 + 1) / 2;             // tiles of the first group; of the second as many or one less
+      if (pair == 0) ntiles = range0 + turns;
+    }
     n_full = min(n_full, ntiles);
     j_last = min(j_last, ntiles - 1);
   }
+  const int t0 = GROUPS == 1 ? range0 : range0 + pair * turns;       // the group's first (two groups: tile j lies in buffer (j - t0) % 2)
+  auto buffer_of = [&](int j) __attribute__((always_inline)) { return (GROUPS == 1 ? j : j - t0) & 1; };
   const int l32 = lane & 31;
   const int hi = lane >> 5;                          // 0/1: which half of the k-slots / rows
   const int qrow = r0 + l32;                         // query row of this lane
@@ -374,7 +387,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   };
   // LDS byte address of this wave's first row in buffer 0 of K; V, buffer 1 and later copies are constants away
   // (the two arrays are laid out back to back by the struct below).
-  const uint32_t lds_wave_base = lds_address(&lds.k[0][0]) + (uint32_t)(ROWS_PER_WAVE * wave * kRowB);
+  const uint32_t lds_wave_base = lds_address(&lds.k[0][0]) + lds_pair + (uint32_t)(ROWS_PER_WAVE * wave * kRowB);
   auto issue_copy = [&](const TileSrc& t, auto BUF, auto C) {               // C < kCopies: K copy C, else V copy C - kCopies
     constexpr int c = decltype(C)::value;
     constexpr bool is_k = c < kCopies;
@@ -489,14 +502,14 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   constexpr int kKOffs = kKS > 8 ? 8 : kKS, kVOffs = kTD > 4 ? 4 : kTD;
   int k_off_[kKOffs];
 #pragma unroll
-  for (int ks = 0; ks < kKOffs; ++ks) k_off_[ks] = l32 * kRowB + (((2 * ks + hi) ^ kswz(l32)) << 4);
+  for (int ks = 0; ks < kKOffs; ++ks) k_off_[ks] = (int)lds_pair + l32 * kRowB + (((2 * ks + hi) ^ kswz(l32)) << 4);
   if constexpr (kHalfStep) k_off_[kKS - 1] = l32 * kRowB + (((hi ? 0 : 2 * (kKS - 1)) ^ kswz(l32)) << 4);
   auto k_off = [&](int ks) __attribute__((always_inline)) { return k_off_[ks & 7] + (ks >> 3) * 256; };
   const int v_row = 4 * hi + (i16 >> 2);
   int v_off_[kVOffs];
 #pragma unroll
   for (int td = 0; td < kVOffs; ++td)
-    v_off_[td] = v_row * kRowB + (((4 * td + 2 * half + ((i16 & 3) >> 1)) ^ vswz(v_row)) << 4) + ((i16 & 1) << 3);
+    v_off_[td] = (int)lds_pair + v_row * kRowB + (((4 * td + 2 * half + ((i16 & 3) >> 1)) ^ vswz(v_row)) << 4) + ((i16 & 1) << 3);
   auto v_off = [&](int td) __attribute__((always_inline)) { return v_off_[td & 3] + (td >> 2) * 256; };
 
   // One K/V tile: scores, softmax, P.V.  Compile-time parameters: BUF, the buffer index (so that all LDS
@@ -717,7 +730,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   auto diag_step = [&](int j, auto NHALF) {
     dma_wait_all();
     __syncthreads();
-    tile_step(j, EitherBuffer{(uint32_t)(j & 1) * kTileBytes}, std::true_type{}, NHALF, j + 1 < ntiles);
+    tile_step(j, EitherBuffer{(uint32_t)buffer_of(j) * kTileBytes}, std::true_type{}, NHALF, j + 1 < ntiles);
   };
   int j = t0;
   if constexpr (I8) {
@@ -768,14 +781,81 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
   for (; !I8 && j < ntiles; ++j) {
     dma_wait_all();
     __syncthreads();
-    if (j + 1 < ntiles) issue_tile(j + 1, (j + 1) & 1);
+    if (j + 1 < ntiles) issue_tile(j + 1, buffer_of(j + 1));
   }
+  if (GROUPS == 2 && pair == 1 && ntiles - t0 < turns) __syncthreads();       // (as many as the first group)
 
   // ---- epilogue: normalise, transpose through LDS (the K buffers are free now), store whole rows ----
   // lane holds row l32, dims 32*td + 8*(r/4) + 4*hi + r%4  ->  wave-private [32 rows][256 B] tile with
   // 16-byte chunks xor-swizzled by row, read back as 16 B per lane so every global store is a full row.
   dma_wait_all();                                    // the zero fill issued during the last tile has landed
   __syncthreads();                                   // every wave is done reading K/V tiles
+  if constexpr (GROUPS == 2) {
+    // Each group finishes half of the dims: what it has of the other half goes through its buffers, in fp32, with its rows' maxima and sums (a sum
+    // of 0: no tile, or no key of the row's).
+    constexpr int kHalf = kTD / 2, kGive = 4 * kHalf * 64, kRoom = sizeof(Tiles) / (2 * kPfWaves);       // blocks, 16-byte pieces and bytes of a wave's
+    __shared__ float2 ml[2][64 * kPfWaves];
+    const float sum = l + __shfl_xor(l, 32, 64), top = sum == 0.f ? -INFINITY : -neg_m[0];
+    auto give = [&](auto FROM) {
+      float4* to = reinterpret_cast<float4*>(&lds_all[pair]) + wave * kGive + lane;
+#pragma unroll
+      for (int i = 0; i < 4 * kHalf; ++i) {
+        const v16f& x = o[decltype(FROM)::value + i / 4];
+        to[64 * i] = make_float4(x[4 * (i % 4)], x[4 * (i % 4) + 1], x[4 * (i % 4) + 2], x[4 * (i % 4) + 3]);
+      }
+    };
+    if (active) {
+      ml[pair][64 * wave + lane] = make_float2(top, sum);
+      if (pair == 0) give(std::integral_constant<int, kHalf>{});
+      else give(std::integral_constant<int, 0>{});
+    }
+    __syncthreads();
+    if (!active) return;
+    const float2 other = ml[1 - pair][64 * wave + lane];
+    const float both = fmaxf(top, other.x), mine = sum == 0.f ? 0.f : fast_exp2(top - both), its = other.y == 0.f ? 0.f : fast_exp2(other.x - both);
+    float lt = sum * mine + other.y * its;
+    if (!in_ranges && a.sink != nullptr) lt = add_sink(lt, both, a.sink[h]);
+    const float inv = in_ranges && !(lt > 0.f) ? 0.f : 1.f / lt, f_mine = mine * inv, f_its = its * inv;
+    const int64_t part_row = (int64_t)blockIdx.y * a.total_tokens + seq_start + r0;
+    if (in_ranges && pair == 0 && hi == 0 && qrow < seq_len) a.lse[(part_row + l32) * a.num_heads + h] = lt > 0.f ? __log2f(lt) + both : -INFINITY;
+    const float4* from = reinterpret_cast<const float4*>(&lds_all[1 - pair]) + wave * kGive + lane;
+    char* ot = reinterpret_cast<char*>(&lds_all[pair]) + sizeof(Tiles) / 2 + wave * kRoom;               // [32 rows][half of the dims], the group's own
+    auto finish = [&](auto FROM, auto ELT) {
+      using E = decltype(ELT);
+      constexpr int kRow = 32 * kHalf * (int)sizeof(E), kPieces = kRow / 16;
+      auto swz = [](int row) __attribute__((always_inline)) { return row / (256 / kRow) & (kPieces - 1); };
+#pragma unroll
+      for (int i = 0; i < 4 * kHalf; ++i) {
+        const v16f& mine_o = o[decltype(FROM)::value + i / 4];
+        const float4 x = from[64 * i];
+        const float w[4] = {mine_o[4 * (i % 4)] * f_mine + x.x * f_its, mine_o[4 * (i % 4) + 1] * f_mine + x.y * f_its,
+                            mine_o[4 * (i % 4) + 2] * f_mine + x.z * f_its, mine_o[4 * (i % 4) + 3] * f_mine + x.w * f_its};
+        if constexpr (sizeof(E) == 4)
+          *reinterpret_cast<float4*>(ot + l32 * kRow + (((2 * i + hi) ^ swz(l32)) << 4)) = make_float4(w[0], w[1], w[2], w[3]);
+        else
+          *reinterpret_cast<uint2*>(ot + l32 * kRow + ((i ^ swz(l32)) << 4) + 8 * hi) = make_uint2(pack2<T>(w[0], w[1]), pack2<T>(w[2], w[3]));
+      }
+#pragma unroll
+      for (int i = 0; i < kWaveRows * kPieces / 64; ++i) {
+        const int row = (64 * i + lane) / kPieces, c = lane % kPieces;
+        const uint4 w = *reinterpret_cast<const uint4*>(ot + row * kRow + ((c ^ swz(row)) << 4));
+        if (r0 + row < seq_len) {
+          if constexpr (sizeof(E) == 4) *reinterpret_cast<uint4*>(a.part + ((part_row + row) * a.num_heads + h) * D + pair * (D / 2) + 4 * c) = w;
+          else store16_stream(reinterpret_cast<T*>(a.out) + ((int64_t)(seq_start + r0 + row) * a.num_heads + h) * D + pair * (D / 2) + 8 * c, w);
+        }
+      }
+    };
+    using First = std::integral_constant<int, 0>;
+    using Second = std::integral_constant<int, kHalf>;
+    if (in_ranges) {
+      if (pair == 0) finish(First{}, float{});
+      else finish(Second{}, float{});
+    } else {
+      if (pair == 0) finish(First{}, T{});
+      else finish(Second{}, T{});
+    }
+    return;
+  }
   if (!active) return;
   if constexpr (RANGES) {
     if (in_ranges) {
@@ -832,7 +912,7 @@ __global__ __launch_bounds__(64 * kPfWaves, D == 256 ? 1 : 2) void prefill_mfma_
 
 // D: the LDS layout (64, 128 or 256), DD: the data's head dimension.
 template <typename T, bool PAGED, bool I8, int D, int DD, bool RANGES = false>
-static int launch_prefill_mfma_as(const PrefillArgs& a, hipStream_t stream, int ranges = 1) {
+static int launch_prefill_mfma_as(const PrefillArgs& a, hipStream_t stream, int ranges = 1, bool pairs = false) {
   const int group = a.num_heads / a.num_kv_heads;
   // query heads of a kv head per workgroup: 4 or 2 where they divide the group, else 1 (the workgroup is then four
   // row tiles of one head)
@@ -852,6 +932,14 @@ static int launch_prefill_mfma_as(const PrefillArgs& a, hipStream_t stream, int 
   dim3 grid(RANGES ? (unsigned)items : (unsigned)((items + span - 1) / span * span), (unsigned)ranges);
   if (!PAGED) add_store_groups(b.store, grid);
   const dim3 block(64 * kPfWaves);
+  if constexpr (RANGES)
+    if (pairs) {
+      const dim3 two(2 * 64 * kPfWaves);
+      if (hpw == 4) prefill_mfma_kernel<T, 4, PAGED, D, I8, DD, true, 2><<<grid, two, 0, stream>>>(b);
+      else if (hpw == 2) prefill_mfma_kernel<T, 2, PAGED, D, I8, DD, true, 2><<<grid, two, 0, stream>>>(b);
+      else prefill_mfma_kernel<T, 1, PAGED, D, I8, DD, true, 2><<<grid, two, 0, stream>>>(b);
+      return launch_status();
+    }
   if (hpw == 4) prefill_mfma_kernel<T, 4, PAGED, D, I8, DD, RANGES><<<grid, block, 0, stream>>>(b);
   else if (hpw == 2) prefill_mfma_kernel<T, 2, PAGED, D, I8, DD, RANGES><<<grid, block, 0, stream>>>(b);
   else prefill_mfma_kernel<T, 1, PAGED, D, I8, DD, RANGES><<<grid, block, 0, stream>>>(b);
@@ -872,7 +960,7 @@ int launch_prefill_paged_16bit(const PrefillArgs& a, int dtype, hipStream_t stre
 // the paged form over an INT8 cache (codes + fp32 scales), head_dim 64 or 128, bf16 / fp16 queries (prefill_varlen.hip)
 int launch_prefill_paged_int8(const PrefillArgs& a, int dtype, hipStream_t stream);
 // key ranges side by side, head_dim 64 or 128, bf16 / fp16, packed or paged (prefill_ranges.hip)
-int launch_prefill_ranges(const PrefillArgs& a, int dtype, bool paged, int ranges, hipStream_t stream);
+int launch_prefill_ranges(const PrefillArgs& a, int dtype, bool paged, int ranges, bool pairs, hipStream_t stream);
 // fp32 tensors, head_dim 128 or 64, packed or over a paged fp32 cache (prefill_f32.hip)
 int launch_prefill_f32(const PrefillArgs& a, bool paged, hipStream_t stream);
 // ... over ranges of their 32-key tiles side by side

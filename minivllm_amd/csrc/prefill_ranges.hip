@@ -7,14 +7,14 @@
 namespace mvllm {
 
 template <typename T, bool PAGED>
-static int launch(const PrefillArgs& a, int ranges, hipStream_t s) {
-  return a.head_dim == 64 ? launch_prefill_mfma_as<T, PAGED, false, 64, 64, true>(a, s, ranges)
-                          : launch_prefill_mfma_as<T, PAGED, false, 128, 128, true>(a, s, ranges);
+static int launch(const PrefillArgs& a, int ranges, bool pairs, hipStream_t s) {
+  return a.head_dim == 64 ? launch_prefill_mfma_as<T, PAGED, false, 64, 64, true>(a, s, ranges, pairs)
+                          : launch_prefill_mfma_as<T, PAGED, false, 128, 128, true>(a, s, ranges, pairs);
 }
 
-int launch_prefill_ranges(const PrefillArgs& a, int dtype, bool paged, int ranges, hipStream_t s) {
-  if (dtype == MVLLM_BF16) return paged ? launch<bf16_t, true>(a, ranges, s) : launch<bf16_t, false>(a, ranges, s);
-  return paged ? launch<f16_t, true>(a, ranges, s) : launch<f16_t, false>(a, ranges, s);
+int launch_prefill_ranges(const PrefillArgs& a, int dtype, bool paged, int ranges, bool pairs, hipStream_t s) {
+  if (dtype == MVLLM_BF16) return paged ? launch<bf16_t, true>(a, ranges, pairs, s) : launch<bf16_t, false>(a, ranges, pairs, s);
+  return paged ? launch<f16_t, true>(a, ranges, pairs, s) : launch<f16_t, false>(a, ranges, pairs, s);
 }
 
 }  // namespace mvllm

@@ -455,17 +455,59 @@ static float busiest_cu(int64_t wgs, int num_seqs, float fresh) {
 // before / now, heads of 128: 12 of 755 rows in all, 95 % cached, 32 heads, up to 50 tiles 72.2 / 54; of 572, 37 tiles 55.4 / 38.9; three of 145, 16 tiles 23.2 /
 // 17.9; furthest behind the best, nine of 12 tiles, 104 workgroups, 1.19 times as long.  From 193 workgroups on equal ones gain nothing (1500 rows behind 1500, 376
 // workgroups: 72 whole, 86 in two), and few sequences may be equal.
-static int64_t cached_range(int64_t wgs, int64_t tiles, int num_seqs, float fresh, int head_dim, float part_us) {
-  const float on_cu = 1.29f * powf((float)num_seqs, -0.4f) * (1.f - 0.29f * fresh) * (float)(wgs * tiles) / 256.f, per_tile = head_dim == 64 ? 0.58f : 0.85f;
-  auto chain = [&](float x) { return fmaxf(x, on_cu) + 0.7f * fminf(x, on_cu); };
+struct CachedBatch {
+  int64_t tiles;
+  float on_cu, per_tile, start, wgs;       // wgs: workgroups of a range that have rows, were all sequences as long as their mean, or half of their last row tiles
+};
+static CachedBatch cached_batch(int num_seqs, int64_t total_q, int64_t max_kv_len, int num_heads, int num_kv_heads, int head_dim) {
+  const int bm = rows_of_tile(num_heads / num_kv_heads);
+  const int64_t slices = (int64_t)num_heads * bm / 128, tiles = ranges_of(max_kv_len, 1), wgs = (total_q / bm + num_seqs) * slices;
+  const float fresh = fminf(1.f, (float)total_q / ((float)num_seqs * (float)max_kv_len)), of_seq = (float)total_q / (float)num_seqs / (float)bm;
+  return {tiles, 1.29f * powf((float)num_seqs, -0.4f) * (1.f - 0.29f * fresh) * (float)(wgs * tiles) / 256.f, head_dim == 64 ? 0.58f : 0.85f,
+          head_dim == 64 ? 0.8f : 2.f, fmaxf(ceilf(of_seq), of_seq + 0.5f) * (float)(num_seqs * slices)};
+}
+static float chain_us(const CachedBatch& b, int64_t x, bool pairs) {
+  const float t = (float)x;
+  return pairs ? b.start + b.per_tile * (0.85f * t + 0.3f * b.on_cu) : b.per_tile * (fmaxf(t, b.on_cu) + 0.7f * fminf(t, b.on_cu));
+}
+// Workgroups of two groups of four waves, each of which walks half of a range's tiles.  Alone on its CU a workgroup of one group takes 1.35 us per tile
+// (870 rows behind 90 %, 14 tiles of 128 dims 18.5 us): products, softmax, LDS reads and trips to memory one after the other.  With two
+// waves per SIMD they cover one another: 0.85 of the time per tile, for 0.8 (dims 64) or 2 us of a second group's start and of the sums' way through LDS.
+// A workgroup takes most of a CU's LDS, so that it pays as long as each has a CU of its own.  Cached batches: the same model, fitted to 2700
+// random ones of 7 tiles and more, 64 to 420 workgroups, caches warm: with the range that it chooses 1.047 times as fast as before on average, 2 % of them more
+// than 3 % slower.  300 others of seven kinds of heads, 1 to 24 sequences: 1.036, between 0.953 and 1.269.  us before and now: one sequence of 451 rows,
+// 141 tiles of 64 dims 42.8 / 35.4; two of 466, 73 tiles 42.0 / 36.7; three of 682, 26 tiles of 64 dims 23.8 / 20.3; one of 980, 31 tiles, 32 heads 46.9 / 42.1;
+// but two of 2752, 67 tiles 113 / 117.  Packed ones, whose row tiles differ, in 1000 batches: 13 to 16 tiles up to 256 workgroups 1.03 times as fast, 16 to 22 up to
+// 320 1.07, 22 to 32 up to 400 1.04 to 1.14, 32 to 50 up to 480 1.15 to 1.24 (3071 rows, 64 dims 41.2 / 34.4); on the line's other side 10 to 13 tiles 0.99, 13 to
+// 16 and 320 to 400 workgroups 0.92, 22 to 32 and 480 to 600 0.93.
+static bool pairs_pay(int num_seqs, int64_t total_q, int64_t max_kv_len, int num_heads, int num_kv_heads, int head_dim, bool paged, int64_t range_tiles) {
+  const CachedBatch b = cached_batch(num_seqs, total_q, max_kv_len, num_heads, num_kv_heads, head_dim);
+  const int64_t x = std::min(range_tiles, b.tiles), n = (b.tiles + x - 1) / x;
+  if (!paged) {
+    const int bm = rows_of_tile(num_heads / num_kv_heads);
+    const int64_t wgs = (total_q / bm + num_seqs) * ((int64_t)num_heads * bm / 128);
+    return x >= 13 && (n == 1 ? wgs <= std::min<int64_t>(480, 256 + 11 * (x - 13)) : wgs * n <= 256);
+  }
+  return x >= 8 && b.wgs * (float)n <= 256.f && chain_us(b, x, true) + (n > 1 ? 1.f : 0.f) < chain_us(b, x, false);
+}
+static int64_t cached_range(const CachedBatch& b, float part_us, bool whole) {       // whole: what is not in pairs is one range
+  const int64_t tiles = b.tiles;
+  const float per_range = 0.6f + 0.81f * part_us;
   int64_t p = (tiles + 1) / 2 * 2;
-  float best = 0.8f;
-  for (int64_t most = kMaxRanges; most > 1; --most) {       // the shortest range that gives so many
+  float best = 0.8f, best_pairs = 0.f;
+  for (int64_t most = kMaxRanges; most >= 1; --most) {      // the shortest range that gives so many
     const int64_t even_tiles = ((tiles + most - 1) / most + 1) / 2 * 2, x = even_tiles < 4 ? 4 : even_tiles, n = (tiles + x - 1) / x;
-    if (x >= tiles) continue;
-    const float gain = per_tile * (chain((float)tiles) - chain((float)x)) - 1.6f - (0.6f + 0.81f * part_us) * (float)n;
-    if (gain > best) {
+    if (x >= tiles && most > 1) continue;
+    const float us = n > 1 ? 1.6f + per_range * (float)n : 0.f, from = chain_us(b, tiles, false);
+    const float gain = from - chain_us(b, x, false) - us;
+    if (!whole && n > 1 && gain > best) {
       best = gain;
+      p = x;
+    }
+    if (b.wgs * (float)n > 256.f || std::min(x, tiles) < 8) continue;
+    const float gain_pairs = from - chain_us(b, std::min(x, tiles), true) - us - (n > 1 ? 1.f : 0.f);
+    if (gain_pairs > best_pairs && gain_pairs > best) {
+      best = best_pairs = gain_pairs;
       p = x;
     }
   }
@@ -543,8 +585,9 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
     if (four && crowded && !paged && fresh >= 0.87f && busiest_cu(even, num_seqs, fresh) > (num_seqs <= 3 ? 1.87f : 2.9f)) return 0;
   }
   int64_t p = (tiles + 1) / 2 * 2;
-  if (paged && (wgs <= 192 || num_seqs >= 5))
-    p = cached_range(wgs, tiles, num_seqs, fresh, head_dim, 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f);
+  if (paged)
+    p = cached_range(cached_batch(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim),
+                     8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f, wgs > 192 && num_seqs < 5);
   if (wgs > 192) return (four || head_dim == 64) && tiles > 112 ? 0 : (int)p;
   const float per_tile = head_dim == 64 ? 0.8f : 0.9f, per_range = 0.3f + 0.7f * 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f;
   float best = 3.f;
@@ -595,7 +638,7 @@ static int run_ranges(void* out, const void* q, const void* k, const void* v, co
   a.part = reinterpret_cast<float*>(workspace);
   a.lse = ranges > 1 ? a.part + (int64_t)ranges * total_q_tokens * num_heads * head_dim : nullptr;
   a.store = store;
-  const int status = launch_prefill_ranges(a, dtype, paged, ranges, s);
+  const int status = launch_prefill_ranges(a, dtype, paged, ranges, pairs_pay(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, paged, range_tiles), s);
   if (status != MVLLM_OK || ranges == 1) return status;
   RangeMergeArgs m;
   m.out = out; m.part = a.part; m.lse = a.lse; m.cu_seqlens_q = cu_seqlens_q; m.cu_seqlens_k = a.cu_seqlens_k; m.sink = sink;

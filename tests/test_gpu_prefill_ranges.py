@@ -64,6 +64,45 @@ def test_the_diagonal_at_every_place_of_a_tile(hq, hkv, d, tiles, new):
         assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (paged, mx, mean)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d,lengths,cached,tiles", [
+    (8, 2, 128, [5000, 2700, 64], [4900, 2650, 0], 40),                # two ranges, one of an odd number of tiles, one of a single tile
+    (8, 4, 64, [3400, 130, 0, 3], [3300, 70, 0, 0], 28),
+    (5, 5, 128, [3000, 1700], [2800, 1699], 24),                       # one head per workgroup
+    (2, 1, 128, [2700, 40], [2000, 10], 14),                           # packed: 14 tiles and 256 workgroups
+    (2, 1, 64, [2200, 900], [100, 0], 36),                             # whole
+])
+@pytest.mark.parametrize("paged", [True, False])
+def test_prefill_over_key_ranges_in_two_groups(hq, hkv, d, lengths, cached, tiles, paged, dtype):
+    """Few workgroups with long ranges: two groups of waves walk the halves of a range, whose sums meet in LDS."""
+    c = make_paged_prefill_case(71, lengths, cached, hq, hkv, d, 16, dtype=dtype)
+    want = oracle.prefill_paged_oracle(c["q_new"].float(), torch.nan_to_num(c["k_cache"].float()), torch.nan_to_num(c["v_cache"].float()),
+                                       c["block_tables"], c["cu_q"], c["cu_k"], 1 / math.sqrt(d), hq, hkv, d, 16)
+    got = _run(c, hq, hkv, d, 16, tiles, max(lengths), paged)
+    mx, mean = error_stats(got if paged else got[c["new_rows"]], want)
+    assert torch.isfinite(got.float()).all() and mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
+
+
+@pytest.mark.parametrize("new", [1, 31, 32, 33, 65, 100])
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 128), (4, 2, 64), (3, 3, 128)])
+def test_the_diagonal_at_every_place_of_a_tile_in_two_groups(hq, hkv, d, new):
+    """As above with a bound of 64 tiles: from a single tile, which leaves the second group without one, to five, the limit in either group's last
+    tile or before it; the sink counts once."""
+    cached = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 192]
+    c = make_paged_prefill_case(87 + new, [n + new for n in cached], cached, hq, hkv, d, 16, dtype=torch.bfloat16)
+    want = oracle.prefill_paged_oracle(c["q_new"].float(), torch.nan_to_num(c["k_cache"].float()), torch.nan_to_num(c["v_cache"].float()),
+                                       c["block_tables"], c["cu_q"], c["cu_k"], 1 / math.sqrt(d), hq, hkv, d, 16)
+    for paged in (True, False):
+        got = _run(c, hq, hkv, d, 16, 64, 4096, paged)
+        mx, mean = error_stats(got if paged else got[c["new_rows"]], want)
+        assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (paged, mx, mean)
+    sink = torch.randn(hq, generator=torch.Generator().manual_seed(1)).to(DEV)
+    got = _run(c, hq, hkv, d, 16, 64, 4096, False, sink)
+    whole = attention.flash_attention_prefill(*(c[n].to(DEV) for n in ("q", "k", "v", "cu_k")), d ** -0.5, hq, hkv, d, sink=sink).cpu()
+    mx, mean = error_stats(got, whole.float())
+    assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
+
+
 @pytest.mark.parametrize("lengths", [[0, 300, 0, 77], [200]])
 def test_prefill_over_key_ranges_sinks_and_empty_sequences(lengths):
     """Against the kernel without ranges: the sink counts once, sequences without tokens have no rows."""
