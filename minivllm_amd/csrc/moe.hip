@@ -6,10 +6,11 @@
 //   moe_plan    (token, choice) pairs sorted by expert, and tiles of 64, 128 or 256 sorted rows per expert
 //   moe_linear  out[row] = x[row] W_e^T, optionally silu(gate) * up or its clamped form behind it: W_e [2 F, K] with gate and up rows in turns of
 //               32, so that both halves of an output are in one lane
-// Products, by the number of rows: very few (no plan; a workgroup finds its expert's rows itself, its waves share K), many (bf16: tiles of 64 x 128,
+// Products, by the number of rows: very few (no plan; a workgroup finds its expert's rows itself, its waves share K), many (bf16: tiles of 32 x 64, 64 x 64, 64 x 128,
 // 128 x 128 or 256 x 256 on the matrix unit over sorted rows), any (fp32, over sorted rows).
 #include "expert_tiles.h"
 #include "prefill_tiles.h"
+#include <cmath>
 
 #pragma clang fp contract(off)
 
@@ -617,6 +618,139 @@ __global__ __launch_bounds__(256, 2) void moe_linear_many_kernel(const ExpertLin
   }
 }
 
+// many, few workgroups: 64 weight rows x 32 kBlocks sorted rows per workgroup, whose waves take a sixteen of K each of every step and add up in LDS, in 32 bits.
+// Weights are the bound as in the 64-row form above, but where that has fewer workgroups than CUs, each of them waits for its own three buffers: 16 KB
+// of weights in flight per CU.  Half as many weight rows are twice as many workgroups, and six buffers (five with 64 rows) 40 KB (32) in flight for each of
+// two per CU.  narrow_pays has when.  us of a product, 64-row form / this: 6 pairs, 64 experts of 1536 x 2048 with the gate 17.5 / 10.2 and of
+// 2048 x 768 9.2 / 7.1; 4 pairs of 2560 x 4096 31.3 / 18.0 (4.7 TB/s), 12 of 4096 x 1280 24.8 / 20.9; one of 4096 x 14336 92.9 / 43.1.
+template <int kGlu, int kBlocks>
+__global__ __launch_bounds__(256, 2) void moe_linear_narrow_kernel(const ExpertLinearArgs a) {
+  constexpr int kStages = kBlocks == 1 ? 6 : 5, kTile = 64, kRows = 32 * kBlocks, kK = 64, kW = kTile * kK * 2, kStage = kW + kRows * kK * 2, kCopies = 2 + kBlocks;
+  __shared__ __attribute__((aligned(16))) char lds[kStages * kStage];     // [buffer][weights, x]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hi = lane >> 5;
+  // ---- which tile ----
+  int n_tile, e, row0, row_end;
+  const bool shared = kGlu != kClampedGlu && (int)blockIdx.x < a.shared.blocks;
+  if (shared) {
+    const int at = (int)(blockIdx.x & 7) * (a.shared.blocks >> 3) + (int)(blockIdx.x >> 3);
+    n_tile = at / a.shared.row_tiles;
+    if (n_tile >= a.shared.n_tiles) return;
+    e = 0;
+    row0 = at % a.shared.row_tiles * kRows;
+    row_end = min(row0 + kRows, a.shared.rows);
+  } else {
+    int tile;
+    if (!find_tile(a, (int)blockIdx.x - a.shared.blocks, tile, n_tile)) return;
+    e = a.tile_expert[tile];
+    row0 = a.tile_row[tile];
+    row_end = min(row0 + kRows, a.row_start[e + 1]);
+  }
+  const int n0 = n_tile * kTile, N = shared ? a.shared.N : a.N, K = shared ? a.shared.K : a.K;
+
+  // ---- copies: two chunks of weights and kBlocks of x per thread and step ----
+  const v4i w_rows = make_rsrc(shared ? reinterpret_cast<const char*>(a.shared.w) : reinterpret_cast<const char*>(a.w) + (int64_t)e * N * K * 2,
+                               (uint32_t)((int64_t)N * K * 2));
+  const v4i x_rows = make_rsrc(shared ? reinterpret_cast<const char*>(a.shared.x) : reinterpret_cast<const char*>(a.x), shared ? a.shared.x_bytes : a.x_bytes);
+  const int r0 = tid >> 3, p0 = (tid & 7) ^ ((r0 >> 1) & 7);       // (row r0 + 32 has the same swizzle)
+  uint32_t from_w[2], from_x[kBlocks];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = min(n0 + r0 + 32 * i, N - 1);
+    from_w[i] = (uint32_t)((shared ? shared_row<kGlu>(a, row) : row) * K + 8 * p0) * 2u;
+  }
+#pragma unroll
+  for (int i = 0; i < kBlocks; ++i) {
+    const int at = min(row0 + r0 + 32 * i, row_end - 1);
+    const uint32_t xr = (uint32_t)(a.per_token && !shared ? a.sorted_pair[at] / a.per_token : at);
+    from_x[i] = (xr * (shared ? (uint32_t)a.shared.x_stride : (uint32_t)a.x_stride) + 8u * p0) * 2u;
+  }
+  const int steps = K / kK, turn = first_step(K, e, n_tile, steps);
+  const uint32_t lds_wave = lds_address(lds) + 1024 * wave;
+  auto copy = [&](int step, int buffer) __attribute__((always_inline)) {      // past the last step nothing is read, and the count stays
+    v4i w = w_rows, x = x_rows;
+    w[2] = step < steps ? w[2] : 0;
+    x[2] = step < steps ? x[2] : 0;
+    const uint32_t at = (uint32_t)(step < steps - turn ? step + turn : step + turn - steps) * (2 * kK), base = lds_wave + buffer * kStage;
+    dma16_to_lds_at<0, true>(w, from_w[0], at, base);
+    dma16_to_lds_at<4096, true>(w, from_w[1], at, base);
+    static_for<kBlocks>([&](auto I) { dma16_to_lds_at<kW + 4096 * decltype(I)::value>(x, from_x[decltype(I)::value], at, base); });
+  };
+  // this lane's fragments of the wave's sixteen: row l32 of a 32-row block, chunk 2 wave + hi
+  const char* frag = lds + l32 * 128 + (((2 * wave + hi) ^ ((l32 >> 1) & 7)) << 4);
+  v16f acc[kBlocks][2];
+#pragma unroll
+  for (int m = 0; m < kBlocks; ++m)
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+
+  static_for<kStages - 1>([&](auto I) { copy(decltype(I)::value, decltype(I)::value); });
+  int buffer = 0;
+  for (int step = 0; step < steps; ++step) {
+    dma_wait_but<kCopies * (kStages - 2)>();
+    workgroup_barrier();                            // this step's operands are there, the buffer of the step before is free
+    copy(step + kStages - 1, buffer == 0 ? kStages - 1 : buffer - 1);
+    const char* at = frag + buffer * kStage;
+    const uint4 w0 = *reinterpret_cast<const uint4*>(at), w1 = *reinterpret_cast<const uint4*>(at + 32 * 128);
+    uint4 x[kBlocks];
+#pragma unroll
+    for (int m = 0; m < kBlocks; ++m) x[m] = *reinterpret_cast<const uint4*>(at + kW + m * 32 * 128);
+#pragma unroll
+    for (int m = 0; m < kBlocks; ++m) {
+      acc[m][0] = mfma32x32x16<bf16_t>(w0, x[m], acc[m][0]);
+      acc[m][1] = mfma32x32x16<bf16_t>(w1, x[m], acc[m][1]);
+    }
+    buffer = buffer + 1 == kStages ? 0 : buffer + 1;
+  }
+  dma_wait_all();                                   // (copies past the last step)
+  __syncthreads();
+  // ---- the waves' sums: 16-byte pieces [wave][block of outputs][four of a lane][lane]; wave w finishes the w-th four of every block.  Lane: row l32,
+  // weight rows 8 w + 4 hi + 0 .. 3 ----
+  static_assert(4 * 2 * kBlocks * 4 * 64 * 16 <= kStages * kStage, "the sums' room");
+  float4* const sums = reinterpret_cast<float4*>(lds);
+#pragma unroll
+  for (int m = 0; m < kBlocks; ++m)
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        sums[(((wave * kBlocks + m) * 2 + n) * 4 + i) * 64 + lane] = make_float4(acc[m][n][4 * i], acc[m][n][4 * i + 1], acc[m][n][4 * i + 2], acc[m][n][4 * i + 3]);
+  __syncthreads();
+  bf16_t* const out_of = shared ? a.shared.out : reinterpret_cast<bf16_t*>(a.out);
+  const int64_t out_stride = shared ? a.shared.out_stride : a.out_stride;
+  const int r = 8 * wave + 4 * hi;
+#pragma unroll
+  for (int m = 0; m < kBlocks; ++m) {
+    const int row = row0 + 32 * m + l32;
+    if (row >= row_end) continue;
+    float v[2][4];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      float4 x[4];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) x[w] = sums[(((w * kBlocks + m) * 2 + n) * 4 + wave) * 64 + lane];
+      v[n][0] = (x[0].x + x[1].x) + (x[2].x + x[3].x);
+      v[n][1] = (x[0].y + x[1].y) + (x[2].y + x[3].y);
+      v[n][2] = (x[0].z + x[1].z) + (x[2].z + x[3].z);
+      v[n][3] = (x[0].w + x[1].w) + (x[2].w + x[3].w);
+    }
+    bf16_t* out = out_of + (int64_t)row * out_stride;
+    if constexpr (kGlu) {
+      float o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = glu_of<kGlu>(a, v[0][i], v[1][i]);
+      *reinterpret_cast<uint2*>(out + n0 / 2 + r) = make_uint2(pack2<bf16_t>(o[0], o[1]), pack2<bf16_t>(o[2], o[3]));
+    } else {
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const int col = n0 + 32 * n + r;
+        if (col < N) *reinterpret_cast<uint2*>(out + col) = make_uint2(pack2<bf16_t>(v[n][0], v[n][1]), pack2<bf16_t>(v[n][2], v[n][3]));
+      }
+    }
+  }
+}
+
 // many, large tiles: 256 sorted rows x 256 weight rows, four waves of 128 x 128 (a wave's accumulators fill half its SIMD's
 // registers; per flop it reads half as much of LDS as with 64 x 64).  The operands of a 16-wide step are read during the
 // products of the one before; a step's last products hide the barrier, after which the next step's operands are there and
@@ -896,6 +1030,18 @@ static int tile_rows(int64_t pairs, int experts) {
   return pairs >= kLargeTileRows * (int64_t)experts ? 256 : pairs > kSmallTileRows * (int64_t)experts ? 128 : 64;
 }
 static int64_t max_tiles(int64_t pairs, int experts, int rows) { return (pairs + rows - 1) / rows + experts; }
+// Whether a product's weights go in 64 rows per workgroup instead of 128, by the workgroups of 128 to be expected where routing is even.  Up to 160 these leave CUs
+// idle: 1.0 to 2.2 times as fast at K of 768 to 14336 (1.27 and more up to 128 workgroups).  From 160 to 248 both fill the chip about once, 0.95 to 1.10.
+// From 248 to 384 a part of the CUs has two of 128 and the others one, while all have two of 64: 1.0 to 1.19 (K 768: 1.05 up to 328, 0.93 at 396).  At 400 to 500
+// 0.91 to 1.03, and above it 0.98 to 1.1 where there are many steps of K, 0.8 to 0.95 where there are few.  K of 512 never (0.65 to 0.85): six buffers'
+// start and the sums at the end are longer than its eight steps.  More than four pairs per expert were not faster (mixtures of 64 experts: 0.98 at six, 0.88 at 28).
+static bool narrow_pays(int64_t pairs, int experts, int N, int K, const ExpertLinearArgs::Shared& shared) {
+  const int least_k = shared.rows != 0 ? std::min(K, shared.K) : K;
+  if (pairs > 4 * (int64_t)experts || least_k < 768) return false;
+  const float with_rows = (float)experts * (1.f - powf(1.f - 1.f / (float)experts, (float)pairs));
+  const float wgs = with_rows * (float)((N + 127) / 128) + (shared.rows != 0 ? (float)((shared.rows + 63) / 64) * (float)((shared.N + 127) / 128) : 0.f);
+  return wgs <= 160.f || (wgs >= 248.f && wgs <= (least_k >= 1024 ? 384.f : 328.f));
+}
 // Tiles of 256 rows and weight rows to be expected.
 static int64_t large_tiles(int64_t pairs, int experts, int N) {
   const int64_t rows = pairs / 256 + experts / 2;
@@ -1052,14 +1198,16 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
     const int rows = second ? 256 : p.tile_rows;
     a.tile_expert = p.tiles[second].expert; a.tile_row = p.tiles[second].row; a.num_tiles = p.tiles[second].num;
     a.max_tiles = (int)max_tiles(pairs, experts, rows);
-    a.n_tiles = rows == 256 ? (N + 255) / 256 : (N + 127) / 128;
+    const bool narrow = rows == 64 && narrow_pays(pairs, experts, N, K, shared), one_block = pairs <= 32 && shared.rows <= 32;      // (one: no expert has more rows)
+    const int tile = rows == 256 ? 256 : narrow ? 64 : 128;              // weight rows
+    a.n_tiles = (N + tile - 1) / tile;
     if (rows == 256 && out_row_stride % 8 != 0) return MVLLM_ERR_UNSUPPORTED;
     const int64_t x_rows = per_token ? (pairs + per_token - 1) / per_token : pairs, x_bytes = ((x_rows - 1) * x_row_stride + K) * 2;
     if (x_bytes >= (int64_t)1 << 32 || (int64_t)N * K * 2 >= (int64_t)1 << 31) return MVLLM_ERR_UNSUPPORTED;
     a.x_bytes = (uint32_t)x_bytes;
     if (shared.rows != 0) {
       a.shared.row_tiles = (shared.rows + rows - 1) / rows;
-      a.shared.n_tiles = rows == 256 ? (sh_N + 255) / 256 : (sh_N + 127) / 128;
+      a.shared.n_tiles = (sh_N + tile - 1) / tile;
       const int64_t tiles = 8 * (((int64_t)a.shared.row_tiles * a.shared.n_tiles + 7) / 8);
       if (tiles > 0x3fffffff) return MVLLM_ERR_BAD_SHAPE;
       a.shared.blocks = (int)tiles;
@@ -1074,6 +1222,8 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
       constexpr int kGlu = decltype(G)::value;
       if (rows == 256) moe_linear_large_kernel<kGlu><<<dim3(8u * (unsigned)a.groups), dim3(256), 0, s>>>(a);
       else if (rows == 128) moe_linear_many_kernel<kGlu, 4><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      else if (narrow && one_block) moe_linear_narrow_kernel<kGlu, 1><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      else if (narrow) moe_linear_narrow_kernel<kGlu, 2><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
       else moe_linear_many_kernel<kGlu, 2><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
     });
   } else {

@@ -657,6 +657,57 @@ def test_moe_linear_shared(rows, top, experts, n, k, sn, sk, glu):
             moe_linear(x, w, ids, **{**dict(plan=plan, per_token=top, glu=glu, shared=(xs, ws)), **bad})
 
 
+@pytest.mark.parametrize("rows,top,experts,n,k", [
+    (1, 1, 1, 64, 768),                                                   # one tile
+    (1, 6, 64, 1536, 2048), (5, 6, 64, 1536, 2048),                       # tiles of 32 rows, on both sides of the line's gap
+    (16, 2, 8, 336, 1088),                                                # 32 pairs, the last weight tile of 16 rows, steps no multiple of the buffers
+    (32, 1, 8, 192, 832),                                                 # experts of up to all 32 rows
+    (33, 1, 9, 192, 832),                                                 # tiles of 64 rows
+    (66, 1, 17, 1040, 768),                                               # ... and an expert of 65 rows: two tiles
+    (40, 3, 30, 960, 4096),
+])
+@pytest.mark.parametrize("glu,side", [(False, None), (True, None), ((1.5, 7.0, 1.0), None), (False, (64, 768)), (True, (64, 768)), (False, (208, 2112)), (True, (208, 2112))])
+def test_moe_linear_few_workgroups(rows, top, experts, n, k, glu, side):
+    """Weights in 64 rows per workgroup, most pairs one expert's: experts and, beside them, an expert of all rows against the products in float32, to a rounding
+    to 16 bits (2^-9 of the value; gated ones to those of its factors)."""
+    g = torch.Generator(device=DEV).manual_seed(rows + n + k)
+    normal = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).bfloat16()
+    n = n // 64 * 64 if glu else n
+    ids = torch.randint(0, experts, (rows, top), generator=g, device=DEV).int()
+    ids[:, 0] = experts - 1                                               # (in the 66-row case one id more, of nobody)
+    if rows == 66:
+        ids[7, 0] = -1
+    x, w = normal(rows, k + 8)[:, :k], normal(experts, n, k, std=k ** -0.5)
+    plan, shared = moe_plan(ids, experts), None
+    if side is not None:
+        sn, sk = side
+        shared = normal(rows, sk), normal(sn // 64 * 64 if glu else sn, sk, std=sk ** -0.5)
+    out = moe_linear(x, w, ids, plan, top, glu, shared=shared)
+
+    def gated(z, turns):
+        if not glu:
+            return z
+        gate, up = z.unflatten(1, (-1, 2, 32)).permute(2, 0, 1, 3).flatten(2) if turns else z.chunk(2, 1)
+        if glu is True:
+            return torch.nn.functional.silu(gate) * up
+        alpha, limit, shift = glu
+        gate = gate.clamp(max=limit)
+        return gate * torch.sigmoid(alpha * gate) * (up.clamp(-limit, limit) + shift)
+
+    def close(got, want):
+        assert got.shape == want.shape
+        worst = (got.float() - want).abs().amax(1) / want.abs().amax(1)
+        assert worst.max() < 2 ** -8, worst.max()
+
+    if shared is not None:
+        out, beside = out
+        close(beside, gated(shared[0].float() @ shared[1].float().T, False))
+    flat, place = ids.flatten().tolist(), plan.place.tolist()
+    for p, e in enumerate(flat):
+        if e >= 0:
+            close(out[place[p]][None], gated(x[p // top][None].float() @ w[e].float().T, True))
+
+
 def test_experts_call_a_shared_expert_that_is_not_as_built():
     """A hook on the shared expert or one of its parts is called, one that was replaced is used."""
     m = SparseExperts(128, 128, 4, 2, 64, shared_ff=64, small_rows=64)
