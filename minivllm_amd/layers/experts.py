@@ -20,10 +20,11 @@ from minivllm_amd.utils.padding import pad_to, round_up
 __all__ = ["ExpertOutput", "ExpertPlan", "SparseExperts", "moe_route", "moe_route_softmax", "moe_plan", "moe_linear", "interleave_gate_up"]
 
 FEW_PAIRS = 16             # (token, choice) pairs up to which the products run without a plan ...
-# ... where the experts are small: without one every expert has workgroups that look for its rows, with one only those that have some have any, and the shared
-# expert is part of the launches.  us of a captured pass at one row, without / with: 8 experts of 256 x 512 13.6 / 17.6, 64 of them 20.8 / 19.4; 16 of 512 x
-# 1024 25.1 / 24.5, 64 32.0 / 25.6; 64 of 768 x 2048 54.6 / 40.0; 64 of 1280 x 4096 109 / 74, two rows 159 / 110; 8 of 14336 x 4096 216 / 175, eight rows 513 / 391.
-FEW_WEIGHTS = 4 << 20      # experts x width x ff
+# ... where rows are short and no shared expert can join the launches: without one every expert has workgroups that look for its rows, with one only those that have
+# some have any, and the shared expert is part of the launches.  us of a captured pass, without / with, one row, top 2: 8 experts of 256 x 512 13.1 / 16.8, 128 of them 15.9 / 19.5,
+# 8 of 512 x 512 18.3 / 19.3 (with a shared expert 23.2 / 19.5); 8 of 768 x 768 23.9 / 17.8, of 128 x 2048 20.3 / 19.5, of 256 x 1024 18.8 / 17.5, 128 of them 21.9 / 19.6, eight rows
+# 28.6 / 21.0; top 6 of 64 of 768 x 2048 44 / 25, top 8 of 1280 x 4096 91 / 61; 8 of 14336 x 4096 197 / 126, eight rows 512 / 387.
+SHORT_ROWS = 768
 
 
 def _ptr(t):
@@ -217,10 +218,12 @@ class SparseExperts(nn.Module):
             ids, weights = moe_route(logits, self.correction, self.experts, self.top, self.groups, self.keep)
         pairs = ids.numel()
         plan = None
-        if h.dtype != torch.bfloat16 or pairs > FEW_PAIRS or self.experts * self.ff * self.inputs > FEW_WEIGHTS:
+        beside = self._shared_beside(h)
+        takes = 4 * self.ff * self.inputs < 1 << 31          # (sorted pairs: offsets into an expert's weights are of 32 bits)
+        if h.dtype != torch.bfloat16 or pairs > FEW_PAIRS or pairs > 0 and takes and (beside or max(self.inputs, self.ff) >= SHORT_ROWS):
             plan = moe_plan(ids, self.experts)
         shared = None
-        if plan is not None and self._shared_beside(h):
+        if plan is not None and beside:
             act, shared = moe_linear(h, self.gate_up, ids, plan, self.top, glu=True, shared=(h, self.shared.gate_up.weight))
             parts, shared = moe_linear(act, self.down, ids, plan, shared=(shared, self.shared.gate_down.weight))
         else:

@@ -729,14 +729,17 @@ def test_experts_call_a_shared_expert_that_is_not_as_built():
         assert m(h).shared is h
 
 
-@pytest.mark.parametrize("experts,sorted_pairs", [(8, False), (9, True)])
-def test_experts_of_one_row(experts, sorted_pairs):
+@pytest.mark.parametrize("width,ff,shared,sorted_pairs", [(704, 704, None, False), (768, 128, None, True), (128, 768, None, True), (128, 64, 64, True)])
+def test_experts_of_one_row(width, ff, shared, sorted_pairs):
     """Few rows, on either side of the line from which their pairs are sorted too: as in a batch, whose products are those over sorted pairs."""
-    m, g = SparseExperts(1024, 1024, experts, 2, 512), torch.Generator(device=DEV).manual_seed(experts)
-    shape = dict(router=(experts, 1024), correction=(experts,), gate=(512, 1024), up=(512, 1024), down=(1024, 512))
-    m.load(lambda name: torch.randn(shape.get(name) or shape[name.split(".")[1]], generator=g, device=DEV).mul_(1024 ** -0.5).bfloat16(), lambda t: t.contiguous())
-    h = torch.randn(40, 1024, generator=g, device=DEV).bfloat16()
+    m, g = SparseExperts(width, width, 8, 2, ff, shared_ff=shared or 0, small_rows=64), torch.Generator(device=DEV).manual_seed(width + ff)
+    shape = {"router": (8, width), "correction": (8,), "gate": (ff, width), "up": (ff, width), "down": (width, ff), "shared.sg": (1, width)}
+    if shared:
+        shape.update({"shared.gate": (shared, width), "shared.up": (shared, width), "shared.down": (width, shared)})
+    m.load(lambda name: torch.randn(shape.get(name) or shape[name.split(".")[1]], generator=g, device=DEV).mul_(width ** -0.5).bfloat16(), lambda t: t.contiguous())
+    h = torch.randn(40, width, generator=g, device=DEV).bfloat16()
     batch = m(h)
+    assert m(h[:0]).parts.shape[0] == 0
     for n in (1, 2, 8):
         out = m(h[:n])
         assert (out.part_row is not None) == sorted_pairs and torch.equal(out.weights, batch.weights[:n])
