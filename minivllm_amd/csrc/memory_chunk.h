@@ -485,7 +485,7 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
     // kOut: what the normaliser and n take of this block before the scores are there
     constexpr int kPer = kThreads / kBlock;         // threads per row
     const int n_t = tid / kPer, n_x = tid % kPer;   // this thread's row, its share of it
-    float nq = 0.f;
+    float nq = 0.f, nq_scale = 0.f;
     auto n_dot = [&]() __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < DIMP / (8 * kPer); ++i) {
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
           nq = fmaf(hi_to_float<bf16_t>(w[e]), nn[2 * e + 1], nq);
         }
       }
-      nq *= sc_in[n_t];
+      nq_scale = sc_in[n_t];
     };
     auto den_of = [&]() __attribute__((always_inline)) {       // the row's normaliser, in the row's first thread
       float sum = 0.f;
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(64 * kWaves, DIMP == 256 ? 1 : 2) void memory_chunk
         for (int e = 0; e < 4; ++e)
           sum += (lo_to_float<bf16_t>(wh[e]) + lo_to_float<bf16_t>(wl[e])) + (hi_to_float<bf16_t>(wh[e]) + hi_to_float<bf16_t>(wl[e]));
       }
-      nq += sum;
+      nq = fmaf(nq, nq_scale, sum);                 // one rounding, whether or not the product was left out
       // over the row's two, four or eight lanes
       auto moved = [&](auto CTRL) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(nq), decltype(CTRL)::value, 0xf, 0xf, false)); };
       nq += moved(std::integral_constant<int, 0xB1>{});

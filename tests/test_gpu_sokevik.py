@@ -2,6 +2,7 @@
 import math
 import random
 
+import numpy as np
 import pytest
 import torch
 
@@ -467,6 +468,46 @@ def test_mlstm_segments_side_by_side(monkeypatch, heads, dim, vdim):
     for i in range(len(lengths)):
         want = _memory_reference(cases[i][0], cases[i][1], weight, heads, dim, vdim, 1e-4)
         assert rel(torch.cat(outs[i]), want) < 4e-3, i
+
+
+def test_mlstm_normaliser_is_rounded_once():
+    """A row's normaliser |q n s + sum| where q n s, rounded, is -sum: what is left is that product's rounding error, which a sum rounded in between loses.  The
+    input gate's level puts the floor below it, and eps of 1 keeps the norm from dividing it out again."""
+    heads, dim, vdim, rows, eps = 8, 128, 256, 64, 1.0
+    scale = np.float32(dim ** -0.5)
+    level, picked = 20.0, []
+    for c in (torch.arange(2 ** 15, 2 ** 17, 2 ** 9).float()).tolist():      # a key's first number, in 16 bits
+        x = torch.tensor(np.float32(c) * scale)
+        high = x.bfloat16()
+        total = np.float32((high.float() + (x - high.float()).bfloat16().float()).item())       # the weighted score as its two halves
+        n = np.float32(-total / scale)
+        left = float(n) * float(scale) + float(total)
+        if n * scale == -total and abs(left) > 1e-4:
+            picked.append((c, float(n), float(total), abs(left)))
+    assert len(picked) >= heads
+    s = Sequence([1] * (2 * rows), block_size=16)
+    manager([], 1, 16, 2).allocate(s)
+    s.num_computed_tokens, s.num_scheduled_tokens = rows, rows
+    step = ragged_step([s], [], 16, DEV, 2 * heads)
+    state = MlstmState.allocate(2, heads, dim, vdim, DEV)
+    state.s.zero_()
+    state.n.zero_()
+    state.m.fill_(level)
+    q, k, gate = torch.zeros(rows, heads, dim), torch.zeros(rows, heads, dim), torch.zeros(rows, heads, vdim)
+    v = torch.zeros(rows, heads, vdim)
+    q[:, :, 0] = 1
+    want = torch.empty(rows, heads, vdim, dtype=torch.float64)
+    signs = torch.randint(0, 2, (heads, vdim), generator=gen(3)).double() * 2 - 1
+    for h, (c, n, total, left) in enumerate(picked[:heads]):
+        k[0, h, 0] = c
+        state.n[:, h, 0] = n
+        v[0, h] = (signs[h] * 0.1 * left / total).bfloat16().float()
+        x = v[0, h].double() * total / (left + 1e-6)
+        want[:, h] = x / torch.sqrt(x.pow(2).mean() + eps) / 2                  # (a gate of 0 is a half)
+    proj = torch.cat([t.flatten(1) for t in (q, k, v, gate)], 1).bfloat16()
+    gates = torch.cat([torch.full((rows, heads), level), torch.zeros(rows, heads)], 1)
+    out = mlstm(step, proj.to(DEV), gates.to(DEV), heads * (2 * dim + vdim), torch.ones(heads * vdim, device=DEV), state, eps).cpu()
+    assert rel(out.view(rows, heads, vdim), want) < 4e-3
 
 
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 256), (3, 24, 136), (1, 64, 200), (2, 72, 144)])
