@@ -204,9 +204,9 @@ class SparseExperts(nn.Module):
         if (m is None or self.glu is not True or h.dtype != torch.bfloat16 or h.dim() != 2 or h.shape[0] == 0 or _has_any_global_hook() or not _as_built(m, Qwen3MLP)
                 or not _as_built(m.gate_up, Linear) or not _as_built(m.gate_down, Linear) or not _as_built(m.activation, SiluAndMul)):
             return False
-        if torch.is_grad_enabled() and h.requires_grad:
-            return False
         up, down = m.gate_up.weight, m.gate_down.weight
+        if torch.is_grad_enabled() and (h.requires_grad or up.requires_grad or down.requires_grad):
+            return False
         return (m.gate_up.bias is None and m.gate_down.bias is None and up.dtype == down.dtype == h.dtype and up.is_contiguous() and down.is_contiguous()
                 and up.shape[0] == 2 * down.shape[1] and up.shape[1] == h.shape[1] and down.shape[1] % 64 == 0 and down.shape[0] % 16 == 0)
 

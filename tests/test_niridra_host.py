@@ -127,6 +127,25 @@ def test_padded_experts_are_the_experts():
     assert torch.allclose(padded @ m.router.T, torch.cat([h @ w["router"].T, h @ w["shared.sg"].T], 1), atol=1e-5)
 
 
+def _with_shared(width=128, ff=64, shared=64, experts=4, small_rows=64):
+    """A layer with a shared expert, loaded with 16-bit weights."""
+    m, g = SparseExperts(width, width, experts, 2, ff, shared_ff=shared, small_rows=small_rows), torch.Generator().manual_seed(0)
+    shape = {"router": (experts, width), "correction": (experts,), "gate": (ff, width), "up": (ff, width), "down": (width, ff), "shared.sg": (1, width),
+             "shared.gate": (shared, width), "shared.up": (shared, width), "shared.down": (width, shared)}
+    m.load(lambda name: (torch.randn(shape.get(name) or shape[name.split(".")[1]], generator=g) / 11).bfloat16(), lambda t: t.contiguous())
+    return m
+
+
+@pytest.mark.parametrize("which", ["gate_up", "gate_down", "h"])
+def test_a_shared_expert_with_gradients_is_called(which):
+    m, h = _with_shared(), torch.zeros(100, 128, dtype=torch.bfloat16)
+    assert m._shared_beside(h)
+    (h if which == "h" else getattr(m.shared, which).weight).requires_grad_(True)
+    assert not m._shared_beside(h)
+    with torch.no_grad():
+        assert m._shared_beside(h)
+
+
 # ---- metadata of layers that cache latents ----
 @pytest.mark.parametrize("seed", range(12))
 def test_latent_arrays_against_row_by_row(seed):
