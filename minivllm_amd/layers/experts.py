@@ -208,6 +208,7 @@ class SparseExperts(nn.Module):
         if torch.is_grad_enabled() and (h.requires_grad or up.requires_grad or down.requires_grad):
             return False
         return (m.gate_up.bias is None and m.gate_down.bias is None and up.dtype == down.dtype == h.dtype and up.is_contiguous() and down.is_contiguous()
+                and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0
                 and up.shape[0] == 2 * down.shape[1] and up.shape[1] == h.shape[1] and down.shape[1] % 64 == 0 and down.shape[0] % 16 == 0)
 
     def forward(self, h) -> ExpertOutput:

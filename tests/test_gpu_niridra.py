@@ -729,6 +729,26 @@ def test_experts_call_a_shared_expert_that_is_not_as_built():
         assert m(h).shared is h
 
 
+@pytest.mark.parametrize("rows", [3, 100])
+@pytest.mark.parametrize("which", ["gate_up", "gate_down"])
+def test_experts_with_a_shared_expert_at_an_odd_address(which, rows):
+    """A contiguous weight that begins two bytes into a buffer: what the module itself gives, as the launches do not take it."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    weights = {"router": (4, 128), "correction": (4,), "gate": (64, 128), "up": (64, 128), "down": (128, 64), "shared.sg": (1, 128), "shared.gate": (64, 128),
+               "shared.up": (64, 128), "shared.down": (128, 64)}
+    m = SparseExperts(128, 128, 4, 2, 64, shared_ff=64)
+    m.load(lambda name: (torch.randn(weights.get(name) or weights[name.split(".")[1]], generator=g, device=DEV) / 11).bfloat16(), lambda t: t.contiguous())
+    h = torch.randn(rows, 128, generator=g, device=DEV).bfloat16()
+    with torch.no_grad():
+        beside = m(h).shared
+        part = getattr(m.shared, which)
+        flat = torch.empty(part.weight.numel() + 1, dtype=torch.bfloat16, device=DEV)
+        flat[1:] = part.weight.flatten()
+        part.weight = torch.nn.Parameter(flat[1:].view_as(part.weight), requires_grad=False)
+        got = m(h).shared
+        assert torch.equal(got, m.shared(h)) and torch.allclose(got.float(), beside.float(), atol=2 ** -6)
+
+
 @pytest.mark.parametrize("width,ff,shared,sorted_pairs", [(704, 704, None, False), (768, 128, None, True), (128, 768, None, True), (128, 64, 64, True)])
 def test_experts_of_one_row(width, ff, shared, sorted_pairs):
     """Few rows, on either side of the line from which their pairs are sorted too: as in a batch, whose products are those over sorted pairs."""

@@ -146,6 +146,21 @@ def test_a_shared_expert_with_gradients_is_called(which):
         assert m._shared_beside(h)
 
 
+def _at_odd_address(weight):
+    """The same numbers in a contiguous view that begins two bytes into a buffer."""
+    flat = torch.empty(weight.numel() + 1, dtype=weight.dtype, device=weight.device)
+    flat[1:] = weight.detach().flatten()
+    return torch.nn.Parameter(flat[1:].view_as(weight), requires_grad=False)
+
+
+@pytest.mark.parametrize("which", ["gate_up", "gate_down"])
+def test_a_shared_expert_at_an_odd_address_is_called(which):
+    m, h = _with_shared(), torch.zeros(100, 128, dtype=torch.bfloat16)
+    part = getattr(m.shared, which)
+    part.weight = _at_odd_address(part.weight)
+    assert part.weight.is_contiguous() and not m._shared_beside(h)
+
+
 # ---- metadata of layers that cache latents ----
 @pytest.mark.parametrize("seed", range(12))
 def test_latent_arrays_against_row_by_row(seed):
