@@ -60,6 +60,11 @@ class ExpertPlan:
         return self.data[:self.pairs]
 
 
+def _span(x) -> int:
+    """Numbers from the first of x (rows, K) to behind the last, rows dense."""
+    return (x.shape[0] - 1) * x.stride(0) + x.shape[1]
+
+
 def moe_route(logits: torch.Tensor, correction: torch.Tensor | None, experts: int, top: int, groups: int = 1, keep: int = 1):
     """(ids int32 (T, top), weights float32 (T, top)) from float32 logits (T, >= experts)."""
     _C.require_cuda(logits, correction)
@@ -208,7 +213,8 @@ class SparseExperts(nn.Module):
         if torch.is_grad_enabled() and (h.requires_grad or up.requires_grad or down.requires_grad):
             return False
         return (m.gate_up.bias is None and m.gate_down.bias is None and up.dtype == down.dtype == h.dtype and up.is_contiguous() and down.is_contiguous()
-                and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0
+                and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0 and 2 * up.numel() < 1 << 31 and 2 * down.numel() < 1 << 31
+                and _span(h) < 1 << 31 and h.shape[0] * down.shape[1] < 1 << 31          # (offsets of 32 bits into weights and, unsigned, rows)
                 and up.shape[0] == 2 * down.shape[1] and up.shape[1] == h.shape[1] and down.shape[1] % 64 == 0 and down.shape[0] % 16 == 0)
 
     def forward(self, h) -> ExpertOutput:

@@ -161,6 +161,20 @@ def test_a_shared_expert_at_an_odd_address_is_called(which):
     assert part.weight.is_contiguous() and not m._shared_beside(h)
 
 
+@pytest.mark.parametrize("inputs,shared,rows,stride,takes", [
+    (4096, 131008, 5, 4096, True), (4096, 131072, 5, 4096, False),              # gate and up of 2 GiB
+    (4096, 1024, 2 ** 19 - 1, 4096, True), (4096, 1024, 2 ** 19, 4096, False),  # rows of 4 GiB
+    (4096, 1024, 3, 2 ** 30 - 4096, True), (4096, 1024, 3, 2 ** 30 - 2048, False),
+    (1024, 4096, 2 ** 19, 1024, False)])                                        # ... of gated units
+def test_a_shared_expert_past_32_bit_offsets_is_called(inputs, shared, rows, stride, takes):
+    with torch.device("meta"):
+        m = SparseExperts(inputs, inputs, 4, 2, 64, shared_ff=shared)
+        m.shared.to(torch.bfloat16)
+        m.shared.requires_grad_(False)
+        h = torch.empty_strided((rows, inputs), (stride, 1), dtype=torch.bfloat16)
+    assert m._shared_beside(h) == takes
+
+
 # ---- metadata of layers that cache latents ----
 @pytest.mark.parametrize("seed", range(12))
 def test_latent_arrays_against_row_by_row(seed):
