@@ -217,6 +217,13 @@ class SparseExperts(nn.Module):
                 and _span(h) < 1 << 31 and h.shape[0] * down.shape[1] < 1 << 31          # (offsets of 32 bits into weights and, unsigned, rows)
                 and up.shape[0] == 2 * down.shape[1] and up.shape[1] == h.shape[1] and down.shape[1] % 64 == 0 and down.shape[0] % 16 == 0)
 
+    def _sorted(self, h, pairs: int, beside: bool) -> bool:
+        """Whether the products go over sorted pairs: always but for few pairs in 16 bits, and for those too where it pays (``SHORT_ROWS``) and offsets into an
+        expert's weights and the rows are of 32 bits."""
+        if h.dtype != torch.bfloat16 or pairs > FEW_PAIRS:
+            return True
+        return (pairs > 0 and (beside or max(self.inputs, self.ff) >= SHORT_ROWS) and 4 * self.ff * self.inputs < 1 << 31 and _span(h) < 1 << 31)
+
     def forward(self, h) -> ExpertOutput:
         logits = gate_linear(h, self.router, None, self.router.shape[0], 0.0)
         if self.softmax:
@@ -226,8 +233,7 @@ class SparseExperts(nn.Module):
         pairs = ids.numel()
         plan = None
         beside = self._shared_beside(h)
-        takes = 4 * self.ff * self.inputs < 1 << 31          # (sorted pairs: offsets into an expert's weights are of 32 bits)
-        if h.dtype != torch.bfloat16 or pairs > FEW_PAIRS or pairs > 0 and takes and (beside or max(self.inputs, self.ff) >= SHORT_ROWS):
+        if self._sorted(h, pairs, beside):
             plan = moe_plan(ids, self.experts)
         shared = None
         if plan is not None and beside:

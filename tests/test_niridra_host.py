@@ -175,6 +175,17 @@ def test_a_shared_expert_past_32_bit_offsets_is_called(inputs, shared, rows, str
     assert m._shared_beside(h) == takes
 
 
+@pytest.mark.parametrize("inputs,ff,rows,stride,is_sorted", [
+    (1024, 512, 3, 1024, True), (512, 704, 3, 512, False), (64, 768, 0, 64, False), (512, 704, 9, 512, True),
+    (4096, 131008, 3, 4096, True), (4096, 131072, 3, 4096, False),              # an expert's gate and up of 2 GiB
+    (1024, 512, 3, 2 ** 30 - 1024, True), (1024, 512, 3, 2 ** 30 - 512, False), # rows that span 4 GiB
+    (1024, 512, 1, 2 ** 31, True)])
+def test_few_pairs_are_sorted_where_sorted_products_take_them(inputs, ff, rows, stride, is_sorted):
+    with torch.device("meta"):
+        h = torch.empty_strided((rows, inputs), (stride, 1), dtype=torch.bfloat16)
+    assert SparseExperts(inputs, inputs, 4, 2, ff)._sorted(h, 2 * rows, False) == is_sorted
+
+
 # ---- metadata of layers that cache latents ----
 @pytest.mark.parametrize("seed", range(12))
 def test_latent_arrays_against_row_by_row(seed):
