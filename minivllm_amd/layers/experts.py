@@ -210,12 +210,27 @@ class SparseExperts(nn.Module):
                 or not _as_built(m.gate_up, Linear) or not _as_built(m.gate_down, Linear) or not _as_built(m.activation, SiluAndMul)):
             return False
         up, down = m.gate_up.weight, m.gate_down.weight
+        if not self._beside_pays(h.shape[0]):
+            return False
         if torch.is_grad_enabled() and (h.requires_grad or up.requires_grad or down.requires_grad):
             return False
         return (m.gate_up.bias is None and m.gate_down.bias is None and up.dtype == down.dtype == h.dtype and up.is_contiguous() and down.is_contiguous()
                 and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0 and 2 * up.numel() < 1 << 31 and 2 * down.numel() < 1 << 31
                 and _span(h) < 1 << 31 and h.shape[0] * down.shape[1] < 1 << 31          # (offsets of 32 bits into weights and, unsigned, rows)
                 and up.shape[0] == 2 * down.shape[1] and up.shape[1] == h.shape[1] and down.shape[1] % 64 == 0 and down.shape[0] % 16 == 0)
+
+    def _beside_pays(self, rows: int) -> bool:
+        """Whether the shared expert's products are better off in the experts' launches.
+
+        They run on tiles made for the experts' rows.  The few long tiles (K of ``shared_ff``) of a shared expert that is large, and much larger than the others, are
+        still running when all others are done, unless large tiles share the rounds out; and tiles of 64 rows (``rows * top`` up to 48 per expert) are far
+        behind the library's product once there are many.  785 mixtures of 8 to 256 experts of 64 to 2048, shared ones of 64 to 10240, 1 to 8192 rows:
+        within these lines 1.14 times as fast on average, 8 of 600 more than 3 % slower (worst 0.914); beyond them 0.99, 69 of 185 more than 3 % slower (worst
+        0.63).  us apart / beside, 2048 wide: 8 experts of 1408 and 7680 shared, 56 rows 83 / 114; top 1 of 64 of 1536 and 8448, 2627 rows 552 / 761; top 1 of
+        256 of 704 and 1344, 7911 rows 540 / 626.  From 96 rows per expert on a large shared expert is as well off: top 4 of 64 of 1408 and 5632, 2048 rows
+        498 / 443."""
+        pairs = rows * self.top
+        return (self.shared_ff <= max(2048, 3.5 * self.ff) or pairs >= 96 * self.experts) and (rows <= 1500 or pairs > 48 * self.experts)
 
     def _sorted(self, h, pairs: int, beside: bool) -> bool:
         """Whether the products go over sorted pairs: always but for few pairs in 16 bits, and for those too where it pays (``SHORT_ROWS``) and offsets into an

@@ -168,7 +168,7 @@ def test_a_shared_expert_at_an_odd_address_is_called(which):
     (1024, 4096, 2 ** 19, 1024, False)])                                        # ... of gated units
 def test_a_shared_expert_past_32_bit_offsets_is_called(inputs, shared, rows, stride, takes):
     with torch.device("meta"):
-        m = SparseExperts(inputs, inputs, 4, 2, 64, shared_ff=shared)
+        m = SparseExperts(inputs, inputs, 4, 2, 40960, shared_ff=shared)
         m.shared.to(torch.bfloat16)
         m.shared.requires_grad_(False)
         h = torch.empty_strided((rows, inputs), (stride, 1), dtype=torch.bfloat16)
@@ -184,6 +184,21 @@ def test_few_pairs_are_sorted_where_sorted_products_take_them(inputs, ff, rows, 
     with torch.device("meta"):
         h = torch.empty_strided((rows, inputs), (stride, 1), dtype=torch.bfloat16)
     assert SparseExperts(inputs, inputs, 4, 2, ff)._sorted(h, 2 * rows, False) == is_sorted
+
+
+@pytest.mark.parametrize("experts,top,ff,shared,rows,joins", [
+    (64, 6, 768, 1536, 1, True), (64, 6, 768, 1536, 8192, True), (64, 8, 1280, 2048, 32, True),
+    (64, 4, 640, 2240, 33, True), (64, 4, 640, 2304, 33, False),                # 3.5 times the others
+    (64, 1, 256, 2048, 33, True), (64, 1, 256, 2112, 33, False),                # ... or 2048
+    (64, 4, 1408, 5632, 1535, False), (64, 4, 1408, 5632, 1536, True),          # 96 rows per expert
+    (128, 2, 704, 1344, 1500, True), (128, 2, 704, 1344, 1501, False), (128, 2, 704, 1344, 3072, False), (128, 2, 704, 1344, 3073, True)])    # more than 48
+def test_which_shared_experts_join_the_others(experts, top, ff, shared, rows, joins):
+    with torch.device("meta"):
+        m = SparseExperts(2048, 2048, experts, top, ff, shared_ff=shared)
+        m.shared.to(torch.bfloat16)
+        m.shared.requires_grad_(False)
+        assert m._beside_pays(rows) == joins
+        assert m._shared_beside(torch.empty(rows, 2048, dtype=torch.bfloat16)) == (joins and shared % 64 == 0)
 
 
 # ---- metadata of layers that cache latents ----
