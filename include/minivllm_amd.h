@@ -96,7 +96,9 @@ size_t mvllm_paged_decode_workspace_bytes(int batch, int num_heads, int head_dim
 /*
  * How mvllm_paged_decode{,_int8} split these static sizes (no counterpart in the reference, whose Triton kernel
  * walks a whole context in one program, attention.py:283-415).  Pure host arithmetic:
- *   *part_tokens      tokens of a partition; partition p of a sequence covers tokens [p, p+1) * part_tokens
+ *   *part_tokens      tokens of a partition at most.  Partition p of a sequence covers tokens [p, p+1) * part_tokens, but where
+ *                     waves share a head (waves_per_head > 1) shorter sequences may be cut into shorter partitions:
+ *                     mvllm_paged_decode_partition has their length
  *   *num_parts        partitions per sequence (1: no workspace is touched and no merge kernel is launched)
  *   *waves_per_head   1: a workgroup holds up to 4 kv heads, one wave each, and every wave walks its partition;
  *                     >1: small-batch form, a workgroup is that many waves on one kv head that share the
@@ -110,6 +112,16 @@ size_t mvllm_paged_decode_workspace_bytes(int batch, int num_heads, int head_dim
 int mvllm_paged_decode_plan(int batch, int num_heads, int num_kv_heads, int head_dim,
                             int max_num_blocks, int block_size, int dtype, int int8_cache,
                             int* part_tokens, int* num_parts, int* waves_per_head);
+
+/*
+ * ... and how long the partitions of a sequence of context_len tokens are in such a call: partition p covers tokens
+ * [p, p+1) * *tokens.  *tokens <= part_tokens, and no sequence has more than num_parts partitions.  Pure host arithmetic.
+ * Returns MVLLM_OK, MVLLM_ERR_BAD_SHAPE (also for a context_len that the table does not hold) / MVLLM_ERR_BAD_DTYPE /
+ * MVLLM_ERR_NULL_POINTER.
+ */
+int mvllm_paged_decode_partition(int batch, int num_heads, int num_kv_heads, int head_dim,
+                                 int max_num_blocks, int block_size, int dtype, int int8_cache,
+                                 int64_t context_len, int* tokens);
 
 /*
  * paged_attention_decode -- src/myvllm/layers/attention.py:418-473 (kernel :283-415).

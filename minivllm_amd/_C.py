@@ -31,6 +31,7 @@ SIGNATURES = {
     "mvllm_store_kvcache_int8": (c_int, [c_void_p] * 7 + [c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
     "mvllm_paged_decode_workspace_bytes": (c_size_t, [c_int] * 5),
     "mvllm_paged_decode_plan": (c_int, [c_int] * 8 + [ctypes.POINTER(c_int)] * 3),
+    "mvllm_paged_decode_partition": (c_int, [c_int] * 8 + [c_int64, ctypes.POINTER(c_int)]),
     "mvllm_paged_decode": (c_int, [c_void_p] * 5 + [c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                                                      c_int64, c_float, c_int, c_void_p, c_size_t, c_void_p]),
     "mvllm_paged_decode_noalloc": (c_int, [c_void_p] * 5 + [c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,

@@ -213,9 +213,9 @@ __device__ __forceinline__ int64_t load_ctx(const DecodeArgs& a, int b) {
 // layers, tables of 2048, before / so: 12 sequences of 200-400 296 / 272, of 900-1200 329 / 310, 16 of 300-1500 358 / 327, 28 of them 422 / 406, of 30-60
 // as before; of a call, tables as wide as the longest context: 15 of 269-640 13.0 / 11.8, 7 of 100-4000 18.4 / 16.8, 23 of 200-4175 with heads of 64 28.7 / 23.7, INT8
 // 33.5 / 29.4, 12 of 1000-8000 with heads of 64 31.5 / 28.3, 20 of 100-16000 with heads of 64 INT8 52.7 / 49.4, 12 of 1000-8000 48.7 / 49.5.
-__device__ __forceinline__ int part_tokens_of(const DecodeArgs& a, int ctx) {
+__host__ __device__ __forceinline__ int part_tokens_of(const DecodeArgs& a, int ctx) {
   if (a.spread == 0) return a.part_tokens;
-  const int even = (int)__umulhi((uint32_t)(ctx + a.spread - 1), a.spread_factor);      // ctx / spread rounded up, or more
+  const int even = (int)(((uint64_t)(uint32_t)(ctx + a.spread - 1) * a.spread_factor) >> 32);      // ctx / spread rounded up, or more
   return min(max((even + 63) & ~63, a.least), a.part_tokens);
 }
 
@@ -1770,6 +1770,14 @@ static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, i
   return plan;
 }
 
+static void set_plan(DecodeArgs& a, const DecodePlan& plan) {
+  a.part_tokens = plan.part_tokens;
+  a.num_parts = plan.num_parts;
+  a.spread = plan.spread;
+  a.spread_factor = plan.spread == 0 ? 0u : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)plan.spread - 1) / (uint64_t)plan.spread);
+  a.least = plan.least;
+}
+
 // INT8 keys of 128 dims in whole rows through LDS, or as operands straight from memory: rows cost the address unit a quarter, and a longer way from a
 // load to its product, which a wave with the SIMD to itself waits for: from more than two waves per SIMD on.  us, rows / operands, 8 kv heads: 5
 // sequences of 30000 tokens (1200 waves) 101 / 94, 8 (1920) 105 / 99, 10 (2400) 118 / 119, 16 222 / 226; 128 of 1000 to 13700 366 / 374, of 4096 209 / 205.
@@ -1907,11 +1915,7 @@ static int decode_entry(void* out, const void* q, const void* k_cache, const voi
                        aligned16(q) && aligned16(out) && aligned16(k_cache) && aligned16(v_cache);
   a.head_chunks = head_chunks_of(num_heads, num_kv_heads);
   const DecodePlan plan = plan_decode(batch, num_kv_heads * a.head_chunks, max_num_blocks, block_size, fast_ok, int8, head_dim, dtype);
-  a.part_tokens = plan.part_tokens;
-  a.num_parts = plan.num_parts;
-  a.spread = plan.spread;
-  a.spread_factor = plan.spread == 0 ? 0u : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)plan.spread - 1) / (uint64_t)plan.spread);
-  a.least = plan.least;
+  set_plan(a, plan);
   a.scale_log2 = scale * kLog2e;
   a.sink = sink;
   a.ws_acc = nullptr; a.ws_ml = nullptr;
@@ -1975,18 +1979,39 @@ extern "C" size_t mvllm_paged_decode_workspace_bytes(int batch, int num_heads, i
   return workspace_bytes_for(batch, num_heads, head_dim, max_num_blocks, block_size);
 }
 
-extern "C" int mvllm_paged_decode_plan(int batch, int num_heads, int num_kv_heads, int head_dim, int max_num_blocks,
-                                       int block_size, int dtype, int int8_cache, int* part_tokens, int* num_parts,
-                                       int* waves_per_head) {
+static int plan_of_sizes(int batch, int num_heads, int num_kv_heads, int head_dim, int max_num_blocks, int block_size, int dtype, int int8_cache,
+                         DecodePlan& plan) {
   if (dtype_size(dtype) == 0) return MVLLM_ERR_BAD_DTYPE;
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || block_size <= 0 || max_num_blocks <= 0 ||
       num_heads % num_kv_heads != 0)
     return MVLLM_ERR_BAD_SHAPE;
-  const DecodePlan plan = plan_decode(batch, num_kv_heads * head_chunks_of(num_heads, num_kv_heads), max_num_blocks, block_size,
-                                      fast_shape(num_heads, num_kv_heads, head_dim, block_size, dtype, int8_cache != 0), int8_cache != 0, head_dim, dtype);
+  plan = plan_decode(batch, num_kv_heads * head_chunks_of(num_heads, num_kv_heads), max_num_blocks, block_size,
+                     fast_shape(num_heads, num_kv_heads, head_dim, block_size, dtype, int8_cache != 0), int8_cache != 0, head_dim, dtype);
+  return MVLLM_OK;
+}
+
+extern "C" int mvllm_paged_decode_plan(int batch, int num_heads, int num_kv_heads, int head_dim, int max_num_blocks,
+                                       int block_size, int dtype, int int8_cache, int* part_tokens, int* num_parts,
+                                       int* waves_per_head) {
+  DecodePlan plan;
+  const int bad = plan_of_sizes(batch, num_heads, num_kv_heads, head_dim, max_num_blocks, block_size, dtype, int8_cache, plan);
+  if (bad != MVLLM_OK) return bad;
   if (part_tokens) *part_tokens = plan.part_tokens;
   if (num_parts) *num_parts = plan.num_parts;
   if (waves_per_head) *waves_per_head = plan.waves_per_head;
+  return MVLLM_OK;
+}
+
+extern "C" int mvllm_paged_decode_partition(int batch, int num_heads, int num_kv_heads, int head_dim, int max_num_blocks,
+                                            int block_size, int dtype, int int8_cache, int64_t context_len, int* tokens) {
+  DecodePlan plan;
+  const int bad = plan_of_sizes(batch, num_heads, num_kv_heads, head_dim, max_num_blocks, block_size, dtype, int8_cache, plan);
+  if (bad != MVLLM_OK) return bad;
+  if (context_len < 0 || context_len > (int64_t)max_num_blocks * block_size || context_len > (int64_t)1 << 30) return MVLLM_ERR_BAD_SHAPE;
+  if (!tokens) return MVLLM_ERR_NULL_POINTER;
+  DecodeArgs a = {};
+  set_plan(a, plan);
+  *tokens = part_tokens_of(a, (int)context_len);
   return MVLLM_OK;
 }
 

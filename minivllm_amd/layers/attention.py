@@ -25,7 +25,7 @@ from minivllm_amd.utils.context import get_context
 __all__ = [
     "store_kvcache", "store_kvcache_int8", "flash_attention_prefill", "flash_attention_prefill_paged",
     "flash_attention_prefill_paged_int8",
-    "paged_attention_decode", "paged_attention_decode_int8", "decode_workspace_bytes", "paged_decode_plan",
+    "paged_attention_decode", "paged_attention_decode_int8", "decode_workspace_bytes", "paged_decode_plan", "paged_decode_partition",
     "prefill_plan", "Attention",
 ]
 
@@ -460,7 +460,7 @@ def _decode_common(query, k_cache, v_cache, block_tables, context_lens, num_head
 def paged_decode_plan(batch: int, num_heads: int, num_kv_heads: int, head_dim: int, max_num_blocks: int,
                       block_size: int, dtype: torch.dtype = torch.bfloat16, int8_cache: bool = False):
     """(part_tokens, num_parts, waves_per_head) a decode call of these static sizes runs with (host arithmetic only).
-    waves_per_head: 1 = one wave per kv head walks a partition, >1 = the small-batch form (that many waves share
+    part_tokens: the most that a partition has (``paged_decode_partition`` for a sequence's own).  waves_per_head: 1 = one wave per kv head walks a partition, >1 = the small-batch form (that many waves share
     one kv head's partition), 0 = the generic kernel."""
     import ctypes
     out = [ctypes.c_int(0) for _ in range(3)]
@@ -468,6 +468,18 @@ def paged_decode_plan(batch: int, num_heads: int, num_kv_heads: int, head_dim: i
                                            _C.dtype_code(dtype), int(int8_cache), *[ctypes.byref(x) for x in out])
     _C.check(st, "paged_decode_plan")
     return tuple(x.value for x in out)
+
+
+def paged_decode_partition(context_len: int, batch: int, num_heads: int, num_kv_heads: int, head_dim: int, max_num_blocks: int,
+                           block_size: int, dtype: torch.dtype = torch.bfloat16, int8_cache: bool = False) -> int:
+    """Tokens of the partitions of a sequence of ``context_len`` tokens in a decode call of these static sizes (host arithmetic only): where
+    waves share a head, shorter sequences may be cut into shorter ones than ``paged_decode_plan``'s part_tokens."""
+    import ctypes
+    out = ctypes.c_int(0)
+    st = _C.load().mvllm_paged_decode_partition(batch, num_heads, num_kv_heads, head_dim, max_num_blocks, block_size,
+                                                _C.dtype_code(dtype), int(int8_cache), context_len, ctypes.byref(out))
+    _C.check(st, "paged_decode_partition")
+    return out.value
 
 
 def prefill_plan(num_heads: int, num_kv_heads: int, head_dim: int, block_size: int = 0,

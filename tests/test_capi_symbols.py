@@ -27,7 +27,7 @@ def _lib():
 def test_header_declares_expected_entry_points():
     names = _declared()
     for n in ["mvllm_store_kvcache", "mvllm_store_kvcache_int8", "mvllm_paged_decode",
-              "mvllm_paged_decode_int8", "mvllm_paged_decode_noalloc", "mvllm_paged_decode_workspace_bytes", "mvllm_paged_decode_plan", "mvllm_prefill_plan", "mvllm_prefill_varlen",
+              "mvllm_paged_decode_int8", "mvllm_paged_decode_noalloc", "mvllm_paged_decode_workspace_bytes", "mvllm_paged_decode_plan", "mvllm_paged_decode_partition", "mvllm_prefill_plan", "mvllm_prefill_varlen",
               "mvllm_prefill_paged", "mvllm_prefill_paged_int8", "mvllm_prefill_paged_int8_staged", "mvllm_prefill_paged_staged", "mvllm_prefill_paged_staged_workspace_bytes", "mvllm_prefill_paged_split", "mvllm_prefill_paged_int8_split", "mvllm_prefill_paged_split_plan", "mvllm_prefill_paged_split_workspace_bytes", "mvllm_qk_norm_rope_store", "mvllm_sample_tokens", "mvllm_sample_tokens_dev_offset", "mvllm_decode_advance", "mvllm_sample_tokens_workspace_bytes",
               "mvllm_add_rms_norm", "mvllm_linear_small_m", "mvllm_norm_linear_small_m", "mvllm_linear_small_m_plan",
               "mvllm_linear_small_m_split", "mvllm_linear_small_m_split_bytes", "mvllm_prefill_ranges", "mvllm_prefill_ranges_plan", "mvllm_prefill_store",
@@ -182,6 +182,33 @@ def test_decode_plan_in_narrow_tables():
     assert thin(33, 2048, 64, 8) == (1024, 2, 4) and thin(33, 2048, 128, 8) == (2048, 1, 4)            # blocks of less than a tile
     assert plan(31, 2064) == (704, 3, 4) and plan(33, 2064) == (1088, 2, 4)
     assert plan(1, 2048, int8_cache=True)[0] == 64 and plan(1, 2048, dtype=torch.float32)[0] == 64
+
+
+def test_decode_partitions_of_a_sequence():
+    """Their length follows the sequence's own where the plan says so, is never past the plan's, and never makes more of them than the workspace has."""
+    import random
+    import torch
+    from minivllm_amd.layers.attention import paged_decode_partition, paged_decode_plan
+    _lib().load()
+    of = lambda ctx, batch, tokens, d=128, block=16, **kw: paged_decode_partition(ctx, batch, 32, 8, d, tokens // block, block, **kw)
+    assert paged_decode_plan(12, 32, 8, 128, 128, 16) == (384, 6, 4)
+    assert [of(n, 12, 2048) for n in (0, 1, 640, 641, 960, 961, 1600, 1601, 2048)] == [128, 128, 128, 192, 192, 256, 320, 384, 384]      # a fifth (512 / 96), in whole 64s
+    assert paged_decode_plan(24, 32, 8, 128, 128, 16) == (704, 3, 4) and [of(n, 24, 2048) for n in (300, 1024, 1025, 2048)] == [512, 512, 576, 704]     # 512 at least
+    assert of(1, 33, 2048) == 2048 and of(300, 64, 32768) == of(32768, 64, 32768) == 1024      # one partition, or one wave per head: the plan's
+    assert of(100, 12, 2048, dtype=torch.float32) == of(2048, 12, 2048, dtype=torch.float32)
+    rng, shorter = random.Random(3), 0
+    for _ in range(3000):
+        batch, tokens, kv = rng.randint(1, 80), 16 * rng.randint(1, 2000), rng.choice((1, 2, 8))
+        sizes = (batch, 4 * kv, kv, rng.choice((32, 64, 128, 256)), tokens // 16, 16, rng.choice((torch.bfloat16, torch.float16, torch.float32)), rng.random() < 0.3)
+        part, parts, waves = paged_decode_plan(*sizes)
+        ctx = rng.randint(0, tokens)
+        own = paged_decode_partition(ctx, *sizes)
+        assert 0 < own <= part and -(-ctx // own) <= parts and (own == part or own % 64 == 0 and waves > 1)
+        shorter += own < part
+    assert shorter > 100
+    for bad in (-1, 2049):
+        with pytest.raises(ValueError):
+            of(bad, 12, 2048)
 
 
 def test_decode_plan_is_host_arithmetic():
