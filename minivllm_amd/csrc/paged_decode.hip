@@ -211,8 +211,10 @@ __device__ __forceinline__ int64_t load_ctx(const DecodeArgs& a, int b) {
 // four of the grid's, 640: 389 / 405).  No shorter than `least`: 128 where CUs would be idle else, 512 where memory is the bound anyway (16-bit heads of 128; 30 of 500 to 2000
 // 31.0 with 512 and 33.4 with 128, 20 of 100 to 16000 72.0 / 75.9), 256 for the others, whose tokens take a wave as long.  us of a decode step of eight
 // layers, tables of 2048, before / so: 12 sequences of 200-400 296 / 272, of 900-1200 329 / 310, 16 of 300-1500 358 / 327, 28 of them 422 / 406, of 30-60
-// as before; of a call, tables as wide as the longest context: 15 of 269-640 13.0 / 11.8, 7 of 100-4000 18.4 / 16.8, 23 of 200-4175 with heads of 64 28.7 / 23.7, INT8
-// 33.5 / 29.4, 12 of 1000-8000 with heads of 64 31.5 / 28.3, 20 of 100-16000 with heads of 64 INT8 52.7 / 49.4, 12 of 1000-8000 48.7 / 49.5.
+// as before; of a call, tables as wide as the longest context: 15 of 269-640 13.0 / 11.8, 7 of 100-4000 18.4 / 16.8, 23 of 200-4175 with heads of 64 28.7 / 23.7,
+// 12 of 1000-8000 with heads of 64 31.5 / 28.3.  In wide tables it is chance whether more and shorter partitions fill the last round better or open another:
+// 126 random batches of 16-bit caches 1.033 times as fast on average, between 0.915 and 1.28, 7 more than 3 % slower (12 of 1000-5840 32.3 / 34.1; 15 of
+// 3500-4600 with heads of 64 33.7 / 30.7); INT8 up to kSpreadInt8Pairs 1.036, 6 of 102.  Beyond that nothing is gained: 88 batches 1.003, 16 more than 3 % slower, 22 of 680-6400 with heads of 64 36 / 41.
 __host__ __device__ __forceinline__ int part_tokens_of(const DecodeArgs& a, int ctx) {
   if (a.spread == 0) return a.part_tokens;
   const int even = (int)(((uint64_t)(uint32_t)(ctx + a.spread - 1) * a.spread_factor) >> 32);      // ctx / spread rounded up, or more
@@ -1748,6 +1750,7 @@ struct DecodePlan {
   int spread, least;      // how many partitions a sequence is to have, and of how many tokens at least (see part_tokens_of); 0: of part_tokens
 };
 constexpr int kSpreadFinePairs = 176;
+constexpr int kSpreadInt8Pairs[2] = {128, 176};     // (sequence, kv head) pairs of INT8 caches in wide tables, heads of 64 and of 128
 static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, int block_size, bool fast_ok, bool int8, int head_dim, int dtype) {
   const int64_t max_ctx = (int64_t)max_num_blocks * block_size;
   const bool split = fast_ok && split_wanted(max_ctx, batch, num_kv_heads, int8);
@@ -1765,7 +1768,7 @@ static DecodePlan plan_decode(int batch, int num_kv_heads, int max_num_blocks, i
   plan.least = wide ? (pairs <= 64 ? 256 : 512) : !heavy ? 256 : pairs > kSpreadFinePairs ? 512 : 128;
   plan.spread = wide || plan.num_parts * pairs <= kSplitMinGroups ? plan.num_parts : (int)(kSplitMinGroups / pairs);
   if (plan.waves_per_head != kSplitWaves || dtype == MVLLM_F32 || (head_dim != 64 && head_dim != 128) || block_size % kTile != 0 || plan.num_parts == 1 ||
-      plan.part_tokens < 256 || plan.part_tokens <= plan.least || plan.spread < 2)
+      plan.part_tokens < 256 || plan.part_tokens <= plan.least || plan.spread < 2 || (int8 && wide && pairs > kSpreadInt8Pairs[head_dim == 128]))
     plan.spread = 0;
   return plan;
 }

@@ -195,6 +195,10 @@ def test_decode_partitions_of_a_sequence():
     assert [of(n, 12, 2048) for n in (0, 1, 640, 641, 960, 961, 1600, 1601, 2048)] == [128, 128, 128, 192, 192, 256, 320, 384, 384]      # a fifth (512 / 96), in whole 64s
     assert paged_decode_plan(24, 32, 8, 128, 128, 16) == (704, 3, 4) and [of(n, 24, 2048) for n in (300, 1024, 1025, 2048)] == [512, 512, 576, 704]     # 512 at least
     assert of(1, 33, 2048) == 2048 and of(300, 64, 32768) == of(32768, 64, 32768) == 1024      # one partition, or one wave per head: the plan's
+    wide = lambda batch, d, int8: of(100, batch, 6144, d, int8_cache=int8) < paged_decode_plan(batch, 32, 8, d, 384, 16, int8_cache=int8)[0]
+    assert wide(24, 64, False) and wide(24, 128, False)                                # wide tables of INT8 caches up to 128 pairs of heads of 64, 176 of 128
+    assert wide(16, 64, True) and not wide(17, 64, True) and wide(22, 128, True) and not wide(23, 128, True)
+    assert of(100, 30, 2048, 64, int8_cache=True) < paged_decode_plan(30, 32, 8, 64, 128, 16, int8_cache=True)[0]
     assert of(100, 12, 2048, dtype=torch.float32) == of(2048, 12, 2048, dtype=torch.float32)
     rng, shorter = random.Random(3), 0
     for _ in range(3000):
