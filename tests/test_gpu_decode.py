@@ -10,7 +10,7 @@ import torch
 
 import oracle
 from helpers import error_stats, extract_sequence, make_paged_case, make_paged_case_on_device
-from minivllm_amd.layers.attention import Attention, paged_attention_decode, paged_decode_plan
+from minivllm_amd.layers.attention import Attention, paged_attention_decode, paged_decode_partition, paged_decode_plan
 from minivllm_amd.utils import reset_context, set_context
 
 pytestmark = pytest.mark.gpu
@@ -307,17 +307,20 @@ def test_both_grid_forms_vs_oracle(dtype, hq, hkv, bs, d, form):
     assert torch.count_nonzero(got[3]) == 0
 
 
-@pytest.mark.parametrize("batch,width,d,bs,dtype", [
-    (12, 2048, 128, 16, torch.bfloat16), (12, 2048, 64, 256, torch.float16),          # as many partitions as the grid has; tables of 128 entries and of 8
-    (20, 2016, 128, 48, torch.bfloat16), (24, 2048, 128, 16, torch.float16),          # fewer than that; partitions of at least 512 tokens
-    (9, 4096, 128, 16, torch.bfloat16), (20, 8192, 64, 32, torch.bfloat16)])          # wide tables
-def test_partitions_as_long_as_the_contexts_ask_for(batch, width, d, bs, dtype):
-    """Sequences of a call whose partitions follow their own lengths: at, in front of and past every length that one partition, a multiple of 64 tokens or
-    as many partitions as there are take, up to the table's."""
-    part, parts, waves = paged_decode_plan(batch, 16, 8, d, width // bs, bs, dtype)
-    assert parts > 1 and waves == 4 and part >= 256
-    edges = [1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 383, 384, 385, 511, 512, 513, 128 * parts, 128 * parts + 1, 256 * parts, 256 * parts + 1, 700, 1030, part * parts]
-    edges = [min(n, width) for n in edges] + [width - 1, width]
+@pytest.mark.parametrize("batch,width,d,bs,dtype,part,parts,spread,least", [
+    (12, 2048, 128, 16, torch.bfloat16, 384, 6, 5, 128), (12, 2048, 64, 256, torch.float16, 384, 6, 5, 256),         # tables of 128 entries and of 8
+    (20, 2016, 128, 48, torch.bfloat16, 512, 4, 3, 128), (24, 2048, 128, 16, torch.float16, 704, 3, 2, 512),         # ... partitions of at least 512 tokens
+    (7, 8192, 128, 16, torch.bfloat16, 512, 16, 16, 256), (24, 8192, 128, 16, torch.float16, 1024, 8, 8, 512),       # wide tables of more than 128 entries ...
+    (24, 8192, 64, 128, torch.bfloat16, 1024, 8, 8, 512), (9, 6144, 64, 256, torch.float16, 768, 8, 8, 512)])        # ... and of less
+def test_partitions_as_long_as_the_contexts_ask_for(batch, width, d, bs, dtype, part, parts, spread, least):
+    """Sequences of a call whose partitions follow their own lengths: at, in front of and past every length that one partition, as many partitions as there
+    are to be, of a multiple of 64 tokens each, and partitions of the plan's length take, up to the table's."""
+    sizes = (batch, 16, 8, d, width // bs, bs, dtype)
+    assert paged_decode_plan(*sizes) == (part, parts, 4)
+    of = lambda ctx: paged_decode_partition(ctx, *sizes)
+    assert of(1) == least < part == of(width) and of(spread * (least + 64)) == least + 64 and of(spread * (least + 64) + 1) > of(spread * (least + 64) - 64 * spread) == least
+    edges = {n + by for n in (64, 128, least, 2 * least, spread * least, spread * (least + 64), part, 2 * part, spread * part, parts * part, 700) for by in (-1, 0, 1)}
+    edges = sorted(n for n in edges | {1, width - 1, width} if 0 < n <= width)
     for at in range(0, len(edges), batch):
         ctx_list = (edges[at:at + batch] + [0, 300] * batch)[:batch]
         q, kc, vc, tables, ctx = make_paged_case(at + d, 0, 0, 0, 16, 8, d, bs, dtype=dtype, ctx_list=ctx_list)

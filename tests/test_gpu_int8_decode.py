@@ -11,7 +11,7 @@ import torch
 
 import oracle
 from helpers import error_stats, half_step, make_paged_case
-from minivllm_amd.layers.attention import paged_attention_decode_int8, paged_decode_plan, store_kvcache_int8
+from minivllm_amd.layers.attention import paged_attention_decode_int8, paged_decode_partition, paged_decode_plan, store_kvcache_int8
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -125,13 +125,17 @@ def test_int8_both_grid_forms(hq, hkv, bs, d, form):
     assert torch.isfinite(got).all() and excess <= 2e-2 and mean <= 2e-3, (mx, excess, mean)
 
 
-@pytest.mark.parametrize("batch,width,d,bs", [(12, 2048, 128, 16), (20, 2016, 64, 48), (9, 4096, 128, 16), (20, 8192, 64, 32)])
-def test_int8_partitions_as_long_as_the_contexts_ask_for(batch, width, d, bs):
+@pytest.mark.parametrize("batch,width,d,bs,part,parts,spread,least", [
+    (12, 2048, 128, 16, 384, 6, 5, 256), (20, 2016, 64, 48, 512, 4, 3, 256), (7, 8192, 128, 16, 512, 16, 16, 256), (7, 8192, 64, 16, 512, 16, 16, 256),
+    (22, 6144, 128, 16, 768, 8, 8, 512), (16, 6144, 64, 256, 768, 8, 8, 512)])
+def test_int8_partitions_as_long_as_the_contexts_ask_for(batch, width, d, bs, part, parts, spread, least):
     """As test_partitions_as_long_as_the_contexts_ask_for of the 16-bit cache."""
-    part, parts, waves = paged_decode_plan(batch, 16, 8, d, width // bs, bs, torch.bfloat16, int8_cache=True)
-    assert parts > 1 and waves == 4 and part >= 256
-    edges = [1, 63, 64, 65, 255, 256, 257, 511, 512, 513, 256 * parts, 256 * parts + 1, 700, 1030, part * parts]
-    edges = [min(n, width) for n in edges] + [width - 1, width]
+    sizes = (batch, 16, 8, d, width // bs, bs, torch.bfloat16, True)
+    assert paged_decode_plan(*sizes) == (part, parts, 4)
+    of = lambda ctx: paged_decode_partition(ctx, *sizes)
+    assert of(1) == least < part == of(width) and of(spread * (least + 64)) == least + 64 and of(spread * (least + 64) + 1) > of(spread * (least + 64) - 64 * spread) == least
+    edges = {n + by for n in (64, least, 2 * least, spread * least, spread * (least + 64), part, spread * part, parts * part) for by in (-1, 0, 1)}
+    edges = sorted(n for n in edges | {1, 700, width - 1, width} if 0 < n <= width)
     for at in range(0, len(edges), batch):
         ctx_list = (edges[at:at + batch] + [129, 300] * batch)[:batch]
         q, ck, cv, sk, sv, tables, ctx = _quantised_case(at + d, 0, 0, 0, 16, 8, d, bs, ctx_list=ctx_list)
