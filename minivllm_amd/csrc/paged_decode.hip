@@ -1582,8 +1582,7 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(const DecodeArgs a) 
   if (h >= a.num_heads) return;
   const int D = a.head_dim;
   const int ctx = (int)load_ctx(a, b);
-  const int part_tokens = part_tokens_of(a, ctx);
-  int np = (ctx + part_tokens - 1) / part_tokens;
+  int np = (ctx + a.part_tokens - 1) / a.part_tokens;       // (partitions of other lengths: aligned outputs, heads of 64 and 128)
   if (np > a.num_parts) np = a.num_parts;
   if (np <= 1) return;                               // written directly by the partition-0 workgroup
   const int64_t slot0 = ((int64_t)b * a.num_parts) * a.num_heads + h;
@@ -1687,10 +1686,14 @@ static void launch_decode_reduce(const DecodeArgs& a, hipStream_t stream) {
   const auto grid = [&](int lanes) { return dim3((unsigned)((a.num_heads + 256 / lanes - 1) / (256 / lanes)), (unsigned)a.batch); };
   // the 16-byte loads and 8- or 16-byte stores need the output rows aligned (the workspace is checked to be)
   const bool vec = (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0;
-  const bool ahead = vec && a.spread != 0 && (int64_t)a.max_num_blocks * a.block_size > kSplitNarrowCtx;
-  if (ahead && a.head_dim == 128) decode_reduce_vec_kernel<T, 128, true><<<grid(32), block, 0, stream>>>(a);
-  else if (ahead && a.head_dim == 64) decode_reduce_vec_kernel<T, 64, true><<<grid(16), block, 0, stream>>>(a);
-  else if (vec && a.head_dim == 128) decode_reduce_vec_kernel<T, 128, false><<<grid(32), block, 0, stream>>>(a);
+  if constexpr (sizeof(T) == 2) {                    // (partitions that follow the contexts are of 16-bit queries)
+    if (vec && a.spread != 0 && (int64_t)a.max_num_blocks * a.block_size > kSplitNarrowCtx) {
+      if (a.head_dim == 128) decode_reduce_vec_kernel<T, 128, true><<<grid(32), block, 0, stream>>>(a);
+      else decode_reduce_vec_kernel<T, 64, true><<<grid(16), block, 0, stream>>>(a);
+      return;
+    }
+  }
+  if (vec && a.head_dim == 128) decode_reduce_vec_kernel<T, 128, false><<<grid(32), block, 0, stream>>>(a);
   else if (vec && a.head_dim == 64) decode_reduce_vec_kernel<T, 64, false><<<grid(16), block, 0, stream>>>(a);
   else if (vec && a.head_dim == 256) decode_reduce_vec_kernel<T, 256, false><<<grid(64), block, 0, stream>>>(a);
   else if (vec && a.head_dim == 32) decode_reduce_vec_kernel<T, 32, false><<<grid(8), block, 0, stream>>>(a);
