@@ -769,6 +769,12 @@ int mvllm_moe_linear_shared(void* out, int64_t out_row_stride, const void* x, in
                             const int32_t* ids, void* plan, int64_t pairs, int experts, int N, int K, int per_token, int glu,
                             void* shared_out, int64_t shared_out_row_stride, const void* shared_x, int64_t shared_x_row_stride,
                             const void* shared_w, int shared_rows, int shared_N, int shared_K, int dtype, void* stream);
+/*
+ * mvllm_moe_linear_tiles: the rows and weight rows of the tiles that a bf16 product over a plan runs on, its outputs' row stride a multiple
+ *   of 8 (shared_rows 0: without a shared expert).  Pure host arithmetic.
+ */
+int mvllm_moe_linear_tiles(int64_t pairs, int experts, int N, int K, int shared_rows, int shared_N, int shared_K,
+                           int* rows, int* weight_rows);
 
 /*
  * ... and for models whose router is a softmax and whose experts have a clamped gate:

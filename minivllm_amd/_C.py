@@ -140,6 +140,7 @@ SIGNATURES = {
     "mvllm_moe_linear": (c_int, [c_void_p, c_int64, c_void_p, c_int64] + [c_void_p] * 3 + [c_int64] + [c_int] * 6 + [c_void_p]),
     "mvllm_moe_linear_shared": (c_int, [c_void_p, c_int64, c_void_p, c_int64] + [c_void_p] * 3 + [c_int64] + [c_int] * 5 +
                                 [c_void_p, c_int64, c_void_p, c_int64, c_void_p] + [c_int] * 4 + [c_void_p]),
+    "mvllm_moe_linear_tiles": (c_int, [c_int64] + [c_int] * 6 + [ctypes.POINTER(c_int)] * 2),
     "mvllm_mlstm_output": (c_int, [c_void_p] * 5 + [c_int64, c_float] + [c_void_p] * 5 + [c_int64, c_int, c_int, c_int,
                                                                                       c_void_p]),
     "mvllm_moe_route_softmax": (c_int, [c_void_p] * 3 + [c_int64, c_void_p, c_int64] + [c_int] * 4 + [c_void_p]),

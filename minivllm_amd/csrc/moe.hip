@@ -1031,10 +1031,11 @@ static int tile_rows(int64_t pairs, int experts) {
 }
 static int64_t max_tiles(int64_t pairs, int experts, int rows) { return (pairs + rows - 1) / rows + experts; }
 // Whether a product's weights go in 64 rows per workgroup instead of 128, by the workgroups of 128 to be expected where routing is even.  Up to 160 these leave CUs
-// idle: 1.0 to 2.2 times as fast at K of 768 to 14336 (1.27 and more up to 128 workgroups).  From 160 to 248 both fill the chip about once, 0.95 to 1.10.
-// From 248 to 384 a part of the CUs has two of 128 and the others one, while all have two of 64: 1.0 to 1.19 (K 768: 1.05 up to 328, 0.93 at 396).  At 400 to 500
-// 0.91 to 1.03, and above it 0.98 to 1.1 where there are many steps of K, 0.8 to 0.95 where there are few.  K of 512 never (0.65 to 0.85): six buffers'
-// start and the sums at the end are longer than its eight steps.  More than four pairs per expert were not faster (mixtures of 64 experts: 0.98 at six, 0.88 at 28).
+// idle: 1.03 to 2.2 times as fast at K of 768 to 14336 (1.27 and more up to 128 workgroups).  From 160 to 248 both fill the chip about once, 0.95 to 1.10.
+// From 248 to 384 a part of the CUs has two of 128 and the others one, while all have two of 64: 1.03 to 1.19 (K 768: 1.05 up to 328, 0.93 at 396).  At 400 to 500
+// 0.89 to 1.04, and above it 0.96 to 1.1 where there are many steps of K, 0.8 to 0.95 where there are few.  More than four pairs per expert were not faster (mixtures
+// of 64 experts: 0.98 at six, 0.88 at 28).  With the gate it is 0.01 to 0.04 more, with the clamped one 0.01 to 0.08.  K of 512 to 704: 1.2
+// to 1.45 up to 115 workgroups too, but 0.78 to 1.06 from 163 on (six buffers' start and the sums at the end are longer than eight to eleven steps): not taken.
 static bool narrow_pays(int64_t pairs, int experts, int N, int K, const ExpertLinearArgs::Shared& shared) {
   const int least_k = shared.rows != 0 ? std::min(K, shared.K) : K;
   if (pairs > 4 * (int64_t)experts || least_k < 768) return false;
@@ -1144,6 +1145,22 @@ extern "C" int mvllm_moe_plan(void* plan, size_t plan_bytes, const int32_t* ids,
 }
 
 // f(a kGlu as a constant)
+// What a bf16 product over sorted pairs runs on.
+struct ExpertForm {
+  int rows, weights;           // of a tile
+  bool second, one_block;      // (second: of the plan's tiles of 256 rows where it has both; one_block: no expert has more than 32 rows)
+};
+static ExpertForm expert_form(int64_t pairs, int experts, int N, int K, const ExpertLinearArgs::Shared& shared, bool wide_stores) {
+  const int plan_rows = tile_rows(pairs, experts);
+  ExpertForm f;
+  f.second = plan_rows == 128 && wide_stores && large_tiles_pay(pairs, experts, N);
+  f.rows = f.second ? 256 : plan_rows;
+  const bool narrow = f.rows == 64 && narrow_pays(pairs, experts, N, K, shared);
+  f.one_block = narrow && pairs <= 32 && shared.rows <= 32;
+  f.weights = f.rows == 256 ? 256 : narrow ? 64 : 128;
+  return f;
+}
+
 template <typename F> static void with_glu(int glu, F f) {
   if (glu == kClampedGlu) f(std::integral_constant<int, kClampedGlu>{});
   else if (glu == kSiluGlu) f(std::integral_constant<int, kSiluGlu>{});
@@ -1194,12 +1211,10 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
   const PlanArgs p = plan_parts_of(plan, ids, pairs, experts);
   a.sorted_pair = p.sorted_pair; a.row_start = p.row_start;
   if (dtype == MVLLM_BF16) {
-    const bool second = p.tile_rows == 128 && out_row_stride % 8 == 0 && large_tiles_pay(pairs, experts, N);
-    const int rows = second ? 256 : p.tile_rows;
-    a.tile_expert = p.tiles[second].expert; a.tile_row = p.tiles[second].row; a.num_tiles = p.tiles[second].num;
+    const ExpertForm form = expert_form(pairs, experts, N, K, shared, out_row_stride % 8 == 0);
+    const int rows = form.rows, tile = form.weights;
+    a.tile_expert = p.tiles[form.second].expert; a.tile_row = p.tiles[form.second].row; a.num_tiles = p.tiles[form.second].num;
     a.max_tiles = (int)max_tiles(pairs, experts, rows);
-    const bool narrow = rows == 64 && narrow_pays(pairs, experts, N, K, shared), one_block = pairs <= 32 && shared.rows <= 32;      // (one: no expert has more rows)
-    const int tile = rows == 256 ? 256 : narrow ? 64 : 128;              // weight rows
     a.n_tiles = (N + tile - 1) / tile;
     if (rows == 256 && out_row_stride % 8 != 0) return MVLLM_ERR_UNSUPPORTED;
     const int64_t x_rows = per_token ? (pairs + per_token - 1) / per_token : pairs, x_bytes = ((x_rows - 1) * x_row_stride + K) * 2;
@@ -1222,8 +1237,8 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
       constexpr int kGlu = decltype(G)::value;
       if (rows == 256) moe_linear_large_kernel<kGlu><<<dim3(8u * (unsigned)a.groups), dim3(256), 0, s>>>(a);
       else if (rows == 128) moe_linear_many_kernel<kGlu, 4><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
-      else if (narrow && one_block) moe_linear_narrow_kernel<kGlu, 1><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
-      else if (narrow) moe_linear_narrow_kernel<kGlu, 2><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      else if (form.one_block) moe_linear_narrow_kernel<kGlu, 1><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+      else if (tile == 64) moe_linear_narrow_kernel<kGlu, 2><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
       else moe_linear_many_kernel<kGlu, 2><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
     });
   } else {
@@ -1232,6 +1247,16 @@ static int expert_linear(void* out, int64_t out_row_stride, const void* x, int64
     with_glu(glu, [&](auto G) { moe_linear_any_kernel<float, decltype(G)::value><<<grid, dim3(256), 0, s>>>(a); });
   }
   return launch_status();
+}
+
+extern "C" int mvllm_moe_linear_tiles(int64_t pairs, int experts, int N, int K, int shared_rows, int shared_N, int shared_K, int* rows, int* weight_rows) {
+  if (pairs <= 0 || experts <= 0 || N <= 0 || K <= 0 || shared_rows < 0 || (shared_rows > 0 && (shared_N <= 0 || shared_K <= 0))) return MVLLM_ERR_BAD_SHAPE;
+  ExpertLinearArgs::Shared shared = {};
+  shared.rows = shared_rows; shared.N = shared_N; shared.K = shared_K;
+  const ExpertForm f = expert_form(pairs, experts, N, K, shared, true);
+  if (rows) *rows = f.one_block ? 32 : f.rows;
+  if (weight_rows) *weight_rows = f.weights;
+  return MVLLM_OK;
 }
 
 extern "C" int mvllm_moe_linear(void* out, int64_t out_row_stride, const void* x, int64_t x_row_stride, const void* w,

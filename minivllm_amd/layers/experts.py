@@ -4,6 +4,7 @@ The module returns the experts' results unsummed (``ExpertOutput``): whoever add
 them with their weights (``layers.fused.stream_norm``)."""
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from typing import Optional
 
@@ -17,7 +18,7 @@ from minivllm_amd.layers.recurrent import gate_linear
 from minivllm_amd.models.qwen3 import Qwen3MLP, _as_built
 from minivllm_amd.utils.padding import pad_to, round_up
 
-__all__ = ["ExpertOutput", "ExpertPlan", "SparseExperts", "moe_route", "moe_route_softmax", "moe_plan", "moe_linear", "interleave_gate_up"]
+__all__ = ["ExpertOutput", "ExpertPlan", "SparseExperts", "moe_route", "moe_route_softmax", "moe_plan", "moe_linear", "moe_linear_tiles", "interleave_gate_up"]
 
 FEW_PAIRS = 16             # (token, choice) pairs up to which the products run without a plan ...
 # ... where rows are short and no shared expert can join the launches: without one every expert has workgroups that look for its rows, with one only those that have
@@ -147,6 +148,14 @@ def moe_linear(x: torch.Tensor, weight: torch.Tensor, ids: torch.Tensor, plan: E
         st = _C.load().mvllm_moe_linear(*head, int(glu), *tail)
     _C.check(st, "moe_linear")
     return out
+
+
+def moe_linear_tiles(pairs: int, experts: int, n: int, k: int, shared: tuple | None = None) -> tuple:
+    """(rows, weight rows) of the tiles that a bf16 ``moe_linear`` of these sizes runs on with a plan, ``shared`` = (rows, N, K); host arithmetic only."""
+    out = [ctypes.c_int(0), ctypes.c_int(0)]
+    st = _C.load().mvllm_moe_linear_tiles(pairs, experts, n, k, *(shared or (0, 0, 0)), *(ctypes.byref(v) for v in out))
+    _C.check(st, "moe_linear_tiles")
+    return tuple(v.value for v in out)
 
 
 def interleave_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:

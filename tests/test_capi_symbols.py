@@ -40,7 +40,7 @@ def test_header_declares_expected_entry_points():
               "mvllm_stream_embed_norm", "mvllm_stream_norm", "mvllm_decay_memory_recurrent", "mvllm_decay_memory_chunked",
               "mvllm_decay_memory_chunked_workspace_bytes", "mvllm_gated_row_norm", "mvllm_latent_norm_store",
               "mvllm_head_linear", "mvllm_latent_decode", "mvllm_latent_decode_workspace_bytes", "mvllm_moe_route",
-              "mvllm_moe_plan", "mvllm_moe_plan_bytes", "mvllm_moe_linear", "mvllm_moe_linear_shared",
+              "mvllm_moe_plan", "mvllm_moe_plan_bytes", "mvllm_moe_linear", "mvllm_moe_linear_shared", "mvllm_moe_linear_tiles",
               "mvllm_moe_route_softmax", "mvllm_moe_linear_clamped", "mvllm_gated_unit", "mvllm_stream_norm_identity", "mvllm_window_prefill",
               "mvllm_window_decode_workspace_bytes", "mvllm_window_decode", "mvllm_latent_rope_store", "mvllm_head_rope", "mvllm_copy_rows",
               "mvllm_head_norm_rope_store", "mvllm_window_decode_split", "mvllm_gelu_tanh", "mvllm_linear_small_m_gelu",
@@ -213,6 +213,25 @@ def test_decode_partitions_of_a_sequence():
     for bad in (-1, 2049):
         with pytest.raises(ValueError):
             of(bad, 12, 2048)
+
+
+def test_tiles_of_products_over_sorted_pairs():
+    """Which tiles a product runs on: edges of every rule."""
+    from minivllm_amd.layers.experts import moe_linear_tiles as tiles
+    _lib().load()
+    assert tiles(32, 8, 1536, 2048) == (32, 64) and tiles(33, 9, 1536, 2048) == (64, 64)          # one block of rows
+    assert tiles(6, 64, 1536, 768) == (32, 64) and tiles(6, 64, 1536, 704) == (64, 128)           # K
+    assert tiles(6, 64, 1536, 2048, (1, 64, 704)) == (64, 128) and tiles(6, 64, 1536, 2048, (1, 64, 768)) == (32, 64)
+    assert tiles(4 * 8, 8, 512, 2048) == (32, 64) and tiles(4 * 8 + 1, 8, 512, 2048) == (64, 128) # pairs per expert
+    assert tiles(1, 1, 160 * 128, 768) == (32, 64) and tiles(1, 1, 161 * 128, 768) == (64, 128)   # workgroups: up to 160,
+    assert tiles(1, 1, 247 * 128, 768) == (64, 128) and tiles(1, 1, 248 * 128, 768) == (32, 64)   # ... from 248
+    assert tiles(1, 1, 328 * 128, 768) == (32, 64) and tiles(1, 1, 329 * 128, 768) == (64, 128)
+    assert tiles(1, 1, 384 * 128, 1024) == (32, 64) and tiles(1, 1, 385 * 128, 1024) == (64, 128)
+    assert tiles(1, 1, 150 * 128, 1024, (1, 10 * 128, 1024)) == (32, 64) and tiles(1, 1, 150 * 128, 1024, (65, 6 * 128, 1024)) == (64, 128)
+    assert tiles(48 * 64, 64, 1536, 2048) == (64, 128) and tiles(48 * 64 + 1, 64, 1536, 2048) == (256, 256)      # rows per expert, large tiles for every CU
+    assert tiles(48 * 16 + 1, 16, 1024, 2048) == (128, 128) and tiles(384 * 16, 16, 1024, 2048) == (256, 256)
+    with pytest.raises(ValueError):
+        tiles(0, 1, 64, 64)
 
 
 def test_decode_plan_is_host_arithmetic():

@@ -12,7 +12,7 @@ from minivllm_amd.engine.hybrid_runner import HybridModelRunner
 from minivllm_amd.engine.ragged import ragged_step
 from minivllm_amd.engine.sequence import Sequence
 from minivllm_amd import _C
-from minivllm_amd.layers.experts import ExpertOutput, SparseExperts, interleave_gate_up, moe_linear, moe_plan, moe_route
+from minivllm_amd.layers.experts import ExpertOutput, SparseExperts, interleave_gate_up, moe_linear, moe_linear_tiles, moe_plan, moe_route
 from minivllm_amd.layers.fused import stream_embed_norm, stream_norm
 from minivllm_amd.layers.latent import head_linear, latent_decode, latent_norm_store, latent_width
 from minivllm_amd.layers.mixers import DecayMemory, LatentAttention
@@ -664,7 +664,7 @@ def test_moe_linear_shared(rows, top, experts, n, k, sn, sk, glu):
     (32, 1, 8, 192, 832),                                                 # experts of up to all 32 rows
     (33, 1, 9, 192, 832),                                                 # tiles of 64 rows
     (66, 1, 17, 1040, 768),                                               # ... and an expert of 65 rows: two tiles
-    (40, 3, 30, 960, 4096),
+    (40, 3, 30, 576, 4096), (40, 3, 30, 1152, 4096),                      # a turned K in 64 rows, on both sides of the gap
 ])
 @pytest.mark.parametrize("glu,side", [(False, None), (True, None), ((1.5, 7.0, 1.0), None), (False, (64, 768)), (True, (64, 768)), (False, (208, 2112)), (True, (208, 2112))])
 def test_moe_linear_few_workgroups(rows, top, experts, n, k, glu, side):
@@ -673,6 +673,7 @@ def test_moe_linear_few_workgroups(rows, top, experts, n, k, glu, side):
     g = torch.Generator(device=DEV).manual_seed(rows + n + k)
     normal = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).bfloat16()
     n = n // 64 * 64 if glu else n
+    assert moe_linear_tiles(rows * top, experts, n, k, None if side is None else (rows, *side)) == (32 if rows * top <= 32 else 64, 64)
     ids = torch.randint(0, experts, (rows, top), generator=g, device=DEV).int()
     ids[:, 0] = experts - 1                                               # (in the 66-row case one id more, of nobody)
     if rows == 66:
