@@ -322,11 +322,14 @@ int mvllm_prefill_paged_int8_split(void* out, const void* q,
  * row tile cut into ranges of `range_tiles` tiles of 64 (an even number), walked side by side: 16-bit element types, head_dim 64 and
  * 128, block_size a multiple of 16, up to 64 sequences.  Partial results are fp32.  sink: fp32 [Hq] or NULL.
  *   _ranges_plan: the range the library would use for a batch of these sizes; 0 = run the calls above.
+ *   _ranges_groups: the groups of four waves that share a range of these tiles, 1 or 2; 0: the call is not built for these sizes.
  *   _ranges_workspace_bytes: 16-byte aligned device memory the call needs.
  * max_kv_len: the host's upper bound of every sequence's key count (keys past it are walked by the last range).
  */
 int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads,
                               int head_dim, int block_size, int dtype);
+int mvllm_prefill_ranges_groups(int num_seqs, int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads,
+                                int head_dim, int block_size, int dtype, int range_tiles);
 size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim,
                                             int range_tiles);
 int mvllm_prefill_ranges(void* out, const void* q, const void* k, const void* v, const int32_t* block_tables,

@@ -61,6 +61,7 @@ SIGNATURES = {
     "mvllm_prefill_paged_split_workspace_bytes": (c_size_t, [c_int, c_int64] + [c_int] * 7),
     "mvllm_prefill_paged_split": (c_int, [c_void_p] * 5 + [c_int, c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int,
                                             c_int, c_int64, c_float, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "mvllm_prefill_ranges_groups": (c_int, [c_int, c_int64] + [c_int] * 7),
     "mvllm_prefill_ranges_plan": (c_int, [c_int, c_int64] + [c_int] * 6),
     "mvllm_prefill_ranges_workspace_bytes": (c_size_t, [c_int64] + [c_int] * 4),
     "mvllm_prefill_ranges": (c_int, [c_void_p] * 5 + [c_int, c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int, c_int,

@@ -609,6 +609,14 @@ extern "C" size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, i
   return ranges < 2 ? 0 : (size_t)ranges * total_q_tokens * num_heads * (head_dim + 1) * sizeof(float);
 }
 
+extern "C" int mvllm_prefill_ranges_groups(int num_seqs, int64_t total_q_tokens, int max_kv_len, int num_heads, int num_kv_heads, int head_dim,
+                                           int block_size, int dtype, int range_tiles) {
+  if (range_tiles <= 0 || range_tiles % 2 != 0 ||
+      !ranges_shape_ok(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size, dtype))
+    return 0;
+  return pairs_pay(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim, block_size > 0, range_tiles) ? 2 : 1;
+}
+
 static int run_ranges(void* out, const void* q, const void* k, const void* v, const int32_t* block_tables, int max_num_blocks,
                       const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int num_seqs, int64_t total_q_tokens, int max_kv_len,
                       int num_heads, int num_kv_heads, int head_dim, int block_size, int64_t num_blocks, float scale, const float* sink,

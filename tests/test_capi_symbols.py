@@ -30,7 +30,7 @@ def test_header_declares_expected_entry_points():
               "mvllm_paged_decode_int8", "mvllm_paged_decode_noalloc", "mvllm_paged_decode_workspace_bytes", "mvllm_paged_decode_plan", "mvllm_paged_decode_partition", "mvllm_prefill_plan", "mvllm_prefill_varlen",
               "mvllm_prefill_paged", "mvllm_prefill_paged_int8", "mvllm_prefill_paged_int8_staged", "mvllm_prefill_paged_staged", "mvllm_prefill_paged_staged_workspace_bytes", "mvllm_prefill_paged_split", "mvllm_prefill_paged_int8_split", "mvllm_prefill_paged_split_plan", "mvllm_prefill_paged_split_workspace_bytes", "mvllm_qk_norm_rope_store", "mvllm_sample_tokens", "mvllm_sample_tokens_dev_offset", "mvllm_decode_advance", "mvllm_sample_tokens_workspace_bytes",
               "mvllm_add_rms_norm", "mvllm_linear_small_m", "mvllm_norm_linear_small_m", "mvllm_linear_small_m_plan",
-              "mvllm_linear_small_m_split", "mvllm_linear_small_m_split_bytes", "mvllm_prefill_ranges", "mvllm_prefill_ranges_plan", "mvllm_prefill_store",
+              "mvllm_linear_small_m_split", "mvllm_linear_small_m_split_bytes", "mvllm_prefill_ranges", "mvllm_prefill_ranges_plan", "mvllm_prefill_ranges_groups", "mvllm_prefill_store",
               "mvllm_prefill_ranges_workspace_bytes", "mvllm_mlstm_chunked_output",
               "mvllm_lm_head_sample", "mvllm_lm_head_sample_workspace_bytes",
               "mvllm_paged_decode_sink", "mvllm_prefill_varlen_sink", "mvllm_prefill_paged_sink",

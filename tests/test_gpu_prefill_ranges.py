@@ -28,6 +28,12 @@ def _run(c, hq, hkv, d, bs, tiles, max_k, paged, sink=None):
     return out.cpu()
 
 
+def _groups(c, hq, hkv, d, bs, tiles, max_k, paged, dtype=torch.bfloat16):
+    """Groups of waves per range that ``_run`` of the same call runs on."""
+    return _C.load().mvllm_prefill_ranges_groups(len(c["cu_k"]) - 1, len(c["q_new"] if paged else c["q"]), max_k, hq, hkv, d, bs if paged else 0,
+                                                 _C.dtype_code(dtype), tiles)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,d,bs,lengths,cached,tiles", [
     (8, 2, 128, 16, [128, 129, 127, 1], [64, 100, 126, 0], 2),         # a last tile that ends a range, starts one, falls short of it
@@ -65,19 +71,22 @@ def test_the_diagonal_at_every_place_of_a_tile(hq, hkv, d, tiles, new):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("hq,hkv,d,lengths,cached,tiles", [
-    (8, 2, 128, [5000, 2700, 64], [4900, 2650, 0], 40),                # two ranges, one of an odd number of tiles, one of a single tile
-    (8, 4, 64, [3400, 130, 0, 3], [3300, 70, 0, 0], 28),
-    (5, 5, 128, [3000, 1700], [2800, 1699], 24),                       # one head per workgroup
-    (2, 1, 128, [2700, 40], [2000, 10], 14),                           # packed: 14 tiles and 256 workgroups
-    (2, 1, 64, [2200, 900], [100, 0], 36),                             # whole
+@pytest.mark.parametrize("hq,hkv,d,lengths,cached,tiles,groups", [
+    (8, 2, 128, [5000, 2700, 64], [4900, 2650, 0], 40, (2, 1)),        # two ranges, one of an odd number of tiles, one of a single tile
+    (8, 4, 64, [3400, 130, 0, 3], [3300, 70, 0, 0], 28, (2, 1)),
+    (5, 5, 128, [3000, 1700], [2800, 1699], 24, (2, 1)),               # one head per workgroup
+    (2, 1, 128, [2700, 40], [2000, 10], 14, (1, 2)),                   # packed: 14 tiles and 256 workgroups
+    (3, 3, 64, [1900, 700, 0], [0, 0, 0], 14, (2, 2)),                 # ... one head per workgroup, two ranges and one
+    (2, 1, 64, [2200, 900], [100, 0], 36, (2, 2)),                     # whole
 ])
 @pytest.mark.parametrize("paged", [True, False])
-def test_prefill_over_key_ranges_in_two_groups(hq, hkv, d, lengths, cached, tiles, paged, dtype):
-    """Few workgroups with long ranges: two groups of waves walk the halves of a range, whose sums meet in LDS."""
+def test_prefill_over_key_ranges_in_two_groups(hq, hkv, d, lengths, cached, tiles, groups, paged, dtype):
+    """Few workgroups with long ranges: two groups of waves walk the halves of a range, whose sums meet in LDS.  groups: what these sizes run on, over a
+    cache and packed."""
     c = make_paged_prefill_case(71, lengths, cached, hq, hkv, d, 16, dtype=dtype)
     want = oracle.prefill_paged_oracle(c["q_new"].float(), torch.nan_to_num(c["k_cache"].float()), torch.nan_to_num(c["v_cache"].float()),
                                        c["block_tables"], c["cu_q"], c["cu_k"], 1 / math.sqrt(d), hq, hkv, d, 16)
+    assert _groups(c, hq, hkv, d, 16, tiles, max(lengths), paged, dtype) == groups[not paged]
     got = _run(c, hq, hkv, d, 16, tiles, max(lengths), paged)
     mx, mean = error_stats(got if paged else got[c["new_rows"]], want)
     assert torch.isfinite(got.float()).all() and mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (mx, mean)
@@ -93,6 +102,7 @@ def test_the_diagonal_at_every_place_of_a_tile_in_two_groups(hq, hkv, d, new):
     want = oracle.prefill_paged_oracle(c["q_new"].float(), torch.nan_to_num(c["k_cache"].float()), torch.nan_to_num(c["v_cache"].float()),
                                        c["block_tables"], c["cu_q"], c["cu_k"], 1 / math.sqrt(d), hq, hkv, d, 16)
     for paged in (True, False):
+        assert _groups(c, hq, hkv, d, 16, 64, 4096, paged) == 2
         got = _run(c, hq, hkv, d, 16, 64, 4096, paged)
         mx, mean = error_stats(got if paged else got[c["new_rows"]], want)
         assert mx <= MAX_ABS_16 and mean <= MEAN_ABS_16, (paged, mx, mean)
