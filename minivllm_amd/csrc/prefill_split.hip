@@ -490,7 +490,9 @@ static bool pairs_pay(int num_seqs, int64_t total_q, int64_t max_kv_len, int num
   }
   return x >= 8 && b.wgs * (float)n <= 256.f && chain_us(b, x, true) + (n > 1 ? 1.f : 0.f) < chain_us(b, x, false);
 }
-static int64_t cached_range(const CachedBatch& b, float part_us, bool whole) {       // whole: what is not in pairs is one range
+// whole: what is not in pairs is one range.  apart: what is one range goes to another kernel, so that there is no pair of one either (taken for one, batches of
+// 12 to 20 tiles of 64 dims lost their ranges: 552 rows behind as many 20.5 / 23.2 us, 324 behind 864, 16 heads 19.3 / 26.1).
+static int64_t cached_range(const CachedBatch& b, float part_us, bool whole, bool apart) {
   const int64_t tiles = b.tiles;
   const float per_range = 0.6f + 0.81f * part_us;
   int64_t p = (tiles + 1) / 2 * 2;
@@ -504,7 +506,7 @@ static int64_t cached_range(const CachedBatch& b, float part_us, bool whole) {  
       best = gain;
       p = x;
     }
-    if (b.wgs * (float)n > 256.f || std::min(x, tiles) < 8) continue;
+    if (b.wgs * (float)n > 256.f || std::min(x, tiles) < 8 || (apart && n == 1)) continue;
     const float gain_pairs = from - chain_us(b, std::min(x, tiles), true) - us - (n > 1 ? 1.f : 0.f);
     if (gain_pairs > best_pairs && gain_pairs > best) {
       best = best_pairs = gain_pairs;
@@ -585,9 +587,10 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
     if (four && crowded && !paged && fresh >= 0.87f && busiest_cu(even, num_seqs, fresh) > (num_seqs <= 3 ? 1.87f : 2.9f)) return 0;
   }
   int64_t p = (tiles + 1) / 2 * 2;
+  const bool apart = wgs <= 192 && (head_dim == 64 ? wgs < (four ? 48 : 80) : odd && tiles < 8);
   if (paged)
     p = cached_range(cached_batch(num_seqs, total_q_tokens, max_kv_len, num_heads, num_kv_heads, head_dim),
-                     8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f, wgs > 192 && num_seqs < 5);
+                     8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f, wgs > 192 && num_seqs < 5, apart);
   if (wgs > 192) return (four || head_dim == 64) && tiles > 112 ? 0 : (int)p;
   const float per_tile = head_dim == 64 ? 0.8f : 0.9f, per_range = 0.3f + 0.7f * 8.f * (float)total_q_tokens * (float)(num_heads * head_dim) / 4.5e6f;
   float best = 3.f;
@@ -600,7 +603,7 @@ extern "C" int mvllm_prefill_ranges_plan(int num_seqs, int64_t total_q_tokens, i
       p = x;
     }
   }
-  return p >= tiles && (head_dim == 64 ? wgs < (four ? 48 : 80) : odd && tiles < 8) ? 0 : (int)p;
+  return p >= tiles && apart ? 0 : (int)p;
 }
 
 extern "C" size_t mvllm_prefill_ranges_workspace_bytes(int64_t total_q_tokens, int max_kv_len, int num_heads, int head_dim, int range_tiles) {

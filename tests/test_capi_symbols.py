@@ -97,6 +97,14 @@ def test_prefill_ranges_plan_looks_at_the_busiest_cu():
     assert plan(4, 1672, 1910, *four, *paged) == 30                                                    # long
 
 
+def test_prefill_ranges_plan_keeps_ranges_where_whole_ones_go_elsewhere():
+    """Few workgroups of heads of 64 over a cache: one range is another kernel's, so ranges are not given up for one in two groups."""
+    plan = _lib().load().mvllm_prefill_ranges_plan
+    for rows, seqs, keys, heads, tiles in [(552, 1, 1104, 16, 6), (799, 2, 1040, 8, 6), (324, 1, 1188, 16, 4), (228, 4, 928, 16, 4)]:
+        kv = 8 if heads == 16 and rows != 324 else heads
+        assert plan(seqs, rows, keys, heads, kv, 64, 16, 1) == tiles, (rows, seqs, keys)
+
+
 def test_prefill_ranges_plan_of_odd_head_groups():
     """Row tiles of 128 in both forms: packed batches go over only where the other form's places pass the chip's 512, cached ones for its
     empty places, for alike tiles or for keys cut into ranges."""
