@@ -225,7 +225,8 @@ class SparseExperts(nn.Module):
             return False
         # (a weight of a class of its own may hold other numbers than its memory, as quantized ones do)
         return (type(up) in (nn.Parameter, torch.Tensor) and type(down) in (nn.Parameter, torch.Tensor)
-                and m.gate_up.bias is None and m.gate_down.bias is None and up.dtype == down.dtype == h.dtype and up.is_contiguous() and down.is_contiguous()
+                and m.gate_up.bias is None and m.gate_down.bias is None and up.dtype == down.dtype == h.dtype and up.device == down.device == h.device
+                and up.is_contiguous() and down.is_contiguous()
                 and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0 and 2 * up.numel() < 1 << 31 and 2 * down.numel() < 1 << 31
                 and _span(h) < 1 << 31 and h.shape[0] * down.shape[1] < 1 << 31          # (offsets of 32 bits into weights and, unsigned, rows)
                 and up.shape[0] == 2 * down.shape[1] and up.shape[1] == h.shape[1] and down.shape[1] % 64 == 0 and down.shape[0] % 16 == 0)

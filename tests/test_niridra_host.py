@@ -157,6 +157,14 @@ def test_a_shared_expert_with_weights_of_their_own_class_is_called(which):
     assert isinstance(part.weight, Weight) and not m._shared_beside(h)
 
 
+@pytest.mark.parametrize("which", ["gate_up", "gate_down"])
+def test_a_shared_expert_on_another_device_is_called(which):
+    m, h = _with_shared(), torch.zeros(100, 128, dtype=torch.bfloat16)
+    part = getattr(m.shared, which)
+    part.weight = torch.nn.Parameter(part.weight.to("meta"), requires_grad=False)
+    assert not m._shared_beside(h)
+
+
 def _at_odd_address(weight):
     """The same numbers in a contiguous view that begins two bytes into a buffer."""
     flat = torch.empty(weight.numel() + 1, dtype=weight.dtype, device=weight.device)
