@@ -26,6 +26,7 @@ FEW_PAIRS = 16             # (token, choice) pairs up to which the products run 
 # 8 of 512 x 512 18.3 / 19.3 (with a shared expert 23.2 / 19.5); 8 of 768 x 768 23.9 / 17.8, of 128 x 2048 20.3 / 19.5, of 256 x 1024 18.8 / 17.5, 128 of them 21.9 / 19.6, eight rows
 # 28.6 / 21.0; top 6 of 64 of 768 x 2048 44 / 25, top 8 of 1280 x 4096 91 / 61; 8 of 14336 x 4096 197 / 126, eight rows 512 / 387.
 SHORT_ROWS = 768
+_PLAIN = (nn.Parameter, torch.Tensor)
 
 
 def _ptr(t):
@@ -215,21 +216,23 @@ class SparseExperts(nn.Module):
         """Whether the shared expert's products may be part of the experts' launches: not where it is not as built here, somebody hooked into it, or the
         launches do not take its sizes."""
         m = self.shared
-        if (m is None or self.glu is not True or h.dtype != torch.bfloat16 or h.dim() != 2 or h.shape[0] == 0 or _has_any_global_hook() or not _as_built(m, Qwen3MLP)
-                or not _as_built(m.gate_up, Linear) or not _as_built(m.gate_down, Linear) or not _as_built(m.activation, SiluAndMul)):
+        if (m is None or self.glu is not True or h.dtype != torch.bfloat16 or h.dim() != 2 or h.shape[0] == 0 or not self._beside_pays(h.shape[0])
+                or _has_any_global_hook() or not _as_built(m, Qwen3MLP)):
             return False
-        up, down = m.gate_up.weight, m.gate_down.weight
-        if not self._beside_pays(h.shape[0]):
+        gate_up, gate_down = m.gate_up, m.gate_down
+        if not _as_built(gate_up, Linear) or not _as_built(gate_down, Linear) or not _as_built(m.activation, SiluAndMul):
             return False
+        up, down = gate_up.weight, gate_down.weight
         if torch.is_grad_enabled() and (h.requires_grad or up.requires_grad or down.requires_grad):
             return False
         # (a weight of a class of its own may hold other numbers than its memory, as quantized ones do)
-        return (type(up) in (nn.Parameter, torch.Tensor) and type(down) in (nn.Parameter, torch.Tensor)
-                and m.gate_up.bias is None and m.gate_down.bias is None and up.dtype == down.dtype == h.dtype and up.device == down.device == h.device
-                and up.is_contiguous() and down.is_contiguous()
-                and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0 and 2 * up.numel() < 1 << 31 and 2 * down.numel() < 1 << 31
-                and _span(h) < 1 << 31 and h.shape[0] * down.shape[1] < 1 << 31          # (offsets of 32 bits into weights and, unsigned, rows)
-                and up.shape[0] == 2 * down.shape[1] and up.shape[1] == h.shape[1] and down.shape[1] % 64 == 0 and down.shape[0] % 16 == 0)
+        if type(up) not in _PLAIN or type(down) not in _PLAIN or gate_up.bias is not None or gate_down.bias is not None:
+            return False
+        (rows, inputs), (n, k), (width, ff) = h.shape, up.shape, down.shape
+        return (up.dtype == down.dtype == h.dtype and up.device == down.device == h.device and up.is_contiguous() and down.is_contiguous()
+                and n == 2 * ff and k == inputs and ff % 64 == 0 and width % 16 == 0 and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0
+                # offsets of 32 bits into weights and, unsigned, rows
+                and n * k < 1 << 30 and width * ff < 1 << 30 and _span(h) < 1 << 31 and rows * ff < 1 << 31)
 
     def _beside_pays(self, rows: int) -> bool:
         """Whether the shared expert's products are better off in the experts' launches.
