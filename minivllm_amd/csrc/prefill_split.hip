@@ -477,7 +477,7 @@ static float chain_us(const CachedBatch& b, int64_t x, bool pairs) {
 // random ones of 7 tiles and more, 64 to 420 workgroups, caches warm: with the range that it chooses 1.047 times as fast as before on average, 2 % of them more
 // than 3 % slower.  300 others of seven kinds of heads, 1 to 24 sequences: 1.036, between 0.953 and 1.269.  us before and now: one sequence of 451 rows,
 // 141 tiles of 64 dims 42.8 / 35.4; two of 466, 73 tiles 42.0 / 36.7; three of 682, 26 tiles of 64 dims 23.8 / 20.3; one of 980, 31 tiles, 32 heads 46.9 / 42.1;
-// but two of 2752, 67 tiles 113 / 117.  Packed ones, whose row tiles differ, in 1000 batches: 13 to 16 tiles up to 256 workgroups 1.03 times as fast, 16 to 22 up to
+// but two of 2752, 67 tiles 113 / 117.  188 more, 30 to 97 % cached: 61 in two groups, 1.085 times as fast, one 0.929 (seven of 742 rows, 98 tiles 52.4 / 56.4).  Packed ones, whose row tiles differ, in 1000 batches: 13 to 16 tiles up to 256 workgroups 1.03 times as fast, 16 to 22 up to
 // 320 1.07, 22 to 32 up to 400 1.04 to 1.14, 32 to 50 up to 480 1.15 to 1.24 (3071 rows, 64 dims 41.2 / 34.4); on the line's other side 10 to 13 tiles 0.99, 13 to
 // 16 and 320 to 400 workgroups 0.92, 22 to 32 and 480 to 600 0.93.
 static bool pairs_pay(int num_seqs, int64_t total_q, int64_t max_kv_len, int num_heads, int num_kv_heads, int head_dim, bool paged, int64_t range_tiles) {
